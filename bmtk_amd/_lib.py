@@ -56,11 +56,11 @@ class Glif3Bwd(C.Structure):
         ("lam_ring", c_void_p), ("gz", c_void_p),
         ("d_rec_w", c_void_p), ("d_inp_w", c_void_p),
         ("blk_count", c_int32), ("gz_planes", c_int32), ("blk_indptr", c_void_p), ("blk_packed", c_void_p),
-        ("d_blk_w", c_void_p),
+        ("d_blk_w", c_void_p), ("swept", c_int32), ("_pad0", c_int32),
     ]
 
 
-ABI_VERSION = 24  # BMTK_AMD_ABI_VERSION of include/bmtk_amd.h that the mirrors above were written for
+ABI_VERSION = 25  # BMTK_AMD_ABI_VERSION of include/bmtk_amd.h that the mirrors above were written for
 
 # name -> (restype, argtypes); every symbol include/bmtk_amd.h declares
 SIGNATURES = {

@@ -1,6 +1,8 @@
 // Reverse-time adjoint of the forward simulation: transposed propagation,
 // state adjoint, event-driven weight gradients.  The differentiable model
 // these kernels transpose is stated in include/bmtk_amd.h (bmtk_glif3_bwd).
+#include <type_traits>
+
 #include "common.hpp"
 #include "glif3_update.hpp"
 
@@ -880,6 +882,278 @@ __global__ __launch_bounds__(kBlock) void bwd_state2_kernel(bmtk_glif3_bwd a, Bw
     }
 }
 
+// The adjoint state of one element, its loss derivative and what of the forward record the swept form needs of it.
+template <bool kTwo>
+struct SweepElem {
+    float lV, lA[GLIF3_NASC], l1[GLIF3_NREC], l2[GLIF3_NREC], dl[kTwo ? 2 : 1], dl_const;
+
+    __device__ __forceinline__ void load(const bmtk_glif3_bwd &a, const BwdStep &q, int64_t e, int64_t ne)
+    {
+        lV = a.lam_V[e];
+#pragma unroll
+        for (int k = 0; k < GLIF3_NASC; ++k) lA[k] = a.lam_asc[k * ne + e];
+#pragma unroll
+        for (int k = 0; k < GLIF3_NREC; ++k) {
+            l1[k] = a.lam_y1[k * ne + e];
+            l2[k] = a.lam_y2[k * ne + e];
+        }
+        dl_const = a.dl_dz_const ? a.dl_dz_const[e] : 0.0f;
+#pragma unroll
+        for (int s = 0; s < (kTwo ? 2 : 1); ++s) dl[s] = a.dl_dz ? a.dl_dz[(q.row - s) * ne + e] : 0.0f;
+    }
+    // steps t and (kTwo) t-1 undone: g[s] = what comes back through the synapses, v[s], f[s] = potential and flags
+    __device__ __forceinline__ void undo(const bmtk_glif3_bwd &a, const BwdStep &q, const Glif3Prop &p, int64_t e, int64_t ne,
+                                         const float (&g)[2], const float (&v)[2], const unsigned (&f)[2])
+    {
+        const int L = a.ring_slots;
+        int slot = (int)(q.t % L);
+#pragma unroll
+        for (int s = 0; s < (kTwo ? 2 : 1); ++s) {
+            float gs = g[s];
+            if (a.dl_dz) gs += dl[s];
+            if (a.dl_dz_const) gs += dl_const;
+            const float sg = (f[s] & BMTK_F_INTEGRATING) ? surrogate(v[s], p.th, a.dampening) * gs : 0.0f;
+            state_adjoint_step(lV, lA, l1, l2, p, a.h, (uint8_t)f[s], sg);
+            // slot t-1 (t-2): what the launches ahead read of the step before
+            slot = slot == 0 ? L - 1 : slot - 1;
+            float *cells = a.lam_ring + (int64_t)slot * GLIF3_NREC * ne + e;
+#pragma unroll
+            for (int k = 0; k < GLIF3_NREC; ++k) cells[k * ne] = p.psc0[k] * l1[k];
+        }
+        a.lam_V[e] = lV;
+#pragma unroll
+        for (int k = 0; k < GLIF3_NASC; ++k) a.lam_asc[k * ne + e] = lA[k];
+#pragma unroll
+        for (int k = 0; k < GLIF3_NREC; ++k) {
+            a.lam_y1[k * ne + e] = l1[k];
+            a.lam_y2[k * ne + e] = l2[k];
+        }
+    }
+};
+
+// The swept form of a backward step, for networks whose adjoint ring the L2s hold (batches that are a multiple of 4 up to
+// 64): transposed propagation, weight gradients and state adjoint of step t -- with kTwo of steps t and t-1 -- in ONE
+// launch through the plain source-major table.  At these sizes a step's launches are short chains of dependent loads,
+// not traffic: what counts is how many launches a step takes and how long the chain in each is.
+//
+// A row's synapses are shared by `splits` neighbouring lane groups of LP lanes (four trials each), as many as the chip
+// has room for (3001 rows x batch 12: 33 / 19 / 12 / 10 us per step with 1 / 2 / 4 / 16 groups a row; 14461 rows: 32 / 32 / 42
+// / 55); they take the row's batches of kF synapses in turn and fold their sums at the end.  A row's sum is then
+// complete in one wavefront and the state adjoint of its elements follows in the same launch.  For that the adjoint
+// ring has two slots more than the table's delays need (ring_slots >= largest delay + 3): while some wavefronts still
+// read the slots t .. t+L-1, others write slots t-1 and t-2.  Slot s holds psc0 times the adjoint of y1 before step s is
+// undone; slot t was written by the launch before (bwd_seed_slot_kernel at the start of a call).
+//
+// Per step, gather and state adjoint as launches of their own against this form: 3001 neurons x batch 12, in-degree 200:
+// 21.8 -> 10.2 us; 6920 x 16, in-degree 525: 56 -> 33; 30000 x 16, in-degree 300: 194 -> 124.  What bounds it: at the smallest sizes the chain
+// row bounds -> records -> adjoint rows -> state (a launch starts with cold L2s, 1 to 2.5 us a link), above some 5,000 rows
+// the rate at which the L2s hand out adjoint rows (2.6e11 lines of 64 bytes per second).  Rings that the L2s do not
+// hold make it pay fabric latency per row, and the blocked table wins (51978 x 32, in-degree 1000: 546 against 740 us).
+struct SweepLaunch {
+    int splits;      // lane groups that share a row, a power of two
+    int n_row_wg;    // workgroups that hold rows; the ones behind them take the input-weight gradients
+    int n_sets;      // sets of rows (what a wavefront holds at a time)
+    int do_grad;
+};
+constexpr int kSweepThreads = 256;
+constexpr int kSweepWaves = kSweepThreads / kWave;
+constexpr int kSweepPerCu = 3;  // workgroups a compute unit holds: 168 vector registers per lane
+
+// kOne: a wavefront holds one row.  What belongs to the row is then the same in all lanes (scalar loads, which leave the
+// vector memory path to the adjoint rows), a lane has at most one element of it to undo, and its state is asked for before
+// the sums are taken.
+template <int LP, bool kOne, bool kTwo>
+__global__ __launch_bounds__(kSweepThreads, kSweepPerCu) void bwd_sweep_kernel(bmtk_glif3_bwd a, BwdStep q, SweepLaunch sw)
+{
+    constexpr int kF = kOne ? 4 : 8;                         // synapses of a row in flight per lane group
+    constexpr int kRecs = kF / LP > 1 ? kF / LP : 1;         // records a lane fetches of them
+    constexpr int kPer = kWave / LP;
+    constexpr int kSteps = kTwo ? 2 : 1;
+    const int batch = a.batch;
+    const int64_t n = a.n_neurons, ne = n * batch;
+    const int L = a.ring_slots;
+    const int lane = lane_id(), wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
+    if ((int)blockIdx.x >= sw.n_row_wg) {
+        const int w = ((int)blockIdx.x - sw.n_row_wg) * kSweepWaves + wave, nw = ((int)gridDim.x - sw.n_row_wg) * kSweepWaves;
+        if (kTwo)
+            bwd_inp_grad2_waves(a, q, w, nw);
+        else
+            bwd_inp_grad_waves(a, q, w, nw);
+        return;
+    }
+    const int grp = lane / LP, in_row = lane & (LP - 1), b4 = in_row * 4;
+    const int S = kOne ? kPer : sw.splits, part = grp & (S - 1);
+    const int rows_set = kPer / S;
+    const bool lane_on = b4 < batch;
+    const uint2 *__restrict__ rows = reinterpret_cast<const uint2 *>(a.rec_packed);
+    const char *__restrict__ ring = reinterpret_cast<const char *>(a.lam_ring);
+    const unsigned lane_off = (unsigned)(lane_on ? b4 : 0) * 4u;
+    const unsigned q_lo = (unsigned)(q.t % L) * 4u, q_wrap = q_lo - 4u * (unsigned)L;
+    const unsigned ne32 = (unsigned)ne, batch32 = (unsigned)batch;
+    // from a synapse's cell for step t to its cell for step t-1: one slot down, or L-1 slots up from slot 0 (bytes)
+    const unsigned slot_down = 0u - 16u * ne32, slot_up = 16u * ne32 * (unsigned)(L - 1);
+    const unsigned long long grp_lanes = (LP == kWave ? ~0ull : ((1ull << LP) - 1ull)) << (grp * LP);
+
+    for (int set = (int)blockIdx.x * kSweepWaves + wave; set < sw.n_sets; set += sw.n_row_wg * kSweepWaves) {
+        const int64_t row_set = kOne ? (int64_t)set : (int64_t)set * rows_set + grp / S;
+        const bool have = row_set < n;
+        const int64_t row = have ? row_set : n - 1;  // (lanes past the last row load what the last one loads)
+        int p = a.rec_indptr[row];
+        const int p1 = have ? a.rec_indptr[row + 1] : p;
+        const int64_t col = a.class_id ? (int64_t)a.class_id[row] : row;
+        const int64_t e4 = row * batch + (lane_on ? b4 : 0);
+        p = min(p + part * kF, p1);
+        // records p .. p+kF-1 of the row, one (kRecs) per lane; places past the row's end repeat its last record
+        uint2 rec[kRecs];
+        const int last = max(p1, 1) - 1;
+        auto fetch = [&](int from) {
+#pragma unroll
+            for (int i = 0; i < kRecs; ++i) rec[i] = rows[min(from + i * LP + in_row, last)];
+        };
+        bool busy = __ballot(p < p1) != 0ull;
+        if (busy) fetch(p);
+        float4 v4[kSteps];
+        uint32_t f4[kSteps];
+        unsigned fire = 0u;  // bits 0-3: the lane's trials in which the source fired in step t, 4-7: in step t-1
+#pragma unroll
+        for (int s = 0; s < kSteps; ++s) {
+            f4[s] = *reinterpret_cast<const uint32_t *>(a.save_flags + (q.row - s) * ne + e4);
+            v4[s] = *reinterpret_cast<const float4 *>(a.save_v + (q.row - s) * ne + e4);
+            if (sw.do_grad && have && lane_on)
+                fire |= ((unsigned)(trial_mask(a.spike_bits + (q.row - s) * a.spike_bits_stride, row, batch, 0, batch) >> b4) & 0xFu) << (4 * s);
+        }
+        Glif3Prop pr;
+        SweepElem<kTwo> el;
+        if (kOne) {
+            pr.load(a.prop, a.prop_stride, col);
+            if (kPer >= 4) el.load(a, q, e4 + (part & 3), ne);
+        }
+        const bool grad = sw.do_grad && __ballot(fire != 0u) != 0ull;
+        const bool row_fired = (__ballot(fire != 0u) & grp_lanes) != 0ull;
+        if (!kOne) {
+            // a row none of whose trials has a surrogate derivative, and whose source did not fire, needs no sum
+            const float th = a.prop[GLIF3_TH * a.prop_stride + col];
+            bool want = fire != 0u;
+#pragma unroll
+            for (int s = 0; s < kSteps; ++s)
+                want = want || ((f4[s] & (BMTK_F_INTEGRATING << 0)) && fabsf((v4[s].x - th) / th) < 1.0f) ||
+                       ((f4[s] & (BMTK_F_INTEGRATING << 8)) && fabsf((v4[s].y - th) / th) < 1.0f) ||
+                       ((f4[s] & (BMTK_F_INTEGRATING << 16)) && fabsf((v4[s].z - th) / th) < 1.0f) ||
+                       ((f4[s] & (BMTK_F_INTEGRATING << 24)) && fabsf((v4[s].w - th) / th) < 1.0f);
+            if ((__ballot(want && lane_on) & grp_lanes) == 0ull) p = p1;
+            busy = __ballot(p < p1) != 0ull;
+        }
+        float4 sum[kSteps];
+#pragma unroll
+        for (int s = 0; s < kSteps; ++s) sum[s] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        // record u of the batch, from the lane that fetched it
+        auto record = [&](int u) {
+            const uint2 r = rec[kRecs > 1 ? u / LP : 0];
+            if (LP == 1) return r;
+            const int src = (lane & ~(LP - 1)) + (u & (LP - 1));
+            return make_uint2((unsigned)__shfl((int)r.x, src, kWave), (unsigned)__shfl((int)r.y, src, kWave));
+        };
+        auto turn = [&](auto with_grad) {
+            constexpr bool kG = decltype(with_grad)::value;
+            float4 x[kSteps][kF];
+            float w[kF];
+#pragma unroll
+            for (int u = 0; u < kF; ++u) {
+                const uint2 sy = record(u);
+                const unsigned dq = sy.x >> 24;
+                const unsigned plane = min(dq + q_lo, dq + q_wrap);  // (slot of step t + delay) * 4 + receptor
+                const unsigned off_t = (mad_u24(sy.x, batch32, mul_u24(plane, ne32)) << 2) + lane_off;
+                w[u] = p + u < p1 ? __uint_as_float(sy.y) : 0.0f;  // (past the row's end: its last record with weight 0)
+                x[0][u] = *reinterpret_cast<const float4 *>(ring + off_t);
+                if (kTwo) x[kSteps - 1][u] = *reinterpret_cast<const float4 *>(ring + (off_t + (plane < 4u ? slot_up : slot_down)));
+            }
+            float old[kRecs];
+            if (kG) {
+#pragma unroll
+                for (int i = 0; i < kRecs; ++i) old[i] = a.d_rec_w[min(p + i * LP + in_row, last)];
+            }
+            const int next = min(p + S * kF, p1);
+            fetch(next);
+#pragma unroll
+            for (int u = 0; u < kF; ++u) {
+#pragma unroll
+                for (int s = 0; s < kSteps; ++s) {
+                    sum[s].x = fmaf(w[u], x[s][u].x, sum[s].x);
+                    sum[s].y = fmaf(w[u], x[s][u].y, sum[s].y);
+                    sum[s].z = fmaf(w[u], x[s][u].z, sum[s].z);
+                    sum[s].w = fmaf(w[u], x[s][u].w, sum[s].w);
+                }
+            }
+            if (kG) {
+                // gradient of a record: over the row's lanes, the adjoint entries of the trials in which the source
+                // fired; every lane gets every sum and keeps those of the records it fetched
+                float keep[kRecs];
+#pragma unroll
+                for (int i = 0; i < kRecs; ++i) keep[i] = 0.0f;
+#pragma unroll
+                for (int u = 0; u < kF; ++u) {
+                    float g = 0.0f;
+#pragma unroll
+                    for (int s = 0; s < kSteps; ++s) {
+                        const unsigned m = fire >> (4 * s);
+                        g += ((m & 1u) ? x[s][u].x : 0.0f) + ((m & 2u) ? x[s][u].y : 0.0f) + ((m & 4u) ? x[s][u].z : 0.0f) +
+                             ((m & 8u) ? x[s][u].w : 0.0f);
+                    }
+                    if (LP > 1) g += dpp_move<0xB1>(g);   // quad_perm [1,0,3,2]
+                    if (LP > 2) g += dpp_move<0x4E>(g);   // quad_perm [2,3,0,1]
+                    if (LP > 4) g += dpp_move<0x141>(g);  // row_half_mirror: the other quad of these eight lanes
+                    if (LP > 8) g += dpp_move<0x140>(g);  // row_mirror: the other eight of these sixteen
+                    if (in_row == (kRecs > 1 ? (u & (LP - 1)) : u)) keep[kRecs > 1 ? u / LP : 0] = g;
+                }
+#pragma unroll
+                for (int i = 0; i < kRecs; ++i) {
+                    const int at = p + i * LP + in_row;
+                    if (row_fired && i * LP + in_row < kF && at < p1) a.d_rec_w[at] = old[i] + keep[i];
+                }
+            }
+            p = next;
+        };
+        while (busy) {
+            if (grad)
+                turn(std::true_type{});
+            else
+                turn(std::false_type{});
+            busy = __ballot(p < p1) != 0ull;
+        }
+        // ---- the row's sum is complete: the state adjoint of its elements ----
+#pragma unroll
+        for (int s = 0; s < kSteps; ++s)
+            for (int off = LP; off < S * LP; off <<= 1) {
+                sum[s].x += __shfl_xor(sum[s].x, off, kWave);
+                sum[s].y += __shfl_xor(sum[s].y, off, kWave);
+                sum[s].z += __shfl_xor(sum[s].z, off, kWave);
+                sum[s].w += __shfl_xor(sum[s].w, off, kWave);
+            }
+        auto undo = [&](int c) {
+            float g[2] = {0.0f, 0.0f}, v[2] = {0.0f, 0.0f};
+            unsigned f[2] = {0u, 0u};
+#pragma unroll
+            for (int s = 0; s < kSteps; ++s) {
+                g[s] = c == 0 ? sum[s].x : c == 1 ? sum[s].y : c == 2 ? sum[s].z : sum[s].w;
+                v[s] = c == 0 ? v4[s].x : c == 1 ? v4[s].y : c == 2 ? v4[s].z : v4[s].w;
+                f[s] = (f4[s] >> (8 * c)) & 0xFFu;
+            }
+            el.undo(a, q, pr, e4 + c, ne, g, v, f);
+        };
+        if (have && lane_on && part < 4) {
+            if (kOne && kPer >= 4) {
+                undo(part);
+            } else {
+                if (!kOne) pr.load(a.prop, a.prop_stride, col);
+                for (int c = part; c < 4; c += S) {
+                    el.load(a, q, e4 + c, ne);
+                    undo(c);
+                }
+            }
+        }
+    }
+}
+
 // ring slot `slot` = psc0 times the present adjoint of y1: what the state adjoint of the step the slot belongs to
 // would write first, done ahead for the two-step form, whose transposed propagation reads it before that
 __global__ __launch_bounds__(kBlock) void bwd_seed_slot_kernel(bmtk_glif3_bwd a, int slot)
@@ -1238,6 +1512,68 @@ int blocked2_launch(const bmtk_glif3_bwd &a, const BwdStep &q, const BlockedPlan
     return BMTK_OK;
 }
 
+
+// ---- the swept form ----
+template <int LP>
+const void *sweep_variant(bool one, bool two)
+{
+    if (one)
+        return two ? reinterpret_cast<const void *>(bwd_sweep_kernel<LP, true, true>)
+                   : reinterpret_cast<const void *>(bwd_sweep_kernel<LP, true, false>);
+    return two ? reinterpret_cast<const void *>(bwd_sweep_kernel<LP, false, true>)
+               : reinterpret_cast<const void *>(bwd_sweep_kernel<LP, false, false>);
+}
+
+struct SweepPlan {
+    int lp;
+    SweepLaunch launch;
+    unsigned grid;
+};
+
+int sweep_plan(const bmtk_glif3_bwd &a, SweepPlan &pl)
+{
+    BMTK_REQUIRE(a.batch % 4 == 0 && a.batch <= kWave, "glif3_simulate_bwd: the swept form serves batches that are a multiple of 4 up to 64");
+    const int64_t ne = a.n_neurons * a.batch;
+    BMTK_REQUIRE(ne < (1ll << 24) && (int64_t)a.ring_slots * GLIF3_NREC * ne < (1ll << 30),
+                 "glif3_simulate_bwd: the swept form needs fewer than 2^24 elements and an adjoint ring below 4 GB");
+    BMTK_REQUIRE(a.rec_indptr && a.rec_packed && a.ring_slots >= 4,
+                 "glif3_simulate_bwd: the swept form needs the recurrent table and ring_slots >= largest delay + 3");
+    int dev = 0, n_cu = 256;
+    (void)hipGetDevice(&dev);
+    (void)hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev);
+    pl.lp = 1;
+    while (pl.lp * 4 < a.batch) pl.lp <<= 1;
+    const int per = kWave / pl.lp;
+    const int64_t groups = (int64_t)n_cu * kSweepPerCu * kSweepWaves * per;  // lane groups the chip holds
+    pl.launch.splits = 1;
+    while (pl.launch.splits < per && a.n_neurons * pl.launch.splits * 2 <= groups) pl.launch.splits *= 2;
+    if (std::getenv("SPL")) pl.launch.splits = std::atoi(getenv("SPL"));
+    if (pl.launch.splits > per) pl.launch.splits = per;
+    const int rows_set = per / pl.launch.splits;
+    pl.launch.n_sets = (int)((a.n_neurons + rows_set - 1) / rows_set);
+    pl.launch.n_row_wg = (pl.launch.n_sets + kSweepWaves - 1) / kSweepWaves;
+    pl.launch.do_grad = a.d_rec_w != nullptr ? 1 : 0;
+    pl.grid = (unsigned)(pl.launch.n_row_wg + (a.d_inp_w ? n_cu : 0));
+    return BMTK_OK;
+}
+
+int sweep_launch(const bmtk_glif3_bwd &a, const SweepPlan &pl, const BwdStep &q, bool two, hipStream_t st)
+{
+    bmtk_glif3_bwd args = a;
+    BwdStep step = q;
+    SweepLaunch launch = pl.launch;
+    void *params[] = {&args, &step, &launch};
+    const bool one = launch.splits == kWave / pl.lp;
+    const void *fn = pl.lp == 1 ? sweep_variant<1>(one, two) : pl.lp == 2 ? sweep_variant<2>(one, two)
+                   : pl.lp == 4 ? sweep_variant<4>(one, two) : pl.lp == 8 ? sweep_variant<8>(one, two) : sweep_variant<16>(one, two);
+    const hipError_t err = hipLaunchKernel(fn, dim3(pl.grid), dim3(kSweepThreads), params, 0, st);
+    if (err != hipSuccess) {
+        set_error("glif3_simulate_bwd: launch failed: %s", hipGetErrorString(err));
+        return BMTK_E_LAUNCH;
+    }
+    return BMTK_OK;
+}
+
 }  // namespace
 
 namespace {
@@ -1295,6 +1631,22 @@ extern "C" int bmtk_glif3_simulate_bwd(const bmtk_glif3_bwd *bwd, int64_t step0,
     int bp = 1;  // trial-tile width: the batch rounded up to a power of two, at most one wavefront
     while (bp < a.batch && bp < kWave) bp <<= 1;
     int64_t k_top = n_steps - 1;
+    if (a.swept) {
+        BMTK_REQUIRE(!blocked, "glif3_simulate_bwd: give the blocked table or ask for the swept form, not both");
+        SweepPlan sp{};
+        int rc = sweep_plan(a, sp);
+        if (rc != BMTK_OK) return rc;
+        if (n_steps > 0)
+            hipLaunchKernelGGL(bwd_seed_slot_kernel, dim3(elem_grid), dim3(kBlock), 0, st, a, (int)((step0 + k_top) % a.ring_slots));
+        while (k_top >= 0) {
+            const bool two = k_top >= 1;
+            rc = sweep_launch(a, sp, BwdStep{step0 + k_top, k_top, 1}, two, st);
+            if (rc != BMTK_OK) return rc;
+            k_top -= two ? 2 : 1;
+        }
+        BMTK_CHECK_LAUNCH("glif3_simulate_bwd");
+        return BMTK_OK;
+    }
     // Two steps per pass over the blocked table where gz has room for both steps' partial sums and a lane holds
     // whole adjoint rows of eight lanes (batches above 16): pairs (k, k-1) from the top, a step left over at the
     // end goes the one-step way.

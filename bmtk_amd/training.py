@@ -47,14 +47,33 @@ class Glif3Bptt:
     """Reverse-time adjoint over a recorded forward run of a ``Glif3Simulator``
     built with ``resident=False``."""
 
-    # adjoint rings above this size use the table regrouped by target range (the ring no longer fits the L2s)
-    BLOCKED_MIN_RING_BYTES = 32 << 20
+    # What a row's sum costs in the swept form grows once the L2s no longer hold the adjoint ring; in the blocked form it
+    # grows as a row's segments (its synapses into one target range) get short.  Measured on one MI355X, us per step swept /
+    # blocked (neurons x trials, in-degree; MB of ring, synapses per segment): 37000 x 32, 200 (114, 12) 198 / 256; 30000 x 32,
+    # 300 (92, 19) 189 / 221; 20000 x 32, 300 (61, 37) 111 / 127; 12000 x 32, 800 (37, 100) 108 / 113; 20000 x 32, 700 (61, 87) 208 / 198;
+    # 51978 x 24, 500 (120, 31) 696 / 558; 12000 x 40, 1000 (46, 125) 276 / 196; 16000 x 64, 400 (98, 25) 248 / 191; 51978 x 32, 1000
+    # (160, 42) 740 / 546.  Up to 16 trials the blocked form takes one step per pass over its table only: 30000 x 16, 1000 (46, 125)
+    # 342 / 403; 52000 x 12, 300 (60, 37) 331 / 357; 51978 x 16, 1000 (80, 62) 842 / 733.
+    BLOCKED_MIN_RING_MB = 40.0
+    BLOCKED_MIN_RING_MB_ONE_STEP = 64.0
+    BLOCKED_MIN_RING_TIMES_SEGMENT = 3000.0    # MB x synapses, at up to 32 trials; less above (longer adjoint rows)
 
-    def __init__(self, sim, dampening=0.3, blocked=None, n_blocks=None, two_steps=True):
-        """``blocked``: use the recurrent table regrouped by target range for the transposed propagation (None:
-        when the adjoint ring exceeds ``BLOCKED_MIN_RING_BYTES`` and the batch allows it); ``n_blocks``: number of
-        target ranges, a multiple of 8 (None: ``ops.blocked_table_blocks``); ``two_steps``: let the blocked form take
-        two steps per pass over its table (batches above 16; ``gz`` then holds the partial sums of both)."""
+    @classmethod
+    def blocked_pays(cls, n, batch, ring_slots, nnz):
+        """Whether the blocked form is expected to take less time per step than the swept form."""
+        from . import ops
+        ring_mb = ring_slots * NREC * n * batch * 4e-6
+        segment = nnz / float(n) / ops.blocked_table_blocks(n, batch, ring_slots)
+        return (ring_mb > (cls.BLOCKED_MIN_RING_MB if batch > 16 else cls.BLOCKED_MIN_RING_MB_ONE_STEP)
+                and ring_mb * segment * max(1.0, batch / 32.0) >= cls.BLOCKED_MIN_RING_TIMES_SEGMENT)
+
+    def __init__(self, sim, dampening=0.3, blocked=None, n_blocks=None, two_steps=True, swept=None):
+        """Three forms of the pass, the same gradients.  ``swept``: one launch per two steps through the plain
+        source-major table (its adjoint ring ``lam_ring`` has two slots more than ``sim.L``); ``blocked``: the recurrent
+        table regrouped by target range for the transposed propagation; neither: a launch per part and step, any batch.
+        None leaves the choice to ``blocked_pays`` where the batch (a multiple of 4 up to 64) allows it.  ``n_blocks``:
+        number of target ranges, a multiple of 8 (None: ``ops.blocked_table_blocks``); ``two_steps``: let the blocked form
+        take two steps per pass over its table (batches above 16; ``gz`` then holds the partial sums of both)."""
         if sim.res_span or sim.delay_offset:
             raise ValueError("the backward pass needs a simulator built with resident=False and delay_offset 0")
         self.sim, self.dampening = sim, float(dampening)
@@ -64,13 +83,21 @@ class Glif3Bptt:
         self.lam_asc = torch.zeros(NASC, ne, device=dev)
         self.lam_y1 = torch.zeros(NREC, ne, device=dev)
         self.lam_y2 = torch.zeros(NREC, ne, device=dev)
-        self.lam_ring = torch.zeros(sim.L, NREC, ne, device=dev)
-        self.d_rec_w = torch.zeros(sim.rec.nnz, device=dev) if sim.rec is not None else None
-        can_block = sim.rec is not None and sim.batch % 4 == 0 and sim.batch <= 64 and sim.L * NREC * ne < (1 << 30)
-        if blocked is None:
-            blocked = can_block and sim.L * NREC * ne * 4 > self.BLOCKED_MIN_RING_BYTES
-        elif blocked and not can_block:
+        grouped = sim.rec is not None and sim.batch % 4 == 0 and sim.batch <= 64
+        can_block = grouped and sim.L * NREC * ne < (1 << 30)
+        can_sweep = grouped and ne < (1 << 24) and sim.L + 2 <= 64 and (sim.L + 2) * NREC * ne < (1 << 30)
+        if swept and (blocked or not can_sweep):
+            raise ValueError("the swept form needs a recurrent table, a batch that is a multiple of 4 up to 64, delays within 61 "
+                             "steps and no blocked table")
+        if blocked and not can_block:
             raise ValueError("the blocked table needs a recurrent table and a batch that is a multiple of 4 up to 64")
+        if blocked is None and not swept:
+            blocked = can_block and (swept is False or not can_sweep or self.blocked_pays(sim.n, sim.batch, sim.L, sim.rec.nnz))
+            swept = not blocked and can_sweep and swept is None
+        self.swept, blocked = bool(swept), bool(blocked)
+        # (the swept form writes the adjoint slots of two steps ahead while others are still read)
+        self.lam_ring = torch.zeros(sim.L + (2 if self.swept else 0), NREC, ne, device=dev)
+        self.d_rec_w = torch.zeros(sim.rec.nnz, device=dev) if sim.rec is not None else None
         self.blk = None
         if blocked:
             from . import ops
@@ -95,7 +122,8 @@ class Glif3Bptt:
             raise ValueError("forward run was made without save_state=True or without spike bits")
         n_steps = bits.shape[0]
         a = _lib.Glif3Bwd()
-        a.n_neurons, a.batch, a.ring_slots, a.h, a.dampening = sim.n, sim.batch, sim.L, sim.h, self.dampening
+        a.n_neurons, a.batch, a.ring_slots, a.h, a.dampening = sim.n, sim.batch, self.lam_ring.shape[0], sim.h, self.dampening
+        a.swept = 1 if self.swept and not blocked else 0
         a.prop, a.prop_stride, a.class_id = _p(sim.prop), sim.prop.shape[1], _p(sim.class_id)
         a.save_v, a.save_flags = _p(saved["v"], torch.float32, n_steps * sim.ne), _p(saved["flags"], torch.uint8)
         a.spike_bits, a.spike_bits_stride = _p(bits, torch.int64), bits.shape[1]

@@ -49,7 +49,7 @@ extern "C" {
 
 /* Bumped whenever a struct layout or a signature below changes; bmtk_amd_abi_version() returns the value the
  * library was built with. */
-#define BMTK_AMD_ABI_VERSION 24
+#define BMTK_AMD_ABI_VERSION 25
 int bmtk_amd_abi_version(void);
 const char *bmtk_amd_last_error(void);
 /* sizeof(bmtk_glif3_sim) as the library was compiled, for bindings that mirror the struct */
@@ -523,6 +523,13 @@ typedef struct bmtk_glif3_bwd {
     const bmtk_synapse *blk_packed;
     float *d_blk_w;                /* [rec nnz] recurrent weight gradient in the order of blk_packed, accumulated,
                                       or NULL (then d_rec_w, if given, is filled through rec_indptr / rec_packed) */
+    /* Optional, for batches that are a multiple of 4 up to 64, without the blocked table: non-zero asks for the swept
+     * form, in which ONE launch per two steps takes the transposed propagation, the weight gradients and the state
+     * adjoint along, all rows under way at once (rows ordered by target keep what the chip reads of lam_ring within the
+     * L2s).  It writes slots of lam_ring ahead of their steps: ring_slots must be at least the largest delay + 3.
+     * Needs fewer than 2^24 elements and a lam_ring below 4 GB; gz is not used. */
+    int32_t swept;
+    int32_t _pad0;
 } bmtk_glif3_bwd;
 
 /* Differentiate steps step0+n_steps-1 down to step0.  Per step: the transposed propagation (the weight gradients

@@ -344,3 +344,52 @@ def test_two_step_backward_on_randomly_shaped_networks(seed):
     for name in ("d_rec_w", "d_inp_w"):
         got, want = getattr(two, name), getattr(one, name)
         assert float((got - want).abs().max()) <= 1e-6 * max(float(want.abs().max()), 1e-30), (name, batch, n)
+
+
+@pytest.mark.parametrize("n,batch,steps,p_conn", [
+    (1, 4, 5, 0.0), (3, 4, 9, 0.7), (63, 8, 17, 0.2), (64, 12, 18, 0.2), (65, 16, 16, 0.2),   # one row per wavefront
+    (700, 64, 12, 0.02), (3073, 32, 7, 0.005),                                                # ... and a few rows beyond
+    (6200, 32, 6, 0.003), (13000, 8, 5, 0.002), (9000, 64, 5, 0.002), (60000, 4, 4, 3e-4)])   # several rows, several sets
+def test_swept_form_equals_the_parts(n, batch, steps, p_conn):
+    """The swept backward pass (one launch per two steps) against the loop over the three per-step entry points, which
+    autograd pins above, over the lane-group splits the launch plan can choose.  A row's products are added in another
+    order, so adjoint state and gradients agree to 4e-6 of the 2-norm: a few fp32 roundings (6e-8 each) per step over at
+    most 18 steps.  An odd number of steps leaves one step for the single-step kernel; two calls on chunks equal one call
+    bit for bit."""
+    rng = np.random.default_rng(n + batch)
+    cells = synthetic.random_cells(rng, 5)
+    nnz = int(n * n * p_conn)
+    src, tgt = rng.integers(0, n, nnz), rng.integers(0, n, nnz)
+    from bmtk_amd import network as net
+    rec = net.coo_to_csr(src, tgt, rng.normal(0, 3, nnz).astype(np.float32), rng.integers(1, 6, nnz), rng.integers(0, 4, nnz), n)
+    n_in = 7
+    isrc, itgt = rng.integers(0, n_in, 40 * n // 10 + 9), rng.integers(0, n, 40 * n // 10 + 9)
+    inp = net.coo_to_csr(isrc, itgt, np.full(isrc.size, 400.0, np.float32), rng.integers(1, 6, isrc.size), np.zeros(isrc.size), n_in)
+    in_ptr, in_ev = synthetic.poisson_events(rng, n_in, 200.0, 1.0, steps, batch)
+    sim = Glif3Simulator(n, cells, 1.0, batch=batch, class_id=rng.integers(0, 5, n), rec=rec, inp=inp, ring_slots=6,
+                         resident=False)
+    sim.set_input_events(in_ptr, in_ev)
+    cut = steps // 2
+    chunks = [sim.run(cut, save_state=True), sim.run(steps - cut, save_state=True)]
+    dl = [torch.as_tensor(rng.normal(size=(c["bits"].shape[0], n * batch)).astype(np.float32), device="cuda") for c in chunks]
+    if nnz == 0:
+        with pytest.raises(ValueError):
+            training.Glif3Bptt(sim, swept=True)
+        return
+    swept = training.Glif3Bptt(sim, swept=True)
+    assert swept.swept and swept.lam_ring.shape[0] == 8
+    parts = training.Glif3Bptt(sim, blocked=False, swept=False)
+    for c, d in zip(reversed(chunks), reversed(dl)):
+        swept.backward(c, dl_dz=d)
+        parts.backward_stepwise(c, dl_dz=d)
+    for name in ("lam_V", "lam_asc", "lam_y1", "lam_y2", "d_rec_w", "d_inp_w"):
+        got, want = getattr(swept, name).double(), getattr(parts, name).double()
+        assert float((got - want).norm()) <= 4e-6 * float(want.norm()), name
+    assert float(swept.lam_V.abs().max()) > 0
+    # (the two calls together as one: same sums, same order)
+    whole = dict(saved=dict(v=torch.cat([c["saved"]["v"] for c in chunks]), flags=torch.cat([c["saved"]["flags"] for c in chunks]),
+                            step0=0), bits=torch.cat([c["bits"] for c in chunks]))
+    one = training.Glif3Bptt(sim, swept=True)
+    one.backward(whole, dl_dz=torch.cat(dl))
+    for name in ("lam_V", "lam_asc", "lam_y1", "lam_y2"):
+        assert torch.equal(getattr(one, name), getattr(swept, name)), name
