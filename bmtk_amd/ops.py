@@ -248,6 +248,12 @@ class SynapseTable:
             self._packed = out
         return self._packed
 
+    def pad_packed(self, records):
+        """Lay the packed records out with ``records`` more behind them (zeros), for kernels that read past the end."""
+        out = torch.zeros(self.nnz + records, 2, dtype=torch.int32, device=self.indices.device)
+        out[:self.nnz] = self.packed()[:self.nnz]
+        self._packed = out
+
     def sorted_by_index(self):
         """The same table with every row ordered by index (stable), as the segment offsets need."""
         rows = torch.repeat_interleave(torch.arange(self.n_rows, device=self.indices.device),

@@ -18,19 +18,24 @@ from .ops import Glif3State, SpikeCompactor, SynapseTable, _dev, _p, _stream, gl
 
 PULL_MAP_BYTES = 40 * 1024      # activity map of bmtk_csr_propagate_pull: what is left of 80 KB beside its accumulators
 PULL_MIN_DENSITY = 0.06         # synaptic events per synapse and step from which "auto" pulls instead of pushing
-                                # (the unfused pull form: batches other than 8, 16, 32, 64)
+                                # (the unfused pull form: batches below 8 and above 64)
 # What a step of a batched run costs on one MI355X, in picoseconds, fitted to runs of 51,978 neurons x 60 M synapses at
 # batches 8, 16, 32 and 0 - 3.2 Hz and of 230,924 neurons x 77 M synapses at batch 8: the fused pull form streams the
 # joint table once per two steps (per synapse, divided by how full a row's blocks of 256 are) and adds a little per
 # synaptic event; the event-driven form pays per element for its update (less with a class table) and an atomic per event.
+# At the smallest sizes either form is a launch or two and its chains of dependent loads (600 neurons x 16: 7.0 us per step
+# fused, 5.6 pushed; 3,001 x 12: 8.3 and 9.1; 1,500 x 8: 7.2 and 10.1).
+FUSE_PS_PER_STEP = 5.05e6
+PUSH_PS_PER_STEP = 4.5e6
 FUSE_PS_PER_SYNAPSE = 1.35
 FUSE_PS_PER_EVENT = 6.0
 PUSH_PS_PER_ELEMENT = 55.0
 PUSH_PS_PER_ELEMENT_CLASS_TABLE = 27.0
 PUSH_PS_PER_EVENT = 48.0
-FUSE_LDS_BYTES = 150 * 1024     # LDS of one workgroup of the fused batched driver (kFuseLdsMax of csrc/simulate_fused.hip)
-FUSE_WAVES = 16                 # wavefronts of one of its workgroups (kFuseWaves)
-FUSE_BATCHES = (8, 16, 32, 64)  # lane = trial, whole bytes of spike bits per neuron
+FUSE_LDS_BYTES = 160 * 1024 - 512   # LDS of one workgroup of the fused batched driver (kFuseLdsMax of csrc/simulate_fused.hip)
+FUSE_LDS_FIXED = 16 * (2 * NREC * 64 * 8 + 128 * 12)   # ... of it sums and stages (kFuseLdsFixed)
+FUSE_BATCHES = range(8, 65)         # lane = trial, at most eight neurons to a wavefront
+FUSE_PAD = 64                       # records behind its table (BMTK_FUSE_PAD)
 RES_LDS_BYTES = 160 * 1024      # LDS of one gfx950 compute unit
 RES_ACT_ENTRIES = 8192          # active-row list of the resident kernel (kActCap of csrc/resident.hip), 4 B each
 RES_LDS_EXTRA = RES_ACT_ENTRIES * 4 + 256   # the list plus the kernel's static LDS (rounded up)
@@ -70,9 +75,9 @@ def fused_pays(n_neurons, batch, n_synapses, class_table, rate_hz, h_ms=1.0):
     events = n_synapses * batch * float(rate_hz) * 1e-3 * h_ms
     row = n_synapses / float(n_neurons)
     blocks_full = row / (256.0 * math.ceil(row / 256.0))
-    fused = FUSE_PS_PER_SYNAPSE * n_synapses / blocks_full + FUSE_PS_PER_EVENT * events
+    fused = FUSE_PS_PER_STEP + FUSE_PS_PER_SYNAPSE * n_synapses / blocks_full + FUSE_PS_PER_EVENT * events
     push = ((PUSH_PS_PER_ELEMENT_CLASS_TABLE if class_table else PUSH_PS_PER_ELEMENT) * n_neurons * batch
-            + PUSH_PS_PER_EVENT * events)
+            + PUSH_PS_PER_EVENT * events + PUSH_PS_PER_STEP)
     return fused < push
 
 
@@ -102,7 +107,7 @@ class Glif3Simulator:
                 against 340 pushed; 230,924 neurons x 8 and x 16 at 2.8 Hz pushed 132 / 237 us against 321 / 358
                 pulled).  Default 3 Hz: batches from 20 at 1 ms steps.  That mark decides the unfused ``pull``;
                 ``fused`` is decided by ``fused_pays``, which compares the fitted cost of a step in either form.
-    fused       launch-per-step mode, batch 8, 16, 32 or 64, delay_offset 0: one launch per step in which a
+    fused       launch-per-step mode, batches of 8 to 64, delay_offset 0: one launch per two steps in which a
                 wavefront sums what arrives at a neuron -- over recurrent and input synapses, from a joint
                 target-major table and a joint history of spike and input-event bits -- and advances the neuron's
                 trials, lane = trial; no arrival sum passes through device memory.  "auto": when ``fused_pays``
@@ -222,6 +227,7 @@ class Glif3Simulator:
         self.in_ptr = self.in_events = None
         self.in_steps = 0
         self.in_duplicates = False
+        self._lists_replaced = False    # since the last run
         self.in_repeat_ptr = self.in_repeat_events = None   # repeated ids of a step, for the pull form of the inputs
         self.step = 0
         self.words = n_words(self.ne)
@@ -252,7 +258,7 @@ class Glif3Simulator:
                     and self.delay_bits == 6 and self.batch in FUSE_BATCHES and pull is not False)
         if fused is True and not can_fuse:
             raise ValueError("the fused form needs a synapse table, launch-per-step mode, delay_offset 0, delays "
-                             "within 63 steps and a batch of 8, 16, 32 or 64")
+                             "within 63 steps and a batch of 8 to 64")
         can_pull = (self.rec is not None and not self.res_span and self.delay_offset == 0
                     and self.L * ((self.n + 31) // 32) * 4 <= PULL_MAP_BYTES)
         # the pull form sums in 64-bit fixed point: weights must be finite and below 2^31 in size
@@ -269,6 +275,12 @@ class Glif3Simulator:
         if pull is True and not can_pull:
             raise ValueError("the pull form needs a recurrent table, launch-per-step mode, delay_offset 0 and "
                              "ring_slots * n_neurons / 8 bytes of LDS (at most 40 KB)")
+        # What separate launches would have pulled: their history of input events is read from the lists step by step, a
+        # call's first step the one before it once more.  The fused form does the same where it takes their place (at
+        # batches that do not divide 64), so that lists replaced between two calls mean what they meant there.
+        pulls = can_pull and (pull is True or (pull == "auto" and dense))
+        self.fuse_rereads = (pulls and 64 % self.batch != 0 and self.inp is not None
+                             and self.L * ((self.n_inputs + 31) // 32) * 4 <= PULL_MAP_BYTES)
         n_syn = sum(t.nnz for t in (self.rec, self.inp) if t is not None)
         if can_fuse and fused and (fused is True or pull is True or
                                    fused_pays(self.n, self.batch, n_syn, self.class_id is not None, expected_rate_hz, self.h)):
@@ -279,7 +291,7 @@ class Glif3Simulator:
                 raise ValueError("the fused form needs finite weights smaller than 2^31 in size")
         if self.fuse_table is not None:
             pass
-        elif can_pull and (pull is True or (pull == "auto" and dense)):
+        elif pulls:
             self.pull_table = self.rec.transposed(self.n)
             self.pull_syn = torch.zeros(NREC, self.ne, device=self.dev)
             need = self.lib.bmtk_csr_propagate_pull_workspace_bytes(self.L, self.n)
@@ -298,19 +310,20 @@ class Glif3Simulator:
     def _setup_fused(self):
         """Joint target-major table, joint history and activity map of the fused batched driver."""
         n, batch, n_in = self.n, self.batch, self.n_inputs if self.inp is not None else 0
-        self.fuse_in_base = -(-n * batch // 64) * 64 // batch
-        if self.fuse_in_base + n_in >= 2 ** 24:
+        rows = 64 // batch                   # neurons of a group: one word of a history row
+        self.fuse_in_base = -(-n // rows) * rows
+        if self.fuse_in_base + n_in + rows >= 2 ** 24:
             return
         self.fuse_table = SynapseTable.joined_by_target(self.rec, self.inp, n, self.fuse_in_base)
-        self.fuse_hist_stride = self.fuse_in_base * batch // 64 + n_words(n_in * batch) + 1
+        self.fuse_table.pad_packed(FUSE_PAD)
+        self.fuse_hist_stride = self.fuse_in_base // rows + -(-n_in // rows) + 1
         self.hist_slots = self.L + 4         # two steps per launch: rows read, written and cleared ahead
         self.ring = torch.zeros(self.L + 2, NREC, self.ne, device=self.dev)   # (its ring: two slots more)
         self.work_bits = torch.zeros(self.hist_slots * self.fuse_hist_stride, dtype=torch.int64, device=self.dev)
         # one bit of the activity map per 2^shift sources: the smallest shift whose map fits the LDS beside the
-        # accumulators (16 wavefronts x 2 arrival steps x (4 x 64 sums + a stage of 64 synapses) x 8 bytes)
-        fixed = FUSE_WAVES * 2 * (NREC * 64 + 64) * 8
+        # accumulators (where it also fits with a byte per source, the library takes that)
         self.fuse_shift = 0
-        while fixed + self.L * self._fuse_any_words() * 4 > FUSE_LDS_BYTES:
+        while FUSE_LDS_FIXED + self.L * self._fuse_any_words() * 4 > FUSE_LDS_BYTES:
             self.fuse_shift += 1
         self.fuse_any = self._new_fuse_any()
 
@@ -319,9 +332,8 @@ class Glif3Simulator:
         whose map fits the LDS).  Before the first run only."""
         if self.fuse_table is None or self.step:
             raise ValueError("set_fuse_shift applies to the fused form before its first run")
-        fixed = FUSE_WAVES * 2 * (NREC * 64 + 64) * 8
         old, self.fuse_shift = self.fuse_shift, int(shift)
-        if not 0 <= self.fuse_shift <= 16 or fixed + self.L * self._fuse_any_words() * 4 > FUSE_LDS_BYTES:
+        if not 0 <= self.fuse_shift <= 16 or FUSE_LDS_FIXED + self.L * self._fuse_any_words() * 4 > FUSE_LDS_BYTES:
             self.fuse_shift = old
             raise ValueError("shift must lie in 0..16 and leave the activity map within the LDS")
         self.fuse_any = self._new_fuse_any()
@@ -329,8 +341,10 @@ class Glif3Simulator:
     def _new_fuse_any(self):
         # the activity map (one row per history row) and, behind it, the map of ring cells that hold something
         # (one row per ring slot, a bit per neuron)
-        return torch.zeros(self.hist_slots * self._fuse_any_words() + (self.L + 2) * (-(-self.n // 32)), dtype=torch.int32,
-                           device=self.dev)
+        # (the form with a byte per source keeps two maps, rows padded to whole words of the history)
+        byte_words = -(-(self.fuse_hist_stride - 1) * (64 // self.batch) // 4)
+        words = max(self.hist_slots * self._fuse_any_words(), 2 * byte_words)
+        return torch.zeros(words + (self.L + 2) * (-(-self.n // 32)), dtype=torch.int32, device=self.dev)
 
     def _fuse_any_words(self):
         groups = -(-(self.fuse_in_base + (self.n_inputs if self.inp is not None else 0)) // (1 << self.fuse_shift))
@@ -433,6 +447,7 @@ class Glif3Simulator:
         self.in_ptr = in_ptr
         self.in_events = in_events if in_events.numel() else in_events.new_zeros(1)
         self.in_steps = in_ptr.numel() - 1
+        self._lists_replaced = self.step > 0
         self.in_duplicates = repeat is not None
         self.in_repeat_ptr = self.in_repeat_events = None
         if repeat is not None and (self.pull_inp_table is not None or self.fuse_table is not None):
@@ -472,6 +487,8 @@ class Glif3Simulator:
             s.fuse_indptr, s.fuse_packed = _p(self.fuse_table.indptr), _p(self.fuse_table.packed())
             s.fuse_any, s.fuse_hist_stride, s.fuse_in_base = _p(self.fuse_any), self.fuse_hist_stride, self.fuse_in_base
             s.fuse_shift, s.fuse_wg_per_cu = self.fuse_shift, self.fuse_wg_per_cu
+            s.fuse_max_team = max(1, -(-self.fuse_table.nnz // (256 * -(-self.n // (64 // self.batch)))))
+            s.in_again = 1 if self.fuse_rereads and self._lists_replaced else 0
             if self.in_repeat_ptr is not None:
                 s.in_repeat_ptr, s.in_repeat_events = _p(self.in_repeat_ptr), _p(self.in_repeat_events)
         if self.res_span:
@@ -563,6 +580,7 @@ class Glif3Simulator:
             s.probe_stride, s.probe_every = self.probe_ids.size, every
         _lib.check(self.lib.bmtk_glif3_simulate_fwd(C.byref(s), self.step, n_steps, _stream()))
         self.step += n_steps
+        self._lists_replaced = self._lists_replaced and n_steps == 0
         self._pending_check = bool(self.res_span)
         return dict(bits=bits, record=record, saved=saved, probe=probe)
 

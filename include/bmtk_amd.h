@@ -49,7 +49,7 @@ extern "C" {
 
 /* Bumped whenever a struct layout or a signature below changes; bmtk_amd_abi_version() returns the value the
  * library was built with. */
-#define BMTK_AMD_ABI_VERSION 25
+#define BMTK_AMD_ABI_VERSION 26
 int bmtk_amd_abi_version(void);
 const char *bmtk_amd_last_error(void);
 /* sizeof(bmtk_glif3_sim) as the library was compiled, for bindings that mirror the struct */
@@ -347,32 +347,43 @@ typedef struct bmtk_glif3_sim {
      * ring. */
     const int64_t *in_repeat_ptr;        /* [total steps + 1] */
     const int32_t *in_repeat_events;
-    /* Fused form of the batched driver (optional; launch-per-step mode, batch 8, 16, 32 or 64, delay_offset 0,
+    /* Fused form of the batched driver (optional; launch-per-step mode, batches of 8 to 64, delay_offset 0,
      * hist_slots == ring_slots + 4, `ring` of ring_slots + 2 slots; takes precedence over pull_*): one launch per TWO
-     * steps in which a wavefront takes 64 / batch target neurons at a time -- in one pass over a joint target-major
-     * table it sums what arrives at them in step t-1 and in step t over recurrent AND input synapses (64-bit fixed
+     * steps in which a wavefront takes R = 64 / batch (rounded down) target neurons at a time -- in one pass over a joint
+     * target-major table it sums what arrives at them in step t-1 and in step t over recurrent AND input synapses (64-bit fixed
      * point in LDS, as bmtk_csr_propagate_pull; both only depend on spikes up to step t-1, delays being at least one
      * step), folds the first sums into y1, advances the neurons' trials through step t, folds the second and
      * advances them through step t+1, lane = (neuron, trial); no arrival sum passes through device memory and the
      * table is read once per two steps.  The joint table's index field names a source of the joint space: neuron j is j,
-     * input source k is fuse_in_base + k, fuse_in_base = ceil(n_neurons*batch/64)*64/batch.  work_bits is then the
-     * joint history [hist_slots][fuse_hist_stride]: bit j*batch+b of row t % hist_slots = source j fired (or had an
-     * input event) in trial b of step t; a launch writes the input parts of the rows of its own two steps from in_ptr /
-     * in_events, for the launches after it.  Repeated ids of a step go through the ring as events (in_repeat_*, with inp_indptr /
-     * inp_packed), as in the pull form.  fuse_any is the "some trial fired" map of the joint sources, one bit per
-     * group of 2^fuse_shift sources and history row; a coarser map (larger shift) costs mask fetches for silent
-     * sources but is what lets any number of sources fit the LDS: ring_slots * fuse_any_words * 4 bytes beside
-     * the 80 KB of accumulators must stay within 150 KB. */
+     * input source k is fuse_in_base + k, fuse_in_base = n_neurons rounded up to a multiple of R.  work_bits is then the
+     * joint history [hist_slots][fuse_hist_stride]: word j / R of row t % hist_slots holds the trials of R sources, bit
+     * (j % R) * batch + b = source j fired (or had an input event) in trial b of step t; a launch writes the input parts of
+     * the rows of its own two steps from in_ptr / in_events, for the launches after it.  Repeated ids of a step go through
+     * the ring as events (in_repeat_*, with inp_indptr / inp_packed), as in the pull form.  fuse_any is the "some trial
+     * fired" map of the joint sources the kernel keeps in LDS beside 88 KB of accumulators.  With fuse_shift 0, ring_slots
+     * at most 8 and as many bytes of LDS as there are sources it holds one byte per source (bit t mod 8 = fired in step t) and
+     * fuse_any two such maps of fuse_byte_words = ceil((fuse_hist_stride - 1) * R / 4) words, which launches read and write in turn.
+     * Otherwise it holds one bit per group of 2^fuse_shift sources and history row; a coarser map (larger shift) costs
+     * mask fetches for silent sources but is what lets any number of sources fit the LDS: ring_slots * fuse_any_words * 4
+     * bytes within 70 KB.  Where R * batch is not 64, groups share words of spike_bits, which the call clears first. */
+#define BMTK_FUSE_PAD 64
     const int32_t *fuse_indptr;        /* [n_neurons + 1] */
-    const bmtk_synapse *fuse_packed;   /* rows = targets, index field = joint source */
-    uint32_t *fuse_any;                /* [hist_slots][fuse_any_words] followed by [ring_slots + 2][ceil(n_neurons/32)]
+    const bmtk_synapse *fuse_packed;   /* rows = targets, index field = joint source; followed by BMTK_FUSE_PAD zeroed records */
+    uint32_t *fuse_any;                /* max(hist_slots * fuse_any_words, 2 * fuse_byte_words) words followed by
+                                        * [ring_slots + 2][ceil(n_neurons/32)]
                                         * words (a bit per neuron and ring slot: the slot holds an arrival of a
                                         * repeated id for the neuron), zeroed with work_bits before the first run;
                                         * fuse_any_words = ceil(ceil((fuse_in_base + n_inputs) / 2^fuse_shift) / 32) */
-    int64_t fuse_hist_stride;          /* words per row of work_bits: >= fuse_in_base*batch/64 + ceil(n_inputs*batch/64) + 1 */
+    int64_t fuse_hist_stride;          /* words per row of work_bits: fuse_in_base / R + ceil(n_inputs / R) + 1 */
     int64_t fuse_in_base;
     int32_t fuse_shift;                /* 0..16 */
     int32_t fuse_wg_per_cu;            /* persistent workgroups per compute unit, 0 = the library's choice */
+    int32_t in_again;                  /* fused form: non-zero = the call begins by reading the input events of step step0 - 1
+                                        * from in_ptr / in_events again, as the pull form in separate launches always does
+                                        * (it matters to a caller that replaced the lists: those that say nothing was
+                                        * emitted in the steps behind take what step0 - 1 still had under way along) */
+    int32_t fuse_max_team;             /* fused form: most wavefronts that share a group of neurons in a network too small to
+                                        * give every wavefront one (0: 16): about as many as the group's run has blocks of 256 */
     /* outputs */
     uint64_t *spike_bits;        /* [n_steps][words] spike bits per step, words = ceil(ne/64); or NULL.
                                   * Row k belongs to step step0+k of the call that wrote it. */

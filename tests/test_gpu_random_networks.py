@@ -200,3 +200,42 @@ def test_many_workgroups_with_volleys_and_delay_offsets(seed):
             got = sim.state.to_numpy()
             for k in ("V", "asc", "y2", "ref"):
                 np.testing.assert_array_equal(got[k], st[k], err_msg="%s %s" % (k, tag))
+
+
+@pytest.mark.parametrize("batch,n,max_delay,shift", [
+    (9, 1, 1, None), (10, 5, 4, None), (10, 7, 7, None), (11, 64, 8, None), (12, 333, 5, None), (13, 66, 3, 2), (17, 3, 6, None),
+    (20, 900, 5, None), (21, 65, 12, None), (22, 17, 2, None), (31, 130, 7, 1), (33, 9, 5, None), (50, 310, 5, None),
+    (63, 21, 9, None)])
+def test_fused_driver_at_batches_that_do_not_divide_64(batch, n, max_delay, shift):
+    """Groups that do not fill a wavefront (one to seven neurons), their words of the history and their pieces of the
+    run's spike bits, ids repeated within a step, both kinds of activity map (a byte per source up to 8 history rows, bits
+    beyond and with a shift), an odd number of steps per call so that the maps change places: bit for bit the fp32
+    oracle, raster and state, over three calls."""
+    from test_gpu_simulate import _with_duplicate_events
+    cfg = synthetic.small_glif3_network(n=n, n_in=23, steps=90, seed=batch, p_conn=min(0.5, 30.0 / n), in_rate=60.0,
+                                        in_fanout=max(1, n // 3), max_delay=max_delay, n_classes=4 if n % 2 else None,
+                                        batch=batch, w_scale=6.0, in_w_scale=40.0)
+    for key in ("rec_src", "inp_src"):
+        indptr, indices, w, d, r = cfg[key]
+        cfg[key] = (indptr, indices, (np.round(w * 4.0) / 4.0 + np.sign(w) * 0.25).astype(np.float32), d, r)
+    in_ptr, in_events = _with_duplicate_events(cfg, np.random.default_rng(batch), batch)
+    i_ext = np.random.default_rng(n).uniform(0.0, 600.0, n * batch).astype(np.float32)
+    rec = cfg["rec_src"] if cfg["rec_src"][1].size else None
+    L = int(max([1] + [int(t[3].max()) for t in (rec, cfg["inp_src"]) if t is not None])) + 1
+    orc.set_threads(1)
+    st = orc.new_state(n, batch, np.float32)
+    want = orc.simulate(st, orc.precompute(cfg["par"], cfg["h"]), cfg["h"], 90, batch=batch, class_id=cfg["class_id"],
+                        ring=np.zeros((L, 4, n * batch), np.float32), rec=rec, inp=cfg["inp_src"], in_ptr=in_ptr,
+                        in_events=in_events, i_ext=i_ext, raster=True)
+    assert want["count"] > 0
+    sim = Glif3Simulator(n, cfg["par"], cfg["h"], batch=batch, class_id=cfg["class_id"], rec=rec, inp=cfg["inp_src"],
+                         i_ext=i_ext, resident=False, fused=True)
+    if shift:
+        sim.set_fuse_shift(shift)
+    sim.set_input_events(in_ptr, in_events)
+    assert sim.fuse_table is not None and sim.in_repeat_ptr is not None
+    ras = np.concatenate([sim.raster(sim.run(k)["bits"]).cpu().numpy() for k in (1, 33, 56)])
+    np.testing.assert_array_equal(ras, want["raster"])
+    got = sim.state.to_numpy()
+    for k in ("V", "asc", "y1", "y2", "ref"):
+        np.testing.assert_array_equal(got[k], st[k], err_msg=k)
