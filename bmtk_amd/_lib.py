@@ -35,6 +35,10 @@ class Glif3Sim(C.Structure):
         ("fuse_indptr", c_void_p), ("fuse_packed", c_void_p), ("fuse_any", c_void_p),
         ("fuse_hist_stride", c_int64), ("fuse_in_base", c_int64), ("fuse_shift", c_int32), ("fuse_wg_per_cu", c_int32),
         ("in_again", c_int32), ("fuse_max_team", c_int32),
+        ("rb_span", c_int32), ("rb_groups", c_int32), ("rb_ways", c_int32), ("rb_team_shift", c_int32),
+        ("rb_list", c_int32), ("rb_late_events", c_int32),
+        ("rb_seg", c_void_p), ("rb_packed", c_void_p), ("rb_ring", c_void_p), ("rb_hist", c_void_p),
+        ("rb_in_ptr", c_void_p), ("rb_in_events", c_void_p), ("rb_pend_until", c_int64),
         ("spike_bits", c_void_p), ("spike_bits_stride", c_int64),
         ("save_v", c_void_p), ("save_flags", c_void_p),
         ("probe_col", c_void_p), ("probe_v", c_void_p), ("probe_stride", c_int64), ("probe_every", c_int32),
@@ -61,7 +65,7 @@ class Glif3Bwd(C.Structure):
     ]
 
 
-ABI_VERSION = 26  # BMTK_AMD_ABI_VERSION of include/bmtk_amd.h that the mirrors above were written for
+ABI_VERSION = 27  # BMTK_AMD_ABI_VERSION of include/bmtk_amd.h that the mirrors above were written for
 
 # name -> (restype, argtypes); every symbol include/bmtk_amd.h declares
 SIGNATURES = {
@@ -101,6 +105,7 @@ SIGNATURES = {
     "bmtk_poisson_fill": (c_int32, [c_int64, c_int32, c_void_p, c_double, c_double, c_double, c_int64, C.c_uint64,
                                     c_void_p, c_void_p, c_void_p, c_void_p]),
     "bmtk_glif3_simulate_fwd": (c_int32, [C.POINTER(Glif3Sim), c_int64, c_int64, c_void_p]),
+    "bmtk_events_by_trial": (c_int32, [c_int32, c_int64, c_int64, c_int32] + [c_void_p] * 6),
     "bmtk_glif3_simulate_bwd": (c_int32, [C.POINTER(Glif3Bwd), c_int64, c_int64, c_void_p]),
     "bmtk_glif3_step_bwd": (c_int32, [C.POINTER(Glif3Bwd), c_int64, c_int64, c_int32, c_void_p]),
     "bmtk_csr_weight_grad": (c_int32, [C.POINTER(Glif3Bwd), c_int64, c_int64, c_void_p]),

@@ -20,6 +20,9 @@ int simulate_resident(const bmtk_glif3_sim &s, int64_t step0, int64_t n_steps, h
 // whole synapse rows walked by a wavefront (resident_solo.hip).
 int simulate_resident_solo(const bmtk_glif3_sim &s, int64_t step0, int64_t n_steps, hipStream_t stream);
 
+// The trials of a batch, several side by side, each with its state in registers and its ring in LDS (resident_batch.hip).
+int simulate_resident_batch(const bmtk_glif3_sim &s, int64_t step0, int64_t n_steps, hipStream_t stream);
+
 // Batched runs, one launch per step with the pull of a step's arrivals and the update fused (simulate_fused.hip).
 int simulate_fused(const bmtk_glif3_sim &s, int64_t step0, int64_t n_steps, hipStream_t stream);
 

@@ -323,6 +323,7 @@ extern "C" int bmtk_glif3_simulate_fwd(const bmtk_glif3_sim *sim, int64_t step0,
     BMTK_REQUIRE((s.save_v == nullptr) == (s.save_flags == nullptr),
                  "glif3_simulate_fwd: save_v and save_flags go together");
     BMTK_REQUIRE(!(s.save_v && s.res_span > 0), "glif3_simulate_fwd: the per-step record needs launch-per-step mode");
+    if (s.rb_groups > 0) return simulate_resident_batch(s, step0, n_steps, (hipStream_t)stream);
     if (s.res_span > 0) {
         BMTK_REQUIRE(s.batch == 1, "glif3_simulate_fwd: resident mode runs batch 1 only");
         BMTK_REQUIRE(s.res_span % 64 == 0 && s.res_span <= 1024, "glif3_simulate_fwd: res_span must be a multiple of 64, at most 1024");

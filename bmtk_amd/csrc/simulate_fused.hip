@@ -72,6 +72,7 @@ struct FusedLaunch {
     int n_w32;           // words per row of the activity map of bits; words of one map of bytes
     int shift;           // sources per bit of the activity map: 2^shift
     int team;            // wavefronts that share a group (1: every wavefront takes groups of its own from the workgroup's counter)
+    int pending;         // bit 0 / 1: the resident form left arrivals of step t0-1 / t0 in rb_ring
     int map_read, map_write;  // which of the two maps of bytes the launch reads and leaves behind (-1: none)
 };
 
@@ -612,6 +613,21 @@ __global__ __launch_bounds__(kFuseBlock) void sim_fused_kernel(bmtk_glif3_sim s,
             }
         }
         float a0[GLIF3_NREC], a1[GLIF3_NREC];
+        const FuseLaunchArgs qp = fresh_launch();
+        if (qp->pending) {
+            // the first steps after a call in the resident form: what that call's spikes still send joins the sums
+            const FuseArgs sp = fresh_args();
+            const int row = fin_grp * kRows + (int)sub_lane, slots = L - 1;
+            if (in_group && row < n) {
+                const unsigned long long *left = reinterpret_cast<const unsigned long long *>(in_memory(sp->rb_ring)) +
+                                                 (int64_t)(lane - sub_bit) * slots * GLIF3_NREC * n + row;
+#pragma unroll
+                for (int r = 0; r < GLIF3_NREC; ++r) {
+                    if (qp->pending & 1) acc[r * kWave + lane] += left[((int64_t)((qp->t0 - 1) % slots) * GLIF3_NREC + r) * n];
+                    if (qp->pending & 2) acc[(GLIF3_NREC + r) * kWave + lane] += left[((int64_t)(qp->t0 % slots) * GLIF3_NREC + r) * n];
+                }
+            }
+        }
 #pragma unroll
         for (int r = 0; r < GLIF3_NREC; ++r) {
             a0[r] = from_fixed(acc[r * kWave + lane]);
@@ -784,6 +800,7 @@ int simulate_fused(const bmtk_glif3_sim &s, int64_t step0, int64_t n_steps, hipS
     const int n_w32 = bytes ? (int)byte_words : (int)((groups + 31) / 32);
     const size_t lds = kFuseLdsFixed + (size_t)n_w32 * 4u * (bytes ? 1u : (unsigned)L);
     BMTK_REQUIRE(lds <= kFuseLdsMax, "glif3_simulate_fwd: the activity map does not fit in LDS; use a larger fuse_shift");
+    BMTK_REQUIRE(s.rb_pend_until == 0 || s.rb_ring, "glif3_simulate_fwd: rb_pend_until needs rb_ring");
     BMTK_REQUIRE(!s.in_repeat_ptr || (s.in_repeat_events && s.inp_indptr && s.inp_packed),
                  "glif3_simulate_fwd: repeat lists need in_repeat_events and the source-major input table");
     BMTK_REQUIRE(!s.probe_col || (s.probe_v && s.probe_every >= 1 && s.probe_stride >= 1),
@@ -856,6 +873,7 @@ int simulate_fused(const bmtk_glif3_sim &s, int64_t step0, int64_t n_steps, hipS
         q.fold0 = k > 0 ? 1 : 0;
         q.in_bits = (has_inp && !closing && n_in_words > 0) ? 1 : 0;
         q.repeats = (s.in_repeat_ptr && !closing) ? 1 : 0;
+        q.pending = (q.fold0 && q.t0 - 1 < s.rb_pend_until ? 1 : 0) | (q.n_sub == 2 && q.t0 < s.rb_pend_until ? 2 : 0);
         q.map_read = map;
         q.map_write = bytes && (!closing || map == 1) ? 1 - map : -1;
         if (q.map_write >= 0) map = q.map_write;

@@ -32,6 +32,14 @@ FUSE_PS_PER_EVENT = 6.0
 PUSH_PS_PER_ELEMENT = 55.0
 PUSH_PS_PER_ELEMENT_CLASS_TABLE = 27.0
 PUSH_PS_PER_EVENT = 48.0
+# The form with resident trials pays a chain of dependent loads and a barrier per launch and step, a visit per row that fired,
+# little per event.  Measured, us per step trials / fused / pushed (neurons x trials, in-degree): 51,978 x 32, 1154: 38 / 95 / - ;
+# 20,011 x 20, 820: 8.3 / 31 / - ; 230,924 x 8, 335: 59 / 134 / 164; 5,000 x 16, 400: 2.8 / 9.8 / - ; 31,000 x 64, 160: 36 / 38 / 87;
+# 120,000 x 16, 150: 41 / 52 / 82; 100,000 x 4, 260: 10 / - / 28; 2,000 x 40, 200: 3.3 / 6.3 / 11.5; 3,000 x 4, 200: 2.7 / - / 11.5.
+TRIALS_PS_PER_PASS = 3.0e6
+TRIALS_PS_PER_ROW = 6.5e3       # per neuron of ONE trial that fires in a step (and the input events that come with it)
+TRIALS_PS_PER_EVENT = 0.8
+FUSE_PS_PER_ELEMENT = 10.0
 FUSE_LDS_BYTES = 160 * 1024 - 512   # LDS of one workgroup of the fused batched driver (kFuseLdsMax of csrc/simulate_fused.hip)
 FUSE_LDS_FIXED = 16 * (2 * NREC * 64 * 8 + 128 * 12)   # ... of it sums and stages (kFuseLdsFixed)
 FUSE_BATCHES = range(8, 65)         # lane = trial, at most eight neurons to a wavefront
@@ -43,6 +51,8 @@ RES_LDS_EXTRA = RES_ACT_ENTRIES * 4 + 256   # the list plus the kernel's static 
 # the items (rows to walk) of two steps and its static LDS (SOLO_LDS_EXTRA)
 SOLO_LDS_PER_ELEMENT = 4 * 4
 SOLO_LDS_EXTRA = 10240 + 2048
+RB_LIST_MIN, RB_LDS_STATIC = 2000, 256   # the form with resident trials: least room for its list of rows, static LDS
+TRIALS_MIN_STEPS = 32           # shorter calls are left to the launch-per-step drivers
 RECORD_WAYS = 64                # lists a large spike record is split into (bmtk_glif3_sim.spike_ways)
 
 
@@ -66,6 +76,25 @@ def resident_span(ne, batch, ring_slots, n_cu, single=True):
     return span
 
 
+def resident_trials_plan(n_neurons, batch, ring_slots, n_cu):
+    """How the trials of a batch share ``n_cu`` compute units when each keeps its state in registers and its arrivals of
+    the next ring_slots - 1 steps in LDS: dict(span, groups, ways, passes, list) -- ``ways`` trials side by side on
+    ``groups`` workgroups of ``span`` neurons each, ``passes`` launches, ``list`` places in the list of rows -- or None
+    where a single trial does not fit.  As few launches as possible: a step costs much the same whatever runs beside it."""
+    cus, slots = n_cu - n_cu % 8, ring_slots - 1
+    if not 2 <= batch <= 64 or cus <= 0 or n_neurons <= 0 or slots < 1:
+        return None
+    per_neuron = slots * NREC * 8
+    span_max = min(1024, (RES_LDS_BYTES - RB_LDS_STATIC - 4 * RB_LIST_MIN) // per_neuron // 64 * 64)
+    if span_max < 64 or -(-n_neurons // span_max) > cus:
+        return None
+    passes = -(-batch // min(batch, cus // -(-n_neurons // span_max)))
+    ways = -(-batch // passes)
+    span = -(-(-(-n_neurons // (cus // ways))) // 64) * 64
+    rows = min(RES_ACT_ENTRIES, (RES_LDS_BYTES - RB_LDS_STATIC - span * per_neuron) // 4)
+    return dict(span=span, groups=-(-n_neurons // span), ways=ways, passes=passes, list=rows)
+
+
 def fused_pays(n_neurons, batch, n_synapses, class_table, rate_hz, h_ms=1.0):
     """Whether the fused pull form of the batched driver is expected to take less time per step than pushing the
     spikes as events, for a network of ``n_neurons`` with ``n_synapses`` recurrent and input synapses at ``batch``
@@ -79,6 +108,21 @@ def fused_pays(n_neurons, batch, n_synapses, class_table, rate_hz, h_ms=1.0):
     push = ((PUSH_PS_PER_ELEMENT_CLASS_TABLE if class_table else PUSH_PS_PER_ELEMENT) * n_neurons * batch
             + PUSH_PS_PER_EVENT * events + PUSH_PS_PER_STEP)
     return fused < push
+
+
+def trials_pay(plan, n_neurons, batch, n_synapses, class_table, rate_hz, h_ms, fused):
+    """Whether the form with resident trials (``plan``: resident_trials_plan) is expected to take less time per step than
+    the driver that would run otherwise, the fused pull form (``fused``) or pushed events."""
+    per_trial = n_neurons * float(rate_hz) * 1e-3 * h_ms
+    events = n_synapses * batch * float(rate_hz) * 1e-3 * h_ms
+    trials = plan["passes"] * (TRIALS_PS_PER_PASS + TRIALS_PS_PER_ROW * per_trial) + TRIALS_PS_PER_EVENT * events
+    if fused:
+        other = (FUSE_PS_PER_STEP + FUSE_PS_PER_SYNAPSE * n_synapses + FUSE_PS_PER_EVENT * events
+                 + FUSE_PS_PER_ELEMENT * n_neurons * batch)
+    else:
+        other = ((PUSH_PS_PER_ELEMENT_CLASS_TABLE if class_table else PUSH_PS_PER_ELEMENT) * n_neurons * batch
+                 + PUSH_PS_PER_EVENT * events + PUSH_PS_PER_STEP)
+    return trials < other
 
 
 class Glif3Simulator:
@@ -121,6 +165,13 @@ class Glif3Simulator:
                 atomics as spikes occur -- the faster form for batched runs.  "auto": by ``expected_rate_hz``
                 (and delay_offset 0, network small enough for the activity map in LDS).  Recurrent arrivals still ahead at the end
                 of a run then live in the history, and ``ring`` holds the input arrivals only.
+    resident_trials  batches of 2 to 64 with a recurrent table and delay_offset 0: trials side by side, each with its state
+                in registers and its ring in LDS for the length of a call, as many at a time as the compute units hold
+                (``resident_trials_plan``).  "auto": where resident, fused and pull are "auto" too, the network fits and
+                ``trials_pay`` says so.  Such a simulator also holds the driver it would have without; a call that asks
+                for more than spike bits (``save_state``, ``record_cap``, probes), covers fewer than TRIALS_MIN_STEPS
+                steps or is captured into a graph, and a look at ``ring``, ``work_bits`` or ``fuse_any``, make it go on with that
+                driver for good.  True: insist (ValueError otherwise); False: off.
     delay_offset  B steps taken off every delay before the tables are built; spikes and input events are
                 then handed to the tables B steps late from a history of spike bits, which gives the same
                 arrivals with a ring B slots shorter.  "auto": 0 while the largest delay is at most 63
@@ -134,7 +185,7 @@ class Glif3Simulator:
     def __init__(self, n_neurons, par, h, batch=1, class_id=None, rec=None, inp=None, ring_slots=None,
                  asc_init=None, u_init=None, i_ext=None, device=None, resident="auto", delay_offset="auto",
                  pull="auto", single_workgroup=True, fired_lists=True, fused="auto", fuse_wg_per_cu=0,
-                 expected_rate_hz=3.0):
+                 expected_rate_hz=3.0, resident_trials="auto"):
         self.lib = _lib.load()
         self.dev = device or _dev()
         self.n, self.batch, self.h = int(n_neurons), int(batch), float(h)
@@ -220,7 +271,8 @@ class Glif3Simulator:
         if self.inp_without_synapses:
             self.inp = None
         self.state = Glif3State.zeros(self.n, self.batch, asc_init=asc_init, u_init=u_init, device=self.dev)
-        self.ring = torch.zeros(self.L, NREC, self.ne, device=self.dev)
+        self._trials = None     # the form with resident trials (_setup_trials), while it is in use
+        self._ring = torch.zeros(self.L, NREC, self.ne, device=self.dev)
         self.i_ext = None if i_ext is None else torch.as_tensor(np.asarray(i_ext, np.float32), device=self.dev)
         if self.i_ext is not None and self.i_ext.numel() != self.ne:
             raise ValueError("i_ext needs one entry per element")
@@ -236,7 +288,7 @@ class Glif3Simulator:
         self.hist_slots = 2 * self.delay_offset + 4
         if self.hist_slots * (self.words + 1) * 8 > 2 ** 30:
             self.hist_slots = self.delay_offset + 3
-        self.work_bits = torch.zeros(self.hist_slots * (self.words + 1), dtype=torch.int64, device=self.dev)
+        self._work_bits = torch.zeros(self.hist_slots * (self.words + 1), dtype=torch.int64, device=self.dev)
         if self.n >= 2 ** 24:
             raise ValueError("the packed synapse tables index at most 2^24 neurons")
         self.res_sync = torch.zeros(_lib.RES_SYNC_WORDS, dtype=torch.int32, device=self.dev)
@@ -252,7 +304,7 @@ class Glif3Simulator:
             self._setup_resident(required=(resident is True))
         self.pull_table = self.pull_syn = self.pull_work = None
         self.pull_inp_table = self.pull_inp_syn = self.pull_inp_work = self.in_hist = None
-        self.fuse_table = self.fuse_any = None
+        self.fuse_table = self._fuse_any = None
         self.fuse_wg_per_cu = int(fuse_wg_per_cu)
         can_fuse = ((self.rec is not None or self.inp is not None) and not self.res_span and self.delay_offset == 0
                     and self.delay_bits == 6 and self.batch in FUSE_BATCHES and pull is not False)
@@ -298,7 +350,7 @@ class Glif3Simulator:
             self.pull_work = torch.zeros(need // 4 + 1, dtype=torch.int32, device=self.dev)
             # the history must hold one row per ring slot, row t % L = spikes of step t
             self.hist_slots = self.L
-            self.work_bits = torch.zeros(self.hist_slots * (self.words + 1), dtype=torch.int64, device=self.dev)
+            self._work_bits = torch.zeros(self.hist_slots * (self.words + 1), dtype=torch.int64, device=self.dev)
             if self.inp is not None and self.L * ((self.n_inputs + 31) // 32) * 4 <= PULL_MAP_BYTES:
                 self.pull_inp_table = self.inp.transposed(self.n)
                 self.pull_inp_syn = torch.zeros(NREC, self.ne, device=self.dev)
@@ -306,6 +358,142 @@ class Glif3Simulator:
                 self.pull_inp_work = torch.zeros(need // 4 + 1, dtype=torch.int32, device=self.dev)
                 self.in_hist_stride = n_words(self.n_inputs * self.batch) + 1
                 self.in_hist = torch.zeros(self.L * self.in_hist_stride, dtype=torch.int64, device=self.dev)
+        self.expected_rate_hz = float(expected_rate_hz)
+        self._trials_left, self._pend_until, self._left_ring = False, 0, None
+        if resident_trials == "auto":
+            wanted = resident == "auto" and fused == "auto" and pull == "auto" and self.pull_table is None
+        else:
+            wanted = bool(resident_trials)
+        plan = None
+        if wanted and self.rec is not None and not self.res_span and self.delay_offset == 0 and self.delay_bits == 6:
+            n_cu = torch.cuda.get_device_properties(self.dev).multi_processor_count
+            plan = resident_trials_plan(self.n, self.batch, self.L, n_cu)
+        if plan and ((self.n + self.n_inputs) * (plan["groups"] + 1) >= 2 ** 32 or self.n + self.n_inputs >= 2 ** 24
+                     or n_syn >= 2 ** 31 or self.pull_table is not None):
+            plan = None
+        if plan and resident_trials == "auto":
+            if not trials_pay(plan, self.n, self.batch, n_syn, self.class_id is not None, expected_rate_hz, self.h,
+                              self.fuse_table is not None):
+                plan = None
+        if plan and not self._trials_weights_ok(fixed_point_ok):
+            plan = None
+        if resident_trials is True and plan is None:
+            raise ValueError("resident trials need a recurrent table, a batch of 2 to 64, delay_offset 0, no pull table, weights "
+                             "that 64-bit fixed point holds and a network whose trial fits the compute units")
+        if plan:
+            self._trials = dict(plan, seg=None)
+
+    def _trials_weights_ok(self, fixed_point_ok):
+        """Whether the 64-bit fixed-point sums of the form with resident trials are at least as good as those of the form
+        it takes the place of: always those of the fused form; the fp32 sums of pushed events where the weights are
+        large against 2^-32 and a neuron's all together small against 2^31."""
+        tables = [t for t in (self.rec, self.inp) if t is not None]
+        if not all(fixed_point_ok(t) for t in tables):
+            return False
+        if self.fuse_table is not None:
+            return True
+        size = sum(t.weights.abs().sum(dtype=torch.float64) for t in tables) / max(1, sum(t.nnz for t in tables))
+        most = sum(t.weights.abs().max().double() * torch.bincount(t.indices, minlength=self.n).max() for t in tables if t.nnz)
+        return bool((size >= 2.0 ** -8) & (most < 2.0 ** 30))
+
+    def _setup_trials(self):
+        """Tables and buffers of the form with resident trials: recurrent and input rows as one table sorted by target,
+        the bounds of every workgroup's segment of every row, the ring behind a call and the ballot history."""
+        tr, n = self._trials, self.n
+        groups = tr["groups"]
+        seg = torch.empty(n + self.n_inputs, groups + 1, dtype=torch.int32, device=self.dev)
+        packed = torch.empty(self.rec.nnz + (self.inp.nnz if self.inp is not None else 0), 2, dtype=torch.int32, device=self.dev)
+        row = at = 0
+        for t in (self.rec, self.inp):
+            if t is None:
+                continue
+            try:
+                own = t.segment_offsets(tr["span"], groups)
+            except ValueError:
+                t = t.sorted_by_index()
+                own = t.segment_offsets(tr["span"], groups)
+            seg[row:row + t.n_rows] = own + at          # (fewer than 2^31 synapses)
+            packed[at:at + t.nnz] = t.packed()[:t.nnz]
+            row, at = row + t.n_rows, at + t.nnz
+        # lanes to a segment at most: about as many as it holds synapses on average
+        segment = int(math.ceil(math.log2(max(1.0, at / float(max(1, row)) / groups))))
+        tr.update(seg=seg, packed=packed, max_team_shift=min(6, segment),
+                  ring=torch.zeros(self.batch, self.L - 1, NREC, n, dtype=torch.int64, device=self.dev),
+                  hist=torch.zeros(tr["ways"], 4, n_words(n) + 1, dtype=torch.int64, device=self.dev))
+
+    def _trials_run(self, s, n_steps):
+        """Fill ``s`` for a call in the form with resident trials.  Returns what has to live until it is launched."""
+        tr = self._trials
+        if tr["seg"] is None:
+            self._setup_trials()
+        s.rb_span, s.rb_groups, s.rb_ways, s.rb_list = tr["span"], tr["groups"], tr["ways"], tr["list"]
+        # as many lanes to a segment as let the workgroup's 1024 take the rows of a step in one go, or in little more
+        # (5,000 neurons x 16 trials, some 20 rows of 21 synapses: 6.5 / 3.5 / 2.8 us per step with 1 / 4 / 32 lanes; 51,978 x 32, 220
+        # of 14: 60 / 38 / 50 / 69 with 1 / 4 / 16 / 32; 230,924 x 8, 1,000 rows of 1.4: one)
+        events = self.in_events.numel() / float(max(1, self.in_steps) * self.batch) if self.in_ptr is not None else 0.0
+        rows = max(1.0, self.n * self.expected_rate_hz * 1e-3 * self.h + events)
+        s.rb_team_shift = max(0, min(tr["max_team_shift"], int(math.log2(max(1.0, 1500.0 / rows)))))
+        s.rb_late_events = 1 if self.fuse_rereads else 0
+        s.rb_seg, s.rb_packed, s.rb_ring, s.rb_hist = _p(tr["seg"]), _p(tr["packed"]), _p(tr["ring"]), _p(tr["hist"])
+        s.res_sync, s.res_spin_limit = _p(self.res_sync), int(self.spin_limit)
+        if self.inp is None or self.in_ptr is None:
+            return None
+        # the events of the steps step - 1 .. step + n_steps - 1, apart by trial
+        args = (self.batch, self.step - 1, n_steps + 1, s.rb_late_events, _p(self.in_ptr), _p(self.in_events))
+        counts = torch.empty(self.batch * (n_steps + 1), dtype=torch.int32, device=self.dev)
+        _lib.check(self.lib.bmtk_events_by_trial(*args, _p(counts), None, None, _stream()))
+        first = torch.zeros(counts.numel() + 1, dtype=torch.int64, device=self.dev)
+        torch.cumsum(counts, 0, out=first[1:])
+        sources = torch.empty_like(self.in_events)
+        _lib.check(self.lib.bmtk_events_by_trial(*args, None, _p(first), _p(sources), _stream()))
+        s.rb_in_ptr, s.rb_in_events = _p(first), _p(sources)
+        return first, sources
+
+    def _leave_trials(self):
+        """From the form with resident trials to the driver that takes its place, for good: what is still under way is
+        handed over."""
+        tr, self._trials = self._trials, None
+        if tr is None or tr["seg"] is None:
+            return
+        left, slots = tr["ring"], self.L - 1
+        if self.fuse_table is not None:
+            self._left_ring, self._pend_until, self._trials_left = left, self.step + slots, True
+            return
+        for t in range(self.step, self.step + slots):
+            cells = (left[:, t % slots].double() * 2.0 ** -32).float()            # [batch][4][n]
+            self._ring[t % self.L] += cells.permute(1, 2, 0).reshape(NREC, self.ne)
+
+    # What the launch-per-step drivers keep between calls.  A caller that looks at it finds it as they would have left it: the
+    # form with resident trials gives way to them first.
+    @property
+    def ring(self):
+        self._leave_trials()
+        return self._ring
+
+    @ring.setter
+    def ring(self, value):
+        self._leave_trials()
+        self._ring = value
+
+    @property
+    def work_bits(self):
+        self._leave_trials()
+        return self._work_bits
+
+    @work_bits.setter
+    def work_bits(self, value):
+        self._leave_trials()
+        self._work_bits = value
+
+    @property
+    def fuse_any(self):
+        self._leave_trials()
+        return self._fuse_any
+
+    @fuse_any.setter
+    def fuse_any(self, value):
+        self._leave_trials()
+        self._fuse_any = value
 
     def _setup_fused(self):
         """Joint target-major table, joint history and activity map of the fused batched driver."""
@@ -318,14 +506,14 @@ class Glif3Simulator:
         self.fuse_table.pad_packed(FUSE_PAD)
         self.fuse_hist_stride = self.fuse_in_base // rows + -(-n_in // rows) + 1
         self.hist_slots = self.L + 4         # two steps per launch: rows read, written and cleared ahead
-        self.ring = torch.zeros(self.L + 2, NREC, self.ne, device=self.dev)   # (its ring: two slots more)
-        self.work_bits = torch.zeros(self.hist_slots * self.fuse_hist_stride, dtype=torch.int64, device=self.dev)
+        self._ring = torch.zeros(self.L + 2, NREC, self.ne, device=self.dev)   # (its ring: two slots more)
+        self._work_bits = torch.zeros(self.hist_slots * self.fuse_hist_stride, dtype=torch.int64, device=self.dev)
         # one bit of the activity map per 2^shift sources: the smallest shift whose map fits the LDS beside the
         # accumulators (where it also fits with a byte per source, the library takes that)
         self.fuse_shift = 0
         while FUSE_LDS_FIXED + self.L * self._fuse_any_words() * 4 > FUSE_LDS_BYTES:
             self.fuse_shift += 1
-        self.fuse_any = self._new_fuse_any()
+        self._fuse_any = self._new_fuse_any()
 
     def set_fuse_shift(self, shift):
         """Fused form: one bit of the activity map per 2^shift sources (the constructor picks the smallest shift
@@ -336,7 +524,7 @@ class Glif3Simulator:
         if not 0 <= self.fuse_shift <= 16 or FUSE_LDS_FIXED + self.L * self._fuse_any_words() * 4 > FUSE_LDS_BYTES:
             self.fuse_shift = old
             raise ValueError("shift must lie in 0..16 and leave the activity map within the LDS")
-        self.fuse_any = self._new_fuse_any()
+        self._fuse_any = self._new_fuse_any()
 
     def _new_fuse_any(self):
         # the activity map (one row per history row) and, behind it, the map of ring cells that hold something
@@ -461,7 +649,7 @@ class Glif3Simulator:
         s.n_neurons, s.batch, s.ring_slots, s.h = self.n, self.batch, self.L, self.h
         s.V, s.asc, s.y1, s.y2, s.ref = (_p(x) for x in (st.V, st.asc, st.y1, st.y2, st.ref))
         s.prop, s.prop_stride, s.class_id = _p(self.prop), self.prop.shape[1], _p(self.class_id)
-        s.ring = _p(self.ring)
+        s.ring = _p(self._ring)
         if self.rec is not None:
             s.rec_indptr, s.rec_indices, s.rec_weights, s.rec_delays, s.rec_receptors = self.rec.pointers()
             s.rec_packed = _p(self.rec.packed())
@@ -471,7 +659,7 @@ class Glif3Simulator:
             s.inp_indptr, s.inp_indices, s.inp_weights, s.inp_delays, s.inp_receptors = self.inp.pointers()
             s.inp_packed = _p(self.inp.packed())
         s.i_ext = _p(self.i_ext)
-        s.work_bits = _p(self.work_bits)
+        s.work_bits = _p(self._work_bits)
         s.delay_offset, s.hist_slots, s.delay_bits = self.delay_offset, self.hist_slots, self.delay_bits
         if self.pull_table is not None:
             s.pull_indptr, s.pull_packed = _p(self.pull_table.indptr), _p(self.pull_table.packed())
@@ -482,13 +670,17 @@ class Glif3Simulator:
                 s.in_hist, s.in_hist_stride = _p(self.in_hist), self.in_hist_stride
                 if self.in_repeat_ptr is not None:
                     s.in_repeat_ptr, s.in_repeat_events = _p(self.in_repeat_ptr), _p(self.in_repeat_events)
+        if self._pend_until <= self.step:
+            self._left_ring = None
         if self.fuse_table is not None:
             s.n_inputs = self.n_inputs if self.inp is not None else 0   # the history's layout, events or not
             s.fuse_indptr, s.fuse_packed = _p(self.fuse_table.indptr), _p(self.fuse_table.packed())
-            s.fuse_any, s.fuse_hist_stride, s.fuse_in_base = _p(self.fuse_any), self.fuse_hist_stride, self.fuse_in_base
+            s.fuse_any, s.fuse_hist_stride, s.fuse_in_base = _p(self._fuse_any), self.fuse_hist_stride, self.fuse_in_base
             s.fuse_shift, s.fuse_wg_per_cu = self.fuse_shift, self.fuse_wg_per_cu
             s.fuse_max_team = max(1, -(-self.fuse_table.nnz // (256 * -(-self.n // (64 // self.batch)))))
-            s.in_again = 1 if self.fuse_rereads and self._lists_replaced else 0
+            s.in_again = 1 if self.fuse_rereads and (self._lists_replaced or self._trials_left) else 0
+            if self._pend_until > self.step:
+                s.rb_ring, s.rb_pend_until = _p(self._left_ring), self._pend_until
             if self.in_repeat_ptr is not None:
                 s.in_repeat_ptr, s.in_repeat_events = _p(self.in_repeat_ptr), _p(self.in_repeat_events)
         if self.res_span:
@@ -561,7 +753,14 @@ class Glif3Simulator:
                           frac=torch.empty(record_cap, dtype=torch.float32, device=self.dev),
                           count=torch.zeros(1 if ways == 1 else ways * _lib.RECORD_COUNT_STRIDE, dtype=torch.int64,
                                             device=self.dev), ways=ways)
+        by_trials = None
+        use_trials = (self._trials is not None and n_steps >= TRIALS_MIN_STEPS and not save_state and record is None
+                      and self.probe_col is None and not torch.cuda.is_current_stream_capturing())
+        if self._trials is not None and n_steps > 0 and not use_trials:
+            self._leave_trials()
         s = self._struct(bits, record)
+        if use_trials:
+            by_trials = self._trials_run(s, n_steps)
         saved = None
         if save_state:
             if self.res_span:
@@ -581,7 +780,9 @@ class Glif3Simulator:
         _lib.check(self.lib.bmtk_glif3_simulate_fwd(C.byref(s), self.step, n_steps, _stream()))
         self.step += n_steps
         self._lists_replaced = self._lists_replaced and n_steps == 0
-        self._pending_check = bool(self.res_span)
+        self._trials_left = self._trials_left and n_steps == 0
+        self._pending_check = self._pending_check or use_trials or bool(self.res_span)
+        del by_trials
         return dict(bits=bits, record=record, saved=saved, probe=probe)
 
     def collect_record(self, record, sort_scale=None):

@@ -49,7 +49,7 @@ extern "C" {
 
 /* Bumped whenever a struct layout or a signature below changes; bmtk_amd_abi_version() returns the value the
  * library was built with. */
-#define BMTK_AMD_ABI_VERSION 26
+#define BMTK_AMD_ABI_VERSION 27
 int bmtk_amd_abi_version(void);
 const char *bmtk_amd_last_error(void);
 /* sizeof(bmtk_glif3_sim) as the library was compiled, for bindings that mirror the struct */
@@ -384,6 +384,27 @@ typedef struct bmtk_glif3_sim {
                                         * emitted in the steps behind take what step0 - 1 still had under way along) */
     int32_t fuse_max_team;             /* fused form: most wavefronts that share a group of neurons in a network too small to
                                         * give every wavefront one (0: 16): about as many as the group's run has blocks of 256 */
+    /* Resident form of a batch's trials (optional, batches of 2 to 64, delay_offset 0; rb_groups == 0 disables it; takes
+     * precedence over everything above): cooperative launches in which rb_ways trials run side by side, each on
+     * rb_groups = ceil(n_neurons / rb_span) workgroups that keep its state in registers and its arrivals of the next
+     * ring_slots - 1 steps in LDS (64-bit fixed point, as the fused form's sums) for the whole call.  Spike bits are the only
+     * output it knows (no save_v, probes or spike record).  The arrivals still ahead at the end of a call are left in
+     * rb_ring, and a call begins with those: neither `ring` nor work_bits is used.  The fused form takes them over
+     * (rb_pend_until).  Uses res_sync and res_spin_limit as the resident mode does. */
+    int32_t rb_span;                   /* neurons of a workgroup: a multiple of 64 up to 1024 */
+    int32_t rb_groups;
+    int32_t rb_ways;                   /* trials of a launch: rb_ways * rb_groups workgroups must be resident at once */
+    int32_t rb_team_shift;             /* 2^rb_team_shift lanes read a row's segment */
+    int32_t rb_list;                   /* places of the list of rows in LDS; (ring_slots-1)*32*rb_span + 4*rb_list + 256 bytes of LDS */
+    int32_t rb_late_events;            /* the input events of a call's last step (each id once; repeats are delivered at once) are
+                                        * left to the next call and its lists, as with in_again */
+    const uint32_t *rb_seg;            /* [n_neurons + n_inputs][rb_groups + 1], bmtk_csr_segment_offsets with rb_span over rb_packed */
+    const bmtk_synapse *rb_packed;     /* recurrent rows followed by the input rows, sorted by target within a row */
+    uint64_t *rb_ring;                 /* [batch][ring_slots - 1][4][n_neurons], zeroed before the first run */
+    uint64_t *rb_hist;                 /* [rb_ways][4][ceil(n_neurons/64) + 1], zeroed once */
+    const int64_t *rb_in_ptr;          /* [batch * (n_steps + 1) + 1], or NULL: input events of trial b in step step0 - 1 + k are */
+    const int32_t *rb_in_events;       /* ... rb_in_events[p[b*(n_steps+1)+k] .. p[b*(n_steps+1)+k+1]) (bmtk_events_by_trial) */
+    int64_t rb_pend_until;             /* fused form: rb_ring holds arrivals of the steps before this one (0: none) */
     /* outputs */
     uint64_t *spike_bits;        /* [n_steps][words] spike bits per step, words = ceil(ne/64); or NULL.
                                   * Row k belongs to step step0+k of the call that wrote it. */
@@ -448,6 +469,15 @@ typedef struct bmtk_glif3_sim {
  * into its LDS ring slice with LDS atomics -- no global atomics and no state
  * traffic.  The barrier spins a bounded number of times; see res_sync. */
 int bmtk_glif3_simulate_fwd(const bmtk_glif3_sim *sim, int64_t step0, int64_t n_steps, void *stream);
+
+/* The input events of the steps step0 .. step0 + n_steps - 1 (step0 may be -1: a step without events) apart by trial.  With
+ * `counts` ([batch][n_steps]) the events of every trial and step are counted; with `first` ([batch][n_steps], the running
+ * sums of those counts, exclusive) and `sources` their sources are written, in no particular order within a trial and step.
+ * With `late` an id counts once in the first of the steps, and in the last one only its occurrences after the first do
+ * (bmtk_glif3_sim.rb_late_events). */
+int bmtk_events_by_trial(int32_t batch, int64_t step0, int64_t n_steps, int32_t late, const int64_t *in_ptr,
+                         const int32_t *in_events, int32_t *counts, const int64_t *first, int32_t *sources, void *stream);
+
 
 /* Poisson spike sources generated on the device: the homogeneous case of bmtk's
  * PoissonSpikeGenerator._build_fixed_fr (bmtk/utils/reports/spike_trains/spike_trains.py:166-206) without

@@ -1,0 +1,139 @@
+"""The form with resident trials (state in registers, ring in LDS, several trials side by side) against the fp32 oracle."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import glif3_oracle as orc
+from bmtk_amd import ops, synthetic
+from bmtk_amd.simulator import Glif3Simulator, resident_trials_plan
+
+pytestmark = pytest.mark.gpu
+STATE = ("V", "asc", "y1", "y2", "ref")
+
+
+def _quarter(table):
+    indptr, indices, w, d, r = table
+    return indptr, indices, (np.round(w * 4.0) / 4.0 + np.sign(w) * 0.25).astype(np.float32), d, r
+
+
+def _case(n, batch, max_delay, classes=None, n_in=120, steps=150, seed=3, in_rate=60.0):
+    cfg = synthetic.small_glif3_network(n=n, n_in=n_in, steps=steps, seed=seed, p_conn=min(0.3, 60.0 / n), in_rate=in_rate,
+                                        in_fanout=max(1, min(n, 30)), max_delay=max_delay, n_classes=classes, batch=batch,
+                                        w_scale=4.0, in_w_scale=20.0)
+    cfg["rec_src"], cfg["inp_src"] = _quarter(cfg["rec_src"]), _quarter(cfg["inp_src"])
+    cfg["i_ext"] = np.random.default_rng(seed).uniform(0.0, 500.0, n * batch).astype(np.float32)
+    # every seventh event twice
+    times = np.where(np.arange(cfg["in_events"].size) % 7 == 0, 2, 1)
+    cfg["in_ptr"] = np.concatenate([[0], np.cumsum(times)])[cfg["in_ptr"]].astype(np.int64)
+    cfg["in_events"] = np.repeat(cfg["in_events"], times)
+    st = orc.new_state(n, batch, np.float32)
+    orc.set_threads(orc.max_threads())
+    # weights in quarters of a pA: sums are exact in fp32 in any order
+    want = orc.simulate(st, orc.precompute(cfg["par"], 1.0), 1.0, steps, batch=batch, class_id=cfg["class_id"],
+                        ring=np.zeros((cfg["L"], 4, n * batch), np.float32), rec=cfg["rec_src"], inp=cfg["inp_src"],
+                        in_ptr=cfg["in_ptr"], in_events=cfg["in_events"], i_ext=cfg["i_ext"], raster=True)
+    assert want["count"] > 0
+    return cfg, want["raster"], st
+
+
+def _sim(cfg, batch, **kw):
+    sim = Glif3Simulator(cfg["n"], cfg["par"], 1.0, batch=batch, class_id=cfg["class_id"], rec=cfg["rec_src"], inp=cfg["inp_src"],
+                         i_ext=cfg["i_ext"], ring_slots=cfg["L"], resident=False, **kw)
+    sim.set_input_events(cfg["in_ptr"], cfg["in_events"])
+    return sim
+
+
+def _same(sim, outs, raster, st):
+    sim.check()
+    np.testing.assert_array_equal(np.concatenate([sim.raster(o["bits"]).cpu().numpy() for o in outs]), raster)
+    got = sim.state.to_numpy()
+    for k in STATE:
+        np.testing.assert_array_equal(got[k], st[k], err_msg=k)
+
+
+@pytest.mark.parametrize("n,batch,max_delay,classes", [
+    (20, 2, 1, None), (63, 5, 2, None), (64, 64, 4, 3), (65, 3, 6, None), (700, 20, 5, 7), (1025, 33, 4, None), (2100, 8, 12, None),
+    (1500, 64, 5, 11)])
+def test_equals_the_oracle_over_two_calls(n, batch, max_delay, classes):
+    """One neuron to a wavefront's worth and one more, one to several workgroups a trial, a ring of one slot, last launches
+    with fewer trials than the others: raster and state bit for bit, arrivals under way between the calls."""
+    cfg, raster, st = _case(n, batch, max_delay, classes)
+    sim = _sim(cfg, batch, resident_trials=True, fused=batch >= 8)
+    outs = [sim.run(50), sim.run(100)]
+    assert sim._trials is not None
+    _same(sim, outs, raster, st)
+
+
+@pytest.mark.parametrize("how", ["short", "record", "ring"])
+@pytest.mark.parametrize("batch,fused", [(6, False), (16, True), (20, True)])
+def test_gives_way_to_the_other_drivers_with_arrivals_under_way(batch, fused, how):
+    """A short call, one that asks for more than spike bits, a look at the ring: the launch-per-step driver goes on with
+    what the calls before left under way, repeated input events included."""
+    cfg, raster, st = _case(900, batch, 5, in_rate=150.0)
+    sim = _sim(cfg, batch, resident_trials=True, fused=fused, **(dict(expected_rate_hz=40.0) if batch == 20 else {}))
+    assert (sim.fuse_table is not None) == fused and sim.in_duplicates and sim.fuse_rereads == (batch == 20)
+    outs = [sim.run(70)]
+    if how == "ring":
+        assert float(sim.ring.abs().sum()) > 0 or fused
+        outs += [sim.run(80)]
+    elif how == "short":
+        outs += [sim.run(1), sim.run(2), sim.run(77)]
+    else:
+        outs += [sim.run(40, save_state=True), sim.run(40, record_cap=100000)]
+    assert sim._trials is None
+    _same(sim, outs, raster, st)
+
+
+def test_input_lists_replaced_between_calls():
+    """Lists that say nothing was emitted in the steps behind take the last step's events back at the batches where the
+    separate pull launches read them again (20), and leave them alone elsewhere (16)."""
+    for batch in (16, 20):
+        cfg, _, _ = _case(900, batch, 5, in_rate=150.0)
+        results = []
+        for kw in (dict(resident_trials=False), dict(resident_trials=True)):
+            sim = _sim(cfg, batch, fused=True, expected_rate_hz=40.0, **kw)
+            a = sim.run(60)
+            ptr = torch.as_tensor(cfg["in_ptr"]).clone()
+            events = torch.as_tensor(cfg["in_events"])[int(ptr[60]):]
+            sim.set_input_events(np.concatenate([np.zeros(60, np.int64), (ptr[60:] - ptr[60]).numpy()]), events.numpy())
+            b = sim.run(90)
+            sim.check()
+            results.append((torch.cat([a["bits"], b["bits"]]).cpu().numpy(), sim.state.to_numpy()))
+        np.testing.assert_array_equal(results[0][0], results[1][0])
+        for k in STATE:
+            np.testing.assert_array_equal(results[0][1][k], results[1][1][k], err_msg=k)
+
+
+def test_more_rows_in_a_step_than_the_list_holds():
+    """Identical neurons driven alike fire together: 5,000 rows in one step against a list of 2,000 places."""
+    n, batch, steps = 5000, 4, 60
+    rng = np.random.default_rng(21)
+    par = synthetic.random_cells(rng, 1)
+    cls = np.zeros(n, np.int32)
+    src, tgt = rng.integers(0, n, 40000), rng.integers(0, n, 40000)
+    rec = _quarter(tuple(t.cpu().numpy() for t in (lambda s: (s.indptr, s.indices, s.weights, s.delays, s.receptors))(
+        ops.SynapseTable.from_edges(src, tgt, np.ones(40000, np.float32), rng.integers(1, 6, 40000), rng.integers(0, 4, 40000), n, n))))
+    i_ext = np.full(n * batch, 900.0, np.float32)
+    st = orc.new_state(n, batch, np.float32)
+    want = orc.simulate(st, orc.precompute(par, 1.0), 1.0, steps, batch=batch, class_id=cls, ring=np.zeros((6, 4, n * batch), np.float32),
+                        rec=rec, i_ext=i_ext, raster=True)
+    assert want["raster"].reshape(steps, n, batch)[:, :, 0].sum(1).max() > 4000
+    sim = Glif3Simulator(n, par, 1.0, batch=batch, class_id=cls, rec=rec, i_ext=i_ext, resident=False, resident_trials=True)
+    sim._trials["list"] = 2000
+    _same(sim, [sim.run(steps)], want["raster"], st)
+
+
+def test_a_barrier_that_gives_up_is_reported():
+    cfg, _, _ = _case(700, 4, 5)
+    sim = _sim(cfg, 4, resident_trials=True)
+    sim.res_sync[1] = 1            # as a workgroup whose wait ran out leaves it
+    sim.run(40)
+    with pytest.raises(RuntimeError):
+        sim.check()
+
+
+def test_what_does_not_fit_is_refused():
+    assert resident_trials_plan(300000, 8, 6, 256) is None and resident_trials_plan(1000, 65, 6, 256) is None
+    cfg, _, _ = _case(200, 2, 3)
+    with pytest.raises(ValueError):
+        Glif3Simulator(cfg["n"], cfg["par"], 1.0, batch=2, inp=cfg["inp_src"], resident=False, resident_trials=True)

@@ -1,0 +1,29 @@
+"""How the trials of a batch are laid out on the compute units, and when that is expected to pay."""
+import pytest
+
+from bmtk_amd.layout import NREC
+from bmtk_amd.simulator import RB_LDS_STATIC, RES_LDS_BYTES, resident_trials_plan, trials_pay
+
+
+@pytest.mark.parametrize("n,batch,slots", [(1, 2, 2), (64, 64, 6), (65, 3, 6), (5000, 16, 6), (20011, 20, 6), (51978, 32, 6), (230924, 8, 6),
+                                           (245000, 2, 6), (2000, 64, 60), (120000, 16, 3)])
+def test_plan_holds_every_neuron_and_trial(n, batch, slots):
+    p = resident_trials_plan(n, batch, slots, 256)
+    assert p["span"] % 64 == 0 and 64 <= p["span"] <= 1024 and p["groups"] == -(-n // p["span"])
+    assert 8 * -(-p["ways"] * p["groups"] // 8) <= 256 and p["ways"] <= batch <= p["ways"] * p["passes"]
+    assert (slots - 1) * NREC * 8 * p["span"] + 4 * p["list"] + RB_LDS_STATIC <= RES_LDS_BYTES and p["list"] >= 64
+
+
+def test_plan_of_what_does_not_fit():
+    for args in ((250000, 8, 6, 256), (1000, 1, 6, 256), (1000, 65, 6, 256), (10000, 8, 63, 64), (1000, 8, 6, 7)):
+        assert resident_trials_plan(*args) is None
+
+
+@pytest.mark.parametrize("n,batch,k,fused,pays", [(51978, 32, 1154, True, True), (230924, 8, 335, False, True), (20011, 20, 820, True, True),
+                                                  (31000, 64, 160, True, True), (3000, 4, 200, False, True), (1500, 8, 400, True, True)])
+def test_choice_agrees_with_measured_steps(n, batch, k, fused, pays):
+    assert trials_pay(resident_trials_plan(n, batch, 6, 256), n, batch, n * k, False, 3.0, 1.0, fused) == pays
+
+
+def test_many_launches_for_a_long_ring_do_not_pay():
+    assert not trials_pay(resident_trials_plan(8000, 64, 60, 256), 8000, 64, 8000 * 100, False, 3.0, 1.0, True)
