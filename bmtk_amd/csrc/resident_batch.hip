@@ -19,6 +19,12 @@
 //
 // What bounds it: a step is a chain of dependent loads (ballots, segment bounds, synapses) and the barrier, 3 us at the
 // smallest sizes, whatever the number of trials side by side; then the table's segments, which every trial reads for itself.
+//
+// One trial of more neurons than the compute units have threads (resident.hip ends at 1024 to a workgroup) runs here with two
+// neurons to a thread and its ring in floats, 80 bytes a neuron: 400,123 neurons, 72 M synapses, 23 -> 9 us per step against a
+// launch per step with an atomic per event (call and set-up included: 25.4 -> 9.8).  What it is short of are the 128 vector
+// registers a thread has: 84 hold two neurons.  Ballots kept over the prefix sum, addresses and products worked out once
+// for all steps spilled 81 of them to memory (13.3 us per step).
 #include <stdlib.h>
 
 #include "glif3_update.hpp"
@@ -32,6 +38,7 @@ constexpr int kRbWaves = kRbBlock / kWave;
 constexpr int kRbHist = 4;                // rows of the ballot history
 constexpr unsigned kRbMaxSpin = 4000000u; // polls of the barrier before giving up (seconds)
 constexpr int kRbCounters = 64;           // arrival counters per way of res_sync, dealt out to the trials of a launch
+constexpr int kRbWideWords = 8;           // ballot words per thread with two neurons to a thread
 constexpr int kRbTogether = 4;            // synapses a lane has in flight
 
 struct RbLaunch {
@@ -59,13 +66,18 @@ struct __attribute__((packed, aligned(4))) RbBounds {
 // arrives for step t after it has seen everybody arrive for step t-1, so that the arrivals of two steps never mix and one
 // counter per trial would do; several used in turn keep a look at step t-1 apart from the arrivals of step t.  A workgroup
 // that writes ballot row t%4 is at most two steps ahead of one that still reads row (t-3)%4.
-// kWords: ballot words per thread.
-template <int kWords>
+// kWords: ballot words per thread.  kPer: neurons per thread; with two, the threads of the last wavefront (the looker) own
+// none.  Sum: what the ring holds, 64-bit fixed point (from_fixed), or floats where a workgroup's neurons are too many for
+// that (batch 1): fp32 atomics into device memory are what it then takes the place of.
+template <int kWords, int kPer, typename Sum>
 __global__ __launch_bounds__(kRbBlock) void sim_resident_batch_kernel(bmtk_glif3_sim s, RbLaunch q)
 {
+    constexpr bool kFixed = sizeof(Sum) == 8;
+    constexpr int kOwners = kPer == 1 ? kRbBlock : kRbBlock - kWave;  // threads that own neurons tid, tid + kOwners, ..
     extern __shared__ unsigned long long rb_lds[];  // ring slice [slots * 4][span], then the list of rows
     __shared__ int go_on;
     __shared__ unsigned scan_l[kRbWaves];
+    __shared__ unsigned listed[2];  // rows in the list of this step and the next (one wide trial)
     const int tid = threadIdx.x, lane = lane_id(), wave = tid / kWave;
     const int span = s.rb_span, G = s.rb_groups;
     // an XCD (block number mod 8) gets consecutive workgroups, hence a trial as few XCDs as hold it
@@ -77,34 +89,40 @@ __global__ __launch_bounds__(kRbBlock) void sim_resident_batch_kernel(bmtk_glif3
     const int n = (int)s.n_neurons, batch = s.batch, S = q.slots;
     const int e0 = g * span;
     const int mine = min(span, n - e0);
-    const bool own = tid < mine;
-    const int i = e0 + tid;
     const int64_t ne = (int64_t)n * batch;
-    const int64_t e = (int64_t)(own ? i : e0) * batch + trial;
-    unsigned long long *ring_l = rb_lds;
-    unsigned *act = reinterpret_cast<unsigned *>(rb_lds + (size_t)S * GLIF3_NREC * span);
+    auto place = [&](int u) { return kPer == 1 ? tid : (tid < kOwners ? u * kOwners + tid : span); };  // in the workgroup's span
+    auto owns = [&](int u) { return place(u) < mine; };
+    auto element = [&](int u) { return (int64_t)(e0 + (owns(u) ? place(u) : 0)) * batch + trial; };
+    Sum *ring_l = reinterpret_cast<Sum *>(rb_lds);
+    unsigned *act = reinterpret_cast<unsigned *>(ring_l + (size_t)S * GLIF3_NREC * span);
     unsigned *abort_word = s.res_sync + 1;
     unsigned *arrivals = s.res_sync + BMTK_RES_SYNC_STRIDE + way * q.sync_slots * BMTK_RES_SYNC_STRIDE;
     constexpr int kWayStride = kRbCounters * BMTK_RES_SYNC_STRIDE;
     unsigned long long *hist = reinterpret_cast<unsigned long long *>(s.rb_hist) + (int64_t)way * kRbHist * (q.words + 1);
-    if (tid == 0) go_on = rb_load(abort_word) == 0u;
+    if (tid == 0) {
+        go_on = rb_load(abort_word) == 0u;
+        listed[0] = listed[1] = 0u;
+    }
     __syncthreads();
     if (!go_on) return;
 
-    unsigned long long *ring_g = reinterpret_cast<unsigned long long *>(s.rb_ring) + (int64_t)trial * S * GLIF3_NREC * n + e0;
+    Sum *ring_g = reinterpret_cast<Sum *>(s.rb_ring) + (int64_t)trial * S * GLIF3_NREC * n + e0;
     for (int c = tid; c < S * GLIF3_NREC * span; c += kRbBlock) {
         const int plane = c / span, k = c - plane * span;
-        ring_l[c] = k < mine ? ring_g[(int64_t)plane * n + k] : 0ull;
+        ring_l[c] = k < mine ? ring_g[(int64_t)plane * n + k] : (Sum)0;
     }
-    Glif3Elem st{};
-    Glif3Prop p{};
-    float I = 0.0f;
-    if (own) {
-        const int64_t col = s.class_id ? (int64_t)s.class_id[i] : (int64_t)i;
-        p.load(s.prop, s.prop_stride, col);
-        glif3_load(st, s.V, s.asc, s.y1, s.y2, s.ref, ne, e);
-        I = s.i_ext ? s.i_ext[e] : 0.0f;
-    }
+    Glif3Elem st[kPer]{};
+    Glif3Prop p[kPer]{};
+    float I[kPer]{};
+#pragma unroll
+    for (int u = 0; u < kPer; ++u)
+        if (owns(u)) {
+            const int i = e0 + place(u);
+            const int64_t col = s.class_id ? (int64_t)s.class_id[i] : (int64_t)i;
+            p[u].load(s.prop, s.prop_stride, col);
+            glif3_load(st[u], s.V, s.asc, s.y1, s.y2, s.ref, ne, element(u));
+            I[u] = s.i_ext ? s.i_ext[element(u)] : 0.0f;
+        }
     __syncthreads();  // (the ring slice is there, and go_on is written again below)
 
     auto counter_of = [&](int j) { return arrivals + (j & (q.sync_slots - 1)) * BMTK_RES_SYNC_STRIDE; };
@@ -140,10 +158,24 @@ __global__ __launch_bounds__(kRbBlock) void sim_resident_batch_kernel(bmtk_glif3
     auto pull_row = [&](unsigned row, unsigned q_lo, unsigned q_wrap) {
         const RbBounds b = *reinterpret_cast<const RbBounds *>(seg + (size_t)row * seg_stride);
         // (slot0 + delay) % slots * 4 + receptor = min(u, u - 4 * slots), u = slot0 * 4 + the record's upper byte
-        auto add = [&](const uint2 sy) {
+        auto add = [&](const uint2 sy, bool crowded) {
             const unsigned dq = sy.x >> 24;
             const unsigned plane = min(dq + q_lo, dq + q_wrap);
-            atomicAdd(ring_l + (mad_u24(plane, (unsigned)span, sy.x & 0xFFFFFFu) - (unsigned)e0), to_fixed(__uint_as_float(sy.y)));
+            Sum *cell = ring_l + (mad_u24(plane, (unsigned)span, sy.x & 0xFFFFFFu) - (unsigned)e0);
+            if constexpr (kFixed)
+                atomicAdd(cell, to_fixed(__uint_as_float(sy.y)));
+            else if (!crowded)
+                atomicAdd(cell, __uint_as_float(sy.y));
+            else {
+                // (where most lanes take part: a float atomic is worked off lane by lane, see resident.hip)
+                unsigned *bits = reinterpret_cast<unsigned *>(cell);
+                unsigned old = *bits;
+                while (true) {
+                    const unsigned seen = atomicCAS(bits, old, __float_as_uint(__uint_as_float(old) + __uint_as_float(sy.y)));
+                    if (seen == old) break;
+                    old = seen;
+                }
+            }
         };
         for (uint32_t at_p = b.lo + part; at_p < b.hi; at_p += kRbTogether * step) {
             uint2 sy[kRbTogether];
@@ -152,13 +184,80 @@ __global__ __launch_bounds__(kRbBlock) void sim_resident_batch_kernel(bmtk_glif3
                 if (at_p + u * step < b.hi) sy[u] = table[at_p + u * step];
 #pragma unroll
             for (int u = 0; u < kRbTogether; ++u)
-                if (at_p + u * step < b.hi) add(sy[u]);
+                if (at_p + u * step < b.hi) add(sy[u], u == 0);
         }
     };
     // Spikes in row `hist_row` of the ballot history (-1: none) and the input events [ka, kb) of the same step, whose ring
     // slot is slot0, into the ring slice.  All threads of the workgroup call it.  `arrival`: the counter to signal once
     // every wavefront's ballot store has been acknowledged.
     const int cap = s.rb_list;
+    // The same for a single wide trial, whose many ballot words would not stay in registers beside two neurons' state: each
+    // wavefront reads them kWideScan per thread at a time and takes its places in the list from a counter in LDS (`turn` tells
+    // which of two: the other is cleared on the way), so that no word outlives its turn and the workgroup meets once less.
+    constexpr int kWideScan = 4, kWideTurns = (kWords + kWideScan - 1) / kWideScan;
+    auto pull_wide = [&](int hist_row, int slot0, unsigned ka, unsigned kb, unsigned *arrival, int turn) {
+        const unsigned q_lo = (unsigned)slot0 * 4u, q_wrap = q_lo - 4u * (unsigned)S;
+        const unsigned n_ev = kb - ka;
+        unsigned base[kWideTurns];
+        // the places from `base` on of the list's window [c0, c0 + cap); the first look takes the places
+        auto list_words = [&](bool first, unsigned c0) {
+            // (not to be worked out once for all steps: that many addresses would push the state out of the registers)
+            int me = tid;
+            asm volatile("" : "+v"(me));
+#pragma unroll
+            for (int b = 0; b < kWideTurns; ++b) {
+                unsigned long long v[kWideScan];
+                unsigned cnt = 0u;
+#pragma unroll
+                for (int u = 0; u < kWideScan; ++u) {
+                    const int w = min((b * kWideScan + u) * kRbBlock + me, q.words);  // (a row's last word stays zero)
+                    v[u] = hist_row >= 0 ? __hip_atomic_load(hist + (int64_t)hist_row * (q.words + 1) + w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0ull;
+                }
+#pragma unroll
+                for (int u = 0; u < kWideScan; ++u) cnt += (unsigned)__popcll(v[u]);
+                const unsigned inc = wave_inclusive_scan(cnt);
+                if (first) {
+                    unsigned to = 0u;
+                    if (lane == kWave - 1) to = inc ? atomicAdd(&listed[turn], inc) : 0u;
+                    base[b] = (unsigned)bcast_i((int)to, kWave - 1);
+                }
+                unsigned pos = base[b] + inc - cnt - c0;  // (wraps below zero for places of an earlier window)
+#pragma unroll
+                for (int u = 0; u < kWideScan; ++u) {
+                    unsigned long long x = v[u];
+                    const unsigned j0 = (unsigned)((b * kWideScan + u) * kRbBlock + me) << 6;
+                    while (x) {
+                        const unsigned bit = (unsigned)__ffsll((long long)x) - 1u;
+                        x &= x - 1ull;
+                        if (pos < (unsigned)cap) act[pos] = j0 + bit;
+                        ++pos;
+                    }
+                }
+            }
+        };
+        // (the events first: their places are known)
+        for (unsigned k = (unsigned)tid; k < n_ev && k < (unsigned)cap; k += kRbBlock) act[k] = (unsigned)n + (unsigned)s.rb_in_events[ka + k];
+        if (tid == 0) listed[turn ^ 1] = 0u;
+#pragma unroll
+        for (int b = 0; b < kWideTurns; ++b) base[b] = 0u;
+        list_words(true, 0u - n_ev);
+        if (arrival) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        if (arrival && tid == 0) __hip_atomic_fetch_add(arrival, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const unsigned total = listed[turn] + n_ev;
+        for (unsigned c0 = 0;;) {
+            const unsigned here = min(total - c0, (unsigned)cap);
+            for (unsigned a = (unsigned)tid >> ts; a < here; a += (unsigned)kRbBlock >> ts) pull_row(act[a], q_lo, q_wrap);
+            __syncthreads();
+            c0 += (unsigned)cap;
+            if (c0 >= total) break;
+            // (a volley outgrows the list: the next window of it)
+            for (unsigned k = (unsigned)tid; k < n_ev; k += kRbBlock)
+                if (k - c0 < (unsigned)cap) act[k - c0] = (unsigned)n + (unsigned)s.rb_in_events[ka + k];
+            list_words(false, c0 - n_ev);
+            __syncthreads();
+        }
+    };
     auto pull = [&](int hist_row, int slot0, unsigned ka, unsigned kb, unsigned *arrival) {
         const unsigned q_lo = (unsigned)slot0 * 4u, q_wrap = q_lo - 4u * (unsigned)S;
         unsigned long long v[kWords];
@@ -206,12 +305,21 @@ __global__ __launch_bounds__(kRbBlock) void sim_resident_batch_kernel(bmtk_glif3
         }
     };
     auto fold = [&](int slot) {
-        unsigned long long *cell = ring_l + (size_t)slot * GLIF3_NREC * span + tid;
+        if (kPer > 1) asm volatile("" : "+s"(slot));
 #pragma unroll
-        for (int r = 0; r < GLIF3_NREC; ++r) {
-            const float a = from_fixed(cell[r * span]);
-            cell[r * span] = 0ull;
-            st.y1[r] = st.y1[r] + a * p.psc0[r];
+        for (int u = 0; u < kPer; ++u) {
+            if (!owns(u)) continue;
+            Sum *cell = ring_l + (size_t)slot * GLIF3_NREC * span + place(u);
+#pragma unroll
+            for (int r = 0; r < GLIF3_NREC; ++r) {
+                float a;
+                if constexpr (kFixed)
+                    a = from_fixed(cell[r * span]);
+                else
+                    a = cell[r * span];
+                cell[r * span] = (Sum)0;
+                st[u].y1[r] = st[u].y1[r] + a * p[u].psc0[r];
+            }
         }
     };
 
@@ -219,7 +327,7 @@ __global__ __launch_bounds__(kRbBlock) void sim_resident_batch_kernel(bmtk_glif3
     const int64_t *in_ptr = q.has_events ? s.rb_in_ptr + (int64_t)trial * (q.n_steps + 1) : nullptr;
     int opaque_zero;
     asm volatile("v_mov_b32 %0, 0" : "=v"(opaque_zero));
-    constexpr int kLooker = kRbBlock - kWave;  // its wavefront owns no neurons at spans up to 960
+    constexpr int kLooker = kRbBlock - kWave;  // its wavefront owns no neurons at spans up to 960, or with two to a thread
     const float zero[GLIF3_NREC] = {0.0f, 0.0f, 0.0f, 0.0f};
     unsigned ka = 0u, kb = 0u;
     if (in_ptr) {
@@ -234,18 +342,24 @@ __global__ __launch_bounds__(kRbBlock) void sim_resident_batch_kernel(bmtk_glif3
         unsigned kn = 0u;
         if (in_ptr) kn = (unsigned)in_ptr[k + 2 + opaque_zero];
         if (k > 0 && tid == kLooker) go_on = poll(k - 1);
-        bool spike = false;
-        float frac;
-        if (own) {
-            if (k > 0) fold(slot);
-            spike = glif3_update(st, p, s.h, zero, I, &frac);
+        if (k > 0) fold(slot);
+        float h = s.h;
+        if (kPer > 1) asm volatile("" : "+s"(h));  // (nor h times a neuron's propagators)
+#pragma unroll
+        for (int u = 0; u < kPer; ++u) {
+            bool spike = false;
+            float frac;
+            if (owns(u)) spike = glif3_update(st[u], p[u], h, zero, I[u], &frac);
+            const unsigned long long m = __ballot(spike);
+            const int i = e0 + place(u);
+            if (lane == 0 && place(u) < span && i < n)
+                __hip_atomic_store(hist + (int64_t)(k & (kRbHist - 1)) * (q.words + 1) + (i >> 6), m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (spike && s.spike_bits) {
+                const int64_t e = element(u);
+                __hip_atomic_fetch_or(reinterpret_cast<unsigned long long *>(s.spike_bits) + (int64_t)k * s.spike_bits_stride + (e >> 6),
+                                      1ull << (e & 63), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
         }
-        const unsigned long long m = __ballot(spike);
-        if (lane == 0 && tid < span && (i & ~(kWave - 1)) < n)
-            __hip_atomic_store(hist + (int64_t)(k & (kRbHist - 1)) * (q.words + 1) + (i >> 6), m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (spike && s.spike_bits)
-            __hip_atomic_fetch_or(reinterpret_cast<unsigned long long *>(s.spike_bits) + (int64_t)k * s.spike_bits_stride + (e >> 6),
-                                  1ull << (e & 63), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         __syncthreads();
         if (k > 0 && !go_on) {
             aborted = true;
@@ -254,8 +368,11 @@ __global__ __launch_bounds__(kRbBlock) void sim_resident_batch_kernel(bmtk_glif3
         // (a call's first step: the spikes of the step before were added by the call before it, and so were its events unless
         //  they are to be taken from this call's lists)
         const bool with_events = k > 0 || s.rb_late_events;
-        pull(k > 0 ? (k - 1) & (kRbHist - 1) : -1, slot, ka, with_events ? kb : ka,
-             counter_of(k) + (g & (BMTK_RES_SYNC_WAYS - 1)) * kWayStride);
+        unsigned *const arrival = counter_of(k) + (g & (BMTK_RES_SYNC_WAYS - 1)) * kWayStride;
+        if constexpr (kPer > 1)
+            pull_wide(k > 0 ? (k - 1) & (kRbHist - 1) : -1, slot, ka, with_events ? kb : ka, arrival, k & 1);
+        else
+            pull(k > 0 ? (k - 1) & (kRbHist - 1) : -1, slot, ka, with_events ? kb : ka, arrival);
         ka = kb;
         kb = (unsigned)__builtin_amdgcn_readfirstlane((int)kn);
         slot = slot + 1 == S ? 0 : slot + 1;
@@ -267,12 +384,17 @@ __global__ __launch_bounds__(kRbBlock) void sim_resident_batch_kernel(bmtk_glif3
     }
     if (!aborted) {
         // closing: what arrived in the last step, then the spikes (and events) of the last step
-        if (own) fold(slot);
+        fold(slot);
         __syncthreads();
-        pull((n_steps - 1) & (kRbHist - 1), slot, ka, kb, nullptr);
+        if constexpr (kPer > 1)
+            pull_wide((n_steps - 1) & (kRbHist - 1), slot, ka, kb, nullptr, n_steps & 1);
+        else
+            pull((n_steps - 1) & (kRbHist - 1), slot, ka, kb, nullptr);
         __syncthreads();
     }
-    if (own) glif3_store(st, s.V, s.asc, s.y1, s.y2, s.ref, ne, e);
+#pragma unroll
+    for (int u = 0; u < kPer; ++u)
+        if (owns(u)) glif3_store(st[u], s.V, s.asc, s.y1, s.y2, s.ref, ne, element(u));
     for (int c = tid; c < S * GLIF3_NREC * span; c += kRbBlock) {
         const int plane = c / span, k = c - plane * span;
         if (k < mine) ring_g[(int64_t)plane * n + k] = ring_l[c];
@@ -319,9 +441,11 @@ int simulate_resident_batch(const bmtk_glif3_sim &s, int64_t step0, int64_t n_st
 {
     const int batch = s.batch, S = s.ring_slots - 1, span = s.rb_span, G = s.rb_groups, W = s.rb_ways;
     const int64_t n = s.n_neurons;
-    BMTK_REQUIRE(batch >= 2 && batch <= kWave, "glif3_simulate_fwd: resident trials come in batches of 2 to 64");
-    BMTK_REQUIRE(span >= kWave && span % kWave == 0 && span <= kRbBlock && G == (n + span - 1) / span,
-                 "glif3_simulate_fwd: rb_span must be a multiple of 64 up to 1024 and rb_groups ceil(n_neurons / rb_span)");
+    BMTK_REQUIRE(batch >= 1 && batch <= kWave, "glif3_simulate_fwd: resident trials come in batches of 1 to 64");
+    const bool wide = span > kRbBlock;
+    BMTK_REQUIRE(span >= kWave && span % kWave == 0 && span <= (batch == 1 ? 2 * (kRbBlock - kWave) : kRbBlock) && G == (n + span - 1) / span,
+                 "glif3_simulate_fwd: rb_span must be a multiple of 64 up to 1024 (one trial: 1920) and rb_groups ceil(n_neurons / rb_span)");
+    BMTK_REQUIRE(wide == (batch == 1), "glif3_simulate_fwd: a single trial is resident in spans above 1024 here, in shorter ones by res_span");
     BMTK_REQUIRE(W >= 1 && W <= batch && s.rb_team_shift >= 0 && s.rb_team_shift <= 6 && s.rb_list >= kWave,
                  "glif3_simulate_fwd: rb_ways must lie in 1..batch, rb_team_shift in 0..6, rb_list from 64 on");
     BMTK_REQUIRE(s.rb_seg && s.rb_packed && s.rb_ring && s.rb_hist && s.res_sync, "glif3_simulate_fwd: resident trials need rb_* and res_sync");
@@ -329,7 +453,7 @@ int simulate_resident_batch(const bmtk_glif3_sim &s, int64_t step0, int64_t n_st
     BMTK_REQUIRE(!s.save_v && !s.probe_col && !s.spike_count, "glif3_simulate_fwd: resident trials return spike bits only");
     BMTK_REQUIRE((s.rb_in_ptr == nullptr) == (s.rb_in_events == nullptr), "glif3_simulate_fwd: rb_in_ptr and rb_in_events go together");
     BMTK_REQUIRE(n_steps < (1ll << 30) && n + s.n_inputs < (1ll << 24), "glif3_simulate_fwd: too many steps or sources for resident trials");
-    const size_t lds = (size_t)S * GLIF3_NREC * span * sizeof(unsigned long long) + (size_t)s.rb_list * sizeof(unsigned);
+    const size_t lds = (size_t)S * GLIF3_NREC * span * (wide ? sizeof(float) : sizeof(unsigned long long)) + (size_t)s.rb_list * sizeof(unsigned);
     BMTK_REQUIRE(lds + 256u <= kResLdsBytes, "glif3_simulate_fwd: the ring slice of resident trials does not fit in LDS");
     RbLaunch q{};
     q.step0 = step0;
@@ -339,9 +463,10 @@ int simulate_resident_batch(const bmtk_glif3_sim &s, int64_t step0, int64_t n_st
     q.has_events = s.rb_in_ptr != nullptr;
     q.sync_slots = kRbCounters;
     while (q.sync_slots * W > kRbCounters) q.sync_slots /= 2;
-    BMTK_REQUIRE(q.words <= 4 * kRbBlock, "glif3_simulate_fwd: more neurons than resident trials can hold");
-    const void *kernel = q.words <= kRbBlock ? reinterpret_cast<const void *>(sim_resident_batch_kernel<1>)
-                                             : reinterpret_cast<const void *>(sim_resident_batch_kernel<4>);
+    BMTK_REQUIRE(q.words <= (wide ? kRbWideWords : 4) * kRbBlock, "glif3_simulate_fwd: more neurons than resident trials can hold");
+    const void *kernel = wide ? reinterpret_cast<const void *>(sim_resident_batch_kernel<kRbWideWords, 2, float>)
+                         : q.words <= kRbBlock ? reinterpret_cast<const void *>(sim_resident_batch_kernel<1, 1, unsigned long long>)
+                                               : reinterpret_cast<const void *>(sim_resident_batch_kernel<4, 1, unsigned long long>);
     hipError_t err = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (err != hipSuccess) {
         set_error("glif3_simulate_fwd: resident trials need %zu bytes of LDS: %s", lds, hipGetErrorString(err));

@@ -35,7 +35,8 @@ PUSH_PS_PER_EVENT = 48.0
 # The form with resident trials pays a chain of dependent loads and a barrier per launch and step, a visit per row that fired,
 # little per event.  Measured, us per step trials / fused / pushed (neurons x trials, in-degree): 51,978 x 32, 1154: 38 / 95 / - ;
 # 20,011 x 20, 820: 8.3 / 31 / - ; 230,924 x 8, 335: 59 / 134 / 164; 5,000 x 16, 400: 2.8 / 9.8 / - ; 31,000 x 64, 160: 36 / 38 / 87;
-# 120,000 x 16, 150: 41 / 52 / 82; 100,000 x 4, 260: 10 / - / 28; 2,000 x 40, 200: 3.3 / 6.3 / 11.5; 3,000 x 4, 200: 2.7 / - / 11.5.
+# 120,000 x 16, 150: 41 / 52 / 82; 100,000 x 4, 260: 10 / - / 28; 2,000 x 40, 200: 3.3 / 6.3 / 11.5; 3,000 x 4, 200: 2.7 / - / 11.5;
+# 400,123 x 1, 180: 9.8 / - / 25.4.
 TRIALS_PS_PER_PASS = 3.0e6
 TRIALS_PS_PER_ROW = 6.5e3       # per neuron of ONE trial that fires in a step (and the input events that come with it)
 TRIALS_PS_PER_EVENT = 0.8
@@ -51,6 +52,7 @@ RES_LDS_EXTRA = RES_ACT_ENTRIES * 4 + 256   # the list plus the kernel's static 
 # the items (rows to walk) of two steps and its static LDS (SOLO_LDS_EXTRA)
 SOLO_LDS_PER_ELEMENT = 4 * 4
 SOLO_LDS_EXTRA = 10240 + 2048
+RB_WIDE_SPAN = 1920             # neurons of a workgroup at most with two to a thread
 RB_LIST_MIN, RB_LDS_STATIC = 2000, 256   # the form with resident trials: least room for its list of rows, static LDS
 TRIALS_MIN_STEPS = 32           # shorter calls are left to the launch-per-step drivers
 RECORD_WAYS = 64                # lists a large spike record is split into (bmtk_glif3_sim.spike_ways)
@@ -80,10 +82,18 @@ def resident_trials_plan(n_neurons, batch, ring_slots, n_cu):
     """How the trials of a batch share ``n_cu`` compute units when each keeps its state in registers and its arrivals of
     the next ring_slots - 1 steps in LDS: dict(span, groups, ways, passes, list) -- ``ways`` trials side by side on
     ``groups`` workgroups of ``span`` neurons each, ``passes`` launches, ``list`` places in the list of rows -- or None
-    where a single trial does not fit.  As few launches as possible: a step costs much the same whatever runs beside it."""
+    where a single trial does not fit.  As few launches as possible: a step costs much the same whatever runs beside it.  One trial:
+    only where the network is too large for the resident mode."""
     cus, slots = n_cu - n_cu % 8, ring_slots - 1
-    if not 2 <= batch <= 64 or cus <= 0 or n_neurons <= 0 or slots < 1:
+    if not 1 <= batch <= 64 or cus <= 0 or n_neurons <= 0 or slots < 1:
         return None
+    if batch == 1:
+        # one trial of more neurons than the compute units have threads: two to a thread, sums in fp32
+        span = -(-(-(-n_neurons // cus)) // 64) * 64
+        rows = min(RES_ACT_ENTRIES, (RES_LDS_BYTES - RB_LDS_STATIC) // 4 - span * slots * NREC)
+        if not 1024 < span <= RB_WIDE_SPAN or rows < RB_LIST_MIN:
+            return None
+        return dict(span=span, groups=-(-n_neurons // span), ways=1, passes=1, list=rows)
     per_neuron = slots * NREC * 8
     span_max = min(1024, (RES_LDS_BYTES - RB_LDS_STATIC - 4 * RB_LIST_MIN) // per_neuron // 64 * 64)
     if span_max < 64 or -(-n_neurons // span_max) > cus:
@@ -165,7 +175,8 @@ class Glif3Simulator:
                 atomics as spikes occur -- the faster form for batched runs.  "auto": by ``expected_rate_hz``
                 (and delay_offset 0, network small enough for the activity map in LDS).  Recurrent arrivals still ahead at the end
                 of a run then live in the history, and ``ring`` holds the input arrivals only.
-    resident_trials  batches of 2 to 64 with a recurrent table and delay_offset 0: trials side by side, each with its state
+    resident_trials  batches of 2 to 64, or one trial of more neurons than ``resident`` holds (1024 to a compute unit; here up
+                to 1920), with a recurrent table and delay_offset 0: trials side by side, each with its state
                 in registers and its ring in LDS for the length of a call, as many at a time as the compute units hold
                 (``resident_trials_plan``).  "auto": where resident, fused and pull are "auto" too, the network fits and
                 ``trials_pay`` says so.  Such a simulator also holds the driver it would have without; a call that asks
@@ -375,10 +386,10 @@ class Glif3Simulator:
             if not trials_pay(plan, self.n, self.batch, n_syn, self.class_id is not None, expected_rate_hz, self.h,
                               self.fuse_table is not None):
                 plan = None
-        if plan and not self._trials_weights_ok(fixed_point_ok):
+        if plan and self.batch > 1 and not self._trials_weights_ok(fixed_point_ok):   # (one trial: sums in fp32)
             plan = None
         if resident_trials is True and plan is None:
-            raise ValueError("resident trials need a recurrent table, a batch of 2 to 64, delay_offset 0, no pull table, weights "
+            raise ValueError("resident trials need a recurrent table, a batch of 2 to 64 (or more neurons than the resident mode holds), delay_offset 0, no pull table, weights "
                              "that 64-bit fixed point holds and a network whose trial fits the compute units")
         if plan:
             self._trials = dict(plan, seg=None)
@@ -418,7 +429,8 @@ class Glif3Simulator:
         # lanes to a segment at most: about as many as it holds synapses on average
         segment = int(math.ceil(math.log2(max(1.0, at / float(max(1, row)) / groups))))
         tr.update(seg=seg, packed=packed, max_team_shift=min(6, segment),
-                  ring=torch.zeros(self.batch, self.L - 1, NREC, n, dtype=torch.int64, device=self.dev),
+                  ring=torch.zeros(self.batch, self.L - 1, NREC, n, device=self.dev,
+                                   dtype=torch.int64 if self.batch > 1 else torch.float32),
                   hist=torch.zeros(tr["ways"], 4, n_words(n) + 1, dtype=torch.int64, device=self.dev))
 
     def _trials_run(self, s, n_steps):
@@ -460,7 +472,9 @@ class Glif3Simulator:
             self._left_ring, self._pend_until, self._trials_left = left, self.step + slots, True
             return
         for t in range(self.step, self.step + slots):
-            cells = (left[:, t % slots].double() * 2.0 ** -32).float()            # [batch][4][n]
+            cells = left[:, t % slots]                                            # [batch][4][n]
+            if cells.dtype == torch.int64:
+                cells = (cells.double() * 2.0 ** -32).float()
             self._ring[t % self.L] += cells.permute(1, 2, 0).reshape(NREC, self.ne)
 
     # What the launch-per-step drivers keep between calls.  A caller that looks at it finds it as they would have left it: the

@@ -384,23 +384,23 @@ typedef struct bmtk_glif3_sim {
                                         * emitted in the steps behind take what step0 - 1 still had under way along) */
     int32_t fuse_max_team;             /* fused form: most wavefronts that share a group of neurons in a network too small to
                                         * give every wavefront one (0: 16): about as many as the group's run has blocks of 256 */
-    /* Resident form of a batch's trials (optional, batches of 2 to 64, delay_offset 0; rb_groups == 0 disables it; takes
-     * precedence over everything above): cooperative launches in which rb_ways trials run side by side, each on
+    /* Resident form of a batch's trials (optional, batches of 2 to 64, or one trial with rb_span above 1024 and its sums in
+     * fp32; delay_offset 0; rb_groups == 0 disables it; takes precedence over everything above): cooperative launches in which rb_ways trials run side by side, each on
      * rb_groups = ceil(n_neurons / rb_span) workgroups that keep its state in registers and its arrivals of the next
      * ring_slots - 1 steps in LDS (64-bit fixed point, as the fused form's sums) for the whole call.  Spike bits are the only
      * output it knows (no save_v, probes or spike record).  The arrivals still ahead at the end of a call are left in
      * rb_ring, and a call begins with those: neither `ring` nor work_bits is used.  The fused form takes them over
      * (rb_pend_until).  Uses res_sync and res_spin_limit as the resident mode does. */
-    int32_t rb_span;                   /* neurons of a workgroup: a multiple of 64 up to 1024 */
+    int32_t rb_span;                   /* neurons of a workgroup: a multiple of 64 up to 1024; one trial: from 1088 to 1920 */
     int32_t rb_groups;
     int32_t rb_ways;                   /* trials of a launch: rb_ways * rb_groups workgroups must be resident at once */
     int32_t rb_team_shift;             /* 2^rb_team_shift lanes read a row's segment */
-    int32_t rb_list;                   /* places of the list of rows in LDS; (ring_slots-1)*32*rb_span + 4*rb_list + 256 bytes of LDS */
+    int32_t rb_list;                   /* places of the list of rows in LDS; (ring_slots-1)*32*rb_span (one trial: *16) + 4*rb_list + 256 bytes of LDS */
     int32_t rb_late_events;            /* the input events of a call's last step (each id once; repeats are delivered at once) are
                                         * left to the next call and its lists, as with in_again */
     const uint32_t *rb_seg;            /* [n_neurons + n_inputs][rb_groups + 1], bmtk_csr_segment_offsets with rb_span over rb_packed */
     const bmtk_synapse *rb_packed;     /* recurrent rows followed by the input rows, sorted by target within a row */
-    uint64_t *rb_ring;                 /* [batch][ring_slots - 1][4][n_neurons], zeroed before the first run */
+    uint64_t *rb_ring;                 /* [batch][ring_slots - 1][4][n_neurons], zeroed before the first run (one trial: floats) */
     uint64_t *rb_hist;                 /* [rb_ways][4][ceil(n_neurons/64) + 1], zeroed once */
     const int64_t *rb_in_ptr;          /* [batch * (n_steps + 1) + 1], or NULL: input events of trial b in step step0 - 1 + k are */
     const int32_t *rb_in_events;       /* ... rb_in_events[p[b*(n_steps+1)+k] .. p[b*(n_steps+1)+k+1]) (bmtk_events_by_trial) */

@@ -123,6 +123,55 @@ def test_more_rows_in_a_step_than_the_list_holds():
     _same(sim, [sim.run(steps)], want["raster"], st)
 
 
+def _wide_case(n, max_delay, classes, steps, seed):
+    """One trial of more neurons than the compute units have threads: sparse, driven by currents and repeated input events."""
+    rng = np.random.default_rng(seed)
+    par = synthetic.random_cells(rng, classes or n)
+    cls = rng.integers(0, classes, n).astype(np.int32) if classes else None
+    tables, n_in = [], 500
+    for rows, nnz in ((n, 12 * n), (n_in, 2 * n)):
+        t = ops.SynapseTable.from_edges(rng.integers(0, rows, nnz), rng.integers(0, n, nnz), rng.normal(0, 20, nnz).astype(np.float32),
+                                        rng.integers(1, max_delay + 1, nnz), rng.integers(0, 4, nnz), rows, n)
+        tables.append(_quarter(tuple(x.cpu().numpy() for x in (t.indptr, t.indices, t.weights, t.delays, t.receptors))))
+    counts = rng.poisson(6.0, steps)
+    counts[::5] = 0
+    events = np.concatenate([np.sort(rng.integers(0, 40, c)) for c in counts]).astype(np.int32)
+    ptr = np.concatenate([[0], np.cumsum(counts)]).astype(np.int64)
+    i_ext = rng.uniform(0.0, 900.0, n).astype(np.float32)
+    st = orc.new_state(n, 1, np.float32)
+    orc.set_threads(orc.max_threads())
+    want = orc.simulate(st, orc.precompute(par, 1.0), 1.0, steps, class_id=cls, ring=np.zeros((max_delay + 1, 4, n), np.float32),
+                        rec=tables[0], inp=tables[1], in_ptr=ptr, in_events=events, i_ext=i_ext, raster=True)
+    sim = Glif3Simulator(n, par, 1.0, class_id=cls, rec=tables[0], inp=tables[1], i_ext=i_ext, ring_slots=max_delay + 1,
+                         resident_trials=True)
+    sim.set_input_events(ptr, events)
+    return sim, want["raster"], st
+
+
+@pytest.mark.parametrize("n,max_delay,classes,places", [(262145, 1, 5, None), (300001, 6, None, None), (491520, 5, 111, 2000)])
+def test_more_neurons_than_threads(n, max_delay, classes, places):
+    """Two neurons to a thread: smallest and largest network, a last workgroup of a few neurons, a list of rows that a step
+    outgrows, arrivals under way between two calls.  Sums of quarters are exact in fp32: bit for bit the oracle's."""
+    sim, raster, st = _wide_case(n, max_delay, classes, 70, n)
+    assert sim._trials is not None and not sim.res_span
+    if places:
+        assert raster.sum(1).max() > places
+        sim._trials["list"] = places
+    _same(sim, [sim.run(33), sim.run(37)], raster, st)
+    assert sim._trials is not None
+
+
+@pytest.mark.parametrize("how", ["short", "record", "ring"])
+def test_more_neurons_than_threads_give_way(how):
+    sim, raster, st = _wide_case(270001, 4, 7, 60, 5)
+    outs = [sim.run(35)]
+    if how == "ring":
+        assert float(sim.ring.abs().sum()) > 0
+    outs += [sim.run(3), sim.run(22)] if how == "short" else [sim.run(25, save_state=how == "record", record_cap=10 ** 6)]
+    assert sim._trials is None
+    _same(sim, outs, raster, st)
+
+
 def test_a_barrier_that_gives_up_is_reported():
     cfg, _, _ = _case(700, 4, 5)
     sim = _sim(cfg, 4, resident_trials=True)

@@ -27,3 +27,12 @@ def test_choice_agrees_with_measured_steps(n, batch, k, fused, pays):
 
 def test_many_launches_for_a_long_ring_do_not_pay():
     assert not trials_pay(resident_trials_plan(8000, 64, 60, 256), 8000, 64, 8000 * 100, False, 3.0, 1.0, True)
+
+
+def test_plan_of_one_trial_with_two_neurons_to_a_thread():
+    for n, slots, span in ((262145, 6, 1088), (400123, 6, 1600), (491520, 6, 1920), (300001, 7, 1216)):
+        p = resident_trials_plan(n, 1, slots, 256)
+        assert p["span"] == span and p["groups"] == -(-n // span) <= 256 and p["ways"] == p["passes"] == 1
+        assert (slots - 1) * NREC * 4 * span + 4 * p["list"] + RB_LDS_STATIC <= RES_LDS_BYTES and p["list"] >= 2000
+    for args in ((262144, 1, 6, 256), (491521, 1, 6, 256), (491520, 1, 7, 256)):
+        assert resident_trials_plan(*args) is None
