@@ -12,18 +12,30 @@ struct Table {
     const uint8_t *delays, *receptors;
 };
 
-// deliver row j of `t` for trial b; all 64 lanes of the wavefront take part
+// deliver row j of `t` for trial b, or of its chunks of 64 synapses every `parts`-th from `part` on; all 64 lanes of the
+// wavefront take part.  Two chunks are in flight at a time: each lane's eight loads travel together, then its additions.
 __device__ __forceinline__ void deliver_row(const Table &t, int j, int b, int batch, float *__restrict__ ring,
-                                            int L, int slot0, int64_t ne)
+                                            int L, int slot0, int64_t ne, int part = 0, int parts = 1)
 {
-    const int p0 = t.indptr[j], p1 = t.indptr[j + 1];
-    for (int p = p0 + lane_id(); p < p1; p += kWave) {
-        const int i = t.indices[p];
-        const float w = t.weights[p];
-        int slot = slot0 + (int)t.delays[p];
-        slot = slot >= L ? slot - L : slot;
-        const int r = t.receptors[p];
-        atomicAdd(ring + ((int64_t)(slot * GLIF3_NREC + r) * ne + (int64_t)i * batch + b), w);
+    constexpr int kTogether = 2;
+    const int p0 = t.indptr[j], p1 = t.indptr[j + 1], stride = parts * kWave;
+    for (int64_t at = (int64_t)p0 + part * kWave + lane_id(); at < p1; at += (int64_t)kTogether * stride) {
+        int i[kTogether], slot[kTogether], r[kTogether];
+        float w[kTogether];
+#pragma unroll
+        for (int u = 0; u < kTogether; ++u) {
+            const int p = (int)min(at + (int64_t)u * stride, (int64_t)p1 - 1);
+            i[u] = t.indices[p];
+            w[u] = t.weights[p];
+            slot[u] = slot0 + (int)t.delays[p];
+            r[u] = t.receptors[p];
+        }
+#pragma unroll
+        for (int u = 0; u < kTogether; ++u) {
+            if (at + (int64_t)u * stride >= p1) continue;
+            const int to = slot[u] >= L ? slot[u] - L : slot[u];
+            atomicAdd(ring + ((int64_t)(to * GLIF3_NREC + r[u]) * ne + (int64_t)i[u] * batch + b), w[u]);
+        }
     }
 }
 

@@ -130,6 +130,31 @@ def test_gather_equals_scatter_and_dense_bruteforce():
     assert rel_err(ring_s.cpu().numpy(), want, 1e-2) < 1e-5
 
 
+@pytest.mark.parametrize("n_active", [0, 1, 127, 128, 129, 4096, 4097, 8193])
+@pytest.mark.parametrize("bound", [None, "exact"])
+def test_scatter_rows_shared_by_wavefronts(n_active, bound):
+    """Few active elements: up to 64 wavefronts to a row, the rows of every length around a chunk and around all chunks of
+    a round.  Weights are small whole numbers, so that the sums are exact in any order."""
+    rng = np.random.default_rng(n_active)
+    n, L = 9000, 5
+    lengths = rng.choice([0, 1, 63, 64, 65, 129], n)
+    lengths[:6] = (64 * 64 - 1, 64 * 64, 64 * 64 + 1, 2 * 64 * 64 + 1, 0, 1)
+    src = np.repeat(np.arange(n, dtype=np.int32), lengths)
+    tgt = rng.integers(0, n, src.size).astype(np.int32)
+    w = rng.integers(1, 9, src.size).astype(np.float32)
+    d, r = rng.integers(1, L, src.size).astype(np.uint8), rng.integers(0, 4, src.size).astype(np.uint8)
+    csr = net.coo_to_csr(src, tgt, w, d, r, n_rows=n, major="source")
+    active = np.arange(n_active, dtype=np.int32)
+    want = np.zeros((L, 4, n))
+    orc.deliver_events(active, 1, csr, want, n, 3)
+    ring = torch.zeros(L, 4, n, device="cuda")
+    ids = torch.zeros(n, dtype=torch.int32, device="cuda")
+    ids[:n_active] = to_dev(active)
+    ops.csr_propagate_scatter(ids, to_dev(np.array([n_active], np.int32)), ops.SynapseTable.from_numpy(csr), ring, n, 1, 3,
+                              max_active=None if bound is None else n_active)
+    np.testing.assert_array_equal(ring.cpu().numpy(), want)
+
+
 def test_empty_rows_and_no_spikes():
     n, L = 70, 4
     csr = net.coo_to_csr(np.array([5], np.int32), np.array([9], np.int32), np.array([2.0], np.float32),
