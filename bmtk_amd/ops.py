@@ -21,7 +21,11 @@ def _dev():
 
 
 def _stream():
-    return torch.cuda.current_stream().cuda_stream
+    """Handle of the current stream.  Asked for without a torch.cuda.Stream around it: that costs 2.3 us per call, a third of
+    what an operation of a caller's own step loop takes on the host."""
+    if not torch.cuda.is_initialized():
+        return torch.cuda.current_stream().cuda_stream
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _p(t, dtype=None, numel=None, name="tensor"):
