@@ -69,7 +69,8 @@ struct __attribute__((packed, aligned(4))) RbBounds {
 // kWords: ballot words per thread.  kPer: neurons per thread; with two, the threads of the last wavefront (the looker) own
 // none.  Sum: what the ring holds, 64-bit fixed point (from_fixed), or floats where a workgroup's neurons are too many for
 // that (batch 1): fp32 atomics into device memory are what it then takes the place of.
-template <int kWords, int kPer, typename Sum>
+// kSave: potentials and step flags of every step go to rb_save_*, trial by trial; by_step_kernel puts them in their order.
+template <int kWords, int kPer, typename Sum, bool kSave>
 __global__ __launch_bounds__(kRbBlock) void sim_resident_batch_kernel(bmtk_glif3_sim s, RbLaunch q)
 {
     constexpr bool kFixed = sizeof(Sum) == 8;
@@ -349,11 +350,18 @@ __global__ __launch_bounds__(kRbBlock) void sim_resident_batch_kernel(bmtk_glif3
         for (int u = 0; u < kPer; ++u) {
             bool spike = false;
             float frac;
+            const int ref_before = st[u].ref;
             if (owns(u)) spike = glif3_update(st[u], p[u], h, zero, I[u], &frac);
             const unsigned long long m = __ballot(spike);
             const int i = e0 + place(u);
             if (lane == 0 && place(u) < span && i < n)
                 __hip_atomic_store(hist + (int64_t)(k & (kRbHist - 1)) * (q.words + 1) + (i >> 6), m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (kSave && owns(u)) {
+                const int64_t to = ((int64_t)trial * n_steps + k) * n + i;
+                s.rb_save_v[to] = st[u].V;
+                s.rb_save_flags[to] = (uint8_t)((spike ? BMTK_F_SPIKE : 0) | (ref_before == 0 ? BMTK_F_INTEGRATING : 0) |
+                                                (ref_before > 0 && st[u].ref == 0 ? BMTK_F_RESET : 0));
+            }
             if (spike && s.spike_bits) {
                 const int64_t e = element(u);
                 __hip_atomic_fetch_or(reinterpret_cast<unsigned long long *>(s.spike_bits) + (int64_t)k * s.spike_bits_stride + (e >> 6),
@@ -398,6 +406,32 @@ __global__ __launch_bounds__(kRbBlock) void sim_resident_batch_kernel(bmtk_glif3
     for (int c = tid; c < S * GLIF3_NREC * span; c += kRbBlock) {
         const int plane = c / span, k = c - plane * span;
         if (k < mine) ring_g[(int64_t)plane * n + k] = ring_l[c];
+    }
+}
+
+// Potentials and flags of 64 neurons and one step from the trials' own rows to the order of the record, [step][neuron][trial].
+// A trial's lane writing its place there itself would store 4 bytes of every 4 * batch, each trial from another XCD: the
+// detour is one more read and write of the record, 0.17 ms for 40 steps of 51,978 x 32 (332 MB).
+constexpr int kByStepPitch = kWave + 1;
+__global__ __launch_bounds__(kBlock) void by_step_kernel(const float *__restrict__ v, const uint8_t *__restrict__ flags, int batch,
+                                                         int n_steps, int n, float *__restrict__ out_v, uint8_t *__restrict__ out_flags)
+{
+    __shared__ float v_l[kWave * kByStepPitch];
+    __shared__ uint8_t flags_l[kWave * kByStepPitch];
+    const int n0 = (int)blockIdx.x * kWave, k = (int)blockIdx.y, mine = min(kWave, n - n0);
+    for (int c = (int)threadIdx.x; c < batch * kWave; c += kBlock) {
+        const int b = c / kWave, j = c % kWave;
+        if (j >= mine) continue;
+        const int64_t from = ((int64_t)b * n_steps + k) * n + n0 + j;
+        v_l[b * kByStepPitch + j] = v[from];
+        flags_l[b * kByStepPitch + j] = flags[from];
+    }
+    __syncthreads();
+    const int64_t to = ((int64_t)k * n + n0) * batch;
+    for (int c = (int)threadIdx.x; c < mine * batch; c += kBlock) {
+        const int j = (int)((unsigned)c / (unsigned)batch), b = c - j * batch;
+        out_v[to + c] = v_l[b * kByStepPitch + j];
+        out_flags[to + c] = flags_l[b * kByStepPitch + j];
     }
 }
 
@@ -450,7 +484,10 @@ int simulate_resident_batch(const bmtk_glif3_sim &s, int64_t step0, int64_t n_st
                  "glif3_simulate_fwd: rb_ways must lie in 1..batch, rb_team_shift in 0..6, rb_list from 64 on");
     BMTK_REQUIRE(s.rb_seg && s.rb_packed && s.rb_ring && s.rb_hist && s.res_sync, "glif3_simulate_fwd: resident trials need rb_* and res_sync");
     BMTK_REQUIRE(s.delay_offset == 0 && (s.delay_bits == 0 || s.delay_bits == 6), "glif3_simulate_fwd: resident trials need delay_offset 0 and the standard packing");
-    BMTK_REQUIRE(!s.save_v && !s.probe_col && !s.spike_count, "glif3_simulate_fwd: resident trials return spike bits only");
+    const bool save = s.save_v != nullptr;
+    BMTK_REQUIRE(!s.probe_col && !s.spike_count, "glif3_simulate_fwd: resident trials take no probes and keep no spike record");
+    BMTK_REQUIRE(!save || (batch > 1 && s.rb_save_v && s.rb_save_flags && n_steps <= 65535),
+                 "glif3_simulate_fwd: resident trials keep the per-step record of batches, up to 65535 steps a call, with rb_save_v and rb_save_flags");
     BMTK_REQUIRE((s.rb_in_ptr == nullptr) == (s.rb_in_events == nullptr), "glif3_simulate_fwd: rb_in_ptr and rb_in_events go together");
     BMTK_REQUIRE(n_steps < (1ll << 30) && n + s.n_inputs < (1ll << 24), "glif3_simulate_fwd: too many steps or sources for resident trials");
     const size_t lds = (size_t)S * GLIF3_NREC * span * (wide ? sizeof(float) : sizeof(unsigned long long)) + (size_t)s.rb_list * sizeof(unsigned);
@@ -464,9 +501,12 @@ int simulate_resident_batch(const bmtk_glif3_sim &s, int64_t step0, int64_t n_st
     q.sync_slots = kRbCounters;
     while (q.sync_slots * W > kRbCounters) q.sync_slots /= 2;
     BMTK_REQUIRE(q.words <= (wide ? kRbWideWords : 4) * kRbBlock, "glif3_simulate_fwd: more neurons than resident trials can hold");
-    const void *kernel = wide ? reinterpret_cast<const void *>(sim_resident_batch_kernel<kRbWideWords, 2, float>)
-                         : q.words <= kRbBlock ? reinterpret_cast<const void *>(sim_resident_batch_kernel<1, 1, unsigned long long>)
-                                               : reinterpret_cast<const void *>(sim_resident_batch_kernel<4, 1, unsigned long long>);
+    const bool few = q.words <= kRbBlock;
+    const void *kernel = wide ? reinterpret_cast<const void *>(sim_resident_batch_kernel<kRbWideWords, 2, float, false>)
+        : few ? (save ? reinterpret_cast<const void *>(sim_resident_batch_kernel<1, 1, unsigned long long, true>)
+                      : reinterpret_cast<const void *>(sim_resident_batch_kernel<1, 1, unsigned long long, false>))
+              : (save ? reinterpret_cast<const void *>(sim_resident_batch_kernel<4, 1, unsigned long long, true>)
+                      : reinterpret_cast<const void *>(sim_resident_batch_kernel<4, 1, unsigned long long, false>));
     hipError_t err = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (err != hipSuccess) {
         set_error("glif3_simulate_fwd: resident trials need %zu bytes of LDS: %s", lds, hipGetErrorString(err));
@@ -501,6 +541,9 @@ int simulate_resident_batch(const bmtk_glif3_sim &s, int64_t step0, int64_t n_st
             return BMTK_E_LAUNCH;
         }
     }
+    if (save)
+        hipLaunchKernelGGL(by_step_kernel, dim3((unsigned)((n + kWave - 1) / kWave), (unsigned)n_steps), dim3(kBlock), 0, stream,
+                           s.rb_save_v, s.rb_save_flags, batch, (int)n_steps, (int)n, s.save_v, s.save_flags);
     BMTK_CHECK_LAUNCH("glif3_simulate_fwd");
     return BMTK_OK;
 }

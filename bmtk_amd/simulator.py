@@ -55,6 +55,7 @@ SOLO_LDS_EXTRA = 10240 + 2048
 RB_WIDE_SPAN = 1920             # neurons of a workgroup at most with two to a thread
 RB_LIST_MIN, RB_LDS_STATIC = 2000, 256   # the form with resident trials: least room for its list of rows, static LDS
 TRIALS_MIN_STEPS = 32           # shorter calls are left to the launch-per-step drivers
+TRIALS_SAVE_BYTES = 1 << 30     # scratch for the per-step record of a call at most: longer calls go in stretches
 RECORD_WAYS = 64                # lists a large spike record is split into (bmtk_glif3_sim.spike_ways)
 
 
@@ -180,7 +181,8 @@ class Glif3Simulator:
                 in registers and its ring in LDS for the length of a call, as many at a time as the compute units hold
                 (``resident_trials_plan``).  "auto": where resident, fused and pull are "auto" too, the network fits and
                 ``trials_pay`` says so.  Such a simulator also holds the driver it would have without; a call that asks
-                for more than spike bits (``save_state``, ``record_cap``, probes), covers fewer than TRIALS_MIN_STEPS
+                for more than spike bits and, of a batch, the per-step record (``record_cap``, probes; ``save_state`` of a single
+                trial or of so many elements that 32 steps of them outgrow TRIALS_SAVE_BYTES), covers fewer than TRIALS_MIN_STEPS
                 steps or is captured into a graph, and a look at ``ring``, ``work_bits`` or ``fuse_any``, make it go on with that
                 driver for good.  True: insist (ValueError otherwise); False: off.
     delay_offset  B steps taken off every delay before the tables are built; spikes and input events are
@@ -372,7 +374,9 @@ class Glif3Simulator:
         self.expected_rate_hz = float(expected_rate_hz)
         self._trials_left, self._pend_until, self._left_ring = False, 0, None
         if resident_trials == "auto":
-            wanted = resident == "auto" and fused == "auto" and pull == "auto" and self.pull_table is None
+            # (resident=False is what the backward pass asks for: no per-step record of a single trial in resident mode)
+            wanted = ((resident == "auto" or (resident is False and self.batch > 1)) and fused == "auto" and pull == "auto"
+                      and self.pull_table is None)
         else:
             wanted = bool(resident_trials)
         plan = None
@@ -460,6 +464,25 @@ class Glif3Simulator:
         _lib.check(self.lib.bmtk_events_by_trial(*args, None, _p(first), _p(sources), _stream()))
         s.rb_in_ptr, s.rb_in_events = _p(first), _p(sources)
         return first, sources
+
+    def _run_trials(self, n_steps, stretch, bits, saved):
+        """A call in the form with resident trials, ``stretch`` steps at a time."""
+        scratch = {}
+        if saved is not None:
+            scratch = dict(v=torch.empty(stretch * self.ne, device=self.dev),
+                           flags=torch.empty(stretch * self.ne, dtype=torch.uint8, device=self.dev))
+        for k in range(0, n_steps, stretch):
+            steps = min(stretch, n_steps - k)
+            s = self._struct(None if bits is None else bits[k:k + steps])
+            lists = self._trials_run(s, steps)
+            if saved is not None:
+                s.save_v, s.save_flags = _p(saved["v"][k:k + steps]), _p(saved["flags"][k:k + steps])
+                s.rb_save_v, s.rb_save_flags = _p(scratch["v"]), _p(scratch["flags"])
+            _lib.check(self.lib.bmtk_glif3_simulate_fwd(C.byref(s), self.step, steps, _stream()))
+            del lists       # (has to live until here)
+            self.step += steps
+            self._lists_replaced = self._trials_left = False
+            self._pending_check = True
 
     def _leave_trials(self):
         """From the form with resident trials to the driver that takes its place, for good: what is still under way is
@@ -767,20 +790,25 @@ class Glif3Simulator:
                           frac=torch.empty(record_cap, dtype=torch.float32, device=self.dev),
                           count=torch.zeros(1 if ways == 1 else ways * _lib.RECORD_COUNT_STRIDE, dtype=torch.int64,
                                             device=self.dev), ways=ways)
-        by_trials = None
-        use_trials = (self._trials is not None and n_steps >= TRIALS_MIN_STEPS and not save_state and record is None
+        use_trials = (self._trials is not None and n_steps >= TRIALS_MIN_STEPS and record is None
                       and self.probe_col is None and not torch.cuda.is_current_stream_capturing())
+        stretch = n_steps
+        if use_trials and save_state:
+            stretch = min(65535, TRIALS_SAVE_BYTES // (5 * self.ne))
+            use_trials = self.batch > 1 and stretch >= TRIALS_MIN_STEPS
         if self._trials is not None and n_steps > 0 and not use_trials:
             self._leave_trials()
-        s = self._struct(bits, record)
-        if use_trials:
-            by_trials = self._trials_run(s, n_steps)
         saved = None
         if save_state:
             if self.res_span:
                 raise ValueError("save_state needs a simulator built with resident=False")
             saved = dict(v=torch.empty(n_steps, self.ne, device=self.dev),
                          flags=torch.empty(n_steps, self.ne, dtype=torch.uint8, device=self.dev), step0=self.step)
+        if use_trials:
+            self._run_trials(n_steps, min(stretch, n_steps), bits, saved)
+            return dict(bits=bits, record=None, saved=saved, probe=None)
+        s = self._struct(bits, record)
+        if saved is not None:
             s.save_v, s.save_flags = _p(saved["v"]), _p(saved["flags"])
         probe = None
         if self.probe_col is not None:
@@ -795,8 +823,7 @@ class Glif3Simulator:
         self.step += n_steps
         self._lists_replaced = self._lists_replaced and n_steps == 0
         self._trials_left = self._trials_left and n_steps == 0
-        self._pending_check = self._pending_check or use_trials or bool(self.res_span)
-        del by_trials
+        self._pending_check = self._pending_check or bool(self.res_span)
         return dict(bits=bits, record=record, saved=saved, probe=probe)
 
     def collect_record(self, record, sort_scale=None):

@@ -49,7 +49,7 @@ extern "C" {
 
 /* Bumped whenever a struct layout or a signature below changes; bmtk_amd_abi_version() returns the value the
  * library was built with. */
-#define BMTK_AMD_ABI_VERSION 27
+#define BMTK_AMD_ABI_VERSION 28
 int bmtk_amd_abi_version(void);
 const char *bmtk_amd_last_error(void);
 /* sizeof(bmtk_glif3_sim) as the library was compiled, for bindings that mirror the struct */
@@ -385,17 +385,19 @@ typedef struct bmtk_glif3_sim {
     int32_t fuse_max_team;             /* fused form: most wavefronts that share a group of neurons in a network too small to
                                         * give every wavefront one (0: 16): about as many as the group's run has blocks of 256 */
     /* Resident form of a batch's trials (optional, batches of 2 to 64, or one trial with rb_span above 1024 and its sums in
-     * fp32; delay_offset 0; rb_groups == 0 disables it; takes precedence over everything above): cooperative launches in which rb_ways trials run side by side, each on
-     * rb_groups = ceil(n_neurons / rb_span) workgroups that keep its state in registers and its arrivals of the next
-     * ring_slots - 1 steps in LDS (64-bit fixed point, as the fused form's sums) for the whole call.  Spike bits are the only
-     * output it knows (no save_v, probes or spike record).  The arrivals still ahead at the end of a call are left in
-     * rb_ring, and a call begins with those: neither `ring` nor work_bits is used.  The fused form takes them over
-     * (rb_pend_until).  Uses res_sync and res_spin_limit as the resident mode does. */
+     * fp32; delay_offset 0; rb_groups == 0 disables it; takes precedence over everything above): cooperative launches in
+     * which rb_ways trials run side by side, each on rb_groups = ceil(n_neurons / rb_span) workgroups that keep its state in
+     * registers and its arrivals of the next ring_slots - 1 steps in LDS (64-bit fixed point, as the fused form's sums) for
+     * the whole call.  Spike bits and, of a batch, the per-step record are the only outputs it knows (no probes or spike
+     * record).  The arrivals still ahead at the end of a call are left in rb_ring, and a call begins with those: neither
+     * `ring` nor work_bits is used.  The fused form takes them over (rb_pend_until).  Uses res_sync and res_spin_limit as
+     * the resident mode does. */
     int32_t rb_span;                   /* neurons of a workgroup: a multiple of 64 up to 1024; one trial: from 1088 to 1920 */
     int32_t rb_groups;
     int32_t rb_ways;                   /* trials of a launch: rb_ways * rb_groups workgroups must be resident at once */
     int32_t rb_team_shift;             /* 2^rb_team_shift lanes read a row's segment */
-    int32_t rb_list;                   /* places of the list of rows in LDS; (ring_slots-1)*32*rb_span (one trial: *16) + 4*rb_list + 256 bytes of LDS */
+    int32_t rb_list;                   /* places of the list of rows in LDS; (ring_slots-1)*32*rb_span (one trial: *16) + 4*rb_list
+                                        * + 256 bytes of LDS */
     int32_t rb_late_events;            /* the input events of a call's last step (each id once; repeats are delivered at once) are
                                         * left to the next call and its lists, as with in_again */
     const uint32_t *rb_seg;            /* [n_neurons + n_inputs][rb_groups + 1], bmtk_csr_segment_offsets with rb_span over rb_packed */
@@ -405,11 +407,13 @@ typedef struct bmtk_glif3_sim {
     const int64_t *rb_in_ptr;          /* [batch * (n_steps + 1) + 1], or NULL: input events of trial b in step step0 - 1 + k are */
     const int32_t *rb_in_events;       /* ... rb_in_events[p[b*(n_steps+1)+k] .. p[b*(n_steps+1)+k+1]) (bmtk_events_by_trial) */
     int64_t rb_pend_until;             /* fused form: rb_ring holds arrivals of the steps before this one (0: none) */
+    float *rb_save_v;                  /* with save_v (batches, up to 65535 steps a call): [batch][n_steps][n_neurons] scratch, and */
+    uint8_t *rb_save_flags;            /* as many bytes with save_flags */
     /* outputs */
     uint64_t *spike_bits;        /* [n_steps][words] spike bits per step, words = ceil(ne/64); or NULL.
                                   * Row k belongs to step step0+k of the call that wrote it. */
     int64_t spike_bits_stride;   /* words per row (>= ceil(ne/64)) */
-    /* optional per-step record for the backward pass (launch-per-step mode only; both or neither):
+    /* optional per-step record for the backward pass (not in resident mode; both or neither):
      * save_v[k][e] = membrane potential after step step0+k, save_flags[k][e] = BMTK_F_* bits */
     float *save_v;
     uint8_t *save_flags;

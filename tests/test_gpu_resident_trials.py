@@ -4,7 +4,7 @@ import pytest
 import torch
 
 from oracle import glif3_oracle as orc
-from bmtk_amd import ops, synthetic
+from bmtk_amd import ops, simulator, synthetic
 from bmtk_amd.simulator import Glif3Simulator, resident_trials_plan
 
 pytestmark = pytest.mark.gpu
@@ -82,6 +82,26 @@ def test_gives_way_to_the_other_drivers_with_arrivals_under_way(batch, fused, ho
         outs += [sim.run(40, save_state=True), sim.run(40, record_cap=100000)]
     assert sim._trials is None
     _same(sim, outs, raster, st)
+
+
+@pytest.mark.parametrize("n,batch,classes,stretch", [(63, 2, None, None), (64, 64, 3, None), (65, 5, None, 32), (1025, 20, 7, 40), (2100, 16, None, None)])
+def test_per_step_record_equals_the_launch_per_step_drivers(monkeypatch, n, batch, classes, stretch):
+    """Potentials and flags in the order [step][neuron][trial], over two calls, in one stretch or several: the bits that the
+    other driver records; then that driver goes on."""
+    cfg, raster, st = _case(n, batch, 4, classes)
+    if stretch:
+        monkeypatch.setattr(simulator, "TRIALS_SAVE_BYTES", 5 * n * batch * stretch)
+    got = []
+    for kw in (dict(resident_trials=True), dict(resident_trials=False)):
+        sim = _sim(cfg, batch, fused=batch >= 8, **kw)
+        a, b = sim.run(100, save_state=True), sim.run(40, save_state=True)
+        assert (sim._trials is not None) == kw["resident_trials"]
+        assert a["saved"]["step0"] == 0 and b["saved"]["step0"] == 100
+        _same(sim, [a, b, sim.run(10, save_state=True)], raster, st)
+        got.append([x[k] for x in (a["saved"], b["saved"]) for k in ("v", "flags")])
+    assert got[0][1].any() and int(got[0][1].max()) <= 7
+    for x, y in zip(*got):
+        assert torch.equal(x, y)
 
 
 def test_input_lists_replaced_between_calls():
