@@ -315,7 +315,8 @@ def bench_bptt(torch, steps=600):
     step_entry = {
         "kernel": "%s (forward), bwd_gather_blocked2_kernel + bwd_state2_kernel (backward, two steps per launch; both "
                   "weight gradients ride in the former)" %
-                  ("sim_fused_kernel: pull and update fused, two steps per launch" if sim.fuse_table is not None
+                  ("sim_resident_batch_kernel: trials side by side, resident for the whole call" if sim._trials is not None
+                   else "sim_fused_kernel: pull and update fused, two steps per launch" if sim.fuse_table is not None
                    else "sim_step_kernel + pull_kernel"),
         "blocked_table_ranges": bptt.n_blocks if bptt.blk is not None else 0,
         "workload": "BPTT step N=51978 nnz=%d inputs=17400 batch=32 steps=%d" % (nnz, steps),
@@ -374,10 +375,9 @@ def bench_bptt(torch, steps=600):
 
 
 def bench_batched_v1(torch, batch=8, steps=300):
-    """The V1-scale network as a batched run, 230,924 neurons x 8 trials, from the settled state, through the
-    launch-per-step driver in the form the simulator picks by itself at this batch and rate (spikes pushed into the
-    ring as events: 0.02 events per synapse and step) and through the fused pull form (248 k sources, so one bit of
-    its activity map stands for several).  Algorithmic bytes: 18 B per synaptic event + 103 B per element update."""
+    """The V1-scale network as a batched run, 230,924 neurons x 8 trials, from the settled state, in the form the
+    simulator picks by itself at this batch and rate (trials side by side, resident for a call) and through the fused
+    pull form (248 k sources, so one bit of its activity map stands for several).  Algorithmic bytes: 18 B per synaptic event + 103 B per element update."""
     import numpy as np
     from bmtk_amd import ops, synthetic, training
     from bmtk_amd.simulator import Glif3Simulator
@@ -399,7 +399,8 @@ def bench_batched_v1(torch, batch=8, steps=300):
         rec_ev, inp_ev = count_events(torch, sim, res["out"]["bits"], 600 + steps // 4)
         per = dev / steps
         alg = (rec_ev + inp_ev) / steps * B_PER_EVENT + sim.ne * B_PER_UPDATE_CLASS
-        out.append({"kernel": "sim_fused_kernel" if sim.fuse_table is not None else "sim_step_kernel",
+        out.append({"kernel": ("sim_resident_batch_kernel" if sim._trials is not None else
+                               "sim_fused_kernel" if sim.fuse_table is not None else "sim_step_kernel"),
                     "workload": "V1-scale batched run: 230,924 neurons x %d trials, %d steps, %s" % (batch, steps, form),
                     "activity_map_sources_per_bit": 1 << sim.fuse_shift if sim.fuse_table is not None else None,
                     "us_per_sim_step": per * 1e6, "neuron_updates_per_s": sim.ne / per,
