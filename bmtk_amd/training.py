@@ -47,31 +47,40 @@ class Glif3Bptt:
     """Reverse-time adjoint over a recorded forward run of a ``Glif3Simulator``
     built with ``resident=False``."""
 
-    # What a row's sum costs in the swept form grows once the L2s no longer hold the adjoint ring; in the blocked form it
-    # grows as a row's segments (its synapses into one target range) get short.  Measured on one MI355X, us per step swept /
-    # blocked (neurons x trials, in-degree; MB of ring, synapses per segment): 37000 x 32, 200 (114, 12) 198 / 256; 30000 x 32,
-    # 300 (92, 19) 189 / 221; 20000 x 32, 300 (61, 37) 111 / 127; 12000 x 32, 800 (37, 100) 108 / 113; 20000 x 32, 700 (61, 87) 208 / 198;
-    # 51978 x 24, 500 (120, 31) 696 / 558; 12000 x 40, 1000 (46, 125) 276 / 196; 16000 x 64, 400 (98, 25) 248 / 191; 51978 x 32, 1000
-    # (160, 42) 740 / 546.  Up to 16 trials the blocked form takes one step per pass over its table only: 30000 x 16, 1000 (46, 125)
-    # 342 / 403; 52000 x 12, 300 (60, 37) 331 / 357; 51978 x 16, 1000 (80, 62) 842 / 733.
-    BLOCKED_MIN_RING_MB = 40.0
-    BLOCKED_MIN_RING_MB_ONE_STEP = 64.0
-    BLOCKED_MIN_RING_TIMES_SEGMENT = 3000.0    # MB x synapses, at up to 32 trials; less above (longer adjoint rows)
+    # A synapse costs the swept form more once the L2s no longer hold the adjoint ring; the blocked form has a fixed part per
+    # row and range, which long rows share among more synapses.  Measured on one MI355X, whole calls of 40 steps, us per step
+    # swept / blocked at in-degree 120, 220, 400, 750 (neurons x trials; MB of ring): 9003 x 32 (28) 25/38 34/42 48/51 78/70;
+    # 15013 x 32 (46) 45/49 58/58 84/76 131/110; 51978 x 32 (160) 198/170 290/212 452/294 753/446; 20011 x 16 (31) 44/54 64/70 98/99
+    # 165/152; 27011 x 16 (41) 63/64 91/87 140/124 244/199; 27011 x 12 (31) 63/65 96/89 156/128 273/203; 15013 x 20 (29) 45/48 63/59
+    # 97/81 160/120; 27011 x 8 (21) 43/53 67/76 107/112 186/174; 51978 x 4 (20) 77/81 127/128 212/195 403/350.  The forms cross
+    # where the ring times the cube root of the in-degree reaches these marks: lower for batches whose adjoint rows (four
+    # bytes a trial) are no whole lines of 64 bytes, so that the swept form's gathers fetch what they do not use.
+    BLOCKED_MIN_RING_MB = 31.0          # at in-degree 400, batch a multiple of 16
+    BLOCKED_MIN_RING_MB_RAGGED = 22.0, 20.0   # other batches up to 16, and above (where it takes two steps per pass)
+    BLOCKED_MIN_RING_MB_FOUR = 17.0     # four trials: a quarter of a line
+    # Four trials through a table of more than 150 MB, which does not stay in the memory-side cache beside the rest: launches of
+    # their own for the parts (27011 x 4, in-degree 750: 139 against 147 swept; 33123 x 4, 598: 155 against 187 and 169 blocked;
+    # 20011 x 4, 750, 120 MB: 106 and 105)
+    PLAIN_MIN_TABLE_BYTES = 150e6
 
     @classmethod
     def blocked_pays(cls, n, batch, ring_slots, nnz):
         """Whether the blocked form is expected to take less time per step than the swept form."""
-        from . import ops
         ring_mb = ring_slots * NREC * n * batch * 4e-6
-        segment = nnz / float(n) / ops.blocked_table_blocks(n, batch, ring_slots)
-        return (ring_mb > (cls.BLOCKED_MIN_RING_MB if batch > 16 else cls.BLOCKED_MIN_RING_MB_ONE_STEP)
-                and ring_mb * segment * max(1.0, batch / 32.0) >= cls.BLOCKED_MIN_RING_TIMES_SEGMENT)
+        least = (cls.BLOCKED_MIN_RING_MB if batch % 16 == 0 else cls.BLOCKED_MIN_RING_MB_FOUR if batch <= 4
+                 else cls.BLOCKED_MIN_RING_MB_RAGGED[batch > 16])
+        return ring_mb * (nnz / (400.0 * n)) ** (1.0 / 3.0) >= least
+
+    @classmethod
+    def plain_pays(cls, batch, nnz):
+        """Whether a launch per part is expected to take less time than the swept form (where the blocked form does not pay)."""
+        return batch <= 4 and 8 * nnz >= cls.PLAIN_MIN_TABLE_BYTES
 
     def __init__(self, sim, dampening=0.3, blocked=None, n_blocks=None, two_steps=True, swept=None):
         """Three forms of the pass, the same gradients.  ``swept``: one launch per two steps through the plain
         source-major table (its adjoint ring ``lam_ring`` has two slots more than ``sim.L``); ``blocked``: the recurrent
         table regrouped by target range for the transposed propagation; neither: a launch per part and step, any batch.
-        None leaves the choice to ``blocked_pays`` where the batch (a multiple of 4 up to 64) allows it.  ``n_blocks``:
+        None leaves the choice to ``blocked_pays`` and ``plain_pays`` where the batch (a multiple of 4 up to 64) allows it.  ``n_blocks``:
         number of target ranges, a multiple of 8 (None: ``ops.blocked_table_blocks``); ``two_steps``: let the blocked form
         take two steps per pass over its table (batches above 16; ``gz`` then holds the partial sums of both)."""
         if sim.res_span or sim.delay_offset:
@@ -93,7 +102,7 @@ class Glif3Bptt:
             raise ValueError("the blocked table needs a recurrent table and a batch that is a multiple of 4 up to 64")
         if blocked is None and not swept:
             blocked = can_block and (swept is False or not can_sweep or self.blocked_pays(sim.n, sim.batch, sim.L, sim.rec.nnz))
-            swept = not blocked and can_sweep and swept is None
+            swept = not blocked and can_sweep and swept is None and not self.plain_pays(sim.batch, sim.rec.nnz)
         self.swept, blocked = bool(swept), bool(blocked)
         # (the swept form writes the adjoint slots of two steps ahead while others are still read)
         self.lam_ring = torch.zeros(sim.L + (2 if self.swept else 0), NREC, ne, device=dev)
