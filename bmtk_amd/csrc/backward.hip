@@ -1547,8 +1547,6 @@ int sweep_plan(const bmtk_glif3_bwd &a, SweepPlan &pl)
     const int64_t groups = (int64_t)n_cu * kSweepPerCu * kSweepWaves * per;  // lane groups the chip holds
     pl.launch.splits = 1;
     while (pl.launch.splits < per && a.n_neurons * pl.launch.splits * 2 <= groups) pl.launch.splits *= 2;
-    if (std::getenv("SPL")) pl.launch.splits = std::atoi(getenv("SPL"));
-    if (pl.launch.splits > per) pl.launch.splits = per;
     const int rows_set = per / pl.launch.splits;
     pl.launch.n_sets = (int)((a.n_neurons + rows_set - 1) / rows_set);
     pl.launch.n_row_wg = (pl.launch.n_sets + kSweepWaves - 1) / kSweepWaves;
