@@ -18,9 +18,10 @@ __device__ __forceinline__ unsigned long long to_fixed(float w)
     return w < 0.0f ? 0ull - v : v;
 }
 
-__device__ __forceinline__ float from_fixed(unsigned long long v)
+// `unit`: what the lowest bit stands for, a power of two (below 2^-32 where the table's weights were scaled up)
+__device__ __forceinline__ float from_fixed(unsigned long long v, double unit = 1.0 / 4294967296.0)
 {
-    return (float)((double)(long long)v * (1.0 / 4294967296.0));
+    return (float)((double)(long long)v * unit);
 }
 
 // One block of a row's synapse stream: positions [base, min(base + kPullChunks*64, p1)) of the packed table.

@@ -25,6 +25,7 @@
 // launch per step with an atomic per event (call and set-up included: 25.4 -> 9.8).  What it is short of are the 128 vector
 // registers a thread has: 84 hold two neurons.  Ballots kept over the prefix sum, addresses and products worked out once
 // for all steps spilled 81 of them to memory (13.3 us per step).
+#include <math.h>
 #include <stdlib.h>
 
 #include "glif3_update.hpp"
@@ -49,6 +50,7 @@ struct RbLaunch {
     int sync_slots;       // arrival counters of a trial, used in turn (a power of two)
     int words;            // ballot words of a trial
     int has_events;
+    double unit;          // of the fixed-point sums
 };
 
 __device__ __forceinline__ unsigned rb_load(const unsigned *p)
@@ -315,7 +317,7 @@ __global__ __launch_bounds__(kRbBlock) void sim_resident_batch_kernel(bmtk_glif3
             for (int r = 0; r < GLIF3_NREC; ++r) {
                 float a;
                 if constexpr (kFixed)
-                    a = from_fixed(cell[r * span]);
+                    a = from_fixed(cell[r * span], q.unit);
                 else
                     a = cell[r * span];
                 cell[r * span] = (Sum)0;
@@ -488,6 +490,7 @@ int simulate_resident_batch(const bmtk_glif3_sim &s, int64_t step0, int64_t n_st
     BMTK_REQUIRE(!s.probe_col && !s.spike_count, "glif3_simulate_fwd: resident trials take no probes and keep no spike record");
     BMTK_REQUIRE(!save || (batch > 1 && s.rb_save_v && s.rb_save_flags && n_steps <= 65535),
                  "glif3_simulate_fwd: resident trials keep the per-step record of batches, up to 65535 steps a call, with rb_save_v and rb_save_flags");
+    BMTK_REQUIRE(s.sum_shift >= 0 && s.sum_shift <= BMTK_SUM_SHIFT_MAX, "glif3_simulate_fwd: sum_shift must lie in 0..BMTK_SUM_SHIFT_MAX");
     BMTK_REQUIRE((s.rb_in_ptr == nullptr) == (s.rb_in_events == nullptr), "glif3_simulate_fwd: rb_in_ptr and rb_in_events go together");
     BMTK_REQUIRE(n_steps < (1ll << 30) && n + s.n_inputs < (1ll << 24), "glif3_simulate_fwd: too many steps or sources for resident trials");
     const size_t lds = (size_t)S * GLIF3_NREC * span * (wide ? sizeof(float) : sizeof(unsigned long long)) + (size_t)s.rb_list * sizeof(unsigned);
@@ -498,6 +501,7 @@ int simulate_resident_batch(const bmtk_glif3_sim &s, int64_t step0, int64_t n_st
     q.slots = S;
     q.words = (int)((n + kWave - 1) / kWave);
     q.has_events = s.rb_in_ptr != nullptr;
+    q.unit = ldexp(1.0, -32 - s.sum_shift);
     q.sync_slots = kRbCounters;
     while (q.sync_slots * W > kRbCounters) q.sync_slots /= 2;
     BMTK_REQUIRE(q.words <= (wide ? kRbWideWords : 4) * kRbBlock, "glif3_simulate_fwd: more neurons than resident trials can hold");

@@ -37,6 +37,8 @@
 // blocks, a stage per arrival step and a map of bits took 113 us per step at 2.4 Hz; runs of rows as blocks (no block
 // cut short at a row's end), one stage for both steps that is worked off when it is full, and a byte per source: 95.
 // Any batch from 8 on: 20,011 x 20 trials, 16 M synapses: 36 us per step against 68 as separate pull and update launches.
+#include <math.h>
+
 #include <type_traits>
 
 #include "common.hpp"
@@ -74,6 +76,7 @@ struct FusedLaunch {
     int team;            // wavefronts that share a group (1: every wavefront takes groups of its own from the workgroup's counter)
     int pending;         // bit 0 / 1: the resident form left arrivals of step t0-1 / t0 in rb_ring
     int map_read, map_write;  // which of the two maps of bytes the launch reads and leaves behind (-1: none)
+    double unit;         // of the fixed-point sums
 };
 
 // One block of the synapse stream a wavefront works through: `left` synapses (up to 256 count) of a group's run, which
@@ -630,8 +633,8 @@ __global__ __launch_bounds__(kFuseBlock) void sim_fused_kernel(bmtk_glif3_sim s,
         }
 #pragma unroll
         for (int r = 0; r < GLIF3_NREC; ++r) {
-            a0[r] = from_fixed(acc[r * kWave + lane]);
-            a1[r] = from_fixed(acc[(GLIF3_NREC + r) * kWave + lane]);
+            a0[r] = from_fixed(acc[r * kWave + lane], qp->unit);
+            a1[r] = from_fixed(acc[(GLIF3_NREC + r) * kWave + lane], qp->unit);
             acc[r * kWave + lane] = 0ull;
             acc[(GLIF3_NREC + r) * kWave + lane] = 0ull;
         }
@@ -779,6 +782,7 @@ int simulate_fused(const bmtk_glif3_sim &s, int64_t step0, int64_t n_steps, hipS
                  "glif3_simulate_fwd: the fused form addresses fewer than 2^30 elements");
     BMTK_REQUIRE(s.delay_offset == 0 && (s.delay_bits == 0 || s.delay_bits == 6) && s.hist_slots == L + 4,
                  "glif3_simulate_fwd: the fused form needs delay_offset 0, the standard packing and hist_slots == ring_slots + 4");
+    BMTK_REQUIRE(s.sum_shift >= 0 && s.sum_shift <= BMTK_SUM_SHIFT_MAX, "glif3_simulate_fwd: sum_shift must lie in 0..BMTK_SUM_SHIFT_MAX");
     BMTK_REQUIRE(s.fuse_shift >= 0 && s.fuse_shift <= 16, "glif3_simulate_fwd: fuse_shift must lie in 0..16");
     const int rows = kWave / batch;  // neurons of a group: one 64-bit word of a history row
     const int64_t n_groups = (s.n_neurons + rows - 1) / rows;
@@ -838,6 +842,7 @@ int simulate_fused(const bmtk_glif3_sim &s, int64_t step0, int64_t n_steps, hipS
     q.H = L + 4;
     q.Lr = L + 2;
     q.n_w32 = n_w32;
+    q.unit = ldexp(1.0, -32 - s.sum_shift);
     q.shift = s.fuse_shift;
     q.n_in_words = (int)n_in_words;
     // (whatever this call's lists hold: repeats of an earlier call's lists may still be under way)

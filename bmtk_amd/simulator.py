@@ -54,6 +54,7 @@ SOLO_LDS_PER_ELEMENT = 4 * 4
 SOLO_LDS_EXTRA = 10240 + 2048
 RB_WIDE_SPAN = 1920             # neurons of a workgroup at most with two to a thread
 RB_LIST_MIN, RB_LDS_STATIC = 2000, 256   # the form with resident trials: least room for its list of rows, static LDS
+SUM_SHIFT_MAX = 120             # BMTK_SUM_SHIFT_MAX
 TRIALS_MIN_STEPS = 32           # shorter calls are left to the launch-per-step drivers
 TRIALS_SAVE_BYTES = 1 << 30     # scratch for the per-step record of a call at most: longer calls go in stretches
 RECORD_WAYS = 64                # lists a large spike record is split into (bmtk_glif3_sim.spike_ways)
@@ -104,6 +105,31 @@ def resident_trials_plan(n_neurons, batch, ring_slots, n_cu):
     span = -(-(-(-n_neurons // (cus // ways))) // 64) * 64
     rows = min(RES_ACT_ENTRIES, (RES_LDS_BYTES - RB_LDS_STATIC - span * per_neuron) // 4)
     return dict(span=span, groups=-(-n_neurons // span), ways=ways, passes=passes, list=rows)
+
+
+def fixed_point_shift(tables, n_neurons):
+    """How far weights have to be scaled up, as a power of two, for 64-bit fixed point with a lowest bit of 2^-32 to hold every
+    one of them exactly, so that no sum has fewer bits than one in fp32: 0 where each weight is a whole multiple of 2^-32 (any
+    fp32 number from 2^-9 on is).  None where they do not fit: what could reach a neuron in a step, scaled, has to stay below
+    2^30 (a factor of two for ids repeated within a step), and weights have to be finite."""
+    lowest, most = 0, 0.0
+    for t in tables:
+        if not t.nnz:
+            continue
+        largest = float(t.weights.abs().max())      # (a NaN carries over)
+        if not math.isfinite(largest):
+            return None
+        most += largest * int(torch.bincount(t.indices, minlength=n_neurons).max())
+        for w in t.weights.split(1 << 26):
+            # the power of two that a weight's lowest set bit stands for
+            bits = w.contiguous().view(torch.int32)
+            exponent, mantissa = (bits >> 23) & 0xFF, bits & 0x7FFFFF
+            mantissa = torch.where(exponent > 0, mantissa | 0x800000, mantissa)
+            low_bit = ((mantissa & -mantissa).to(torch.float32).view(torch.int32) >> 23) - 127
+            place = torch.where(mantissa != 0, exponent.clamp(min=1) - 150 + low_bit, torch.zeros_like(low_bit))
+            lowest = min(lowest, int(place.min()))
+    shift = max(0, -32 - lowest)
+    return shift if shift <= SUM_SHIFT_MAX and most * 2.0 ** shift < 2.0 ** 30 else None
 
 
 def fused_pays(n_neurons, batch, n_synapses, class_table, rate_hz, h_ms=1.0):
@@ -318,6 +344,7 @@ class Glif3Simulator:
         self.pull_table = self.pull_syn = self.pull_work = None
         self.pull_inp_table = self.pull_inp_syn = self.pull_inp_work = self.in_hist = None
         self.fuse_table = self._fuse_any = None
+        self.sum_shift = 0      # power of two that the weights of the tables summed in fixed point are scaled by
         self.fuse_wg_per_cu = int(fuse_wg_per_cu)
         can_fuse = ((self.rec is not None or self.inp is not None) and not self.res_span and self.delay_offset == 0
                     and self.delay_bits == 6 and self.batch in FUSE_BATCHES and pull is not False)
@@ -344,14 +371,19 @@ class Glif3Simulator:
         # call's first step the one before it once more.  The fused form does the same where it takes their place (at
         # batches that do not divide 64), so that lists replaced between two calls mean what they meant there.
         pulls = can_pull and (pull is True or (pull == "auto" and dense))
-        self.fuse_rereads = (pulls and 64 % self.batch != 0 and self.inp is not None
-                             and self.L * ((self.n_inputs + 31) // 32) * 4 <= PULL_MAP_BYTES)
+        inp_pulls = self.inp is not None and self.L * ((self.n_inputs + 31) // 32) * 4 <= PULL_MAP_BYTES
+        self.fuse_rereads = pulls and 64 % self.batch != 0 and inp_pulls
         n_syn = sum(t.nnz for t in (self.rec, self.inp) if t is not None)
         if can_fuse and fused and (fused is True or pull is True or
                                    fused_pays(self.n, self.batch, n_syn, self.class_id is not None, expected_rate_hz, self.h)):
             tables = [t for t in (self.rec, self.inp) if t is not None]
             if all(fixed_point_ok(t) for t in tables):
-                self._setup_fused()
+                # Whatever its batches (or separate pull launches in their place) hold in fixed point stays there; where
+                # events would be pushed, as fp32, the sums have to be as good.
+                shift = fixed_point_shift(tables, self.n)
+                if fused is True or shift is not None or 64 % self.batch == 0 or (pulls and (self.inp is None or inp_pulls)):
+                    self.sum_shift = shift or 0
+                    self._setup_fused()
             elif fused is True:
                 raise ValueError("the fused form needs finite weights smaller than 2^31 in size")
         if self.fuse_table is not None:
@@ -364,7 +396,7 @@ class Glif3Simulator:
             # the history must hold one row per ring slot, row t % L = spikes of step t
             self.hist_slots = self.L
             self._work_bits = torch.zeros(self.hist_slots * (self.words + 1), dtype=torch.int64, device=self.dev)
-            if self.inp is not None and self.L * ((self.n_inputs + 31) // 32) * 4 <= PULL_MAP_BYTES:
+            if inp_pulls:
                 self.pull_inp_table = self.inp.transposed(self.n)
                 self.pull_inp_syn = torch.zeros(NREC, self.ne, device=self.dev)
                 need = self.lib.bmtk_csr_propagate_pull_workspace_bytes(self.L, self.n_inputs)
@@ -389,8 +421,11 @@ class Glif3Simulator:
             if not trials_pay(plan, self.n, self.batch, n_syn, self.class_id is not None, expected_rate_hz, self.h,
                               self.fuse_table is not None):
                 plan = None
-        if plan and self.batch > 1 and not self._trials_weights_ok(fixed_point_ok):   # (one trial: sums in fp32)
-            plan = None
+        if plan and self.batch > 1 and self.fuse_table is None:     # (one trial: sums in fp32; the fused form: as good as its own)
+            shift = fixed_point_shift([t for t in (self.rec, self.inp) if t is not None], self.n)
+            if shift is None and not (resident_trials is True and self._trials_weights_ok(fixed_point_ok)):
+                plan = None
+            self.sum_shift = shift or 0
         if resident_trials is True and plan is None:
             raise ValueError("resident trials need a recurrent table, a batch of 2 to 64 (or more neurons than the resident mode holds), delay_offset 0, no pull table, weights "
                              "that 64-bit fixed point holds and a network whose trial fits the compute units")
@@ -398,14 +433,11 @@ class Glif3Simulator:
             self._trials = dict(plan, seg=None)
 
     def _trials_weights_ok(self, fixed_point_ok):
-        """Whether the 64-bit fixed-point sums of the form with resident trials are at least as good as those of the form
-        it takes the place of: always those of the fused form; the fp32 sums of pushed events where the weights are
-        large against 2^-32 and a neuron's all together small against 2^31."""
+        """Whether weights that 64-bit fixed point does not all hold exactly are good enough for a caller who insists on the form
+        with resident trials: large against 2^-32 on average, a neuron's all together small against 2^31."""
         tables = [t for t in (self.rec, self.inp) if t is not None]
         if not all(fixed_point_ok(t) for t in tables):
             return False
-        if self.fuse_table is not None:
-            return True
         size = sum(t.weights.abs().sum(dtype=torch.float64) for t in tables) / max(1, sum(t.nnz for t in tables))
         most = sum(t.weights.abs().max().double() * torch.bincount(t.indices, minlength=self.n).max() for t in tables if t.nnz)
         return bool((size >= 2.0 ** -8) & (most < 2.0 ** 30))
@@ -429,6 +461,8 @@ class Glif3Simulator:
             seg[row:row + t.n_rows] = own + at          # (fewer than 2^31 synapses)
             packed[at:at + t.nnz] = t.packed()[:t.nnz]
             row, at = row + t.n_rows, at + t.nnz
+        if self.sum_shift:
+            packed.view(torch.float32)[:, 1] *= 2.0 ** self.sum_shift
         # lanes to a segment at most: about as many as it holds synapses on average
         segment = int(math.ceil(math.log2(max(1.0, at / float(max(1, row)) / groups))))
         tr.update(seg=seg, packed=packed, max_team_shift=min(6, segment),
@@ -496,7 +530,7 @@ class Glif3Simulator:
         for t in range(self.step, self.step + slots):
             cells = left[:, t % slots]                                            # [batch][4][n]
             if cells.dtype == torch.int64:
-                cells = (cells.double() * 2.0 ** -32).float()
+                cells = (cells.double() * 2.0 ** -(32 + self.sum_shift)).float()
             self._ring[t % self.L] += cells.permute(1, 2, 0).reshape(NREC, self.ne)
 
     # What the launch-per-step drivers keep between calls.  A caller that looks at it finds it as they would have left it: the
@@ -539,6 +573,8 @@ class Glif3Simulator:
         if self.fuse_in_base + n_in + rows >= 2 ** 24:
             return
         self.fuse_table = SynapseTable.joined_by_target(self.rec, self.inp, n, self.fuse_in_base)
+        if self.sum_shift:
+            self.fuse_table.weights *= 2.0 ** self.sum_shift
         self.fuse_table.pad_packed(FUSE_PAD)
         self.fuse_hist_stride = self.fuse_in_base // rows + -(-n_in // rows) + 1
         self.hist_slots = self.L + 4         # two steps per launch: rows read, written and cleared ahead
@@ -697,6 +733,7 @@ class Glif3Simulator:
         s.i_ext = _p(self.i_ext)
         s.work_bits = _p(self._work_bits)
         s.delay_offset, s.hist_slots, s.delay_bits = self.delay_offset, self.hist_slots, self.delay_bits
+        s.sum_shift = self.sum_shift
         if self.pull_table is not None:
             s.pull_indptr, s.pull_packed = _p(self.pull_table.indptr), _p(self.pull_table.packed())
             s.pull_syn, s.pull_work = _p(self.pull_syn), _p(self.pull_work)

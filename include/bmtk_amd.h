@@ -49,7 +49,7 @@ extern "C" {
 
 /* Bumped whenever a struct layout or a signature below changes; bmtk_amd_abi_version() returns the value the
  * library was built with. */
-#define BMTK_AMD_ABI_VERSION 28
+#define BMTK_AMD_ABI_VERSION 29
 int bmtk_amd_abi_version(void);
 const char *bmtk_amd_last_error(void);
 /* sizeof(bmtk_glif3_sim) as the library was compiled, for bindings that mirror the struct */
@@ -409,6 +409,12 @@ typedef struct bmtk_glif3_sim {
     int64_t rb_pend_until;             /* fused form: rb_ring holds arrivals of the steps before this one (0: none) */
     float *rb_save_v;                  /* with save_v (batches, up to 65535 steps a call): [batch][n_steps][n_neurons] scratch, and */
     uint8_t *rb_save_flags;            /* as many bytes with save_flags */
+    /* Fixed-point sums of the fused and the resident form: their tables (fuse_packed, rb_packed) hold the weights times
+     * 2^sum_shift, and a sum's lowest bit (rb_ring's too) stands for 2^-(32 + sum_shift).  A weight is held exactly when that
+     * divides it, otherwise cut off towards zero; what may reach a neuron in a step must stay below 2^(31 - sum_shift). */
+#define BMTK_SUM_SHIFT_MAX 120
+    int32_t sum_shift;                 /* 0..BMTK_SUM_SHIFT_MAX */
+    int32_t _pad3;
     /* outputs */
     uint64_t *spike_bits;        /* [n_steps][words] spike bits per step, words = ceil(ne/64); or NULL.
                                   * Row k belongs to step step0+k of the call that wrote it. */

@@ -5,7 +5,7 @@ import torch
 
 from oracle import glif3_oracle as orc
 from bmtk_amd import ops, simulator, synthetic
-from bmtk_amd.simulator import Glif3Simulator, resident_trials_plan
+from bmtk_amd.simulator import Glif3Simulator, fixed_point_shift, resident_trials_plan
 
 pytestmark = pytest.mark.gpu
 STATE = ("V", "asc", "y1", "y2", "ref")
@@ -16,11 +16,15 @@ def _quarter(table):
     return indptr, indices, (np.round(w * 4.0) / 4.0 + np.sign(w) * 0.25).astype(np.float32), d, r
 
 
-def _case(n, batch, max_delay, classes=None, n_in=120, steps=150, seed=3, in_rate=60.0, once=(0, 0)):
+def _case(n, batch, max_delay, classes=None, n_in=120, steps=150, seed=3, in_rate=60.0, once=(0, 0), small=None):
     cfg = synthetic.small_glif3_network(n=n, n_in=n_in, steps=steps, seed=seed, p_conn=min(0.3, 60.0 / n), in_rate=in_rate,
                                         in_fanout=max(1, min(n, 30)), max_delay=max_delay, n_classes=classes, batch=batch,
                                         w_scale=4.0, in_w_scale=20.0)
     cfg["rec_src"], cfg["inp_src"] = _quarter(cfg["rec_src"]), _quarter(cfg["inp_src"])
+    if small is not None:      # the weights of two of the four receptors
+        for k in ("rec_src", "inp_src"):
+            indptr, indices, w, d, r = cfg[k]
+            cfg[k] = indptr, indices, np.where(r >= 2, w * np.float32(small), w).astype(np.float32), d, r
     cfg["i_ext"] = np.random.default_rng(seed).uniform(0.0, 500.0, n * batch).astype(np.float32)
     # every seventh event twice, but for those of the steps once[0] .. once[1] - 1
     times = np.where(np.arange(cfg["in_events"].size) % 7 == 0, 2, 1)
@@ -150,6 +154,40 @@ def test_repeated_ids_under_way_outlive_their_lists(batch, ends, kw):
         at = end
     assert (sim._trials is not None) == (kw["resident_trials"] and ends[1] - ends[0] >= simulator.TRIALS_MIN_STEPS)
     _same(sim, outs, raster, st)
+
+
+@pytest.mark.parametrize("small", [2.0 ** -12 / 3.0, 2.0 ** -38])
+@pytest.mark.parametrize("batch,kw,calls", [
+    (12, dict(resident_trials=False, fused=True), (150,)), (16, dict(resident_trials=False, fused=True), (150,)),
+    (5, dict(resident_trials=True), (60, 90)), (5, dict(resident_trials=True), (60, 20, 70)), (20, dict(resident_trials=True, fused=True), (60, 20, 70))])
+def test_small_weights_keep_their_bits(batch, kw, calls, small):
+    """Two receptors of ordinary weights, two of weights a 12,000th (all 24 bits in use) or 2^-38 as large: a weight below 2^-9
+    may have bits under 2^-32, one below 2^-32 has no others.  y1 agrees to a few of its last places, receptor by receptor."""
+    cfg, raster, st = _case(900, batch, 5, small=small)
+    sim = _sim(cfg, batch, **kw)
+    outs = [sim.run(n) for n in calls]
+    sim.check()
+    np.testing.assert_array_equal(np.concatenate([sim.raster(o["bits"]).cpu().numpy() for o in outs]), raster)
+    y1 = sim.state.to_numpy()["y1"]
+    for r in range(4):
+        size = np.abs(st["y1"][r]).max()
+        assert size > 0
+        # a sum of up to 16 fp32 addends, each addition within half a last place of the sum of their sizes
+        np.testing.assert_allclose(y1[r], st["y1"][r], rtol=16 * 2.0 ** -24, atol=16 * 2.0 ** -24 * size, err_msg=str(r))
+    assert sim.sum_shift == fixed_point_shift([sim.rec, sim.inp], sim.n) > 0
+
+
+def test_weights_that_fixed_point_does_not_hold_stay_pushed():
+    """2^24 pA beside 2^-40 pA: more than 63 bits.  Left to itself the simulator adds such weights in fp32, as before."""
+    for batch in (5, 12):
+        cfg, raster, st = _case(900, batch, 5, small=2.0 ** -40)
+        auto = dict(i_ext=cfg["i_ext"], ring_slots=cfg["L"], expected_rate_hz=4.0)
+        held = Glif3Simulator(cfg["n"], cfg["par"], 1.0, batch=batch, rec=cfg["rec_src"], inp=cfg["inp_src"], **auto)
+        assert held._trials is not None and held.sum_shift == 10
+        indptr, indices, w, d, r = cfg["rec_src"]
+        far = np.where(r == 0, w * np.float32(2.0 ** 24), w)
+        sim = Glif3Simulator(cfg["n"], cfg["par"], 1.0, batch=batch, rec=(indptr, indices, far, d, r), inp=cfg["inp_src"], **auto)
+        assert sim._trials is None and sim.fuse_table is None
 
 
 def test_more_rows_in_a_step_than_the_list_holds():
