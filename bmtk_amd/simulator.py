@@ -524,6 +524,8 @@ class Glif3Simulator:
         if tr is None or tr["seg"] is None:
             return
         left, slots = tr["ring"], self.L - 1
+        for t in (left, tr["hist"], tr["seg"], tr["packed"]):
+            self._in_use(t)
         if self.fuse_table is not None:
             self._left_ring, self._pend_until, self._trials_left = left, self.step + slots, True
             return
@@ -532,6 +534,11 @@ class Glif3Simulator:
             if cells.dtype == torch.int64:
                 cells = (cells.double() * 2.0 ** -(32 + self.sum_shift)).float()
             self._ring[t % self.L] += cells.permute(1, 2, 0).reshape(NREC, self.ne)
+
+    @staticmethod
+    def _in_use(t):
+        """``t``, about to be let go, is read by launches on the current stream, which need not be the one it was made on."""
+        t.record_stream(torch.cuda.current_stream(t.device))
 
     # What the launch-per-step drivers keep between calls.  A caller that looks at it finds it as they would have left it: the
     # form with resident trials gives way to them first.
@@ -754,6 +761,7 @@ class Glif3Simulator:
             s.in_again = 1 if self.fuse_rereads and (self._lists_replaced or self._trials_left) else 0
             if self._pend_until > self.step:
                 s.rb_ring, s.rb_pend_until = _p(self._left_ring), self._pend_until
+                self._in_use(self._left_ring)
             if self.in_repeat_ptr is not None:
                 s.in_repeat_ptr, s.in_repeat_events = _p(self.in_repeat_ptr), _p(self.in_repeat_events)
         if self.res_span:

@@ -258,6 +258,32 @@ def test_more_neurons_than_threads_give_way(how):
     _same(sim, outs, raster, st)
 
 
+@pytest.mark.parametrize("batch,fused", [(6, False), (16, True)])
+def test_buffers_given_up_wait_for_the_stream_that_reads_them(batch, fused):
+    """Built and first run on the default stream, run and left for the other driver on a second one: the memory of the form's
+    tables and of what it handed over is not given out again on the first stream while the second still works."""
+    cfg, raster, st = _case(900, batch, 5, in_rate=150.0)
+    sim = _sim(cfg, batch, resident_trials=True, fused=fused)
+    outs = [sim.run(40)]
+    own = torch.cuda.Stream()
+    own.wait_stream(torch.cuda.current_stream())
+    torch.cuda.synchronize()
+    with torch.cuda.stream(own):
+        torch.cuda._sleep(100_000_000)
+        outs.append(sim.run(40))
+        given_up = [(t.data_ptr(), t.numel() * t.element_size()) for t in (sim._trials[k] for k in ("ring", "hist", "seg", "packed"))]
+        outs += [sim.run(20), sim.run(20), sim.run(30)]
+        done = torch.cuda.Event()
+        done.record()
+    assert sim._trials is None and sim._left_ring is None
+    others = [torch.empty(size, dtype=torch.uint8, device="cuda") for _, size in given_up for _ in range(4)]
+    assert not done.query()
+    for at, size in given_up:
+        assert all(o.data_ptr() + o.numel() <= at or at + size <= o.data_ptr() for o in others)
+    torch.cuda.synchronize()
+    _same(sim, outs, raster, st)
+
+
 def test_a_barrier_that_gives_up_is_reported():
     cfg, _, _ = _case(700, 4, 5)
     sim = _sim(cfg, 4, resident_trials=True)
