@@ -618,16 +618,22 @@ __global__ __launch_bounds__(kFuseBlock) void sim_fused_kernel(bmtk_glif3_sim s,
         float a0[GLIF3_NREC], a1[GLIF3_NREC];
         const FuseLaunchArgs qp = fresh_launch();
         if (qp->pending) {
-            // the first steps after a call in the resident form: what that call's spikes still send joins the sums
+            // the first steps after a call in the resident form: what that call's spikes still send joins the sums, once (the
+            // launch may be replayed from a graph)
             const FuseArgs sp = fresh_args();
             const int row = fin_grp * kRows + (int)sub_lane, slots = L - 1;
             if (in_group && row < n) {
-                const unsigned long long *left = reinterpret_cast<const unsigned long long *>(in_memory(sp->rb_ring)) +
-                                                 (int64_t)(lane - sub_bit) * slots * GLIF3_NREC * n + row;
+                uint64_t *left = in_memory(sp->rb_ring) + (int64_t)(lane - sub_bit) * slots * GLIF3_NREC * n + row;
+                auto take = [&](int64_t step, int r) {
+                    uint64_t *cell = left + ((int64_t)(step % slots) * GLIF3_NREC + r) * n;
+                    const unsigned long long v = *cell;
+                    *cell = 0ull;
+                    return v;
+                };
 #pragma unroll
                 for (int r = 0; r < GLIF3_NREC; ++r) {
-                    if (qp->pending & 1) acc[r * kWave + lane] += left[((int64_t)((qp->t0 - 1) % slots) * GLIF3_NREC + r) * n];
-                    if (qp->pending & 2) acc[(GLIF3_NREC + r) * kWave + lane] += left[((int64_t)(qp->t0 % slots) * GLIF3_NREC + r) * n];
+                    if (qp->pending & 1) acc[r * kWave + lane] += take(qp->t0 - 1, r);
+                    if (qp->pending & 2) acc[(GLIF3_NREC + r) * kWave + lane] += take(qp->t0, r);
                 }
             }
         }

@@ -404,7 +404,7 @@ class Glif3Simulator:
                 self.in_hist_stride = n_words(self.n_inputs * self.batch) + 1
                 self.in_hist = torch.zeros(self.L * self.in_hist_stride, dtype=torch.int64, device=self.dev)
         self.expected_rate_hz = float(expected_rate_hz)
-        self._trials_left, self._pend_until, self._left_ring = False, 0, None
+        self._trials_left, self._pend_until, self._left_ring, self._kept = False, 0, None, []
         if resident_trials == "auto":
             # (resident=False, as training simulators have it, asks for the launch-per-step drivers; the form is theirs on request)
             wanted = resident == "auto" and fused == "auto" and pull == "auto" and self.pull_table is None
@@ -534,11 +534,16 @@ class Glif3Simulator:
             if cells.dtype == torch.int64:
                 cells = (cells.double() * 2.0 ** -(32 + self.sum_shift)).float()
             self._ring[t % self.L] += cells.permute(1, 2, 0).reshape(NREC, self.ne)
+        if torch.cuda.is_current_stream_capturing():
+            left.zero_()        # (handed over once, however often the graph is replayed)
 
-    @staticmethod
-    def _in_use(t):
-        """``t``, about to be let go, is read by launches on the current stream, which need not be the one it was made on."""
-        t.record_stream(torch.cuda.current_stream(t.device))
+    def _in_use(self, t):
+        """``t``, which will be let go, is read by launches on the current stream, which need not be the one it was made on, or by a
+        graph, with every replay."""
+        if torch.cuda.is_current_stream_capturing():
+            self._kept.append(t)
+        else:
+            t.record_stream(torch.cuda.current_stream(t.device))
 
     # What the launch-per-step drivers keep between calls.  A caller that looks at it finds it as they would have left it: the
     # form with resident trials gives way to them first.

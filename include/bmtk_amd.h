@@ -406,7 +406,8 @@ typedef struct bmtk_glif3_sim {
     uint64_t *rb_hist;                 /* [rb_ways][4][ceil(n_neurons/64) + 1], zeroed once */
     const int64_t *rb_in_ptr;          /* [batch * (n_steps + 1) + 1], or NULL: input events of trial b in step step0 - 1 + k are */
     const int32_t *rb_in_events;       /* ... rb_in_events[p[b*(n_steps+1)+k] .. p[b*(n_steps+1)+k+1]) (bmtk_events_by_trial) */
-    int64_t rb_pend_until;             /* fused form: rb_ring holds arrivals of the steps before this one (0: none) */
+    int64_t rb_pend_until;             /* fused form: rb_ring holds arrivals of the steps before this one (0: none); it takes and
+                                        * clears them */
     float *rb_save_v;                  /* with save_v (batches, up to 65535 steps a call): [batch][n_steps][n_neurons] scratch, and */
     uint8_t *rb_save_flags;            /* as many bytes with save_flags */
     /* Fixed-point sums of the fused and the resident form: their tables (fuse_packed, rb_packed) hold the weights times

@@ -284,6 +284,30 @@ def test_buffers_given_up_wait_for_the_stream_that_reads_them(batch, fused):
     _same(sim, outs, raster, st)
 
 
+@pytest.mark.parametrize("batch,fused", [(6, False), (16, True)])
+def test_arrivals_handed_over_under_capture_come_once(batch, fused):
+    """A call captured behind one with resident trials goes on with the other driver; what the first had under way arrives in the
+    first replay and in no other.  Every replay against the same call made again by a simulator without the form."""
+    cfg, _, _ = _case(900, batch, 5, in_rate=150.0)
+    first, again = 40, 40           # (a whole number of rounds of the fused form's histories)
+    sim, other = _sim(cfg, batch, resident_trials=True, fused=fused), _sim(cfg, batch, resident_trials=False, fused=fused)
+    sim.run(first)
+    other.run(first)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = sim.run(again)
+    assert sim._trials is None and sim.step == first + again
+    for k in range(4):
+        graph.replay()
+        other.step = first
+        want = other.run(again)
+        torch.cuda.synchronize()
+        assert torch.equal(out["bits"], want["bits"]), k
+        for name in STATE:
+            assert torch.equal(getattr(sim.state, name), getattr(other.state, name)), (k, name)
+
+
 def test_a_barrier_that_gives_up_is_reported():
     cfg, _, _ = _case(700, 4, 5)
     sim = _sim(cfg, 4, resident_trials=True)
