@@ -327,14 +327,14 @@ class SynapseTable:
         packed[:self.nnz] = self.packed()[:self.nnz][order]
         return indptr, packed, order
 
-    def segment_offsets(self, span, n_groups):
+    def segment_offsets(self, span, n_groups, out=None):
         """uint32 [n_rows, n_groups+1] offsets of the first synapse per row whose index is >= g*span
-        (stored in an int32 tensor).  Raises if a row is not sorted by index."""
+        (stored in an int32 tensor, ``out`` if given).  Raises if a row is not sorted by index."""
         lib = _lib.load()
-        seg = torch.empty(self.n_rows, n_groups + 1, dtype=torch.int32, device=self.indices.device)
+        seg = torch.empty(self.n_rows, n_groups + 1, dtype=torch.int32, device=self.indices.device) if out is None else out
         flag = torch.zeros(1, dtype=torch.int32, device=self.indices.device)
         _lib.check(lib.bmtk_csr_segment_offsets(self.n_rows, _p(self.indptr), _p(self.indices), span, n_groups,
-                                                _p(seg), _p(flag), _stream()))
+                                                _p(seg, torch.int32, self.n_rows * (n_groups + 1), "out"), _p(flag), _stream()))
         if int(flag.item()):
             raise ValueError("synapse table rows are not sorted by index")
         return seg

@@ -55,6 +55,8 @@ SOLO_LDS_EXTRA = 10240 + 2048
 RB_WIDE_SPAN = 1920             # neurons of a workgroup at most with two to a thread
 RB_LIST_MIN, RB_LDS_STATIC = 2000, 256   # the form with resident trials: least room for its list of rows, static LDS
 SUM_SHIFT_MAX = 120             # BMTK_SUM_SHIFT_MAX
+TRIALS_TABLE_BYTES = 1 << 30    # tables and ring of the form with resident trials at most, or TRIALS_TABLE_RATIO times the synapses' 10 bytes
+TRIALS_TABLE_RATIO = 4
 TRIALS_MIN_STEPS = 32           # shorter calls are left to the launch-per-step drivers
 TRIALS_SAVE_BYTES = 1 << 30     # scratch for the per-step record of a call at most: longer calls go in stretches
 RECORD_WAYS = 64                # lists a large spike record is split into (bmtk_glif3_sim.spike_ways)
@@ -147,6 +149,20 @@ def fused_pays(n_neurons, batch, n_synapses, class_table, rate_hz, h_ms=1.0):
     return fused < push
 
 
+def trials_bytes(plan, n_neurons, batch, ring_slots, n_inputs, n_synapses):
+    """Device memory that the form with resident trials takes beside the synapse tables: bounds of every workgroup's segment of
+    every row, packed records, the ring behind a call."""
+    return ((n_neurons + n_inputs) * (plan["groups"] + 1) * 4 + n_synapses * 8
+            + batch * (ring_slots - 1) * NREC * n_neurons * (8 if batch > 1 else 4))
+
+
+def trials_fit(plan, n_neurons, batch, ring_slots, n_inputs, n_synapses):
+    """Whether that memory is in proportion to the synapses'.  With many sources of few synapses (millions of virtual cells) the bounds
+    alone, a thousand bytes a source, would be many times the network; the other drivers need none."""
+    return (trials_bytes(plan, n_neurons, batch, ring_slots, n_inputs, n_synapses)
+            <= max(TRIALS_TABLE_BYTES, TRIALS_TABLE_RATIO * 10 * n_synapses))
+
+
 def trials_pay(plan, n_neurons, batch, n_synapses, class_table, rate_hz, h_ms, fused):
     """Whether the form with resident trials (``plan``: resident_trials_plan) is expected to take less time per step than
     the driver that would run otherwise, the fused pull form (``fused``) or pushed events."""
@@ -205,8 +221,9 @@ class Glif3Simulator:
     resident_trials  batches of 2 to 64, or one trial of more neurons than ``resident`` holds (1024 to a compute unit; here up
                 to 1920), with a recurrent table and delay_offset 0: trials side by side, each with its state
                 in registers and its ring in LDS for the length of a call, as many at a time as the compute units hold
-                (``resident_trials_plan``).  "auto": where resident, fused and pull are "auto" too, the network fits and
-                ``trials_pay`` says so.  Such a simulator also holds the driver it would have without; a call that asks
+                (``resident_trials_plan``).  "auto": where resident, fused and pull are "auto" too, the network fits,
+                ``trials_pay`` says so and its tables are in proportion to the network (``trials_fit``); where there turns out to be no
+                memory for them the other driver runs.  Such a simulator also holds the driver it would have without; a call that asks
                 for more than spike bits and, of a batch, the per-step record (``record_cap``, probes; ``save_state`` of a single
                 trial or of so many elements that 32 steps of them outgrow TRIALS_SAVE_BYTES), covers fewer than TRIALS_MIN_STEPS
                 steps or is captured into a graph, and a look at ``ring``, ``work_bits`` or ``fuse_any``, make it go on with that
@@ -418,8 +435,9 @@ class Glif3Simulator:
                      or n_syn >= 2 ** 31 or self.pull_table is not None):
             plan = None
         if plan and resident_trials == "auto":
-            if not trials_pay(plan, self.n, self.batch, n_syn, self.class_id is not None, expected_rate_hz, self.h,
-                              self.fuse_table is not None):
+            if not (trials_pay(plan, self.n, self.batch, n_syn, self.class_id is not None, expected_rate_hz, self.h,
+                               self.fuse_table is not None)
+                    and trials_fit(plan, self.n, self.batch, self.L, self.n_inputs, n_syn)):
                 plan = None
         if plan and self.batch > 1 and self.fuse_table is None:     # (one trial: sums in fp32; the fused form: as good as its own)
             shift = fixed_point_shift([t for t in (self.rec, self.inp) if t is not None], self.n)
@@ -430,7 +448,7 @@ class Glif3Simulator:
             raise ValueError("resident trials need a recurrent table, a batch of 2 to 64 (or more neurons than the resident mode holds), delay_offset 0, no pull table, weights "
                              "that 64-bit fixed point holds and a network whose trial fits the compute units")
         if plan:
-            self._trials = dict(plan, seg=None)
+            self._trials = dict(plan, seg=None, insisted=resident_trials is True)
 
     def _trials_weights_ok(self, fixed_point_ok):
         """Whether weights that 64-bit fixed point does not all hold exactly are good enough for a caller who insists on the form
@@ -453,12 +471,13 @@ class Glif3Simulator:
         for t in (self.rec, self.inp):
             if t is None:
                 continue
+            own = seg[row:row + t.n_rows]
             try:
-                own = t.segment_offsets(tr["span"], groups)
+                t.segment_offsets(tr["span"], groups, out=own)
             except ValueError:
                 t = t.sorted_by_index()
-                own = t.segment_offsets(tr["span"], groups)
-            seg[row:row + t.n_rows] = own + at          # (fewer than 2^31 synapses)
+                t.segment_offsets(tr["span"], groups, out=own)
+            own += at                                   # (fewer than 2^31 synapses)
             packed[at:at + t.nnz] = t.packed()[:t.nnz]
             row, at = row + t.n_rows, at + t.nnz
         if self.sum_shift:
@@ -473,8 +492,6 @@ class Glif3Simulator:
     def _trials_run(self, s, n_steps):
         """Fill ``s`` for a call in the form with resident trials.  Returns what has to live until it is launched."""
         tr = self._trials
-        if tr["seg"] is None:
-            self._setup_trials()
         s.rb_span, s.rb_groups, s.rb_ways, s.rb_list = tr["span"], tr["groups"], tr["ways"], tr["list"]
         # as many lanes to a segment as let the workgroup's 1024 take the rows of a step in one go, or in little more
         # (5,000 neurons x 16 trials, some 20 rows of 21 synapses: 6.5 / 3.5 / 2.8 us per step with 1 / 4 / 32 lanes; 51,978 x 32, 220
@@ -499,11 +516,19 @@ class Glif3Simulator:
         return first, sources
 
     def _run_trials(self, n_steps, stretch, bits, saved):
-        """A call in the form with resident trials, ``stretch`` steps at a time."""
+        """A call in the form with resident trials, ``stretch`` steps at a time.  False, and nothing done, if that was the
+        constructor's choice and there is no memory for it."""
         scratch = {}
-        if saved is not None:
-            scratch = dict(v=torch.empty(stretch * self.ne, device=self.dev),
-                           flags=torch.empty(stretch * self.ne, dtype=torch.uint8, device=self.dev))
+        try:
+            if self._trials["seg"] is None:
+                self._setup_trials()
+            if saved is not None:
+                scratch = dict(v=torch.empty(stretch * self.ne, device=self.dev),
+                               flags=torch.empty(stretch * self.ne, dtype=torch.uint8, device=self.dev))
+        except torch.OutOfMemoryError:
+            if self._trials["insisted"]:
+                raise
+            return False
         for k in range(0, n_steps, stretch):
             steps = min(stretch, n_steps - k)
             s = self._struct(None if bits is None else bits[k:k + steps])
@@ -516,6 +541,7 @@ class Glif3Simulator:
             self.step += steps
             self._lists_replaced = self._trials_left = False
             self._pending_check = True
+        return True
 
     def _leave_trials(self):
         """From the form with resident trials to the driver that takes its place, for good: what is still under way is
@@ -854,8 +880,9 @@ class Glif3Simulator:
             saved = dict(v=torch.empty(n_steps, self.ne, device=self.dev),
                          flags=torch.empty(n_steps, self.ne, dtype=torch.uint8, device=self.dev), step0=self.step)
         if use_trials:
-            self._run_trials(n_steps, min(stretch, n_steps), bits, saved)
-            return dict(bits=bits, record=None, saved=saved, probe=None)
+            if self._run_trials(n_steps, min(stretch, n_steps), bits, saved):
+                return dict(bits=bits, record=None, saved=saved, probe=None)
+            self._leave_trials()
         s = self._struct(bits, record)
         if saved is not None:
             s.save_v, s.save_flags = _p(saved["v"]), _p(saved["flags"])

@@ -317,6 +317,26 @@ def test_a_barrier_that_gives_up_is_reported():
         sim.check()
 
 
+@pytest.mark.parametrize("save", [False, True])
+def test_no_memory_for_the_tables(monkeypatch, save):
+    """Chosen by the constructor: the call runs with the driver that the simulator holds beside it.  Insisted on: the error."""
+    def full(self):
+        raise torch.OutOfMemoryError("no memory")
+
+    monkeypatch.setattr(Glif3Simulator, "_setup_trials", full)
+    cfg, raster, st = _case(900, 5, 5)
+    kw = dict(batch=5, class_id=cfg["class_id"], rec=cfg["rec_src"], inp=cfg["inp_src"], i_ext=cfg["i_ext"], ring_slots=cfg["L"])
+    sim = Glif3Simulator(cfg["n"], cfg["par"], 1.0, **kw)
+    assert sim._trials is not None
+    sim.set_input_events(cfg["in_ptr"], cfg["in_events"])
+    outs = [sim.run(50, save_state=save), sim.run(100, save_state=save)]
+    assert sim._trials is None and all((o["saved"] is not None) == save for o in outs)
+    _same(sim, outs, raster, st)
+    sim = _sim(cfg, 5, resident_trials=True)
+    with pytest.raises(torch.OutOfMemoryError):
+        sim.run(50, save_state=save)
+
+
 def test_what_does_not_fit_is_refused():
     assert resident_trials_plan(300000, 8, 6, 256) is None and resident_trials_plan(1000, 65, 6, 256) is None
     cfg, _, _ = _case(200, 2, 3)

@@ -2,7 +2,7 @@
 import pytest
 
 from bmtk_amd.layout import NREC
-from bmtk_amd.simulator import RB_LDS_STATIC, RES_LDS_BYTES, resident_trials_plan, trials_pay
+from bmtk_amd.simulator import RB_LDS_STATIC, RES_LDS_BYTES, resident_trials_plan, trials_bytes, trials_fit, trials_pay
 
 
 @pytest.mark.parametrize("n,batch,slots", [(1, 2, 2), (64, 64, 6), (65, 3, 6), (5000, 16, 6), (20011, 20, 6), (51978, 32, 6), (230924, 8, 6),
@@ -27,6 +27,16 @@ def test_choice_agrees_with_measured_steps(n, batch, k, fused, pays):
 
 def test_many_launches_for_a_long_ring_do_not_pay():
     assert not trials_pay(resident_trials_plan(8000, 64, 60, 256), 8000, 64, 8000 * 100, False, 3.0, 1.0, True)
+
+
+def test_tables_stay_in_proportion_to_the_network():
+    for n, batch, n_in, k in ((230924, 8, 17400, 335), (400123, 1, 30000, 180), (51978, 32, 17400, 1154), (2000, 64, 500, 150), (491520, 1, 60000, 125)):
+        assert trials_fit(resident_trials_plan(n, batch, 6, 256), n, batch, 6, n_in, n * k)
+    # ten million virtual cells of a few synapses each: 10 GB of segment bounds beside 0.5 GB of synapses
+    for n, batch in ((230924, 8), (400123, 1)):
+        plan = resident_trials_plan(n, batch, 6, 256)
+        assert trials_bytes(plan, n, batch, 6, 10 ** 7, 5 * 10 ** 7) > 9e9
+        assert not trials_fit(plan, n, batch, 6, 10 ** 7, 5 * 10 ** 7)
 
 
 def test_plan_of_one_trial_with_two_neurons_to_a_thread():
