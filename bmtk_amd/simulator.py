@@ -421,7 +421,7 @@ class Glif3Simulator:
                 self.in_hist_stride = n_words(self.n_inputs * self.batch) + 1
                 self.in_hist = torch.zeros(self.L * self.in_hist_stride, dtype=torch.int64, device=self.dev)
         self.expected_rate_hz = float(expected_rate_hz)
-        self._trials_left, self._pend_until, self._left_ring, self._kept = False, 0, None, []
+        self._trials_left, self._pend_from, self._pend_until, self._left_ring, self._kept = False, 0, 0, None, []
         if resident_trials == "auto":
             # (resident=False, as training simulators have it, asks for the launch-per-step drivers; the form is theirs on request)
             wanted = resident == "auto" and fused == "auto" and pull == "auto" and self.pull_table is None
@@ -553,7 +553,7 @@ class Glif3Simulator:
         for t in (left, tr["hist"], tr["seg"], tr["packed"]):
             self._in_use(t)
         if self.fuse_table is not None:
-            self._left_ring, self._pend_until, self._trials_left = left, self.step + slots, True
+            self._left_ring, self._pend_from, self._pend_until, self._trials_left = left, self.step, self.step + slots, True
             return
         for t in range(self.step, self.step + slots):
             cells = left[:, t % slots]                                            # [batch][4][n]
@@ -571,8 +571,9 @@ class Glif3Simulator:
         else:
             t.record_stream(torch.cuda.current_stream(t.device))
 
-    # What the launch-per-step drivers keep between calls.  A caller that looks at it finds it as they would have left it: the
-    # form with resident trials gives way to them first.
+    # What the launch-per-step drivers keep between calls.  For a caller that looks at it, the form with resident trials gives way
+    # to them first.  Pushed events are then handed over in the ring; for the fused form, whose history of spike bits cannot
+    # be had from sums, they wait apart (_left_ring) and join its sums in the steps they are due in, unless ``step`` is set back.
     @property
     def ring(self):
         self._leave_trials()
@@ -715,7 +716,12 @@ class Glif3Simulator:
         resolution step, which NEST delivers both): every occurrence is delivered.
         The pull form of the inputs turns a step's events into bits, which hold an id
         once; the second and later occurrences are then listed apart
-        (``in_repeat_ptr`` / ``in_repeat_events``) and delivered as events on top."""
+        (``in_repeat_ptr`` / ``in_repeat_events``) and delivered as events on top.
+
+        Lists that replace others between two calls should still name the events of the step behind (``step - 1``): the
+        separate pull launches read that step once more at the start of a call, and so does the fused form in their
+        place (``fuse_rereads``: batches that do not divide 64, from some ``expected_rate_hz`` on).  Lists without them take
+        back what those events still had under way there; the other forms have delivered them and look at later steps only."""
         if self.inp is None and not self.inp_without_synapses:
             raise ValueError("no input synapse table")
         if torch.is_tensor(in_ptr):
@@ -781,8 +787,9 @@ class Glif3Simulator:
                 s.in_hist, s.in_hist_stride = _p(self.in_hist), self.in_hist_stride
                 if self.in_repeat_ptr is not None:
                     s.in_repeat_ptr, s.in_repeat_events = _p(self.in_repeat_ptr), _p(self.in_repeat_events)
-        if self._pend_until <= self.step:
-            self._left_ring = None
+        if not self._pend_from <= self.step < self._pend_until:
+            # (all of it has arrived, or the caller began anew with an earlier step)
+            self._left_ring, self._pend_until = None, 0
         if self.fuse_table is not None:
             s.n_inputs = self.n_inputs if self.inp is not None else 0   # the history's layout, events or not
             s.fuse_indptr, s.fuse_packed = _p(self.fuse_table.indptr), _p(self.fuse_table.packed())
@@ -790,7 +797,7 @@ class Glif3Simulator:
             s.fuse_shift, s.fuse_wg_per_cu = self.fuse_shift, self.fuse_wg_per_cu
             s.fuse_max_team = max(1, -(-self.fuse_table.nnz // (256 * -(-self.n // (64 // self.batch)))))
             s.in_again = 1 if self.fuse_rereads and (self._lists_replaced or self._trials_left) else 0
-            if self._pend_until > self.step:
+            if self._left_ring is not None:
                 s.rb_ring, s.rb_pend_until = _p(self._left_ring), self._pend_until
                 self._in_use(self._left_ring)
             if self.in_repeat_ptr is not None:

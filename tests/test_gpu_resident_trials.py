@@ -109,6 +109,22 @@ def test_per_step_record_equals_the_launch_per_step_drivers(monkeypatch, n, batc
         assert torch.equal(x, y)
 
 
+@pytest.mark.parametrize("batch,fused", [(6, False), (12, True), (16, True)])
+def test_beginning_anew_leaves_nothing_under_way(batch, fused):
+    """State, ring, history and step set back after calls with resident trials: the run from rest once more, without the
+    arrivals that were under way."""
+    cfg, raster, st = _case(900, batch, 5, in_rate=150.0)
+    sim = _sim(cfg, batch, resident_trials=True, fused=fused)
+    rest = {k: getattr(sim.state, k).clone() for k in STATE}
+    sim.run(70)
+    for t in (sim.ring, sim.work_bits) + ((sim.fuse_any,) if fused else ()):
+        t.zero_()
+    for k in STATE:
+        getattr(sim.state, k).copy_(rest[k])
+    sim.step = 0
+    _same(sim, [sim.run(31), sim.run(119)], raster, st)
+
+
 def test_input_lists_replaced_between_calls():
     """Lists that say nothing was emitted in the steps behind take the last step's events back at the batches where the
     separate pull launches read them again (20), and leave them alone elsewhere (16)."""
@@ -127,6 +143,26 @@ def test_input_lists_replaced_between_calls():
         np.testing.assert_array_equal(results[0][0], results[1][0])
         for k in STATE:
             np.testing.assert_array_equal(results[0][1][k], results[1][1][k], err_msg=k)
+
+
+def test_replaced_lists_mean_what_they_mean_to_separate_pull_launches():
+    """At batches that do not divide 64 the fused form takes the place of separate pull launches, which read a call's first step
+    from the step before it once more: lists that no longer name that step's events take them back in either form."""
+    cfg, _, _ = _case(900, 20, 5, in_rate=150.0)
+    results = []
+    for kw in (dict(fused=False, pull=True, resident_trials=False), dict(fused=True), dict(fused=True, resident_trials=True)):
+        sim = _sim(cfg, 20, expected_rate_hz=40.0, **kw)
+        assert (sim.pull_inp_table is None) == kw["fused"] and sim.fuse_rereads
+        a = sim.run(60)
+        ptr = cfg["in_ptr"]
+        sim.set_input_events(np.concatenate([np.zeros(60, np.int64), ptr[60:] - ptr[60]]), cfg["in_events"][ptr[60]:])
+        b = sim.run(90)
+        sim.check()
+        results.append((torch.cat([a["bits"], b["bits"]]), sim.state.to_numpy()))
+    for bits, state in results[1:]:
+        assert torch.equal(bits, results[0][0])
+        for k in STATE:
+            np.testing.assert_array_equal(state[k], results[0][1][k], err_msg=k)
 
 
 @pytest.mark.parametrize("ends,kw", [
