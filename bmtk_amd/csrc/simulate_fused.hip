@@ -39,6 +39,7 @@
 // Any batch from 8 on: 20,011 x 20 trials, 16 M synapses: 36 us per step against 68 as separate pull and update launches.
 #include <math.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "common.hpp"
@@ -75,6 +76,7 @@ struct FusedLaunch {
     int shift;           // sources per bit of the activity map: 2^shift
     int team;            // wavefronts that share a group (1: every wavefront takes groups of its own from the workgroup's counter)
     int pending;         // bit 0 / 1: the resident form left arrivals of step t0-1 / t0 in rb_ring
+    int pend_slot[2];    // their slots of rb_ring
     int map_read, map_write;  // which of the two maps of bytes the launch reads and leaves behind (-1: none)
     double unit;         // of the fixed-point sums
 };
@@ -618,22 +620,17 @@ __global__ __launch_bounds__(kFuseBlock) void sim_fused_kernel(bmtk_glif3_sim s,
         float a0[GLIF3_NREC], a1[GLIF3_NREC];
         const FuseLaunchArgs qp = fresh_launch();
         if (qp->pending) {
-            // the first steps after a call in the resident form: what that call's spikes still send joins the sums, once (the
-            // launch may be replayed from a graph)
+            // the first steps after a call in the resident form: what that call's spikes still send joins the sums (and is cleared
+            // behind the launches, see clear_taken_kernel)
             const FuseArgs sp = fresh_args();
-            const int row = fin_grp * kRows + (int)sub_lane, slots = L - 1;
+            const int row = fin_grp * kRows + (int)sub_lane;
             if (in_group && row < n) {
-                uint64_t *left = in_memory(sp->rb_ring) + (int64_t)(lane - sub_bit) * slots * GLIF3_NREC * n + row;
-                auto take = [&](int64_t step, int r) {
-                    uint64_t *cell = left + ((int64_t)(step % slots) * GLIF3_NREC + r) * n;
-                    const unsigned long long v = *cell;
-                    *cell = 0ull;
-                    return v;
-                };
+                uint64_t *left = in_memory(sp->rb_ring) + (int64_t)(lane - sub_bit) * (L - 1) * GLIF3_NREC * n + row;
+                // (a cell at a time: 16 of them at once spill registers that every turn of a launch without any needs)
 #pragma unroll
                 for (int r = 0; r < GLIF3_NREC; ++r) {
-                    if (qp->pending & 1) acc[r * kWave + lane] += take(qp->t0 - 1, r);
-                    if (qp->pending & 2) acc[(GLIF3_NREC + r) * kWave + lane] += take(qp->t0, r);
+                    if (qp->pending & 1) acc[r * kWave + lane] += left[(int64_t)(qp->pend_slot[0] * GLIF3_NREC + r) * n];
+                    if (qp->pending & 2) acc[(GLIF3_NREC + r) * kWave + lane] += left[(int64_t)(qp->pend_slot[1] * GLIF3_NREC + r) * n];
                 }
             }
         }
@@ -779,6 +776,19 @@ __global__ __launch_bounds__(kBlock) void zero_bits_kernel(uint64_t *__restrict_
     for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlock) bits[i] = 0ull;
 }
 
+// What a call took from rb_ring, [trial][slot][receptor][neuron], cleared behind its launches: `count` slots from `slot0` on.  A
+// call that is captured into a graph thereby takes it over in the first replay only.  (Cleared by the launches themselves,
+// each cell as it was read, it cost all of them two spilled registers and 12 bytes of scratch: 1 % of a training step of
+// 3,001 neurons x 12 trials, which never leaves anything there.)
+__global__ __launch_bounds__(kBlock) void clear_taken_kernel(uint64_t *__restrict__ ring, int64_t words, int slot_words, int slots, int slot0, int count)
+{
+    for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < words; i += (int64_t)gridDim.x * kBlock) {
+        const int64_t row = i / slot_words, trial = row / count;
+        const int slot = (slot0 + (int)(row - trial * count)) % slots;
+        ring[(trial * slots + slot) * slot_words + (i - row * slot_words)] = 0ull;
+    }
+}
+
 int simulate_fused(const bmtk_glif3_sim &s, int64_t step0, int64_t n_steps, hipStream_t stream)
 {
     const int batch = s.batch, L = s.ring_slots;
@@ -886,6 +896,7 @@ int simulate_fused(const bmtk_glif3_sim &s, int64_t step0, int64_t n_steps, hipS
         q.in_bits = (has_inp && !closing && n_in_words > 0) ? 1 : 0;
         q.repeats = (s.in_repeat_ptr && !closing) ? 1 : 0;
         q.pending = (q.fold0 && q.t0 - 1 < s.rb_pend_until ? 1 : 0) | (q.n_sub == 2 && q.t0 < s.rb_pend_until ? 2 : 0);
+        for (int i = 0; i < 2; ++i) q.pend_slot[i] = (int)((q.t0 + (L - 1) + i - 1) % (L - 1));
         q.map_read = map;
         q.map_write = bytes && (!closing || map == 1) ? 1 - map : -1;
         if (q.map_write >= 0) map = q.map_write;
@@ -900,6 +911,15 @@ int simulate_fused(const bmtk_glif3_sim &s, int64_t step0, int64_t n_steps, hipS
             return BMTK_E_LAUNCH;
         }
     }
+    if (n_steps > 0 && step0 < s.rb_pend_until) {
+        const int64_t left = s.rb_pend_until - step0;
+        const int slots = L - 1, slot_words = GLIF3_NREC * (int)s.n_neurons;
+        const int count = (int)std::min<int64_t>(std::min<int64_t>(n_steps, left), slots);
+        const int64_t words = (int64_t)batch * count * slot_words, blocks = (words + kBlock - 1) / kBlock;
+        hipLaunchKernelGGL(clear_taken_kernel, dim3((unsigned)std::min<int64_t>(blocks, 4096)), dim3(kBlock), 0, stream, s.rb_ring, words, slot_words,
+                           slots, (int)(step0 % slots), count);
+    }
+    BMTK_CHECK_LAUNCH("glif3_simulate_fwd");
     return BMTK_OK;
 }
 
