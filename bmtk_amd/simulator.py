@@ -114,24 +114,32 @@ def fixed_point_shift(tables, n_neurons):
     one of them exactly, so that no sum has fewer bits than one in fp32: 0 where each weight is a whole multiple of 2^-32 (any
     fp32 number from 2^-9 on is).  None where they do not fit: what could reach a neuron in a step, scaled, has to stay below
     2^30 (a factor of two for ids repeated within a step), and weights have to be finite."""
-    lowest, most = 0, 0.0
+    tables = [t for t in tables if t.nnz]
+    lowest, sizes = 0, []
     for t in tables:
-        if not t.nnz:
-            continue
-        largest = float(t.weights.abs().max())      # (a NaN carries over)
+        size = t.weights.abs()
+        least, largest = torch.stack(torch.aminmax(size)).tolist()      # (a NaN carries over)
         if not math.isfinite(largest):
             return None
-        most += largest * int(torch.bincount(t.indices, minlength=n_neurons).max())
-        for w in t.weights.split(1 << 26):
+        sizes.append(largest)
+        # (from 2^-9 on every number's bits lie above 2^-33)
+        for w in size.split(1 << 26) if least < 2.0 ** -9 else ():
             # the power of two that a weight's lowest set bit stands for
             bits = w.contiguous().view(torch.int32)
-            exponent, mantissa = (bits >> 23) & 0xFF, bits & 0x7FFFFF
+            exponent, mantissa = bits >> 23, bits & 0x7FFFFF
             mantissa = torch.where(exponent > 0, mantissa | 0x800000, mantissa)
             low_bit = ((mantissa & -mantissa).to(torch.float32).view(torch.int32) >> 23) - 127
             place = torch.where(mantissa != 0, exponent.clamp(min=1) - 150 + low_bit, torch.zeros_like(low_bit))
             lowest = min(lowest, int(place.min()))
     shift = max(0, -32 - lowest)
-    return shift if shift <= SUM_SHIFT_MAX and most * 2.0 ** shift < 2.0 ** 30 else None
+    if shift > SUM_SHIFT_MAX:
+        return None
+    limit = 2.0 ** (30 - shift)
+    # (all synapses on one neuron; only where that is too much, the synapses of the neuron that has most)
+    if (sum(size * t.nnz for size, t in zip(sizes, tables)) >= limit
+            and sum(size * int(torch.bincount(t.indices, minlength=n_neurons).max()) for size, t in zip(sizes, tables)) >= limit):
+        return None
+    return shift
 
 
 def fused_pays(n_neurons, batch, n_synapses, class_table, rate_hz, h_ms=1.0):
