@@ -388,8 +388,8 @@ def bench_batched_v1(torch, batch=8, steps=300):
     inp = synthetic.device_input_table(N_IN, N_V1, N_IN_SYN, seed=4, w_scale=IN_W_SCALE)
     in_ptr, in_ev = ops.poisson_events(N_IN, IN_RATE_HZ, 1.0, 600 + 2 * steps, batch=batch, seed=5)
     out = []
-    for form, kw in (("the simulator's choice", dict()), ("fused pull form", dict(fused=True))):
-        sim = Glif3Simulator(N_V1, par, 1.0, batch=batch, class_id=class_id, rec=by_src, inp=inp, resident=False, **kw)
+    for form, kw in (("the simulator's choice", dict()), ("fused pull form", dict(fused=True, resident=False))):
+        sim = Glif3Simulator(N_V1, par, 1.0, batch=batch, class_id=class_id, rec=by_src, inp=inp, **kw)
         sim.set_input_events(in_ptr, in_ev)
         sim.run(600, spike_bits=False)
         sim.run(steps // 4, spike_bits=False)
