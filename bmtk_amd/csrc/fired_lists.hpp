@@ -1,0 +1,128 @@
+// How the workgroups of a resident run tell one another which neurons fired: lists whose words say themselves which step
+// they belong to.
+//
+// A list is eight 64-bit words per workgroup and step.  Every word carries a tag of its step in its upper nine bits, is
+// stored with ONE agent-scope store and read with agent-scope loads: a reader that finds the tag it wants has the word,
+// one that does not asks again.  Nothing has to be ordered between two words, so the writer waits for no acknowledgement
+// and signals no counter, and a step needs no grid barrier: whoever has read the lists of step t of all workgroups knows
+// that all have finished step t.  (With ballots and arrival counters three trips to memory followed one another -- the
+// stores' acknowledgement, the arrivals, the look at the counters -- before the ballots could be asked for.)
+//
+//   word 0       tag | number that fired (11 bits) | 4 neurons (11 bits each, counted within the workgroup's span)
+//   words 1..7   tag | 5 neurons
+//
+// A step in which more than 39 neurons of a workgroup fired says so in the number (kListMany): its ballots are read then,
+// which the writer has waited for before it published the word.  All eight words are written in every step: the word a
+// reader meets in place of the one it wants is then that row's last user's, `rows` steps ago, and nothing older, which
+// is what makes eight bits of step number enough.  The rows are cleared before a launch, and a tag is never zero.
+#pragma once
+
+#include "common.hpp"
+
+namespace bmtk {
+
+constexpr int kListWords = BMTK_RES_FIRED_SLOTS / 2;
+constexpr int kListQuickWords = 2;          // these of all workgroups side by side: what a reader asks for first
+constexpr unsigned kListQuick = 9, kListHalf = 19, kListMax = 39;  // neurons in words 0..1, 0..3, 0..7
+constexpr unsigned kListMany = 2047;        // in place of the number: more than kListMax, see the ballots
+constexpr int kListRounds = 4;              // workgroups a lane of the reading wavefront looks after
+constexpr int kListGroups = kListRounds * kWave;
+constexpr int kListIdBits = 11, kListCountAt = 44, kListTagAt = 55;
+static_assert(kListWords == 8 && kListCountAt == 4 * kListIdBits && kListTagAt == 5 * kListIdBits, "list layout");
+
+__device__ __forceinline__ unsigned list_tag(int k) { return 256u | ((unsigned)k & 255u); }
+
+__device__ __forceinline__ unsigned long long load_agent64(const unsigned long long *p)
+{
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// The lists of one step: words 0 and 1 of every list, then words 2..7 of every list (a writer's stores and a reader's loads meet
+// as few lines as that allows).
+constexpr int kListRows = 4;   // lists of so many steps are kept
+constexpr int kListRowWords = kListWords * kListGroups;
+struct ListRow {
+    unsigned long long *w;
+    __device__ __forceinline__ unsigned long long *at(int g, int j) const
+    {
+        return w + (j < kListQuickWords ? kListQuickWords * g + j
+                                        : kListQuickWords * kListGroups + (kListWords - kListQuickWords) * g + j - kListQuickWords);
+    }
+};
+
+// The lane's number, worked out where it is used: addresses and products of it, hoisted out of a loop over the steps, would
+// push a neuron's state out of the registers.
+__device__ __forceinline__ int lane_here()
+{
+    int l = lane_id();
+    asm volatile("" : "+v"(l));
+    return l;
+}
+
+// One wavefront: the list of workgroup g, of n neurons that stand in fired_l.  In two parts, so that its reads of LDS go out
+// beside others of the caller.
+struct ListWrite {
+    unsigned first, id[5];
+
+    __device__ __forceinline__ void read(const unsigned short *fired_l)
+    {
+        const unsigned j = (unsigned)lane_here() & (kListWords - 1u);
+        first = max(5u * j, 1u) - 1u;  // (39 entries are looked at, whatever their number)
+#pragma unroll
+        for (unsigned i = 0; i < 5u; ++i) id[i] = fired_l[first + i];
+    }
+    __device__ __forceinline__ void publish(const ListRow &row, int g, unsigned tag, unsigned n) const
+    {
+        const int j = lane_here();
+        unsigned long long word = (unsigned long long)tag << kListTagAt;
+#pragma unroll
+        for (unsigned i = 0; i < 4u; ++i) word |= (unsigned long long)(first + i < n ? id[i] : 0u) << (kListIdBits * i);
+        // (word 0: the number stands where the others have their fifth neuron)
+        const unsigned fifth = first + 4u < n ? id[4] : 0u;
+        word |= (unsigned long long)(j > 0 ? fifth : n > kListMax ? kListMany : n) << kListCountAt;
+        if (j < kListWords) __hip_atomic_store(row.at(g, j), word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+};
+// What the reading wavefront holds of a step's lists: words 0 and 1, lane l those of workgroups l, l + 64, ..
+struct ListLook {
+    unsigned long long v[kListRounds][kListQuickWords];
+
+    __device__ __forceinline__ void none()
+    {
+#pragma unroll
+        for (int u = 0; u < kListRounds; ++u) v[u][0] = v[u][1] = 0ull;
+    }
+    // asks once for words `from`, `from` + 1 of all G lists; true when every workgroup has published them in the wanted step
+    __device__ __forceinline__ bool look(const ListRow &row, int G, unsigned tag, int from = 0)
+    {
+        const unsigned lane = (unsigned)lane_here();
+        const char *base = reinterpret_cast<const char *>(row.at(0, from));
+        const unsigned stride = 8u * (from ? kListWords - kListQuickWords : kListQuickWords);
+#pragma unroll
+        for (int u = 0; u < kListRounds; ++u) {
+            const unsigned long long *p = reinterpret_cast<const unsigned long long *>(base + min(u * kWave + lane, (unsigned)G - 1u) * stride);
+            v[u][0] = load_agent64(p);
+            v[u][1] = load_agent64(p + 1);
+        }
+        unsigned differs = 0u;
+#pragma unroll
+        for (int u = 0; u < kListRounds; ++u)
+            differs |= ((unsigned)(v[u][0] >> 32) ^ (tag << (kListTagAt - 32))) | ((unsigned)(v[u][1] >> 32) ^ (tag << (kListTagAt - 32)));
+        return __ballot((differs >> (kListTagAt - 32)) != 0u) == 0ull;
+    }
+    __device__ __forceinline__ unsigned count(int u, int G) const
+    {
+        return u * kWave + lane_id() < G ? (unsigned)(v[u][0] >> kListCountAt) & kListMany : 0u;
+    }
+};
+
+// the i-th neuron of a word
+__device__ __forceinline__ unsigned list_id(unsigned long long word, int i)
+{
+    const unsigned lo = (unsigned)word, hi = (unsigned)(word >> 32);
+    const int at = kListIdBits * i;
+    const unsigned bits = at + kListIdBits <= 32 ? lo >> at : at >= 32 ? hi >> (at - 32) : __builtin_amdgcn_alignbit(hi, lo, at);
+    return bits & ((1u << kListIdBits) - 1u);
+}
+
+}  // namespace bmtk

@@ -19,14 +19,9 @@
 // Nothing but spike ballots, segment offsets and the synapses actually used
 // crosses the memory system: no global atomics, no state traffic.
 //
-// Without slack (see below) a workgroup publishes, beside its ballots, the
-// neurons that fired as a list of 16 places (res_fired: filled in LDS with one
-// LDS atomic per spiking lane, written out by one wavefront once the workgroup
-// has met after the update), and step 2 reads the lists -- four places per
-// thread -- instead of taking the ballots of the whole network apart bit by
-// bit, which every workgroup would do for itself; a step in which some list
-// did not suffice is read from the ballots.  The same count gives a spike its
-// place in the spike record when the workgroup has a record list of its own.
+// That is the form for runs with slack (below), and without where the caller does
+// not ask for lists.  Without slack the workgroups exchange lists of fired neurons
+// and meet at no grid barrier: sim_resident_lists_kernel, further down.
 //
 // Ballots live in a history of D rows, row t%D for step t.  With D = 3 a
 // workgroup waits for the barrier of step t at the end of step t: row t%3 is
@@ -57,6 +52,7 @@
 // grid always drains.
 #include <stdlib.h>
 
+#include "fired_lists.hpp"
 #include "glif3_update.hpp"
 #include "sim_internal.hpp"
 
@@ -107,7 +103,7 @@ __device__ __forceinline__ unsigned load_agent(const unsigned *p)
 // fence of workgroup scope does NOT do this: on this target it waits for LDS and scalar operations only, because
 // the wavefronts of a workgroup share one vector cache.
 //
-// THE GRID BARRIER'S CONTRACT.  Four kinds of words in device memory are written by one workgroup and read by
+// THE GRID BARRIER'S CONTRACT.  Three kinds of words in device memory are written by one workgroup and read by
 // others during a launch; every such access is a relaxed atomic of AGENT scope (it passes the compute unit's
 // vector cache and the XCD's L2 and is served where all XCDs see the same value), and the order between them is
 // made by hand, because HIP's memory model offers no fence of the needed kind that does not also invalidate the
@@ -115,8 +111,6 @@ __device__ __forceinline__ unsigned load_agent(const unsigned *p)
 //   work_bits   (ballots)   written by: lane 0 of every wavefront that owns elements, right after its update of
 //                           step t (row t % hist).  Read by: every workgroup's pull of step t, after it has seen
 //                           the barrier of step t complete.
-//   res_fired   (lists)     written by: the first 16 threads of a workgroup after the workgroup has met (row t %
-//                           hist, the workgroup's 16 places).  Read by: every workgroup's pull of step t, as above.
 //   arrival counters        written by: thread 0 of a workgroup, one increment per step, on the counter of (step,
 //                           the workgroup's XCD), AFTER every wavefront of the workgroup has executed
 //                           wait_vector_memory() and the workgroup has passed __syncthreads().  Read by: one look
@@ -124,9 +118,9 @@ __device__ __forceinline__ unsigned load_agent(const unsigned *p)
 //                           bounded spin.
 //   abort word              written by: any workgroup whose spin ran out.  Read by: every workgroup inside its spin
 //                           and at the start of a launch.  Sticky: only the host clears it.
-// The one ordering that makes the barrier a barrier: a workgroup's ballot and list stores of step t are
+// The one ordering that makes the barrier a barrier: a workgroup's ballot stores of step t are
 // ACKNOWLEDGED (wait_vector_memory in every wavefront that stored, then the workgroup barrier) before its arrival
-// for step t is sent.  A reader that has counted all arrivals of step t therefore loads ballots and lists that
+// for step t is sent.  A reader that has counted all arrivals of step t therefore loads ballots that
 // are already where agent-scope loads look.  Nothing else is assumed: readers do not rely on the order of two
 // stores of another workgroup, and no acquire fence runs inside the loop (every read of another workgroup's words
 // is an agent-scope load, which is not served from a copy that an earlier read left in the compute unit's cache).
@@ -135,8 +129,8 @@ __device__ __forceinline__ unsigned load_agent(const unsigned *p)
 // workgroups for many steps against a driver without this barrier would differ in single synaptic segments --
 // tests/test_gpu_simulate.py::test_v1_scale_resident_equals_per_step_launches and
 // ::test_lists_of_fired_neurons_equal_the_ballots, tests/test_gpu_random_networks.py::
-// test_many_workgroups_with_volleys_and_delay_offsets, tests/test_gpu_fullsize.py::
-// test_v1_scale_forward_run_against_both_oracles.
+// test_many_workgroups_with_volleys_and_delay_offsets.
+// (The lists of sim_resident_lists_kernel need none of this: every word of theirs carries its step.)
 __device__ __forceinline__ void wait_vector_memory()
 {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -152,13 +146,17 @@ struct __attribute__((packed, aligned(4))) SegBounds {
     uint32_t lo, hi;
 };
 
-__device__ __forceinline__ void pull_segment(const uint32_t *__restrict__ seg_row, int g,
-                                             const bmtk_synapse *__restrict__ tab, float *ring_l, int span, int e0,
-                                             int L, int slot0)
-{
-    const SegBounds sb = *reinterpret_cast<const SegBounds *>(seg_row + g);
-    const uint32_t len = sb.hi - sb.lo;  // the offsets never decrease
-    const uint2 *__restrict__ rows = reinterpret_cast<const uint2 *>(tab) + sb.lo;
+struct RingSlice {
+    float *origin;     // the slice's origin less e0
+    unsigned span_v;   // in a vector register once, not before every multiply
+    unsigned q_lo, q_wrap;
+
+    // additions to the slots behind slot0
+    __device__ __forceinline__ RingSlice(float *ring_l, int span, int e0, int L, int slot0)
+        : origin(ring_l - e0), q_lo((unsigned)slot0 * 4u), q_wrap((unsigned)slot0 * 4u - 4u * (unsigned)L)
+    {
+        asm("v_mov_b32 %0, %1" : "=v"(span_v) : "s"(span));
+    }
     // An LDS float atomic costs about three clocks per LANE on gfx950 (its lanes are worked off one after the
     // other), an integer compare-and-swap a few clocks per INSTRUCTION.  Where most lanes of a wavefront take
     // part -- the first synapse of the segments -- the addition is therefore a compare-and-swap loop (a
@@ -170,11 +168,8 @@ __device__ __forceinline__ void pull_segment(const uint32_t *__restrict__ seg_ro
     // wavefront instruction for a handful of lanes): the cell's address takes six instructions -- two byte adds, min,
     // mask, one 24-bit multiply-add, one shift-add onto the slice's origin less e0 -- and a synapse's load a compare
     // against the segment's length and an immediate offset.
-    const unsigned q_lo = (unsigned)slot0 * 4u, q_wrap = q_lo - 4u * (unsigned)L;
-    float *origin = ring_l - e0;
-    unsigned span_v;  // in a vector register once, not before every multiply
-    asm("v_mov_b32 %0, %1" : "=v"(span_v) : "s"(span));
-    auto add = [&](const uint2 sy, bool crowded) {
+    __device__ __forceinline__ void add(const uint2 sy, bool crowded) const
+    {
         const unsigned dq = sy.x >> 24;
         const unsigned plane = min(dq + q_lo, dq + q_wrap);
         float *cell = origin + mad_u24(plane, span_v, sy.x & 0xFFFFFFu);
@@ -190,19 +185,34 @@ __device__ __forceinline__ void pull_segment(const uint32_t *__restrict__ seg_ro
             if (seen == old) break;
             old = seen;
         }
-    };
+    }
+};
+
+__device__ __forceinline__ void pull_bounds(uint32_t lo, uint32_t len, uint32_t part, uint32_t team,
+                                            const bmtk_synapse *__restrict__ tab, const RingSlice &ring)
+{
+    const uint2 *__restrict__ rows = reinterpret_cast<const uint2 *>(tab) + lo;
     // all of a segment's loads go out together: a loop of dependent loads for the few long segments would
     // hold up the whole wavefront (1 in 25 segments has more than 3 synapses, 1 in 5000 more than 6); measured at V1
     // scale: four together and the compare-and-swap for the first only, 5.35 us per step; six and two, 5.43
     constexpr int kTogether = 4;
-    uint2 first[kTogether];
+    for (uint32_t q = part; q < len; q += kTogether * team) {
+        uint2 sy[kTogether];
 #pragma unroll
-    for (int u = 0; u < kTogether; ++u)
-        if ((uint32_t)u < len) first[u] = rows[u];
+        for (int u = 0; u < kTogether; ++u)
+            if (q + u * team < len) sy[u] = rows[q + u * team];
 #pragma unroll
-    for (int u = 0; u < kTogether; ++u)
-        if ((uint32_t)u < len) add(first[u], u < 1);
-    for (uint32_t q = (uint32_t)kTogether; q < len; ++q) add(rows[q], false);
+        for (int u = 0; u < kTogether; ++u)
+            if (q + u * team < len) ring.add(sy[u], u < 1);
+    }
+}
+
+__device__ __forceinline__ void pull_segment(const uint32_t *__restrict__ seg_row, int g,
+                                             const bmtk_synapse *__restrict__ tab, float *ring_l, int span, int e0,
+                                             int L, int slot0)
+{
+    const SegBounds sb = *reinterpret_cast<const SegBounds *>(seg_row + g);
+    pull_bounds(sb.lo, sb.hi - sb.lo, 0u, 1u, tab, RingSlice(ring_l, span, e0, L, slot0));  // the offsets never decrease
 }
 
 constexpr int kScanWords = 4;   // ballot words per thread and round
@@ -222,11 +232,7 @@ constexpr unsigned kInputTag = 0x80000000u;
 // Returns true when the bump has been made.
 // kUnified: the input rows follow the recurrent rows in ONE table (inp_seg = rec_seg + n_neurons*(n_groups+1), both
 // sets of offsets index rec_packed), so a listed row needs no choice between two tables.
-// kLists: the workgroups publish the neurons that fired as short lists (res_fired) and a step is read from those
-// when every list sufficed: two 8-byte loads per thread bring four places of the lists, the occupied ones go
-// straight to the row list -- no ballot words to take apart bit by bit, which is the larger part of the
-// instructions a quiet step costs.
-template <bool kUnified, bool kLists>
+template <bool kUnified>
 __device__ __forceinline__ bool pull_step(const bmtk_glif3_sim &s, const Resident &r, int g, int hist_row, int slot0,
                                           float *ring_l, unsigned *act, unsigned *scan_l, int e0, int words,
                                           int64_t k0, int64_t k1, unsigned *arrival = nullptr)
@@ -253,57 +259,6 @@ __device__ __forceinline__ bool pull_step(const bmtk_glif3_sim &s, const Residen
             }
         }
     };
-    bool arrived_above = false;
-    if (kLists && s.res_fired && k1 - k0 <= kResBlock) {
-        PROF_T(p0);
-        constexpr unsigned kManyFlag = 1u << 20;  // in a count: some list did not suffice (1024 of them still fit 32 bits)
-        static_assert(kManyFlag > (unsigned)kActCap && 5 * kResBlock <= kActCap, "a step read from the lists always fits the row list");
-        const unsigned long long *lists = reinterpret_cast<const unsigned long long *>(
-            s.res_fired + (int64_t)hist_row * r.n_groups * BMTK_RES_FIRED_SLOTS);
-        unsigned long long w0 = 0ull, w1 = 0ull;  // four places: kResBlock threads cover 256 workgroups' lists
-        if (has_rec && tid < r.n_groups * (BMTK_RES_FIRED_SLOTS / 4)) {
-            w0 = __hip_atomic_load(lists + 2 * tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            w1 = __hip_atomic_load(lists + 2 * tid + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-        const int64_t ke = k0 + tid;
-        const bool has_event = ke < k1;
-        const unsigned event_row = has_event ? (unsigned)s.in_events[ke] : 0u;
-        const unsigned id[4] = {(unsigned)w0, (unsigned)(w0 >> 32), (unsigned)w1, (unsigned)(w1 >> 32)};
-        unsigned cnt = has_event ? 1u : 0u;
-#pragma unroll
-        for (int u = 0; u < 4; ++u) cnt += id[u] != 0u ? 1u : 0u;
-        if (id[0] == BMTK_RES_FIRED_MANY) cnt = kManyFlag;  // such a list is marked in every place
-        const unsigned inc = wave_inclusive_scan(cnt);
-        if (lane_id() == kWave - 1) scan_l[wave] = inc;
-        if (arrival) wait_vector_memory();  // the loads are back already; this is for the stores of the update
-        __syncthreads();
-        if (arrival && tid == 0) __hip_atomic_fetch_add(arrival, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        PROF_T(p1);
-        const unsigned part = wave_inclusive_scan(lane_id() < kResBlock / kWave ? scan_l[lane_id()] : 0u);
-        const unsigned total = (unsigned)bcast_i((int)part, kResBlock / kWave - 1);
-        const unsigned base = wave > 0 ? (unsigned)__shfl((int)part, wave - 1, kWave) : 0u;
-        if (total <= (unsigned)kActCap) {  // workgroup-uniform: every list sufficed, and the row list holds them
-            unsigned pos = base + inc - cnt;
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-                if (id[u] != 0u) act[pos++] = id[u] - 1u;
-            if (has_event) act[pos] = kUnified ? event_row + (unsigned)s.n_neurons : event_row | kInputTag;
-            __syncthreads();
-            PROF_T(p2);
-            pull_listed(total);
-            __syncthreads();
-            PROF_T(p3);
-            PROF_ADD(4, p0, p1);
-            PROF_ADD(5, p1, p2);
-            PROF_ADD(6, p2, p3);
-            PROF_BLK(3, p2, p3);
-            return arrival != nullptr;
-        }
-        // this step from the ballots (the arrival has been made)
-        __syncthreads();  // scan_l is written again below
-        arrived_above = arrival != nullptr;
-        arrival = nullptr;
-    }
     const unsigned long long *bits =
         reinterpret_cast<const unsigned long long *>(s.work_bits) + (int64_t)hist_row * (words + 1);
     // 32-bit counters wherever the sizes allow: the loop is short of scalar registers
@@ -390,7 +345,7 @@ __device__ __forceinline__ bool pull_step(const bmtk_glif3_sim &s, const Residen
         PROF_ADD(6, p2, p3);
         PROF_BLK(3, p2, p3);
     }
-    return arrived_above || (arrival != nullptr && rounds > 0);
+    return arrival != nullptr && rounds > 0;
 }
 
 // kLate: the run has slack (S > 0), see the loop body.  kForm: what the launch asks for beyond the simulation
@@ -405,7 +360,6 @@ template <bool kLate, int kForm>
 __global__ __launch_bounds__(kResBlock) void sim_resident_kernel(bmtk_glif3_sim s, Resident r)
 {
     constexpr bool kUnifiedTables = kForm != kFormAny;
-    constexpr bool kLists = !kLate;  // lists of fired neurons beside the ballots (res_fired), see pull_step
     if (kForm != kFormAny) {
         s.probe_col = nullptr;
         s.inp_seg = nullptr;
@@ -415,7 +369,6 @@ __global__ __launch_bounds__(kResBlock) void sim_resident_kernel(bmtk_glif3_sim 
     extern __shared__ float ring_l[];  // [L*4][span], then the active-row list
     __shared__ int go_on;
     __shared__ unsigned scan_l[kResBlock / kWave];
-    __shared__ unsigned fired_l[BMTK_RES_FIRED_SLOTS];  // this workgroup's list of the step: neuron + 1
     __shared__ unsigned fired_n[2];  // how many fired in this step and the one before
     const int tid = threadIdx.x;
     const int lane = lane_id();
@@ -477,7 +430,7 @@ __global__ __launch_bounds__(kResBlock) void sim_resident_kernel(bmtk_glif3_sim 
     // waits for an atomic on device memory, which the arrivals of a step would queue up behind.
     const bool own_record = !kLate && s.spike_count != nullptr && rec_ways >= gridDim.x;
     unsigned long long rec_count = own_record ? s.spike_count[rec_way * BMTK_RECORD_COUNT_STRIDE] : 0ull;
-    const bool count_fired = own_record || (kLists && s.res_fired != nullptr);
+    const bool count_fired = own_record;
     // the input events of the step pulled in step t, u = t-1-B, are in_events[ka, kb); the bound for the
     // next step is fetched a step ahead.  Steps before 0 have no events (in_ptr[0] = 0).
     const int B = r.offset;
@@ -589,7 +542,6 @@ __global__ __launch_bounds__(kResBlock) void sim_resident_kernel(bmtk_glif3_sim 
         // barrier).
         if (count_fired && m != 0ull && spike) {
             const unsigned at = atomicAdd(&fired_n[k & 1], 1u);
-            if (kLists && s.res_fired && at < BMTK_RES_FIRED_SLOTS) fired_l[at] = (unsigned)e + 1u;
             if (own_record && rec_count + at < rec_cap) {
                 const unsigned long long idx = rec_way * rec_cap + rec_count + at;
                 s.spike_step[idx] = (int32_t)t;
@@ -624,12 +576,6 @@ __global__ __launch_bounds__(kResBlock) void sim_resident_kernel(bmtk_glif3_sim 
             // the list of this step, complete since the workgroup met: out with it, like the ballots (the arrival
             // waits for the store), and the count back to zero (it is added to again after the barriers of the pull)
             if (own_record) rec_count += fired_n[k & 1];
-            if (kLists && s.res_fired && tid < BMTK_RES_FIRED_SLOTS && g < r.n_groups) {  // (the grid is rounded up)
-                const unsigned n = fired_n[k & 1];
-                const unsigned word = n > BMTK_RES_FIRED_SLOTS ? BMTK_RES_FIRED_MANY : ((unsigned)tid < n ? fired_l[tid] : 0u);
-                __hip_atomic_store(s.res_fired + ((int64_t)row_t * r.n_groups + g) * BMTK_RES_FIRED_SLOTS + tid, word,
-                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            }
             // the other count, last read a barrier ago and next added to a barrier on, back to zero
             if (count_fired && tid == 0) fired_n[(k + 1) & 1] = 0u;
         }
@@ -646,7 +592,7 @@ __global__ __launch_bounds__(kResBlock) void sim_resident_kernel(bmtk_glif3_sim 
         //    inside the loop is read by another workgroup before the kernel ends.
         bool arrived = false;
         if (k > 0 && t - 1 - B >= 0 && mine > 0)
-            arrived = pull_step<kUnifiedTables, kLists>(s, r, g, row_p, slot_prev, ring_l, act, scan_l, e0, words, ka, kb,
+            arrived = pull_step<kUnifiedTables>(s, r, g, row_p, slot_prev, ring_l, act, scan_l, e0, words, ka, kb,
                                                late ? nullptr : my_counter);
         if (!late && !arrived) {
             wait_vector_memory();
@@ -702,7 +648,7 @@ __global__ __launch_bounds__(kResBlock) void sim_resident_kernel(bmtk_glif3_sim 
         // closing: spikes and inputs of the last step (less the delay offset), then fold the last slot
         const int64_t tl = r.step0 + done - 1;
         if (tl - B >= 0 && mine > 0)
-            pull_step<kUnifiedTables, kLists>(s, r, g, wrap(tl - B, r.hist), wrap(tl, L), ring_l, act, scan_l, e0, words, ka,
+            pull_step<kUnifiedTables>(s, r, g, wrap(tl - B, r.hist), wrap(tl, L), ring_l, act, scan_l, e0, words, ka,
                                               kb);
         __syncthreads();
         if (own) {
@@ -724,9 +670,523 @@ __global__ __launch_bounds__(kResBlock) void sim_resident_kernel(bmtk_glif3_sim 
     }
 }
 
-__global__ void zero_words_kernel(unsigned *w, int n)
+// The form without slack (delay offset 0), several workgroups.  What sets its pace is a chain through memory: a spike of
+// step t has to be in every workgroup's ring slice before the update of step t+2.  Here little but that chain is left of
+// the exchange.  The neurons that fired travel in lists that carry their step (fired_lists.hpp): no acknowledgement, no
+// arrival, no barrier over the grid.  And the wavefronts divide the memory traffic, because a wavefront's accesses complete
+// in the order issued (one that waits for a load waits for its stores before it, and a store is acknowledged after a trip
+// to the far side of the L2):
+//   reader (the last)       asks for the lists of step t until every workgroup's are there and puts the rows that fired, and
+//                           those of the step's input events, into one list in LDS.  Stores nothing.
+//   writer (last but one)   stores what the workgroup leaves in LDS: its list first, ballots, the spike record.  Pulls
+//                           nothing.
+//   the others              pull: a thread takes a row, reads the bounds of this workgroup's segment of it and adds the
+//                           segment's synapses to the ring slice.
+// All but the reader (the reader too at spans above 960) own neurons and update them.  A round k of the loop:
+//     fold slot k-1, update; who fired -> LDS; writer: list of step k   (reader: lists of step k-1 -> rows)
+//   --------------------------------- the workgroup meets --------------------------------------------------
+//     pull step k-1                                                     (reader: on to the lists of step k)
+//   ------------------ all but the reader wait for one another's pulls (a count in LDS) --------------------
+// A workgroup that publishes step t has seen everybody's step t-2, so four rows of lists are enough.
+//
+// The reader waits half a thousand clocks before its first look: lists looked at while they are being written cost the
+// writers' stores, and the pulls, more than the look brings (120,000 neurons: 4.2 us per step looking at once, 3.9 so).
+// A look then finds all lists there nearly always.
+//
+// A row's segment is read by a team of neighbouring lanes, as many as a segment holds synapses on average, rounded up, if
+// the step has threads for it (a small network has few rows a step and long segments).
+//
+// Steps in which a list does not hold its neurons, or the rows have no room, are crowded: all sixteen wavefronts read
+// the lists (or ballots) and work the rows off.
+//
+// Measured per step, ballots or lists behind a grid barrier -> this: 10,007 neurons of in-degree 600 3.27 -> 2.16 us; 60,000 of
+// 660 4.15 -> 2.88; 120,000 of 440 4.63 -> 3.92; the V1 network's 230,924 of 335 5.46 -> 4.96.  What it spends there: update
+// 0.5, list out 0.5, pull 2.5 (two dependent trips to memory for 700 rows), and 1.1 until the slowest wavefront has pulled.
+// Bounds and first synapses of a segment in one 16-byte cell (a gigabyte): 4.89 us at V1, slower elsewhere, dropped; flags in
+// LDS in place of the meeting, so that the list need not be out before the pull begins: 5.4 us, the pulls and the reader
+// then share the way to memory; another order of rows for each workgroup of an XCD: no difference.
+constexpr int kReader = kResBlock / kWave - 1, kWriter = kReader - 1;
+constexpr int kPullThreads = kWriter * kWave;
+static_assert((kWays * kBarrierWords) * kBarrierStride * 4 >= kListRows * kListRowWords * 8, "res_sync holds the lists");
+constexpr unsigned kCrowded = 0xFFFFFFFFu;
+constexpr int kReaderEvents = 4;    // input events a lane of the reader asks for ahead
+// the room of the row list (kActCap words) divided up: rows of two steps, a place per lane of the reader for what is none, the
+// neurons of this workgroup that fired and, for a record, their crossing fractions
+constexpr unsigned row_cap(bool record)
 {
-    if ((int)threadIdx.x < n) w[threadIdx.x] = 0u;
+    return (unsigned)((kActCap * 4 - 2 * kResBlock - (record ? 4 * kResBlock : 0) - 4 * kWave) / 8);
+}
+
+// Words of LDS that wavefronts of the workgroup tell one another how far they are by.  A wavefront's accesses to LDS are worked
+// off in the order it issues them; only the compiler has to be kept from another order.
+__device__ __forceinline__ unsigned load_lds(unsigned *p)
+{
+    const unsigned v = __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    asm volatile("" ::: "memory");
+    return v;
+}
+__device__ __forceinline__ void store_lds(unsigned *p, unsigned v)
+{
+    asm volatile("" ::: "memory");
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+__device__ __forceinline__ void count_lds(unsigned *p)
+{
+    asm volatile("" ::: "memory");
+    if (lane_id() == 0) __hip_atomic_fetch_add(p, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+template <int kForm, bool kReaderOwns>
+__global__ __launch_bounds__(kResBlock) void sim_resident_lists_kernel(bmtk_glif3_sim s, Resident r)
+{
+    constexpr bool kUnified = kForm != kFormAny, kRecord = kForm != kFormLean;
+    constexpr unsigned kRowCap = row_cap(kRecord), kCrowdedCap = 2u * kRowCap;
+    if (kForm != kFormAny) {
+        s.probe_col = nullptr;
+        s.inp_seg = nullptr;
+        s.inp_packed = nullptr;
+    }
+    extern __shared__ float ring_l[];  // [L*4][span], then kActCap words
+    __shared__ int go_on;
+    __shared__ unsigned rows_l[2], spikes_l[2], team_l[2], crowd_l[2], done_l, updated_l, listed_l;  // rows of a step, of neurons (the others: of inputs), ..
+    __shared__ unsigned fired_n[2];                               // how many fired in this step and the one before
+    __shared__ unsigned long long ballot_l[kResBlock / kWave];
+    const int tid = threadIdx.x, lane = lane_id();
+    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int per_xcd = (int)gridDim.x >> 3;  // an XCD gets consecutive groups, see sim_resident_kernel
+    const int g = (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
+    if (g >= r.n_groups) return;  // (the grid is rounded up; nobody waits for these)
+    const int ne = (int)s.n_neurons;
+    const int words = (ne + 63) >> 6;
+    const int L = s.ring_slots, G = r.n_groups;
+    const int span = r.span;
+    const int e0 = g * span;
+    const int mine = min(span, ne - e0);
+    const bool own = tid < mine;
+    const int e = e0 + tid;
+    unsigned *rows = reinterpret_cast<unsigned *>(ring_l + L * GLIF3_NREC * span);  // [2][kRowCap], a place per lane behind
+    unsigned short *fired_l = reinterpret_cast<unsigned short *>(rows + 2 * kRowCap + kWave);
+    float *frac_l = reinterpret_cast<float *>(fired_l + kResBlock);
+    unsigned *abort_word = s.res_sync + 1;
+    unsigned long long *lists = reinterpret_cast<unsigned long long *>(s.res_sync + kBarrierStride);
+    unsigned long long *hist = reinterpret_cast<unsigned long long *>(s.work_bits);
+    const bool alone = s.rec_seg == nullptr;  // nobody's spikes arrive anywhere
+    // a run before this one gave up and nobody has looked yet: do nothing, so that the failure is still there to see
+    if (tid == 0) {
+        go_on = load_agent(abort_word) == 0u;
+        fired_n[0] = fired_n[1] = rows_l[0] = rows_l[1] = spikes_l[0] = spikes_l[1] = team_l[0] = team_l[1] = crowd_l[0] = crowd_l[1] = done_l = updated_l = listed_l = 0u;
+    }
+    __syncthreads();
+    if (!go_on) return;
+
+    for (int c = tid; c < L * GLIF3_NREC * span; c += kResBlock) {
+        const int dr = c / span, i = c - dr * span;
+        ring_l[c] = i < mine ? s.ring[(int64_t)dr * ne + e0 + i] : 0.0f;
+    }
+    Glif3Elem st{};
+    Glif3Prop p{};
+    float I = 0.0f;
+    if (own) {
+        const int64_t col = s.class_id ? (int64_t)s.class_id[e] : e;
+        p.load(s.prop, s.prop_stride, col);
+        glif3_load(st, s.V, s.asc, s.y1, s.y2, s.ref, ne, e);
+        I = s.i_ext ? s.i_ext[e] : 0.0f;
+    }
+    __syncthreads();
+
+    const int n_steps = (int)r.n_steps;
+    auto wrap = [](int64_t a, int m) { return (int)(((a % m) + m) % m); };
+    int slot_prev = wrap(r.step0 - 1, L), row_t = wrap(r.step0, r.hist);  // ring slot of step t-1, history row of step t
+    auto next = [](int a, int m) { return a + 1 == m ? 0 : a + 1; };
+    auto row_before = [&]() { return row_t == 0 ? r.hist - 1 : row_t - 1; };
+    auto events_at = [&](int k) -> int64_t { return s.in_ptr ? s.in_ptr[r.step0 + k] : 0; };
+    auto lists_of = [&](int k) { return ListRow{lists + (k & (kListRows - 1)) * kListRowWords}; };
+
+    auto fold = [&](int slot) __attribute__((always_inline)) {
+        float *prev = ring_l + slot * GLIF3_NREC * span + tid;
+#pragma unroll
+        for (int q = 0; q < GLIF3_NREC; ++q) {
+            const float a = prev[q * span];
+            prev[q * span] = 0.0f;
+            st.y1[q] = st.y1[q] + a * p.psc0[q];
+        }
+    };
+    const int probe_col = (own && s.probe_col) ? s.probe_col[e] : -1;
+    int probe_phase = s.probe_col ? (int)((r.step0 + 1) % s.probe_every) : 1;  // 0: sample after this step
+    int64_t probe_row = 0;
+    const float zero[GLIF3_NREC] = {0.0f, 0.0f, 0.0f, 0.0f};
+    // fold and update of step step0 + k; what fired stays in LDS
+    auto update = [&](int k) __attribute__((always_inline)) {
+        bool spike = false;
+        float frac = 0.0f;
+        if (own) {
+            if (k > 0) fold(slot_prev);
+            spike = glif3_update(st, p, s.h, zero, I, &frac);
+        }
+        if (s.probe_col) {
+            if (probe_phase == 0) {
+                if (probe_col >= 0) s.probe_v[probe_row * s.probe_stride + probe_col] = st.V;
+                ++probe_row;
+            }
+            probe_phase = probe_phase + 1 == s.probe_every ? 0 : probe_phase + 1;
+        }
+        const unsigned long long m = __ballot(spike);
+        if (lane == 0) ballot_l[wave] = m;
+        if (m != 0ull && spike) {
+            const unsigned at = atomicAdd(&fired_n[k & 1], 1u);  // (at most span)
+            fired_l[at] = (unsigned short)tid;
+            if (kRecord) frac_l[at] = frac;
+        }
+    };
+    auto row_bounds = [&](unsigned row) __attribute__((always_inline)) -> SegBounds {
+        if (kUnified)  // rows * (n_groups + 1) stays below 2^32 (checked before the launch)
+            return *reinterpret_cast<const SegBounds *>(s.rec_seg + mul_u24(row, (unsigned)(G + 1)) + g);
+        const uint32_t *seg = row & kInputTag ? s.inp_seg : s.rec_seg;
+        return *reinterpret_cast<const SegBounds *>(seg + (int64_t)(row & ~kInputTag) * (G + 1) + g);
+    };
+    auto input_row = [&](int32_t source) { return kUnified ? (unsigned)source + (unsigned)s.n_neurons : (unsigned)source | kInputTag; };
+    auto add_bounds = [&](SegBounds b, bool of_input, unsigned part, unsigned team) __attribute__((always_inline)) {
+        const bmtk_synapse *tab = !kUnified && of_input ? s.inp_packed : s.rec_packed;
+        pull_bounds(b.lo, b.hi - b.lo, part, team, tab, RingSlice(ring_l, span, e0, L, slot_prev));  // the offsets never decrease
+    };
+    // The rows of step k-1 into the ring slice.  Where they are listed before the update of step k already (`ask` ahead of it),
+    // the bounds of a thread's first row are on their way meanwhile.
+    unsigned n_rows = 0u, team = 0u, at_row = 0u;
+    SegBounds first_row{0u, 0u};
+    auto ask = [&](int k) __attribute__((always_inline)) {
+        unsigned me = (unsigned)tid;
+        asm volatile("" : "+v"(me));
+        const int buf = (k - 1) & 1;
+        n_rows = (unsigned)__builtin_amdgcn_readfirstlane((int)rows_l[buf]);
+        team = (unsigned)__builtin_amdgcn_readfirstlane((int)team_l[buf]);
+        if (n_rows == kCrowded || wave == kWriter) n_rows = 0u;
+        at_row = me >> team;
+        if (at_row < n_rows) first_row = row_bounds(rows[buf * kRowCap + at_row]);
+    };
+    auto pull = [&](int k) __attribute__((always_inline)) {
+        const int buf = (k - 1) & 1;
+        const unsigned part = (unsigned)lane & ((1u << team) - 1u), step = (unsigned)kPullThreads >> team, n_spikes = spikes_l[buf];
+        while (at_row < n_rows) {
+            const SegBounds b = first_row;
+            const bool of_input = at_row >= n_spikes;
+            at_row += step;
+            if (at_row < n_rows) first_row = row_bounds(rows[buf * kRowCap + at_row]);
+            add_bounds(b, of_input, part, 1u << team);
+        }
+    };
+    // The same in a crowded step, by all threads: lists (row `row` of the history), ballots where a list did not suffice,
+    // and the events in_events[lo, hi).  What finds no room in the row list is pulled on the spot.
+    auto pull_crowded = [&](int k) __attribute__((always_inline)) {
+        const int row = row_before();
+        const int64_t lo = events_at(k - 1), hi = events_at(k);
+        unsigned *act = rows;
+        const ListRow from = lists_of(k - 1);
+        const unsigned long long *ballots = hist + (int64_t)row * (words + 1);
+        int me = tid;
+        asm volatile("" : "+v"(me));
+        const int of = me >> 2, sub = me & 3;  // four threads to a list
+        unsigned long long head = 0ull;
+        if (!alone && of < G) head = load_agent64(from.at(of, 0));
+        const unsigned n = (unsigned)(head >> kListCountAt) & kListMany;
+        const bool many = n == kListMany;
+        const int event_rounds = (int)((hi - lo + kResBlock - 1) / kResBlock);  // a step's events are below 2^31
+        for (int round = -event_rounds; round < 4; ++round) {
+            unsigned long long v = 0ull;
+            unsigned cnt = 0u, base = (unsigned)(of * span);
+            bool bits = false;
+            if (round < 0) {
+                const int64_t at = lo + (int64_t)(round + event_rounds) * kResBlock + tid;
+                if (at < hi) base = input_row(s.in_events[at]), cnt = 1u;
+            } else {
+                const int j = round * 4 + sub;  // word of the list, or of the workgroup's ballots (up to 16)
+                const unsigned first = j == 0 ? 0u : 5u * (unsigned)j - 1u;
+                if (many) {
+                    const int w = of * (span >> 6) + j;
+                    if (j < (span >> 6) && w < words) v = load_agent64(ballots + w);
+                    cnt = (unsigned)__popcll(v);
+                    base += 64u * (unsigned)j;
+                    bits = true;
+                } else if (j < kListWords && n > first) {
+                    // (words 0 and 1 have been seen; the others left with them)
+                    cnt = min(n - first, j == 0 ? 4u : 5u);
+                    unsigned spins = 0u;
+                    while (((v = load_agent64(from.at(of, j))) ^ head) >> kListTagAt) {
+                        if (++spins > kMaxSpin) {
+                            __hip_atomic_store(abort_word, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                            cnt = 0u;
+                            break;
+                        }
+                    }
+                }
+            }
+            const unsigned inc = wave_inclusive_scan(cnt);
+            unsigned at = 0u;
+            if (lane == kWave - 1 && inc) at = atomicAdd(&crowd_l[k & 1], inc);
+            at = (unsigned)bcast_i((int)at, kWave - 1) + inc - cnt;
+            for (; cnt > 0u; --cnt, ++at) {
+                unsigned id = base;
+                if (bits) {
+                    id += (unsigned)(__ffsll((long long)v) - 1);
+                    v &= v - 1ull;
+                } else if (round >= 0) {
+                    id += (unsigned)v & ((1u << kListIdBits) - 1u);
+                    v >>= kListIdBits;
+                }
+                if (at < kCrowdedCap)
+                    act[at] = id;
+                else
+                    add_bounds(row_bounds(id), (id & kInputTag) != 0u, 0u, 1u);
+            }
+        }
+        __syncthreads();
+        const unsigned total = min(crowd_l[k & 1], kCrowdedCap);
+        for (unsigned a = (unsigned)tid; a < total; a += kResBlock) add_bounds(row_bounds(act[a]), (act[a] & kInputTag) != 0u, 0u, 1u);
+        __syncthreads();
+    };
+    // The writer's part of a step: the list (the others wait for it), ballots, record.
+    const unsigned rec_ways = s.spike_ways > 1 ? (unsigned)s.spike_ways : 1u;
+    const unsigned long long rec_way = blockIdx.x & (rec_ways - 1u), rec_cap = (unsigned long long)s.spike_cap / rec_ways;
+    // with as many lists of the record as workgroups this one appends to its own alone and keeps the count in a register
+    const bool own_record = kRecord && s.spike_count != nullptr && rec_ways >= gridDim.x;
+    unsigned long long rec_count = own_record ? s.spike_count[rec_way * BMTK_RECORD_COUNT_STRIDE] : 0ull;
+    auto write = [&](int k) __attribute__((always_inline)) {
+        const int w = lane_here();
+        ListWrite list;
+        list.read(fired_l);
+        const unsigned n = fired_n[k & 1];
+        const unsigned long long m = ballot_l[w & (kResBlock / kWave - 1)];
+        const bool has = w < (span >> 6) && (e0 >> 6) + w < words;
+        auto ballots = [&]() {
+            if (has) __hip_atomic_store(hist + (int64_t)row_t * (words + 1) + (e0 >> 6) + w, m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        };
+        if (n > kListMax) {  // the ballots will be read: they have to have arrived before the list says so
+            ballots();
+            wait_vector_memory();
+        }
+        list.publish(lists_of(k), g, list_tag(k), n);
+        if (n <= kListMax) ballots();
+        if (s.spike_bits && has) s.spike_bits[k * s.spike_bits_stride + (e0 >> 6) + w] = m;
+        if (lane == 0) fired_n[(k + 1) & 1] = 0u;
+        if (kRecord && s.spike_count && n > 0u) {
+            unsigned long long base = rec_count;
+            if (!own_record) {
+                if (lane == 0) base = atomicAdd(s.spike_count + rec_way * BMTK_RECORD_COUNT_STRIDE, (unsigned long long)n);
+                base = bcast_u64(base, 0);
+            }
+            for (unsigned i = (unsigned)lane; i < n; i += kWave) {
+                if (base + i >= rec_cap) break;
+                const unsigned long long to = rec_way * rec_cap + base + i;
+                s.spike_step[to] = (int32_t)(r.step0 + k);
+                s.spike_elem[to] = e0 + (int)fired_l[i];
+                if (s.spike_frac) s.spike_frac[to] = frac_l[i];
+            }
+            rec_count += n;
+        }
+    };
+
+    // the pulls of round k are complete
+    auto pulled = [&](int k) __attribute__((always_inline)) {
+        while ((int)(load_lds(&done_l) - (unsigned)(k + 1) * kWriter) < 0) {}
+    };
+
+    bool aborted = false;
+    if (wave != kReader) {
+        for (int k = 0; k <= n_steps; ++k) {  // (one round more than steps: the closing pull)
+            const bool asked = k > 0 && load_lds(&listed_l) == (unsigned)k;
+            if (asked) ask(k);
+            if (k < n_steps) {
+                update(k);
+                if (wave != kWriter) {
+                    count_lds(&updated_l);
+                } else {
+                    const unsigned all = (unsigned)(k + 1) * (kReaderOwns ? kReader : kWriter);
+                    while ((int)(load_lds(&updated_l) - all) < 0) {}
+                    write(k);
+                }
+            }
+            __syncthreads();  // X
+            if (k > 0 && !go_on) {
+                aborted = true;
+                break;
+            }
+            if (k > 0) {
+                if (!asked) ask(k);
+                if (rows_l[(k - 1) & 1] == kCrowded)
+                    pull_crowded(k);
+                else
+                    pull(k);
+            }
+            if (k < n_steps) {
+                slot_prev = next(slot_prev, L);
+                row_t = next(row_t, r.hist);
+            }
+            if (wave != kWriter) count_lds(&done_l);
+            pulled(k);  // Y
+        }
+    } else {
+        ListLook seen;
+        seen.none();
+        bool have = false, lost = false;  // the step in hand: its bounds are in LDS; given up
+        unsigned failed = 0u;
+        int opaque_zero;
+        asm volatile("v_mov_b32 %0, 0" : "=v"(opaque_zero));
+        // lanes to a segment at most: its synapses on average, rounded up to a power of two
+        unsigned max_team = 0u;
+        {
+            float synapses = 0.0f, segments = 0.0f;
+            if (!alone) synapses += (float)s.rec_indptr[s.n_neurons], segments += (float)s.n_neurons;
+            if (s.in_ptr) synapses += (float)s.inp_indptr[s.n_inputs], segments += (float)s.n_inputs;
+            segments *= (float)G;
+            while (max_team < 6u && segments * (float)(1u << max_team) < synapses) ++max_team;
+        }
+        // the input events of the step in hand, the first of them on their way
+        int64_t ev_lo = events_at(0), ev_hi = events_at(1);
+        long long ev_next = 0;
+        int32_t ev[kReaderEvents] = {0, 0, 0, 0};
+        // one more look in vain: false when it is time to give up
+        auto again = [&]() __attribute__((always_inline)) -> bool {
+            const unsigned limit = s.res_spin_limit ? s.res_spin_limit : kMaxSpin;
+            if (++failed > limit) __hip_atomic_store(abort_word, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            return failed <= limit && load_agent(abort_word) == 0u;
+        };
+        // The rows of step k, whose lists have been seen, into LDS.  Every instruction here is one of a single wavefront, four
+        // clocks each and more beside three others on its SIMD: what no list holds is not stepped through, and a store too many
+        // (to the lane's spare place) is cheaper than a branch of lanes.
+        auto take = [&](int k) __attribute__((always_inline)) {
+            const int buf = k & 1;
+            const unsigned n_ev = (unsigned)(ev_hi - ev_lo);
+            unsigned c[kListRounds], sum = 0u;
+#pragma unroll
+            for (int u = 0; u < kListRounds; ++u) {
+                c[u] = seen.count(u, G);
+                sum += c[u];
+            }
+            have = true;
+            const unsigned inc = wave_inclusive_scan(sum);
+            const unsigned total = (unsigned)bcast_i((int)inc, kWave - 1);
+            const unsigned most = max(max(c[0], c[1]), max(c[2], c[3]));
+            unsigned n = total + n_ev;
+            if (__any(most > kListHalf) || n_ev > kRowCap || n > kRowCap) n = kCrowded;
+            if (n != kCrowded) {
+                const unsigned me = (unsigned)lane_here(), spare = 2u * kRowCap + me, at_buf = (unsigned)buf * kRowCap;
+                // the neurons in words `seen` of the lists, from the j0-th on
+                auto emit = [&](unsigned j0, bool first) __attribute__((always_inline)) {
+                    unsigned pos = at_buf + inc - sum + j0;
+#pragma unroll
+                    for (int u = 0; u < kListRounds; ++u) {
+                        if (u * kWave >= G) break;
+                        const unsigned base = (u * kWave + me) * (unsigned)span;
+#pragma unroll
+                        for (int i = 0; i < (first ? 9 : 10); ++i) {
+                            const bool is = c[u] > j0 + (unsigned)i;
+                            if (__ballot(is) == 0ull) break;
+                            const int at = first && i > 3 ? i + 1 : i;  // (word 0 holds four)
+                            rows[is ? pos + (unsigned)i : spare] = base + list_id(seen.v[u][at / 5], at % 5);
+                        }
+                        pos += c[u];
+                    }
+                };
+                emit(0u, true);
+#pragma unroll
+                for (int i = 0; i < kReaderEvents; ++i) {
+                    if ((unsigned)(i * kWave) >= n_ev) break;
+                    const unsigned a = i * kWave + me;
+                    int32_t source = ev[i];
+                    asm volatile("" : "+v"(source));  // (not looked at ahead of the lists)
+                    rows[a < n_ev ? at_buf + total + a : spare] = input_row(source);
+                }
+                for (unsigned a = kReaderEvents * kWave + me; a < n_ev; a += kWave) rows[at_buf + total + a] = input_row(s.in_events[ev_lo + a]);
+                if (__any(most > kListQuick)) {
+                    while (!seen.look(lists_of(k), G, list_tag(k), kListQuickWords)) {
+                        if (!again()) {
+                            lost = true;
+                            break;
+                        }
+                    }
+                    if (!lost) emit(kListQuick, false);
+                }
+            }
+            unsigned ts = 0u;
+            if (n != kCrowded)
+                while (ts < max_team && (n << (ts + 1u)) <= (unsigned)kPullThreads) ++ts;
+            if (lane == 0) {
+                rows_l[buf] = n;
+                spikes_l[buf] = total;
+                team_l[buf] = ts;
+                store_lds(&listed_l, lost ? 0u : (unsigned)k + 1u);
+            }
+        };
+        for (int k = 0; k <= n_steps; ++k) {
+            if (kReaderOwns && k < n_steps) {
+                if (k > 0) pulled(k - 1);
+                update(k);
+                count_lds(&updated_l);
+            }
+            if (k > 0) {
+                if (!alone) __builtin_amdgcn_s_sleep(8);
+                while (!have && !lost) {
+                    if (alone || seen.look(lists_of(k - 1), G, list_tag(k - 1)))
+                        take(k - 1);
+                    else
+                        lost = !again();
+                }
+                if (lane == 0) {
+                    go_on = !lost;
+                    crowd_l[k & 1] = 0u;
+                }
+            }
+            // vmcnt(0): nothing is on its way here, and with that said the compiler does not wait for loads below before it
+            // uses their registers again (a trip to memory at the busiest time)
+            __builtin_amdgcn_s_waitcnt(0x0F70);
+            const int64_t ev_end = ((int64_t)__builtin_amdgcn_readfirstlane((int)(ev_next >> 32)) << 32) |
+                                   (int64_t)(unsigned)__builtin_amdgcn_readfirstlane((int)ev_next);
+            __syncthreads();  // X
+            if (k > 0 && !go_on) {
+                aborted = true;
+                break;
+            }
+            // (as vector loads: a scalar load's answer would be waited for at the next LDS access)
+            if (s.in_ptr) ev_next = s.in_ptr[r.step0 + min(k + 2, n_steps) + opaque_zero];
+            if (k > 0 && k < n_steps) {  // the events of step k are next: their end was asked for a step ago
+                ev_lo = ev_hi;
+                ev_hi = ev_end;
+            }
+            if (k < n_steps) {
+                const unsigned n_ev = (unsigned)(ev_hi - ev_lo);
+                const int32_t *const from = s.in_events + ev_lo;
+                const unsigned me = (unsigned)lane_here();
+#pragma unroll
+                for (int i = 0; i < kReaderEvents; ++i)
+                    if (i * kWave + me < n_ev) ev[i] = from[i * kWave + me];
+            }
+            have = false;
+            failed = 0u;
+            if (k > 0 && rows_l[(k - 1) & 1] == kCrowded) pull_crowded(k);
+            if (k < n_steps) {
+                slot_prev = next(slot_prev, L);
+                row_t = next(row_t, r.hist);
+            }
+        }
+        if (kReaderOwns && !aborted) pulled(n_steps);
+    }
+    if (wave != kReader || kReaderOwns) {
+        if (own && !aborted) fold(slot_prev);
+        if (own) glif3_store(st, s.V, s.asc, s.y1, s.y2, s.ref, ne, e);
+    }
+    if (own_record && wave == kWriter && lane == 0) s.spike_count[rec_way * BMTK_RECORD_COUNT_STRIDE] = rec_count;
+    __syncthreads();
+    for (int c = tid; c < L * GLIF3_NREC * span; c += kResBlock) {
+        const int dr = c / span, i = c - dr * span;
+        if (i < mine) s.ring[(int64_t)dr * ne + e0 + i] = ring_l[c];
+    }
+}
+
+
+// the lists of a run back to no step's
+__global__ __launch_bounds__(kBlock) void zero_words_kernel(unsigned *w, int64_t n)
+{
+    const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (i < n) w[i] = 0u;
 }
 
 // abort flag and arrival counters of a resident run
@@ -786,14 +1246,23 @@ int simulate_resident(const bmtk_glif3_sim &s, int64_t step0, int64_t n_steps, h
                          (!has_inputs || (s.inp_packed == s.rec_packed &&
                                           s.inp_seg == s.rec_seg + s.n_neurons * (int64_t)(s.res_groups + 1)));
     const int form = !unified || s.probe_col != nullptr ? kFormAny : (s.spike_count != nullptr ? kFormRecord : kFormLean);
-    const void *const kernels[2][3] = {
+    // without slack the workgroups exchange lists (a history of four rows: see sim_resident_lists_kernel)
+    const bool lists = slack == 0 && s.delay_offset == 0 && s.res_fired != nullptr && s.res_groups <= kListGroups && hist >= 4;
+    const bool reader_owns = s.res_span > kReader * kWave;
+    const void *const kernels[4][3] = {
         {reinterpret_cast<const void *>(sim_resident_kernel<false, kFormAny>),
          reinterpret_cast<const void *>(sim_resident_kernel<false, kFormRecord>),
          reinterpret_cast<const void *>(sim_resident_kernel<false, kFormLean>)},
         {reinterpret_cast<const void *>(sim_resident_kernel<true, kFormAny>),
          reinterpret_cast<const void *>(sim_resident_kernel<true, kFormRecord>),
-         reinterpret_cast<const void *>(sim_resident_kernel<true, kFormLean>)}};
-    const void *kernel = kernels[slack > 0 ? 1 : 0][form];
+         reinterpret_cast<const void *>(sim_resident_kernel<true, kFormLean>)},
+        {reinterpret_cast<const void *>(sim_resident_lists_kernel<kFormAny, false>),
+         reinterpret_cast<const void *>(sim_resident_lists_kernel<kFormRecord, false>),
+         reinterpret_cast<const void *>(sim_resident_lists_kernel<kFormLean, false>)},
+        {reinterpret_cast<const void *>(sim_resident_lists_kernel<kFormAny, true>),
+         reinterpret_cast<const void *>(sim_resident_lists_kernel<kFormRecord, true>),
+         reinterpret_cast<const void *>(sim_resident_lists_kernel<kFormLean, true>)}};
+    const void *kernel = kernels[lists ? (reader_owns ? 3 : 2) : (slack > 0 ? 1 : 0)][form];
     hipError_t err = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (err != hipSuccess) {
         set_error("glif3_simulate_fwd: resident mode needs %zu bytes of LDS: %s", lds, hipGetErrorString(err));
@@ -810,7 +1279,11 @@ int simulate_resident(const bmtk_glif3_sim &s, int64_t step0, int64_t n_steps, h
                   n_cu, per_cu);
         return BMTK_E_LAUNCH;
     }
-    hipLaunchKernelGGL(zero_sync_kernel, dim3(1), dim3(kBlock), 0, stream, s.res_sync);
+    const int64_t list_words = 2 * kListRows * kListRowWords;
+    if (lists)
+        hipLaunchKernelGGL(zero_words_kernel, dim3((unsigned)((list_words + kBlock - 1) / kBlock)), dim3(kBlock), 0, stream, s.res_sync + kBarrierStride, list_words);
+    else
+        hipLaunchKernelGGL(zero_sync_kernel, dim3(1), dim3(kBlock), 0, stream, s.res_sync);
     bmtk_glif3_sim s_copy = s;
     // BMTK_AMD_PLAIN_LAUNCH=1 uses an ordinary launch (co-residency then rests on the occupancy check
     // above and an otherwise idle device); for tools that cannot follow cooperative launches.

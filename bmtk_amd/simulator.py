@@ -202,9 +202,8 @@ class Glif3Simulator:
                 workgroup, without a grid barrier (about 1 us per step instead of 2.5); False keeps such a network
                 on the many-workgroup form
     fired_lists  resident mode with several workgroups: every workgroup publishes the neurons that fired in a step
-                as a short list beside its ballots, and the others read the lists instead of expanding the whole
-                network's ballots (steps in which a list does not suffice are read from the ballots); False: always
-                from the ballots.  Same results either way.
+                as a short list whose words carry the step, and nobody waits at a grid barrier (neurons that a list does
+                not hold are read from the ballots); False: ballots behind a grid barrier.  Same results either way.
     expected_rate_hz  what "auto" decides ``pull`` / ``fused`` by.  Pushing spikes into the ring costs an atomic per
                 synaptic event, pulling a pass over the whole table per step whatever the activity; a synapse
                 carries batch * rate * h events per step, and on one MI355X the pass is the cheaper of the two from
@@ -692,7 +691,7 @@ class Glif3Simulator:
             self.rec_seg, self.inp_seg = seg[:self.n], seg[self.n:]
             self.res_unified = (packed, seg)
         self.res_span, self.res_groups = span, groups
-        # the lists of fired neurons the workgroups publish beside their ballots (bmtk_glif3_sim.res_fired)
+        # asks for the exchange by lists of fired neurons (bmtk_glif3_sim.res_fired)
         self.res_fired = (torch.zeros(self.hist_slots * groups * _lib.RES_FIRED_SLOTS, dtype=torch.int32, device=self.dev)
                           if groups > 1 and self.fired_lists else None)
 

@@ -235,8 +235,7 @@ int bmtk_csr_segment_offsets(int64_t n_rows, const int32_t *indptr, const int32_
 
 #define BMTK_RES_SYNC_STRIDE 1088                          /* words: 4 KiB + 256 B */
 #define BMTK_RES_SYNC_WAYS 8                               /* counters a step's arrivals are spread over */
-#define BMTK_RES_FIRED_SLOTS 16       /* places of a workgroup's list in bmtk_glif3_sim.res_fired */
-#define BMTK_RES_FIRED_MANY 0xFFFFFFFFu /* ... more neurons fired than the list holds */
+#define BMTK_RES_FIRED_SLOTS 16       /* words per workgroup and row of bmtk_glif3_sim.res_fired */
 #define BMTK_RES_SYNC_WORDS ((1 + 64 * BMTK_RES_SYNC_WAYS) * BMTK_RES_SYNC_STRIDE) /* size of bmtk_glif3_sim.res_sync */
 
 /* Everything nest.Simulate needs for a forward run (bmtk/simulator/pointnet/pointsimulator.py:159-166). */
@@ -307,21 +306,16 @@ typedef struct bmtk_glif3_sim {
     const uint32_t *inp_seg;     /* [inputs][res_groups+1] */
     uint32_t *res_sync;          /* BMTK_RES_SYNC_WORDS words of scratch, zeroed by the caller once: word 1 =
                                   * abort flag, from word BMTK_RES_SYNC_STRIDE on 64 x BMTK_RES_SYNC_WAYS arrival
-                                  * counters that many words apart, which every call zeroes again.  Word 1 != 0
+                                  * counters that many words apart (or lists, see res_fired), which every call clears for itself.  Word 1 != 0
                                   * after a run means a grid barrier timed out and the results are invalid.  The
                                   * flag is sticky: no call clears it, and a call that finds it set does nothing,
                                   * so a failure cannot be overwritten before the host has seen it; the host
                                   * clears it after reading. */
     uint32_t *res_fired;         /* optional, several workgroups only: [hist_slots][res_groups][BMTK_RES_FIRED_SLOTS]
-                                  * words (3 rows when hist_slots is 0), zeroed by the caller once and then left to
-                                  * the library.  Beside its
-                                  * ballots a workgroup publishes the neurons that fired in a step as a short list
-                                  * (number + 1; 0 = free place; all places BMTK_RES_FIRED_MANY when the list does not
-                                  * hold them), and the other workgroups read the lists instead of expanding the
-                                  * ballots of the whole network, each for itself; steps in which some list did not
-                                  * suffice are read from the ballots.  NULL: always from the ballots (a simulation passes it in
-                                  * every call or in none: the lists of a call's last steps are read by the next).  Used by runs
-                                  * without slack only (largest delay offset: the others do not wait per step). */
+                                  * words.  Given, runs without slack (delay offset 0, hist_slots of at least 4) exchange lists
+                                  * of the neurons that fired, whose words say themselves which step they belong to, instead of
+                                  * ballots behind a grid barrier.  The lists themselves are kept in res_sync.  NULL: always
+                                  * ballots and the barrier. */
     /* Pull form of the recurrent delivery for batched runs (optional; launch-per-step mode with delay_offset 0
      * and hist_slots == ring_slots): a TARGET-major packed copy of the recurrent table.  The recurrent arrivals
      * of step t-1 are then summed in one pass over that table from the spike-bit history

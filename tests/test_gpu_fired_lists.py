@@ -1,0 +1,104 @@
+"""The exchange by lists of fired neurons (sim_resident_lists_kernel) at the edges of what a list holds: 9, 19 and 39 neurons
+of a workgroup, more (its ballots), all of them, and more input events in a step than the row list has room for; spans with one
+wavefront of neurons, with all wavefronts but the reader's and with all sixteen."""
+import numpy as np
+import pytest
+import torch
+
+from bmtk_amd import simulator, synthetic
+from bmtk_amd.layout import PAR
+
+pytestmark = pytest.mark.gpu
+N, STEPS = 3000, 60
+
+
+def _network(seed):
+    rng = np.random.default_rng(seed)
+    n_in = 6000
+
+    def table(n_src, per_row):
+        indptr = np.arange(n_src + 1, dtype=np.int32) * per_row
+        idx = rng.integers(0, N, n_src * per_row).astype(np.int32)
+        w = (rng.integers(1, 200, idx.size) / 4.0).astype(np.float32)       # sums exact in fp32 in any order
+        return (indptr, idx, w, rng.integers(1, 6, idx.size).astype(np.uint8), rng.integers(0, 4, idx.size).astype(np.uint8))
+
+    per_step = rng.integers(0, 40, STEPS)
+    per_step[7], per_step[21] = 5000, 300
+    events = [np.sort(rng.integers(0, n_in, c)) for c in per_step]
+    ptr = np.concatenate([[0], np.cumsum(per_step)]).astype(np.int64)
+    return synthetic.random_cells(rng, N), table(N, 40), table(n_in, 7), ptr, np.concatenate(events).astype(np.int32)
+
+
+def _start(par, span, seed):
+    """Potentials above threshold for a chosen number of neurons of every workgroup: they fire in the first step."""
+    rng = np.random.default_rng(seed)
+    u = np.zeros(N, np.float32)
+    counts = [0, 1, 4, 5, 9, 10, 14, 19, 20, 34, 38, 39, 40, 64, span]
+    for g, e0 in enumerate(range(0, N, span)):
+        mine = min(span, N - e0)
+        pick = e0 + rng.permutation(mine)[:min(mine, counts[(g + seed) % len(counts)])]
+        u[pick] = (par[PAR["V_TH"]] - par[PAR["E_L"]])[pick] * 3.0
+    return u
+
+
+@pytest.mark.parametrize("form", ["bits", "record", "shared_record", "probes"])
+@pytest.mark.parametrize("span", [64, 960, 1024])
+def test_lists_at_their_edges_equal_per_step_launches(span, form, monkeypatch):
+    for seed in ((0, 5) if span == 64 else (8, 11, 12, 14)):
+        par, rec, inp, ptr, events = _network(seed)
+        u = _start(par, span, seed)
+
+        def run(resident):
+            monkeypatch.setattr(simulator, "resident_span", lambda *a, **k: span)
+            sim = simulator.Glif3Simulator(N, par, 1.0, rec=rec, inp=inp, u_init=u, resident=resident)
+            assert not resident or (sim.res_groups == -(-N // span) and sim.res_fired is not None)
+            sim.set_input_events(ptr, events)
+            if form == "probes":
+                sim.set_probes(np.arange(0, N, 7), every=2)
+            cap, ways = (N * STEPS * 256 if form == "record" else N * STEPS * 2), (256 if form == "record" else 2)
+            out = [sim.run(k, record_cap=cap if "record" in form else 0, record_ways=ways if "record" in form else None)
+                   for k in (1, 30, STEPS - 31)]
+            st = sim.state
+            got = dict(bits=torch.cat([o["bits"] for o in out]), V=st.V, y1=st.y1, y2=st.y2, asc=st.asc, ref=st.ref)
+            if "record" in form:
+                recs = [sim.collect_record(o["record"], sort_scale=1.0) for o in out]
+                assert not any(r["overflow"] for r in recs)
+                for key in ("step", "elem", "frac"):
+                    got[key] = torch.cat([r[key] for r in recs])
+            if form == "probes":
+                got["probe"] = torch.cat([o["probe"]["v"] for o in out])
+            sim.check()
+            return got
+
+        want, got = run(False), run(True)
+        assert int(want["bits"].ne(0).sum()) > 50
+        for key in want:
+            assert torch.equal(want[key], got[key]), (seed, key)
+
+
+def test_a_reader_gives_up_cleanly(monkeypatch):
+    """With a limit of one look in vain some reader gives up (workgroups do not start together): every wavefront leaves its loop,
+    check() reports the run, and the next one is right."""
+    par, rec, inp, ptr, events = _network(1)
+    monkeypatch.setattr(simulator, "resident_span", lambda *a, **k: 64)
+
+    def make():
+        sim = simulator.Glif3Simulator(N, par, 1.0, rec=rec, inp=inp, resident=True)
+        sim.set_input_events(ptr, events)
+        return sim
+    sim = make()
+    sim.spin_limit = 1
+    sim.run(40)
+    gave_up = int(sim.res_sync[1].item()) != 0
+    sim.spin_limit = 0
+    sim.run(20)             # finds the word set, if it is, and does nothing
+    if gave_up:
+        with pytest.raises(RuntimeError, match="barrier"):
+            sim.check()
+        assert int(sim.res_sync[1].item()) == 0
+    want = make()
+    want.run(60)
+    sim = make()
+    sim.run(60)
+    sim.check()
+    assert torch.equal(want.state.V, sim.state.V)
