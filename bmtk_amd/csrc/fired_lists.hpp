@@ -43,8 +43,10 @@ constexpr int kListRows = 4;   // lists of so many steps are kept
 constexpr int kListRowWords = kListWords * kListGroups;
 struct ListRow {
     unsigned long long *w;
+    int first, G;  // the lists that belong together: first .. first + G - 1
     __device__ __forceinline__ unsigned long long *at(int g, int j) const
     {
+        g += first;
         return w + (j < kListQuickWords ? kListQuickWords * g + j
                                         : kListQuickWords * kListGroups + (kListWords - kListQuickWords) * g + j - kListQuickWords);
     }
@@ -93,21 +95,26 @@ struct ListLook {
         for (int u = 0; u < kListRounds; ++u) v[u][0] = v[u][1] = 0ull;
     }
     // asks once for words `from`, `from` + 1 of all G lists; true when every workgroup has published them in the wanted step
-    __device__ __forceinline__ bool look(const ListRow &row, int G, unsigned tag, int from = 0)
+    // (kFew: lists are seldom more than a wavefront's lanes, and a branch past the rest is worth it)
+    template <bool kFew>
+    __device__ __forceinline__ bool look(const ListRow &row, unsigned tag, int from = 0)
     {
         const unsigned lane = (unsigned)lane_here();
         const char *base = reinterpret_cast<const char *>(row.at(0, from));
         const unsigned stride = 8u * (from ? kListWords - kListQuickWords : kListQuickWords);
 #pragma unroll
         for (int u = 0; u < kListRounds; ++u) {
-            const unsigned long long *p = reinterpret_cast<const unsigned long long *>(base + min(u * kWave + lane, (unsigned)G - 1u) * stride);
+            if (kFew && u * kWave >= row.G) break;
+            const unsigned long long *p = reinterpret_cast<const unsigned long long *>(base + min(u * kWave + lane, (unsigned)row.G - 1u) * stride);
             v[u][0] = load_agent64(p);
             v[u][1] = load_agent64(p + 1);
         }
         unsigned differs = 0u;
 #pragma unroll
-        for (int u = 0; u < kListRounds; ++u)
+        for (int u = 0; u < kListRounds; ++u) {
+            if (kFew && u * kWave >= row.G) break;
             differs |= ((unsigned)(v[u][0] >> 32) ^ (tag << (kListTagAt - 32))) | ((unsigned)(v[u][1] >> 32) ^ (tag << (kListTagAt - 32)));
+        }
         return __ballot((differs >> (kListTagAt - 32)) != 0u) == 0ull;
     }
     __device__ __forceinline__ unsigned count(int u, int G) const
@@ -123,6 +130,143 @@ __device__ __forceinline__ unsigned list_id(unsigned long long word, int i)
     const int at = kListIdBits * i;
     const unsigned bits = at + kListIdBits <= 32 ? lo >> at : at >= 32 ? hi >> (at - 32) : __builtin_amdgcn_alignbit(hi, lo, at);
     return bits & ((1u << kListIdBits) - 1u);
+}
+
+// One wavefront: the neurons in the lists `seen`, whose workgroups own `span` neurons each, to rows[to ..] in LDS.  Returns their
+// number, or kCrowded where a list holds too many for this or there is no room for them and `more` rows in `cap` places; false
+// of `again` (called with every look in vain) gives up.  rows[spare] is the lane's own place for what is no row.
+// Every instruction here is one of a single wavefront, four clocks each and more beside three others on its SIMD: what no
+// list holds is not stepped through, and a store too many is cheaper than a branch of lanes.
+constexpr unsigned kCrowded = 0xFFFFFFFFu;  // in place of a number of rows
+template <bool kFew, typename Again>
+__device__ __forceinline__ unsigned rows_from_lists(ListLook &seen, const ListRow &lists, unsigned tag, int span, unsigned *rows,
+                                                    unsigned to, unsigned cap, unsigned spare, unsigned more, Again again, bool &lost)
+{
+    unsigned c[kListRounds], sum = 0u;
+#pragma unroll
+    for (int u = 0; u < kListRounds; ++u) {
+        c[u] = seen.count(u, lists.G);
+        sum += c[u];
+    }
+    const unsigned inc = wave_inclusive_scan(sum);
+    const unsigned total = (unsigned)bcast_i((int)inc, kWave - 1);
+    const unsigned most = max(max(c[0], c[1]), max(c[2], c[3]));
+    if (__any(most > kListHalf) || more > cap || total + more > cap) return kCrowded;
+    const unsigned me = (unsigned)lane_here();
+    // the neurons in the words of `seen`, from the j0-th of a list on
+    auto emit = [&](unsigned j0, bool first) __attribute__((always_inline)) {
+        unsigned pos = to + inc - sum + j0;
+#pragma unroll
+        for (int u = 0; u < kListRounds; ++u) {
+            if (u * kWave >= lists.G) break;
+            const unsigned base = (u * kWave + me) * (unsigned)span;
+#pragma unroll
+            for (int i = 0; i < (first ? 9 : 10); ++i) {
+                const bool is = c[u] > j0 + (unsigned)i;
+                if (__ballot(is) == 0ull) break;
+                const int at = first && i > 3 ? i + 1 : i;  // (word 0 holds four)
+                rows[is ? pos + (unsigned)i : spare] = base + list_id(seen.v[u][at / 5], at % 5);
+            }
+            pos += c[u];
+        }
+    };
+    emit(0u, true);
+    if (__any(most > kListQuick)) {
+        while (!seen.template look<kFew>(lists, tag, kListQuickWords)) {
+            if (!again()) {
+                lost = true;
+                return kCrowded;
+            }
+        }
+        emit(kListQuick, false);
+    }
+    return total;
+}
+
+// All 1024 threads: the rows of a crowded step -- the neurons in `lists` (ballots where a list did not suffice, `ballot_words` to a
+// workgroup, `words` in all) and n_ev rows event(i) -- to act[0 .. cap), their number to *count, which was zero.  What finds no
+// room goes to spot(row) at once.  kWordRounds: 4 * kWordRounds words cover a list or a workgroup's ballots.
+template <int kWordRounds, typename Event, typename Spot>
+__device__ __forceinline__ void crowded_rows(const ListRow &lists, bool any, int span, const unsigned long long *ballots, int words,
+                                             unsigned n_ev, unsigned *act, unsigned cap, unsigned *count, unsigned *abort_word,
+                                             unsigned max_spin, Event event, Spot spot)
+{
+    constexpr unsigned kThreads = 1024u;
+    int me = (int)threadIdx.x;
+    asm volatile("" : "+v"(me));
+    const int of = me >> 2, sub = me & 3;  // four threads to a list
+    unsigned long long head = 0ull;
+    if (any && of < lists.G) head = load_agent64(lists.at(of, 0));
+    const unsigned n = (unsigned)(head >> kListCountAt) & kListMany;
+    const bool many = n == kListMany;
+    const int event_rounds = (int)((n_ev + kThreads - 1u) / kThreads);
+    for (int round = -event_rounds; round < kWordRounds; ++round) {
+        unsigned long long v = 0ull;
+        unsigned cnt = 0u, base = (unsigned)(of * span);
+        bool bits = false;
+        if (round < 0) {
+            const unsigned at = (unsigned)(round + event_rounds) * kThreads + (unsigned)me;
+            if (at < n_ev) base = event(at), cnt = 1u;
+        } else {
+            const int j = round * 4 + sub;  // word of the list, or of the workgroup's ballots
+            const unsigned first = j == 0 ? 0u : 5u * (unsigned)j - 1u;
+            if (many) {
+                const int w = of * (span >> 6) + j;
+                if (j < (span >> 6) && w < words) v = load_agent64(ballots + w);
+                cnt = (unsigned)__popcll(v);
+                base += 64u * (unsigned)j;
+                bits = true;
+            } else if (j < kListWords && n > first) {
+                // (words 0 and 1 have been seen; the others left with them)
+                cnt = min(n - first, j == 0 ? 4u : 5u);
+                unsigned spins = 0u;
+                while (((v = load_agent64(lists.at(of, j))) ^ head) >> kListTagAt) {
+                    if (++spins > max_spin) {
+                        __hip_atomic_store(abort_word, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        cnt = 0u;
+                        break;
+                    }
+                }
+            }
+        }
+        const unsigned inc = wave_inclusive_scan(cnt);
+        unsigned at = 0u;
+        if (lane_id() == kWave - 1 && inc) at = atomicAdd(count, inc);
+        at = (unsigned)bcast_i((int)at, kWave - 1) + inc - cnt;
+        for (; cnt > 0u; --cnt, ++at) {
+            unsigned id = base;
+            if (bits) {
+                id += (unsigned)(__ffsll((long long)v) - 1);
+                v &= v - 1ull;
+            } else if (round >= 0) {
+                id += (unsigned)v & ((1u << kListIdBits) - 1u);
+                v >>= kListIdBits;
+            }
+            if (at < cap)
+                act[at] = id;
+            else
+                spot(id);
+        }
+    }
+}
+
+// Words of LDS that wavefronts of the workgroup tell one another how far they are by.  A wavefront's accesses to LDS are worked
+// off in the order it issues them; only the compiler has to be kept from another order.
+__device__ __forceinline__ unsigned load_lds(unsigned *p)
+{
+    const unsigned v = __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    asm volatile("" ::: "memory");
+    return v;
+}
+__device__ __forceinline__ void store_lds(unsigned *p, unsigned v)
+{
+    asm volatile("" ::: "memory");
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+__device__ __forceinline__ void count_lds(unsigned *p)
+{
+    asm volatile("" ::: "memory");
+    if (lane_id() == 0) __hip_atomic_fetch_add(p, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
 }  // namespace bmtk

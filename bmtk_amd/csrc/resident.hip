@@ -708,32 +708,12 @@ __global__ __launch_bounds__(kResBlock) void sim_resident_kernel(bmtk_glif3_sim 
 constexpr int kReader = kResBlock / kWave - 1, kWriter = kReader - 1;
 constexpr int kPullThreads = kWriter * kWave;
 static_assert((kWays * kBarrierWords) * kBarrierStride * 4 >= kListRows * kListRowWords * 8, "res_sync holds the lists");
-constexpr unsigned kCrowded = 0xFFFFFFFFu;
 constexpr int kReaderEvents = 4;    // input events a lane of the reader asks for ahead
 // the room of the row list (kActCap words) divided up: rows of two steps, a place per lane of the reader for what is none, the
 // neurons of this workgroup that fired and, for a record, their crossing fractions
 constexpr unsigned row_cap(bool record)
 {
     return (unsigned)((kActCap * 4 - 2 * kResBlock - (record ? 4 * kResBlock : 0) - 4 * kWave) / 8);
-}
-
-// Words of LDS that wavefronts of the workgroup tell one another how far they are by.  A wavefront's accesses to LDS are worked
-// off in the order it issues them; only the compiler has to be kept from another order.
-__device__ __forceinline__ unsigned load_lds(unsigned *p)
-{
-    const unsigned v = __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    asm volatile("" ::: "memory");
-    return v;
-}
-__device__ __forceinline__ void store_lds(unsigned *p, unsigned v)
-{
-    asm volatile("" ::: "memory");
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-}
-__device__ __forceinline__ void count_lds(unsigned *p)
-{
-    asm volatile("" ::: "memory");
-    if (lane_id() == 0) __hip_atomic_fetch_add(p, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
 template <int kForm, bool kReaderOwns>
@@ -800,7 +780,7 @@ __global__ __launch_bounds__(kResBlock) void sim_resident_lists_kernel(bmtk_glif
     auto next = [](int a, int m) { return a + 1 == m ? 0 : a + 1; };
     auto row_before = [&]() { return row_t == 0 ? r.hist - 1 : row_t - 1; };
     auto events_at = [&](int k) -> int64_t { return s.in_ptr ? s.in_ptr[r.step0 + k] : 0; };
-    auto lists_of = [&](int k) { return ListRow{lists + (k & (kListRows - 1)) * kListRowWords}; };
+    auto lists_of = [&](int k) { return ListRow{lists + (k & (kListRows - 1)) * kListRowWords, 0, G}; };
 
     auto fold = [&](int slot) __attribute__((always_inline)) {
         float *prev = ring_l + slot * GLIF3_NREC * span + tid;
@@ -877,70 +857,14 @@ __global__ __launch_bounds__(kResBlock) void sim_resident_lists_kernel(bmtk_glif
     // The same in a crowded step, by all threads: lists (row `row` of the history), ballots where a list did not suffice,
     // and the events in_events[lo, hi).  What finds no room in the row list is pulled on the spot.
     auto pull_crowded = [&](int k) __attribute__((always_inline)) {
-        const int row = row_before();
-        const int64_t lo = events_at(k - 1), hi = events_at(k);
-        unsigned *act = rows;
-        const ListRow from = lists_of(k - 1);
-        const unsigned long long *ballots = hist + (int64_t)row * (words + 1);
-        int me = tid;
-        asm volatile("" : "+v"(me));
-        const int of = me >> 2, sub = me & 3;  // four threads to a list
-        unsigned long long head = 0ull;
-        if (!alone && of < G) head = load_agent64(from.at(of, 0));
-        const unsigned n = (unsigned)(head >> kListCountAt) & kListMany;
-        const bool many = n == kListMany;
-        const int event_rounds = (int)((hi - lo + kResBlock - 1) / kResBlock);  // a step's events are below 2^31
-        for (int round = -event_rounds; round < 4; ++round) {
-            unsigned long long v = 0ull;
-            unsigned cnt = 0u, base = (unsigned)(of * span);
-            bool bits = false;
-            if (round < 0) {
-                const int64_t at = lo + (int64_t)(round + event_rounds) * kResBlock + tid;
-                if (at < hi) base = input_row(s.in_events[at]), cnt = 1u;
-            } else {
-                const int j = round * 4 + sub;  // word of the list, or of the workgroup's ballots (up to 16)
-                const unsigned first = j == 0 ? 0u : 5u * (unsigned)j - 1u;
-                if (many) {
-                    const int w = of * (span >> 6) + j;
-                    if (j < (span >> 6) && w < words) v = load_agent64(ballots + w);
-                    cnt = (unsigned)__popcll(v);
-                    base += 64u * (unsigned)j;
-                    bits = true;
-                } else if (j < kListWords && n > first) {
-                    // (words 0 and 1 have been seen; the others left with them)
-                    cnt = min(n - first, j == 0 ? 4u : 5u);
-                    unsigned spins = 0u;
-                    while (((v = load_agent64(from.at(of, j))) ^ head) >> kListTagAt) {
-                        if (++spins > kMaxSpin) {
-                            __hip_atomic_store(abort_word, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                            cnt = 0u;
-                            break;
-                        }
-                    }
-                }
-            }
-            const unsigned inc = wave_inclusive_scan(cnt);
-            unsigned at = 0u;
-            if (lane == kWave - 1 && inc) at = atomicAdd(&crowd_l[k & 1], inc);
-            at = (unsigned)bcast_i((int)at, kWave - 1) + inc - cnt;
-            for (; cnt > 0u; --cnt, ++at) {
-                unsigned id = base;
-                if (bits) {
-                    id += (unsigned)(__ffsll((long long)v) - 1);
-                    v &= v - 1ull;
-                } else if (round >= 0) {
-                    id += (unsigned)v & ((1u << kListIdBits) - 1u);
-                    v >>= kListIdBits;
-                }
-                if (at < kCrowdedCap)
-                    act[at] = id;
-                else
-                    add_bounds(row_bounds(id), (id & kInputTag) != 0u, 0u, 1u);
-            }
-        }
+        const int64_t lo = events_at(k - 1), hi = events_at(k);  // (a step's events are below 2^31)
+        auto pull_row = [&](unsigned row) __attribute__((always_inline)) { add_bounds(row_bounds(row), (row & kInputTag) != 0u, 0u, 1u); };
+        crowded_rows<4>(lists_of(k - 1), !alone, span, hist + (int64_t)row_before() * (words + 1), words, (unsigned)(hi - lo), rows,
+                        kCrowdedCap, &crowd_l[k & 1], abort_word, kMaxSpin,
+                        [&](unsigned i) { return input_row(s.in_events[lo + i]); }, pull_row);
         __syncthreads();
         const unsigned total = min(crowd_l[k & 1], kCrowdedCap);
-        for (unsigned a = (unsigned)tid; a < total; a += kResBlock) add_bounds(row_bounds(act[a]), (act[a] & kInputTag) != 0u, 0u, 1u);
+        for (unsigned a = (unsigned)tid; a < total; a += kResBlock) pull_row(rows[a]);
         __syncthreads();
     };
     // The writer's part of a step: the list (the others wait for it), ballots, record.
@@ -1049,44 +973,16 @@ __global__ __launch_bounds__(kResBlock) void sim_resident_lists_kernel(bmtk_glif
             if (++failed > limit) __hip_atomic_store(abort_word, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             return failed <= limit && load_agent(abort_word) == 0u;
         };
-        // The rows of step k, whose lists have been seen, into LDS.  Every instruction here is one of a single wavefront, four
-        // clocks each and more beside three others on its SIMD: what no list holds is not stepped through, and a store too many
-        // (to the lane's spare place) is cheaper than a branch of lanes.
+        // the rows of step k, whose lists have been seen, into LDS
         auto take = [&](int k) __attribute__((always_inline)) {
             const int buf = k & 1;
             const unsigned n_ev = (unsigned)(ev_hi - ev_lo);
-            unsigned c[kListRounds], sum = 0u;
-#pragma unroll
-            for (int u = 0; u < kListRounds; ++u) {
-                c[u] = seen.count(u, G);
-                sum += c[u];
-            }
+            const unsigned me = (unsigned)lane_here(), spare = 2u * kRowCap + me, at_buf = (unsigned)buf * kRowCap;
             have = true;
-            const unsigned inc = wave_inclusive_scan(sum);
-            const unsigned total = (unsigned)bcast_i((int)inc, kWave - 1);
-            const unsigned most = max(max(c[0], c[1]), max(c[2], c[3]));
-            unsigned n = total + n_ev;
-            if (__any(most > kListHalf) || n_ev > kRowCap || n > kRowCap) n = kCrowded;
-            if (n != kCrowded) {
-                const unsigned me = (unsigned)lane_here(), spare = 2u * kRowCap + me, at_buf = (unsigned)buf * kRowCap;
-                // the neurons in words `seen` of the lists, from the j0-th on
-                auto emit = [&](unsigned j0, bool first) __attribute__((always_inline)) {
-                    unsigned pos = at_buf + inc - sum + j0;
-#pragma unroll
-                    for (int u = 0; u < kListRounds; ++u) {
-                        if (u * kWave >= G) break;
-                        const unsigned base = (u * kWave + me) * (unsigned)span;
-#pragma unroll
-                        for (int i = 0; i < (first ? 9 : 10); ++i) {
-                            const bool is = c[u] > j0 + (unsigned)i;
-                            if (__ballot(is) == 0ull) break;
-                            const int at = first && i > 3 ? i + 1 : i;  // (word 0 holds four)
-                            rows[is ? pos + (unsigned)i : spare] = base + list_id(seen.v[u][at / 5], at % 5);
-                        }
-                        pos += c[u];
-                    }
-                };
-                emit(0u, true);
+            const unsigned total = rows_from_lists<false>(seen, lists_of(k), list_tag(k), span, rows, at_buf, kRowCap, spare, n_ev, again, lost);
+            unsigned n = kCrowded;
+            if (total != kCrowded) {
+                n = total + n_ev;
 #pragma unroll
                 for (int i = 0; i < kReaderEvents; ++i) {
                     if ((unsigned)(i * kWave) >= n_ev) break;
@@ -1096,15 +992,6 @@ __global__ __launch_bounds__(kResBlock) void sim_resident_lists_kernel(bmtk_glif
                     rows[a < n_ev ? at_buf + total + a : spare] = input_row(source);
                 }
                 for (unsigned a = kReaderEvents * kWave + me; a < n_ev; a += kWave) rows[at_buf + total + a] = input_row(s.in_events[ev_lo + a]);
-                if (__any(most > kListQuick)) {
-                    while (!seen.look(lists_of(k), G, list_tag(k), kListQuickWords)) {
-                        if (!again()) {
-                            lost = true;
-                            break;
-                        }
-                    }
-                    if (!lost) emit(kListQuick, false);
-                }
             }
             unsigned ts = 0u;
             if (n != kCrowded)
@@ -1125,7 +1012,7 @@ __global__ __launch_bounds__(kResBlock) void sim_resident_lists_kernel(bmtk_glif
             if (k > 0) {
                 if (!alone) __builtin_amdgcn_s_sleep(8);
                 while (!have && !lost) {
-                    if (alone || seen.look(lists_of(k - 1), G, list_tag(k - 1)))
+                    if (alone || seen.look<false>(lists_of(k - 1), list_tag(k - 1)))
                         take(k - 1);
                     else
                         lost = !again();

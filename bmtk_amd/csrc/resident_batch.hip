@@ -2,14 +2,14 @@
 // resident.hip, with the workgroups of the chip divided among several trials.
 //
 // The trials of a batch do not touch one another.  `ways` of them run side by side in one cooperative launch, each on
-// `groups` workgroups with a grid barrier of its own; launches follow one another until every trial has had its turn.
-// A workgroup owns `span` neurons of its trial.  Per step it
-//   1. folds the arrivals of slot t-1 (LDS) into y1, updates its neurons from registers and publishes their ballots;
-//   2. reads the ballots that its trial's workgroups published a step ago, packs the neurons that fired and the trial's
-//      input events into a list of rows, signals the barrier of step t on the way, and adds its own segment of every
-//      listed row (rows sorted by target, segment bounds in a table) to its ring slice.  A row's segment is read by
-//      `1 << team_shift` neighbouring lanes: with few workgroups to a trial a segment holds tens of synapses, which one
-//      lane would take one after the other.
+// `groups` workgroups that exchange lists of the neurons that fired (fired_lists.hpp); launches follow one another until
+// every trial has had its turn.  A workgroup owns `span` neurons of its trial, and its wavefronts divide the work as those of
+// sim_resident_lists_kernel (resident.hip) do: a reader, a writer, the others pull; all but the reader update.  Round k
+//   1. folds the arrivals of slot k-1 (LDS) into y1 and updates from registers; the writer publishes who fired, the reader
+//      makes the lists of step k-1 and the trial's input events into a list of rows;
+//   2. behind the workgroup's meeting, adds its own segment of every listed row (rows sorted by target, segment bounds in a
+//      table) to its ring slice.  A row's segment is read by `1 << team_shift` neighbouring lanes: with few workgroups to a
+//      trial a segment holds tens of synapses, which one lane would take one after the other.
 // Neither state nor arrival sums cross the memory system, and of the table only the segments of rows that fired.
 //
 // Sums are 64-bit fixed point, exact and independent of the order, as in the fused batched driver (and an integer
@@ -17,17 +17,20 @@
 // spikes of step t-1 are added, so that ring_slots - 1 slots suffice: 160 bytes of LDS per neuron and trial at delays of
 // up to five steps.  Behind a call the arrivals still ahead wait in rb_ring, trial by trial.
 //
-// What bounds it: a step is a chain of dependent loads (ballots, segment bounds, synapses) and the barrier, 3 us at the
-// smallest sizes, whatever the number of trials side by side; then the table's segments, which every trial reads for itself.
+// What bounds it: a step is a chain of dependent loads (lists, segment bounds, synapses), 2.5 us at the smallest sizes,
+// whatever the number of trials side by side; then the table's segments, which every trial reads for itself.  Per step and
+// launch, ballots and a grid barrier per trial -> lists: 230,924 neurons x 8 6.9 -> 6.1 us, 20,011 x 20 5.0 -> 4.7,
+// 400,123 x 1 9.3 -> 6.6; 51,978 x 32, which reads 18 synapses a segment for 243 rows of each of four trials, 5.2 as before.
 //
 // One trial of more neurons than the compute units have threads (resident.hip ends at 1024 to a workgroup) runs here with two
-// neurons to a thread and its ring in floats, 80 bytes a neuron: 400,123 neurons, 72 M synapses, 23 -> 9 us per step against a
-// launch per step with an atomic per event (call and set-up included: 25.4 -> 9.8).  What it is short of are the 128 vector
-// registers a thread has: 84 hold two neurons.  Ballots kept over the prefix sum, addresses and products worked out once
-// for all steps spilled 81 of them to memory (13.3 us per step).
+// neurons to a thread and its ring in floats, 80 bytes a neuron: 400,123 neurons, 72 M synapses, 23 -> 6.6 us per step against
+// a launch per step with an atomic per event.  What it is short of are the 128 vector
+// registers a thread has: 84 hold two neurons.  Addresses and products worked out once for all steps spill
+// half of them to memory, hence the opaque thread numbers below.
 #include <math.h>
 #include <stdlib.h>
 
+#include "fired_lists.hpp"
 #include "glif3_update.hpp"
 #include "pull_common.hpp"
 #include "sim_internal.hpp"
@@ -36,18 +39,18 @@ namespace bmtk {
 
 constexpr int kRbBlock = 1024;
 constexpr int kRbWaves = kRbBlock / kWave;
-constexpr int kRbHist = 4;                // rows of the ballot history
-constexpr unsigned kRbMaxSpin = 4000000u; // polls of the barrier before giving up (seconds)
-constexpr int kRbCounters = 64;           // arrival counters per way of res_sync, dealt out to the trials of a launch
-constexpr int kRbWideWords = 8;           // ballot words per thread with two neurons to a thread
-constexpr int kRbTogether = 4;            // synapses a lane has in flight
+constexpr int kRbReader = kRbWaves - 1, kRbWriter = kRbReader - 1;  // wavefronts with a part of their own, see resident.hip
+constexpr int kRbPullThreads = kRbWriter * kWave;
+constexpr unsigned kRbMaxSpin = 4000000u; // looks in vain before giving up (seconds)
+constexpr int kRbTogether = 6;            // synapses a lane has in flight (20,011 x 20, 8 lanes to 33: 4 of them 9.6 us per step, 6 9.3)
+constexpr int kRbEvents = 4;              // input events a lane of the reader asks for ahead
+static_assert(BMTK_RES_SYNC_WORDS >= BMTK_RES_SYNC_STRIDE + 2 * kListRows * kListRowWords, "res_sync holds the lists");
 
 struct RbLaunch {
     int64_t step0;
     int n_steps;
     int trial0, trials;   // trials of this launch
     int slots;            // of the ring slice: ring_slots - 1
-    int sync_slots;       // arrival counters of a trial, used in turn (a power of two)
     int words;            // ballot words of a trial
     int has_events;
     double unit;          // of the fixed-point sums
@@ -62,26 +65,22 @@ struct __attribute__((packed, aligned(4))) RbBounds {
     uint32_t lo, hi;
 };
 
-// The barrier's contract is that of resident.hip: ballots are stored and read with agent-scope accesses, every wavefront
-// waits until its stores have been acknowledged (s_waitcnt vmcnt(0)) before its workgroup meets and one thread arrives,
-// and a reader has counted all arrivals of the step before.  A trial's workgroups only count one another.  A workgroup
-// arrives for step t after it has seen everybody arrive for step t-1, so that the arrivals of two steps never mix and one
-// counter per trial would do; several used in turn keep a look at step t-1 apart from the arrivals of step t.  A workgroup
-// that writes ballot row t%4 is at most two steps ahead of one that still reads row (t-3)%4.
-// kWords: ballot words per thread.  kPer: neurons per thread; with two, the threads of the last wavefront (the looker) own
-// none.  Sum: what the ring holds, 64-bit fixed point (from_fixed), or floats where a workgroup's neurons are too many for
-// that (batch 1): fp32 atomics into device memory are what it then takes the place of.
-// kSave: potentials and step flags of every step go to rb_save_*, trial by trial; by_step_kernel puts them in their order.
-template <int kWords, int kPer, typename Sum, bool kSave>
+// kPer: neurons per thread; with two, the threads of the reader own none.  Sum: what the ring holds, 64-bit fixed point
+// (from_fixed), or floats where a workgroup's neurons are too many for that (batch 1): fp32 atomics into device memory are what
+// it then takes the place of.  kSave: potentials and step flags of every step go to rb_save_*, trial by trial; by_step_kernel
+// puts them in their order.  kReaderOwns: spans above 960 with a neuron to a thread.
+template <int kPer, typename Sum, bool kSave, bool kReaderOwns>
 __global__ __launch_bounds__(kRbBlock) void sim_resident_batch_kernel(bmtk_glif3_sim s, RbLaunch q)
 {
     constexpr bool kFixed = sizeof(Sum) == 8;
-    constexpr int kOwners = kPer == 1 ? kRbBlock : kRbBlock - kWave;  // threads that own neurons tid, tid + kOwners, ..
-    extern __shared__ unsigned long long rb_lds[];  // ring slice [slots * 4][span], then the list of rows
+    constexpr int kOwners = kRbReader * kWave;  // with two neurons to a thread: threads that own tid, tid + kOwners
+    extern __shared__ unsigned long long rb_lds[];  // ring slice [slots * 4][span], then rb_list words for rows
     __shared__ int go_on;
-    __shared__ unsigned scan_l[kRbWaves];
-    __shared__ unsigned listed[2];  // rows in the list of this step and the next (one wide trial)
-    const int tid = threadIdx.x, lane = lane_id(), wave = tid / kWave;
+    __shared__ unsigned rows_l[2], crowd_l[2], done_l, updated_l, listed_l;  // rows of a round, ..
+    __shared__ unsigned fired_n[2];                  // how many fired in this step and the one before
+    __shared__ unsigned short fired_l[kListMax + 1]; // the first of them, counted within the span
+    const int tid = threadIdx.x, lane = lane_id();
+    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
     const int span = s.rb_span, G = s.rb_groups;
     // an XCD (block number mod 8) gets consecutive workgroups, hence a trial as few XCDs as hold it
     const int per_xcd = (int)gridDim.x >> 3;
@@ -93,18 +92,24 @@ __global__ __launch_bounds__(kRbBlock) void sim_resident_batch_kernel(bmtk_glif3
     const int e0 = g * span;
     const int mine = min(span, n - e0);
     const int64_t ne = (int64_t)n * batch;
-    auto place = [&](int u) { return kPer == 1 ? tid : (tid < kOwners ? u * kOwners + tid : span); };  // in the workgroup's span
-    auto owns = [&](int u) { return place(u) < mine; };
+    auto place = [&](int u) __attribute__((always_inline)) {
+        int me = tid;
+        if (kPer > 1) asm volatile("" : "+v"(me));  // (addresses and products of it, kept for all steps, would push the state out)
+        return kPer == 1 ? me : (me < kOwners ? u * kOwners + me : span);
+    };  // in the workgroup's span
+    auto owns = [&](int u) __attribute__((always_inline)) { return place(u) < mine; };
     auto element = [&](int u) { return (int64_t)(e0 + (owns(u) ? place(u) : 0)) * batch + trial; };
     Sum *ring_l = reinterpret_cast<Sum *>(rb_lds);
-    unsigned *act = reinterpret_cast<unsigned *>(ring_l + (size_t)S * GLIF3_NREC * span);
+    unsigned *rows = reinterpret_cast<unsigned *>(ring_l + (size_t)S * GLIF3_NREC * span);  // [2][row_cap], a place per lane behind
+    const unsigned row_cap = ((unsigned)s.rb_list - kWave) / 2u;
     unsigned *abort_word = s.res_sync + 1;
-    unsigned *arrivals = s.res_sync + BMTK_RES_SYNC_STRIDE + way * q.sync_slots * BMTK_RES_SYNC_STRIDE;
-    constexpr int kWayStride = kRbCounters * BMTK_RES_SYNC_STRIDE;
-    unsigned long long *hist = reinterpret_cast<unsigned long long *>(s.rb_hist) + (int64_t)way * kRbHist * (q.words + 1);
+    unsigned long long *lists = reinterpret_cast<unsigned long long *>(s.res_sync + BMTK_RES_SYNC_STRIDE);
+    unsigned long long *hist = reinterpret_cast<unsigned long long *>(s.rb_hist) + (int64_t)way * kListRows * (q.words + 1);
+    auto lists_of = [&](int k) { return ListRow{lists + (k & (kListRows - 1)) * kListRowWords, way * G, G}; };
+    auto ballots_of = [&](int k) { return hist + (int64_t)(k & (kListRows - 1)) * (q.words + 1); };
     if (tid == 0) {
         go_on = rb_load(abort_word) == 0u;
-        listed[0] = listed[1] = 0u;
+        rows_l[0] = rows_l[1] = crowd_l[0] = crowd_l[1] = done_l = updated_l = listed_l = fired_n[0] = fired_n[1] = 0u;
     }
     __syncthreads();
     if (!go_on) return;
@@ -128,39 +133,102 @@ __global__ __launch_bounds__(kRbBlock) void sim_resident_batch_kernel(bmtk_glif3
         }
     __syncthreads();  // (the ring slice is there, and go_on is written again below)
 
-    auto counter_of = [&](int j) { return arrivals + (j & (q.sync_slots - 1)) * BMTK_RES_SYNC_STRIDE; };
-    auto poll = [&](int j) -> int {  // one thread: 1 = the trial's workgroups have all arrived at step j, 0 = given up
-        const unsigned *word = counter_of(j);
-        const unsigned target = (unsigned)G * ((unsigned)j / (unsigned)q.sync_slots + 1u);
-        unsigned spins = 0;
-        auto arrived = [&]() {
-            unsigned v[BMTK_RES_SYNC_WAYS], sum = 0;
+    const int n_steps = q.n_steps;
+    int slot = (int)((q.step0 - 1 + S) % S);  // of step k-1
+    const float zero[GLIF3_NREC] = {0.0f, 0.0f, 0.0f, 0.0f};
+    auto fold = [&](int at_slot) __attribute__((always_inline)) {
+        if (kPer > 1) asm volatile("" : "+s"(at_slot));
 #pragma unroll
-            for (int x = 0; x < BMTK_RES_SYNC_WAYS; ++x) v[x] = rb_load(word + x * kWayStride);
+        for (int u = 0; u < kPer; ++u) {
+            if (!owns(u)) continue;
+            Sum *cell = ring_l + (size_t)at_slot * GLIF3_NREC * span + place(u);
 #pragma unroll
-            for (int x = 0; x < BMTK_RES_SYNC_WAYS; ++x) sum += v[x];
-            return sum;
-        };
-        while (arrived() < target) {
-            if (rb_load(abort_word) != 0u) return 0;
-            if (++spins > (s.res_spin_limit ? s.res_spin_limit : kRbMaxSpin)) {
-                __hip_atomic_store(abort_word, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                return 0;
+            for (int r = 0; r < GLIF3_NREC; ++r) {
+                float a;
+                if constexpr (kFixed)
+                    a = from_fixed(cell[r * span], q.unit);
+                else
+                    a = cell[r * span];
+                cell[r * span] = (Sum)0;
+                st[u].y1[r] = st[u].y1[r] + a * p[u].psc0[r];
             }
-            __builtin_amdgcn_s_sleep(2);
         }
-        return 1;
+    };
+    auto spike_bit = [&](int k, int i) {  // (a word of the output holds several trials)
+        const int64_t e = (int64_t)i * batch + trial;
+        __hip_atomic_fetch_or(reinterpret_cast<unsigned long long *>(s.spike_bits) + (int64_t)k * s.spike_bits_stride + (e >> 6),
+                              1ull << (e & 63), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+    // fold and update of step step0 + k (the fold alone behind the last step)
+    unsigned fired = 0u;  // bit u: this thread's u-th neuron
+    auto update = [&](int k) __attribute__((always_inline)) {
+        if (k > 0) fold(slot);
+        if (k == n_steps) return;
+        float h = s.h;
+        if (kPer > 1) asm volatile("" : "+s"(h));  // (h times a neuron's propagators: not to be worked out once for all steps)
+        fired = 0u;
+#pragma unroll
+        for (int u = 0; u < kPer; ++u) {
+            if (!owns(u)) continue;
+            float frac;
+            const int ref_before = st[u].ref;
+            const bool spike = glif3_update(st[u], p[u], h, zero, I[u], &frac);
+            if (kSave) {
+                const int64_t to = ((int64_t)trial * n_steps + k) * n + e0 + place(u);
+                s.rb_save_v[to] = st[u].V;
+                s.rb_save_flags[to] = (uint8_t)((spike ? BMTK_F_SPIKE : 0) | (ref_before == 0 ? BMTK_F_INTEGRATING : 0) |
+                                                (ref_before > 0 && st[u].ref == 0 ? BMTK_F_RESET : 0));
+            }
+            if (spike) {
+                fired |= 1u << u;
+                const unsigned to = atomicAdd(&fired_n[k & 1], 1u);
+                if (to < kListMax) fired_l[to] = (unsigned short)place(u);
+            }
+        }
+    };
+    // Writer, before the workgroup meets: the list, where it holds the neurons, then their bits in the output.
+    auto write = [&](int k) __attribute__((always_inline)) {
+        ListWrite list;
+        list.read(fired_l);
+        const unsigned m = fired_n[k & 1];
+        const int i = lane_here();
+        const int id = fired_l[min((unsigned)i, kListMax)];
+        if (m <= kListMax) {
+            list.publish(lists_of(k), g, list_tag(k), m);
+            if (s.spike_bits && (unsigned)i < m) spike_bit(k, e0 + id);
+        }
+        if (lane == 0) fired_n[(k + 1) & 1] = 0u;
+    };
+    // All, behind the meeting: a volley's ballots, which have to have arrived before the list says that they are to be read.
+    auto volley = [&](int k) __attribute__((always_inline)) {
+        if (fired_n[k & 1] <= kListMax) return;
+#pragma unroll
+        for (int u = 0; u < kPer; ++u) {
+            const bool spike = (fired >> u) & 1u;
+            const unsigned long long m = __ballot(spike);
+            const int i = e0 + place(u);
+            if (lane == 0 && place(u) < span && i < n)
+                __hip_atomic_store(ballots_of(k) + (i >> 6), m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (spike && s.spike_bits) spike_bit(k, i);
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        if (wave == kRbWriter) {
+            ListWrite list;
+            list.read(fired_l);
+            list.publish(lists_of(k), g, list_tag(k), fired_n[k & 1]);
+        }
     };
 
-    // this workgroup's segment of one row, `part` of 1 << team_shift lanes, into the slots behind slot0
+    // this workgroup's segment of a row into the slots behind `slot`, lane `part` of `step`
     const int ts = s.rb_team_shift;
-    const unsigned part = (unsigned)tid & ((1u << ts) - 1u), step = 1u << ts;
     const uint32_t *__restrict__ seg = s.rb_seg + g;
     const uint2 *__restrict__ table = reinterpret_cast<const uint2 *>(s.rb_packed);
     const unsigned seg_stride = (unsigned)G + 1u;
-    auto pull_row = [&](unsigned row, unsigned q_lo, unsigned q_wrap) {
-        const RbBounds b = *reinterpret_cast<const RbBounds *>(seg + (size_t)row * seg_stride);
-        // (slot0 + delay) % slots * 4 + receptor = min(u, u - 4 * slots), u = slot0 * 4 + the record's upper byte
+    auto row_bounds = [&](unsigned row) __attribute__((always_inline)) { return *reinterpret_cast<const RbBounds *>(seg + (size_t)row * seg_stride); };
+    auto add_segment = [&](RbBounds b, unsigned part, unsigned step) __attribute__((always_inline)) {
+        const unsigned q_lo = (unsigned)slot * 4u, q_wrap = q_lo - 4u * (unsigned)S;
+        // (slot + delay) % slots * 4 + receptor = min(u, u - 4 * slots), u = slot * 4 + the record's upper byte
         auto add = [&](const uint2 sy, bool crowded) {
             const unsigned dq = sy.x >> 24;
             const unsigned plane = min(dq + q_lo, dq + q_wrap);
@@ -190,221 +258,168 @@ __global__ __launch_bounds__(kRbBlock) void sim_resident_batch_kernel(bmtk_glif3
                 if (at_p + u * step < b.hi) add(sy[u], u == 0);
         }
     };
-    // Spikes in row `hist_row` of the ballot history (-1: none) and the input events [ka, kb) of the same step, whose ring
-    // slot is slot0, into the ring slice.  All threads of the workgroup call it.  `arrival`: the counter to signal once
-    // every wavefront's ballot store has been acknowledged.
-    const int cap = s.rb_list;
-    // The same for a single wide trial, whose many ballot words would not stay in registers beside two neurons' state: each
-    // wavefront reads them kWideScan per thread at a time and takes its places in the list from a counter in LDS (`turn` tells
-    // which of two: the other is cleared on the way), so that no word outlives its turn and the workgroup meets once less.
-    constexpr int kWideScan = 4, kWideTurns = (kWords + kWideScan - 1) / kWideScan;
-    auto pull_wide = [&](int hist_row, int slot0, unsigned ka, unsigned kb, unsigned *arrival, int turn) {
-        const unsigned q_lo = (unsigned)slot0 * 4u, q_wrap = q_lo - 4u * (unsigned)S;
-        const unsigned n_ev = kb - ka;
-        unsigned base[kWideTurns];
-        // the places from `base` on of the list's window [c0, c0 + cap); the first look takes the places
-        auto list_words = [&](bool first, unsigned c0) {
-            // (not to be worked out once for all steps: that many addresses would push the state out of the registers)
-            int me = tid;
-            asm volatile("" : "+v"(me));
-#pragma unroll
-            for (int b = 0; b < kWideTurns; ++b) {
-                unsigned long long v[kWideScan];
-                unsigned cnt = 0u;
-#pragma unroll
-                for (int u = 0; u < kWideScan; ++u) {
-                    const int w = min((b * kWideScan + u) * kRbBlock + me, q.words);  // (a row's last word stays zero)
-                    v[u] = hist_row >= 0 ? __hip_atomic_load(hist + (int64_t)hist_row * (q.words + 1) + w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0ull;
-                }
-#pragma unroll
-                for (int u = 0; u < kWideScan; ++u) cnt += (unsigned)__popcll(v[u]);
-                const unsigned inc = wave_inclusive_scan(cnt);
-                if (first) {
-                    unsigned to = 0u;
-                    if (lane == kWave - 1) to = inc ? atomicAdd(&listed[turn], inc) : 0u;
-                    base[b] = (unsigned)bcast_i((int)to, kWave - 1);
-                }
-                unsigned pos = base[b] + inc - cnt - c0;  // (wraps below zero for places of an earlier window)
-#pragma unroll
-                for (int u = 0; u < kWideScan; ++u) {
-                    unsigned long long x = v[u];
-                    const unsigned j0 = (unsigned)((b * kWideScan + u) * kRbBlock + me) << 6;
-                    while (x) {
-                        const unsigned bit = (unsigned)__ffsll((long long)x) - 1u;
-                        x &= x - 1ull;
-                        if (pos < (unsigned)cap) act[pos] = j0 + bit;
-                        ++pos;
-                    }
-                }
-            }
-        };
-        // (the events first: their places are known)
-        for (unsigned k = (unsigned)tid; k < n_ev && k < (unsigned)cap; k += kRbBlock) act[k] = (unsigned)n + (unsigned)s.rb_in_events[ka + k];
-        if (tid == 0) listed[turn ^ 1] = 0u;
-#pragma unroll
-        for (int b = 0; b < kWideTurns; ++b) base[b] = 0u;
-        list_words(true, 0u - n_ev);
-        if (arrival) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
-        if (arrival && tid == 0) __hip_atomic_fetch_add(arrival, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const unsigned total = listed[turn] + n_ev;
-        for (unsigned c0 = 0;;) {
-            const unsigned here = min(total - c0, (unsigned)cap);
-            for (unsigned a = (unsigned)tid >> ts; a < here; a += (unsigned)kRbBlock >> ts) pull_row(act[a], q_lo, q_wrap);
-            __syncthreads();
-            c0 += (unsigned)cap;
-            if (c0 >= total) break;
-            // (a volley outgrows the list: the next window of it)
-            for (unsigned k = (unsigned)tid; k < n_ev; k += kRbBlock)
-                if (k - c0 < (unsigned)cap) act[k - c0] = (unsigned)n + (unsigned)s.rb_in_events[ka + k];
-            list_words(false, c0 - n_ev);
-            __syncthreads();
+    // The rows of round k: what fired in step k-1, and the input events handed over with it.  Where they are listed before the
+    // update of step k (`ask` ahead of it), the bounds of a thread's first row are on their way meanwhile.
+    unsigned n_rows = 0u, at_row = 0u;
+    RbBounds first_row{0u, 0u};
+    auto ask = [&](int k) __attribute__((always_inline)) {
+        unsigned me = (unsigned)tid;
+        asm volatile("" : "+v"(me));
+        n_rows = (unsigned)__builtin_amdgcn_readfirstlane((int)rows_l[k & 1]);
+        if (n_rows == kCrowded || wave == kRbWriter) n_rows = 0u;
+        at_row = me >> ts;
+        if (at_row < n_rows) first_row = row_bounds(rows[(k & 1) * row_cap + at_row]);
+    };
+    auto pull = [&](int k) __attribute__((always_inline)) {
+        const unsigned part = (unsigned)lane & ((1u << ts) - 1u);
+        while (at_row < n_rows) {
+            const RbBounds b = first_row;
+            at_row += (unsigned)kRbPullThreads >> ts;
+            if (at_row < n_rows) first_row = row_bounds(rows[(k & 1) * row_cap + at_row]);
+            add_segment(b, part, 1u << ts);
         }
     };
-    auto pull = [&](int hist_row, int slot0, unsigned ka, unsigned kb, unsigned *arrival) {
-        const unsigned q_lo = (unsigned)slot0 * 4u, q_wrap = q_lo - 4u * (unsigned)S;
-        unsigned long long v[kWords];
-        unsigned cnt = 0u;
-#pragma unroll
-        for (int u = 0; u < kWords; ++u) {
-            // (the last word of a row is never written: it stays zero)
-            const int w = min(u * kRbBlock + tid, q.words);
-            v[u] = hist_row >= 0 ? __hip_atomic_load(hist + (int64_t)hist_row * (q.words + 1) + w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0ull;
-        }
-        const unsigned n_ev = kb - ka;
-        const unsigned ev = (unsigned)tid < n_ev ? (unsigned)s.rb_in_events[ka + tid] : 0u;
-#pragma unroll
-        for (int u = 0; u < kWords; ++u) cnt += (unsigned)__popcll(v[u]);
-        const unsigned inc = wave_inclusive_scan(cnt);
-        if (lane == kWave - 1) scan_l[wave] = inc;
-        if (arrival) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    // the input events of round k: rb_in_events[in_ptr[k] .. in_ptr[k + 1])
+    const int64_t *in_ptr = q.has_events ? s.rb_in_ptr + (int64_t)trial * (n_steps + 1) : nullptr;
+    // (a call's first step: the spikes of the step before were added by the call before it, and so were its events unless
+    //  they are to be taken from this call's lists)
+    auto with_events = [&](int k) { return in_ptr && (k > 0 || s.rb_late_events); };
+    auto pull_crowded = [&](int k) __attribute__((always_inline)) {
+        const unsigned lo = with_events(k) ? (unsigned)in_ptr[k] : 0u, hi = with_events(k) ? (unsigned)in_ptr[k + 1] : 0u;
+        const unsigned cap = (unsigned)s.rb_list;
+        auto pull_row = [&](unsigned row) __attribute__((always_inline)) { add_segment(row_bounds(row), 0u, 1u); };
+        crowded_rows<kPer == 1 ? 4 : 8>(lists_of(k - 1), k > 0, span, ballots_of(k - 1), q.words, hi - lo, rows, cap, &crowd_l[k & 1],
+                                        abort_word, kRbMaxSpin, [&](unsigned i) { return (unsigned)n + (unsigned)s.rb_in_events[lo + i]; },
+                                        pull_row);
         __syncthreads();
-        if (arrival && tid == 0) __hip_atomic_fetch_add(arrival, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const unsigned parts = wave_inclusive_scan(lane < kRbWaves ? scan_l[lane] : 0u);
-        const unsigned n_spk = (unsigned)bcast_i((int)parts, kRbWaves - 1);
-        const unsigned base = wave > 0 ? (unsigned)__shfl((int)parts, wave - 1, kWave) : 0u;
-        const unsigned total = n_spk + n_ev;
-        for (unsigned c0 = 0; c0 < total; c0 += (unsigned)cap) {  // (one round unless a volley outgrows the list)
-            unsigned pos = base + inc - cnt - c0;  // (wraps below zero for places of an earlier round)
-#pragma unroll
-            for (int u = 0; u < kWords; ++u) {
-                unsigned long long x = v[u];
-                const unsigned j0 = (unsigned)(u * kRbBlock + tid) << 6;
-                while (x) {
-                    const unsigned bit = (unsigned)__ffsll((long long)x) - 1u;
-                    x &= x - 1ull;
-                    if (pos < (unsigned)cap) act[pos] = j0 + bit;
-                    ++pos;
-                }
-            }
-            for (unsigned k = (unsigned)tid; k < n_ev; k += kRbBlock) {
-                const unsigned to = n_spk + k - c0;
-                if (to < (unsigned)cap) act[to] = (unsigned)n + (k == (unsigned)tid ? ev : (unsigned)s.rb_in_events[ka + k]);
-            }
-            __syncthreads();
-            const unsigned here = min(total - c0, (unsigned)cap);
-            for (unsigned a = (unsigned)tid >> ts; a < here; a += (unsigned)kRbBlock >> ts) pull_row(act[a], q_lo, q_wrap);
-            __syncthreads();
-        }
+        const unsigned total = min(crowd_l[k & 1], cap);
+        for (unsigned a = (unsigned)tid >> ts; a < total; a += (unsigned)kRbBlock >> ts)
+            add_segment(row_bounds(rows[a]), (unsigned)lane & ((1u << ts) - 1u), 1u << ts);
+        __syncthreads();
     };
-    auto fold = [&](int slot) {
-        if (kPer > 1) asm volatile("" : "+s"(slot));
-#pragma unroll
-        for (int u = 0; u < kPer; ++u) {
-            if (!owns(u)) continue;
-            Sum *cell = ring_l + (size_t)slot * GLIF3_NREC * span + place(u);
-#pragma unroll
-            for (int r = 0; r < GLIF3_NREC; ++r) {
-                float a;
-                if constexpr (kFixed)
-                    a = from_fixed(cell[r * span], q.unit);
-                else
-                    a = cell[r * span];
-                cell[r * span] = (Sum)0;
-                st[u].y1[r] = st[u].y1[r] + a * p[u].psc0[r];
-            }
-        }
+    // the pulls of round k are complete
+    auto pulled = [&](int k) __attribute__((always_inline)) {
+        while ((int)(load_lds(&done_l) - (unsigned)(k + 1) * kRbWriter) < 0) {}
     };
 
-    // the input events of the call's steps, trial by trial: those of step step0 - 1 + k are rb_in_events[in_ptr[k], in_ptr[k+1])
-    const int64_t *in_ptr = q.has_events ? s.rb_in_ptr + (int64_t)trial * (q.n_steps + 1) : nullptr;
-    int opaque_zero;
-    asm volatile("v_mov_b32 %0, 0" : "=v"(opaque_zero));
-    constexpr int kLooker = kRbBlock - kWave;  // its wavefront owns no neurons at spans up to 960, or with two to a thread
-    const float zero[GLIF3_NREC] = {0.0f, 0.0f, 0.0f, 0.0f};
-    unsigned ka = 0u, kb = 0u;
-    if (in_ptr) {
-        ka = (unsigned)in_ptr[0];
-        kb = (unsigned)in_ptr[1];
-    }
-    int slot = (int)((q.step0 - 1 + S) % S);  // of step t-1
-    const int n_steps = q.n_steps;
+    auto store = [&]() __attribute__((always_inline)) {
+        int64_t all = ne;
+        asm volatile("" : "+s"(all));  // (its addresses are not those of the loads, kept all along)
+#pragma unroll
+        for (int u = 0; u < kPer; ++u)
+            if (owns(u)) glif3_store(st[u], s.V, s.asc, s.y1, s.y2, s.ref, all, element(u));
+    };
+
     bool aborted = false;
-    for (int k = 0; k < n_steps; ++k) {
-        // the bound of the next step's events: asked for here, looked at after the pull (see resident.hip)
-        unsigned kn = 0u;
-        if (in_ptr) kn = (unsigned)in_ptr[k + 2 + opaque_zero];
-        if (k > 0 && tid == kLooker) go_on = poll(k - 1);
-        if (k > 0) fold(slot);
-        float h = s.h;
-        if (kPer > 1) asm volatile("" : "+s"(h));  // (nor h times a neuron's propagators)
-#pragma unroll
-        for (int u = 0; u < kPer; ++u) {
-            bool spike = false;
-            float frac;
-            const int ref_before = st[u].ref;
-            if (owns(u)) spike = glif3_update(st[u], p[u], h, zero, I[u], &frac);
-            const unsigned long long m = __ballot(spike);
-            const int i = e0 + place(u);
-            if (lane == 0 && place(u) < span && i < n)
-                __hip_atomic_store(hist + (int64_t)(k & (kRbHist - 1)) * (q.words + 1) + (i >> 6), m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (kSave && owns(u)) {
-                const int64_t to = ((int64_t)trial * n_steps + k) * n + i;
-                s.rb_save_v[to] = st[u].V;
-                s.rb_save_flags[to] = (uint8_t)((spike ? BMTK_F_SPIKE : 0) | (ref_before == 0 ? BMTK_F_INTEGRATING : 0) |
-                                                (ref_before > 0 && st[u].ref == 0 ? BMTK_F_RESET : 0));
+    if (wave != kRbReader) {
+        for (int k = 0; k <= n_steps; ++k) {  // (one round more than steps: the closing pull)
+            const bool asked = kPer == 1 && load_lds(&listed_l) == (unsigned)k + 1u;  // (two neurons leave no registers for it)
+            if (asked) ask(k);
+            update(k);
+            if (wave != kRbWriter) {
+                count_lds(&updated_l);
+            } else if (k < n_steps) {
+                const unsigned all = (unsigned)(k + 1) * (kReaderOwns ? kRbReader : kRbWriter);
+                while ((int)(load_lds(&updated_l) - all) < 0) {}
+                write(k);
             }
-            if (spike && s.spike_bits) {
-                const int64_t e = element(u);
-                __hip_atomic_fetch_or(reinterpret_cast<unsigned long long *>(s.spike_bits) + (int64_t)k * s.spike_bits_stride + (e >> 6),
-                                      1ull << (e & 63), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __syncthreads();  // the workgroup meets: every slot k-1 is folded, the rows of the round are there
+            if (!go_on) {
+                aborted = true;
+                break;
             }
+            if (k < n_steps) volley(k);
+            if (!asked) ask(k);
+            if (rows_l[k & 1] == kCrowded)
+                pull_crowded(k);
+            else
+                pull(k);
+            slot = slot + 1 == S ? 0 : slot + 1;
+            if (wave != kRbWriter) count_lds(&done_l);
+            pulled(k);
         }
-        __syncthreads();
-        if (k > 0 && !go_on) {
-            aborted = true;
-            break;
-        }
-        // (a call's first step: the spikes of the step before were added by the call before it, and so were its events unless
-        //  they are to be taken from this call's lists)
-        const bool with_events = k > 0 || s.rb_late_events;
-        unsigned *const arrival = counter_of(k) + (g & (BMTK_RES_SYNC_WAYS - 1)) * kWayStride;
-        if constexpr (kPer > 1)
-            pull_wide(k > 0 ? (k - 1) & (kRbHist - 1) : -1, slot, ka, with_events ? kb : ka, arrival, k & 1);
-        else
-            pull(k > 0 ? (k - 1) & (kRbHist - 1) : -1, slot, ka, with_events ? kb : ka, arrival);
-        ka = kb;
-        kb = (unsigned)__builtin_amdgcn_readfirstlane((int)kn);
-        slot = slot + 1 == S ? 0 : slot + 1;
-    }
-    if (!aborted) {
-        if (tid == 0) go_on = poll(n_steps - 1);
-        __syncthreads();
-        aborted = go_on == 0;
-    }
-    if (!aborted) {
-        // closing: what arrived in the last step, then the spikes (and events) of the last step
-        fold(slot);
-        __syncthreads();
-        if constexpr (kPer > 1)
-            pull_wide((n_steps - 1) & (kRbHist - 1), slot, ka, kb, nullptr, n_steps & 1);
-        else
-            pull((n_steps - 1) & (kRbHist - 1), slot, ka, kb, nullptr);
-        __syncthreads();
-    }
+        store();
+    } else {
+        ListLook seen;
+        bool lost = false;  // given up
+        unsigned failed = 0u;
+        int opaque_zero;
+        asm volatile("v_mov_b32 %0, 0" : "=v"(opaque_zero));
+        // the input events of the round in hand, the first of them on their way
+        unsigned ev_lo = with_events(0) ? (unsigned)in_ptr[0] : 0u, ev_hi = with_events(0) ? (unsigned)in_ptr[1] : 0u;
+        unsigned next_lo = 0u, next_hi = 0u;
+        if (in_ptr) next_lo = (unsigned)in_ptr[1], next_hi = (unsigned)in_ptr[min(2, n_steps + 1)];
+        int32_t ev[kRbEvents] = {0, 0, 0, 0};
+        auto ask_events = [&]() __attribute__((always_inline)) {
+            const unsigned n_ev = ev_hi - ev_lo, me = (unsigned)lane_here();
+            const int32_t *const from = s.rb_in_events + ev_lo;
 #pragma unroll
-    for (int u = 0; u < kPer; ++u)
-        if (owns(u)) glif3_store(st[u], s.V, s.asc, s.y1, s.y2, s.ref, ne, element(u));
+            for (int i = 0; i < kRbEvents; ++i)
+                if (i * kWave + me < n_ev) ev[i] = from[i * kWave + me];
+        };
+        ask_events();
+        // one more look in vain: false when it is time to give up
+        auto again = [&]() __attribute__((always_inline)) -> bool {
+            const unsigned limit = s.res_spin_limit ? s.res_spin_limit : kRbMaxSpin;
+            if (++failed > limit) __hip_atomic_store(abort_word, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            return failed <= limit && rb_load(abort_word) == 0u;
+        };
+        for (int k = 0; k <= n_steps; ++k) {
+            if (kReaderOwns) {
+                if (k > 0) pulled(k - 1);
+                update(k);
+                count_lds(&updated_l);
+            }
+            seen.none();
+            failed = 0u;
+            if (k > 0) {
+                __builtin_amdgcn_s_sleep(8);  // (see resident.hip)
+                while (!lost && !seen.look<kPer == 1>(lists_of(k - 1), list_tag(k - 1))) lost = !again();
+            }
+            if (!lost) {
+                const unsigned me = (unsigned)lane_here(), spare = 2u * row_cap + me, to = (unsigned)(k & 1) * row_cap, n_ev = ev_hi - ev_lo;
+                const unsigned total = rows_from_lists<kPer == 1>(seen, lists_of(k - 1), list_tag(k - 1), span, rows, to, row_cap, spare, n_ev, again, lost);
+                if (total != kCrowded) {
+#pragma unroll
+                    for (int i = 0; i < kRbEvents; ++i) {
+                        if ((unsigned)(i * kWave) >= n_ev) break;
+                        const unsigned a = i * kWave + me;
+                        int32_t source = ev[i];
+                        asm volatile("" : "+v"(source));  // (not looked at ahead of the lists)
+                        rows[a < n_ev ? to + total + a : spare] = (unsigned)n + (unsigned)source;
+                    }
+                    for (unsigned a = kRbEvents * kWave + me; a < n_ev; a += kWave) rows[to + total + a] = (unsigned)n + (unsigned)s.rb_in_events[ev_lo + a];
+                }
+                if (lane == 0) {
+                    rows_l[k & 1] = total == kCrowded ? kCrowded : total + n_ev;
+                    crowd_l[k & 1] = 0u;
+                    if (!lost) store_lds(&listed_l, (unsigned)k + 1u);
+                }
+            }
+            if (lane == 0) go_on = !lost;
+            // vmcnt(0): nothing is on its way here, and with that said the compiler does not wait for loads below before it
+            // uses their registers again
+            __builtin_amdgcn_s_waitcnt(0x0F70);
+            ev_lo = next_lo;
+            ev_hi = (unsigned)__builtin_amdgcn_readfirstlane((int)next_hi);
+            __syncthreads();
+            if (!go_on) {
+                aborted = true;
+                break;
+            }
+            if (in_ptr) {
+                next_lo = ev_hi;
+                next_hi = (unsigned)in_ptr[min(k + 3, n_steps + 1) + opaque_zero];
+                if (k < n_steps) ask_events();
+            }
+            if (k < n_steps) volley(k);
+            if (rows_l[k & 1] == kCrowded) pull_crowded(k);
+            slot = slot + 1 == S ? 0 : slot + 1;
+        }
+        if (kReaderOwns && !aborted) pulled(n_steps);
+        if (kReaderOwns) store();
+    }
+    __syncthreads();
     for (int c = tid; c < S * GLIF3_NREC * span; c += kRbBlock) {
         const int plane = c / span, k = c - plane * span;
         if (k < mine) ring_g[(int64_t)plane * n + k] = ring_l[c];
@@ -435,12 +450,6 @@ __global__ __launch_bounds__(kBlock) void by_step_kernel(const float *__restrict
         out_v[to + c] = v_l[b * kByStepPitch + j];
         out_flags[to + c] = flags_l[b * kByStepPitch + j];
     }
-}
-
-// arrival counters of a launch back to zero (the abort word stays until the host has seen it)
-__global__ void rb_zero_sync_kernel(unsigned *sync)
-{
-    for (int c = threadIdx.x; c < BMTK_RES_SYNC_WAYS * kRbCounters; c += blockDim.x) sync[(1 + c) * BMTK_RES_SYNC_STRIDE] = 0u;
 }
 
 __global__ __launch_bounds__(kBlock) void rb_zero_bits_kernel(uint64_t *__restrict__ bits, int64_t n)
@@ -502,15 +511,13 @@ int simulate_resident_batch(const bmtk_glif3_sim &s, int64_t step0, int64_t n_st
     q.words = (int)((n + kWave - 1) / kWave);
     q.has_events = s.rb_in_ptr != nullptr;
     q.unit = ldexp(1.0, -32 - s.sum_shift);
-    q.sync_slots = kRbCounters;
-    while (q.sync_slots * W > kRbCounters) q.sync_slots /= 2;
-    BMTK_REQUIRE(q.words <= (wide ? kRbWideWords : 4) * kRbBlock, "glif3_simulate_fwd: more neurons than resident trials can hold");
-    const bool few = q.words <= kRbBlock;
-    const void *kernel = wide ? reinterpret_cast<const void *>(sim_resident_batch_kernel<kRbWideWords, 2, float, false>)
-        : few ? (save ? reinterpret_cast<const void *>(sim_resident_batch_kernel<1, 1, unsigned long long, true>)
-                      : reinterpret_cast<const void *>(sim_resident_batch_kernel<1, 1, unsigned long long, false>))
-              : (save ? reinterpret_cast<const void *>(sim_resident_batch_kernel<4, 1, unsigned long long, true>)
-                      : reinterpret_cast<const void *>(sim_resident_batch_kernel<4, 1, unsigned long long, false>));
+    BMTK_REQUIRE((wide ? 2 * kRbReader * kWave : kRbBlock) * (int64_t)kListGroups >= n, "glif3_simulate_fwd: more neurons than resident trials can hold");
+    const bool owns = span > kRbReader * kWave;
+    const void *kernel = wide ? reinterpret_cast<const void *>(sim_resident_batch_kernel<2, float, false, false>)
+        : owns ? (save ? reinterpret_cast<const void *>(sim_resident_batch_kernel<1, unsigned long long, true, true>)
+                       : reinterpret_cast<const void *>(sim_resident_batch_kernel<1, unsigned long long, false, true>))
+               : (save ? reinterpret_cast<const void *>(sim_resident_batch_kernel<1, unsigned long long, true, false>)
+                       : reinterpret_cast<const void *>(sim_resident_batch_kernel<1, unsigned long long, false, false>));
     hipError_t err = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (err != hipSuccess) {
         set_error("glif3_simulate_fwd: resident trials need %zu bytes of LDS: %s", lds, hipGetErrorString(err));
@@ -525,6 +532,7 @@ int simulate_resident_batch(const bmtk_glif3_sim &s, int64_t step0, int64_t n_st
         set_error("glif3_simulate_fwd: %u resident workgroups do not fit the device (%d compute units x %d)", grid, n_cu, per_cu);
         return BMTK_E_LAUNCH;
     }
+    BMTK_REQUIRE(W * G <= kListGroups, "glif3_simulate_fwd: a launch of resident trials has at most 256 workgroups");
     if (s.spike_bits) {
         // (a spike is one bit in a word its trials share)
         const int64_t words = n_steps * s.spike_bits_stride, blocks = (words + kBlock - 1) / kBlock;
@@ -534,7 +542,10 @@ int simulate_resident_batch(const bmtk_glif3_sim &s, int64_t step0, int64_t n_st
     for (int trial0 = 0; trial0 < batch; trial0 += W) {
         q.trial0 = trial0;
         q.trials = batch - trial0 < W ? batch - trial0 : W;
-        hipLaunchKernelGGL(rb_zero_sync_kernel, dim3(1), dim3(kBlock), 0, stream, s.res_sync);
+        // the lists of the launch before back to no step's
+        const int64_t list_words = (int64_t)kListRows * kListRowWords;
+        hipLaunchKernelGGL(rb_zero_bits_kernel, dim3((unsigned)((list_words + kBlock - 1) / kBlock)), dim3(kBlock), 0, stream,
+                           reinterpret_cast<uint64_t *>(s.res_sync + BMTK_RES_SYNC_STRIDE), list_words);
         bmtk_glif3_sim copy = s;
         RbLaunch launch = q;
         void *args[] = {&copy, &launch};

@@ -500,12 +500,12 @@ class Glif3Simulator:
         """Fill ``s`` for a call in the form with resident trials.  Returns what has to live until it is launched."""
         tr = self._trials
         s.rb_span, s.rb_groups, s.rb_ways, s.rb_list = tr["span"], tr["groups"], tr["ways"], tr["list"]
-        # as many lanes to a segment as let the workgroup's 1024 take the rows of a step in one go, or in little more
-        # (5,000 neurons x 16 trials, some 20 rows of 21 synapses: 6.5 / 3.5 / 2.8 us per step with 1 / 4 / 32 lanes; 51,978 x 32, 220
-        # of 14: 60 / 38 / 50 / 69 with 1 / 4 / 16 / 32; 230,924 x 8, 1,000 rows of 1.4: one)
+        # as many lanes to a segment as let the workgroup's 896 that pull take the rows of a step in one go (51,978 x 32, 243 rows
+        # of 18 synapses: 47 / 40 / 42 us per step with 1 / 2 / 4 lanes; 20,011 x 20, 85 of 33: 10.6 / 9.3 / 9.5 with 4 / 8 / 16;
+        # 230,924 x 8, 780 rows of 1.4: one)
         events = self.in_events.numel() / float(max(1, self.in_steps) * self.batch) if self.in_ptr is not None else 0.0
         rows = max(1.0, self.n * self.expected_rate_hz * 1e-3 * self.h + events)
-        s.rb_team_shift = max(0, min(tr["max_team_shift"], int(math.log2(max(1.0, 1500.0 / rows)))))
+        s.rb_team_shift = max(0, min(tr["max_team_shift"], int(math.log2(max(1.0, 900.0 / rows)))))
         s.rb_late_events = 1 if self.fuse_rereads else 0
         s.rb_seg, s.rb_packed, s.rb_ring, s.rb_hist = _p(tr["seg"]), _p(tr["packed"]), _p(tr["ring"]), _p(tr["hist"])
         s.res_sync, s.res_spin_limit = _p(self.res_sync), int(self.spin_limit)

@@ -9,7 +9,7 @@ from bmtk_amd import simulator, synthetic
 from bmtk_amd.layout import PAR
 
 pytestmark = pytest.mark.gpu
-N, STEPS = 3000, 60
+N, STEPS = 3000, 70
 
 
 def _network(seed):
@@ -74,6 +74,38 @@ def test_lists_at_their_edges_equal_per_step_launches(span, form, monkeypatch):
         assert int(want["bits"].ne(0).sum()) > 50
         for key in want:
             assert torch.equal(want[key], got[key]), (seed, key)
+
+
+@pytest.mark.parametrize("span,places,save", [(64, 2000, False), (64, 64, False), (832, 700, True), (960, 2000, False), (1024, 2000, True),
+                                              (1024, 64, False)])
+def test_lists_of_trials_side_by_side_at_their_edges(span, places, save, monkeypatch):
+    """The same in the form with resident trials, five of them two at a time; `places` 64 leaves the row list no room at all."""
+    batch = 5
+    par, rec, inp, ptr, events = _network(3)
+    rec, inp = [t[:3] + (np.minimum(t[3], 4),) + t[4:] for t in (rec, inp)]
+    rng = np.random.default_rng(4)
+    by_step = [np.sort(events[a:b] * batch + rng.integers(0, batch, b - a)).astype(np.int32) for a, b in zip(ptr[:-1], ptr[1:])]
+    u = np.stack([_start(par, span, seed) for seed in (0, 5, 8, 12, 14)], axis=1).reshape(-1)
+    groups = -(-N // span)
+
+    def run(trials):
+        monkeypatch.setattr(simulator, "resident_trials_plan", lambda *a: dict(span=span, groups=groups, ways=2, passes=3, list=places))
+        sim = simulator.Glif3Simulator(N, par, 1.0, batch=batch, rec=rec, inp=inp, resident=False, resident_trials=trials)
+        sim.state.V.copy_(torch.as_tensor(u))
+        sim.set_input_events(ptr, np.concatenate(by_step))
+        out = [sim.run(k, save_state=save) for k in (33, STEPS - 33)]
+        st = sim.state
+        got = dict(bits=torch.cat([o["bits"] for o in out]), V=st.V, y1=st.y1, y2=st.y2, asc=st.asc, ref=st.ref)
+        if save:
+            got.update(v=torch.cat([o["saved"]["v"] for o in out]), flags=torch.cat([o["saved"]["flags"] for o in out]))
+        sim.check()
+        assert (sim._trials is not None) == trials
+        return got
+
+    want, got = run(False), run(True)
+    assert int(want["bits"].ne(0).sum()) > 50
+    for key in want:
+        assert torch.equal(want[key], got[key]), key
 
 
 def test_a_reader_gives_up_cleanly(monkeypatch):
