@@ -377,23 +377,31 @@ def bin_spike_times(trains, dt, n_steps, batch=1, trial=0):
     ``static_synapse`` delivery) and is emitted in step stamp-1.  An event is
     the element id ``source*batch + trial``; events of one step are ascending.
     """
-    steps, elems = [], []
-    for j, st in enumerate(trains):
-        st = check_spike_times(st)
-        if st is None:
-            continue
-        stamp = np.ceil(st / dt - 1e-6).astype(np.int64)
-        stamp = np.maximum(stamp, 1)
-        emit = stamp - 1
-        emit = emit[emit < n_steps]
-        steps.append(emit)
-        elems.append(np.full(emit.size, j * batch + trial, np.int64))
-    if steps:
-        steps, elems = np.concatenate(steps), np.concatenate(elems)
+    # all trains at once: a run script has a train per virtual cell, and three array operations on each cost 5 ms per thousand
+    trains = list(trains)
+    used = [j for j, st in enumerate(trains) if st is not None and len(st)]
+    try:
+        times = [np.asarray(trains[j], np.float64).ravel() for j in used]
+        bad = any(t.min() <= 0.0 for t in times if t.size) if used else False   # (a NaN is not)
+    except (TypeError, ValueError):
+        bad = True
+    if bad or any(np.isnan(t).any() for t in times):
+        for st in trains:
+            check_spike_times(st)       # raises for the first train that is not valid
+        times = [np.asarray(trains[j], np.float64).ravel() for j in used]
+    times_all = np.concatenate(times) if times else np.zeros(0)
+    stamp = np.maximum(np.ceil(times_all / dt - 1e-6).astype(np.int64), 1)
+    elems = np.repeat(np.asarray(used, np.int64) * batch + trial, [t.size for t in times])
+    steps = stamp - 1
+    early = steps < n_steps
+    steps, elems = steps[early], elems[early]
+    stride = int(elems.max()) + 1 if elems.size else 1
+    if elems.size and 0 <= int(elems.min()) and n_steps * stride < 2 ** 62:
+        key = np.sort(steps * stride + elems)
+        steps, elems = key // stride, key % stride
     else:
-        steps, elems = np.zeros(0, np.int64), np.zeros(0, np.int64)
-    order = np.lexsort((elems, steps))
-    steps, elems = steps[order], elems[order]
+        order = np.lexsort((elems, steps))
+        steps, elems = steps[order], elems[order]
     in_ptr = np.zeros(n_steps + 1, np.int64)
-    np.add.at(in_ptr, steps + 1, 1)
-    return np.cumsum(in_ptr), elems.astype(np.int32)
+    in_ptr[1:] = np.cumsum(np.bincount(steps, minlength=n_steps)[:n_steps])
+    return in_ptr, elems.astype(np.int32)

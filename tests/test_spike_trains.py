@@ -168,3 +168,26 @@ def test_gamma_generator_draws_and_statistics():
         g.add(node_ids=[0], firing_rate=5.0, a=-1.0)
     with pytest.raises(ValueError):
         g.add(node_ids=[0], firing_rate=5.0, a=2.0, times=(2.0, 1.0))
+
+
+@pytest.mark.parametrize("seed", range(8))
+def test_binning_all_trains_at_once_equals_one_by_one(seed):
+    rng = np.random.default_rng(seed)
+    trains = [None if rng.random() < 0.2 else rng.uniform(0.01, 60, rng.integers(0, 9)) for _ in range(rng.integers(0, 40))]
+    trains = [t.tolist() if t is not None and rng.random() < 0.3 else t for t in trains]
+    dt, n_steps, batch, trial = float(rng.choice([0.1, 0.25, 1.0])), int(rng.integers(1, 90)), 3, 2
+    in_ptr, ev = bin_spike_times(trains, dt, n_steps, batch=batch, trial=trial)
+    want = [[] for _ in range(n_steps)]
+    for j, st in enumerate(trains):
+        st = check_spike_times(st)
+        for t in [] if st is None else st:
+            step = max(int(np.ceil(t / dt - 1e-6)), 1) - 1
+            if step < n_steps:
+                want[step].append(j * batch + trial)
+    assert in_ptr.dtype == np.int64 and ev.dtype == np.int32 and in_ptr.size == n_steps + 1
+    assert [ev[in_ptr[k]:in_ptr[k + 1]].tolist() for k in range(n_steps)] == [sorted(w) for w in want]
+
+
+def test_the_first_train_that_is_not_valid_is_named():
+    with pytest.raises(ValueError, match=r"\[0\. 2\.\]"):
+        bin_spike_times([[1.0], [0.0, 2.0], [-1.0]], 1.0, 5)
