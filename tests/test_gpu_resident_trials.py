@@ -378,3 +378,13 @@ def test_what_does_not_fit_is_refused():
     cfg, _, _ = _case(200, 2, 3)
     with pytest.raises(ValueError):
         Glif3Simulator(cfg["n"], cfg["par"], 1.0, batch=2, inp=cfg["inp_src"], resident=False, resident_trials=True)
+
+
+def test_training_simulators_take_resident_trials_where_they_pay():
+    """resident=False of a batch: the form with resident trials by itself, the per-step drivers for a short call and on request."""
+    batch = 12
+    cfg, _, _ = _case(700, batch, 3)
+    for kw, steps, trials in ((dict(), 64, True), (dict(), 20, False), (dict(resident_trials=False), 64, False)):
+        sim = _sim(cfg, batch, **kw)
+        sim.run(steps, save_state=True)
+        assert (sim._trials is not None) == trials
