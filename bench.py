@@ -509,7 +509,7 @@ def bench_front_end(torch, sim, steps):
     times, senders = sim.to_host(rec["time"], rec["elem"])
     collect = time.perf_counter() - t0
     alg_step = N_V1 * B_PER_UPDATE_CLASS   # the state update alone; the events ride on top as in the headline
-    out = [{"kernel": "sim_resident_kernel (spike record on) + collect_record",
+    out = [{"kernel": "sim_resident_lists_kernel (spike record on) + collect_record",
             "workload": "V1-scale forward simulation as the front ends run it, %d steps" % steps,
             "us_per_sim_step": dev / steps * 1e6, "neuron_updates_per_s": N_V1 * steps / wall,
             "spikes": int(times.size), "record_overflow": bool(rec["overflow"]),
@@ -731,7 +731,7 @@ def main():
     events = rec_ev + in_ev
     total_steps = K * S
     resident = bool(sim.res_span)
-    # resident mode: every pass is ONE launch of sim_resident_kernel covering its S steps;
+    # resident mode: every pass is ONE launch of sim_resident_lists_kernel covering its S steps;
     # otherwise S+1 launches of sim_step_kernel per pass
     launches = K if resident else K * (S + 1)
     per_launch = dev / launches
@@ -760,7 +760,7 @@ def main():
                    "events_per_sim_step": events / total_steps, "us_per_sim_step": wall / total_steps * 1e6,
                    "input_weight_scale": IN_W_SCALE,
                    "same_network_at_input_weight_x1": unscaled_activity(torch)},
-        "roofline": {"bound": "hbm", "kernel": "sim_resident_kernel" if resident else "sim_step_kernel",
+        "roofline": {"bound": "hbm", "kernel": "sim_resident_lists_kernel" if resident else "sim_step_kernel",
                      "achieved": alg / per_launch / 1e9, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": alg / per_launch / 1e9 / HBM_PEAK_GBS,
                      "traffic": None if traffic_step is None else traffic_step * total_steps / launches,
