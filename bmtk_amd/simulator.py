@@ -36,7 +36,7 @@ PUSH_PS_PER_EVENT = 48.0
 # little per event.  Measured, us per step trials / fused / pushed (neurons x trials, in-degree): 51,978 x 32, 1154: 38 / 95 / - ;
 # 20,011 x 20, 820: 8.3 / 31 / - ; 230,924 x 8, 335: 59 / 134 / 164; 5,000 x 16, 400: 2.8 / 9.8 / - ; 31,000 x 64, 160: 36 / 38 / 87;
 # 120,000 x 16, 150: 41 / 52 / 82; 100,000 x 4, 260: 10 / - / 28; 2,000 x 40, 200: 3.3 / 6.3 / 11.5; 3,000 x 4, 200: 2.7 / - / 11.5;
-# 400,123 x 1, 180: 9.8 / - / 25.4.
+# 400,123 x 1, 180: 9.8 / - / 25.4.  (Fitted with a grid barrier per trial; with lists the first figures are up to a third lower.)
 TRIALS_PS_PER_PASS = 3.0e6
 TRIALS_PS_PER_ROW = 6.5e3       # per neuron of ONE trial that fires in a step (and the input events that come with it)
 TRIALS_PS_PER_EVENT = 0.8
@@ -53,7 +53,7 @@ RES_LDS_EXTRA = RES_ACT_ENTRIES * 4 + 256   # the list plus the kernel's static 
 SOLO_LDS_PER_ELEMENT = 4 * 4
 SOLO_LDS_EXTRA = 10240 + 2048
 RB_WIDE_SPAN = 1920             # neurons of a workgroup at most with two to a thread
-RB_LIST_MIN, RB_LDS_STATIC = 2000, 256   # the form with resident trials: least room for its list of rows, static LDS
+RB_LIST_MIN, RB_LDS_STATIC = 2000, 256   # the form with resident trials: least room (words) for its lists of rows, static LDS
 SUM_SHIFT_MAX = 120             # BMTK_SUM_SHIFT_MAX
 TRIALS_TABLE_BYTES = 1 << 30    # tables and ring of the form with resident trials at most, or TRIALS_TABLE_RATIO times the synapses' 10 bytes
 TRIALS_TABLE_RATIO = 4

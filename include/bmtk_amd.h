@@ -390,7 +390,8 @@ typedef struct bmtk_glif3_sim {
     int32_t rb_groups;
     int32_t rb_ways;                   /* trials of a launch: rb_ways * rb_groups workgroups must be resident at once */
     int32_t rb_team_shift;             /* 2^rb_team_shift lanes read a row's segment */
-    int32_t rb_list;                   /* places of the list of rows in LDS; (ring_slots-1)*32*rb_span (one trial: *16) + 4*rb_list
+    int32_t rb_list;                   /* words of LDS for the rows of two steps, at least 64 (a step with more than (rb_list - 64) / 2
+                                        * rows takes longer); (ring_slots-1)*32*rb_span (one trial: *16) + 4*rb_list
                                         * + 256 bytes of LDS */
     int32_t rb_late_events;            /* the input events of a call's last step (each id once; repeats are delivered at once) are
                                         * left to the next call and its lists, as with in_again */
