@@ -332,8 +332,8 @@ def bench_bptt(torch, steps=600):
         "roofline_forward": {"bound": "hbm", "achieved": fwd_step * steps / t_f / 1e9, "peak": HBM_PEAK_GBS,
                              "unit": "GB/s", "frac": fwd_step * steps / t_f / 1e9 / HBM_PEAK_GBS,
                              "algorithmic_bytes_per_step": fwd_step,
-                             "what": "the joint table once per step + state in and out + record out (the kernel reads "
-                                     "the table once per TWO steps, so its traffic is below this)",
+                             "what": "the joint table once per step + state in and out + record out (trials side by side read "
+                                     "only the rows that fired and keep their state: traffic is far below this)",
                              "frac_by_update_and_event_bytes":
                                  (ne * B_PER_UPDATE_PLAIN + (events / steps + in_ev.numel() / (2 * steps) * (nnz_in / n_in)) * B_PER_EVENT)
                                  * steps / t_f / 1e9 / HBM_PEAK_GBS,
