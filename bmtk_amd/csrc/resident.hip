@@ -697,7 +697,9 @@ __global__ __launch_bounds__(kResBlock) void sim_resident_kernel(bmtk_glif3_sim 
 // the step has threads for it (a small network has few rows a step and long segments).
 //
 // Steps in which a list does not hold its neurons, or the rows have no room, are crowded: all sixteen wavefronts read
-// the lists (or ballots) and work the rows off.
+// the lists (or ballots) and work the rows off.  At rates far above a network's usual few Hz that is every step: 60,000 neurons
+// at 40 / 60 / 92 Hz 10.3 / 14.8 / 20.4 us against 10.3 / 13.4 / 19.5 with ballots and a grid barrier, 230,924 at 49 Hz 48.8
+// against 44.1, 5,000 at 70 Hz 3.5 against 4.2.
 //
 // Measured per step, ballots or lists behind a grid barrier -> this: 10,007 neurons of in-degree 600 3.27 -> 2.16 us; 60,000 of
 // 660 4.15 -> 2.88; 120,000 of 440 4.63 -> 3.92; the V1 network's 230,924 of 335 5.46 -> 4.96.  What it spends there: update
