@@ -729,7 +729,7 @@ __global__ __launch_bounds__(kResBlock) void sim_resident_lists_kernel(bmtk_glif
         s.inp_packed = nullptr;
     }
     extern __shared__ float ring_l[];  // [L*4][span], then kActCap words
-    __shared__ int go_on;
+    __shared__ int go_on[2];  // by the round, as rows_l is: a slot is written again only after a meeting behind all reads of it
     __shared__ unsigned rows_l[2], spikes_l[2], team_l[2], crowd_l[2], done_l, updated_l, listed_l;  // rows of a step, of neurons (the others: of inputs), ..
     __shared__ unsigned fired_n[2];                               // how many fired in this step and the one before
     __shared__ unsigned long long ballot_l[kResBlock / kWave];
@@ -755,11 +755,11 @@ __global__ __launch_bounds__(kResBlock) void sim_resident_lists_kernel(bmtk_glif
     const bool alone = s.rec_seg == nullptr;  // nobody's spikes arrive anywhere
     // a run before this one gave up and nobody has looked yet: do nothing, so that the failure is still there to see
     if (tid == 0) {
-        go_on = load_agent(abort_word) == 0u;
+        go_on[0] = load_agent(abort_word) == 0u;
         fired_n[0] = fired_n[1] = rows_l[0] = rows_l[1] = spikes_l[0] = spikes_l[1] = team_l[0] = team_l[1] = crowd_l[0] = crowd_l[1] = done_l = updated_l = listed_l = 0u;
     }
     __syncthreads();
-    if (!go_on) return;
+    if (!go_on[0]) return;
 
     for (int c = tid; c < L * GLIF3_NREC * span; c += kResBlock) {
         const int dr = c / span, i = c - dr * span;
@@ -931,7 +931,7 @@ __global__ __launch_bounds__(kResBlock) void sim_resident_lists_kernel(bmtk_glif
                 }
             }
             __syncthreads();  // X
-            if (k > 0 && !go_on) {
+            if (k > 0 && !go_on[k & 1]) {
                 aborted = true;
                 break;
             }
@@ -1020,7 +1020,7 @@ __global__ __launch_bounds__(kResBlock) void sim_resident_lists_kernel(bmtk_glif
                         lost = !again();
                 }
                 if (lane == 0) {
-                    go_on = !lost;
+                    go_on[k & 1] = !lost;
                     crowd_l[k & 1] = 0u;
                 }
             }
@@ -1030,7 +1030,7 @@ __global__ __launch_bounds__(kResBlock) void sim_resident_lists_kernel(bmtk_glif
             const int64_t ev_end = ((int64_t)__builtin_amdgcn_readfirstlane((int)(ev_next >> 32)) << 32) |
                                    (int64_t)(unsigned)__builtin_amdgcn_readfirstlane((int)ev_next);
             __syncthreads();  // X
-            if (k > 0 && !go_on) {
+            if (k > 0 && !go_on[k & 1]) {
                 aborted = true;
                 break;
             }

@@ -75,7 +75,7 @@ __global__ __launch_bounds__(kRbBlock) void sim_resident_batch_kernel(bmtk_glif3
     constexpr bool kFixed = sizeof(Sum) == 8;
     constexpr int kOwners = kRbReader * kWave;  // with two neurons to a thread: threads that own tid, tid + kOwners
     extern __shared__ unsigned long long rb_lds[];  // ring slice [slots * 4][span], then rb_list words for rows
-    __shared__ int go_on;
+    __shared__ int go_on[2];  // by the round, as rows_l is: a slot is written again only after a meeting behind all reads of it
     __shared__ unsigned rows_l[2], crowd_l[2], done_l, updated_l, listed_l;  // rows of a round, ..
     __shared__ unsigned fired_n[2];                  // how many fired in this step and the one before
     __shared__ unsigned short fired_l[kListMax + 1]; // the first of them, counted within the span
@@ -108,11 +108,11 @@ __global__ __launch_bounds__(kRbBlock) void sim_resident_batch_kernel(bmtk_glif3
     auto lists_of = [&](int k) { return ListRow{lists + (k & (kListRows - 1)) * kListRowWords, way * G, G}; };
     auto ballots_of = [&](int k) { return hist + (int64_t)(k & (kListRows - 1)) * (q.words + 1); };
     if (tid == 0) {
-        go_on = rb_load(abort_word) == 0u;
+        go_on[0] = rb_load(abort_word) == 0u;
         rows_l[0] = rows_l[1] = crowd_l[0] = crowd_l[1] = done_l = updated_l = listed_l = fired_n[0] = fired_n[1] = 0u;
     }
     __syncthreads();
-    if (!go_on) return;
+    if (!go_on[0]) return;
 
     Sum *ring_g = reinterpret_cast<Sum *>(s.rb_ring) + (int64_t)trial * S * GLIF3_NREC * n + e0;
     for (int c = tid; c < S * GLIF3_NREC * span; c += kRbBlock) {
@@ -324,7 +324,7 @@ __global__ __launch_bounds__(kRbBlock) void sim_resident_batch_kernel(bmtk_glif3
                 write(k);
             }
             __syncthreads();  // the workgroup meets: every slot k-1 is folded, the rows of the round are there
-            if (!go_on) {
+            if (!go_on[k & 1]) {
                 aborted = true;
                 break;
             }
@@ -396,14 +396,14 @@ __global__ __launch_bounds__(kRbBlock) void sim_resident_batch_kernel(bmtk_glif3
                     if (!lost) store_lds(&listed_l, (unsigned)k + 1u);
                 }
             }
-            if (lane == 0) go_on = !lost;
+            if (lane == 0) go_on[k & 1] = !lost;
             // vmcnt(0): nothing is on its way here, and with that said the compiler does not wait for loads below before it
             // uses their registers again
             __builtin_amdgcn_s_waitcnt(0x0F70);
             ev_lo = next_lo;
             ev_hi = (unsigned)__builtin_amdgcn_readfirstlane((int)next_hi);
             __syncthreads();
-            if (!go_on) {
+            if (!go_on[k & 1]) {
                 aborted = true;
                 break;
             }
