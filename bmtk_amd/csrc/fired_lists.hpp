@@ -185,7 +185,7 @@ __device__ __forceinline__ unsigned rows_from_lists(ListLook &seen, const ListRo
 
 // All 1024 threads: the rows of a crowded step -- the neurons in `lists` (ballots where a list did not suffice, `ballot_words` to a
 // workgroup, `words` in all) and n_ev rows event(i) -- to act[0 .. cap), their number to *count, which was zero.  What finds no
-// room goes to spot(row) at once.  kWordRounds: 4 * kWordRounds words cover a list or a workgroup's ballots.
+// room goes to spot(row) at once.  A word is looked for max_spin times in vain at most.  kWordRounds: 4 * kWordRounds words cover a list or a workgroup's ballots.
 template <int kWordRounds, typename Event, typename Spot>
 __device__ __forceinline__ void crowded_rows(const ListRow &lists, bool any, int span, const unsigned long long *ballots, int words,
                                              unsigned n_ev, unsigned *act, unsigned cap, unsigned *count, unsigned *abort_word,
@@ -221,8 +221,9 @@ __device__ __forceinline__ void crowded_rows(const ListRow &lists, bool any, int
                 cnt = min(n - first, j == 0 ? 4u : 5u);
                 unsigned spins = 0u;
                 while (((v = load_agent64(lists.at(of, j))) ^ head) >> kListTagAt) {
-                    if (++spins > max_spin) {
-                        __hip_atomic_store(abort_word, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    // (given up, here or elsewhere: nothing of the run is valid, and check() will say so)
+                    if (++spins > max_spin) __hip_atomic_store(abort_word, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    if (spins > max_spin || __hip_atomic_load(abort_word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u) {
                         cnt = 0u;
                         break;
                     }

@@ -752,6 +752,7 @@ __global__ __launch_bounds__(kResBlock) void sim_resident_lists_kernel(bmtk_glif
     unsigned *abort_word = s.res_sync + 1;
     unsigned long long *lists = reinterpret_cast<unsigned long long *>(s.res_sync + kBarrierStride);
     unsigned long long *hist = reinterpret_cast<unsigned long long *>(s.work_bits);
+    const unsigned spin_limit = s.res_spin_limit ? s.res_spin_limit : kMaxSpin;
     const bool alone = s.rec_seg == nullptr;  // nobody's spikes arrive anywhere
     // a run before this one gave up and nobody has looked yet: do nothing, so that the failure is still there to see
     if (tid == 0) {
@@ -862,7 +863,7 @@ __global__ __launch_bounds__(kResBlock) void sim_resident_lists_kernel(bmtk_glif
         const int64_t lo = events_at(k - 1), hi = events_at(k);  // (a step's events are below 2^31)
         auto pull_row = [&](unsigned row) __attribute__((always_inline)) { add_bounds(row_bounds(row), (row & kInputTag) != 0u, 0u, 1u); };
         crowded_rows<4>(lists_of(k - 1), !alone, span, hist + (int64_t)row_before() * (words + 1), words, (unsigned)(hi - lo), rows,
-                        kCrowdedCap, &crowd_l[k & 1], abort_word, kMaxSpin,
+                        kCrowdedCap, &crowd_l[k & 1], abort_word, spin_limit,
                         [&](unsigned i) { return input_row(s.in_events[lo + i]); }, pull_row);
         __syncthreads();
         const unsigned total = min(crowd_l[k & 1], kCrowdedCap);
@@ -971,9 +972,8 @@ __global__ __launch_bounds__(kResBlock) void sim_resident_lists_kernel(bmtk_glif
         int32_t ev[kReaderEvents] = {0, 0, 0, 0};
         // one more look in vain: false when it is time to give up
         auto again = [&]() __attribute__((always_inline)) -> bool {
-            const unsigned limit = s.res_spin_limit ? s.res_spin_limit : kMaxSpin;
-            if (++failed > limit) __hip_atomic_store(abort_word, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            return failed <= limit && load_agent(abort_word) == 0u;
+            if (++failed > spin_limit) __hip_atomic_store(abort_word, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            return failed <= spin_limit && load_agent(abort_word) == 0u;
         };
         // the rows of step k, whose lists have been seen, into LDS
         auto take = [&](int k) __attribute__((always_inline)) {

@@ -103,6 +103,7 @@ __global__ __launch_bounds__(kRbBlock) void sim_resident_batch_kernel(bmtk_glif3
     unsigned *rows = reinterpret_cast<unsigned *>(ring_l + (size_t)S * GLIF3_NREC * span);  // [2][row_cap], a place per lane behind
     const unsigned row_cap = ((unsigned)s.rb_list - kWave) / 2u;
     unsigned *abort_word = s.res_sync + 1;
+    const unsigned spin_limit = s.res_spin_limit ? s.res_spin_limit : kRbMaxSpin;
     unsigned long long *lists = reinterpret_cast<unsigned long long *>(s.res_sync + BMTK_RES_SYNC_STRIDE);
     unsigned long long *hist = reinterpret_cast<unsigned long long *>(s.rb_hist) + (int64_t)way * kListRows * (q.words + 1);
     auto lists_of = [&](int k) { return ListRow{lists + (k & (kListRows - 1)) * kListRowWords, way * G, G}; };
@@ -289,7 +290,7 @@ __global__ __launch_bounds__(kRbBlock) void sim_resident_batch_kernel(bmtk_glif3
         const unsigned cap = (unsigned)s.rb_list;
         auto pull_row = [&](unsigned row) __attribute__((always_inline)) { add_segment(row_bounds(row), 0u, 1u); };
         crowded_rows<kPer == 1 ? 4 : 8>(lists_of(k - 1), k > 0, span, ballots_of(k - 1), q.words, hi - lo, rows, cap, &crowd_l[k & 1],
-                                        abort_word, kRbMaxSpin, [&](unsigned i) { return (unsigned)n + (unsigned)s.rb_in_events[lo + i]; },
+                                        abort_word, spin_limit, [&](unsigned i) { return (unsigned)n + (unsigned)s.rb_in_events[lo + i]; },
                                         pull_row);
         __syncthreads();
         const unsigned total = min(crowd_l[k & 1], cap);
@@ -360,9 +361,8 @@ __global__ __launch_bounds__(kRbBlock) void sim_resident_batch_kernel(bmtk_glif3
         ask_events();
         // one more look in vain: false when it is time to give up
         auto again = [&]() __attribute__((always_inline)) -> bool {
-            const unsigned limit = s.res_spin_limit ? s.res_spin_limit : kRbMaxSpin;
-            if (++failed > limit) __hip_atomic_store(abort_word, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            return failed <= limit && rb_load(abort_word) == 0u;
+            if (++failed > spin_limit) __hip_atomic_store(abort_word, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            return failed <= spin_limit && rb_load(abort_word) == 0u;
         };
         for (int k = 0; k <= n_steps; ++k) {
             if (kReaderOwns) {

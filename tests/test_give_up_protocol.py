@@ -99,3 +99,13 @@ def test_the_model_sees_a_word_that_is_read_late():
     """With one word for all rounds a wavefront may read the next round's in place of its own and leave without adding to done_l;
     the others wait for that.  (A reader that owns neurons waits for the pulling wavefronts first: only the writer can be late.)"""
     assert _stuck(1, False, False) is not None and _stuck(1, False, True) is not None
+
+
+@pytest.mark.parametrize("source,kernel,limit", [("resident.hip", "sim_resident_lists_kernel", "kMaxSpin"),
+                                                 ("resident_batch.hip", "sim_resident_batch_kernel", "kRbMaxSpin")])
+def test_the_callers_limit_holds_for_every_wait(source, kernel, limit):
+    """res_spin_limit, where one is given, takes the built-in limit's place in all waits for other workgroups."""
+    with open(os.path.join(CSRC, source)) as f:
+        body = f.read().split("void %s(" % kernel)[1].split("\n}\n")[0]
+    used = [line for line in body.splitlines() if limit in line]
+    assert len(used) == 1 and "s.res_spin_limit ? s.res_spin_limit : " + limit in used[0]

@@ -134,3 +134,28 @@ def test_a_reader_gives_up_cleanly(monkeypatch):
     sim.run(60)
     sim.check()
     assert torch.equal(want.state.V, sim.state.V)
+
+
+@pytest.mark.parametrize("batch", [1, 5])
+def test_crowded_steps_give_up_cleanly(batch, monkeypatch):
+    """The same in steps that all wavefronts work off (39 neurons and more of a workgroup, more events than there is room for): the
+    limit holds for the lists' further words too.  The run ends and is reported, or nobody had to wait and it is right."""
+    par, rec, inp, ptr, events = _network(1)
+    rec, inp = [t[:3] + (np.minimum(t[3], 4),) + t[4:] for t in (rec, inp)]
+    ptr, events = np.arange(41, dtype=np.int64) * 3000, np.tile(np.arange(3000, dtype=np.int32) * batch, 40)
+    monkeypatch.setattr(simulator, "resident_span", lambda *a, **k: 64)
+    monkeypatch.setattr(simulator, "resident_trials_plan", lambda *a: dict(span=64, groups=47, ways=2, passes=3, list=64))
+    bits = {}
+    for limit in (0, 1):
+        sim = simulator.Glif3Simulator(N, par, 1.0, batch=batch, rec=rec, inp=inp, resident=batch == 1, resident_trials=batch > 1)
+        sim.state.V.copy_(torch.as_tensor(np.repeat(_start(par, 64, 8), batch)))
+        sim.set_input_events(ptr, events)
+        sim.spin_limit = limit
+        bits[limit] = sim.run(40)["bits"]
+        gave_up = int(sim.res_sync[1].item()) != 0
+        assert not (gave_up and limit == 0)
+        if gave_up:
+            with pytest.raises(RuntimeError, match="barrier"):
+                sim.check()
+        else:
+            assert torch.equal(bits[limit], bits[0])
