@@ -280,7 +280,7 @@ def bench_bptt(torch, steps=600):
     _, by_src, _ = synthetic.device_network(n, 1000, "poisson", seed=2, w_scale=0.2)
     inp = synthetic.device_input_table(n_in, n, 8_000_000, seed=4, w_scale=2.0)
     in_ptr, in_ev = ops.poisson_events(n_in, 5.0, 1.0, 2 * steps, batch=batch, seed=5)
-    sim = Glif3Simulator(n, par, 1.0, batch=batch, rec=by_src, inp=inp, resident=False)
+    sim = Glif3Simulator(n, par, 1.0, batch=batch, rec=by_src, inp=inp)
     sim.set_input_events(in_ptr, in_ev)
     g = torch.Generator(device="cuda").manual_seed(11)
     pop = torch.randint(0, 17, (n,), device="cuda", generator=g)

@@ -197,7 +197,7 @@ class Glif3Simulator:
     resident    "auto": every ``run`` is one cooperative launch that keeps the state in registers and the ring in
                 LDS (the resident kernel) whenever the network fits it -- batch 1, at most 1024 elements per
                 compute unit, ring slice within LDS; True: insist on it (ValueError otherwise); False: one launch
-                per step, which takes any batch and size (a batch's trials: see ``resident_trials``)
+                per step, which takes any batch and size (``resident_trials`` then has to be asked for)
     single_workgroup  resident mode: a network of up to 1024 elements whose whole ring fits LDS runs in ONE
                 workgroup, without a grid barrier (about 1 us per step instead of 2.5); False keeps such a network
                 on the many-workgroup form
@@ -228,7 +228,7 @@ class Glif3Simulator:
     resident_trials  batches of 2 to 64, or one trial of more neurons than ``resident`` holds (1024 to a compute unit; here up
                 to 1920), with a recurrent table and delay_offset 0: trials side by side, each with its state
                 in registers and its ring in LDS for the length of a call, as many at a time as the compute units hold
-                (``resident_trials_plan``).  "auto": where resident (of a batch: also False), fused and pull are "auto" too, the network fits,
+                (``resident_trials_plan``).  "auto": where resident, fused and pull are "auto" too, the network fits,
                 ``trials_pay`` says so and its tables are in proportion to the network (``trials_fit``); where there turns out to be no
                 memory for them the other driver runs.  Such a simulator also holds the driver it would have without; a call that asks
                 for more than spike bits and, of a batch, the per-step record (``record_cap``, probes; ``save_state`` of a single
@@ -430,8 +430,8 @@ class Glif3Simulator:
         self.expected_rate_hz = float(expected_rate_hz)
         self._trials_left, self._pend_from, self._pend_until, self._left_ring, self._kept = False, 0, 0, None, []
         if resident_trials == "auto":
-            # (batches with resident=False, as training simulators have it, too: their forward part is a call of many steps)
-            wanted = (resident == "auto" or (resident is False and self.batch > 1)) and fused == "auto" and pull == "auto" and self.pull_table is None
+            # (resident=False asks for the launch-per-step drivers, of a batch too)
+            wanted = resident == "auto" and fused == "auto" and pull == "auto" and self.pull_table is None
         else:
             wanted = bool(resident_trials)
         plan = None

@@ -44,8 +44,9 @@ def rate_mse(counts, n_steps, batch, pop_id, targets):
 
 
 class Glif3Bptt:
-    """Reverse-time adjoint over a recorded forward run of a ``Glif3Simulator``
-    built with ``resident=False``."""
+    """Reverse-time adjoint over a recorded forward run of a ``Glif3Simulator``: of a batch, or of a single trial
+    built with ``resident=False``.  (A batch whose simulator leaves ``resident`` at "auto" runs the forward part with
+    resident trials where they pay: 1.76 instead of 2.19 ms a step of training at 3,001 neurons x 12 trials x 100 steps.)"""
 
     # A synapse costs the swept form more once the L2s no longer hold the adjoint ring; the blocked form has a fixed part per
     # row and range, which long rows share among more synapses.  Measured on one MI355X, whole calls of 40 steps, us per step
@@ -84,7 +85,7 @@ class Glif3Bptt:
         number of target ranges, a multiple of 8 (None: ``ops.blocked_table_blocks``); ``two_steps``: let the blocked form
         take two steps per pass over its table (batches above 16; ``gz`` then holds the partial sums of both)."""
         if sim.res_span or sim.delay_offset:
-            raise ValueError("the backward pass needs a simulator built with resident=False and delay_offset 0")
+            raise ValueError("the backward pass needs a simulator built with resident=False (or a batch) and delay_offset 0")
         self.sim, self.dampening = sim, float(dampening)
         self.lib = _lib.load()
         dev, ne = sim.dev, sim.ne

@@ -4,7 +4,7 @@ import pytest
 import torch
 
 from oracle import glif3_oracle as orc
-from bmtk_amd import ops, simulator, synthetic
+from bmtk_amd import ops, simulator, synthetic, training
 from bmtk_amd.simulator import Glif3Simulator, fixed_point_shift, resident_trials_plan
 
 pytestmark = pytest.mark.gpu
@@ -380,11 +380,26 @@ def test_what_does_not_fit_is_refused():
         Glif3Simulator(cfg["n"], cfg["par"], 1.0, batch=2, inp=cfg["inp_src"], resident=False, resident_trials=True)
 
 
-def test_training_simulators_take_resident_trials_where_they_pay():
-    """resident=False of a batch: the form with resident trials by itself, the per-step drivers for a short call and on request."""
+def test_resident_false_keeps_the_launches_and_auto_takes_trials_for_training():
+    """resident=False is one launch per step (or two), whatever a step would cost otherwise; a training simulator of a batch that
+    leaves ``resident`` alone, or asks for them, runs its trials resident, with the same record, and the backward pass takes it."""
     batch = 12
     cfg, _, _ = _case(700, batch, 3)
-    for kw, steps, trials in ((dict(), 64, True), (dict(), 20, False), (dict(resident_trials=False), 64, False)):
-        sim = _sim(cfg, batch, **kw)
-        sim.run(steps, save_state=True)
-        assert (sim._trials is not None) == trials
+    want = None
+    for kw, trials in ((dict(resident=False), False), (dict(resident_trials=False), False), (dict(), True),
+                       (dict(resident=False, resident_trials=True), True)):
+        sim = Glif3Simulator(cfg["n"], cfg["par"], 1.0, batch=batch, class_id=cfg["class_id"], rec=cfg["rec_src"], inp=cfg["inp_src"],
+                             i_ext=cfg["i_ext"], ring_slots=cfg["L"], **kw)
+        sim.set_input_events(cfg["in_ptr"], cfg["in_events"])
+        assert (sim._trials is not None) == trials, kw
+        out = sim.run(64, save_state=True)
+        assert (sim._trials is not None) == trials, kw
+        bptt = training.Glif3Bptt(sim)
+        bptt.backward(out, dl_dz_const=torch.ones(sim.ne, device="cuda"))
+        got = dict(bits=out["bits"], v=out["saved"]["v"], flags=out["saved"]["flags"])
+        want = want or dict(got, d_rec_w=bptt.d_rec_w)
+        for key in got:
+            assert torch.equal(got[key], want[key]), (kw, key)
+        assert float(bptt.d_rec_w.abs().max()) > 0.0
+        # (the same adjoint; only sums of atomic additions in another order)
+        assert float((bptt.d_rec_w - want["d_rec_w"]).norm()) <= 4e-6 * float(want["d_rec_w"].norm())
