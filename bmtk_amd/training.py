@@ -130,6 +130,10 @@ class Glif3Bptt:
         sim, saved, bits = self.sim, fwd["saved"], fwd["bits"]
         if saved is None or bits is None:
             raise ValueError("forward run was made without save_state=True or without spike bits")
+        # (resident trials can give up on one another and then leave a record that was never written; no later step of a training
+        #  would show it.  A capture cannot look.)
+        if sim._pending_check and not torch.cuda.is_current_stream_capturing():
+            sim.check()
         n_steps = bits.shape[0]
         a = _lib.Glif3Bwd()
         a.n_neurons, a.batch, a.ring_slots, a.h, a.dampening = sim.n, sim.batch, self.lam_ring.shape[0], sim.h, self.dampening
@@ -158,7 +162,8 @@ class Glif3Bptt:
     def backward(self, fwd, dl_dz_const=None, dl_dz=None):
         """``fwd`` is what ``sim.run(n, save_state=True)`` returned.  Accumulates
         into ``d_rec_w`` / ``d_inp_w`` (same order as ``sim.rec`` / ``sim.inp``).
-        Calls for consecutive chunks must come in reverse time order."""
+        Calls for consecutive chunks must come in reverse time order.  Synchronises once behind runs with resident trials,
+        to raise if they gave up (``Glif3Simulator.check``)."""
         a, step0, n_steps = self._struct(fwd, dl_dz_const, dl_dz, self.blk is not None)
         _lib.check(self.lib.bmtk_glif3_simulate_bwd(C.byref(a), step0, n_steps, _stream()))
         if self.blk is not None:  # the blocked kernel accumulates in its table's order: back to the order of sim.rec

@@ -403,3 +403,23 @@ def test_resident_false_keeps_the_launches_and_auto_takes_trials_for_training():
         assert float(bptt.d_rec_w.abs().max()) > 0.0
         # (the same adjoint; only sums of atomic additions in another order)
         assert float((bptt.d_rec_w - want["d_rec_w"]).norm()) <= 4e-6 * float(want["d_rec_w"].norm())
+
+
+@pytest.mark.parametrize("stepwise", [False, True])
+def test_the_backward_pass_refuses_the_record_of_a_run_that_gave_up(stepwise):
+    """The abort word set from the host: the forward run does nothing, its record is whatever the memory held, and the backward pass
+    says so instead of taking gradients from it.  The next run is right."""
+    batch = 12
+    cfg, _, _ = _case(300, batch, 3)
+    sim = _sim(cfg, batch, resident_trials=True)
+    bptt = training.Glif3Bptt(sim)
+    backward = bptt.backward_stepwise if stepwise else bptt.backward
+    dl_dz = torch.ones(sim.ne, device="cuda")
+    backward(sim.run(40, save_state=True), dl_dz_const=dl_dz)
+    bptt.zero()
+    sim.res_sync[1] = 1
+    with pytest.raises(RuntimeError, match="aborted"):
+        backward(sim.run(40, save_state=True), dl_dz_const=dl_dz)
+    assert float(bptt.d_rec_w.abs().max()) == 0.0
+    backward(sim.run(40, save_state=True), dl_dz_const=dl_dz)
+    assert int(sim.res_sync[1].item()) == 0 and bool(torch.isfinite(bptt.d_rec_w).all())
