@@ -41,6 +41,14 @@ __device__ __forceinline__ unsigned long long load_agent64(const unsigned long l
 // as few lines as that allows).
 constexpr int kListRows = 4;   // lists of so many steps are kept
 constexpr int kListRowWords = kListWords * kListGroups;
+// They begin behind the first line of res_sync, at the next whole 64-bit word: that is scratch of 32-bit words, and as long as
+// they were all that it held a caller's could lie on any of them.
+constexpr size_t kListSyncWords = BMTK_RES_SYNC_STRIDE + 1 + (size_t)2 * kListRows * kListRowWords;  // of res_sync
+static_assert(BMTK_RES_SYNC_WORDS >= kListSyncWords, "res_sync holds the lists");
+__host__ __device__ inline unsigned long long *lists_in(unsigned *res_sync)
+{
+    return reinterpret_cast<unsigned long long *>((reinterpret_cast<uintptr_t>(res_sync + BMTK_RES_SYNC_STRIDE) + 7u) & ~(uintptr_t)7u);
+}
 struct ListRow {
     unsigned long long *w;
     int first, G;  // the lists that belong together: first .. first + G - 1

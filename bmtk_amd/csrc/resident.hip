@@ -709,7 +709,6 @@ __global__ __launch_bounds__(kResBlock) void sim_resident_kernel(bmtk_glif3_sim 
 // then share the way to memory; another order of rows for each workgroup of an XCD: no difference.
 constexpr int kReader = kResBlock / kWave - 1, kWriter = kReader - 1;
 constexpr int kPullThreads = kWriter * kWave;
-static_assert((kWays * kBarrierWords) * kBarrierStride * 4 >= kListRows * kListRowWords * 8, "res_sync holds the lists");
 constexpr int kReaderEvents = 4;    // input events a lane of the reader asks for ahead
 // the room of the row list (kActCap words) divided up: rows of two steps, a place per lane of the reader for what is none, the
 // neurons of this workgroup that fired and, for a record, their crossing fractions
@@ -750,7 +749,7 @@ __global__ __launch_bounds__(kResBlock) void sim_resident_lists_kernel(bmtk_glif
     unsigned short *fired_l = reinterpret_cast<unsigned short *>(rows + 2 * kRowCap + kWave);
     float *frac_l = reinterpret_cast<float *>(fired_l + kResBlock);
     unsigned *abort_word = s.res_sync + 1;
-    unsigned long long *lists = reinterpret_cast<unsigned long long *>(s.res_sync + kBarrierStride);
+    unsigned long long *lists = lists_in(s.res_sync);
     unsigned long long *hist = reinterpret_cast<unsigned long long *>(s.work_bits);
     const unsigned spin_limit = s.res_spin_limit ? s.res_spin_limit : kMaxSpin;
     const bool alone = s.rec_seg == nullptr;  // nobody's spikes arrive anywhere
@@ -1168,9 +1167,10 @@ int simulate_resident(const bmtk_glif3_sim &s, int64_t step0, int64_t n_steps, h
                   n_cu, per_cu);
         return BMTK_E_LAUNCH;
     }
-    const int64_t list_words = 2 * kListRows * kListRowWords;
+    const int64_t list_words = 2 * kListRows * kListRowWords;  // (32-bit ones)
     if (lists)
-        hipLaunchKernelGGL(zero_words_kernel, dim3((unsigned)((list_words + kBlock - 1) / kBlock)), dim3(kBlock), 0, stream, s.res_sync + kBarrierStride, list_words);
+        hipLaunchKernelGGL(zero_words_kernel, dim3((unsigned)((list_words + kBlock - 1) / kBlock)), dim3(kBlock), 0, stream,
+                           reinterpret_cast<unsigned *>(lists_in(s.res_sync)), list_words);
     else
         hipLaunchKernelGGL(zero_sync_kernel, dim3(1), dim3(kBlock), 0, stream, s.res_sync);
     bmtk_glif3_sim s_copy = s;

@@ -44,7 +44,6 @@ constexpr int kRbPullThreads = kRbWriter * kWave;
 constexpr unsigned kRbMaxSpin = 4000000u; // looks in vain before giving up (seconds)
 constexpr int kRbTogether = 6;            // synapses a lane has in flight (20,011 x 20, 8 lanes to 33: 4 of them 9.6 us per step, 6 9.3)
 constexpr int kRbEvents = 4;              // input events a lane of the reader asks for ahead
-static_assert(BMTK_RES_SYNC_WORDS >= BMTK_RES_SYNC_STRIDE + 2 * kListRows * kListRowWords, "res_sync holds the lists");
 
 struct RbLaunch {
     int64_t step0;
@@ -104,7 +103,7 @@ __global__ __launch_bounds__(kRbBlock) void sim_resident_batch_kernel(bmtk_glif3
     const unsigned row_cap = ((unsigned)s.rb_list - kWave) / 2u;
     unsigned *abort_word = s.res_sync + 1;
     const unsigned spin_limit = s.res_spin_limit ? s.res_spin_limit : kRbMaxSpin;
-    unsigned long long *lists = reinterpret_cast<unsigned long long *>(s.res_sync + BMTK_RES_SYNC_STRIDE);
+    unsigned long long *lists = lists_in(s.res_sync);
     unsigned long long *hist = reinterpret_cast<unsigned long long *>(s.rb_hist) + (int64_t)way * kListRows * (q.words + 1);
     auto lists_of = [&](int k) { return ListRow{lists + (k & (kListRows - 1)) * kListRowWords, way * G, G}; };
     auto ballots_of = [&](int k) { return hist + (int64_t)(k & (kListRows - 1)) * (q.words + 1); };
@@ -553,7 +552,7 @@ int simulate_resident_batch(const bmtk_glif3_sim &s, int64_t step0, int64_t n_st
         // the lists of the launch before back to no step's
         const int64_t list_words = (int64_t)kListRows * kListRowWords;
         hipLaunchKernelGGL(rb_zero_bits_kernel, dim3((unsigned)((list_words + kBlock - 1) / kBlock)), dim3(kBlock), 0, stream,
-                           reinterpret_cast<uint64_t *>(s.res_sync + BMTK_RES_SYNC_STRIDE), list_words);
+                           reinterpret_cast<uint64_t *>(lists_in(s.res_sync)), list_words);
         bmtk_glif3_sim copy = s;
         RbLaunch launch = q;
         void *args[] = {&copy, &launch};

@@ -306,7 +306,8 @@ typedef struct bmtk_glif3_sim {
     const uint32_t *inp_seg;     /* [inputs][res_groups+1] */
     uint32_t *res_sync;          /* BMTK_RES_SYNC_WORDS words of scratch, zeroed by the caller once: word 1 =
                                   * abort flag, from word BMTK_RES_SYNC_STRIDE on 64 x BMTK_RES_SYNC_WAYS arrival
-                                  * counters that many words apart (or lists, see res_fired), which every call clears for itself.  Word 1 != 0
+                                  * counters that many words apart (or lists, see res_fired, from the next whole 64-bit word on), which every call
+                                  * clears for itself.  Word 1 != 0
                                   * after a run means a grid barrier timed out and the results are invalid.  The
                                   * flag is sticky: no call clears it, and a call that finds it set does nothing,
                                   * so a failure cannot be overwritten before the host has seen it; the host

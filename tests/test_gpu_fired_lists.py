@@ -159,3 +159,21 @@ def test_crowded_steps_give_up_cleanly(batch, monkeypatch):
                 sim.check()
         else:
             assert torch.equal(bits[limit], bits[0])
+
+
+@pytest.mark.parametrize("batch", [1, 5])
+def test_scratch_on_any_32_bit_word(batch, monkeypatch):
+    """res_sync is scratch of 32-bit words: the lists in it, whose words are of 64 bits, find their own alignment."""
+    from bmtk_amd import _lib
+    par, rec, inp, ptr, events = _network(2)
+    rec, inp = [t[:3] + (np.minimum(t[3], 4),) + t[4:] for t in (rec, inp)]
+    monkeypatch.setattr(simulator, "resident_span", lambda *a, **k: 64)
+    bits = []
+    for words in (0, 1):
+        sim = simulator.Glif3Simulator(N, par, 1.0, batch=batch, rec=rec, inp=inp, resident=batch == 1, resident_trials=batch > 1)
+        sim.res_sync = torch.zeros(words + _lib.RES_SYNC_WORDS, dtype=torch.int32, device="cuda")[words:]
+        assert sim.res_sync.data_ptr() % 8 == 4 * words
+        sim.set_input_events(ptr, events * batch)
+        bits.append(sim.run(STEPS)["bits"])
+        sim.check()
+    assert int(bits[0].ne(0).sum()) > 50 and torch.equal(bits[0], bits[1])
