@@ -23,7 +23,7 @@ namespace bmtk {
 
 constexpr int kListWords = BMTK_RES_FIRED_SLOTS / 2;
 constexpr int kListQuickWords = 2;          // these of all workgroups side by side: what a reader asks for first
-constexpr unsigned kListQuick = 9, kListHalf = 19, kListMax = 39;  // neurons in words 0..1, 0..3, 0..7
+constexpr unsigned kListQuick = 9, kListMax = 39;  // neurons in words 0..1, 0..7
 constexpr unsigned kListMany = 2047;        // in place of the number: more than kListMax, see the ballots
 constexpr int kListRounds = 4;              // workgroups a lane of the reading wavefront looks after
 constexpr int kListGroups = kListRounds * kWave;
@@ -159,7 +159,7 @@ __device__ __forceinline__ unsigned rows_from_lists(ListLook &seen, const ListRo
     const unsigned inc = wave_inclusive_scan(sum);
     const unsigned total = (unsigned)bcast_i((int)inc, kWave - 1);
     const unsigned most = max(max(c[0], c[1]), max(c[2], c[3]));
-    if (__any(most > kListHalf) || more > cap || total + more > cap) return kCrowded;
+    if (__any(most > kListMax) || more > cap || total + more > cap) return kCrowded;
     const unsigned me = (unsigned)lane_here();
     // the neurons in the words of `seen`, from the j0-th of a list on
     auto emit = [&](unsigned j0, bool first) __attribute__((always_inline)) {
@@ -179,82 +179,127 @@ __device__ __forceinline__ unsigned rows_from_lists(ListLook &seen, const ListRo
         }
     };
     emit(0u, true);
-    if (__any(most > kListQuick)) {
-        while (!seen.template look<kFew>(lists, tag, kListQuickWords)) {
+    // (two more words of all lists at a time)
+#pragma unroll
+    for (int from = kListQuickWords; from < kListWords; from += 2) {
+        const unsigned j0 = 5u * from - 1u;
+        if (!__any(most > j0)) break;
+        while (!seen.template look<kFew>(lists, tag, from)) {
             if (!again()) {
                 lost = true;
                 return kCrowded;
             }
         }
-        emit(kListQuick, false);
+        emit(j0, false);
     }
     return total;
 }
 
-// All 1024 threads: the rows of a crowded step -- the neurons in `lists` (ballots where a list did not suffice, `ballot_words` to a
-// workgroup, `words` in all) and n_ev rows event(i) -- to act[0 .. cap), their number to *count, which was zero.  What finds no
-// room goes to spot(row) at once.  A word is looked for max_spin times in vain at most.  kWordRounds: 4 * kWordRounds words cover a list or a workgroup's ballots.
-template <int kWordRounds, typename Event, typename Spot>
-__device__ __forceinline__ void crowded_rows(const ListRow &lists, bool any, int span, const unsigned long long *ballots, int words,
-                                             unsigned n_ev, unsigned *act, unsigned cap, unsigned *count, unsigned *abort_word,
-                                             unsigned max_spin, Event event, Spot spot)
+// All 1024 threads: the rows of a crowded step -- n_first rows first(i), at most one to a thread and cap, and the neurons in `lists`,
+// ballots where a list did not suffice (`words` in all) -- to act[0 .. cap), as many at a time as there is room for; pull(n) works act[0 .. n) off.  count: three words of LDS.  A word is
+// looked for max_spin times in vain at most.  kBallotWords: of a workgroup, at most.
+// A thread holds two words a round, and as many threads share a list as let all lists have theirs: eight words of every
+// list are one round, sixteen ballots of every workgroup one or two.
+template <int kBallotWords, typename First, typename Pull>
+__device__ __forceinline__ void crowded_rows(const ListRow &lists, unsigned tag, int span, const unsigned long long *ballots, int words,
+                                             unsigned n_first, First first_row, unsigned *act, unsigned cap, unsigned *count, unsigned *abort_word,
+                                             unsigned max_spin, Pull pull)
 {
-    constexpr unsigned kThreads = 1024u;
-    int me = (int)threadIdx.x;
-    asm volatile("" : "+v"(me));
-    const int of = me >> 2, sub = me & 3;  // four threads to a list
-    unsigned long long head = 0ull;
-    if (any && of < lists.G) head = load_agent64(lists.at(of, 0));
-    const unsigned n = (unsigned)(head >> kListCountAt) & kListMany;
-    const bool many = n == kListMany;
-    const int event_rounds = (int)((n_ev + kThreads - 1u) / kThreads);
-    for (int round = -event_rounds; round < kWordRounds; ++round) {
-        unsigned long long v = 0ull;
-        unsigned cnt = 0u, base = (unsigned)(of * span);
-        bool bits = false;
-        if (round < 0) {
-            const unsigned at = (unsigned)(round + event_rounds) * kThreads + (unsigned)me;
-            if (at < n_ev) base = event(at), cnt = 1u;
-        } else {
-            const int j = round * 4 + sub;  // word of the list, or of the workgroup's ballots
-            const unsigned first = j == 0 ? 0u : 5u * (unsigned)j - 1u;
-            if (many) {
-                const int w = of * (span >> 6) + j;
-                if (j < (span >> 6) && w < words) v = load_agent64(ballots + w);
-                cnt = (unsigned)__popcll(v);
-                base += 64u * (unsigned)j;
-                bits = true;
-            } else if (j < kListWords && n > first) {
-                // (words 0 and 1 have been seen; the others left with them)
-                cnt = min(n - first, j == 0 ? 4u : 5u);
-                unsigned spins = 0u;
-                while (((v = load_agent64(lists.at(of, j))) ^ head) >> kListTagAt) {
-                    // (given up, here or elsewhere: nothing of the run is valid, and check() will say so)
-                    if (++spins > max_spin) __hip_atomic_store(abort_word, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    if (spins > max_spin || __hip_atomic_load(abort_word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u) {
-                        cnt = 0u;
-                        break;
+    constexpr unsigned kManyAt = 24u;  // upper bits of a counter: wavefronts that met a list that did not suffice
+    // (worked out where it is used: beside a neuron's state there are no registers for it)
+    auto here = []() __attribute__((always_inline)) {
+        int me = (int)threadIdx.x;
+        asm volatile("" : "+v"(me));
+        return me;
+    };
+    if (here() < 3) count[here()] = 0u;
+    __syncthreads();
+    const int sharing = lists.G <= 64 ? 4 : lists.G <= 128 ? 3 : 2;  // 1 << sharing threads to a list
+    unsigned filled = n_first;  // places taken
+    int turn = 0;          // a counter for every handing out of places: the one before may still be read, the one after is cleared
+    bool ballots_too = false, last = false;
+    bool bits = false;     // this thread's words are ballots
+    for (int round = 0; !last; ++round) {
+        unsigned long long v[2] = {0ull, 0ull};
+        auto word = [&](int i) __attribute__((always_inline)) { return ((2 * round + i) << sharing) + (here() & ((1 << sharing) - 1)); };
+        const int of = here() >> sharing;
+        const unsigned first_one = round == 0 && (unsigned)here() < n_first ? first_row((unsigned)here()) : 0u;
+        if (of < lists.G && (round == 0 || bits)) {
+            // (the reader has seen all lists, so their ballots are there: both are asked for at once.  A list's words end in the first round)
+            unsigned long long ballot[2] = {0ull, 0ull}, head = 0ull;
+            if (round == 0) head = load_agent64(lists.at(of, 0));
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const int w = of * (span >> 6) + word(i);
+                if (round == 0 && word(i) < kListWords) v[i] = load_agent64(lists.at(of, word(i)));
+                if (word(i) < (span >> 6) && w < words) ballot[i] = load_agent64(ballots + w);
+            }
+            const unsigned n = (unsigned)(head >> kListCountAt) & kListMany;
+            bits = bits || n == kListMany;
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                if (bits) {
+                    v[i] = ballot[i];
+                    continue;
+                }
+                const int j = word(i);
+                const unsigned first = j == 0 ? 0u : 5u * (unsigned)j - 1u;
+                unsigned left = 0u;
+                if (j < kListWords && n > first) {
+                    // (words 0 and 1 have been seen; the others left with them)
+                    left = min(n - first, j == 0 ? 4u : 5u);
+                    for (unsigned spins = 0u; (unsigned)(v[i] >> kListTagAt) != tag; v[i] = load_agent64(lists.at(of, j))) {
+                        // (given up, here or elsewhere: nothing of the run is valid, and check() will say so)
+                        if (++spins > max_spin) __hip_atomic_store(abort_word, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        if (spins > max_spin || __hip_atomic_load(abort_word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u) {
+                            left = 0u;
+                            break;
+                        }
                     }
                 }
+                // (in place of the tag: the neurons left in the word)
+                v[i] = (v[i] & ((1ull << kListTagAt) - 1ull)) | (unsigned long long)left << kListTagAt;
             }
         }
-        const unsigned inc = wave_inclusive_scan(cnt);
-        unsigned at = 0u;
-        if (lane_id() == kWave - 1 && inc) at = atomicAdd(count, inc);
-        at = (unsigned)bcast_i((int)at, kWave - 1) + inc - cnt;
-        for (; cnt > 0u; --cnt, ++at) {
-            unsigned id = base;
-            if (bits) {
-                id += (unsigned)(__ffsll((long long)v) - 1);
-                v &= v - 1ull;
-            } else if (round >= 0) {
-                id += (unsigned)v & ((1u << kListIdBits) - 1u);
-                v >>= kListIdBits;
+        if (round == 0 && (unsigned)here() < n_first) act[here()] = first_one;
+        while (true) {
+            unsigned mine = 0u;
+#pragma unroll
+            for (int i = 0; i < 2; ++i) mine += bits ? (unsigned)__popcll(v[i]) : (unsigned)(v[i] >> kListTagAt);
+            const unsigned inc = wave_inclusive_scan(mine);
+            const unsigned flag = __any(bits) ? 1u << kManyAt : 0u;
+            unsigned at = 0u;
+            if (lane_id() == kWave - 1 && (inc | flag)) at = atomicAdd(&count[turn], inc + flag);
+            at = filled + ((unsigned)bcast_i((int)at, kWave - 1) & ((1u << kManyAt) - 1u)) + inc - mine;
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const unsigned base = (unsigned)((here() >> sharing) * span + (bits ? 64 * word(i) : 0));
+                while (at < cap && (bits ? v[i] : v[i] >> kListTagAt)) {
+                    unsigned id = (unsigned)v[i];
+                    if (bits) {
+                        id = (unsigned)__ffsll((long long)v[i]) - 1u;
+                        v[i] &= v[i] - 1ull;
+                    } else {
+                        id &= (1u << kListIdBits) - 1u;
+                        const unsigned long long left = (v[i] >> kListTagAt) - 1ull;
+                        v[i] = ((v[i] & ((1ull << kListTagAt) - 1ull)) >> kListIdBits) | left << kListTagAt;
+                    }
+                    act[at++] = base + id;
+                }
             }
-            if (at < cap)
-                act[at] = id;
-            else
-                spot(id);
+            __syncthreads();
+            const unsigned handed = count[turn];
+            turn = turn == 2 ? 0 : turn + 1;
+            if (here() == 0) count[turn == 2 ? 0 : turn + 1] = 0u;
+            ballots_too = ballots_too || (handed >> kManyAt) != 0u;
+            const unsigned total = filled + (handed & ((1u << kManyAt) - 1u));
+            last = total <= cap && (2 * (round + 1)) << sharing >= (ballots_too ? kBallotWords : kListWords);
+            filled = total;
+            if (total <= cap && !last) break;
+            pull(min(total, cap));
+            __syncthreads();
+            filled = 0u;
+            if (last) break;
         }
     }
 }

@@ -91,6 +91,7 @@ struct Resident {
     int span, n_groups;
     int offset, hist, slack;  // B, D, S of the note above
     int check;                // the arrival counters are looked at every `check` steps (1 when S = 0)
+    int row_cap;              // lists: rows of a step that there is room for
 };
 
 __device__ __forceinline__ unsigned load_agent(const unsigned *p)
@@ -696,10 +697,11 @@ __global__ __launch_bounds__(kResBlock) void sim_resident_kernel(bmtk_glif3_sim 
 // A row's segment is read by a team of neighbouring lanes, as many as a segment holds synapses on average, rounded up, if
 // the step has threads for it (a small network has few rows a step and long segments).
 //
-// Steps in which a list does not hold its neurons, or the rows have no room, are crowded: all sixteen wavefronts read
-// the lists (or ballots) and work the rows off.  At rates far above a network's usual few Hz that is every step: 60,000 neurons
-// at 40 / 60 / 92 Hz 10.3 / 14.8 / 20.4 us against 10.3 / 13.4 / 19.5 with ballots and a grid barrier, 230,924 at 49 Hz 48.8
-// against 44.1, 5,000 at 70 Hz 3.5 against 4.2.
+// Steps in which more than 39 neurons of a workgroup fire, or whose rows have no room, are crowded: all sixteen wavefronts read the
+// lists (or ballots) and work the rows off.  A network's usual few Hz are far below that; us per step, ballots behind a grid barrier /
+// the reader taking lists of up to 19 neurons and 3,808 rows / of 39 and all that LDS holds: 60,000 neurons at 35, 45, 56, 71, 92 Hz
+// 8.9 / 8.5 / 7.9, 10.3 / 12.2 / 9.3, 12.1 / 14.5 / 10.8, 14.2 / 17.1 / 13.0, 17.4 / 20.7 / 17.5; 230,924 neurons at 24, 35, 46, 60 Hz
+// 17.3 / 19.4 / 18.4, 23.1 / 33.8 / 29.0, 38.4 / 41.7 / 36.5, 47.0 / 52.1 / 45.4 (crowded from 25 Hz on).
 //
 // Measured per step, ballots or lists behind a grid barrier -> this: 10,007 neurons of in-degree 600 3.27 -> 2.16 us; 60,000 of
 // 660 4.15 -> 2.88; 120,000 of 440 4.63 -> 3.92; the V1 network's 230,924 of 335 5.46 -> 4.96.  What it spends there: update
@@ -710,26 +712,27 @@ __global__ __launch_bounds__(kResBlock) void sim_resident_kernel(bmtk_glif3_sim 
 constexpr int kReader = kResBlock / kWave - 1, kWriter = kReader - 1;
 constexpr int kPullThreads = kWriter * kWave;
 constexpr int kReaderEvents = 4;    // input events a lane of the reader asks for ahead
-// the room of the row list (kActCap words) divided up: rows of two steps, a place per lane of the reader for what is none, the
-// neurons of this workgroup that fired and, for a record, their crossing fractions
-constexpr unsigned row_cap(bool record)
+// LDS behind the ring slice, `bytes` of it: rows of two steps, a place per lane of the reader for what is none, the neurons of this
+// workgroup that fired and, for a record, their crossing fractions.  At least kActCap words (3,808 rows of a step, with a record 3,296),
+// and all that the ring slice leaves, up to four times as many: crowded steps cost half as much again.
+constexpr int row_cap(size_t bytes, bool record)
 {
-    return (unsigned)((kActCap * 4 - 2 * kResBlock - (record ? 4 * kResBlock : 0) - 4 * kWave) / 8);
+    return (int)((bytes - 2 * kResBlock - (record ? 4 * kResBlock : 0) - 4 * kWave) / 8);
 }
 
 template <int kForm, bool kReaderOwns>
 __global__ __launch_bounds__(kResBlock) void sim_resident_lists_kernel(bmtk_glif3_sim s, Resident r)
 {
     constexpr bool kUnified = kForm != kFormAny, kRecord = kForm != kFormLean;
-    constexpr unsigned kRowCap = row_cap(kRecord), kCrowdedCap = 2u * kRowCap;
+    const unsigned row_cap = (unsigned)r.row_cap;
     if (kForm != kFormAny) {
         s.probe_col = nullptr;
         s.inp_seg = nullptr;
         s.inp_packed = nullptr;
     }
-    extern __shared__ float ring_l[];  // [L*4][span], then kActCap words
+    extern __shared__ float ring_l[];  // [L*4][span], then see row_cap
     __shared__ int go_on[2];  // by the round, as rows_l is: a slot is written again only after a meeting behind all reads of it
-    __shared__ unsigned rows_l[2], spikes_l[2], team_l[2], crowd_l[2], done_l, updated_l, listed_l;  // rows of a step, of neurons (the others: of inputs), ..
+    __shared__ unsigned rows_l[2], spikes_l[2], team_l[2], crowd_l[3], done_l, updated_l, listed_l;  // rows of a step, of neurons (the others: of inputs), ..
     __shared__ unsigned fired_n[2];                               // how many fired in this step and the one before
     __shared__ unsigned long long ballot_l[kResBlock / kWave];
     const int tid = threadIdx.x, lane = lane_id();
@@ -745,8 +748,8 @@ __global__ __launch_bounds__(kResBlock) void sim_resident_lists_kernel(bmtk_glif
     const int mine = min(span, ne - e0);
     const bool own = tid < mine;
     const int e = e0 + tid;
-    unsigned *rows = reinterpret_cast<unsigned *>(ring_l + L * GLIF3_NREC * span);  // [2][kRowCap], a place per lane behind
-    unsigned short *fired_l = reinterpret_cast<unsigned short *>(rows + 2 * kRowCap + kWave);
+    unsigned *rows = reinterpret_cast<unsigned *>(ring_l + L * GLIF3_NREC * span);  // [2][row_cap], a place per lane behind
+    unsigned short *fired_l = reinterpret_cast<unsigned short *>(rows + 2 * row_cap + kWave);
     float *frac_l = reinterpret_cast<float *>(fired_l + kResBlock);
     unsigned *abort_word = s.res_sync + 1;
     unsigned long long *lists = lists_in(s.res_sync);
@@ -756,7 +759,7 @@ __global__ __launch_bounds__(kResBlock) void sim_resident_lists_kernel(bmtk_glif
     // a run before this one gave up and nobody has looked yet: do nothing, so that the failure is still there to see
     if (tid == 0) {
         go_on[0] = load_agent(abort_word) == 0u;
-        fired_n[0] = fired_n[1] = rows_l[0] = rows_l[1] = spikes_l[0] = spikes_l[1] = team_l[0] = team_l[1] = crowd_l[0] = crowd_l[1] = done_l = updated_l = listed_l = 0u;
+        fired_n[0] = fired_n[1] = rows_l[0] = rows_l[1] = spikes_l[0] = spikes_l[1] = team_l[0] = team_l[1] = done_l = updated_l = listed_l = 0u;
     }
     __syncthreads();
     if (!go_on[0]) return;
@@ -831,19 +834,30 @@ __global__ __launch_bounds__(kResBlock) void sim_resident_lists_kernel(bmtk_glif
         const bmtk_synapse *tab = !kUnified && of_input ? s.inp_packed : s.rec_packed;
         pull_bounds(b.lo, b.hi - b.lo, part, team, tab, RingSlice(ring_l, span, e0, L, slot_prev));  // the offsets never decrease
     };
+    // Input events events[a], events[a + step], .. of n, for a thread or team, without a stay in LDS; the first of them is at hand already.
+    auto pull_events = [&](const int32_t *events, unsigned a, unsigned step, unsigned n, int32_t next_source, unsigned part, unsigned team)
+        __attribute__((always_inline)) {
+        while (a < n) {
+            const int32_t source = next_source;
+            a += step;
+            if (a < n) next_source = events[a];
+            add_bounds(row_bounds(input_row(source)), true, part, team);
+        }
+    };
     // The rows of step k-1 into the ring slice.  Where they are listed before the update of step k already (`ask` ahead of it),
     // the bounds of a thread's first row are on their way meanwhile.
-    unsigned n_rows = 0u, team = 0u, at_row = 0u;
+    unsigned listed = 0u, n_rows = 0u, team = 0u, at_row = 0u;
     SegBounds first_row{0u, 0u};
     auto ask = [&](int k) __attribute__((always_inline)) {
         unsigned me = (unsigned)tid;
         asm volatile("" : "+v"(me));
         const int buf = (k - 1) & 1;
-        n_rows = (unsigned)__builtin_amdgcn_readfirstlane((int)rows_l[buf]);
+        listed = (unsigned)__builtin_amdgcn_readfirstlane((int)rows_l[buf]);
         team = (unsigned)__builtin_amdgcn_readfirstlane((int)team_l[buf]);
-        if (n_rows == kCrowded || wave == kWriter) n_rows = 0u;
+        const bool pulls = listed != kCrowded && wave != kWriter;
+        n_rows = pulls ? listed : 0u;
         at_row = me >> team;
-        if (at_row < n_rows) first_row = row_bounds(rows[buf * kRowCap + at_row]);
+        if (at_row < n_rows) first_row = row_bounds(rows[buf * row_cap + at_row]);
     };
     auto pull = [&](int k) __attribute__((always_inline)) {
         const int buf = (k - 1) & 1;
@@ -852,21 +866,28 @@ __global__ __launch_bounds__(kResBlock) void sim_resident_lists_kernel(bmtk_glif
             const SegBounds b = first_row;
             const bool of_input = at_row >= n_spikes;
             at_row += step;
-            if (at_row < n_rows) first_row = row_bounds(rows[buf * kRowCap + at_row]);
+            if (at_row < n_rows) first_row = row_bounds(rows[buf * row_cap + at_row]);
             add_bounds(b, of_input, part, 1u << team);
         }
     };
     // The same in a crowded step, by all threads: lists (row `row` of the history), ballots where a list did not suffice,
-    // and the events in_events[lo, hi).  What finds no room in the row list is pulled on the spot.
+    // and the events in_events[lo, hi).
     auto pull_crowded = [&](int k) __attribute__((always_inline)) {
-        const int64_t lo = events_at(k - 1), hi = events_at(k);  // (a step's events are below 2^31)
-        auto pull_row = [&](unsigned row) __attribute__((always_inline)) { add_bounds(row_bounds(row), (row & kInputTag) != 0u, 0u, 1u); };
-        crowded_rows<4>(lists_of(k - 1), !alone, span, hist + (int64_t)row_before() * (words + 1), words, (unsigned)(hi - lo), rows,
-                        kCrowdedCap, &crowd_l[k & 1], abort_word, spin_limit,
-                        [&](unsigned i) { return input_row(s.in_events[lo + i]); }, pull_row);
-        __syncthreads();
-        const unsigned total = min(crowd_l[k & 1], kCrowdedCap);
-        for (unsigned a = (unsigned)tid; a < total; a += kResBlock) pull_row(rows[a]);
+        const int64_t lo = events_at(k - 1);
+        const unsigned n_ev = (unsigned)(events_at(k) - lo);  // (a step's events are below 2^31)
+        const int32_t *const events = s.in_events + lo;
+        const bool beside = !alone && n_ev <= (unsigned)kResBlock && n_ev <= 2u * row_cap;  // listed with the neurons
+        if (!beside) pull_events(events, (unsigned)tid, kResBlock, n_ev, (unsigned)tid < n_ev ? events[tid] : 0, 0u, 1u);
+        if (!alone)
+            crowded_rows<kResBlock / kWave>(
+                lists_of(k - 1), list_tag(k - 1), span, hist + (int64_t)row_before() * (words + 1), words, beside ? n_ev : 0u,
+                [&](unsigned i) { return input_row(events[i]); }, rows, 2u * row_cap, crowd_l, abort_word, spin_limit,
+                [&](unsigned total) __attribute__((always_inline)) {
+                    for (unsigned a = (unsigned)tid; a < total; a += kResBlock) {
+                        const unsigned row = rows[a];
+                        add_bounds(row_bounds(row), (row & kInputTag) != 0u, 0u, 1u);
+                    }
+                });
         __syncthreads();
     };
     // The writer's part of a step: the list (the others wait for it), ballots, record.
@@ -937,7 +958,7 @@ __global__ __launch_bounds__(kResBlock) void sim_resident_lists_kernel(bmtk_glif
             }
             if (k > 0) {
                 if (!asked) ask(k);
-                if (rows_l[(k - 1) & 1] == kCrowded)
+                if (listed == kCrowded)
                     pull_crowded(k);
                 else
                     pull(k);
@@ -952,7 +973,7 @@ __global__ __launch_bounds__(kResBlock) void sim_resident_lists_kernel(bmtk_glif
     } else {
         ListLook seen;
         seen.none();
-        bool have = false, lost = false;  // the step in hand: its bounds are in LDS; given up
+        bool have = false, lost = false;  // the step in hand: its rows are in LDS; given up
         unsigned failed = 0u;
         int opaque_zero;
         asm volatile("v_mov_b32 %0, 0" : "=v"(opaque_zero));
@@ -968,7 +989,7 @@ __global__ __launch_bounds__(kResBlock) void sim_resident_lists_kernel(bmtk_glif
         // the input events of the step in hand, the first of them on their way
         int64_t ev_lo = events_at(0), ev_hi = events_at(1);
         long long ev_next = 0;
-        int32_t ev[kReaderEvents] = {0, 0, 0, 0};
+        int32_t ev[kReaderEvents] = {};
         // one more look in vain: false when it is time to give up
         auto again = [&]() __attribute__((always_inline)) -> bool {
             if (++failed > spin_limit) __hip_atomic_store(abort_word, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -978,9 +999,9 @@ __global__ __launch_bounds__(kResBlock) void sim_resident_lists_kernel(bmtk_glif
         auto take = [&](int k) __attribute__((always_inline)) {
             const int buf = k & 1;
             const unsigned n_ev = (unsigned)(ev_hi - ev_lo);
-            const unsigned me = (unsigned)lane_here(), spare = 2u * kRowCap + me, at_buf = (unsigned)buf * kRowCap;
+            const unsigned me = (unsigned)lane_here(), spare = 2u * row_cap + me, at_buf = (unsigned)buf * row_cap;
             have = true;
-            const unsigned total = rows_from_lists<false>(seen, lists_of(k), list_tag(k), span, rows, at_buf, kRowCap, spare, n_ev, again, lost);
+            const unsigned total = rows_from_lists<false>(seen, lists_of(k), list_tag(k), span, rows, at_buf, row_cap, spare, n_ev, again, lost);
             unsigned n = kCrowded;
             if (total != kCrowded) {
                 n = total + n_ev;
@@ -1018,10 +1039,7 @@ __global__ __launch_bounds__(kResBlock) void sim_resident_lists_kernel(bmtk_glif
                     else
                         lost = !again();
                 }
-                if (lane == 0) {
-                    go_on[k & 1] = !lost;
-                    crowd_l[k & 1] = 0u;
-                }
+                if (lane == 0) go_on[k & 1] = !lost;
             }
             // vmcnt(0): nothing is on its way here, and with that said the compiler does not wait for loads below before it
             // uses their registers again (a trip to memory at the busiest time)
@@ -1044,8 +1062,10 @@ __global__ __launch_bounds__(kResBlock) void sim_resident_lists_kernel(bmtk_glif
                 const int32_t *const from = s.in_events + ev_lo;
                 const unsigned me = (unsigned)lane_here();
 #pragma unroll
-                for (int i = 0; i < kReaderEvents; ++i)
+                for (int i = 0; i < kReaderEvents; ++i) {
+                    if ((unsigned)(i * kWave) >= n_ev) break;
                     if (i * kWave + me < n_ev) ev[i] = from[i * kWave + me];
+                }
             }
             have = false;
             failed = 0u;
@@ -1125,8 +1145,9 @@ int simulate_resident(const bmtk_glif3_sim &s, int64_t step0, int64_t n_steps, h
     const int hist = s.hist_slots ? s.hist_slots : 3;
     int slack = s.delay_offset < hist - 3 - s.delay_offset ? s.delay_offset : hist - 3 - s.delay_offset;
     slack = slack < kMaxSlack ? slack : kMaxSlack;
-    Resident r{step0, n_steps, s.res_span, s.res_groups, s.delay_offset, hist, slack, slack / 2 + 1};
-    const size_t lds = (size_t)s.ring_slots * GLIF3_NREC * s.res_span * sizeof(float) + kActCap * sizeof(int);
+    Resident r{step0, n_steps, s.res_span, s.res_groups, s.delay_offset, hist, slack, slack / 2 + 1, 0};
+    const size_t ring_bytes = (size_t)s.ring_slots * GLIF3_NREC * s.res_span * sizeof(float);
+    size_t lds = ring_bytes + kActCap * sizeof(int);
     // one table for recurrent and input rows lets the kernel drop the second set of pointers
     const bool has_inputs = s.in_ptr != nullptr;
     const int64_t rows = s.n_neurons + (has_inputs ? s.n_inputs : 0);
@@ -1136,6 +1157,11 @@ int simulate_resident(const bmtk_glif3_sim &s, int64_t step0, int64_t n_steps, h
     const int form = !unified || s.probe_col != nullptr ? kFormAny : (s.spike_count != nullptr ? kFormRecord : kFormLean);
     // without slack the workgroups exchange lists (a history of four rows: see sim_resident_lists_kernel)
     const bool lists = slack == 0 && s.delay_offset == 0 && s.res_fired != nullptr && s.res_groups <= kListGroups && hist >= 4;
+    if (lists) {
+        const size_t most = 4 * kActCap * sizeof(int), rest = kResLdsBytes - 256u - ring_bytes;
+        lds = ring_bytes + (rest < most ? rest : most) / 16 * 16;
+        r.row_cap = row_cap(lds - ring_bytes, form != kFormLean);
+    }
     const bool reader_owns = s.res_span > kReader * kWave;
     const void *const kernels[4][3] = {
         {reinterpret_cast<const void *>(sim_resident_kernel<false, kFormAny>),

@@ -21,6 +21,9 @@
 // whatever the number of trials side by side; then the table's segments, which every trial reads for itself.  Per step and
 // launch, ballots and a grid barrier per trial -> lists: 230,924 neurons x 8 6.9 -> 6.1 us, 20,011 x 20 5.0 -> 4.7,
 // 400,123 x 1 9.3 -> 6.6; 51,978 x 32, which reads 18 synapses a segment for 243 rows of each of four trials, 5.2 as before.
+// At tens of Hz, where steps are crowded (see resident.hip), the ballots were the faster exchange still: 60,000 x 4 at 24 / 45 Hz 12.3 /
+// 20.3 us a step against 14.9 / 24.8 (15.1 / 35.7 with every list of more than 19 neurons crowded), 230,924 x 2 at 28 Hz 56 against 62;
+// at 19 Hz 60,000 x 4 take 5.4 against 10.0.
 //
 // One trial of more neurons than the compute units have threads (resident.hip ends at 1024 to a workgroup) runs here with two
 // neurons to a thread and its ring in floats, 80 bytes a neuron: 400,123 neurons, 72 M synapses, 23 -> 6.6 us per step against
@@ -75,7 +78,7 @@ __global__ __launch_bounds__(kRbBlock) void sim_resident_batch_kernel(bmtk_glif3
     constexpr int kOwners = kRbReader * kWave;  // with two neurons to a thread: threads that own tid, tid + kOwners
     extern __shared__ unsigned long long rb_lds[];  // ring slice [slots * 4][span], then rb_list words for rows
     __shared__ int go_on[2];  // by the round, as rows_l is: a slot is written again only after a meeting behind all reads of it
-    __shared__ unsigned rows_l[2], crowd_l[2], done_l, updated_l, listed_l;  // rows of a round, ..
+    __shared__ unsigned rows_l[2], crowd_l[3], done_l, updated_l, listed_l;  // rows of a round, ..
     __shared__ unsigned fired_n[2];                  // how many fired in this step and the one before
     __shared__ unsigned short fired_l[kListMax + 1]; // the first of them, counted within the span
     const int tid = threadIdx.x, lane = lane_id();
@@ -109,7 +112,7 @@ __global__ __launch_bounds__(kRbBlock) void sim_resident_batch_kernel(bmtk_glif3
     auto ballots_of = [&](int k) { return hist + (int64_t)(k & (kListRows - 1)) * (q.words + 1); };
     if (tid == 0) {
         go_on[0] = rb_load(abort_word) == 0u;
-        rows_l[0] = rows_l[1] = crowd_l[0] = crowd_l[1] = done_l = updated_l = listed_l = fired_n[0] = fired_n[1] = 0u;
+        rows_l[0] = rows_l[1] = done_l = updated_l = listed_l = fired_n[0] = fired_n[1] = 0u;
     }
     __syncthreads();
     if (!go_on[0]) return;
@@ -258,43 +261,58 @@ __global__ __launch_bounds__(kRbBlock) void sim_resident_batch_kernel(bmtk_glif3
                 if (at_p + u * step < b.hi) add(sy[u], u == 0);
         }
     };
-    // The rows of round k: what fired in step k-1, and the input events handed over with it.  Where they are listed before the
-    // update of step k (`ask` ahead of it), the bounds of a thread's first row are on their way meanwhile.
-    unsigned n_rows = 0u, at_row = 0u;
-    RbBounds first_row{0u, 0u};
-    auto ask = [&](int k) __attribute__((always_inline)) {
-        unsigned me = (unsigned)tid;
-        asm volatile("" : "+v"(me));
-        n_rows = (unsigned)__builtin_amdgcn_readfirstlane((int)rows_l[k & 1]);
-        if (n_rows == kCrowded || wave == kRbWriter) n_rows = 0u;
-        at_row = me >> ts;
-        if (at_row < n_rows) first_row = row_bounds(rows[(k & 1) * row_cap + at_row]);
-    };
-    auto pull = [&](int k) __attribute__((always_inline)) {
-        const unsigned part = (unsigned)lane & ((1u << ts) - 1u);
-        while (at_row < n_rows) {
-            const RbBounds b = first_row;
-            at_row += (unsigned)kRbPullThreads >> ts;
-            if (at_row < n_rows) first_row = row_bounds(rows[(k & 1) * row_cap + at_row]);
-            add_segment(b, part, 1u << ts);
-        }
-    };
     // the input events of round k: rb_in_events[in_ptr[k] .. in_ptr[k + 1])
     const int64_t *in_ptr = q.has_events ? s.rb_in_ptr + (int64_t)trial * (n_steps + 1) : nullptr;
     // (a call's first step: the spikes of the step before were added by the call before it, and so were its events unless
     //  they are to be taken from this call's lists)
     auto with_events = [&](int k) { return in_ptr && (k > 0 || s.rb_late_events); };
+    // Input events events[a], events[a + step], .. of n, without a stay in LDS; the first of them is at hand already
+    auto pull_events = [&](const int32_t *events, unsigned a, unsigned step, unsigned n_ev, int32_t next_source) __attribute__((always_inline)) {
+        while (a < n_ev) {
+            const int32_t source = next_source;
+            a += step;
+            if (a < n_ev) next_source = events[a];
+            add_segment(row_bounds((unsigned)n + (unsigned)source), (unsigned)lane & ((1u << ts) - 1u), 1u << ts);
+        }
+    };
+    // The rows of round k: what fired in step k-1, and the input events handed over with it.  Where they are listed before the
+    // update of step k (`ask` ahead of it), the bounds of a thread's first row are on their way meanwhile.
+    unsigned listed = 0u, n_rows = 0u, at_row = 0u;
+    RbBounds first_row{0u, 0u};
+    auto ask = [&](int k) __attribute__((always_inline)) {
+        unsigned me = (unsigned)tid;
+        asm volatile("" : "+v"(me));
+        listed = (unsigned)__builtin_amdgcn_readfirstlane((int)rows_l[k & 1]);
+        const bool pulls = listed != kCrowded && wave != kRbWriter;
+        n_rows = pulls ? listed : 0u;
+        at_row = me >> ts;
+        if (at_row < n_rows) first_row = row_bounds(rows[(k & 1) * row_cap + at_row]);
+    };
+    auto pull = [&](int k) __attribute__((always_inline)) {
+        const unsigned part = (unsigned)lane & ((1u << ts) - 1u), step = (unsigned)kRbPullThreads >> ts;
+        while (at_row < n_rows) {
+            const RbBounds b = first_row;
+            at_row += step;
+            if (at_row < n_rows) first_row = row_bounds(rows[(k & 1) * row_cap + at_row]);
+            add_segment(b, part, 1u << ts);
+        }
+    };
     auto pull_crowded = [&](int k) __attribute__((always_inline)) {
-        const unsigned lo = with_events(k) ? (unsigned)in_ptr[k] : 0u, hi = with_events(k) ? (unsigned)in_ptr[k + 1] : 0u;
-        const unsigned cap = (unsigned)s.rb_list;
-        auto pull_row = [&](unsigned row) __attribute__((always_inline)) { add_segment(row_bounds(row), 0u, 1u); };
-        crowded_rows<kPer == 1 ? 4 : 8>(lists_of(k - 1), k > 0, span, ballots_of(k - 1), q.words, hi - lo, rows, cap, &crowd_l[k & 1],
-                                        abort_word, spin_limit, [&](unsigned i) { return (unsigned)n + (unsigned)s.rb_in_events[lo + i]; },
-                                        pull_row);
-        __syncthreads();
-        const unsigned total = min(crowd_l[k & 1], cap);
-        for (unsigned a = (unsigned)tid >> ts; a < total; a += (unsigned)kRbBlock >> ts)
-            add_segment(row_bounds(rows[a]), (unsigned)lane & ((1u << ts) - 1u), 1u << ts);
+        const unsigned lo = with_events(k) ? (unsigned)in_ptr[k] : 0u, n_ev = with_events(k) ? (unsigned)in_ptr[k + 1] - lo : 0u;
+        const int32_t *const events = s.rb_in_events + lo;
+        const bool beside = k > 0 && n_ev <= (unsigned)kRbBlock && n_ev <= (unsigned)s.rb_list;  // listed with the neurons
+        if (!beside) {
+            const unsigned a = (unsigned)tid >> ts;
+            pull_events(events, a, (unsigned)kRbBlock >> ts, n_ev, a < n_ev ? events[a] : 0);
+        }
+        if (k > 0)
+            crowded_rows<kPer * kRbWaves>(
+                lists_of(k - 1), list_tag(k - 1), span, ballots_of(k - 1), q.words, beside ? n_ev : 0u,
+                [&](unsigned i) { return (unsigned)n + (unsigned)events[i]; }, rows, (unsigned)s.rb_list, crowd_l, abort_word, spin_limit,
+                [&](unsigned total) __attribute__((always_inline)) {
+                    for (unsigned a = (unsigned)tid >> ts; a < total; a += (unsigned)kRbBlock >> ts)
+                        add_segment(row_bounds(rows[a]), (unsigned)lane & ((1u << ts) - 1u), 1u << ts);
+                });
         __syncthreads();
     };
     // the pulls of round k are complete
@@ -330,7 +348,7 @@ __global__ __launch_bounds__(kRbBlock) void sim_resident_batch_kernel(bmtk_glif3
             }
             if (k < n_steps) volley(k);
             if (!asked) ask(k);
-            if (rows_l[k & 1] == kCrowded)
+            if (listed == kCrowded)
                 pull_crowded(k);
             else
                 pull(k);
@@ -349,13 +367,15 @@ __global__ __launch_bounds__(kRbBlock) void sim_resident_batch_kernel(bmtk_glif3
         unsigned ev_lo = with_events(0) ? (unsigned)in_ptr[0] : 0u, ev_hi = with_events(0) ? (unsigned)in_ptr[1] : 0u;
         unsigned next_lo = 0u, next_hi = 0u;
         if (in_ptr) next_lo = (unsigned)in_ptr[1], next_hi = (unsigned)in_ptr[min(2, n_steps + 1)];
-        int32_t ev[kRbEvents] = {0, 0, 0, 0};
+        int32_t ev[kRbEvents] = {};
         auto ask_events = [&]() __attribute__((always_inline)) {
             const unsigned n_ev = ev_hi - ev_lo, me = (unsigned)lane_here();
             const int32_t *const from = s.rb_in_events + ev_lo;
 #pragma unroll
-            for (int i = 0; i < kRbEvents; ++i)
+            for (int i = 0; i < kRbEvents; ++i) {
+                if ((unsigned)(i * kWave) >= n_ev) break;
                 if (i * kWave + me < n_ev) ev[i] = from[i * kWave + me];
+            }
         };
         ask_events();
         // one more look in vain: false when it is time to give up
@@ -391,7 +411,6 @@ __global__ __launch_bounds__(kRbBlock) void sim_resident_batch_kernel(bmtk_glif3
                 }
                 if (lane == 0) {
                     rows_l[k & 1] = total == kCrowded ? kCrowded : total + n_ev;
-                    crowd_l[k & 1] = 0u;
                     if (!lost) store_lds(&listed_l, (unsigned)k + 1u);
                 }
             }

@@ -177,3 +177,40 @@ def test_scratch_on_any_32_bit_word(batch, monkeypatch):
         bits.append(sim.run(STEPS)["bits"])
         sim.check()
     assert int(bits[0].ne(0).sum()) > 50 and torch.equal(bits[0], bits[1])
+
+
+@pytest.mark.parametrize("form", ["bits", "two_tables", "trials"])
+@pytest.mark.parametrize("n", [4100, 6000, 12300])
+def test_volleys_of_any_number_of_workgroups(n, form, monkeypatch):
+    """Volleys (the ballots of some workgroups, the lists of others) of 65, 94 and 193 workgroups: 16, 8 and 4 threads share a
+    workgroup's words, and rows come in one handing out or several.  Two tables: membrane probes rule out the joint one."""
+    span, batch = 64, 3 if form == "trials" else 1
+    rng = np.random.default_rng(n)
+    indptr = np.arange(n + 1, dtype=np.int32) * 30
+    idx = rng.integers(0, n, n * 30).astype(np.int32)
+    rec = (indptr, idx, (rng.integers(1, 200, idx.size) / 4.0).astype(np.float32), rng.integers(1, 5, idx.size).astype(np.uint8),
+           rng.integers(0, 4, idx.size).astype(np.uint8))
+    par = synthetic.random_cells(rng, n)
+    u = np.zeros((n, batch), np.float32)
+    for b in range(batch):
+        for g, e0 in enumerate(range(0, n, span)):
+            mine = min(span, n - e0)
+            pick = e0 + rng.permutation(mine)[:min(mine, (0, 3, 20, 39, 40, 52, 64)[(g + b) % 7])]
+            u[pick, b] = (par[PAR["V_TH"]] - par[PAR["E_L"]])[pick] * 3.0
+    i_ext = rng.uniform(0.0, 300.0, n * batch).astype(np.float32)
+    groups = -(-n // span)
+    monkeypatch.setattr(simulator, "resident_span", lambda *a, **k: span)
+    monkeypatch.setattr(simulator, "resident_trials_plan", lambda *a: dict(span=span, groups=groups, ways=1, passes=3, list=2100))
+    got = []
+    for resident in (False, True):
+        sim = simulator.Glif3Simulator(n, par, 1.0, batch=batch, rec=rec, i_ext=i_ext, resident=resident and batch == 1,
+                                       resident_trials=resident and batch > 1)
+        sim.state.V.copy_(torch.as_tensor(u.reshape(-1)))
+        if form == "two_tables":
+            sim.set_probes(np.arange(0, n, 11), every=3)
+        out = sim.run(40)
+        got.append(dict(bits=out["bits"], V=sim.state.V, y1=sim.state.y1, y2=sim.state.y2))
+        sim.check()
+    assert int(got[0]["bits"][0].ne(0).sum()) > groups // 2
+    for key in got[0]:
+        assert torch.equal(got[0][key], got[1][key]), key
