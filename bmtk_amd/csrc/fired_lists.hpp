@@ -146,6 +146,7 @@ __device__ __forceinline__ unsigned list_id(unsigned long long word, int i)
 // Every instruction here is one of a single wavefront, four clocks each and more beside three others on its SIMD: what no
 // list holds is not stepped through, and a store too many is cheaper than a branch of lanes.
 constexpr unsigned kCrowded = 0xFFFFFFFFu;  // in place of a number of rows
+constexpr unsigned kMoreEvents = 1u << 30;  // beside it: the step has more input events than the reader has listed
 template <bool kFew, typename Again>
 __device__ __forceinline__ unsigned rows_from_lists(ListLook &seen, const ListRow &lists, unsigned tag, int span, unsigned *rows,
                                                     unsigned to, unsigned cap, unsigned spare, unsigned more, Again again, bool &lost)

@@ -711,7 +711,7 @@ __global__ __launch_bounds__(kResBlock) void sim_resident_kernel(bmtk_glif3_sim 
 // then share the way to memory; another order of rows for each workgroup of an XCD: no difference.
 constexpr int kReader = kResBlock / kWave - 1, kWriter = kReader - 1;
 constexpr int kPullThreads = kWriter * kWave;
-constexpr int kReaderEvents = 4;    // input events a lane of the reader asks for ahead
+constexpr int kReaderEvents = 8;    // input events a lane of the reader asks for ahead
 // LDS behind the ring slice, `bytes` of it: rows of two steps, a place per lane of the reader for what is none, the neurons of this
 // workgroup that fired and, for a record, their crossing fractions.  At least kActCap words (3,808 rows of a step, with a record 3,296),
 // and all that the ring slice leaves, up to four times as many: crowded steps cost half as much again.
@@ -846,7 +846,12 @@ __global__ __launch_bounds__(kResBlock) void sim_resident_lists_kernel(bmtk_glif
     };
     // The rows of step k-1 into the ring slice.  Where they are listed before the update of step k already (`ask` ahead of it),
     // the bounds of a thread's first row are on their way meanwhile.
-    unsigned listed = 0u, n_rows = 0u, team = 0u, at_row = 0u;
+    // What the reader has no lanes for, input events from the kReaderEvents * kWave-th on, follows the listed rows, straight from the input
+    // lists.  (Put into the rows by the reader, 64 at a time, they made it the one all waited for: 60,000 neurons, 800 / 2,000 / 3,600
+    // events a step 4.5 / 10.0 / 17.1 us, with ballots 4.0 / 7.5 / 12.9, so 3.7 / 5.6 / 7.6; eight of a lane under way at a time 3.8 / 5.9 / 8.3.)
+    unsigned listed = 0u, n_rows = 0u, team = 0u, at_row = 0u, n_more = 0u;
+    const int32_t *more_events = nullptr;
+    int32_t next_source = 0;
     SegBounds first_row{0u, 0u};
     auto ask = [&](int k) __attribute__((always_inline)) {
         unsigned me = (unsigned)tid;
@@ -855,19 +860,32 @@ __global__ __launch_bounds__(kResBlock) void sim_resident_lists_kernel(bmtk_glif
         listed = (unsigned)__builtin_amdgcn_readfirstlane((int)rows_l[buf]);
         team = (unsigned)__builtin_amdgcn_readfirstlane((int)team_l[buf]);
         const bool pulls = listed != kCrowded && wave != kWriter;
-        n_rows = pulls ? listed : 0u;
+        n_rows = pulls ? listed & ~kMoreEvents : 0u;
         at_row = me >> team;
         if (at_row < n_rows) first_row = row_bounds(rows[buf * row_cap + at_row]);
+        n_more = 0u;
+        if (pulls && (listed & kMoreEvents)) {
+            const int64_t from = events_at(k - 1) + kReaderEvents * kWave;
+            n_more = (unsigned)(events_at(k) - from);
+            more_events = s.in_events + from;
+            if (at_row >= n_rows && at_row - n_rows < n_more) next_source = more_events[at_row - n_rows];
+        }
     };
     auto pull = [&](int k) __attribute__((always_inline)) {
         const int buf = (k - 1) & 1;
         const unsigned part = (unsigned)lane & ((1u << team) - 1u), step = (unsigned)kPullThreads >> team, n_spikes = spikes_l[buf];
+        const bool at_hand = at_row >= n_rows;
         while (at_row < n_rows) {
             const SegBounds b = first_row;
             const bool of_input = at_row >= n_spikes;
             at_row += step;
             if (at_row < n_rows) first_row = row_bounds(rows[buf * row_cap + at_row]);
             add_bounds(b, of_input, part, 1u << team);
+        }
+        if (n_more != 0u) {
+            const unsigned a = at_row - n_rows;
+            if (!at_hand && a < n_more) next_source = more_events[a];
+            pull_events(more_events, a, step, n_more, next_source, part, 1u << team);
         }
     };
     // The same in a crowded step, by all threads: lists (row `row` of the history), ballots where a list did not suffice,
@@ -998,13 +1016,13 @@ __global__ __launch_bounds__(kResBlock) void sim_resident_lists_kernel(bmtk_glif
         // the rows of step k, whose lists have been seen, into LDS
         auto take = [&](int k) __attribute__((always_inline)) {
             const int buf = k & 1;
-            const unsigned n_ev = (unsigned)(ev_hi - ev_lo);
+            const unsigned n_ev = (unsigned)(ev_hi - ev_lo), n_listed = min(n_ev, (unsigned)(kReaderEvents * kWave));
             const unsigned me = (unsigned)lane_here(), spare = 2u * row_cap + me, at_buf = (unsigned)buf * row_cap;
             have = true;
-            const unsigned total = rows_from_lists<false>(seen, lists_of(k), list_tag(k), span, rows, at_buf, row_cap, spare, n_ev, again, lost);
+            const unsigned total = rows_from_lists<false>(seen, lists_of(k), list_tag(k), span, rows, at_buf, row_cap, spare, n_listed, again, lost);
             unsigned n = kCrowded;
             if (total != kCrowded) {
-                n = total + n_ev;
+                n = total + n_listed;
 #pragma unroll
                 for (int i = 0; i < kReaderEvents; ++i) {
                     if ((unsigned)(i * kWave) >= n_ev) break;
@@ -1013,13 +1031,12 @@ __global__ __launch_bounds__(kResBlock) void sim_resident_lists_kernel(bmtk_glif
                     asm volatile("" : "+v"(source));  // (not looked at ahead of the lists)
                     rows[a < n_ev ? at_buf + total + a : spare] = input_row(source);
                 }
-                for (unsigned a = kReaderEvents * kWave + me; a < n_ev; a += kWave) rows[at_buf + total + a] = input_row(s.in_events[ev_lo + a]);
             }
             unsigned ts = 0u;
             if (n != kCrowded)
-                while (ts < max_team && (n << (ts + 1u)) <= (unsigned)kPullThreads) ++ts;
+                while (ts < max_team && ((n + n_ev - n_listed) << (ts + 1u)) <= (unsigned)kPullThreads) ++ts;
             if (lane == 0) {
-                rows_l[buf] = n;
+                rows_l[buf] = n == kCrowded || n_ev == n_listed ? n : n | kMoreEvents;
                 spikes_l[buf] = total;
                 team_l[buf] = ts;
                 store_lds(&listed_l, lost ? 0u : (unsigned)k + 1u);

@@ -46,7 +46,7 @@ constexpr int kRbReader = kRbWaves - 1, kRbWriter = kRbReader - 1;  // wavefront
 constexpr int kRbPullThreads = kRbWriter * kWave;
 constexpr unsigned kRbMaxSpin = 4000000u; // looks in vain before giving up (seconds)
 constexpr int kRbTogether = 6;            // synapses a lane has in flight (20,011 x 20, 8 lanes to 33: 4 of them 9.6 us per step, 6 9.3)
-constexpr int kRbEvents = 4;              // input events a lane of the reader asks for ahead
+constexpr int kRbEvents = 8;              // input events a lane of the reader asks for ahead
 
 struct RbLaunch {
     int64_t step0;
@@ -277,24 +277,40 @@ __global__ __launch_bounds__(kRbBlock) void sim_resident_batch_kernel(bmtk_glif3
     };
     // The rows of round k: what fired in step k-1, and the input events handed over with it.  Where they are listed before the
     // update of step k (`ask` ahead of it), the bounds of a thread's first row are on their way meanwhile.
-    unsigned listed = 0u, n_rows = 0u, at_row = 0u;
+    // Events that the reader has no lanes for follow the listed rows (see resident.hip).
+    unsigned listed = 0u, n_rows = 0u, at_row = 0u, n_more = 0u;
+    const int32_t *more_events = nullptr;
+    int32_t next_source = 0;
     RbBounds first_row{0u, 0u};
     auto ask = [&](int k) __attribute__((always_inline)) {
         unsigned me = (unsigned)tid;
         asm volatile("" : "+v"(me));
         listed = (unsigned)__builtin_amdgcn_readfirstlane((int)rows_l[k & 1]);
         const bool pulls = listed != kCrowded && wave != kRbWriter;
-        n_rows = pulls ? listed : 0u;
+        n_rows = pulls ? listed & ~kMoreEvents : 0u;
         at_row = me >> ts;
         if (at_row < n_rows) first_row = row_bounds(rows[(k & 1) * row_cap + at_row]);
+        n_more = 0u;
+        if (pulls && (listed & kMoreEvents)) {
+            const unsigned from = (unsigned)in_ptr[k] + kRbEvents * kWave;
+            n_more = (unsigned)in_ptr[k + 1] - from;
+            more_events = s.rb_in_events + from;
+            if (at_row >= n_rows && at_row - n_rows < n_more) next_source = more_events[at_row - n_rows];
+        }
     };
     auto pull = [&](int k) __attribute__((always_inline)) {
         const unsigned part = (unsigned)lane & ((1u << ts) - 1u), step = (unsigned)kRbPullThreads >> ts;
+        const bool at_hand = at_row >= n_rows;
         while (at_row < n_rows) {
             const RbBounds b = first_row;
             at_row += step;
             if (at_row < n_rows) first_row = row_bounds(rows[(k & 1) * row_cap + at_row]);
             add_segment(b, part, 1u << ts);
+        }
+        if (n_more != 0u) {
+            const unsigned a = at_row - n_rows;
+            if (!at_hand && a < n_more) next_source = more_events[a];
+            pull_events(more_events, a, step, n_more, next_source);
         }
     };
     auto pull_crowded = [&](int k) __attribute__((always_inline)) {
@@ -397,7 +413,8 @@ __global__ __launch_bounds__(kRbBlock) void sim_resident_batch_kernel(bmtk_glif3
             }
             if (!lost) {
                 const unsigned me = (unsigned)lane_here(), spare = 2u * row_cap + me, to = (unsigned)(k & 1) * row_cap, n_ev = ev_hi - ev_lo;
-                const unsigned total = rows_from_lists<kFew>(seen, lists_of(k - 1), list_tag(k - 1), span, rows, to, row_cap, spare, n_ev, again, lost);
+                const unsigned n_listed = min(n_ev, (unsigned)(kRbEvents * kWave));
+                const unsigned total = rows_from_lists<kFew>(seen, lists_of(k - 1), list_tag(k - 1), span, rows, to, row_cap, spare, n_listed, again, lost);
                 if (total != kCrowded) {
 #pragma unroll
                     for (int i = 0; i < kRbEvents; ++i) {
@@ -407,10 +424,9 @@ __global__ __launch_bounds__(kRbBlock) void sim_resident_batch_kernel(bmtk_glif3
                         asm volatile("" : "+v"(source));  // (not looked at ahead of the lists)
                         rows[a < n_ev ? to + total + a : spare] = (unsigned)n + (unsigned)source;
                     }
-                    for (unsigned a = kRbEvents * kWave + me; a < n_ev; a += kWave) rows[to + total + a] = (unsigned)n + (unsigned)s.rb_in_events[ev_lo + a];
                 }
                 if (lane == 0) {
-                    rows_l[k & 1] = total == kCrowded ? kCrowded : total + n_ev;
+                    rows_l[k & 1] = total == kCrowded ? kCrowded : (total + n_listed) | (n_ev > n_listed ? kMoreEvents : 0u);
                     if (!lost) store_lds(&listed_l, (unsigned)k + 1u);
                 }
             }

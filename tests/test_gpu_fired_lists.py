@@ -214,3 +214,36 @@ def test_volleys_of_any_number_of_workgroups(n, form, monkeypatch):
     assert int(got[0]["bits"][0].ne(0).sum()) > groups // 2
     for key in got[0]:
         assert torch.equal(got[0][key], got[1][key]), key
+
+
+@pytest.mark.parametrize("form", ["bits", "record", "probes"])
+@pytest.mark.parametrize("batch,places", [(1, 0), (5, 700), (5, 8192)])
+def test_steps_of_many_input_events(batch, places, form, monkeypatch):
+    """Around the numbers of events that the reader lists (512), that one turn of the pulling threads takes beside them, that trials'
+    rows have room for (half of `places` less 64), and far more of them, on any side of a step with few."""
+    if form != "bits" and batch > 1:
+        pytest.skip("trials keep no record and no probes")
+    par, rec, inp, _, _ = _network(6)
+    rec, inp = [t[:3] + (np.minimum(t[3], 4),) + t[4:] for t in (rec, inp)]
+    inp = inp[:2] + (inp[2] / 32,) + inp[3:]
+    n_in, rng = 6000, np.random.default_rng(8)
+    edges = [0, 1, 63, 64, 255, 256, 257, 317, 318, 319, 511, 512, 513, 1023, 1025, 1407, 1408, 1409, 2048, 3297, 3809, 4063, 4064, 4065, 5999]
+    per_step = np.array([e for e in edges] + [300, 300, 5000, 300, 2000, 4000, 2000] + list(rng.permutation(edges)))
+    ptr = np.concatenate([[0], np.cumsum(per_step)]).astype(np.int64)
+    events = np.concatenate([np.sort(rng.choice(n_in, c, replace=False)) for c in per_step]).astype(np.int32)
+    monkeypatch.setattr(simulator, "resident_span", lambda *a, **k: 64)
+    monkeypatch.setattr(simulator, "resident_trials_plan", lambda *a: dict(span=64, groups=47, ways=2, passes=3, list=places))
+    got = []
+    for resident in (False, True):
+        sim = simulator.Glif3Simulator(N, par, 1.0, batch=batch, rec=rec, inp=inp, resident=resident and batch == 1,
+                                       resident_trials=resident and batch > 1)
+        sim.state.V.copy_(torch.as_tensor(np.repeat(_start(par, 64, 5), batch)))
+        sim.set_input_events(ptr, events * batch + (2 if batch > 1 else 0))
+        if form == "probes":
+            sim.set_probes(np.arange(0, N, 7), every=2)
+        out = sim.run(per_step.size, record_cap=N * per_step.size * 2 if form == "record" else 0)
+        got.append(dict(bits=out["bits"], V=sim.state.V, y1=sim.state.y1, y2=sim.state.y2))
+        sim.check()
+    assert int(got[0]["bits"].ne(0).sum()) > 50
+    for key in got[0]:
+        assert torch.equal(got[0][key], got[1][key]), key
