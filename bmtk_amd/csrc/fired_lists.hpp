@@ -103,8 +103,7 @@ struct ListLook {
         for (int u = 0; u < kListRounds; ++u) v[u][0] = v[u][1] = 0ull;
     }
     // asks once for words `from`, `from` + 1 of all G lists; true when every workgroup has published them in the wanted step
-    // (kFew: lists are seldom more than a wavefront's lanes, and a branch past the rest is worth it)
-    template <bool kFew>
+    // (beyond the G-th the last list over again: with a branch past those, 16 to 256 lists took the same time within 2 %)
     __device__ __forceinline__ bool look(const ListRow &row, unsigned tag, int from = 0)
     {
         const unsigned lane = (unsigned)lane_here();
@@ -112,17 +111,14 @@ struct ListLook {
         const unsigned stride = 8u * (from ? kListWords - kListQuickWords : kListQuickWords);
 #pragma unroll
         for (int u = 0; u < kListRounds; ++u) {
-            if (kFew && u * kWave >= row.G) break;
             const unsigned long long *p = reinterpret_cast<const unsigned long long *>(base + min(u * kWave + lane, (unsigned)row.G - 1u) * stride);
             v[u][0] = load_agent64(p);
             v[u][1] = load_agent64(p + 1);
         }
         unsigned differs = 0u;
 #pragma unroll
-        for (int u = 0; u < kListRounds; ++u) {
-            if (kFew && u * kWave >= row.G) break;
+        for (int u = 0; u < kListRounds; ++u)
             differs |= ((unsigned)(v[u][0] >> 32) ^ (tag << (kListTagAt - 32))) | ((unsigned)(v[u][1] >> 32) ^ (tag << (kListTagAt - 32)));
-        }
         return __ballot((differs >> (kListTagAt - 32)) != 0u) == 0ull;
     }
     __device__ __forceinline__ unsigned count(int u, int G) const
@@ -147,7 +143,7 @@ __device__ __forceinline__ unsigned list_id(unsigned long long word, int i)
 // list holds is not stepped through, and a store too many is cheaper than a branch of lanes.
 constexpr unsigned kCrowded = 0xFFFFFFFFu;  // in place of a number of rows
 constexpr unsigned kMoreEvents = 1u << 30;  // beside it: the step has more input events than the reader has listed
-template <bool kFew, typename Again>
+template <typename Again>
 __device__ __forceinline__ unsigned rows_from_lists(ListLook &seen, const ListRow &lists, unsigned tag, int span, unsigned *rows,
                                                     unsigned to, unsigned cap, unsigned spare, unsigned more, Again again, bool &lost)
 {
@@ -185,7 +181,7 @@ __device__ __forceinline__ unsigned rows_from_lists(ListLook &seen, const ListRo
     for (int from = kListQuickWords; from < kListWords; from += 2) {
         const unsigned j0 = 5u * from - 1u;
         if (!__any(most > j0)) break;
-        while (!seen.template look<kFew>(lists, tag, from)) {
+        while (!seen.look(lists, tag, from)) {
             if (!again()) {
                 lost = true;
                 return kCrowded;

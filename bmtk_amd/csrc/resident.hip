@@ -1019,7 +1019,7 @@ __global__ __launch_bounds__(kResBlock) void sim_resident_lists_kernel(bmtk_glif
             const unsigned n_ev = (unsigned)(ev_hi - ev_lo), n_listed = min(n_ev, (unsigned)(kReaderEvents * kWave));
             const unsigned me = (unsigned)lane_here(), spare = 2u * row_cap + me, at_buf = (unsigned)buf * row_cap;
             have = true;
-            const unsigned total = rows_from_lists<false>(seen, lists_of(k), list_tag(k), span, rows, at_buf, row_cap, spare, n_listed, again, lost);
+            const unsigned total = rows_from_lists(seen, lists_of(k), list_tag(k), span, rows, at_buf, row_cap, spare, n_listed, again, lost);
             unsigned n = kCrowded;
             if (total != kCrowded) {
                 n = total + n_listed;
@@ -1051,7 +1051,7 @@ __global__ __launch_bounds__(kResBlock) void sim_resident_lists_kernel(bmtk_glif
             if (k > 0) {
                 if (!alone) __builtin_amdgcn_s_sleep(8);
                 while (!have && !lost) {
-                    if (alone || seen.look<false>(lists_of(k - 1), list_tag(k - 1)))
+                    if (alone || seen.look(lists_of(k - 1), list_tag(k - 1)))
                         take(k - 1);
                     else
                         lost = !again();

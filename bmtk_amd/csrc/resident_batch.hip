@@ -71,7 +71,7 @@ struct __attribute__((packed, aligned(4))) RbBounds {
 // (from_fixed), or floats where a workgroup's neurons are too many for that (batch 1): fp32 atomics into device memory are what
 // it then takes the place of.  kSave: potentials and step flags of every step go to rb_save_*, trial by trial; by_step_kernel
 // puts them in their order.  kReaderOwns: spans above 960 with a neuron to a thread.
-template <int kPer, typename Sum, bool kSave, bool kReaderOwns, bool kFew>
+template <int kPer, typename Sum, bool kSave, bool kReaderOwns>
 __global__ __launch_bounds__(kRbBlock) void sim_resident_batch_kernel(bmtk_glif3_sim s, RbLaunch q)
 {
     constexpr bool kFixed = sizeof(Sum) == 8;
@@ -409,12 +409,12 @@ __global__ __launch_bounds__(kRbBlock) void sim_resident_batch_kernel(bmtk_glif3
             failed = 0u;
             if (k > 0) {
                 __builtin_amdgcn_s_sleep(8);  // (see resident.hip)
-                while (!lost && !seen.look<kFew>(lists_of(k - 1), list_tag(k - 1))) lost = !again();
+                while (!lost && !seen.look(lists_of(k - 1), list_tag(k - 1))) lost = !again();
             }
             if (!lost) {
                 const unsigned me = (unsigned)lane_here(), spare = 2u * row_cap + me, to = (unsigned)(k & 1) * row_cap, n_ev = ev_hi - ev_lo;
                 const unsigned n_listed = min(n_ev, (unsigned)(kRbEvents * kWave));
-                const unsigned total = rows_from_lists<kFew>(seen, lists_of(k - 1), list_tag(k - 1), span, rows, to, row_cap, spare, n_listed, again, lost);
+                const unsigned total = rows_from_lists(seen, lists_of(k - 1), list_tag(k - 1), span, rows, to, row_cap, spare, n_listed, again, lost);
                 if (total != kCrowded) {
 #pragma unroll
                     for (int i = 0; i < kRbEvents; ++i) {
@@ -547,19 +547,12 @@ int simulate_resident_batch(const bmtk_glif3_sim &s, int64_t step0, int64_t n_st
     q.unit = ldexp(1.0, -32 - s.sum_shift);
     BMTK_REQUIRE((wide ? 2 * kRbReader * kWave : kRbBlock) * (int64_t)kListGroups >= n, "glif3_simulate_fwd: more neurons than resident trials can hold");
     const bool owns = span > kRbReader * kWave;
-    // few: a trial of up to 128 workgroups, whose lists take a wavefront's lanes once or twice; one of more (or a wide one) asks
-    // for all four lists of a lane without a branch (230,924 x 8, 241 workgroups to a trial: 53.2 -> 52.5 us per step)
-    const bool few = G <= 2 * kWave;
-    const void *const kernels[2][2][2] = {
-        {{reinterpret_cast<const void *>(sim_resident_batch_kernel<1, unsigned long long, false, false, false>),
-          reinterpret_cast<const void *>(sim_resident_batch_kernel<1, unsigned long long, false, false, true>)},
-         {reinterpret_cast<const void *>(sim_resident_batch_kernel<1, unsigned long long, false, true, false>),
-          reinterpret_cast<const void *>(sim_resident_batch_kernel<1, unsigned long long, false, true, true>)}},
-        {{reinterpret_cast<const void *>(sim_resident_batch_kernel<1, unsigned long long, true, false, false>),
-          reinterpret_cast<const void *>(sim_resident_batch_kernel<1, unsigned long long, true, false, true>)},
-         {reinterpret_cast<const void *>(sim_resident_batch_kernel<1, unsigned long long, true, true, false>),
-          reinterpret_cast<const void *>(sim_resident_batch_kernel<1, unsigned long long, true, true, true>)}}};
-    const void *kernel = wide ? reinterpret_cast<const void *>(sim_resident_batch_kernel<2, float, false, false, false>) : kernels[save][owns][few];
+    const void *const kernels[2][2] = {
+        {reinterpret_cast<const void *>(sim_resident_batch_kernel<1, unsigned long long, false, false>),
+         reinterpret_cast<const void *>(sim_resident_batch_kernel<1, unsigned long long, false, true>)},
+        {reinterpret_cast<const void *>(sim_resident_batch_kernel<1, unsigned long long, true, false>),
+         reinterpret_cast<const void *>(sim_resident_batch_kernel<1, unsigned long long, true, true>)}};
+    const void *kernel = wide ? reinterpret_cast<const void *>(sim_resident_batch_kernel<2, float, false, false>) : kernels[save][owns];
     hipError_t err = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (err != hipSuccess) {
         set_error("glif3_simulate_fwd: resident trials need %zu bytes of LDS: %s", lds, hipGetErrorString(err));
