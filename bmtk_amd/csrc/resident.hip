@@ -834,16 +834,6 @@ __global__ __launch_bounds__(kResBlock) void sim_resident_lists_kernel(bmtk_glif
         const bmtk_synapse *tab = !kUnified && of_input ? s.inp_packed : s.rec_packed;
         pull_bounds(b.lo, b.hi - b.lo, part, team, tab, RingSlice(ring_l, span, e0, L, slot_prev));  // the offsets never decrease
     };
-    // Input events events[a], events[a + step], .. of n, for a thread or team, without a stay in LDS; the first of them is at hand already.
-    auto pull_events = [&](const int32_t *events, unsigned a, unsigned step, unsigned n, int32_t next_source, unsigned part, unsigned team)
-        __attribute__((always_inline)) {
-        while (a < n) {
-            const int32_t source = next_source;
-            a += step;
-            if (a < n) next_source = events[a];
-            add_bounds(row_bounds(input_row(source)), true, part, team);
-        }
-    };
     // The rows of step k-1 into the ring slice.  Where they are listed before the update of step k already (`ask` ahead of it),
     // the bounds of a thread's first row are on their way meanwhile.
     // What the reader has no lanes for, input events from the kReaderEvents * kWave-th on, follows the listed rows, straight from the input
@@ -883,22 +873,26 @@ __global__ __launch_bounds__(kResBlock) void sim_resident_lists_kernel(bmtk_glif
             add_bounds(b, of_input, part, 1u << team);
         }
         if (n_more != 0u) {
-            const unsigned a = at_row - n_rows;
+            unsigned a = at_row - n_rows;
             if (!at_hand && a < n_more) next_source = more_events[a];
-            pull_events(more_events, a, step, n_more, next_source, part, 1u << team);
+            while (a < n_more) {
+                const int32_t source = next_source;
+                a += step;
+                if (a < n_more) next_source = more_events[a];
+                add_bounds(row_bounds(input_row(source)), true, part, 1u << team);
+            }
         }
     };
-    // The same in a crowded step, by all threads: lists (row `row` of the history), ballots where a list did not suffice,
-    // and the events in_events[lo, hi).
+    // A crowded step, by all threads: lists (row `row` of the history), ballots where a list did not suffice, a thread's input event.
+    // Further events are left to pull.
     auto pull_crowded = [&](int k) __attribute__((always_inline)) {
         const int64_t lo = events_at(k - 1);
         const unsigned n_ev = (unsigned)(events_at(k) - lo);  // (a step's events are below 2^31)
         const int32_t *const events = s.in_events + lo;
-        const bool beside = !alone && n_ev <= (unsigned)kResBlock && n_ev <= 2u * row_cap;  // listed with the neurons
-        if (!beside) pull_events(events, (unsigned)tid, kResBlock, n_ev, (unsigned)tid < n_ev ? events[tid] : 0, 0u, 1u);
+        const unsigned n_first = alone ? 0u : min(n_ev, min((unsigned)kResBlock, 2u * row_cap));
         if (!alone)
             crowded_rows<kResBlock / kWave>(
-                lists_of(k - 1), list_tag(k - 1), span, hist + (int64_t)row_before() * (words + 1), words, beside ? n_ev : 0u,
+                lists_of(k - 1), list_tag(k - 1), span, hist + (int64_t)row_before() * (words + 1), words, n_first,
                 [&](unsigned i) { return input_row(events[i]); }, rows, 2u * row_cap, crowd_l, abort_word, spin_limit,
                 [&](unsigned total) __attribute__((always_inline)) {
                     for (unsigned a = (unsigned)tid; a < total; a += kResBlock) {
@@ -906,7 +900,9 @@ __global__ __launch_bounds__(kResBlock) void sim_resident_lists_kernel(bmtk_glif
                         add_bounds(row_bounds(row), (row & kInputTag) != 0u, 0u, 1u);
                     }
                 });
-        __syncthreads();
+        n_more = wave < kWriter ? n_ev - n_first : 0u;
+        more_events = events + n_first;
+        if (at_row < n_more) next_source = more_events[at_row];  // (n_rows is 0, and a team one lane)
     };
     // The writer's part of a step: the list (the others wait for it), ballots, record.
     const unsigned rec_ways = s.spike_ways > 1 ? (unsigned)s.spike_ways : 1u;
@@ -976,10 +972,8 @@ __global__ __launch_bounds__(kResBlock) void sim_resident_lists_kernel(bmtk_glif
             }
             if (k > 0) {
                 if (!asked) ask(k);
-                if (listed == kCrowded)
-                    pull_crowded(k);
-                else
-                    pull(k);
+                if (listed == kCrowded) pull_crowded(k);
+                pull(k);
             }
             if (k < n_steps) {
                 slot_prev = next(slot_prev, L);

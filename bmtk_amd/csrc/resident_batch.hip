@@ -266,15 +266,6 @@ __global__ __launch_bounds__(kRbBlock) void sim_resident_batch_kernel(bmtk_glif3
     // (a call's first step: the spikes of the step before were added by the call before it, and so were its events unless
     //  they are to be taken from this call's lists)
     auto with_events = [&](int k) { return in_ptr && (k > 0 || s.rb_late_events); };
-    // Input events events[a], events[a + step], .. of n, without a stay in LDS; the first of them is at hand already
-    auto pull_events = [&](const int32_t *events, unsigned a, unsigned step, unsigned n_ev, int32_t next_source) __attribute__((always_inline)) {
-        while (a < n_ev) {
-            const int32_t source = next_source;
-            a += step;
-            if (a < n_ev) next_source = events[a];
-            add_segment(row_bounds((unsigned)n + (unsigned)source), (unsigned)lane & ((1u << ts) - 1u), 1u << ts);
-        }
-    };
     // The rows of round k: what fired in step k-1, and the input events handed over with it.  Where they are listed before the
     // update of step k (`ask` ahead of it), the bounds of a thread's first row are on their way meanwhile.
     // Events that the reader has no lanes for follow the listed rows (see resident.hip).
@@ -308,28 +299,32 @@ __global__ __launch_bounds__(kRbBlock) void sim_resident_batch_kernel(bmtk_glif3
             add_segment(b, part, 1u << ts);
         }
         if (n_more != 0u) {
-            const unsigned a = at_row - n_rows;
+            unsigned a = at_row - n_rows;
             if (!at_hand && a < n_more) next_source = more_events[a];
-            pull_events(more_events, a, step, n_more, next_source);
+            while (a < n_more) {
+                const int32_t source = next_source;
+                a += step;
+                if (a < n_more) next_source = more_events[a];
+                add_segment(row_bounds((unsigned)n + (unsigned)source), part, 1u << ts);
+            }
         }
     };
     auto pull_crowded = [&](int k) __attribute__((always_inline)) {
         const unsigned lo = with_events(k) ? (unsigned)in_ptr[k] : 0u, n_ev = with_events(k) ? (unsigned)in_ptr[k + 1] - lo : 0u;
         const int32_t *const events = s.rb_in_events + lo;
-        const bool beside = k > 0 && n_ev <= (unsigned)kRbBlock && n_ev <= (unsigned)s.rb_list;  // listed with the neurons
-        if (!beside) {
-            const unsigned a = (unsigned)tid >> ts;
-            pull_events(events, a, (unsigned)kRbBlock >> ts, n_ev, a < n_ev ? events[a] : 0);
-        }
+        const unsigned n_first = k > 0 ? min(n_ev, min((unsigned)kRbBlock, (unsigned)s.rb_list)) : 0u;
         if (k > 0)
             crowded_rows<kPer * kRbWaves>(
-                lists_of(k - 1), list_tag(k - 1), span, ballots_of(k - 1), q.words, beside ? n_ev : 0u,
+                lists_of(k - 1), list_tag(k - 1), span, ballots_of(k - 1), q.words, n_first,
                 [&](unsigned i) { return (unsigned)n + (unsigned)events[i]; }, rows, (unsigned)s.rb_list, crowd_l, abort_word, spin_limit,
                 [&](unsigned total) __attribute__((always_inline)) {
                     for (unsigned a = (unsigned)tid >> ts; a < total; a += (unsigned)kRbBlock >> ts)
                         add_segment(row_bounds(rows[a]), (unsigned)lane & ((1u << ts) - 1u), 1u << ts);
                 });
-        __syncthreads();
+        // (further events are left to pull; n_rows is 0)
+        n_more = wave < kRbWriter ? n_ev - n_first : 0u;
+        more_events = events + n_first;
+        if (at_row < n_more) next_source = more_events[at_row];
     };
     // the pulls of round k are complete
     auto pulled = [&](int k) __attribute__((always_inline)) {
@@ -364,10 +359,8 @@ __global__ __launch_bounds__(kRbBlock) void sim_resident_batch_kernel(bmtk_glif3
             }
             if (k < n_steps) volley(k);
             if (!asked) ask(k);
-            if (listed == kCrowded)
-                pull_crowded(k);
-            else
-                pull(k);
+            if (listed == kCrowded) pull_crowded(k);
+            pull(k);
             slot = slot + 1 == S ? 0 : slot + 1;
             if (wave != kRbWriter) count_lds(&done_l);
             pulled(k);
