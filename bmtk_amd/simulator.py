@@ -47,6 +47,7 @@ FUSE_BATCHES = range(8, 65)         # lane = trial, at most eight neurons to a w
 FUSE_PAD = 64                       # records behind its table (BMTK_FUSE_PAD)
 RES_LDS_BYTES = 160 * 1024      # LDS of one gfx950 compute unit
 RES_ACT_ENTRIES = 8192          # active-row list of the resident kernel (kActCap of csrc/resident.hip), 4 B each
+LIST_MAX = 39                   # neurons of a workgroup's list (kListMax of csrc/fired_lists.hpp)
 RES_LDS_EXTRA = RES_ACT_ENTRIES * 4 + 256   # the list plus the kernel's static LDS (rounded up)
 # the single-workgroup form: per element the spike offsets and probed potentials of two steps (SOLO_LDS_PER_ELEMENT);
 # the items (rows to walk) of two steps and its static LDS (SOLO_LDS_EXTRA)
@@ -80,6 +81,17 @@ def resident_span(ne, batch, ring_slots, n_cu, single=True):
     if span > 1024 or ring_slots * NREC * span * 4 + RES_LDS_EXTRA > RES_LDS_BYTES:
         return 0
     return span
+
+
+def lists_pay(span, groups, rate_hz, h_ms=1.0):
+    """Whether ``groups`` workgroups of ``span`` neurons that fire at ``rate_hz`` are expected to fit what they fire in a step into lists
+    (of up to LIST_MAX neurons), which they then exchange in less time than ballots behind a grid barrier.  Measured on one MI355X,
+    us per step lists / ballots, and the busiest workgroup of a step: 230,924 neurons at 21, 24, 28, 35, 46, 60 Hz 17.0 / 18.0 (34),
+    18.4 / 17.2 (37), 26.3 / 22.4 (43), 29.0 / 23.1 (50), 36.5 / 38.4 (63), 45.4 / 47.0 (79); 120,000 at 45, 57, 71 Hz 15.2 / 15.7 (37),
+    22.9 / 18.8 (44), 28.7 / 28.5 (53); 60,000 at 71, 92 Hz 13.0 / 14.2 (30), 17.5 / 17.4 (38); 3,000 at 91 Hz 4.0 / 5.2 (12)."""
+    fired = span * float(rate_hz) * 1e-3 * h_ms
+    # (the largest of so many Poisson numbers, a little above it)
+    return fired + math.sqrt(2.0 * fired * math.log(max(2, groups))) <= LIST_MAX
 
 
 def resident_trials_plan(n_neurons, batch, ring_slots, n_cu):
@@ -203,8 +215,9 @@ class Glif3Simulator:
                 on the many-workgroup form
     fired_lists  resident mode with several workgroups: every workgroup publishes the neurons that fired in a step
                 as a short list whose words carry the step, and nobody waits at a grid barrier (neurons that a list does
-                not hold are read from the ballots); False: ballots behind a grid barrier.  Same results either way.
-    expected_rate_hz  what "auto" decides ``pull`` / ``fused`` by.  Pushing spikes into the ring costs an atomic per
+                not hold are read from the ballots), unless at ``expected_rate_hz`` lists would seldom do (``lists_pay``);
+                False: ballots behind a grid barrier.  Same results either way.
+    expected_rate_hz  what ``fired_lists`` goes by, and "auto" decides ``pull`` / ``fused`` by.  Pushing spikes into the ring costs an atomic per
                 synaptic event, pulling a pass over the whole table per step whatever the activity; a synapse
                 carries batch * rate * h events per step, and on one MI355X the pass is the cheaper of the two from
                 about 0.06 events per synapse and step (measured: 51,978 neurons x 32 trials at 3.2 Hz pull 168 us
@@ -363,6 +376,7 @@ class Glif3Simulator:
         self.spin_limit = 0  # resident mode: polls of the grid barrier before giving up (0 = built-in limit)
         self.single_workgroup = bool(single_workgroup)
         self.fired_lists = bool(fired_lists)
+        self.expected_rate_hz = float(expected_rate_hz)
         if resident:
             self._setup_resident(required=(resident is True))
         self.pull_table = self.pull_syn = self.pull_work = None
@@ -427,7 +441,6 @@ class Glif3Simulator:
                 self.pull_inp_work = torch.zeros(need // 4 + 1, dtype=torch.int32, device=self.dev)
                 self.in_hist_stride = n_words(self.n_inputs * self.batch) + 1
                 self.in_hist = torch.zeros(self.L * self.in_hist_stride, dtype=torch.int64, device=self.dev)
-        self.expected_rate_hz = float(expected_rate_hz)
         self._trials_left, self._pend_from, self._pend_until, self._left_ring, self._kept = False, 0, 0, None, []
         if resident_trials == "auto":
             # (resident=False asks for the launch-per-step drivers, of a batch too)
@@ -692,8 +705,8 @@ class Glif3Simulator:
             self.res_unified = (packed, seg)
         self.res_span, self.res_groups = span, groups
         # asks for the exchange by lists of fired neurons (bmtk_glif3_sim.res_fired)
-        self.res_fired = (torch.zeros(self.hist_slots * groups * _lib.RES_FIRED_SLOTS, dtype=torch.int32, device=self.dev)
-                          if groups > 1 and self.fired_lists else None)
+        lists = groups > 1 and self.fired_lists and lists_pay(span, groups, self.expected_rate_hz, self.h)
+        self.res_fired = torch.zeros(self.hist_slots * groups * _lib.RES_FIRED_SLOTS, dtype=torch.int32, device=self.dev) if lists else None
 
     def check(self):
         """Raise if a resident run since the last check gave up on its grid barrier (synchronises).  The abort

@@ -247,3 +247,19 @@ def test_steps_of_many_input_events(batch, places, form, monkeypatch):
     assert int(got[0]["bits"].ne(0).sum()) > 50
     for key in got[0]:
         assert torch.equal(got[0][key], got[1][key]), key
+
+
+@pytest.mark.parametrize("rate,lists,ask", [(3.0, True, True), (100.0, True, True), (600.0, False, True), (3.0, False, False)])
+def test_the_expected_rate_picks_the_exchange(rate, lists, ask, monkeypatch):
+    """Lists unless more neurons of a workgroup are expected to fire in a step than they hold; the same results either way."""
+    par, rec, inp, ptr, events = _network(4)
+    monkeypatch.setattr(simulator, "resident_span", lambda *a, **k: 64)
+    got = []
+    for resident in (False, True):
+        sim = simulator.Glif3Simulator(N, par, 1.0, rec=rec, inp=inp, u_init=_start(par, 64, 8), resident=resident, expected_rate_hz=rate,
+                                       fired_lists=ask, **({} if resident else dict(pull=False)))
+        assert not resident or (sim.res_fired is not None) == lists
+        sim.set_input_events(ptr, events)
+        got.append(sim.run(STEPS)["bits"])
+        sim.check()
+    assert torch.equal(got[0], got[1])

@@ -2,7 +2,7 @@
 import pytest
 
 from bmtk_amd.layout import NREC
-from bmtk_amd.simulator import RB_LDS_STATIC, RES_LDS_BYTES, resident_trials_plan, trials_bytes, trials_fit, trials_pay
+from bmtk_amd.simulator import RB_LDS_STATIC, RES_LDS_BYTES, lists_pay, resident_trials_plan, trials_bytes, trials_fit, trials_pay
 
 
 @pytest.mark.parametrize("n,batch,slots", [(1, 2, 2), (64, 64, 6), (65, 3, 6), (5000, 16, 6), (20011, 20, 6), (51978, 32, 6), (230924, 8, 6),
@@ -46,3 +46,13 @@ def test_plan_of_one_trial_with_two_neurons_to_a_thread():
         assert (slots - 1) * NREC * 4 * span + 4 * p["list"] + RB_LDS_STATIC <= RES_LDS_BYTES and p["list"] >= 2000
     for args in ((262144, 1, 6, 256), (491521, 1, 6, 256), (491520, 1, 7, 256)):
         assert resident_trials_plan(*args) is None
+
+
+def test_lists_are_exchanged_where_they_were_measured_to_pay():
+    """(span, workgroups, Hz): lists against ballots behind a grid barrier, as measured; never ballots at the default rate."""
+    for span, groups, rate, lists in ((960, 241, 20.8, True), (960, 241, 24.2, False), (960, 241, 27.8, False), (960, 241, 34.6, False),
+                                      (512, 235, 45.1, True), (512, 235, 56.6, False), (256, 235, 70.9, True), (64, 157, 91.0, True),
+                                      (64, 47, 91.0, True)):
+        assert lists_pay(span, groups, rate) == lists, (span, groups, rate)
+    assert all(lists_pay(span, groups, 3.0, h) for span in (64, 512, 1024) for groups in (2, 256) for h in (0.1, 1.0))
+    assert lists_pay(64, 5, 0.0)
