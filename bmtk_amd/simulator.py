@@ -704,9 +704,9 @@ class Glif3Simulator:
             self.rec_seg, self.inp_seg = seg[:self.n], seg[self.n:]
             self.res_unified = (packed, seg)
         self.res_span, self.res_groups = span, groups
-        # asks for the exchange by lists of fired neurons (bmtk_glif3_sim.res_fired)
+        # asks for the exchange by lists of fired neurons (bmtk_glif3_sim.res_fired: that it is there is all that is looked at)
         lists = groups > 1 and self.fired_lists and lists_pay(span, groups, self.expected_rate_hz, self.h)
-        self.res_fired = torch.zeros(self.hist_slots * groups * _lib.RES_FIRED_SLOTS, dtype=torch.int32, device=self.dev) if lists else None
+        self.res_fired = torch.zeros(1, dtype=torch.int32, device=self.dev) if lists else None
 
     def check(self):
         """Raise if a resident run since the last check gave up on its grid barrier (synchronises).  The abort

@@ -235,7 +235,8 @@ int bmtk_csr_segment_offsets(int64_t n_rows, const int32_t *indptr, const int32_
 
 #define BMTK_RES_SYNC_STRIDE 1088                          /* words: 4 KiB + 256 B */
 #define BMTK_RES_SYNC_WAYS 8                               /* counters a step's arrivals are spread over */
-#define BMTK_RES_FIRED_SLOTS 16       /* words per workgroup and row of bmtk_glif3_sim.res_fired */
+#define BMTK_RES_FIRED_SLOTS 16       /* 32-bit words of a workgroup's list of fired neurons */
+#define BMTK_RES_FIRED_MANY 0xFFFFFFFFu /* no longer used: for programs that name it */
 #define BMTK_RES_SYNC_WORDS ((1 + 64 * BMTK_RES_SYNC_WAYS) * BMTK_RES_SYNC_STRIDE) /* size of bmtk_glif3_sim.res_sync */
 
 /* Everything nest.Simulate needs for a forward run (bmtk/simulator/pointnet/pointsimulator.py:159-166). */
@@ -304,19 +305,18 @@ typedef struct bmtk_glif3_sim {
     int32_t res_groups;
     const uint32_t *rec_seg;     /* [neurons][res_groups+1] */
     const uint32_t *inp_seg;     /* [inputs][res_groups+1] */
-    uint32_t *res_sync;          /* BMTK_RES_SYNC_WORDS words of scratch, zeroed by the caller once: word 1 =
-                                  * abort flag, from word BMTK_RES_SYNC_STRIDE on 64 x BMTK_RES_SYNC_WAYS arrival
-                                  * counters that many words apart (or lists, see res_fired, from the next whole 64-bit word on), which every call
-                                  * clears for itself.  Word 1 != 0
+    uint32_t *res_sync;          /* BMTK_RES_SYNC_WORDS words of scratch, zeroed by the caller once: word 1 = abort flag, from word
+                                  * BMTK_RES_SYNC_STRIDE on 64 x BMTK_RES_SYNC_WAYS arrival counters that many words apart, or (see
+                                  * res_fired) lists, from the next whole 64-bit word on; every call clears them for itself.  Word 1 != 0
                                   * after a run means a grid barrier timed out and the results are invalid.  The
                                   * flag is sticky: no call clears it, and a call that finds it set does nothing,
                                   * so a failure cannot be overwritten before the host has seen it; the host
                                   * clears it after reading. */
-    uint32_t *res_fired;         /* optional, several workgroups only: [hist_slots][res_groups][BMTK_RES_FIRED_SLOTS]
-                                  * words.  Given, runs without slack (delay offset 0, hist_slots of at least 4) exchange lists
-                                  * of the neurons that fired, whose words say themselves which step they belong to, instead of
-                                  * ballots behind a grid barrier.  The lists themselves are kept in res_sync.  NULL: always
-                                  * ballots and the barrier. */
+    uint32_t *res_fired;         /* optional, several workgroups only: not NULL asks for the exchange by lists (the memory is neither read
+                                  * nor written).  Runs without slack (delay offset 0, hist_slots of at least 4) then exchange lists of
+                                  * the neurons that fired, kept in res_sync, whose words say themselves which step they belong to,
+                                  * instead of ballots behind a grid barrier.  The faster exchange unless more than 39 neurons of a
+                                  * workgroup fire in most steps.  NULL: always ballots and the barrier. */
     /* Pull form of the recurrent delivery for batched runs (optional; launch-per-step mode with delay_offset 0
      * and hist_slots == ring_slots): a TARGET-major packed copy of the recurrent table.  The recurrent arrivals
      * of step t-1 are then summed in one pass over that table from the spike-bit history
