@@ -427,11 +427,10 @@ __global__ __launch_bounds__(kResBlock) void sim_resident_kernel(bmtk_glif3_sim 
     const unsigned long long rec_way = blockIdx.x & (rec_ways - 1u), rec_cap = (unsigned long long)s.spike_cap / rec_ways;
     // With as many lists as workgroups this one appends to its list alone: its count lives in a register of every
     // thread (first loaded, written back at the end), a spike's place is that count plus the spike's rank among the
-    // workgroup's spikes of the step (the LDS atomic that also builds the list of fired neurons), and no wavefront
+    // workgroup's spikes of the step (an LDS atomic), and no wavefront
     // waits for an atomic on device memory, which the arrivals of a step would queue up behind.
     const bool own_record = !kLate && s.spike_count != nullptr && rec_ways >= gridDim.x;
     unsigned long long rec_count = own_record ? s.spike_count[rec_way * BMTK_RECORD_COUNT_STRIDE] : 0ull;
-    const bool count_fired = own_record;
     // the input events of the step pulled in step t, u = t-1-B, are in_events[ka, kb); the bound for the
     // next step is fetched a step ahead.  Steps before 0 have no events (in_ptr[0] = 0).
     const int B = r.offset;
@@ -541,9 +540,9 @@ __global__ __launch_bounds__(kResBlock) void sim_resident_kernel(bmtk_glif3_sim 
         // memory round trip away.  It is only asked for here and looked at after the pull, so that no wavefront
         // stops for it in the update (which every other wavefront of the workgroup would wait out at the next
         // barrier).
-        if (count_fired && m != 0ull && spike) {
+        if (own_record && m != 0ull && spike) {
             const unsigned at = atomicAdd(&fired_n[k & 1], 1u);
-            if (own_record && rec_count + at < rec_cap) {
+            if (rec_count + at < rec_cap) {
                 const unsigned long long idx = rec_way * rec_cap + rec_count + at;
                 s.spike_step[idx] = (int32_t)t;
                 s.spike_elem[idx] = (int32_t)e;
@@ -574,11 +573,10 @@ __global__ __launch_bounds__(kResBlock) void sim_resident_kernel(bmtk_glif3_sim 
                 aborted = true;
                 break;
             }
-            // the list of this step, complete since the workgroup met: out with it, like the ballots (the arrival
-            // waits for the store), and the count back to zero (it is added to again after the barriers of the pull)
+            // the number of this step, complete since the workgroup met; the other one, last read a barrier ago and next added
+            // to a barrier on, back to zero
             if (own_record) rec_count += fired_n[k & 1];
-            // the other count, last read a barrier ago and next added to a barrier on, back to zero
-            if (count_fired && tid == 0) fired_n[(k + 1) & 1] = 0u;
+            if (own_record && tid == 0) fired_n[(k + 1) & 1] = 0u;
         }
         PROF_T(c2);
 #ifdef BMTK_RES_PROFILE

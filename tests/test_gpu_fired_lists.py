@@ -216,13 +216,10 @@ def test_volleys_of_any_number_of_workgroups(n, form, monkeypatch):
         assert torch.equal(got[0][key], got[1][key]), key
 
 
-@pytest.mark.parametrize("form", ["bits", "record", "probes"])
-@pytest.mark.parametrize("batch,places", [(1, 0), (5, 700), (5, 8192)])
+@pytest.mark.parametrize("batch,places,form", [(1, 0, "bits"), (1, 0, "record"), (1, 0, "probes"), (5, 700, "bits"), (5, 8192, "bits")])
 def test_steps_of_many_input_events(batch, places, form, monkeypatch):
     """Around the numbers of events that the reader lists (512), that one turn of the pulling threads takes beside them, that trials'
     rows have room for (half of `places` less 64), and far more of them, on any side of a step with few."""
-    if form != "bits" and batch > 1:
-        pytest.skip("trials keep no record and no probes")
     par, rec, inp, _, _ = _network(6)
     rec, inp = [t[:3] + (np.minimum(t[3], 4),) + t[4:] for t in (rec, inp)]
     inp = inp[:2] + (inp[2] / 32,) + inp[3:]

@@ -271,13 +271,13 @@ def test_v1_scale_forward_run_against_both_oracles():
     assert agree[np.float64] >= 0.999, agree
 
 
-@pytest.mark.parametrize("fused", [True, False])
-def test_training_size_forward_run_is_bit_identical_to_the_oracle(fused):
+@pytest.mark.parametrize("fused,trials", [(True, False), (False, False), (True, True)], ids=["True", "False", "trials"])
+def test_training_size_forward_run_is_bit_identical_to_the_oracle(fused, trials):
     """The forward pass of the training configuration at its own size -- 51,978 neurons x batch 32, 52 M recurrent
     and 8 M input synapses, 17,400 Poisson inputs at 5 Hz, per-step record on -- through the batched driver: pull
-    and update fused in one launch per step over the joint table (what a simulator picks at this batch), and as
-    separate launches (pull form for recurrent and input synapses); repeat lists for ids that occur twice in a step
-    either way.  Quarter-pA weights: raster, state and the recorded potentials must equal the fp32 oracle's bit for
+    and update fused in one launch per two steps over the joint table (what resident=False takes at this batch), as
+    separate launches (pull form for recurrent and input synapses), and its trials resident, four at a time; ids that
+    occur twice in a step in all of them.  Quarter-pA weights: raster, state and the recorded potentials must equal the fp32 oracle's bit for
     bit."""
     n, n_in, batch, steps = N52K, 17400, 32, 120
     rng = np.random.default_rng(4)
@@ -287,7 +287,8 @@ def test_training_size_forward_run_is_bit_identical_to_the_oracle(fused):
     inp = synthetic.device_input_table(n_in, n, 8_000_000, seed=4, w_scale=2.0)
     inp = (inp[0], inp[1], _quarter(inp[2]), inp[3], inp[4])
     in_ptr, in_ev = ops.poisson_events(n_in, 5.0, 1.0, steps, batch=batch, seed=5)
-    sim = Glif3Simulator(n, par, 1.0, batch=batch, rec=by_src, inp=inp, resident=False, fused="auto" if fused else False)
+    sim = Glif3Simulator(n, par, 1.0, batch=batch, rec=by_src, inp=inp, resident=False, fused="auto" if fused else False,
+                         resident_trials=trials)
     if fused:
         assert sim.fuse_table is not None and sim.pull_table is None and sim.fuse_shift == 0
     else:
@@ -296,6 +297,7 @@ def test_training_size_forward_run_is_bit_identical_to_the_oracle(fused):
     assert sim.in_duplicates and sim.in_repeat_events.numel() > 0   # a few ids occur twice within a step
     a = sim.run(50, save_state=True)
     b = sim.run(steps - 50, save_state=True)
+    assert (sim._trials is not None) == trials
     ras = torch.cat([sim.raster(a["bits"]), sim.raster(b["bits"])]).cpu().numpy()
     rec_h = tuple(t.cpu().numpy() for t in by_src)
     inp_h = tuple(t.cpu().numpy() for t in inp)

@@ -216,9 +216,10 @@ def test_exact_weights_make_every_path_bit_identical():
 
 
 def test_v1_scale_resident_equals_per_step_launches():
-    """230,924 neurons, ~70 M synapses, exact weights: the resident kernel (242
-    workgroups, one grid barrier per step) and the per-step launches must emit
-    identical spikes for 2000 steps, the resident run split into two calls."""
+    """230,924 neurons, ~70 M synapses, exact weights: the resident kernels (241
+    workgroups that exchange lists, or ballots behind a grid barrier per step) and
+    the per-step launches must emit identical spikes for 2000 steps, the resident
+    runs split into two calls."""
     import torch
     rng = np.random.default_rng(3)
     n, n_in, steps = 230924, 17400, 2000
@@ -231,9 +232,9 @@ def test_v1_scale_resident_equals_per_step_launches():
     inp = (inp[0], inp[1], torch.round(inp[2] * 4) / 4 + 0.25, inp[3], inp[4])
     in_ptr, in_ev = synthetic.device_poisson_events(n_in, 5.0, 1.0, steps, seed=5)
     bits = []
-    for resident in (False, True):
-        sim = Glif3Simulator(n, par, 1.0, class_id=cid, rec=by_src, inp=inp, resident=resident)
-        assert bool(sim.res_span) == resident
+    for resident, lists in ((False, True), (True, True), (True, False)):
+        sim = Glif3Simulator(n, par, 1.0, class_id=cid, rec=by_src, inp=inp, resident=resident, fired_lists=lists)
+        assert bool(sim.res_span) == resident and (sim.res_fired is not None) == (resident and lists)
         sim.set_input_events(in_ptr, in_ev)
         if resident:
             out = {"bits": torch.cat([sim.run(777)["bits"], sim.run(steps - 777)["bits"]])}
@@ -248,7 +249,7 @@ def test_v1_scale_resident_equals_per_step_launches():
         first_state = state
         del sim
     assert int(ops_popcount(bits[0])) > 1000000
-    assert torch.equal(bits[0], bits[1])
+    assert torch.equal(bits[0], bits[1]) and torch.equal(bits[0], bits[2])
 
 
 def test_resident_with_every_thread_owning_an_element():
