@@ -19,8 +19,9 @@
 //
 // What bounds it: a step is a chain of dependent loads (lists, segment bounds, synapses), 2.5 us at the smallest sizes,
 // whatever the number of trials side by side; then the table's segments, which every trial reads for itself.  Per step and
-// launch, ballots and a grid barrier per trial -> lists: 230,924 neurons x 8 6.9 -> 6.1 us, 20,011 x 20 5.0 -> 4.7,
-// 400,123 x 1 9.3 -> 6.6; 51,978 x 32, which reads 18 synapses a segment for 243 rows of each of four trials, 5.2 as before.
+// launch, ballots and a grid barrier per trial -> lists, in turn in one process: 230,924 neurons x 4 6.0 -> 5.6 us, 20,011 x 20 4.5 ->
+// 4.3, 3,001 x 12 3.0 -> 2.8, 400,123 x 1 with 1,024 spikes a step 10.5 -> 7.6; 51,978 x 32, which reads 18 synapses a segment for 243
+// rows of each of four trials, as before.
 // At tens of Hz, where steps are crowded (see resident.hip), the ballots were the faster exchange still: 60,000 x 4 at 24 / 45 Hz 12.3 /
 // 20.3 us a step against 14.9 / 24.8 (15.1 / 35.7 with every list of more than 19 neurons crowded), 230,924 x 2 at 28 Hz 56 against 62;
 // at 19 Hz 60,000 x 4 take 5.4 against 10.0.

@@ -32,11 +32,15 @@ FUSE_PS_PER_EVENT = 6.0
 PUSH_PS_PER_ELEMENT = 55.0
 PUSH_PS_PER_ELEMENT_CLASS_TABLE = 27.0
 PUSH_PS_PER_EVENT = 48.0
-# The form with resident trials pays a chain of dependent loads and a barrier per launch and step, a visit per row that fired,
-# little per event.  Measured, us per step trials / fused / pushed (neurons x trials, in-degree): 51,978 x 32, 1154: 38 / 95 / - ;
-# 20,011 x 20, 820: 8.3 / 31 / - ; 230,924 x 8, 335: 59 / 134 / 164; 5,000 x 16, 400: 2.8 / 9.8 / - ; 31,000 x 64, 160: 36 / 38 / 87;
-# 120,000 x 16, 150: 41 / 52 / 82; 100,000 x 4, 260: 10 / - / 28; 2,000 x 40, 200: 3.3 / 6.3 / 11.5; 3,000 x 4, 200: 2.7 / - / 11.5;
-# 400,123 x 1, 180: 9.8 / - / 25.4.  (Fitted with a grid barrier per trial; with lists the first figures are up to a third lower.)
+# The form with resident trials pays a chain of dependent loads per launch and step, a visit per row that fired, little per event.
+# Measured at 2 to 3 Hz in calls of 100 to 300 steps, us per step trials / fused / pushed (neurons x trials, in-degree): 51,978 x 32, 1154:
+# 40 / 92 / 255; 20,011 x 20, 820: 8.3 / 31 / 55; 230,924 x 8, 335: 48 / 134 / 140; 5,000 x 16, 400: 2.8 / 10.0 / 21; 31,000 x 64, 160:
+# 35 / 37 / 83; 60,000 x 64, 130: 70 / 65 / 145; 120,000 x 16, 150: 35 / 51 / 81; 115,000 x 20, 130: 46 / 57 / 91; 12,000 x 64, 130:
+# 12.1 / 16.1 / 28; 100,000 x 4, 260: 7.3 / - / 28; 2,000 x 40, 200: 2.7 / 6.7 / 8.7; 3,000 x 4, 200: 2.5 / - / 7.0; 600 x 16, 100:
+# 2.2 / - / 4.8; 400,123 x 1, 180: 6.6 / - / 22.  The constants were fitted with a grid barrier per trial and ask for up to a half
+# more than lists take; at all of these sizes they pick the faster form still.  What they leave out: a call's own cost (state and
+# ring in and out, its events put apart by trial: 31,000 x 64 in calls of 40 steps 59 us a step against 39 fused) and the detour of
+# the per-step record (51,978 x 32 6 us a step, 31,000 x 64 7, against 2 and 4 in the fused form).
 TRIALS_PS_PER_PASS = 3.0e6
 TRIALS_PS_PER_ROW = 6.5e3       # per neuron of ONE trial that fires in a step (and the input events that come with it)
 TRIALS_PS_PER_EVENT = 0.8
