@@ -39,7 +39,8 @@ class Glif3Sim(C.Structure):
         ("rb_list", c_int32), ("rb_late_events", c_int32),
         ("rb_seg", c_void_p), ("rb_packed", c_void_p), ("rb_ring", c_void_p), ("rb_hist", c_void_p),
         ("rb_in_ptr", c_void_p), ("rb_in_events", c_void_p), ("rb_pend_until", c_int64),
-        ("rb_save_v", c_void_p), ("rb_save_flags", c_void_p), ("sum_shift", c_int32), ("_pad3", c_int32),
+        ("rb_save_v", c_void_p), ("rb_save_flags", c_void_p),
+        ("rb_cells", c_void_p), ("rb_extra", c_int32), ("_pad4", c_int32), ("sum_shift", c_int32), ("_pad3", c_int32),
         ("spike_bits", c_void_p), ("spike_bits_stride", c_int64),
         ("save_v", c_void_p), ("save_flags", c_void_p),
         ("probe_col", c_void_p), ("probe_v", c_void_p), ("probe_stride", c_int64), ("probe_every", c_int32),
@@ -66,7 +67,7 @@ class Glif3Bwd(C.Structure):
     ]
 
 
-ABI_VERSION = 29  # BMTK_AMD_ABI_VERSION of include/bmtk_amd.h that the mirrors above were written for
+ABI_VERSION = 30  # BMTK_AMD_ABI_VERSION of include/bmtk_amd.h that the mirrors above were written for
 
 # name -> (restype, argtypes); every symbol include/bmtk_amd.h declares
 SIGNATURES = {
@@ -106,6 +107,8 @@ SIGNATURES = {
     "bmtk_poisson_fill": (c_int32, [c_int64, c_int32, c_void_p, c_double, c_double, c_double, c_int64, C.c_uint64,
                                     c_void_p, c_void_p, c_void_p, c_void_p]),
     "bmtk_glif3_simulate_fwd": (c_int32, [C.POINTER(Glif3Sim), c_int64, c_int64, c_void_p]),
+    "bmtk_csr_receptors_used": (c_int32, [c_int64] + [c_void_p] * 4),
+    "bmtk_csr_pack_cells": (c_int32, [c_int64, c_int32] + [c_void_p] * 3),
     "bmtk_events_by_trial": (c_int32, [c_int32, c_int64, c_int64, c_int32] + [c_void_p] * 6),
     "bmtk_glif3_simulate_bwd": (c_int32, [C.POINTER(Glif3Bwd), c_int64, c_int64, c_void_p]),
     "bmtk_glif3_step_bwd": (c_int32, [C.POINTER(Glif3Bwd), c_int64, c_int64, c_int32, c_void_p]),

@@ -15,7 +15,15 @@
 // Sums are 64-bit fixed point, exact and independent of the order, as in the fused batched driver (and an integer
 // addition in LDS costs 28 clocks per wavefront where a float's costs 194).  Slot t-1 is folded and cleared before the
 // spikes of step t-1 are added, so that ring_slots - 1 slots suffice: 160 bytes of LDS per neuron and trial at delays of
-// up to five steps.  Behind a call the arrivals still ahead wait in rb_ring, trial by trial.
+// up to five steps with sums for all four receptors.  Behind a call the arrivals still ahead wait in rb_ring, trial by trial.
+//
+// Where that saves launches a neuron has sums only for the receptors that some synapse of it ends on (rb_cells): of four ports the cells
+// of a population mostly use two, which is 80 bytes, and with two neurons to a thread (1088 to 1920 a workgroup) twice the
+// trials run side by side.  The first two sums of every neuron are planes over the span (the fold reads them without bank
+// conflicts), the rarer third and fourth stand behind; a record names its cell, so that the pull asks nothing.  A step then takes 1.2 to 1.4
+// times as long: update 0.7 -> 1.4 us (the issue of two neurons' instructions), the pull's chain as before with twice the
+// synapses in a segment.  At 2.2 sums a neuron, 200 steps: 51,978 x 32 in 4 launches of 32 workgroups a trial 5.85 ms, in 8 of 63 8.03;
+// 20,011 x 20 in one launch 1.47, in two 1.74.  230,924 x 8 have no room for two trials either way.
 //
 // What bounds it: a step is a chain of dependent loads (lists, segment bounds, synapses), 2.5 us at the smallest sizes,
 // whatever the number of trials side by side; then the table's segments, which every trial reads for itself.  Per step and
@@ -46,6 +54,7 @@ constexpr int kRbWaves = kRbBlock / kWave;
 constexpr int kRbReader = kRbWaves - 1, kRbWriter = kRbReader - 1;  // wavefronts with a part of their own, see resident.hip
 constexpr int kRbPullThreads = kRbWriter * kWave;
 constexpr unsigned kRbMaxSpin = 4000000u; // looks in vain before giving up (seconds)
+// (two neurons to a thread and their sums leave registers for four: with six the compiler spills)
 constexpr int kRbTogether = 6;            // synapses a lane has in flight (20,011 x 20, 8 lanes to 33: 4 of them 9.6 us per step, 6 9.3)
 constexpr int kRbEvents = 8;              // input events a lane of the reader asks for ahead
 
@@ -64,20 +73,31 @@ __device__ __forceinline__ unsigned rb_load(const unsigned *p)
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// Where the sums of a neuron's receptor r stand within a slot of its workgroup's slice.  `word` is rb_cells': bits 0..3 the
+// receptors that some synapse of the neuron ends on, above them where its third sum stands among the workgroup's.
+__host__ __device__ inline int rb_cell(unsigned word, int r, int place, int span)
+{
+    const unsigned below = word & ((1u << r) - 1u);
+    const int j = (int)((below & 1u) + (below >> 1 & 1u) + (below >> 2 & 1u));
+    return j < 2 ? j * span + place : 2 * span + (int)(word >> GLIF3_NREC) + j - 2;
+}
+
 struct __attribute__((packed, aligned(4))) RbBounds {
     uint32_t lo, hi;
 };
 
 // kPer: neurons per thread; with two, the threads of the reader own none.  Sum: what the ring holds, 64-bit fixed point
 // (from_fixed), or floats where a workgroup's neurons are too many for that (batch 1): fp32 atomics into device memory are what
-// it then takes the place of.  kSave: potentials and step flags of every step go to rb_save_*, trial by trial; by_step_kernel
+// it then takes the place of.  kAllSums: every neuron has all four sums, in planes (no rb_cells); at 1,000 neurons and less to a
+// workgroup the fold's selections cost 0.1 us a step, so that few sums are for where they save launches.  kSave: potentials and step flags of every step go to rb_save_*, trial by trial; by_step_kernel
 // puts them in their order.  kReaderOwns: spans above 960 with a neuron to a thread.
-template <int kPer, typename Sum, bool kSave, bool kReaderOwns>
+template <int kPer, typename Sum, bool kAllSums, bool kSave, bool kReaderOwns>
 __global__ __launch_bounds__(kRbBlock) void sim_resident_batch_kernel(bmtk_glif3_sim s, RbLaunch q)
 {
     constexpr bool kFixed = sizeof(Sum) == 8;
+    constexpr int kTogether = kPer > 1 && kFixed ? 4 : kRbTogether;
     constexpr int kOwners = kRbReader * kWave;  // with two neurons to a thread: threads that own tid, tid + kOwners
-    extern __shared__ unsigned long long rb_lds[];  // ring slice [slots * 4][span], then rb_list words for rows
+    extern __shared__ unsigned long long rb_lds[];  // ring slice [slots][cells], then rb_list words for rows
     __shared__ int go_on[2];  // by the round, as rows_l is: a slot is written again only after a meeting behind all reads of it
     __shared__ unsigned rows_l[2], crowd_l[3], done_l, updated_l, listed_l;  // rows of a round, ..
     __shared__ unsigned fired_n[2];                  // how many fired in this step and the one before
@@ -102,8 +122,10 @@ __global__ __launch_bounds__(kRbBlock) void sim_resident_batch_kernel(bmtk_glif3
     };  // in the workgroup's span
     auto owns = [&](int u) __attribute__((always_inline)) { return place(u) < mine; };
     auto element = [&](int u) { return (int64_t)(e0 + (owns(u) ? place(u) : 0)) * batch + trial; };
+    // cells of a slot: two planes of the workgroup's neurons, then the third and fourth sums of those that have any
+    const int cells = kAllSums ? GLIF3_NREC * span : 2 * span + s.rb_extra;
     Sum *ring_l = reinterpret_cast<Sum *>(rb_lds);
-    unsigned *rows = reinterpret_cast<unsigned *>(ring_l + (size_t)S * GLIF3_NREC * span);  // [2][row_cap], a place per lane behind
+    unsigned *rows = reinterpret_cast<unsigned *>(ring_l + (size_t)S * cells);  // [2][row_cap], a place per lane behind
     const unsigned row_cap = ((unsigned)s.rb_list - kWave) / 2u;
     unsigned *abort_word = s.res_sync + 1;
     const unsigned spin_limit = s.res_spin_limit ? s.res_spin_limit : kRbMaxSpin;
@@ -118,10 +140,30 @@ __global__ __launch_bounds__(kRbBlock) void sim_resident_batch_kernel(bmtk_glif3
     __syncthreads();
     if (!go_on[0]) return;
 
-    Sum *ring_g = reinterpret_cast<Sum *>(s.rb_ring) + (int64_t)trial * S * GLIF3_NREC * n + e0;
-    for (int c = tid; c < S * GLIF3_NREC * span; c += kRbBlock) {
-        const int plane = c / span, k = c - plane * span;
-        ring_l[c] = k < mine ? ring_g[(int64_t)plane * n + k] : (Sum)0;
+    // the arrivals that the call before left; some slots' are asked for together, before the state takes the registers
+    auto cell_of = [&](unsigned word, int r, int at) __attribute__((always_inline)) { return kAllSums ? r * span + at : rb_cell(word, r, at, span); };
+    Sum *const ring_g = reinterpret_cast<Sum *>(s.rb_ring) + (int64_t)trial * S * GLIF3_NREC * n + e0;  // (all receptors' planes)
+    unsigned sums[kPer]{};  // a neuron's word of rb_cells
+#pragma unroll
+    for (int u = 0; u < kPer; ++u)
+        if (owns(u)) sums[u] = kAllSums ? 15u : s.rb_cells[e0 + place(u)];
+    for (int c = tid; c < S * cells; c += kRbBlock) ring_l[c] = (Sum)0;
+    __syncthreads();
+    constexpr int kSlots = kPer > 1 ? 2 : 4;
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) {
+        if (!owns(u)) continue;
+#pragma unroll 1
+        for (int k = 0; k < S; k += kSlots) {
+            Sum v[kSlots * GLIF3_NREC];
+#pragma unroll
+            for (int j = 0; j < kSlots * GLIF3_NREC; ++j)
+                if (k + j / GLIF3_NREC < S && (sums[u] >> j % GLIF3_NREC & 1u)) v[j] = ring_g[((int64_t)k * GLIF3_NREC + j) * n + place(u)];
+#pragma unroll
+            for (int j = 0; j < kSlots * GLIF3_NREC; ++j)
+                if (k + j / GLIF3_NREC < S && (sums[u] >> j % GLIF3_NREC & 1u))
+                    ring_l[(k + j / GLIF3_NREC) * cells + cell_of(sums[u], j % GLIF3_NREC, place(u))] = v[j];
+        }
     }
     Glif3Elem st[kPer]{};
     Glif3Prop p[kPer]{};
@@ -145,16 +187,39 @@ __global__ __launch_bounds__(kRbBlock) void sim_resident_batch_kernel(bmtk_glif3
 #pragma unroll
         for (int u = 0; u < kPer; ++u) {
             if (!owns(u)) continue;
-            Sum *cell = ring_l + (size_t)at_slot * GLIF3_NREC * span + place(u);
+            Sum *const row = ring_l + (size_t)at_slot * cells;
+            auto take = [&](int cell) __attribute__((always_inline)) {
+                const Sum v = row[cell];
+                row[cell] = (Sum)0;
+                if constexpr (kFixed)
+                    return from_fixed(v, q.unit);
+                else
+                    return v;
+            };
+            if constexpr (kAllSums) {
+#pragma unroll
+                for (int r = 0; r < GLIF3_NREC; ++r) st[u].y1[r] = st[u].y1[r] + take(r * span + place(u)) * p[u].psc0[r];
+                continue;
+            }
+            unsigned word = sums[u];
+            if (kPer > 1) asm volatile("" : "+v"(word));
+            float a[GLIF3_NREC];
+            a[0] = take(place(u));
+            a[1] = take(span + place(u));
+            a[2] = a[3] = 0.0f;
+            const int third = 2 * span + (int)(word >> GLIF3_NREC);
+            if (__popc(word & 15u) > 2) a[2] = take(third);
+            if ((word & 15u) == 15u) a[3] = take(third + 1);
+            // (a sum for every receptor used, in their order: receptor r has as many before it as bits are set below bit r)
 #pragma unroll
             for (int r = 0; r < GLIF3_NREC; ++r) {
-                float a;
-                if constexpr (kFixed)
-                    a = from_fixed(cell[r * span], q.unit);
-                else
-                    a = cell[r * span];
-                cell[r * span] = (Sum)0;
-                st[u].y1[r] = st[u].y1[r] + a * p[u].psc0[r];
+                const unsigned below = word & ((1u << r) - 1u);
+                float x = a[0];
+                if (r > 0) x = below ? a[1] : x;
+                if (r > 1) x = (below & (below - 1u)) ? a[2] : x;
+                if (r > 2) x = below == 7u ? a[3] : x;
+                x = (word >> r & 1u) ? x : 0.0f;
+                st[u].y1[r] = st[u].y1[r] + x * p[u].psc0[r];
             }
         }
     };
@@ -231,12 +296,11 @@ __global__ __launch_bounds__(kRbBlock) void sim_resident_batch_kernel(bmtk_glif3
     const unsigned seg_stride = (unsigned)G + 1u;
     auto row_bounds = [&](unsigned row) __attribute__((always_inline)) { return *reinterpret_cast<const RbBounds *>(seg + (size_t)row * seg_stride); };
     auto add_segment = [&](RbBounds b, unsigned part, unsigned step) __attribute__((always_inline)) {
-        const unsigned q_lo = (unsigned)slot * 4u, q_wrap = q_lo - 4u * (unsigned)S;
-        // (slot + delay) % slots * 4 + receptor = min(u, u - 4 * slots), u = slot * 4 + the record's upper byte
+        const unsigned q_lo = (unsigned)slot, q_wrap = q_lo - (unsigned)S;
+        // (slot + delay) % slots = min(u, u - slots), u = slot + the record's upper byte; below it the cell
         auto add = [&](const uint2 sy, bool crowded) {
             const unsigned dq = sy.x >> 24;
-            const unsigned plane = min(dq + q_lo, dq + q_wrap);
-            Sum *cell = ring_l + (mad_u24(plane, (unsigned)span, sy.x & 0xFFFFFFu) - (unsigned)e0);
+            Sum *cell = ring_l + mad_u24(min(dq + q_lo, dq + q_wrap), (unsigned)cells, sy.x & 0xFFFFFFu);
             if constexpr (kFixed)
                 atomicAdd(cell, to_fixed(__uint_as_float(sy.y)));
             else if (!crowded)
@@ -252,13 +316,13 @@ __global__ __launch_bounds__(kRbBlock) void sim_resident_batch_kernel(bmtk_glif3
                 }
             }
         };
-        for (uint32_t at_p = b.lo + part; at_p < b.hi; at_p += kRbTogether * step) {
-            uint2 sy[kRbTogether];
+        for (uint32_t at_p = b.lo + part; at_p < b.hi; at_p += kTogether * step) {
+            uint2 sy[kTogether];
 #pragma unroll
-            for (int u = 0; u < kRbTogether; ++u)
+            for (int u = 0; u < kTogether; ++u)
                 if (at_p + u * step < b.hi) sy[u] = table[at_p + u * step];
 #pragma unroll
-            for (int u = 0; u < kRbTogether; ++u)
+            for (int u = 0; u < kTogether; ++u)
                 if (at_p + u * step < b.hi) add(sy[u], u == 0);
         }
     };
@@ -448,9 +512,16 @@ __global__ __launch_bounds__(kRbBlock) void sim_resident_batch_kernel(bmtk_glif3
         if (kReaderOwns) store();
     }
     __syncthreads();
-    for (int c = tid; c < S * GLIF3_NREC * span; c += kRbBlock) {
-        const int plane = c / span, k = c - plane * span;
-        if (k < mine) ring_g[(int64_t)plane * n + k] = ring_l[c];
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) {
+        if (!owns(u)) continue;
+        unsigned word = sums[u];
+        asm volatile("" : "+v"(word));  // (what the reads of the ring worked out from it is not kept for this)
+#pragma unroll 1
+        for (int k = 0; k < S; ++k)
+#pragma unroll
+            for (int r = 0; r < GLIF3_NREC; ++r)
+                if (word >> r & 1u) ring_g[(int64_t)(k * GLIF3_NREC + r) * n + place(u)] = ring_l[k * cells + cell_of(word, r, place(u))];
     }
 }
 
@@ -516,9 +587,11 @@ int simulate_resident_batch(const bmtk_glif3_sim &s, int64_t step0, int64_t n_st
     const int64_t n = s.n_neurons;
     BMTK_REQUIRE(batch >= 1 && batch <= kWave, "glif3_simulate_fwd: resident trials come in batches of 1 to 64");
     const bool wide = span > kRbBlock;
-    BMTK_REQUIRE(span >= kWave && span % kWave == 0 && span <= (batch == 1 ? 2 * (kRbBlock - kWave) : kRbBlock) && G == (n + span - 1) / span,
-                 "glif3_simulate_fwd: rb_span must be a multiple of 64 up to 1024 (one trial: 1920) and rb_groups ceil(n_neurons / rb_span)");
-    BMTK_REQUIRE(wide == (batch == 1), "glif3_simulate_fwd: a single trial is resident in spans above 1024 here, in shorter ones by res_span");
+    BMTK_REQUIRE(span >= kWave && span % kWave == 0 && span <= 2 * kRbReader * kWave && G == (n + span - 1) / span,
+                 "glif3_simulate_fwd: rb_span must be a multiple of 64 up to 1920 and rb_groups ceil(n_neurons / rb_span)");
+    BMTK_REQUIRE(wide || batch > 1, "glif3_simulate_fwd: a single trial is resident in spans above 1024 here, in shorter ones by res_span");
+    BMTK_REQUIRE(s.rb_cells ? batch > 1 && s.rb_extra >= 0 && s.rb_extra <= 2 * span : s.rb_extra == 2 * span && (batch == 1 || !wide),
+                 "glif3_simulate_fwd: rb_extra must lie in 0..2 * rb_span with rb_cells (batches; spans above 1024 need it) and be 2 * rb_span without");
     BMTK_REQUIRE(W >= 1 && W <= batch && s.rb_team_shift >= 0 && s.rb_team_shift <= 6 && s.rb_list >= kWave,
                  "glif3_simulate_fwd: rb_ways must lie in 1..batch, rb_team_shift in 0..6, rb_list from 64 on");
     BMTK_REQUIRE(s.rb_seg && s.rb_packed && s.rb_ring && s.rb_hist && s.res_sync, "glif3_simulate_fwd: resident trials need rb_* and res_sync");
@@ -530,7 +603,7 @@ int simulate_resident_batch(const bmtk_glif3_sim &s, int64_t step0, int64_t n_st
     BMTK_REQUIRE(s.sum_shift >= 0 && s.sum_shift <= BMTK_SUM_SHIFT_MAX, "glif3_simulate_fwd: sum_shift must lie in 0..BMTK_SUM_SHIFT_MAX");
     BMTK_REQUIRE((s.rb_in_ptr == nullptr) == (s.rb_in_events == nullptr), "glif3_simulate_fwd: rb_in_ptr and rb_in_events go together");
     BMTK_REQUIRE(n_steps < (1ll << 30) && n + s.n_inputs < (1ll << 24), "glif3_simulate_fwd: too many steps or sources for resident trials");
-    const size_t lds = (size_t)S * GLIF3_NREC * span * (wide ? sizeof(float) : sizeof(unsigned long long)) + (size_t)s.rb_list * sizeof(unsigned);
+    const size_t lds = (size_t)S * (2 * span + s.rb_extra) * (batch == 1 ? sizeof(float) : sizeof(unsigned long long)) + (size_t)s.rb_list * sizeof(unsigned);
     BMTK_REQUIRE(lds + 256u <= kResLdsBytes, "glif3_simulate_fwd: the ring slice of resident trials does not fit in LDS");
     RbLaunch q{};
     q.step0 = step0;
@@ -540,13 +613,18 @@ int simulate_resident_batch(const bmtk_glif3_sim &s, int64_t step0, int64_t n_st
     q.has_events = s.rb_in_ptr != nullptr;
     q.unit = ldexp(1.0, -32 - s.sum_shift);
     BMTK_REQUIRE((wide ? 2 * kRbReader * kWave : kRbBlock) * (int64_t)kListGroups >= n, "glif3_simulate_fwd: more neurons than resident trials can hold");
-    const bool owns = span > kRbReader * kWave;
-    const void *const kernels[2][2] = {
-        {reinterpret_cast<const void *>(sim_resident_batch_kernel<1, unsigned long long, false, false>),
-         reinterpret_cast<const void *>(sim_resident_batch_kernel<1, unsigned long long, false, true>)},
-        {reinterpret_cast<const void *>(sim_resident_batch_kernel<1, unsigned long long, true, false>),
-         reinterpret_cast<const void *>(sim_resident_batch_kernel<1, unsigned long long, true, true>)}};
-    const void *kernel = wide ? reinterpret_cast<const void *>(sim_resident_batch_kernel<2, float, false, false>) : kernels[save][owns];
+    using Fixed = unsigned long long;
+    auto address = [](auto *k) { return reinterpret_cast<const void *>(k); };
+    const bool owns = span > kRbReader * kWave, few = s.rb_cells != nullptr;
+    const void *const kernels[2][2][2] = {  // one neuron to a thread: few sums, record, neurons of the reader's
+        {{address(sim_resident_batch_kernel<1, Fixed, true, false, false>), address(sim_resident_batch_kernel<1, Fixed, true, false, true>)},
+         {address(sim_resident_batch_kernel<1, Fixed, true, true, false>), address(sim_resident_batch_kernel<1, Fixed, true, true, true>)}},
+        {{address(sim_resident_batch_kernel<1, Fixed, false, false, false>), address(sim_resident_batch_kernel<1, Fixed, false, false, true>)},
+         {address(sim_resident_batch_kernel<1, Fixed, false, true, false>), address(sim_resident_batch_kernel<1, Fixed, false, true, true>)}}};
+    const void *kernel = batch == 1 ? address(sim_resident_batch_kernel<2, float, true, false, false>)
+                         : !wide    ? kernels[few][save][owns]
+                         : save     ? address(sim_resident_batch_kernel<2, Fixed, false, true, false>)
+                                    : address(sim_resident_batch_kernel<2, Fixed, false, false, false>);
     hipError_t err = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (err != hipSuccess) {
         set_error("glif3_simulate_fwd: resident trials need %zu bytes of LDS: %s", lds, hipGetErrorString(err));
@@ -594,7 +672,52 @@ int simulate_resident_batch(const bmtk_glif3_sim &s, int64_t step0, int64_t n_st
 
 }  // namespace bmtk
 
+namespace bmtk {
+
+__global__ __launch_bounds__(kBlock) void receptors_used_kernel(int64_t nnz, const int32_t *__restrict__ indices, const uint8_t *__restrict__ receptors,
+                                                                uint32_t *__restrict__ used)
+{
+    for (int64_t p = (int64_t)blockIdx.x * kBlock + threadIdx.x; p < nnz; p += (int64_t)gridDim.x * kBlock) {
+        const unsigned bit = 1u << (receptors[p] & 3u);
+        uint32_t *const word = used + indices[p];
+        // (nearly always there already: a look costs less than an atomic)
+        if (!(__hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & bit)) atomicOr(word, bit);
+    }
+}
+
+__global__ __launch_bounds__(kBlock) void pack_cells_kernel(int64_t nnz, int span, const uint32_t *__restrict__ words, uint2 *__restrict__ packed)
+{
+    for (int64_t p = (int64_t)blockIdx.x * kBlock + threadIdx.x; p < nnz; p += (int64_t)gridDim.x * kBlock) {
+        const unsigned x = packed[p].x, i = x & 0xFFFFFFu;
+        const int r = (int)(x >> 24 & 3u), place = (int)(i % (unsigned)span);
+        packed[p].x = (x >> 26) << 24 | (unsigned)(words ? rb_cell(words[i], r, place, span) : r * span + place);
+    }
+}
+
+}  // namespace bmtk
+
 using namespace bmtk;
+
+extern "C" int bmtk_csr_receptors_used(int64_t nnz, const int32_t *indices, const uint8_t *receptors, uint32_t *used, void *stream)
+{
+    BMTK_REQUIRE(nnz >= 0 && (nnz == 0 || (indices && receptors && used)), "csr_receptors_used: bad arguments");
+    if (nnz == 0) return BMTK_OK;
+    const int64_t blocks = (nnz + kBlock - 1) / kBlock;
+    hipLaunchKernelGGL(receptors_used_kernel, dim3((unsigned)(blocks < 4096 ? blocks : 4096)), dim3(kBlock), 0, (hipStream_t)stream, nnz, indices, receptors, used);
+    BMTK_CHECK_LAUNCH("csr_receptors_used");
+    return BMTK_OK;
+}
+
+extern "C" int bmtk_csr_pack_cells(int64_t nnz, int32_t span, const uint32_t *cells, bmtk_synapse *packed, void *stream)
+{
+    BMTK_REQUIRE(nnz >= 0 && span > 0 && (nnz == 0 || packed), "csr_pack_cells: bad arguments");
+    if (nnz == 0) return BMTK_OK;
+    const int64_t blocks = (nnz + kBlock - 1) / kBlock;
+    hipLaunchKernelGGL(pack_cells_kernel, dim3((unsigned)(blocks < 4096 ? blocks : 4096)), dim3(kBlock), 0, (hipStream_t)stream, nnz, span, cells,
+                       reinterpret_cast<uint2 *>(packed));
+    BMTK_CHECK_LAUNCH("csr_pack_cells");
+    return BMTK_OK;
+}
 
 extern "C" int bmtk_events_by_trial(int32_t batch, int64_t step0, int64_t n_steps, int32_t late, const int64_t *in_ptr,
                                     const int32_t *in_events, int32_t *counts, const int64_t *first, int32_t *sources, void *stream)

@@ -58,6 +58,7 @@ RES_LDS_EXTRA = RES_ACT_ENTRIES * 4 + 256   # the list plus the kernel's static 
 SOLO_LDS_PER_ELEMENT = 4 * 4
 SOLO_LDS_EXTRA = 10240 + 2048
 RB_WIDE_SPAN = 1920             # neurons of a workgroup at most with two to a thread
+RB_TWO_COST = 1.35              # a step of resident trials with two neurons to a thread against one (51,978 x 32: 1.40, 20,011 x 20: 1.3)
 RB_LIST_MIN, RB_LDS_STATIC = 2000, 256   # the form with resident trials: least room (words) for its lists of rows, static LDS
 SUM_SHIFT_MAX = 120             # BMTK_SUM_SHIFT_MAX
 TRIALS_TABLE_BYTES = 1 << 30    # tables and ring of the form with resident trials at most, or TRIALS_TABLE_RATIO times the synapses' 10 bytes
@@ -98,31 +99,49 @@ def lists_pay(span, groups, rate_hz, h_ms=1.0):
     return fired + math.sqrt(2.0 * fired * math.log(max(2, groups))) <= LIST_MAX
 
 
-def resident_trials_plan(n_neurons, batch, ring_slots, n_cu):
+def resident_trials_plan(n_neurons, batch, ring_slots, n_cu, third=None):
     """How the trials of a batch share ``n_cu`` compute units when each keeps its state in registers and its arrivals of
-    the next ring_slots - 1 steps in LDS: dict(span, groups, ways, passes, list) -- ``ways`` trials side by side on
+    the next ring_slots - 1 steps in LDS: dict(span, groups, ways, passes, list, few) -- ``ways`` trials side by side on
     ``groups`` workgroups of ``span`` neurons each, ``passes`` launches, ``list`` places in the list of rows -- or None
-    where a single trial does not fit.  As few launches as possible: a step costs much the same whatever runs beside it.  One trial:
-    only where the network is too large for the resident mode."""
+    where a single trial does not fit.  ``third``: how many third and fourth receptors the neurons before the i-th use
+    (n_neurons + 1 numbers; receptors that no synapse of a neuron ends on have no sums), or None where every neuron is to have all four.
+    One trial: only where the network is too large for the resident mode, and with four sums in fp32.
+
+    A step costs much the same whatever runs beside it: as few launches as possible, if need be with sums only for what is in use
+    (``few``) and two neurons to a thread (spans above 1024), which take RB_TWO_COST times as long a step."""
     cus, slots = n_cu - n_cu % 8, ring_slots - 1
     if not 1 <= batch <= 64 or cus <= 0 or n_neurons <= 0 or slots < 1:
         return None
+
+    def places(span, few=False):
+        """Words of LDS beside the sums of so many neurons."""
+        extra = 2 * span
+        if few:
+            first = np.arange(0, n_neurons, span)
+            extra = int((third[np.minimum(first + span, n_neurons)] - third[first]).max())
+        return (RES_LDS_BYTES - RB_LDS_STATIC - slots * (2 * span + extra) * (4 if batch == 1 else 8)) // 4
+
+    def plan(span, ways, passes, few=False):
+        return dict(span=span, groups=-(-n_neurons // span), ways=ways, passes=passes, list=min(RES_ACT_ENTRIES, places(span, few)), few=few)
+
     if batch == 1:
         # one trial of more neurons than the compute units have threads: two to a thread, sums in fp32
         span = -(-(-(-n_neurons // cus)) // 64) * 64
-        rows = min(RES_ACT_ENTRIES, (RES_LDS_BYTES - RB_LDS_STATIC) // 4 - span * slots * NREC)
-        if not 1024 < span <= RB_WIDE_SPAN or rows < RB_LIST_MIN:
-            return None
-        return dict(span=span, groups=-(-n_neurons // span), ways=1, passes=1, list=rows)
-    per_neuron = slots * NREC * 8
-    span_max = min(1024, (RES_LDS_BYTES - RB_LDS_STATIC - 4 * RB_LIST_MIN) // per_neuron // 64 * 64)
-    if span_max < 64 or -(-n_neurons // span_max) > cus:
-        return None
-    passes = -(-batch // min(batch, cus // -(-n_neurons // span_max)))
-    ways = -(-batch // passes)
-    span = -(-(-(-n_neurons // (cus // ways))) // 64) * 64
-    rows = min(RES_ACT_ENTRIES, (RES_LDS_BYTES - RB_LDS_STATIC - span * per_neuron) // 4)
-    return dict(span=span, groups=-(-n_neurons // span), ways=ways, passes=passes, list=rows)
+        return plan(span, 1, 1) if 1024 < span <= RB_WIDE_SPAN and places(span) >= RB_LIST_MIN else None
+    best, best_cost = None, None
+    # (of equals the first: few sums cost 0.1 us a step to tell apart)
+    for few, most, cost in ((False, 1024, 1.0), (True, 1024, 1.05), (True, RB_WIDE_SPAN, RB_TWO_COST))[:1 if third is None else 3]:
+        most = next((span for span in range(most, 0, -64) if places(span, few) >= RB_LIST_MIN), 0)
+        if not most or -(-n_neurons // most) > cus:
+            continue
+        passes = -(-batch // min(batch, cus // -(-n_neurons // most)))
+        ways = -(-batch // passes)
+        span = -(-(-(-n_neurons // (cus // ways))) // 64) * 64
+        if places(span, few) < RB_LIST_MIN:      # (sums dealt out unevenly)
+            span = most
+        if best is None or passes * cost < best_cost:
+            best, best_cost = plan(span, ways, passes, few), passes * cost
+    return best
 
 
 def fixed_point_shift(tables, n_neurons):
@@ -176,7 +195,7 @@ def fused_pays(n_neurons, batch, n_synapses, class_table, rate_hz, h_ms=1.0):
 def trials_bytes(plan, n_neurons, batch, ring_slots, n_inputs, n_synapses):
     """Device memory that the form with resident trials takes beside the synapse tables: bounds of every workgroup's segment of
     every row, packed records, the ring behind a call."""
-    return ((n_neurons + n_inputs) * (plan["groups"] + 1) * 4 + n_synapses * 8
+    return ((n_neurons + n_inputs) * (plan["groups"] + 1) * 4 + n_synapses * 8 + n_neurons * 4
             + batch * (ring_slots - 1) * NREC * n_neurons * (8 if batch > 1 else 4))
 
 
@@ -192,7 +211,8 @@ def trials_pay(plan, n_neurons, batch, n_synapses, class_table, rate_hz, h_ms, f
     the driver that would run otherwise, the fused pull form (``fused``) or pushed events."""
     per_trial = n_neurons * float(rate_hz) * 1e-3 * h_ms
     events = n_synapses * batch * float(rate_hz) * 1e-3 * h_ms
-    trials = plan["passes"] * (TRIALS_PS_PER_PASS + TRIALS_PS_PER_ROW * per_trial) + TRIALS_PS_PER_EVENT * events
+    step = (TRIALS_PS_PER_PASS + TRIALS_PS_PER_ROW * per_trial) * (RB_TWO_COST if batch > 1 and plan["span"] > 1024 else 1.0)
+    trials = plan["passes"] * step + TRIALS_PS_PER_EVENT * events
     if fused:
         other = (FUSE_PS_PER_STEP + FUSE_PS_PER_SYNAPSE * n_synapses + FUSE_PS_PER_EVENT * events
                  + FUSE_PS_PER_ELEMENT * n_neurons * batch)
@@ -451,10 +471,16 @@ class Glif3Simulator:
             wanted = resident == "auto" and fused == "auto" and pull == "auto" and self.pull_table is None
         else:
             wanted = bool(resident_trials)
-        plan = None
+        plan = used = None
         if wanted and self.rec is not None and not self.res_span and self.delay_offset == 0 and self.delay_bits == 6:
             n_cu = torch.cuda.get_device_properties(self.dev).multi_processor_count
-            plan = resident_trials_plan(self.n, self.batch, self.L, n_cu)
+            # (of a batch: what it takes at best, before the tables are looked at)
+            plan = resident_trials_plan(self.n, self.batch, self.L, n_cu, np.zeros(self.n + 1, np.int64) if self.batch > 1 else None)
+            if plan and self.batch > 1:
+                used = self._receptors_used()
+                third = torch.zeros(self.n + 1, dtype=torch.int64, device=self.dev)
+                torch.cumsum(self._third_and_fourth(used), 0, out=third[1:])
+                plan = resident_trials_plan(self.n, self.batch, self.L, n_cu, third.cpu().numpy())
         if plan and ((self.n + self.n_inputs) * (plan["groups"] + 1) >= 2 ** 32 or self.n + self.n_inputs >= 2 ** 24
                      or n_syn >= 2 ** 31 or self.pull_table is not None):
             plan = None
@@ -472,7 +498,7 @@ class Glif3Simulator:
             raise ValueError("resident trials need a recurrent table, a batch of 2 to 64 (or more neurons than the resident mode holds), delay_offset 0, no pull table, weights "
                              "that 64-bit fixed point holds and a network whose trial fits the compute units")
         if plan:
-            self._trials = dict(plan, seg=None, insisted=resident_trials is True)
+            self._trials = dict(plan, seg=None, insisted=resident_trials is True, used=used)
 
     def _trials_weights_ok(self, fixed_point_ok):
         """Whether weights that 64-bit fixed point does not all hold exactly are good enough for a caller who insists on the form
@@ -483,6 +509,18 @@ class Glif3Simulator:
         size = sum(t.weights.abs().sum(dtype=torch.float64) for t in tables) / max(1, sum(t.nnz for t in tables))
         most = sum(t.weights.abs().max().double() * torch.bincount(t.indices, minlength=self.n).max() for t in tables if t.nnz)
         return bool((size >= 2.0 ** -8) & (most < 2.0 ** 30))
+
+    def _receptors_used(self):
+        """Which receptors some synapse of a neuron ends on, a bit each."""
+        used = torch.zeros(self.n, dtype=torch.int32, device=self.dev)
+        for t in (self.rec, self.inp):
+            if t is not None:
+                _lib.check(self.lib.bmtk_csr_receptors_used(t.nnz, _p(t.indices), _p(t.receptors), _p(used), _stream()))
+        return used
+
+    @staticmethod
+    def _third_and_fourth(used):
+        return (sum((used >> r) & 1 for r in range(NREC)) - 2).clamp_(min=0)
 
     def _setup_trials(self):
         """Tables and buffers of the form with resident trials: recurrent and input rows as one table sorted by target,
@@ -506,9 +544,17 @@ class Glif3Simulator:
             row, at = row + t.n_rows, at + t.nnz
         if self.sum_shift:
             packed.view(torch.float32)[:, 1] *= 2.0 ** self.sum_shift
+        cells, extra = None, 2 * tr["span"]
+        if tr["few"]:           # where a neuron's third sum stands among its workgroup's
+            own = self._third_and_fourth(tr["used"])
+            before = torch.cumsum(own, 0) - own
+            begin = torch.arange(groups, device=self.dev) * tr["span"]
+            before -= before[begin].repeat_interleave(tr["span"])[:n]
+            cells, extra = (tr["used"] | before << NREC).to(torch.int32), int((before + own).max())
+        _lib.check(self.lib.bmtk_csr_pack_cells(at, tr["span"], _p(cells), _p(packed), _stream()))
         # lanes to a segment at most: about as many as it holds synapses on average
         segment = int(math.ceil(math.log2(max(1.0, at / float(max(1, row)) / groups))))
-        tr.update(seg=seg, packed=packed, max_team_shift=min(6, segment),
+        tr.update(seg=seg, packed=packed, cells=cells, extra=extra, max_team_shift=min(6, segment),
                   ring=torch.zeros(self.batch, self.L - 1, NREC, n, device=self.dev,
                                    dtype=torch.int64 if self.batch > 1 else torch.float32),
                   hist=torch.zeros(tr["ways"], 4, n_words(n) + 1, dtype=torch.int64, device=self.dev))
@@ -524,6 +570,7 @@ class Glif3Simulator:
         rows = max(1.0, self.n * self.expected_rate_hz * 1e-3 * self.h + events)
         s.rb_team_shift = max(0, min(tr["max_team_shift"], int(math.log2(max(1.0, 900.0 / rows)))))
         s.rb_late_events = 1 if self.fuse_rereads else 0
+        s.rb_cells, s.rb_extra = _p(tr["cells"]), tr["extra"]
         s.rb_seg, s.rb_packed, s.rb_ring, s.rb_hist = _p(tr["seg"]), _p(tr["packed"]), _p(tr["ring"]), _p(tr["hist"])
         s.res_sync, s.res_spin_limit = _p(self.res_sync), int(self.spin_limit)
         if self.inp is None or self.in_ptr is None:
@@ -574,8 +621,9 @@ class Glif3Simulator:
         if tr is None or tr["seg"] is None:
             return
         left, slots = tr["ring"], self.L - 1
-        for t in (left, tr["hist"], tr["seg"], tr["packed"]):
-            self._in_use(t)
+        for t in (left, tr["hist"], tr["seg"], tr["packed"], tr["cells"]):
+            if t is not None:
+                self._in_use(t)
         if self.fuse_table is not None:
             self._left_ring, self._pend_from, self._pend_until, self._trials_left = left, self.step, self.step + slots, True
             return

@@ -49,7 +49,7 @@ extern "C" {
 
 /* Bumped whenever a struct layout or a signature below changes; bmtk_amd_abi_version() returns the value the
  * library was built with. */
-#define BMTK_AMD_ABI_VERSION 29
+#define BMTK_AMD_ABI_VERSION 30
 int bmtk_amd_abi_version(void);
 const char *bmtk_amd_last_error(void);
 /* sizeof(bmtk_glif3_sim) as the library was compiled, for bindings that mirror the struct */
@@ -387,17 +387,19 @@ typedef struct bmtk_glif3_sim {
      * record).  The arrivals still ahead at the end of a call are left in rb_ring, and a call begins with those: neither
      * `ring` nor work_bits is used.  The fused form takes them over (rb_pend_until).  Uses res_sync and res_spin_limit as
      * the resident mode does. */
-    int32_t rb_span;                   /* neurons of a workgroup: a multiple of 64 up to 1024; one trial: from 1088 to 1920 */
+    int32_t rb_span;                   /* neurons of a workgroup: a multiple of 64 up to 1920 (above 1024 a thread holds two); one trial:
+                                        * from 1088 on */
     int32_t rb_groups;
     int32_t rb_ways;                   /* trials of a launch: rb_ways * rb_groups workgroups must be resident at once */
     int32_t rb_team_shift;             /* 2^rb_team_shift lanes read a row's segment */
     int32_t rb_list;                   /* words of LDS for the rows of two steps, at least 64 (a step with more than (rb_list - 64) / 2
-                                        * rows takes longer); (ring_slots-1)*32*rb_span (one trial: *16) + 4*rb_list
-                                        * + 256 bytes of LDS */
+                                        * rows takes longer); (ring_slots-1)*8*(2*rb_span + rb_extra) (one trial: *4)
+                                        * + 4*rb_list + 256 bytes of LDS */
     int32_t rb_late_events;            /* the input events of a call's last step (each id once; repeats are delivered at once) are
                                         * left to the next call and its lists, as with in_again */
     const uint32_t *rb_seg;            /* [n_neurons + n_inputs][rb_groups + 1], bmtk_csr_segment_offsets with rb_span over rb_packed */
-    const bmtk_synapse *rb_packed;     /* recurrent rows followed by the input rows, sorted by target within a row */
+    const bmtk_synapse *rb_packed;     /* recurrent rows followed by the input rows, sorted by target within a row, with the cells
+                                        * of rb_cells in place of target and receptor (bmtk_csr_pack_cells) */
     uint64_t *rb_ring;                 /* [batch][ring_slots - 1][4][n_neurons], zeroed before the first run (one trial: floats) */
     uint64_t *rb_hist;                 /* [rb_ways][4][ceil(n_neurons/64) + 1], zeroed once */
     const int64_t *rb_in_ptr;          /* [batch * (n_steps + 1) + 1], or NULL: input events of trial b in step step0 - 1 + k are */
@@ -406,6 +408,12 @@ typedef struct bmtk_glif3_sim {
                                         * clears them */
     float *rb_save_v;                  /* with save_v (batches, up to 65535 steps a call): [batch][n_steps][n_neurons] scratch, and */
     uint8_t *rb_save_flags;            /* as many bytes with save_flags */
+    const uint32_t *rb_cells;          /* batches: [n_neurons], bits 0..3 the receptors that some synapse ends on
+                                        * (bmtk_csr_receptors_used).  Only those have sums in LDS: the first two of every neuron in
+                                        * planes of rb_span, third and fourth behind these; from bit 4 on, where the neuron's third
+                                        * stands among its workgroup's.  NULL (one trial; spans up to 1024): four planes */
+    int32_t rb_extra;                  /* third and fourth sums of a workgroup's neurons at most; without rb_cells 2 * rb_span */
+    int32_t _pad4;
     /* Fixed-point sums of the fused and the resident form: their tables (fuse_packed, rb_packed) hold the weights times
      * 2^sum_shift, and a sum's lowest bit (rb_ring's too) stands for 2^-(32 + sum_shift).  A weight is held exactly when that
      * divides it, otherwise cut off towards zero; what may reach a neuron in a step must stay below 2^(31 - sum_shift). */
@@ -476,6 +484,13 @@ typedef struct bmtk_glif3_sim {
  * into its LDS ring slice with LDS atomics -- no global atomics and no state
  * traffic.  The barrier spins a bounded number of times; see res_sync. */
 int bmtk_glif3_simulate_fwd(const bmtk_glif3_sim *sim, int64_t step0, int64_t n_steps, void *stream);
+
+/* Sets bit r of used[i] (zeroed by the caller) where a synapse of the table ends on receptor r of neuron i. */
+int bmtk_csr_receptors_used(int64_t nnz, const int32_t *indices, const uint8_t *receptors, uint32_t *used, void *stream);
+
+/* Packed records of the standard packing (6-bit delays) in place: the cell of bmtk_glif3_sim.rb_cells that a record's target and
+ * receptor have, workgroups of `span` neurons, takes the lower 24 bits, the delay the upper eight.  NULL: four planes a neuron. */
+int bmtk_csr_pack_cells(int64_t nnz, int32_t span, const uint32_t *cells, bmtk_synapse *packed, void *stream);
 
 /* The input events of the steps step0 .. step0 + n_steps - 1 (step0 may be -1: a step without events) apart by trial.  With
  * `counts` ([batch][n_steps]) the events of every trial and step are counted; with `first` ([batch][n_steps], the running

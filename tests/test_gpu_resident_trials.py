@@ -69,6 +69,36 @@ def test_equals_the_oracle_over_two_calls(n, batch, max_delay, classes):
     _same(sim, outs, raster, st)
 
 
+PAIRS = ((0, 1), (2, 3), (1, 3), (0, 0), (0, 3), (2, 2), (1, 2))
+
+
+@pytest.mark.parametrize("n,batch,max_delay,classes,span,four", [
+    (65, 3, 6, None, None, 2), (64, 64, 1, 3, None, 0), (1010, 33, 4, None, 1024, 5), (1025, 5, 5, 7, 1088, 3), (1921, 12, 4, None, 1920, 97),
+    (1920, 64, 5, 11, 1920, 0), (4100, 16, 3, 5, 1408, 1)])
+def test_only_receptors_in_use_have_sums(n, batch, max_delay, classes, span, four):
+    """One or two of the four receptors in any combination, every `four`-th neuron with all four, one neuron to a thread and
+    two, a last workgroup of one neuron: raster and state bit for bit, over two calls in the form, one with the per-step record and one
+    with the driver that takes its place."""
+    cfg, _, _ = _case(n, batch, max_delay, classes, steps=200)
+    for k in ("rec_src", "inp_src"):
+        indptr, indices, w, d, r = cfg[k]
+        some = np.asarray(PAIRS, np.uint8)[indices % len(PAIRS), r & 1]
+        cfg[k] = indptr, indices, w, d, np.where(indices % four == four - 1, r, some).astype(np.uint8) if four else some
+    st = orc.new_state(n, batch, np.float32)
+    raster = orc.simulate(st, orc.precompute(cfg["par"], 1.0), 1.0, 200, batch=batch, class_id=cfg["class_id"],
+                          ring=np.zeros((cfg["L"], 4, n * batch), np.float32), rec=cfg["rec_src"], inp=cfg["inp_src"],
+                          in_ptr=cfg["in_ptr"], in_events=cfg["in_events"], i_ext=cfg["i_ext"], raster=True)["raster"]
+    sim = _sim(cfg, batch, resident_trials=True, fused=batch >= 8)
+    if span:
+        sim._trials.update(span=span, groups=-(-n // span), ways=min(batch, 256 // -(-n // span)), list=400)
+    sim._trials["few"] = True
+    outs = [sim.run(50), sim.run(60), sim.run(70, save_state=True)]
+    assert sim._trials["extra"] > 0 if four else sim._trials["extra"] == 0
+    outs.append(sim.run(20))
+    assert sim._trials is None
+    _same(sim, outs, raster, st)
+
+
 @pytest.mark.parametrize("how", ["short", "record", "ring"])
 @pytest.mark.parametrize("batch,fused", [(6, False), (16, True), (20, True)])
 def test_gives_way_to_the_other_drivers_with_arrivals_under_way(batch, fused, how):

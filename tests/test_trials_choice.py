@@ -1,4 +1,5 @@
 """How the trials of a batch are laid out on the compute units, and when that is expected to pay."""
+import numpy as np
 import pytest
 
 from bmtk_amd.layout import NREC
@@ -12,6 +13,22 @@ def test_plan_holds_every_neuron_and_trial(n, batch, slots):
     assert p["span"] % 64 == 0 and 64 <= p["span"] <= 1024 and p["groups"] == -(-n // p["span"])
     assert 8 * -(-p["ways"] * p["groups"] // 8) <= 256 and p["ways"] <= batch <= p["ways"] * p["passes"]
     assert (slots - 1) * NREC * 8 * p["span"] + 4 * p["list"] + RB_LDS_STATIC <= RES_LDS_BYTES and p["list"] >= 64
+
+
+@pytest.mark.parametrize("n,batch,slots,share", [(51978, 32, 6, 0.2), (20011, 20, 6, 0.2), (230924, 8, 6, 0.0), (230924, 8, 6, 0.2), (5000, 64, 20, 1.0),
+                                                 (120000, 16, 3, 2.0), (64, 2, 2, 2.0)])
+def test_plan_with_the_receptors_in_use(n, batch, slots, share):
+    """Third and fourth sums in the last neurons only: the workgroup that has most of them counts."""
+    extra = np.zeros(n, np.int64)
+    extra[n - int(n * share / 2):] = 2
+    third = np.concatenate([[0], np.cumsum(extra)])
+    p = resident_trials_plan(n, batch, slots, 256, third)
+    sums = 2 * p["span"] + max(third[min(k + p["span"], n)] - third[k] for k in range(0, n, p["span"]))
+    assert p["span"] % 64 == 0 and 64 <= p["span"] <= 1920 and p["groups"] == -(-n // p["span"])
+    assert 8 * -(-p["ways"] * p["groups"] // 8) <= 256 and p["ways"] <= batch <= p["ways"] * p["passes"]
+    assert (slots - 1) * 8 * sums + 4 * p["list"] + RB_LDS_STATIC <= RES_LDS_BYTES and p["list"] >= 2000
+    old = resident_trials_plan(n, batch, slots, 256)
+    assert p["passes"] <= old["passes"]
 
 
 def test_plan_of_what_does_not_fit():
