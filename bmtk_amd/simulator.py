@@ -356,6 +356,7 @@ class Glif3Simulator:
                     d = d.astype(np.int32 if wide else np.uint8)
                 return (t[0], t[1], t[2], d, t[4])
             rec, inp = shorten(rec), shorten(inp)
+        self.least_delay = min_delay - self.delay_offset    # ... of the tables' records
         self.L = int(ring_slots) if ring_slots else max_delay - self.delay_offset + 1
         self.rec = self._table(rec, self.n) if rec is not None else None
         self.inp = self._table(inp, None) if inp is not None else None
@@ -545,7 +546,7 @@ class Glif3Simulator:
         if self.sum_shift:
             packed.view(torch.float32)[:, 1] *= 2.0 ** self.sum_shift
         cells, extra = None, 2 * tr["span"]
-        if tr["few"]:           # where a neuron's third sum stands among its workgroup's
+        if tr.get("few"):           # where a neuron's third sum stands among its workgroup's
             own = self._third_and_fourth(tr["used"])
             before = torch.cumsum(own, 0) - own
             begin = torch.arange(groups, device=self.dev) * tr["span"]
@@ -879,6 +880,7 @@ class Glif3Simulator:
             s.res_spin_limit = int(self.spin_limit)
             s.rec_seg, s.inp_seg = _p(self.rec_seg), _p(self.inp_seg)
             s.res_fired = _p(self.res_fired)
+            s.res_min_delay = self.least_delay
             if self.res_unified is not None and s.inp_packed and self.res_groups > 1:
                 s.inp_packed = s.rec_packed      # the input offsets count from the start of the joint table
         if bits is not None:
