@@ -46,7 +46,7 @@ class Glif3Sim(C.Structure):
         ("probe_col", c_void_p), ("probe_v", c_void_p), ("probe_stride", c_int64), ("probe_every", c_int32),
         ("_pad1", c_int32),
         ("spike_step", c_void_p), ("spike_elem", c_void_p), ("spike_frac", c_void_p),
-        ("spike_cap", c_int64), ("spike_count", c_void_p), ("spike_ways", c_int32), ("_pad2", c_int32),
+        ("spike_cap", c_int64), ("spike_count", c_void_p), ("spike_ways", c_int32), ("res_min_delay", c_int32),
     ]
 
 
@@ -67,7 +67,7 @@ class Glif3Bwd(C.Structure):
     ]
 
 
-ABI_VERSION = 30  # BMTK_AMD_ABI_VERSION of include/bmtk_amd.h that the mirrors above were written for
+ABI_VERSION = 31  # BMTK_AMD_ABI_VERSION of include/bmtk_amd.h that the mirrors above were written for
 
 # name -> (restype, argtypes); every symbol include/bmtk_amd.h declares
 SIGNATURES = {
@@ -106,6 +106,7 @@ SIGNATURES = {
                                      c_void_p, c_void_p]),
     "bmtk_poisson_fill": (c_int32, [c_int64, c_int32, c_void_p, c_double, c_double, c_double, c_int64, C.c_uint64,
                                     c_void_p, c_void_p, c_void_p, c_void_p]),
+    "bmtk_resident_window_steps": (c_int32, [C.POINTER(Glif3Sim)]),
     "bmtk_glif3_simulate_fwd": (c_int32, [C.POINTER(Glif3Sim), c_int64, c_int64, c_void_p]),
     "bmtk_csr_receptors_used": (c_int32, [c_int64] + [c_void_p] * 4),
     "bmtk_csr_pack_cells": (c_int32, [c_int64, c_int32] + [c_void_p] * 3),

@@ -118,6 +118,40 @@ __device__ __forceinline__ bool glif3_update(Glif3Elem &s, const Glif3Prop &p, f
     return spike;
 }
 
+// The same step, operation for operation, for a wavefront that runs many steps on end: lanes choose between results instead of
+// taking branches (which cost some ten scalar instructions each, and keep independent arithmetic apart).
+// *fired: the ballot of the lanes with ``own`` that spiked; *frac is set in those only.
+__device__ __forceinline__ void glif3_update_wave(Glif3Elem &s, const Glif3Prop &p, float h, const float syn[GLIF3_NREC],
+                                                  float I, bool own, unsigned long long *fired, float *frac)
+{
+    const float v_old = s.V;
+    const bool held = s.ref > 0, leaves = s.ref == 1;
+    float S = 0.0f;
+#pragma unroll
+    for (int a = 0; a < GLIF3_NASC; ++a) S = S + p.c[a] * s.asc[a];
+    float U = v_old * p.P33 + (I + S) * p.P30;
+#pragma unroll
+    for (int k = 0; k < GLIF3_NREC; ++k) U = U + (p.P31[k] * s.y1[k] + p.P32[k] * s.y2[k]);
+    const float U_free = U;
+    const bool spike = own && !held && U > p.th;
+#pragma unroll
+    for (int a = 0; a < GLIF3_NASC; ++a) {
+        const float reset = p.amp[a] + s.asc[a] * p.r[a], decayed = s.asc[a] * p.d[a];
+        s.asc[a] = leaves ? reset : held ? s.asc[a] : decayed;
+    }
+    s.V = leaves ? p.Ur : held ? v_old : U;
+    s.ref = spike ? p.n_ref : held ? s.ref - 1 : s.ref;
+#pragma unroll
+    for (int k = 0; k < GLIF3_NREC; ++k) {
+        const float P21 = h * p.P11[k];
+        const float a1 = s.y1[k], a2 = s.y2[k];
+        s.y2[k] = P21 * a1 + p.P11[k] * a2;
+        s.y1[k] = a1 * p.P11[k] + syn[k] * p.psc0[k];
+    }
+    *fired = __ballot(spike);
+    if (*fired != 0ull) *frac = (p.th - v_old) / (U_free - v_old);
+}
+
 __device__ __forceinline__ void glif3_load(Glif3Elem &s, const float *V, const float *asc, const float *y1,
                                            const float *y2, const int32_t *ref, int64_t ne, int64_t e)
 {

@@ -11,6 +11,8 @@
 // microsecond, i.e. millions of steps) are this case: a step costs about a
 // microsecond instead of the two and a half the grid barrier sets as a floor.
 //
+// Where spikes arrive several steps late, resident_windows.hip does better.
+//
 // One compute unit runs it all, so what sets the pace of a step is how many
 // instructions its sixteen wavefronts issue (a SIMD issues for one of its four
 // wavefronts every four cycles; scalar bookkeeping counts like arithmetic), the
@@ -558,6 +560,9 @@ int simulate_resident_solo(const bmtk_glif3_sim &s, int64_t step0, int64_t n_ste
         set_error("glif3_simulate_fwd: a resident call covers fewer than 2^31 steps");
         return BMTK_E_ARG;
     }
+    bool windows = false;
+    const int status = simulate_resident_windows(s, step0, n_steps, stream, &windows);
+    if (windows || status != BMTK_OK) return status;
     const int hist = s.hist_slots ? s.hist_slots : 3;
     Solo r{step0, (int)n_steps, s.res_span, s.delay_offset, hist, 0};
     size_t lds = solo_lds_bytes(s.ring_slots, s.res_span);

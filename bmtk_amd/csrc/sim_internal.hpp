@@ -20,6 +20,10 @@ int simulate_resident(const bmtk_glif3_sim &s, int64_t step0, int64_t n_steps, h
 // whole synapse rows walked by a wavefront (resident_solo.hip).
 int simulate_resident_solo(const bmtk_glif3_sim &s, int64_t step0, int64_t n_steps, hipStream_t stream);
 
+// ... and where spikes arrive late enough for its wavefronts to run several steps between barriers (resident_windows.hip).
+// *taken: whether they do; if not, nothing has been launched.
+int simulate_resident_windows(const bmtk_glif3_sim &s, int64_t step0, int64_t n_steps, hipStream_t stream, bool *taken);
+
 // The trials of a batch, several side by side, each with its state in registers and its ring in LDS (resident_batch.hip).
 int simulate_resident_batch(const bmtk_glif3_sim &s, int64_t step0, int64_t n_steps, hipStream_t stream);
 

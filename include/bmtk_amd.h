@@ -49,7 +49,7 @@ extern "C" {
 
 /* Bumped whenever a struct layout or a signature below changes; bmtk_amd_abi_version() returns the value the
  * library was built with. */
-#define BMTK_AMD_ABI_VERSION 30
+#define BMTK_AMD_ABI_VERSION 31
 int bmtk_amd_abi_version(void);
 const char *bmtk_amd_last_error(void);
 /* sizeof(bmtk_glif3_sim) as the library was compiled, for bindings that mirror the struct */
@@ -454,7 +454,10 @@ typedef struct bmtk_glif3_sim {
      * resident mode launches at most 256) and no delay offset, a workgroup has a list of its own and keeps the count
      * in a register for the length of a call: no atomics on device memory at all. */
     int32_t spike_ways;
-    int32_t _pad2;
+    /* Single-workgroup form: no synapse of the two packed tables has a delay (as its record holds it, after the delay offset)
+     * below this many steps; 0 or 1: not known.  With delay_offset it says how long after its spike a first arrival comes,
+     * and the form runs up to half that many steps (8 at most) between two barriers. */
+    int32_t res_min_delay;
 } bmtk_glif3_sim;
 
 #define BMTK_RECORD_COUNT_STRIDE 16 /* 64-bit words between two counters of a record in several lists */
@@ -484,6 +487,10 @@ typedef struct bmtk_glif3_sim {
  * into its LDS ring slice with LDS atomics -- no global atomics and no state
  * traffic.  The barrier spins a bounded number of times; see res_sync. */
 int bmtk_glif3_simulate_fwd(const bmtk_glif3_sim *sim, int64_t step0, int64_t n_steps, void *stream);
+
+/* Steps that the single-workgroup form (res_groups == 1) runs between two barriers for this simulation: 0 where it takes a
+ * barrier every step. */
+int bmtk_resident_window_steps(const bmtk_glif3_sim *sim);
 
 /* Sets bit r of used[i] (zeroed by the caller) where a synapse of the table ends on receptor r of neuron i. */
 int bmtk_csr_receptors_used(int64_t nnz, const int32_t *indices, const uint8_t *receptors, uint32_t *used, void *stream);
