@@ -307,6 +307,68 @@ __global__ __launch_bounds__(kBlock) void compact_write_fused_kernel(const uint6
     }
 }
 
+// Input event lists looked over, a wavefront per step.  Bounded by launches and the one look at `found` that follows: the same in
+// array operations (marks at every step's start, differences, comparisons, reductions, four of them waited for) took 270 us a
+// call, 350 with repeats to list, beside runs of 1.5 to 2.3 ms; this takes 55, and 105 with repeats.
+__global__ __launch_bounds__(kBlock) void events_check_kernel(int64_t n_steps, const int64_t *__restrict__ in_ptr, int64_t n_events,
+                                                              const int32_t *__restrict__ in_events, int64_t n_ids, int32_t *__restrict__ repeats,
+                                                              unsigned *__restrict__ found)
+{
+    const int lane = lane_id();
+    const int64_t wave = (int64_t)blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave, n_waves = (int64_t)gridDim.x * (kBlock / kWave);
+    constexpr int kTogether = 4;
+    unsigned bad = 0u, total = 0u;
+    if (wave == 0 && (in_ptr[0] != 0 || in_ptr[n_steps] != n_events)) bad = BMTK_EVENTS_INCONSISTENT;
+    for (int64_t t = wave; t < n_steps; t += n_waves) {
+        const int64_t p0 = in_ptr[t], p1 = in_ptr[t + 1];
+        unsigned again = 0u;
+        if (p0 < 0 || p1 < p0 || p1 > n_events)
+            bad |= BMTK_EVENTS_INCONSISTENT;    // (nothing is read through them)
+        else
+            for (int64_t base = p0; base < p1; base += kTogether * kWave) {
+                int32_t id[kTogether], before[kTogether];
+#pragma unroll
+                for (int u = 0; u < kTogether; ++u) {
+                    const int64_t p = min(base + u * kWave + lane, p1 - 1);
+                    id[u] = in_events[p];
+                    before[u] = in_events[max(p - 1, p0)];
+                }
+#pragma unroll
+                for (int u = 0; u < kTogether; ++u) {
+                    const int64_t p = base + u * kWave + lane;
+                    if (p < p1 && (id[u] < 0 || id[u] >= n_ids)) bad |= BMTK_EVENTS_INCONSISTENT;
+                    if (p < p1 && id[u] < before[u]) bad |= BMTK_EVENTS_UNORDERED;
+                    again += (unsigned)__popcll(__ballot(p > p0 && p < p1 && id[u] == before[u]));
+                }
+            }
+        if (lane == 0) repeats[t] = (int32_t)again;
+        total += again;
+    }
+    if (bad) atomicOr(found, bad);
+    if (lane == 0 && total) atomicAdd(found + 1, total);
+}
+
+// The second and later occurrences of an id in its step, in order: those of step t from to[first[t]] on.
+__global__ __launch_bounds__(kBlock) void events_repeated_kernel(int64_t n_steps, const int64_t *__restrict__ in_ptr,
+                                                                 const int32_t *__restrict__ in_events, const int64_t *__restrict__ first,
+                                                                 int32_t *__restrict__ to)
+{
+    const int lane = lane_id();
+    const int64_t wave = (int64_t)blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave, n_waves = (int64_t)gridDim.x * (kBlock / kWave);
+    for (int64_t t = wave; t < n_steps; t += n_waves) {
+        int64_t at = first[t];
+        if (first[t + 1] == at) continue;
+        const int64_t p0 = in_ptr[t], p1 = in_ptr[t + 1];
+        for (int64_t base = p0; base < p1; base += kWave) {
+            const int64_t p = base + lane;
+            const bool same = p > p0 && p < p1 && in_events[p] == in_events[p - 1];
+            const unsigned long long m = __ballot(same);
+            if (same) to[at + lane_prefix(m)] = in_events[p];
+            at += __popcll(m);
+        }
+    }
+}
+
 // ---------------------------------------------------------------------------
 // Event-driven scatter: wavefronts walk the out-going synapses of the active
 // elements 64 at a time (coalesced table reads), fp32 atomics into the ring.
@@ -568,6 +630,29 @@ int bmtk_spikes_compact_bits(const uint64_t *zbits, int64_t n, int32_t *ids, int
     BMTK_REQUIRE(zbits && ids && count && workspace, "spikes_compact_bits: pointers must be non-null");
     uint32_t *block_count = (uint32_t *)((uint64_t *)workspace + n_words_of(n) + 1);
     return compact_from_bits(zbits, n, ids, count, block_count, (hipStream_t)stream);
+}
+
+int bmtk_events_check(int64_t n_steps, const int64_t *in_ptr, int64_t n_events, const int32_t *in_events, int64_t n_ids, int32_t *repeats,
+                      uint32_t *found, void *stream)
+{
+    BMTK_REQUIRE(n_steps >= 0 && n_events >= 0 && n_ids >= 0, "events_check: bad sizes");
+    BMTK_REQUIRE(in_ptr && (in_events || n_events == 0) && (repeats || n_steps == 0) && found, "events_check: pointers must be non-null");
+    const int64_t blocks = (n_steps + kBlock / kWave - 1) / (kBlock / kWave);
+    hipLaunchKernelGGL(events_check_kernel, dim3((unsigned)(blocks < 1 ? 1 : blocks < 8192 ? blocks : 8192)), dim3(kBlock), 0, (hipStream_t)stream,
+                       n_steps, in_ptr, n_events, in_events, n_ids, repeats, found);
+    BMTK_CHECK_LAUNCH("events_check");
+    return BMTK_OK;
+}
+
+int bmtk_events_repeated(int64_t n_steps, const int64_t *in_ptr, const int32_t *in_events, const int64_t *first, int32_t *to, void *stream)
+{
+    BMTK_REQUIRE(n_steps > 0, "events_repeated: bad sizes");
+    BMTK_REQUIRE(in_ptr && in_events && first && to, "events_repeated: pointers must be non-null");
+    const int64_t blocks = (n_steps + kBlock / kWave - 1) / (kBlock / kWave);
+    hipLaunchKernelGGL(events_repeated_kernel, dim3((unsigned)(blocks < 8192 ? blocks : 8192)), dim3(kBlock), 0, (hipStream_t)stream, n_steps,
+                       in_ptr, in_events, first, to);
+    BMTK_CHECK_LAUNCH("events_repeated");
+    return BMTK_OK;
 }
 
 int bmtk_csr_propagate_scatter(const int32_t *active, const int32_t *n_active, int64_t max_active, int32_t batch,

@@ -797,40 +797,49 @@ class Glif3Simulator:
         back what those events still had under way there; the other forms have delivered them and look at later steps only."""
         if self.inp is None and not self.inp_without_synapses:
             raise ValueError("no input synapse table")
+        n_ids = self.n_inputs * self.batch
         if torch.is_tensor(in_ptr):
-            ok = bool((in_ptr[0] == 0) & (in_ptr[1:] >= in_ptr[:-1]).all() & (in_ptr[-1] == in_events.numel()))
-            if in_events.numel():
-                ok = ok and bool((in_events.min() >= 0) & (in_events.max() < self.n_inputs * self.batch))
-            if not ok or in_ptr.dtype != torch.int64 or in_events.dtype != torch.int32:
+            if (not torch.is_tensor(in_events) or in_ptr.dtype != torch.int64 or in_events.dtype != torch.int32
+                    or in_ptr.dim() != 1 or in_events.dim() != 1 or not in_ptr.numel()):
                 raise ValueError("device input event lists are inconsistent")
             in_ptr, in_events = in_ptr.contiguous(), in_events.contiguous()
+            look = True
         else:
             in_ptr = np.ascontiguousarray(in_ptr, np.int64)
             in_events = np.ascontiguousarray(in_events, np.int32)
-            net.check_input_events(in_ptr, in_events, self.n_inputs * self.batch)
+            look = net.check_input_events(in_ptr, in_events, n_ids)
             in_ptr = torch.as_tensor(in_ptr, device=self.dev)
             in_events = torch.as_tensor(in_events, device=self.dev)
-        repeat = None
-        if in_events.numel() > 1:
-            step_start = torch.zeros(in_events.numel() + 1, dtype=torch.bool, device=in_events.device)
-            step_start[in_ptr] = True                      # an event that opens a step may be smaller than the last
-            d = in_events[1:] - in_events[:-1]
-            inside = ~step_start[1:-1]
-            if bool(((d < 0) & inside).any()):
-                raise ValueError("input events must be ascending within every step")
-            repeat = (d == 0) & inside                     # event k+1 repeats event k of the same step
-            if not bool(repeat.any()):
-                repeat = None
+        repeated = self._look_over_events(in_ptr, in_events, n_ids) if look else None
         self.in_ptr = in_ptr
         self.in_events = in_events if in_events.numel() else in_events.new_zeros(1)
         self.in_steps = in_ptr.numel() - 1
         self._lists_replaced = self.step > 0
-        self.in_duplicates = repeat is not None
-        self.in_repeat_ptr = self.in_repeat_events = None
-        if repeat is not None and (self.pull_inp_table is not None or self.fuse_table is not None):
-            where = repeat.nonzero().flatten() + 1         # positions of the second and later occurrences
-            self.in_repeat_events = in_events[where].contiguous()
-            self.in_repeat_ptr = torch.searchsorted(where, in_ptr).to(torch.int64).contiguous()
+        self.in_duplicates = repeated is not None
+        self.in_repeat_ptr, self.in_repeat_events = repeated or (None, None)
+
+    def _look_over_events(self, in_ptr, in_events, n_ids):
+        """ValueError for lists that are not what they should be; the running sum of the repeated ids of a step and these ids
+        (both None where no form at hand asks for them), or None where no id is repeated."""
+        ptr, events = in_ptr.to(self.dev), in_events.to(self.dev)
+        steps = ptr.numel() - 1
+        found = torch.zeros(steps + 2, dtype=torch.int32, device=self.dev)     # ... and behind the two words what each step repeats
+        repeats = found[2:]
+        _lib.check(self.lib.bmtk_events_check(steps, _p(ptr), events.numel(), _p(events), n_ids, _p(repeats), _p(found), _stream()))
+        bad, count = found[:2].tolist()
+        if bad & _lib.EVENTS_INCONSISTENT:
+            raise ValueError("device input event lists are inconsistent")
+        if bad:
+            raise ValueError("input events must be ascending within every step")
+        if not count:
+            return None
+        if self.pull_inp_table is None and self.fuse_table is None:
+            return None, None
+        first = torch.zeros(steps + 1, dtype=torch.int64, device=self.dev)
+        torch.cumsum(repeats, 0, out=first[1:])
+        again = torch.empty(count, dtype=torch.int32, device=self.dev)
+        _lib.check(self.lib.bmtk_events_repeated(steps, _p(ptr), _p(events), _p(first), _p(again), _stream()))
+        return first, again
 
     def _struct(self, bits=None, record=None):
         s = _lib.Glif3Sim()

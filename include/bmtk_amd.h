@@ -499,6 +499,19 @@ int bmtk_csr_receptors_used(int64_t nnz, const int32_t *indices, const uint8_t *
  * receptor have, workgroups of `span` neurons, takes the lower 24 bits, the delay the upper eight.  NULL: four planes a neuron. */
 int bmtk_csr_pack_cells(int64_t nnz, int32_t span, const uint32_t *cells, bmtk_synapse *packed, void *stream);
 
+/* Looks over per-step event lists (in_events[in_ptr[t] .. in_ptr[t + 1]) are the ids of step t; in_ptr has n_steps + 1 entries)
+ * before anything else reads them: found[0] |= BMTK_EVENTS_INCONSISTENT where in_ptr does not ascend from 0 to n_events or an id
+ * lies outside 0 .. n_ids - 1, BMTK_EVENTS_UNORDERED where ids of a step descend; repeats[t] = how many ids of step t equal the
+ * one before them, found[1] += their number in all.  The caller clears the two words of found. */
+#define BMTK_EVENTS_INCONSISTENT 1
+#define BMTK_EVENTS_UNORDERED 2
+int bmtk_events_check(int64_t n_steps, const int64_t *in_ptr, int64_t n_events, const int32_t *in_events, int64_t n_ids, int32_t *repeats,
+                      uint32_t *found, void *stream);
+
+/* Those repeated ids, of lists without fault: step t's into to[first[t] .. first[t + 1]), first being the running sum of repeats
+ * (n_steps + 1 entries, 0 first). */
+int bmtk_events_repeated(int64_t n_steps, const int64_t *in_ptr, const int32_t *in_events, const int64_t *first, int32_t *to, void *stream);
+
 /* The input events of the steps step0 .. step0 + n_steps - 1 (step0 may be -1: a step without events) apart by trial.  With
  * `counts` ([batch][n_steps]) the events of every trial and step are counted; with `first` ([batch][n_steps], the running
  * sums of those counts, exclusive) and `sources` their sources are written, in no particular order within a trial and step.

@@ -1,0 +1,72 @@
+"""Input event lists looked over on the device: what is refused, and the repeated ids listed apart."""
+import numpy as np
+import pytest
+
+from bmtk_amd import synthetic
+from bmtk_amd.simulator import Glif3Simulator
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def sim():
+    cfg = synthetic.small_glif3_network(n=100, n_in=400, steps=10, seed=1)
+    return Glif3Simulator(cfg["n"], cfg["par"], cfg["h"], batch=8, rec=cfg["rec_src"], inp=cfg["inp_src"], class_id=cfg["class_id"],
+                          resident=False, fused=True)
+
+
+def _lists(counts, seed, repeats):
+    rng = np.random.default_rng(seed)
+    by_step = [np.sort(rng.choice(3200, c, replace=False)) for c in counts]
+    for ids in by_step if repeats else ():
+        if ids.size > 1:
+            where = np.unique(np.concatenate([rng.integers(1, ids.size, 3), [ids.size - 1], [k for k in (1, 63, 64, 65, 255, 256, 257) if k < ids.size]]))
+            for k in where:
+                ids[k] = ids[k - 1]
+    return np.concatenate([[0], np.cumsum(counts)]).astype(np.int64), np.concatenate(by_step + [np.zeros(0)]).astype(np.int32)
+
+
+@pytest.mark.parametrize("counts", [[0], [], [1], [2, 0, 0, 1], [63, 64, 65, 0, 255, 256, 257, 1, 2], [0] * 500 + [1000, 3, 2900], [1] * 40000])
+@pytest.mark.parametrize("repeats", [False, True])
+@pytest.mark.parametrize("device", [False, True])
+def test_repeated_ids_are_listed_apart(sim, counts, repeats, device):
+    import torch
+    ptr, events = _lists(counts, len(counts), repeats)
+    again = np.concatenate([[False], events[1:] == events[:-1]])[:events.size]
+    again[ptr[:-1][np.diff(ptr) > 0]] = False
+    sim.set_input_events(*((torch.as_tensor(ptr, device="cuda"), torch.as_tensor(events, device="cuda")) if device else (ptr, events)))
+    assert sim.in_duplicates == bool(again.any())
+    if again.any():
+        np.testing.assert_array_equal(sim.in_repeat_events.cpu().numpy(), events[again])
+        np.testing.assert_array_equal(sim.in_repeat_ptr.cpu().numpy(), np.concatenate([[0], np.cumsum(again)])[ptr])
+    else:
+        assert sim.in_repeat_ptr is None and sim.in_repeat_events is None
+
+
+def test_lists_with_faults_are_refused(sim):
+    import torch
+    ptr, events = _lists([3, 0, 70, 300], 5, True)
+
+    def device(p, e):
+        return torch.as_tensor(p, device="cuda"), torch.as_tensor(e, device="cuda")
+    sim.set_input_events(*device(ptr, events))
+    kept = sim.in_ptr
+    for at, value in ((0, 1), (1, 4), (2, -1), (4, 372), (4, 374), (3, 1 << 40)):
+        p = ptr.copy()
+        p[at] = value
+        with pytest.raises(ValueError, match="inconsistent" if at != 1 else "inconsistent|ascending"):
+            sim.set_input_events(*device(p, events))
+    for at, value in ((0, -1), (372, 3200), (100, -5)):
+        e = events.copy()
+        e[at] = value
+        with pytest.raises(ValueError, match="inconsistent"):
+            sim.set_input_events(*device(ptr, e))
+    for at in (2, 72, 73 + 64, 372):     # the last of a step, one behind 64 others
+        e = events.copy()
+        e[at] = e[at - 1] - 1
+        with pytest.raises(ValueError, match="ascending"):
+            sim.set_input_events(*device(ptr, e))
+    for p, e in ((ptr.astype(np.int32), events), (ptr, events.astype(np.int64)), (ptr[:0], events), (ptr[:, None], events)):
+        with pytest.raises(ValueError, match="inconsistent"):
+            sim.set_input_events(*device(p, e))
+    assert sim.in_ptr is kept
