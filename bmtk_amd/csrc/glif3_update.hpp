@@ -118,28 +118,31 @@ __device__ __forceinline__ bool glif3_update(Glif3Elem &s, const Glif3Prop &p, f
     return spike;
 }
 
-// The same step, operation for operation, for a wavefront that runs many steps on end: lanes choose between results instead of
+// The same step, operation for operation, in two parts, for kernels that run many steps on end.  What the step after waits for is who
+// fired; the other half of the step can be done where the wavefront waits for memory.  Lanes choose between results instead of
 // taking branches (which cost some ten scalar instructions each, and keep independent arithmetic apart).
-// *fired: the ballot of the lanes with ``own`` that spiked; *frac is set in those only.
-__device__ __forceinline__ void glif3_update_wave(Glif3Elem &s, const Glif3Prop &p, float h, const float syn[GLIF3_NREC],
-                                                  float I, bool own, unsigned long long *fired, float *frac)
+__device__ __forceinline__ float glif3_potential(const Glif3Elem &s, const Glif3Prop &p, float I)
 {
-    const float v_old = s.V;
-    const bool held = s.ref > 0, leaves = s.ref == 1;
     float S = 0.0f;
 #pragma unroll
     for (int a = 0; a < GLIF3_NASC; ++a) S = S + p.c[a] * s.asc[a];
-    float U = v_old * p.P33 + (I + S) * p.P30;
+    float U = s.V * p.P33 + (I + S) * p.P30;
 #pragma unroll
     for (int k = 0; k < GLIF3_NREC; ++k) U = U + (p.P31[k] * s.y1[k] + p.P32[k] * s.y2[k]);
-    const float U_free = U;
-    const bool spike = own && !held && U > p.th;
+    return U;
+}
+
+__device__ __forceinline__ bool glif3_fires(const Glif3Elem &s, const Glif3Prop &p, float U) { return s.ref <= 0 && U > p.th; }
+
+__device__ __forceinline__ void glif3_finish(Glif3Elem &s, const Glif3Prop &p, float h, const float syn[GLIF3_NREC], float U, bool spike)
+{
+    const bool held = s.ref > 0, leaves = s.ref == 1;
 #pragma unroll
     for (int a = 0; a < GLIF3_NASC; ++a) {
         const float reset = p.amp[a] + s.asc[a] * p.r[a], decayed = s.asc[a] * p.d[a];
         s.asc[a] = leaves ? reset : held ? s.asc[a] : decayed;
     }
-    s.V = leaves ? p.Ur : held ? v_old : U;
+    s.V = leaves ? p.Ur : held ? s.V : U;
     s.ref = spike ? p.n_ref : held ? s.ref - 1 : s.ref;
 #pragma unroll
     for (int k = 0; k < GLIF3_NREC; ++k) {
@@ -148,8 +151,17 @@ __device__ __forceinline__ void glif3_update_wave(Glif3Elem &s, const Glif3Prop 
         s.y2[k] = P21 * a1 + p.P11[k] * a2;
         s.y1[k] = a1 * p.P11[k] + syn[k] * p.psc0[k];
     }
+}
+
+// Both parts.  *fired: the ballot of the lanes with ``own`` that spiked; *frac is set in those only.
+__device__ __forceinline__ void glif3_update_wave(Glif3Elem &s, const Glif3Prop &p, float h, const float syn[GLIF3_NREC],
+                                                  float I, bool own, unsigned long long *fired, float *frac)
+{
+    const float v_old = s.V, U = glif3_potential(s, p, I);
+    const bool spike = own && glif3_fires(s, p, U);
+    glif3_finish(s, p, h, syn, U, spike);
     *fired = __ballot(spike);
-    if (*fired != 0ull) *frac = (p.th - v_old) / (U_free - v_old);
+    if (*fired != 0ull) *frac = (p.th - v_old) / (U - v_old);
 }
 
 __device__ __forceinline__ void glif3_load(Glif3Elem &s, const float *V, const float *asc, const float *y1,
