@@ -40,7 +40,7 @@ class Glif3Sim(C.Structure):
         ("rb_seg", c_void_p), ("rb_packed", c_void_p), ("rb_ring", c_void_p), ("rb_hist", c_void_p),
         ("rb_in_ptr", c_void_p), ("rb_in_events", c_void_p), ("rb_pend_until", c_int64),
         ("rb_save_v", c_void_p), ("rb_save_flags", c_void_p),
-        ("rb_cells", c_void_p), ("rb_extra", c_int32), ("_pad4", c_int32), ("sum_shift", c_int32), ("_pad3", c_int32),
+        ("rb_cells", c_void_p), ("rb_extra", c_int32), ("rb_whole", c_int32), ("sum_shift", c_int32), ("_pad3", c_int32),
         ("spike_bits", c_void_p), ("spike_bits_stride", c_int64),
         ("save_v", c_void_p), ("save_flags", c_void_p),
         ("probe_col", c_void_p), ("probe_v", c_void_p), ("probe_stride", c_int64), ("probe_every", c_int32),
@@ -68,7 +68,7 @@ class Glif3Bwd(C.Structure):
 
 
 EVENTS_INCONSISTENT = 1     # BMTK_EVENTS_INCONSISTENT
-ABI_VERSION = 31  # BMTK_AMD_ABI_VERSION of include/bmtk_amd.h that the mirrors above were written for
+ABI_VERSION = 32  # BMTK_AMD_ABI_VERSION of include/bmtk_amd.h that the mirrors above were written for
 
 # name -> (restype, argtypes); every symbol include/bmtk_amd.h declares
 SIGNATURES = {

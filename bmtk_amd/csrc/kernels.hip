@@ -317,7 +317,7 @@ __global__ __launch_bounds__(kBlock) void events_check_kernel(int64_t n_steps, c
     const int lane = lane_id();
     const int64_t wave = (int64_t)blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave, n_waves = (int64_t)gridDim.x * (kBlock / kWave);
     constexpr int kTogether = 4;
-    unsigned bad = 0u, total = 0u;
+    unsigned bad = 0u, total = 0u, most = 0u;
     if (wave == 0 && (in_ptr[0] != 0 || in_ptr[n_steps] != n_events)) bad = BMTK_EVENTS_INCONSISTENT;
     for (int64_t t = wave; t < n_steps; t += n_waves) {
         const int64_t p0 = in_ptr[t], p1 = in_ptr[t + 1];
@@ -343,9 +343,13 @@ __global__ __launch_bounds__(kBlock) void events_check_kernel(int64_t n_steps, c
             }
         if (lane == 0) repeats[t] = (int32_t)again;
         total += again;
+        most = max(most, again);
     }
     if (bad) atomicOr(found, bad);
-    if (lane == 0 && total) atomicAdd(found + 1, total);
+    if (lane == 0 && total) {
+        atomicAdd(found + 1, total);
+        atomicMax(found + 2, most);
+    }
 }
 
 // The second and later occurrences of an id in its step, in order: those of step t from to[first[t]] on.

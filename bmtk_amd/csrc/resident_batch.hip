@@ -42,6 +42,8 @@
 #include <math.h>
 #include <stdlib.h>
 
+#include <type_traits>
+
 #include "fired_lists.hpp"
 #include "glif3_update.hpp"
 #include "pull_common.hpp"
@@ -65,7 +67,8 @@ struct RbLaunch {
     int slots;            // of the ring slice: ring_slots - 1
     int words;            // ballot words of a trial
     int has_events;
-    double unit;          // of the fixed-point sums
+    double unit;          // of the sums
+    int down;             // whole numbers: bits that a kept sum is shifted by (Kept)
 };
 
 __device__ __forceinline__ unsigned rb_load(const unsigned *p)
@@ -88,13 +91,16 @@ struct __attribute__((packed, aligned(4))) RbBounds {
 
 // kPer: neurons per thread; with two, the threads of the reader own none.  Sum: what the ring holds, 64-bit fixed point
 // (from_fixed), or floats where a workgroup's neurons are too many for that (batch 1): fp32 atomics into device memory are what
-// it then takes the place of.  kAllSums: every neuron has all four sums, in planes (no rb_cells); at 1,000 neurons and less to a
+// it then takes the place of, or 32-bit whole numbers where every weight is a whole multiple of one power of two and all that
+// reaches a neuron in a step stays below 2^31 of it (rb_whole): the same sums, bit for bit, in half the room, which is what decides how
+// many trials share a launch (230,924 x 8, 100 steps: 5.38 -> 3.40 ms; 10,000 x 8, 200 steps in one launch either way: 0.74 -> 0.59).  kAllSums: every neuron has all four sums, in planes (no rb_cells); at 1,000 neurons and less to a
 // workgroup the fold's selections cost 0.1 us a step, so that few sums are for where they save launches.  kSave: potentials and step flags of every step go to rb_save_*, trial by trial; by_step_kernel
 // puts them in their order.  kReaderOwns: spans above 960 with a neuron to a thread.
 template <int kPer, typename Sum, bool kAllSums, bool kSave, bool kReaderOwns>
 __global__ __launch_bounds__(kRbBlock) void sim_resident_batch_kernel(bmtk_glif3_sim s, RbLaunch q)
 {
-    constexpr bool kFixed = sizeof(Sum) == 8;
+    constexpr bool kFixed = sizeof(Sum) == 8, kWhole = std::is_same<Sum, unsigned>::value;
+    using Kept = typename std::conditional<std::is_same<Sum, float>::value, float, unsigned long long>::type;   // of rb_ring
     constexpr int kTogether = kPer > 1 ? 4 : kRbTogether;
     constexpr int kOwners = kRbReader * kWave;  // with two neurons to a thread: threads that own tid, tid + kOwners
     extern __shared__ unsigned long long rb_lds[];  // ring slice [slots][cells], then rb_list words for rows
@@ -142,7 +148,19 @@ __global__ __launch_bounds__(kRbBlock) void sim_resident_batch_kernel(bmtk_glif3
 
     // the arrivals that the call before left; some slots' are asked for together, before the state takes the registers
     auto cell_of = [&](unsigned word, int r, int at) __attribute__((always_inline)) { return kAllSums ? r * span + at : rb_cell(word, r, at, span); };
-    Sum *const ring_g = reinterpret_cast<Sum *>(s.rb_ring) + (int64_t)trial * S * GLIF3_NREC * n + e0;  // (all receptors' planes)
+    auto from_kept = [&](Kept v) __attribute__((always_inline)) -> Sum {
+        if constexpr (kWhole)
+            return (Sum)((long long)v >> q.down);
+        else
+            return v;
+    };
+    auto to_kept = [&](Sum v) __attribute__((always_inline)) -> Kept {
+        if constexpr (kWhole)
+            return (Kept)((long long)(int)v << q.down);
+        else
+            return v;
+    };
+    Kept *const ring_g = reinterpret_cast<Kept *>(s.rb_ring) + (int64_t)trial * S * GLIF3_NREC * n + e0;  // (all receptors' planes)
     unsigned sums[kPer]{};  // a neuron's word of rb_cells
 #pragma unroll
     for (int u = 0; u < kPer; ++u)
@@ -155,14 +173,14 @@ __global__ __launch_bounds__(kRbBlock) void sim_resident_batch_kernel(bmtk_glif3
         if (!owns(u)) continue;
 #pragma unroll 1
         for (int k = 0; k < S; k += kSlots) {
-            Sum v[kSlots * GLIF3_NREC];
+            Kept v[kSlots * GLIF3_NREC];
 #pragma unroll
             for (int j = 0; j < kSlots * GLIF3_NREC; ++j)
                 if (k + j / GLIF3_NREC < S && (sums[u] >> j % GLIF3_NREC & 1u)) v[j] = ring_g[((int64_t)k * GLIF3_NREC + j) * n + place(u)];
 #pragma unroll
             for (int j = 0; j < kSlots * GLIF3_NREC; ++j)
                 if (k + j / GLIF3_NREC < S && (sums[u] >> j % GLIF3_NREC & 1u))
-                    ring_l[(k + j / GLIF3_NREC) * cells + cell_of(sums[u], j % GLIF3_NREC, place(u))] = v[j];
+                    ring_l[(k + j / GLIF3_NREC) * cells + cell_of(sums[u], j % GLIF3_NREC, place(u))] = from_kept(v[j]);
         }
     }
     Glif3Elem st[kPer]{};
@@ -193,6 +211,8 @@ __global__ __launch_bounds__(kRbBlock) void sim_resident_batch_kernel(bmtk_glif3
                 row[cell] = (Sum)0;
                 if constexpr (kFixed)
                     return from_fixed(v, q.unit);
+                else if constexpr (kWhole)
+                    return (float)(int)v * (float)q.unit;
                 else
                     return v;
             };
@@ -326,6 +346,8 @@ __global__ __launch_bounds__(kRbBlock) void sim_resident_batch_kernel(bmtk_glif3
             Sum *cell = ring_l + mad_u24(min(dq + q_lo, dq + q_wrap), (unsigned)cells, sy.x & 0xFFFFFFu);
             if constexpr (kFixed)
                 atomicAdd(cell, to_fixed(__uint_as_float(sy.y)));
+            else if constexpr (kWhole)
+                atomicAdd(cell, sy.y);
             else if (!crowded)
                 atomicAdd(cell, __uint_as_float(sy.y));
             else {
@@ -545,7 +567,7 @@ __global__ __launch_bounds__(kRbBlock) void sim_resident_batch_kernel(bmtk_glif3
         for (int k = 0; k < S; ++k)
 #pragma unroll
             for (int r = 0; r < GLIF3_NREC; ++r)
-                if (word >> r & 1u) ring_g[(int64_t)(k * GLIF3_NREC + r) * n + place(u)] = ring_l[k * cells + cell_of(word, r, place(u))];
+                if (word >> r & 1u) ring_g[(int64_t)(k * GLIF3_NREC + r) * n + place(u)] = to_kept(ring_l[k * cells + cell_of(word, r, place(u))]);
     }
 }
 
@@ -614,8 +636,12 @@ int simulate_resident_batch(const bmtk_glif3_sim &s, int64_t step0, int64_t n_st
     BMTK_REQUIRE(span >= kWave && span % kWave == 0 && span <= 2 * kRbReader * kWave && G == (n + span - 1) / span,
                  "glif3_simulate_fwd: rb_span must be a multiple of 64 up to 1920 and rb_groups ceil(n_neurons / rb_span)");
     BMTK_REQUIRE(wide || batch > 1, "glif3_simulate_fwd: a single trial is resident in spans above 1024 here, in shorter ones by res_span");
-    BMTK_REQUIRE(s.rb_cells ? batch > 1 && s.rb_extra >= 0 && s.rb_extra <= 2 * span : s.rb_extra == 2 * span && (batch == 1 || !wide),
-                 "glif3_simulate_fwd: rb_extra must lie in 0..2 * rb_span with rb_cells (batches; spans above 1024 need it) and be 2 * rb_span without");
+    BMTK_REQUIRE(s.rb_cells ? batch > 1 && s.rb_extra >= 0 && s.rb_extra <= 2 * span : s.rb_extra == 2 * span && (batch == 1 || !wide || s.rb_whole),
+                 "glif3_simulate_fwd: rb_extra must lie in 0..2 * rb_span with rb_cells (batches; spans above 1024 need it or rb_whole) and be 2 * rb_span without");
+    BMTK_REQUIRE(s.sum_shift >= 0 && s.sum_shift <= BMTK_SUM_SHIFT_MAX, "glif3_simulate_fwd: sum_shift must lie in 0..BMTK_SUM_SHIFT_MAX");
+    const bool whole = s.rb_whole != 0;
+    BMTK_REQUIRE(s.rb_whole >= 0 && s.rb_whole <= 33 + s.sum_shift && !(whole && (batch == 1 || s.rb_cells)),
+                 "glif3_simulate_fwd: rb_whole must lie in 0..33 + sum_shift and is for batches without rb_cells");
     BMTK_REQUIRE(W >= 1 && W <= batch && s.rb_team_shift >= 0 && s.rb_team_shift <= 6 && s.rb_list >= kWave,
                  "glif3_simulate_fwd: rb_ways must lie in 1..batch, rb_team_shift in 0..6, rb_list from 64 on");
     BMTK_REQUIRE(s.rb_seg && s.rb_packed && s.rb_ring && s.rb_hist && s.res_sync, "glif3_simulate_fwd: resident trials need rb_* and res_sync");
@@ -624,10 +650,9 @@ int simulate_resident_batch(const bmtk_glif3_sim &s, int64_t step0, int64_t n_st
     BMTK_REQUIRE(!s.probe_col && !s.spike_count, "glif3_simulate_fwd: resident trials take no probes and keep no spike record");
     BMTK_REQUIRE(!save || (batch > 1 && s.rb_save_v && s.rb_save_flags && n_steps <= 65535),
                  "glif3_simulate_fwd: resident trials keep the per-step record of batches, up to 65535 steps a call, with rb_save_v and rb_save_flags");
-    BMTK_REQUIRE(s.sum_shift >= 0 && s.sum_shift <= BMTK_SUM_SHIFT_MAX, "glif3_simulate_fwd: sum_shift must lie in 0..BMTK_SUM_SHIFT_MAX");
     BMTK_REQUIRE((s.rb_in_ptr == nullptr) == (s.rb_in_events == nullptr), "glif3_simulate_fwd: rb_in_ptr and rb_in_events go together");
     BMTK_REQUIRE(n_steps < (1ll << 30) && n + s.n_inputs < (1ll << 24), "glif3_simulate_fwd: too many steps or sources for resident trials");
-    const size_t lds = (size_t)S * (2 * span + s.rb_extra) * (batch == 1 ? sizeof(float) : sizeof(unsigned long long)) + (size_t)s.rb_list * sizeof(unsigned);
+    const size_t lds = (size_t)S * (2 * span + s.rb_extra) * (batch == 1 || whole ? sizeof(float) : sizeof(unsigned long long)) + (size_t)s.rb_list * sizeof(unsigned);
     BMTK_REQUIRE(lds + 256u <= kResLdsBytes, "glif3_simulate_fwd: the ring slice of resident trials does not fit in LDS");
     RbLaunch q{};
     q.step0 = step0;
@@ -635,7 +660,8 @@ int simulate_resident_batch(const bmtk_glif3_sim &s, int64_t step0, int64_t n_st
     q.slots = S;
     q.words = (int)((n + kWave - 1) / kWave);
     q.has_events = s.rb_in_ptr != nullptr;
-    q.unit = ldexp(1.0, -32 - s.sum_shift);
+    q.unit = ldexp(1.0, whole ? 1 - s.rb_whole : -32 - s.sum_shift);
+    q.down = whole ? 33 + s.sum_shift - s.rb_whole : 0;
     BMTK_REQUIRE((wide ? 2 * kRbReader * kWave : kRbBlock) * (int64_t)kListGroups >= n, "glif3_simulate_fwd: more neurons than resident trials can hold");
     using Fixed = unsigned long long;
     auto address = [](auto *k) { return reinterpret_cast<const void *>(k); };
@@ -645,7 +671,13 @@ int simulate_resident_batch(const bmtk_glif3_sim &s, int64_t step0, int64_t n_st
          {address(sim_resident_batch_kernel<1, Fixed, true, true, false>), address(sim_resident_batch_kernel<1, Fixed, true, true, true>)}},
         {{address(sim_resident_batch_kernel<1, Fixed, false, false, false>), address(sim_resident_batch_kernel<1, Fixed, false, false, true>)},
          {address(sim_resident_batch_kernel<1, Fixed, false, true, false>), address(sim_resident_batch_kernel<1, Fixed, false, true, true>)}}};
-    const void *kernel = batch == 1 ? address(sim_resident_batch_kernel<2, float, true, false, false>)
+    const void *const whole_kernels[2][2] = {  // record, neurons of the reader's
+        {address(sim_resident_batch_kernel<1, unsigned, true, false, false>), address(sim_resident_batch_kernel<1, unsigned, true, false, true>)},
+        {address(sim_resident_batch_kernel<1, unsigned, true, true, false>), address(sim_resident_batch_kernel<1, unsigned, true, true, true>)}};
+    const void *kernel = whole && !wide ? whole_kernels[save][owns]
+                         : whole        ? (save ? address(sim_resident_batch_kernel<2, unsigned, true, true, false>)
+                                                : address(sim_resident_batch_kernel<2, unsigned, true, false, false>))
+                         : batch == 1   ? address(sim_resident_batch_kernel<2, float, true, false, false>)
                          : !wide    ? kernels[few][save][owns]
                          : save     ? address(sim_resident_batch_kernel<2, Fixed, false, true, false>)
                                     : address(sim_resident_batch_kernel<2, Fixed, false, false, false>);

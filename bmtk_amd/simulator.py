@@ -59,6 +59,11 @@ SOLO_LDS_PER_ELEMENT = 4 * 4
 SOLO_LDS_EXTRA = 10240 + 2048
 RB_WIDE_SPAN = 1920             # neurons of a workgroup at most with two to a thread
 RB_TWO_COST = 1.35              # a step of resident trials with two neurons to a thread against one (51,978 x 32: 1.40, 20,011 x 20: 1.3)
+# ... with sums as 32-bit whole numbers (230,924 x 8: 1.27).  They take less time in as many launches too, no conversion of each weight
+# among other things: 200 steps with sums of 64 / 32 bits 5,000 x 16 630 / 614 us, 10,000 x 8 742 / 594, 31,000 x 8 1,091 / 902, 2,000 x 40 620 / 593, 60,000 x 4
+# 1,163 / 975, 4,000 x 64 1,030 / 878; two to a thread 51,978 x 32 5,484 / 4,901, 20,011 x 20 1,212 / 1,060, 100,000 x 4 2,406 / 2,020, 31,000 x 64
+# 6,239 / 5,363; in half the launches 230,924 x 8 5,376 / 3,401 (100 steps), 120,000 x 16 12,264 / 9,702
+RB_TWO_COST_WHOLE = 1.22
 RB_LIST_MIN, RB_LDS_STATIC = 2000, 256   # the form with resident trials: least room (words) for its lists of rows, static LDS
 SUM_SHIFT_MAX = 120             # BMTK_SUM_SHIFT_MAX
 TRIALS_TABLE_BYTES = 1 << 30    # tables and ring of the form with resident trials at most, or TRIALS_TABLE_RATIO times the synapses' 10 bytes
@@ -99,13 +104,14 @@ def lists_pay(span, groups, rate_hz, h_ms=1.0):
     return fired + math.sqrt(2.0 * fired * math.log(max(2, groups))) <= LIST_MAX
 
 
-def resident_trials_plan(n_neurons, batch, ring_slots, n_cu, third=None):
+def resident_trials_plan(n_neurons, batch, ring_slots, n_cu, third=None, sum_bytes=8):
     """How the trials of a batch share ``n_cu`` compute units when each keeps its state in registers and its arrivals of
     the next ring_slots - 1 steps in LDS: dict(span, groups, ways, passes, list, few) -- ``ways`` trials side by side on
     ``groups`` workgroups of ``span`` neurons each, ``passes`` launches, ``list`` places in the list of rows -- or None
     where a single trial does not fit.  ``third``: how many third and fourth receptors the neurons before the i-th use
     (n_neurons + 1 numbers; receptors that no synapse of a neuron ends on have no sums), or None where every neuron is to have all four.
-    One trial: only where the network is too large for the resident mode, and with four sums in fp32.
+    One trial: only where the network is too large for the resident mode, and with four sums in fp32.  ``sum_bytes`` 4: sums as 32-bit
+    whole numbers (``whole_numbers``), four to a neuron.
 
     A step costs much the same whatever runs beside it: as few launches as possible, if need be with sums only for what is in use
     (``few``) and two neurons to a thread (spans above 1024), which take RB_TWO_COST times as long a step."""
@@ -119,7 +125,7 @@ def resident_trials_plan(n_neurons, batch, ring_slots, n_cu, third=None):
         if few:
             first = np.arange(0, n_neurons, span)
             extra = int((third[np.minimum(first + span, n_neurons)] - third[first]).max())
-        return (RES_LDS_BYTES - RB_LDS_STATIC - slots * (2 * span + extra) * (4 if batch == 1 else 8)) // 4
+        return (RES_LDS_BYTES - RB_LDS_STATIC - slots * (2 * span + extra) * (4 if batch == 1 else sum_bytes)) // 4
 
     def plan(span, ways, passes, few=False):
         return dict(span=span, groups=-(-n_neurons // span), ways=ways, passes=passes, list=min(RES_ACT_ENTRIES, places(span, few)), few=few)
@@ -130,7 +136,9 @@ def resident_trials_plan(n_neurons, batch, ring_slots, n_cu, third=None):
         return plan(span, 1, 1) if 1024 < span <= RB_WIDE_SPAN and places(span) >= RB_LIST_MIN else None
     best, best_cost = None, None
     # (of equals the first: few sums cost 0.1 us a step to tell apart)
-    for few, most, cost in ((False, 1024, 1.0), (True, 1024, 1.05), (True, RB_WIDE_SPAN, RB_TWO_COST))[:1 if third is None else 3]:
+    kinds = (((False, 1024, 1.0), (False, RB_WIDE_SPAN, RB_TWO_COST_WHOLE)) if sum_bytes == 4 else
+             ((False, 1024, 1.0), (True, 1024, 1.05), (True, RB_WIDE_SPAN, RB_TWO_COST))[:1 if third is None else 3])
+    for few, most, cost in kinds:
         most = next((span for span in range(most, 0, -64) if places(span, few) >= RB_LIST_MIN), 0)
         if not most or -(-n_neurons // most) > cus:
             continue
@@ -142,6 +150,24 @@ def resident_trials_plan(n_neurons, batch, ring_slots, n_cu, third=None):
         if best is None or passes * cost < best_cost:
             best, best_cost = plan(span, ways, passes, few), passes * cost
     return best
+
+
+def _lowest_place(size):
+    """The lowest power of two that some set bit of these numbers (fp32, none negative) stands for, 0 if that is above 1."""
+    lowest = 0
+    for w in size.split(1 << 26):
+        bits = w.contiguous().view(torch.int32)
+        exponent, mantissa = bits >> 23, bits & 0x7FFFFF
+        mantissa = torch.where(exponent > 0, mantissa | 0x800000, mantissa)
+        low_bit = ((mantissa & -mantissa).to(torch.float32).view(torch.int32) >> 23) - 127
+        place = torch.where(mantissa != 0, exponent.clamp(min=1) - 150 + low_bit, torch.zeros_like(low_bit))
+        lowest = min(lowest, int(place.min()))
+    return lowest
+
+
+def plan_cost(plan):
+    """What the launches of a plan come to, in steps with a neuron to a thread."""
+    return plan["passes"] * (1.0 if plan["span"] <= 1024 else RB_TWO_COST if plan.get("few") else RB_TWO_COST_WHOLE)
 
 
 def fixed_point_shift(tables, n_neurons):
@@ -158,14 +184,8 @@ def fixed_point_shift(tables, n_neurons):
             return None
         sizes.append(largest)
         # (from 2^-9 on every number's bits lie above 2^-33)
-        for w in size.split(1 << 26) if least < 2.0 ** -9 else ():
-            # the power of two that a weight's lowest set bit stands for
-            bits = w.contiguous().view(torch.int32)
-            exponent, mantissa = bits >> 23, bits & 0x7FFFFF
-            mantissa = torch.where(exponent > 0, mantissa | 0x800000, mantissa)
-            low_bit = ((mantissa & -mantissa).to(torch.float32).view(torch.int32) >> 23) - 127
-            place = torch.where(mantissa != 0, exponent.clamp(min=1) - 150 + low_bit, torch.zeros_like(low_bit))
-            lowest = min(lowest, int(place.min()))
+        if least < 2.0 ** -9:
+            lowest = min(lowest, _lowest_place(size))
     shift = max(0, -32 - lowest)
     if shift > SUM_SHIFT_MAX:
         return None
@@ -175,6 +195,23 @@ def fixed_point_shift(tables, n_neurons):
             and sum(size * int(torch.bincount(t.indices, minlength=n_neurons).max()) for size, t in zip(sizes, tables)) >= limit):
         return None
     return shift
+
+
+def whole_numbers(rec, inp, n_neurons, slots):
+    """Whether the sums of arrivals fit 32-bit whole numbers of a power of two that every weight is a multiple of: (k, most repeated
+    input events of a step) for multiples of 2^-k pA, or None.  All synapses of a neuron at once may come to half of what 32 bits hold,
+    the other half is for input ids repeated within a step, which ``slots`` steps may bring to one sum."""
+    tables = [t for t in (rec, inp) if t is not None and t.nnz]
+    sizes = [t.weights.abs() for t in tables]
+    if not all(bool(torch.isfinite(size).all()) for size in sizes):
+        return None
+    k = -min([_lowest_place(size) for size in sizes], default=0)
+    reach = [torch.bincount(t.indices, weights=size.double(), minlength=n_neurons) for t, size in zip(tables, sizes)]
+    most = float(sum(reach).max()) if reach else 0.0
+    of_inputs = float(reach[-1].max()) if inp is not None and inp.nnz else 0.0
+    if k > 30 or most * 2.0 ** k > 2.0 ** 30:
+        return None
+    return k, int(2.0 ** 30 / max(1.0, of_inputs * 2.0 ** k * slots))
 
 
 def fused_pays(n_neurons, batch, n_synapses, class_table, rate_hz, h_ms=1.0):
@@ -211,8 +248,8 @@ def trials_pay(plan, n_neurons, batch, n_synapses, class_table, rate_hz, h_ms, f
     the driver that would run otherwise, the fused pull form (``fused``) or pushed events."""
     per_trial = n_neurons * float(rate_hz) * 1e-3 * h_ms
     events = n_synapses * batch * float(rate_hz) * 1e-3 * h_ms
-    step = (TRIALS_PS_PER_PASS + TRIALS_PS_PER_ROW * per_trial) * (RB_TWO_COST if batch > 1 and plan["span"] > 1024 else 1.0)
-    trials = plan["passes"] * step + TRIALS_PS_PER_EVENT * events
+    step = TRIALS_PS_PER_PASS + TRIALS_PS_PER_ROW * per_trial
+    trials = (plan_cost(plan) if batch > 1 else plan["passes"]) * step + TRIALS_PS_PER_EVENT * events
     if fused:
         other = (FUSE_PS_PER_STEP + FUSE_PS_PER_SYNAPSE * n_synapses + FUSE_PS_PER_EVENT * events
                  + FUSE_PS_PER_ELEMENT * n_neurons * batch)
@@ -380,6 +417,7 @@ class Glif3Simulator:
         self.in_ptr = self.in_events = None
         self.in_steps = 0
         self.in_duplicates = False
+        self.in_most_repeats = 0    # of a step
         self._lists_replaced = False    # since the last run
         self.in_repeat_ptr = self.in_repeat_events = None   # repeated ids of a step, for the pull form of the inputs
         self.step = 0
@@ -482,6 +520,12 @@ class Glif3Simulator:
                 third = torch.zeros(self.n + 1, dtype=torch.int64, device=self.dev)
                 torch.cumsum(self._third_and_fourth(used), 0, out=third[1:])
                 plan = resident_trials_plan(self.n, self.batch, self.L, n_cu, third.cpu().numpy())
+            # 32-bit sums where the weights allow them: 3 to 25 % faster in as many launches (see RB_TWO_COST_WHOLE)
+            small = resident_trials_plan(self.n, self.batch, self.L, n_cu, None, 4) if self.batch > 1 else None
+            if small and (plan is None or plan_cost(small) <= plan_cost(plan)):
+                whole = whole_numbers(self.rec, self.inp, self.n, self.L - 1)
+                if whole:
+                    plan = dict(small, whole=whole[0] + 1, room=whole[1])
         if plan and ((self.n + self.n_inputs) * (plan["groups"] + 1) >= 2 ** 32 or self.n + self.n_inputs >= 2 ** 24
                      or n_syn >= 2 ** 31 or self.pull_table is not None):
             plan = None
@@ -543,7 +587,10 @@ class Glif3Simulator:
             own += at                                   # (fewer than 2^31 synapses)
             packed[at:at + t.nnz] = t.packed()[:t.nnz]
             row, at = row + t.n_rows, at + t.nnz
-        if self.sum_shift:
+        tr["whole"] = 0 if tr.get("few") else tr.get("whole", 0)
+        if tr["whole"]:
+            packed[:, 1] = (packed.view(torch.float32)[:, 1] * 2.0 ** (tr["whole"] - 1)).to(torch.int32)
+        elif self.sum_shift:
             packed.view(torch.float32)[:, 1] *= 2.0 ** self.sum_shift
         cells, extra = None, 2 * tr["span"]
         if tr.get("few"):           # where a neuron's third sum stands among its workgroup's
@@ -571,7 +618,7 @@ class Glif3Simulator:
         rows = max(1.0, self.n * self.expected_rate_hz * 1e-3 * self.h + events)
         s.rb_team_shift = max(0, min(tr["max_team_shift"], int(math.log2(max(1.0, 900.0 / rows)))))
         s.rb_late_events = 1 if self.fuse_rereads else 0
-        s.rb_cells, s.rb_extra = _p(tr["cells"]), tr["extra"]
+        s.rb_cells, s.rb_extra, s.rb_whole = _p(tr["cells"]), tr["extra"], tr["whole"]
         s.rb_seg, s.rb_packed, s.rb_ring, s.rb_hist = _p(tr["seg"]), _p(tr["packed"]), _p(tr["ring"]), _p(tr["hist"])
         s.res_sync, s.res_spin_limit = _p(self.res_sync), int(self.spin_limit)
         if self.inp is None or self.in_ptr is None:
@@ -810,36 +857,34 @@ class Glif3Simulator:
             look = net.check_input_events(in_ptr, in_events, n_ids)
             in_ptr = torch.as_tensor(in_ptr, device=self.dev)
             in_events = torch.as_tensor(in_events, device=self.dev)
-        repeated = self._look_over_events(in_ptr, in_events, n_ids) if look else None
+        most, repeated = self._look_over_events(in_ptr, in_events, n_ids) if look else (0, None)
         self.in_ptr = in_ptr
         self.in_events = in_events if in_events.numel() else in_events.new_zeros(1)
         self.in_steps = in_ptr.numel() - 1
         self._lists_replaced = self.step > 0
-        self.in_duplicates = repeated is not None
+        self.in_duplicates, self.in_most_repeats = most > 0, most
         self.in_repeat_ptr, self.in_repeat_events = repeated or (None, None)
 
     def _look_over_events(self, in_ptr, in_events, n_ids):
-        """ValueError for lists that are not what they should be; the running sum of the repeated ids of a step and these ids
-        (both None where no form at hand asks for them), or None where no id is repeated."""
+        """ValueError for lists that are not what they should be; the most repeated ids of a step, and the running sum of their numbers
+        with the ids themselves where a form at hand asks for them, or None."""
         ptr, events = in_ptr.to(self.dev), in_events.to(self.dev)
         steps = ptr.numel() - 1
-        found = torch.zeros(steps + 2, dtype=torch.int32, device=self.dev)     # ... and behind the two words what each step repeats
-        repeats = found[2:]
+        found = torch.zeros(steps + 3, dtype=torch.int32, device=self.dev)     # ... and behind the three words what each step repeats
+        repeats = found[3:]
         _lib.check(self.lib.bmtk_events_check(steps, _p(ptr), events.numel(), _p(events), n_ids, _p(repeats), _p(found), _stream()))
-        bad, count = found[:2].tolist()
+        bad, count, most = found[:3].tolist()
         if bad & _lib.EVENTS_INCONSISTENT:
             raise ValueError("device input event lists are inconsistent")
         if bad:
             raise ValueError("input events must be ascending within every step")
-        if not count:
-            return None
-        if self.pull_inp_table is None and self.fuse_table is None:
-            return None, None
+        if not count or (self.pull_inp_table is None and self.fuse_table is None):
+            return most, None
         first = torch.zeros(steps + 1, dtype=torch.int64, device=self.dev)
         torch.cumsum(repeats, 0, out=first[1:])
         again = torch.empty(count, dtype=torch.int32, device=self.dev)
         _lib.check(self.lib.bmtk_events_repeated(steps, _p(ptr), _p(events), _p(first), _p(again), _stream()))
-        return first, again
+        return most, (first, again)
 
     def _struct(self, bits=None, record=None):
         s = _lib.Glif3Sim()
@@ -956,7 +1001,8 @@ class Glif3Simulator:
                           count=torch.zeros(1 if ways == 1 else ways * _lib.RECORD_COUNT_STRIDE, dtype=torch.int64,
                                             device=self.dev), ways=ways)
         use_trials = (self._trials is not None and n_steps >= TRIALS_MIN_STEPS and record is None
-                      and self.probe_col is None and not torch.cuda.is_current_stream_capturing())
+                      and self.probe_col is None and not torch.cuda.is_current_stream_capturing()
+                      and self.in_most_repeats <= self._trials.get("room", self.in_most_repeats))
         stretch = n_steps
         if use_trials and save_state:
             stretch = min(65535, TRIALS_SAVE_BYTES // (5 * self.ne))

@@ -49,7 +49,7 @@ extern "C" {
 
 /* Bumped whenever a struct layout or a signature below changes; bmtk_amd_abi_version() returns the value the
  * library was built with. */
-#define BMTK_AMD_ABI_VERSION 31
+#define BMTK_AMD_ABI_VERSION 32
 int bmtk_amd_abi_version(void);
 const char *bmtk_amd_last_error(void);
 /* sizeof(bmtk_glif3_sim) as the library was compiled, for bindings that mirror the struct */
@@ -393,7 +393,7 @@ typedef struct bmtk_glif3_sim {
     int32_t rb_ways;                   /* trials of a launch: rb_ways * rb_groups workgroups must be resident at once */
     int32_t rb_team_shift;             /* 2^rb_team_shift lanes read a row's segment */
     int32_t rb_list;                   /* words of LDS for the rows of two steps, at least 64 (a step with more than (rb_list - 64) / 2
-                                        * rows takes longer); (ring_slots-1)*8*(2*rb_span + rb_extra) (one trial: *4)
+                                        * rows takes longer); (ring_slots-1)*8*(2*rb_span + rb_extra) (one trial, or rb_whole: *4)
                                         * + 4*rb_list + 256 bytes of LDS */
     int32_t rb_late_events;            /* the input events of a call's last step (each id once; repeats are delivered at once) are
                                         * left to the next call and its lists, as with in_again */
@@ -411,9 +411,11 @@ typedef struct bmtk_glif3_sim {
     const uint32_t *rb_cells;          /* batches: [n_neurons], bits 0..3 the receptors that some synapse ends on
                                         * (bmtk_csr_receptors_used).  Only those have sums in LDS: the first two of every neuron in
                                         * planes of rb_span, third and fourth behind these; from bit 4 on, where the neuron's third
-                                        * stands among its workgroup's.  NULL (one trial; spans up to 1024): four planes */
+                                        * stands among its workgroup's.  NULL (one trial; spans up to 1024; rb_whole): four planes */
     int32_t rb_extra;                  /* third and fourth sums of a workgroup's neurons at most; without rb_cells 2 * rb_span */
-    int32_t _pad4;
+    int32_t rb_whole;                  /* batches without rb_cells; 0, or k + 1: the weight field of rb_packed holds a 32-bit whole number of 2^-k pA
+                                        * (exactly), and so do the sums in LDS: what may reach a receptor of a neuron in a step must
+                                        * stay below 2^31 of them.  rb_ring keeps its 64 bits and unit.  Half the LDS a sum */
     /* Fixed-point sums of the fused and the resident form: their tables (fuse_packed, rb_packed) hold the weights times
      * 2^sum_shift, and a sum's lowest bit (rb_ring's too) stands for 2^-(32 + sum_shift).  A weight is held exactly when that
      * divides it, otherwise cut off towards zero; what may reach a neuron in a step must stay below 2^(31 - sum_shift). */
@@ -502,7 +504,7 @@ int bmtk_csr_pack_cells(int64_t nnz, int32_t span, const uint32_t *cells, bmtk_s
 /* Looks over per-step event lists (in_events[in_ptr[t] .. in_ptr[t + 1]) are the ids of step t; in_ptr has n_steps + 1 entries)
  * before anything else reads them: found[0] |= BMTK_EVENTS_INCONSISTENT where in_ptr does not ascend from 0 to n_events or an id
  * lies outside 0 .. n_ids - 1, BMTK_EVENTS_UNORDERED where ids of a step descend; repeats[t] = how many ids of step t equal the
- * one before them, found[1] += their number in all.  The caller clears the two words of found. */
+ * one before them, found[1] += their number in all, found[2] = the most of a step.  The caller clears the three words of found. */
 #define BMTK_EVENTS_INCONSISTENT 1
 #define BMTK_EVENTS_UNORDERED 2
 int bmtk_events_check(int64_t n_steps, const int64_t *in_ptr, int64_t n_events, const int32_t *in_events, int64_t n_ids, int32_t *repeats,

@@ -453,3 +453,79 @@ def test_the_backward_pass_refuses_the_record_of_a_run_that_gave_up(stepwise):
     assert float(bptt.d_rec_w.abs().max()) == 0.0
     backward(sim.run(40, save_state=True), dl_dz_const=dl_dz)
     assert int(sim.res_sync[1].item()) == 0 and bool(torch.isfinite(bptt.d_rec_w).all())
+
+
+@pytest.mark.parametrize("whole", [True, False])
+@pytest.mark.parametrize("n,batch,max_delay,classes,span", [
+    (64, 64, 4, 3, None), (700, 20, 5, 7, None), (1025, 33, 1, None, 1024), (1025, 5, 5, 7, 1088), (1921, 12, 4, None, 1920), (4100, 8, 6, 5, 1408)])
+def test_sums_of_32_and_of_64_bits(monkeypatch, n, batch, max_delay, classes, span, whole):
+    """Weights in quarters of a pA: sums as 32-bit whole numbers of them, or in 64 bits where the weights are taken not to allow that.  One
+    neuron to a thread and two, the per-step record, arrivals under way between calls and to the driver that takes its place."""
+    cfg, _, _ = _case(n, batch, max_delay, classes, steps=200)
+    if not whole:
+        monkeypatch.setattr(simulator, "whole_numbers", lambda *a: None)
+    st = orc.new_state(n, batch, np.float32)
+    raster = orc.simulate(st, orc.precompute(cfg["par"], 1.0), 1.0, 200, batch=batch, class_id=cfg["class_id"],
+                          ring=np.zeros((cfg["L"], 4, n * batch), np.float32), rec=cfg["rec_src"], inp=cfg["inp_src"],
+                          in_ptr=cfg["in_ptr"], in_events=cfg["in_events"], i_ext=cfg["i_ext"], raster=True)["raster"]
+    sim = _sim(cfg, batch, resident_trials=True, fused=batch >= 8)
+    assert sim._trials.get("whole", 0) == (3 if whole else 0)      # multiples of 2^-2
+    if span:
+        sim._trials.update(span=span, groups=-(-n // span), ways=min(batch, 256 // -(-n // span)), list=400, few=not whole and span > 1024)
+    outs = [sim.run(50), sim.run(60), sim.run(70, save_state=True)]
+    assert sim._trials is not None
+    outs.append(sim.run(20))
+    assert sim._trials is None
+    _same(sim, outs, raster, st)
+
+
+def test_weights_that_32_bit_sums_take():
+    n = 50
+    rng = np.random.default_rng(1)
+
+    def table(w, rows=n):
+        return ops.SynapseTable.from_edges(rng.integers(0, rows, w.size), rng.integers(0, n, w.size), w.astype(np.float32),
+                                           np.ones(w.size, np.int64), np.zeros(w.size, np.int64), rows, n)
+    quarters = np.round(rng.normal(0, 20, 400)) / 4
+    rec, inp = table(quarters), table(np.full(100, 2.0), 10)
+    k, room = simulator.whole_numbers(rec, inp, n, 5)
+    most = np.bincount(inp.indices.cpu().numpy(), minlength=n).max() * 2.0
+    assert k == 2 and room == int(2.0 ** 30 / (most * 4 * 5))
+    assert simulator.whole_numbers(rec, None, n, 5)[0] == 2 and simulator.whole_numbers(table(np.zeros(3)), None, n, 1)[0] == 0
+    assert simulator.whole_numbers(table(np.array([2.0 ** -30])), None, n, 1)[0] == 30
+    for bad in ([2.0 ** -31], [np.nan], [np.inf, 1.0], [2.0 ** 31], [2.0 ** 20, 2.0 ** -11], np.full(100000, 2.0 ** 21)):
+        assert simulator.whole_numbers(rec, table(np.array(bad)), n, 5) is None
+        assert simulator.whole_numbers(table(np.array(bad)), inp, n, 5) is None
+    # sums as large as they may come out as they are: every synapse of a neuron at once, either sign
+    for sign in (1.0, -1.0):
+        w = np.full(3, sign * 2.0 ** 28)
+        src, tgt = np.arange(3), np.zeros(3, np.int64)
+        one = ops.SynapseTable.from_edges(src, tgt, w.astype(np.float32), np.ones(3, np.int64), np.zeros(3, np.int64), 4, 4)
+        tabs = tuple(t.cpu().numpy() for t in (one.indptr, one.indices, one.weights, one.delays, one.receptors))
+        par = synthetic.random_cells(np.random.default_rng(2), 4)
+        got = {}
+        for trials in (True, False):
+            sim = Glif3Simulator(4, par, 1.0, batch=2, rec=table_of(4), inp=tabs, resident=False, resident_trials=trials)
+            assert not trials or sim._trials["whole"] == 1
+            sim.set_input_events(np.concatenate([[0], np.full(40, 3)]).astype(np.int64), np.arange(3, dtype=np.int32) * 2)
+            sim.run(40)
+            sim.check()
+            got[trials] = sim.state.to_numpy()
+        for key in STATE:
+            np.testing.assert_array_equal(got[True][key], got[False][key], err_msg=key)
+
+
+def table_of(n):
+    """A recurrent table of one synapse that carries nothing."""
+    return (np.array([0] + [1] * n, np.int32), np.array([n - 1], np.int32), np.zeros(1, np.float32), np.ones(1, np.uint8), np.zeros(1, np.uint8))
+
+
+def test_more_repeated_events_than_32_bit_sums_take():
+    """A step that repeats an id more often than there is room for: the other driver runs, whatever the sums come to."""
+    cfg, raster, st = _case(300, 8, 3)
+    sim = _sim(cfg, 8, resident_trials=True, fused=True)
+    assert 0 < sim.in_most_repeats <= sim._trials["room"]
+    sim._trials["room"] = sim.in_most_repeats - 1
+    outs = [sim.run(60), sim.run(90)]
+    assert sim._trials is None
+    _same(sim, outs, raster, st)
