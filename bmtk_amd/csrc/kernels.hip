@@ -307,6 +307,33 @@ __global__ __launch_bounds__(kBlock) void compact_write_fused_kernel(const uint6
     }
 }
 
+// What 32-bit sums of arrivals have to know of a table's weights, in one pass: the lowest power of two that a set bit of some weight
+// stands for, the largest size (both reduced per wavefront first), and how much could reach each target at once, in multiples of 2^-10
+// rounded up.  Bounded by the additions, 47 ps each: 2.9 ms for 62 M synapses, where a count in doubles and ten array operations took 9.
+__global__ __launch_bounds__(kBlock) void weight_reach_kernel(int64_t nnz, const int32_t *__restrict__ indices, const float *__restrict__ weights,
+                                                              unsigned long long *__restrict__ reach, int32_t *__restrict__ found)
+{
+    int lowest = 0, largest = 0;
+    for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < nnz; i += (int64_t)gridDim.x * kBlock) {
+        const unsigned bits = __float_as_uint(weights[i]) & 0x7FFFFFFFu, exponent = bits >> 23;
+        const unsigned mantissa = (bits & 0x7FFFFFu) | (exponent ? 0x800000u : 0u);
+        largest = max(largest, (int)bits);
+        if (mantissa == 0u) continue;
+        lowest = min(lowest, (int)max(exponent, 1u) - 150 + __ffs((int)mantissa) - 1);
+        // (sizes of 2^30 and more, infinities and NaN are told by found[1])
+        if (bits < 0x4E800000u) atomicAdd(reach + indices[i], (unsigned long long)ceilf(__uint_as_float(bits) * 1024.0f));
+    }
+#pragma unroll
+    for (int step = kWave / 2; step > 0; step >>= 1) {
+        lowest = min(lowest, __shfl_xor(lowest, step, kWave));
+        largest = max(largest, __shfl_xor(largest, step, kWave));
+    }
+    if (lane_id() == 0) {
+        atomicMin(found, lowest);
+        atomicMax(found + 1, largest);
+    }
+}
+
 // Input event lists looked over, a wavefront per step.  Bounded by launches and the one look at `found` that follows: the same in
 // array operations (marks at every step's start, differences, comparisons, reductions, four of them waited for) took 270 us a
 // call, 350 with repeats to list, beside runs of 1.5 to 2.3 ms; this takes 55, and 105 with repeats.
@@ -634,6 +661,17 @@ int bmtk_spikes_compact_bits(const uint64_t *zbits, int64_t n, int32_t *ids, int
     BMTK_REQUIRE(zbits && ids && count && workspace, "spikes_compact_bits: pointers must be non-null");
     uint32_t *block_count = (uint32_t *)((uint64_t *)workspace + n_words_of(n) + 1);
     return compact_from_bits(zbits, n, ids, count, block_count, (hipStream_t)stream);
+}
+
+int bmtk_csr_weight_reach(int64_t nnz, const int32_t *indices, const float *weights, uint64_t *reach, int32_t *found, void *stream)
+{
+    BMTK_REQUIRE(nnz >= 0 && found && reach && (nnz == 0 || (indices && weights)), "csr_weight_reach: bad sizes or null pointers");
+    if (nnz == 0) return BMTK_OK;
+    const int64_t blocks = (nnz + kBlock - 1) / kBlock;
+    hipLaunchKernelGGL(weight_reach_kernel, dim3((unsigned)(blocks < 4096 ? blocks : 4096)), dim3(kBlock), 0, (hipStream_t)stream, nnz, indices,
+                       weights, reinterpret_cast<unsigned long long *>(reach), found);
+    BMTK_CHECK_LAUNCH("csr_weight_reach");
+    return BMTK_OK;
 }
 
 int bmtk_events_check(int64_t n_steps, const int64_t *in_ptr, int64_t n_events, const int32_t *in_events, int64_t n_ids, int32_t *repeats,

@@ -152,19 +152,6 @@ def resident_trials_plan(n_neurons, batch, ring_slots, n_cu, third=None, sum_byt
     return best
 
 
-def _lowest_place(size):
-    """The lowest power of two that some set bit of these numbers (fp32, none negative) stands for, 0 if that is above 1."""
-    lowest = 0
-    for w in size.split(1 << 26):
-        bits = w.contiguous().view(torch.int32)
-        exponent, mantissa = bits >> 23, bits & 0x7FFFFF
-        mantissa = torch.where(exponent > 0, mantissa | 0x800000, mantissa)
-        low_bit = ((mantissa & -mantissa).to(torch.float32).view(torch.int32) >> 23) - 127
-        place = torch.where(mantissa != 0, exponent.clamp(min=1) - 150 + low_bit, torch.zeros_like(low_bit))
-        lowest = min(lowest, int(place.min()))
-    return lowest
-
-
 def plan_cost(plan):
     """What the launches of a plan come to, in steps with a neuron to a thread."""
     return plan["passes"] * (1.0 if plan["span"] <= 1024 else RB_TWO_COST if plan.get("few") else RB_TWO_COST_WHOLE)
@@ -184,8 +171,14 @@ def fixed_point_shift(tables, n_neurons):
             return None
         sizes.append(largest)
         # (from 2^-9 on every number's bits lie above 2^-33)
-        if least < 2.0 ** -9:
-            lowest = min(lowest, _lowest_place(size))
+        for w in size.split(1 << 26) if least < 2.0 ** -9 else ():
+            # the power of two that a weight's lowest set bit stands for
+            bits = w.contiguous().view(torch.int32)
+            exponent, mantissa = bits >> 23, bits & 0x7FFFFF
+            mantissa = torch.where(exponent > 0, mantissa | 0x800000, mantissa)
+            low_bit = ((mantissa & -mantissa).to(torch.float32).view(torch.int32) >> 23) - 127
+            place = torch.where(mantissa != 0, exponent.clamp(min=1) - 150 + low_bit, torch.zeros_like(low_bit))
+            lowest = min(lowest, int(place.min()))
     shift = max(0, -32 - lowest)
     if shift > SUM_SHIFT_MAX:
         return None
@@ -201,15 +194,19 @@ def whole_numbers(rec, inp, n_neurons, slots):
     """Whether the sums of arrivals fit 32-bit whole numbers of a power of two that every weight is a multiple of: (k, most repeated
     input events of a step) for multiples of 2^-k pA, or None.  All synapses of a neuron at once may come to half of what 32 bits hold,
     the other half is for input ids repeated within a step, which ``slots`` steps may bring to one sum."""
-    tables = [t for t in (rec, inp) if t is not None and t.nnz]
-    sizes = [t.weights.abs() for t in tables]
-    if not all(bool(torch.isfinite(size).all()) for size in sizes):
-        return None
-    k = -min([_lowest_place(size) for size in sizes], default=0)
-    reach = [torch.bincount(t.indices, weights=size.double(), minlength=n_neurons) for t, size in zip(tables, sizes)]
-    most = float(sum(reach).max()) if reach else 0.0
-    of_inputs = float(reach[-1].max()) if inp is not None and inp.nnz else 0.0
-    if k > 30 or most * 2.0 ** k > 2.0 ** 30:
+    lib, tables = _lib.load(), [t for t in (inp, rec) if t is not None and t.nnz]
+    if not tables:
+        return 0, 1 << 30
+    dev = tables[0].weights.device
+    reach, found = torch.zeros(n_neurons, dtype=torch.int64, device=dev), torch.zeros(2, dtype=torch.int32, device=dev)
+    of_inputs = torch.zeros(1, device=dev)
+    for t in tables:      # (the inputs first, so that what they come to is known by itself)
+        _lib.check(lib.bmtk_csr_weight_reach(t.nnz, _p(t.indices), _p(t.weights), _p(reach), _p(found), _stream()))
+        if t is inp:
+            of_inputs = reach.max()
+    (lowest, largest), of_inputs, most = found.tolist(), float(of_inputs.max()) / 1024.0, float(reach.max()) / 1024.0
+    k = -lowest
+    if largest >= 0x4E800000 or k > 30 or most * 2.0 ** k > 2.0 ** 30:      # (2^30 as a float's bits)
         return None
     return k, int(2.0 ** 30 / max(1.0, of_inputs * 2.0 ** k * slots))
 
@@ -515,17 +512,16 @@ class Glif3Simulator:
             n_cu = torch.cuda.get_device_properties(self.dev).multi_processor_count
             # (of a batch: what it takes at best, before the tables are looked at)
             plan = resident_trials_plan(self.n, self.batch, self.L, n_cu, np.zeros(self.n + 1, np.int64) if self.batch > 1 else None)
-            if plan and self.batch > 1:
+            # 32-bit sums where the weights allow them: 3 to 25 % faster in as many launches (see RB_TWO_COST_WHOLE)
+            small = resident_trials_plan(self.n, self.batch, self.L, n_cu, None, 4) if self.batch > 1 else None
+            whole = whole_numbers(self.rec, self.inp, self.n, self.L - 1) if small and (plan is None or plan_cost(small) <= plan_cost(plan)) else None
+            if whole:
+                plan = dict(small, whole=whole[0] + 1, room=whole[1])
+            elif plan and self.batch > 1:
                 used = self._receptors_used()
                 third = torch.zeros(self.n + 1, dtype=torch.int64, device=self.dev)
                 torch.cumsum(self._third_and_fourth(used), 0, out=third[1:])
                 plan = resident_trials_plan(self.n, self.batch, self.L, n_cu, third.cpu().numpy())
-            # 32-bit sums where the weights allow them: 3 to 25 % faster in as many launches (see RB_TWO_COST_WHOLE)
-            small = resident_trials_plan(self.n, self.batch, self.L, n_cu, None, 4) if self.batch > 1 else None
-            if small and (plan is None or plan_cost(small) <= plan_cost(plan)):
-                whole = whole_numbers(self.rec, self.inp, self.n, self.L - 1)
-                if whole:
-                    plan = dict(small, whole=whole[0] + 1, room=whole[1])
         if plan and ((self.n + self.n_inputs) * (plan["groups"] + 1) >= 2 ** 32 or self.n + self.n_inputs >= 2 ** 24
                      or n_syn >= 2 ** 31 or self.pull_table is not None):
             plan = None
@@ -594,6 +590,8 @@ class Glif3Simulator:
             packed.view(torch.float32)[:, 1] *= 2.0 ** self.sum_shift
         cells, extra = None, 2 * tr["span"]
         if tr.get("few"):           # where a neuron's third sum stands among its workgroup's
+            if tr["used"] is None:
+                tr["used"] = self._receptors_used()
             own = self._third_and_fourth(tr["used"])
             before = torch.cumsum(own, 0) - own
             begin = torch.arange(groups, device=self.dev) * tr["span"]

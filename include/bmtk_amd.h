@@ -501,6 +501,11 @@ int bmtk_csr_receptors_used(int64_t nnz, const int32_t *indices, const uint8_t *
  * receptor have, workgroups of `span` neurons, takes the lower 24 bits, the delay the upper eight.  NULL: four planes a neuron. */
 int bmtk_csr_pack_cells(int64_t nnz, int32_t span, const uint32_t *cells, bmtk_synapse *packed, void *stream);
 
+/* reach[target] += |weight| in multiples of 2^-10, each rounded up (weights of 2^30 and more, infinities and NaN left out), over the
+ * synapses of a table whose indices are targets; found[0] = the lowest power of two that a set bit of some weight stands for if that is lower,
+ * found[1] = the bits of the largest |weight| if that is larger.  The caller clears them. */
+int bmtk_csr_weight_reach(int64_t nnz, const int32_t *indices, const float *weights, uint64_t *reach, int32_t *found, void *stream);
+
 /* Looks over per-step event lists (in_events[in_ptr[t] .. in_ptr[t + 1]) are the ids of step t; in_ptr has n_steps + 1 entries)
  * before anything else reads them: found[0] |= BMTK_EVENTS_INCONSISTENT where in_ptr does not ascend from 0 to n_events or an id
  * lies outside 0 .. n_ids - 1, BMTK_EVENTS_UNORDERED where ids of a step descend; repeats[t] = how many ids of step t equal the
