@@ -189,9 +189,14 @@ class SynapseTable:
         dev = device or _dev()
         src = torch.as_tensor(np.ascontiguousarray(src) if not torch.is_tensor(src) else src, device=dev).long()
         tgt = torch.as_tensor(np.ascontiguousarray(tgt) if not torch.is_tensor(tgt) else tgt, device=dev).long()
-        if src.numel() and (int(src.min()) < 0 or int(src.max()) >= n_rows or int(tgt.min()) < 0
-                            or int(tgt.max()) >= n_cols):
+        d = torch.as_tensor(np.ascontiguousarray(d) if not torch.is_tensor(d) else d, device=dev)
+        looks = [d.max().long()] if d.numel() else [src.new_zeros(())]
+        if src.numel():
+            looks += [*torch.aminmax(src), *torch.aminmax(tgt)]
+        longest, *ends = torch.stack(looks).tolist()      # (one look at the device)
+        if ends and (ends[0] < 0 or ends[1] >= n_rows or ends[2] < 0 or ends[3] >= n_cols):
             raise ValueError("edge endpoints outside 0..{} / 0..{}".format(n_rows - 1, n_cols - 1))
+        wide = longest > 255
         order = torch.sort(src * n_cols + tgt, stable=True).indices
         counts = torch.bincount(src, minlength=n_rows)
         indptr = torch.zeros(n_rows + 1, dtype=torch.int32, device=dev)
@@ -201,8 +206,6 @@ class SynapseTable:
             a = torch.as_tensor(np.ascontiguousarray(a) if not torch.is_tensor(a) else a, device=dev)
             return a.to(dtype)[order].contiguous()
 
-        d = torch.as_tensor(np.ascontiguousarray(d) if not torch.is_tensor(d) else d, device=dev)
-        wide = bool(d.numel()) and int(d.max()) > 255
         return cls(indptr, tgt[order].to(torch.int32).contiguous(), col(w, torch.float32),
                    d.to(torch.int32 if wide else torch.uint8)[order].contiguous(), col(r, torch.uint8),
                    n_rows=n_rows, max_row=int(counts.max().item()) if counts.numel() else 0)
@@ -212,16 +215,21 @@ class SynapseTable:
         """Adopt device tensors after the same checks ``network.check_csr`` makes on the host."""
         indptr, indices, w, d, r = (t.contiguous() for t in csr)
         nnz = indices.numel()
-        ok = indptr.numel() == n_rows + 1 and int(indptr[0]) == 0 and int(indptr[-1]) == nnz
-        ok = ok and bool((indptr[1:] >= indptr[:-1]).all())
-        ok = ok and w.numel() == nnz and d.numel() == nnz and r.numel() == nnz
-        if ok and nnz:
-            ok = bool((indices.min() >= 0) & (indices.max() < n_cols) & (d.min() >= 1) & (d.max() < ring_slots)
-                      & (r.max() < NREC))
+        max_row, ok = 0, indptr.numel() == n_rows + 1 and w.numel() == nnz and d.numel() == nnz and r.numel() == nnz
+        if ok:
+            # (one look at the device)
+            fine = (indptr[0] == 0) & (indptr[-1] == nnz)
+            if nnz:
+                fine = fine & (indices.min() >= 0) & (indices.max() < n_cols) & (d.min() >= 1) & (d.max() < ring_slots) & (r.max() < NREC)
+            if n_rows:
+                least, most = torch.aminmax(indptr[1:] - indptr[:-1])
+                ok, least, max_row = torch.stack([fine.to(least.dtype), least, most]).tolist()
+                ok = bool(ok) and least >= 0
+            else:
+                ok = bool(fine)
         if not ok:
             raise ValueError("inconsistent synapse table (indptr, index range, delay range or receptor range)")
-        deg = indptr[1:] - indptr[:-1]
-        return cls(indptr, indices, w, d, r, n_rows=n_rows, max_row=int(deg.max()) if deg.numel() else 0)
+        return cls(indptr, indices, w, d, r, n_rows=n_rows, max_row=max_row)
 
     @property
     def nnz(self):

@@ -337,12 +337,12 @@ class Glif3Simulator:
             raise ValueError("par needs one column per neuron when class_id is not given")
         self.prop = glif3_precompute(par, h)
         self.class_id = None if class_id is None else torch.as_tensor(class_id, device=self.dev)
-        lo, hi = [], []
-        for t in (rec, inp):
-            if t is not None and len(t[3]):
-                lo.append(int(t[3].min()))
-                hi.append(int(t[3].max()))
-        min_delay, max_delay = (min(lo), max(hi)) if lo else (1, 1)
+        ends = [x for t in (rec, inp) if t is not None and len(t[3])
+                for x in (torch.aminmax(t[3]) if torch.is_tensor(t[3]) else (t[3].min(), t[3].max()))]
+        if ends and all(torch.is_tensor(x) for x in ends):
+            ends = torch.stack([x.long() for x in ends]).tolist()      # (one look at the device)
+        ends = [int(x) for x in ends]
+        min_delay, max_delay = (min(ends[::2]), max(ends[1::2])) if ends else (1, 1)
         if min_delay < 1:
             raise ValueError("delays must be at least one step")
         if delay_offset == "auto":
@@ -780,6 +780,13 @@ class Glif3Simulator:
                                      RES_LDS_EXTRA, RES_LDS_BYTES))
             return
         groups = -(-self.ne // span)
+        if groups == 1:
+            # (whole rows are read, in any order: their bounds are the row's)
+            for t in (self.rec, self.inp):
+                if t is not None:
+                    setattr(self, "rec_seg" if t is self.rec else "inp_seg", torch.stack([t.indptr[:-1], t.indptr[1:]], 1))
+            self.res_span, self.res_groups, self.res_fired = span, groups, None
+            return
         if self.rec is not None:
             self.rec = self.rec.sorted_by_index()
             self.rec_seg = self.rec.segment_offsets(span, groups)
@@ -803,7 +810,7 @@ class Glif3Simulator:
             self.res_unified = (packed, seg)
         self.res_span, self.res_groups = span, groups
         # asks for the exchange by lists of fired neurons (bmtk_glif3_sim.res_fired: that it is there is all that is looked at)
-        lists = groups > 1 and self.fired_lists and lists_pay(span, groups, self.expected_rate_hz, self.h)
+        lists = self.fired_lists and lists_pay(span, groups, self.expected_rate_hz, self.h)
         self.res_fired = torch.zeros(1, dtype=torch.int32, device=self.dev) if lists else None
 
     def check(self):

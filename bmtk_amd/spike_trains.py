@@ -377,21 +377,23 @@ def bin_spike_times(trains, dt, n_steps, batch=1, trial=0):
     ``static_synapse`` delivery) and is emitted in step stamp-1.  An event is
     the element id ``source*batch + trial``; events of one step are ascending.
     """
-    # all trains at once: a run script has a train per virtual cell, and three array operations on each cost 5 ms per thousand
+    # all trains at once: a run script has a train per virtual cell, and an array operation on each costs more than a millisecond
+    # per thousand
     trains = list(trains)
     used = [j for j, st in enumerate(trains) if st is not None and len(st)]
     try:
-        times = [np.asarray(trains[j], np.float64).ravel() for j in used]
-        bad = any(t.min() <= 0.0 for t in times if t.size) if used else False   # (a NaN is not)
+        times = [st if type(st) is np.ndarray and st.ndim == 1 else np.asarray(st, np.float64).ravel() for st in (trains[j] for j in used)]
+        times_all = np.concatenate(times).astype(np.float64, copy=False) if times else np.zeros(0)
+        bad = times_all.size and not times_all.min() > 0.0      # (a NaN is the least)
     except (TypeError, ValueError):
         bad = True
-    if bad or any(np.isnan(t).any() for t in times):
+    if bad:
         for st in trains:
             check_spike_times(st)       # raises for the first train that is not valid
         times = [np.asarray(trains[j], np.float64).ravel() for j in used]
-    times_all = np.concatenate(times) if times else np.zeros(0)
+        times_all = np.concatenate(times) if times else np.zeros(0)
     stamp = np.maximum(np.ceil(times_all / dt - 1e-6).astype(np.int64), 1)
-    elems = np.repeat(np.asarray(used, np.int64) * batch + trial, [t.size for t in times])
+    elems = np.repeat(np.asarray(used, np.int64) * batch + trial, [len(t) for t in times])
     steps = stamp - 1
     early = steps < n_steps
     steps, elems = steps[early], elems[early]

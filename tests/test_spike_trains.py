@@ -191,3 +191,17 @@ def test_binning_all_trains_at_once_equals_one_by_one(seed):
 def test_the_first_train_that_is_not_valid_is_named():
     with pytest.raises(ValueError, match=r"\[0\. 2\.\]"):
         bin_spike_times([[1.0], [0.0, 2.0], [-1.0]], 1.0, 5)
+
+
+def test_trains_of_every_form_are_binned_alike():
+    """Arrays of several types, lists, tuples, columns and reversed views among the trains: what each gives by itself."""
+    x = np.array([0.3, 2.0, 2.0, 7.5])
+    forms = [x, None, list(x), x.astype(np.float32), np.array([1, 4]), [], x[:, None], x[::-1], tuple(x), np.zeros(0), np.array([3], np.uint8)]
+    ptr, events = bin_spike_times(forms, 0.1, 60)
+    alone = [bin_spike_times([None] * j + [np.asarray(f, np.float64).ravel()], 0.1, 60) if f is not None else None for j, f in enumerate(forms)]
+    for t in range(60):
+        want = sorted(int(e) for a in alone if a is not None for e in a[1][a[0][t]:a[0][t + 1]])
+        assert events[ptr[t]:ptr[t + 1]].tolist() == want
+    for bad in ([0.0], np.array([1.0, -2.0]), [2.0, 0.0, np.nan], np.zeros(2, np.float32)):
+        with pytest.raises(ValueError, match="negative/zero"):
+            bin_spike_times([x, None, bad, x], 0.1, 60)
