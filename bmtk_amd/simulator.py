@@ -269,7 +269,8 @@ class Glif3Simulator:
                 compute unit, ring slice within LDS; True: insist on it (ValueError otherwise); False: one launch
                 per step, which takes any batch and size (``resident_trials`` then has to be asked for)
     single_workgroup  resident mode: a network of up to 1024 elements whose whole ring fits LDS runs in ONE
-                workgroup, without a grid barrier (about 1 us per step instead of 2.5); False keeps such a network
+                workgroup, without a grid barrier (about 1 us per step instead of 2.5, a third of that where no delay is below some ten
+                steps, which it then runs several of between two barriers); False keeps such a network
                 on the many-workgroup form
     fired_lists  resident mode with several workgroups: every workgroup publishes the neurons that fired in a step
                 as a short list whose words carry the step, and nobody waits at a grid barrier (neurons that a list does
@@ -305,7 +306,9 @@ class Glif3Simulator:
                 for more than spike bits and, of a batch, the per-step record (``record_cap``, probes; ``save_state`` of a single
                 trial or of so many elements that 32 steps of them outgrow TRIALS_SAVE_BYTES), covers fewer than TRIALS_MIN_STEPS
                 steps or is captured into a graph, and a look at ``ring``, ``work_bits`` or ``fuse_any``, make it go on with that
-                driver for good.  True: insist (ValueError otherwise); False: off.
+                driver for good.  True: insist (ValueError otherwise); False: off.  Sums of a batch's arrivals have 64 bits, or 32 where the
+                weights are whole multiples of one power of two that those hold exactly (``whole_numbers``); input lists that repeat
+                more ids in a step than these have room for make it go on with the other driver, too.
     delay_offset  B steps taken off every delay before the tables are built; spikes and input events are
                 then handed to the tables B steps late from a history of spike bits, which gives the same
                 arrivals with a ring B slots shorter.  "auto": 0 while the largest delay is at most 63
