@@ -339,7 +339,7 @@ __global__ __launch_bounds__(kBlock) void weight_reach_kernel(int64_t nnz, const
 // call, 350 with repeats to list, beside runs of 1.5 to 2.3 ms; this takes 55, and 105 with repeats.
 __global__ __launch_bounds__(kBlock) void events_check_kernel(int64_t n_steps, const int64_t *__restrict__ in_ptr, int64_t n_events,
                                                               const int32_t *__restrict__ in_events, int64_t n_ids, int32_t *__restrict__ repeats,
-                                                              unsigned *__restrict__ found)
+                                                              int32_t *__restrict__ longest, unsigned *__restrict__ found)
 {
     const int lane = lane_id();
     const int64_t wave = (int64_t)blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave, n_waves = (int64_t)gridDim.x * (kBlock / kWave);
@@ -348,7 +348,7 @@ __global__ __launch_bounds__(kBlock) void events_check_kernel(int64_t n_steps, c
     if (wave == 0 && (in_ptr[0] != 0 || in_ptr[n_steps] != n_events)) bad = BMTK_EVENTS_INCONSISTENT;
     for (int64_t t = wave; t < n_steps; t += n_waves) {
         const int64_t p0 = in_ptr[t], p1 = in_ptr[t + 1];
-        unsigned again = 0u;
+        unsigned again = 0u, run = 0u, of_one = 0u;   // run: repeats of one id on end up to here
         if (p0 < 0 || p1 < p0 || p1 > n_events)
             bad |= BMTK_EVENTS_INCONSISTENT;    // (nothing is read through them)
         else
@@ -365,12 +365,30 @@ __global__ __launch_bounds__(kBlock) void events_check_kernel(int64_t n_steps, c
                     const int64_t p = base + u * kWave + lane;
                     if (p < p1 && (id[u] < 0 || id[u] >= n_ids)) bad |= BMTK_EVENTS_INCONSISTENT;
                     if (p < p1 && id[u] < before[u]) bad |= BMTK_EVENTS_UNORDERED;
-                    again += (unsigned)__popcll(__ballot(p > p0 && p < p1 && id[u] == before[u]));
+                    unsigned long long same = __ballot(p > p0 && p < p1 && id[u] == before[u]);
+                    if (same == 0ull) {
+                        run = 0u;
+                        continue;
+                    }
+                    again += (unsigned)__popcll(same);
+                    if (same == ~0ull) {
+                        run += kWave;
+                        of_one = max(of_one, run);
+                        continue;
+                    }
+                    of_one = max(of_one, run + (unsigned)__ffsll((long long)~same) - 1u);
+                    run = (unsigned)__clzll((long long)~same);
+                    unsigned on_end = 0u;
+                    for (; same; same &= same << 1) ++on_end;
+                    of_one = max(of_one, on_end);
                 }
             }
-        if (lane == 0) repeats[t] = (int32_t)again;
+        if (lane == 0) {
+            repeats[t] = (int32_t)again;
+            longest[t] = (int32_t)of_one;
+        }
         total += again;
-        most = max(most, again);
+        most = max(most, of_one);
     }
     if (bad) atomicOr(found, bad);
     if (lane == 0 && total) {
@@ -675,13 +693,13 @@ int bmtk_csr_weight_reach(int64_t nnz, const int32_t *indices, const float *weig
 }
 
 int bmtk_events_check(int64_t n_steps, const int64_t *in_ptr, int64_t n_events, const int32_t *in_events, int64_t n_ids, int32_t *repeats,
-                      uint32_t *found, void *stream)
+                      int32_t *longest, uint32_t *found, void *stream)
 {
     BMTK_REQUIRE(n_steps >= 0 && n_events >= 0 && n_ids >= 0, "events_check: bad sizes");
-    BMTK_REQUIRE(in_ptr && (in_events || n_events == 0) && (repeats || n_steps == 0) && found, "events_check: pointers must be non-null");
+    BMTK_REQUIRE(in_ptr && (in_events || n_events == 0) && ((repeats && longest) || n_steps == 0) && found, "events_check: pointers must be non-null");
     const int64_t blocks = (n_steps + kBlock / kWave - 1) / (kBlock / kWave);
     hipLaunchKernelGGL(events_check_kernel, dim3((unsigned)(blocks < 1 ? 1 : blocks < 8192 ? blocks : 8192)), dim3(kBlock), 0, (hipStream_t)stream,
-                       n_steps, in_ptr, n_events, in_events, n_ids, repeats, found);
+                       n_steps, in_ptr, n_events, in_events, n_ids, repeats, longest, found);
     BMTK_CHECK_LAUNCH("events_check");
     return BMTK_OK;
 }

@@ -190,10 +190,11 @@ def fixed_point_shift(tables, n_neurons):
     return shift
 
 
-def whole_numbers(rec, inp, n_neurons, slots):
-    """Whether the sums of arrivals fit 32-bit whole numbers of a power of two that every weight is a multiple of: (k, most repeated
-    input events of a step) for multiples of 2^-k pA, or None.  All synapses of a neuron at once may come to half of what 32 bits hold,
-    the other half is for input ids repeated within a step, which ``slots`` steps may bring to one sum."""
+def whole_numbers(rec, inp, n_neurons):
+    """Whether the sums of arrivals fit 32-bit whole numbers of a power of two that every weight is a multiple of: (k, how often a step may
+    repeat an input id) for multiples of 2^-k pA, or None.  A synapse has one delay, so what it brings to a sum comes from the
+    events of one step: all synapses of a neuron once, and those of the inputs once more for every time that a step may repeat their id, have
+    to come to less than half of what 32 bits hold (the other half is for arrivals under way where ``step`` is set back)."""
     lib, tables = _lib.load(), [t for t in (inp, rec) if t is not None and t.nnz]
     if not tables:
         return 0, 1 << 30
@@ -206,9 +207,10 @@ def whole_numbers(rec, inp, n_neurons, slots):
             of_inputs = reach.max()
     (lowest, largest), of_inputs, most = found.tolist(), float(of_inputs.max()) / 1024.0, float(reach.max()) / 1024.0
     k = -lowest
-    if largest >= 0x4E800000 or k > 30 or most * 2.0 ** k > 2.0 ** 30:      # (2^30 as a float's bits)
+    left = 2.0 ** 30 - most * 2.0 ** k
+    if largest >= 0x4E800000 or k > 30 or left <= 0.0:      # (2^30 as a float's bits)
         return None
-    return k, int(2.0 ** 30 / max(1.0, of_inputs * 2.0 ** k * slots))
+    return k, math.ceil(left / max(1.0, of_inputs * 2.0 ** k)) - 1
 
 
 def fused_pays(n_neurons, batch, n_synapses, class_table, rate_hz, h_ms=1.0):
@@ -308,7 +310,7 @@ class Glif3Simulator:
                 steps or is captured into a graph, and a look at ``ring``, ``work_bits`` or ``fuse_any``, make it go on with that
                 driver for good.  True: insist (ValueError otherwise); False: off.  Sums of a batch's arrivals have 64 bits, or 32 where the
                 weights are whole multiples of one power of two that those hold exactly (``whole_numbers``); input lists that repeat
-                more ids in a step than these have room for make it go on with the other driver, too.
+                an id in a step more often than these have room for make it go on with the other driver, too.
     delay_offset  B steps taken off every delay before the tables are built; spikes and input events are
                 then handed to the tables B steps late from a history of spike bits, which gives the same
                 arrivals with a ring B slots shorter.  "auto": 0 while the largest delay is at most 63
@@ -417,7 +419,7 @@ class Glif3Simulator:
         self.in_ptr = self.in_events = None
         self.in_steps = 0
         self.in_duplicates = False
-        self.in_most_repeats = 0    # of a step
+        self.in_most_repeats = 0    # of one id, of any step
         self._lists_replaced = False    # since the last run
         self.in_repeat_ptr = self.in_repeat_events = None   # repeated ids of a step, for the pull form of the inputs
         self.step = 0
@@ -517,7 +519,7 @@ class Glif3Simulator:
             plan = resident_trials_plan(self.n, self.batch, self.L, n_cu, np.zeros(self.n + 1, np.int64) if self.batch > 1 else None)
             # 32-bit sums where the weights allow them: 3 to 25 % faster in as many launches (see RB_TWO_COST_WHOLE)
             small = resident_trials_plan(self.n, self.batch, self.L, n_cu, None, 4) if self.batch > 1 else None
-            whole = whole_numbers(self.rec, self.inp, self.n, self.L - 1) if small and (plan is None or plan_cost(small) <= plan_cost(plan)) else None
+            whole = whole_numbers(self.rec, self.inp, self.n) if small and (plan is None or plan_cost(small) <= plan_cost(plan)) else None
             if whole:
                 plan = dict(small, whole=whole[0] + 1, room=whole[1])
             elif plan and self.batch > 1:
@@ -874,13 +876,13 @@ class Glif3Simulator:
         self.in_repeat_ptr, self.in_repeat_events = repeated or (None, None)
 
     def _look_over_events(self, in_ptr, in_events, n_ids):
-        """ValueError for lists that are not what they should be; the most repeated ids of a step, and the running sum of their numbers
-        with the ids themselves where a form at hand asks for them, or None."""
+        """ValueError for lists that are not what they should be; how often a step repeats an id at most, and the running sum of the repeats
+        of the steps with the ids themselves where a form at hand asks for them, or None."""
         ptr, events = in_ptr.to(self.dev), in_events.to(self.dev)
         steps = ptr.numel() - 1
-        found = torch.zeros(steps + 3, dtype=torch.int32, device=self.dev)     # ... and behind the three words what each step repeats
-        repeats = found[3:]
-        _lib.check(self.lib.bmtk_events_check(steps, _p(ptr), events.numel(), _p(events), n_ids, _p(repeats), _p(found), _stream()))
+        found = torch.zeros(2 * steps + 3, dtype=torch.int32, device=self.dev)  # ... and behind the three words what each step repeats
+        repeats, longest = found[3:steps + 3], found[steps + 3:]
+        _lib.check(self.lib.bmtk_events_check(steps, _p(ptr), events.numel(), _p(events), n_ids, _p(repeats), _p(longest), _p(found), _stream()))
         bad, count, most = found[:3].tolist()
         if bad & _lib.EVENTS_INCONSISTENT:
             raise ValueError("device input event lists are inconsistent")

@@ -49,7 +49,7 @@ extern "C" {
 
 /* Bumped whenever a struct layout or a signature below changes; bmtk_amd_abi_version() returns the value the
  * library was built with. */
-#define BMTK_AMD_ABI_VERSION 32
+#define BMTK_AMD_ABI_VERSION 33
 int bmtk_amd_abi_version(void);
 const char *bmtk_amd_last_error(void);
 /* sizeof(bmtk_glif3_sim) as the library was compiled, for bindings that mirror the struct */
@@ -509,11 +509,12 @@ int bmtk_csr_weight_reach(int64_t nnz, const int32_t *indices, const float *weig
 /* Looks over per-step event lists (in_events[in_ptr[t] .. in_ptr[t + 1]) are the ids of step t; in_ptr has n_steps + 1 entries)
  * before anything else reads them: found[0] |= BMTK_EVENTS_INCONSISTENT where in_ptr does not ascend from 0 to n_events or an id
  * lies outside 0 .. n_ids - 1, BMTK_EVENTS_UNORDERED where ids of a step descend; repeats[t] = how many ids of step t equal the
- * one before them, found[1] += their number in all, found[2] = the most of a step.  The caller clears the three words of found. */
+ * one before them, found[1] += their number in all; longest[t] = how many of those on end are the same id, at most, found[2] = the most
+ * of any step.  The caller clears the three words of found. */
 #define BMTK_EVENTS_INCONSISTENT 1
 #define BMTK_EVENTS_UNORDERED 2
 int bmtk_events_check(int64_t n_steps, const int64_t *in_ptr, int64_t n_events, const int32_t *in_events, int64_t n_ids, int32_t *repeats,
-                      uint32_t *found, void *stream);
+                      int32_t *longest, uint32_t *found, void *stream);
 
 /* Those repeated ids, of lists without fault: step t's into to[first[t] .. first[t + 1]), first being the running sum of repeats
  * (n_steps + 1 entries, 0 first). */

@@ -43,6 +43,18 @@ def test_repeated_ids_are_listed_apart(sim, counts, repeats, device):
         assert sim.in_repeat_ptr is None and sim.in_repeat_events is None
 
 
+@pytest.mark.parametrize("before", [0, 1, 5, 63, 200])
+@pytest.mark.parametrize("times", [1, 2, 63, 64, 65, 66, 128, 129, 256, 257, 258, 700])
+def test_how_often_a_step_repeats_one_id(sim, before, times):
+    """An id that occurs `times` times behind `before` others, beside steps that repeat many ids once or twice."""
+    import torch
+    steps = [np.repeat(np.arange(300), 2), np.concatenate([np.arange(before), np.full(times, 1000), np.arange(1001, 1090)]), np.zeros(0, int),
+             np.repeat(np.arange(90), 3), np.arange(90)]
+    ptr = np.concatenate([[0], np.cumsum([s.size for s in steps])]).astype(np.int64)
+    sim.set_input_events(torch.as_tensor(ptr, device="cuda"), torch.as_tensor(np.concatenate(steps).astype(np.int32), device="cuda"))
+    assert sim.in_most_repeats == max(2, times - 1) and sim.in_repeat_events.numel() == 300 + times - 1 + 180
+
+
 def test_lists_with_faults_are_refused(sim):
     import torch
     ptr, events = _lists([3, 0, 70, 300], 5, True)

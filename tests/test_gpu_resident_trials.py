@@ -488,14 +488,15 @@ def test_weights_that_32_bit_sums_take():
                                            np.ones(w.size, np.int64), np.zeros(w.size, np.int64), rows, n)
     quarters = np.round(rng.normal(0, 20, 400)) / 4
     rec, inp = table(quarters), table(np.full(100, 2.0), 10)
-    k, room = simulator.whole_numbers(rec, inp, n, 5)
-    most = np.bincount(inp.indices.cpu().numpy(), minlength=n).max() * 2.0
-    assert k == 2 and room == int(2.0 ** 30 / (most * 4 * 5))
-    assert simulator.whole_numbers(rec, None, n, 5)[0] == 2 and simulator.whole_numbers(table(np.zeros(3)), None, n, 1)[0] == 0
-    assert simulator.whole_numbers(table(np.array([2.0 ** -30])), None, n, 1)[0] == 30
+    k, room = simulator.whole_numbers(rec, inp, n)
+    of_inputs = np.bincount(inp.indices.cpu().numpy(), minlength=n) * 2.0
+    together = of_inputs + np.bincount(rec.indices.cpu().numpy(), np.abs(rec.weights.cpu().numpy()), n)
+    assert k == 2 and (together.max() + room * of_inputs.max()) * 4 < 2 ** 30 <= (together.max() + (room + 1) * of_inputs.max()) * 4
+    assert simulator.whole_numbers(rec, None, n)[0] == 2 and simulator.whole_numbers(table(np.zeros(3)), None, n)[0] == 0
+    assert simulator.whole_numbers(table(np.array([2.0 ** -30])), None, n)[0] == 30
     for bad in ([2.0 ** -31], [np.nan], [np.inf, 1.0], [2.0 ** 31], [2.0 ** 20, 2.0 ** -11], np.full(100000, 2.0 ** 21)):
-        assert simulator.whole_numbers(rec, table(np.array(bad)), n, 5) is None
-        assert simulator.whole_numbers(table(np.array(bad)), inp, n, 5) is None
+        assert simulator.whole_numbers(rec, table(np.array(bad)), n) is None
+        assert simulator.whole_numbers(table(np.array(bad)), inp, n) is None
     # sums as large as they may come out as they are: every synapse of a neuron at once, either sign
     for sign in (1.0, -1.0):
         w = np.full(3, sign * 2.0 ** 28)
@@ -518,6 +519,37 @@ def test_weights_that_32_bit_sums_take():
 def table_of(n):
     """A recurrent table of one synapse that carries nothing."""
     return (np.array([0] + [1] * n, np.int32), np.array([n - 1], np.int32), np.zeros(1, np.float32), np.ones(1, np.uint8), np.zeros(1, np.uint8))
+
+
+def _heavy(cfg, weight):
+    """An input source that never fires (the last), but could bring a neuron ``weight``."""
+    indptr, indices, w, d, r = (a.copy() for a in cfg["inp_src"])
+    assert indptr[-1] > indptr[-2]
+    w[-1] = weight
+    cfg["inp_src"] = indptr, indices, w, d, r
+    last = cfg["n_in"] - 1
+    batch = cfg["i_ext"].size // cfg["n"]
+    keep = cfg["in_events"] // batch != last
+    cfg["in_ptr"], cfg["in_events"] = np.concatenate([[0], np.cumsum(keep)])[cfg["in_ptr"]].astype(np.int64), cfg["in_events"][keep]
+
+
+def test_many_repeated_events_leave_32_bit_sums_alone():
+    """Hundreds of ids twice in a step: a sum takes one repeat of each where it has room for that of an id that reaches a neuron with all
+    its inputs."""
+    n, batch = 300, 8
+    cfg, _, _ = _case(n, batch, 5, in_rate=400.0)
+    _heavy(cfg, 2.0 ** 26)      # 2^28 of 2^30: room for two repeats of an id
+    steps = np.repeat(np.arange(150), np.diff(cfg["in_ptr"]))
+    repeats = np.bincount(steps[1:][(np.diff(cfg["in_events"]) == 0) & (np.diff(steps) == 0)], minlength=150)
+    st = orc.new_state(n, batch, np.float32)
+    raster = orc.simulate(st, orc.precompute(cfg["par"], 1.0), 1.0, 150, batch=batch, class_id=cfg["class_id"],
+                          ring=np.zeros((cfg["L"], 4, n * batch), np.float32), rec=cfg["rec_src"], inp=cfg["inp_src"],
+                          in_ptr=cfg["in_ptr"], in_events=cfg["in_events"], i_ext=cfg["i_ext"], raster=True)["raster"]
+    sim = _sim(cfg, batch, resident_trials=True, fused=True)
+    assert sim._trials["whole"] == 3 and sim._trials["room"] == 2 and sim.in_most_repeats == 1 and repeats.max() > 40
+    outs = [sim.run(60), sim.run(90)]
+    assert sim._trials["whole"] == 3
+    _same(sim, outs, raster, st)
 
 
 def test_more_repeated_events_than_32_bit_sums_take():
