@@ -309,8 +309,9 @@ class Glif3Simulator:
                 trial or of so many elements that 32 steps of them outgrow TRIALS_SAVE_BYTES), covers fewer than TRIALS_MIN_STEPS
                 steps or is captured into a graph, and a look at ``ring``, ``work_bits`` or ``fuse_any``, make it go on with that
                 driver for good.  True: insist (ValueError otherwise); False: off.  Sums of a batch's arrivals have 64 bits, or 32 where the
-                weights are whole multiples of one power of two that those hold exactly (``whole_numbers``); input lists that repeat
-                an id in a step more often than these have room for make it go on with the other driver, too.
+                weights are whole multiples of one power of two that those hold exactly (``whole_numbers``); a call whose
+                input events repeat an id in a step more often than these have room for makes it go on with 64-bit sums, or with the
+                other driver where those do not fit or pay.
     delay_offset  B steps taken off every delay before the tables are built; spikes and input events are
                 then handed to the tables B steps late from a history of spike bits, which gives the same
                 arrivals with a ring B slots shorter.  "auto": 0 while the largest delay is at most 63
@@ -419,7 +420,7 @@ class Glif3Simulator:
         self.in_ptr = self.in_events = None
         self.in_steps = 0
         self.in_duplicates = False
-        self.in_most_repeats = 0    # of one id, of any step
+        self.in_most_repeats, self.in_repeats_of_one = 0, None   # how often one id is repeated in any step, and in each
         self._lists_replaced = False    # since the last run
         self.in_repeat_ptr = self.in_repeat_events = None   # repeated ids of a step, for the pull form of the inputs
         self.step = 0
@@ -523,18 +524,9 @@ class Glif3Simulator:
             if whole:
                 plan = dict(small, whole=whole[0] + 1, room=whole[1])
             elif plan and self.batch > 1:
-                used = self._receptors_used()
-                third = torch.zeros(self.n + 1, dtype=torch.int64, device=self.dev)
-                torch.cumsum(self._third_and_fourth(used), 0, out=third[1:])
-                plan = resident_trials_plan(self.n, self.batch, self.L, n_cu, third.cpu().numpy())
-        if plan and ((self.n + self.n_inputs) * (plan["groups"] + 1) >= 2 ** 32 or self.n + self.n_inputs >= 2 ** 24
-                     or n_syn >= 2 ** 31 or self.pull_table is not None):
+                plan, used = self._fixed_point_plan()
+        if plan and not self._trials_possible(plan, resident_trials != "auto"):
             plan = None
-        if plan and resident_trials == "auto":
-            if not (trials_pay(plan, self.n, self.batch, n_syn, self.class_id is not None, expected_rate_hz, self.h,
-                               self.fuse_table is not None)
-                    and trials_fit(plan, self.n, self.batch, self.L, self.n_inputs, n_syn)):
-                plan = None
         if plan and self.batch > 1 and self.fuse_table is None:     # (one trial: sums in fp32; the fused form: as good as its own)
             shift = fixed_point_shift([t for t in (self.rec, self.inp) if t is not None], self.n)
             if shift is None and not (resident_trials is True and self._trials_weights_ok(fixed_point_ok)):
@@ -545,6 +537,24 @@ class Glif3Simulator:
                              "that 64-bit fixed point holds and a network whose trial fits the compute units")
         if plan:
             self._trials = dict(plan, seg=None, insisted=resident_trials is True, used=used)
+
+    def _fixed_point_plan(self):
+        """The plan of a batch with 64-bit sums, and the receptors in use that it was made from."""
+        used = self._receptors_used()
+        third = torch.zeros(self.n + 1, dtype=torch.int64, device=self.dev)
+        torch.cumsum(self._third_and_fourth(used), 0, out=third[1:])
+        n_cu = torch.cuda.get_device_properties(self.dev).multi_processor_count
+        return resident_trials_plan(self.n, self.batch, self.L, n_cu, third.cpu().numpy()), used
+
+    def _trials_possible(self, plan, insisted):
+        """Whether the tables of a plan can be had and, unless it is asked for, whether it is expected to pay."""
+        n_syn = sum(t.nnz for t in (self.rec, self.inp) if t is not None)
+        if ((self.n + self.n_inputs) * (plan["groups"] + 1) >= 2 ** 32 or self.n + self.n_inputs >= 2 ** 24
+                or n_syn >= 2 ** 31 or self.pull_table is not None):
+            return False
+        return insisted or (trials_pay(plan, self.n, self.batch, n_syn, self.class_id is not None, self.expected_rate_hz, self.h,
+                                       self.fuse_table is not None)
+                            and trials_fit(plan, self.n, self.batch, self.L, self.n_inputs, n_syn))
 
     def _trials_weights_ok(self, fixed_point_ok):
         """Whether weights that 64-bit fixed point does not all hold exactly are good enough for a caller who insists on the form
@@ -588,6 +598,8 @@ class Glif3Simulator:
             own += at                                   # (fewer than 2^31 synapses)
             packed[at:at + t.nnz] = t.packed()[:t.nnz]
             row, at = row + t.n_rows, at + t.nnz
+        if tr.get("ring") is None:
+            tr["ring"] = torch.zeros(self.batch, self.L - 1, NREC, n, device=self.dev, dtype=torch.int64 if self.batch > 1 else torch.float32)
         tr["whole"] = 0 if tr.get("few") else tr.get("whole", 0)
         if tr["whole"]:
             packed[:, 1] = (packed.view(torch.float32)[:, 1] * 2.0 ** (tr["whole"] - 1)).to(torch.int32)
@@ -606,8 +618,6 @@ class Glif3Simulator:
         # lanes to a segment at most: about as many as it holds synapses on average
         segment = int(math.ceil(math.log2(max(1.0, at / float(max(1, row)) / groups))))
         tr.update(seg=seg, packed=packed, cells=cells, extra=extra, max_team_shift=min(6, segment),
-                  ring=torch.zeros(self.batch, self.L - 1, NREC, n, device=self.dev,
-                                   dtype=torch.int64 if self.batch > 1 else torch.float32),
                   hist=torch.zeros(tr["ways"], 4, n_words(n) + 1, dtype=torch.int64, device=self.dev))
 
     def _trials_run(self, s, n_steps):
@@ -665,16 +675,38 @@ class Glif3Simulator:
             self._pending_check = True
         return True
 
+    def _room_for_repeats(self, n_steps):
+        """Whether sums of 32 bits, where that is what a batch has, hold the input events of a call of ``n_steps`` steps."""
+        tr = self._trials
+        if not tr.get("whole") or tr.get("few") or self.in_most_repeats <= tr["room"]:
+            return True
+        # (some step of the lists repeats an id too often: a call before that step, or behind it, has nothing to do with it)
+        most = self.in_repeats_of_one[max(self.step - 1, 0):self.step + n_steps]
+        return not most.numel() or int(most.max()) <= tr["room"]
+
+    def _trials_in_fixed_point(self):
+        """From 32-bit sums to 64-bit ones, for good, where a plan with those pays as well; what is under way is in rb_ring either way."""
+        tr = self._trials
+        plan, used = self._fixed_point_plan()
+        if plan is None or not self._trials_possible(plan, tr["insisted"]):
+            return
+        self._let_trials_tables_go(tr)
+        self._trials = dict(plan, seg=None, insisted=tr["insisted"], used=used, ring=tr.get("ring"))
+
+    def _let_trials_tables_go(self, tr):
+        for key in ("hist", "seg", "packed", "cells"):
+            if tr.get(key) is not None:
+                self._in_use(tr.pop(key))
+
     def _leave_trials(self):
         """From the form with resident trials to the driver that takes its place, for good: what is still under way is
         handed over."""
         tr, self._trials = self._trials, None
-        if tr is None or tr["seg"] is None:
+        if tr is None or tr.get("ring") is None:
             return
         left, slots = tr["ring"], self.L - 1
-        for t in (left, tr["hist"], tr["seg"], tr["packed"], tr["cells"]):
-            if t is not None:
-                self._in_use(t)
+        self._in_use(left)
+        self._let_trials_tables_go(tr)
         if self.fuse_table is not None:
             self._left_ring, self._pend_from, self._pend_until, self._trials_left = left, self.step, self.step + slots, True
             return
@@ -867,17 +899,17 @@ class Glif3Simulator:
             look = net.check_input_events(in_ptr, in_events, n_ids)
             in_ptr = torch.as_tensor(in_ptr, device=self.dev)
             in_events = torch.as_tensor(in_events, device=self.dev)
-        most, repeated = self._look_over_events(in_ptr, in_events, n_ids) if look else (0, None)
+        most, longest, repeated = self._look_over_events(in_ptr, in_events, n_ids) if look else (0, None, None)
         self.in_ptr = in_ptr
         self.in_events = in_events if in_events.numel() else in_events.new_zeros(1)
         self.in_steps = in_ptr.numel() - 1
         self._lists_replaced = self.step > 0
-        self.in_duplicates, self.in_most_repeats = most > 0, most
+        self.in_duplicates, self.in_most_repeats, self.in_repeats_of_one = most > 0, most, longest
         self.in_repeat_ptr, self.in_repeat_events = repeated or (None, None)
 
     def _look_over_events(self, in_ptr, in_events, n_ids):
-        """ValueError for lists that are not what they should be; how often a step repeats an id at most, and the running sum of the repeats
-        of the steps with the ids themselves where a form at hand asks for them, or None."""
+        """ValueError for lists that are not what they should be; how often a step repeats an id at most, the same of each step, and the running
+        sum of the repeats of the steps with the ids themselves where a form at hand asks for them, or None."""
         ptr, events = in_ptr.to(self.dev), in_events.to(self.dev)
         steps = ptr.numel() - 1
         found = torch.zeros(2 * steps + 3, dtype=torch.int32, device=self.dev)  # ... and behind the three words what each step repeats
@@ -889,12 +921,12 @@ class Glif3Simulator:
         if bad:
             raise ValueError("input events must be ascending within every step")
         if not count or (self.pull_inp_table is None and self.fuse_table is None):
-            return most, None
+            return most, longest, None
         first = torch.zeros(steps + 1, dtype=torch.int64, device=self.dev)
         torch.cumsum(repeats, 0, out=first[1:])
         again = torch.empty(count, dtype=torch.int32, device=self.dev)
         _lib.check(self.lib.bmtk_events_repeated(steps, _p(ptr), _p(events), _p(first), _p(again), _stream()))
-        return most, (first, again)
+        return most, longest, (first, again)
 
     def _struct(self, bits=None, record=None):
         s = _lib.Glif3Sim()
@@ -1011,12 +1043,14 @@ class Glif3Simulator:
                           count=torch.zeros(1 if ways == 1 else ways * _lib.RECORD_COUNT_STRIDE, dtype=torch.int64,
                                             device=self.dev), ways=ways)
         use_trials = (self._trials is not None and n_steps >= TRIALS_MIN_STEPS and record is None
-                      and self.probe_col is None and not torch.cuda.is_current_stream_capturing()
-                      and self.in_most_repeats <= self._trials.get("room", self.in_most_repeats))
+                      and self.probe_col is None and not torch.cuda.is_current_stream_capturing())
         stretch = n_steps
         if use_trials and save_state:
             stretch = min(65535, TRIALS_SAVE_BYTES // (5 * self.ne))
             use_trials = self.batch > 1 and stretch >= TRIALS_MIN_STEPS
+        if use_trials and not self._room_for_repeats(n_steps):
+            self._trials_in_fixed_point()
+            use_trials = not self._trials.get("whole")
         if self._trials is not None and n_steps > 0 and not use_trials:
             self._leave_trials()
         saved = None

@@ -552,12 +552,51 @@ def test_many_repeated_events_leave_32_bit_sums_alone():
     _same(sim, outs, raster, st)
 
 
-def test_more_repeated_events_than_32_bit_sums_take():
-    """A step that repeats an id more often than there is room for: the other driver runs, whatever the sums come to."""
-    cfg, raster, st = _case(300, 8, 3)
-    sim = _sim(cfg, 8, resident_trials=True, fused=True)
-    assert 0 < sim.in_most_repeats <= sim._trials["room"]
-    sim._trials["room"] = sim.in_most_repeats - 1
+@pytest.mark.parametrize("n,batch,max_delay,span", [(300, 8, 3, None), (1025, 12, 5, 1088), (2100, 16, 1, None)])
+def test_more_repeated_events_than_32_bit_sums_take(n, batch, max_delay, span):
+    """A call with a step that repeats an id more often than there is room for: sums of 64 bits from there on, in the same form, with what
+    the calls before left under way.  Calls before that step keep 32 bits, lists that hold it or not."""
+    cfg, _, _ = _case(n, batch, max_delay, steps=200)
+    _heavy(cfg, 2.0 ** 26)
+    # an id five times in step 150: four repeats, room for two
+    at = cfg["in_ptr"][150]
+    assert cfg["in_ptr"][151] > at
+    cfg["in_events"] = np.insert(cfg["in_events"], at, np.full(4, cfg["in_events"][at]))
+    cfg["in_ptr"][151:] += 4
+    st = orc.new_state(n, batch, np.float32)
+    raster = orc.simulate(st, orc.precompute(cfg["par"], 1.0), 1.0, 200, batch=batch, class_id=cfg["class_id"],
+                          ring=np.zeros((cfg["L"], 4, n * batch), np.float32), rec=cfg["rec_src"], inp=cfg["inp_src"],
+                          in_ptr=cfg["in_ptr"], in_events=cfg["in_events"], i_ext=cfg["i_ext"], raster=True)["raster"]
+    sim = _sim(cfg, batch, resident_trials=True, fused=True)
+    assert sim._trials["whole"] == 3 and sim._trials["room"] == 2 and sim.in_most_repeats >= 4
+    if span:
+        sim._trials.update(span=span, groups=-(-n // span), ways=min(batch, 256 // -(-n // span)), list=400)
     outs = [sim.run(60), sim.run(90)]
-    assert sim._trials is None
+    assert sim._trials["whole"] == 3
+    outs.append(sim.run(50))
+    assert sim._trials is not None and sim._trials["whole"] == 0
     _same(sim, outs, raster, st)
+
+
+def test_repeated_events_where_64_bit_sums_do_not_fit(monkeypatch):
+    """... then the driver that takes the form's place goes on, also where memory for the other tables is not there."""
+    cfg, raster, st = _case(300, 8, 3)
+    for how in ("no plan", "no memory"):
+        sim = _sim(cfg, 8, resident_trials=True, fused=True)
+        outs = [sim.run(60)]
+        assert 0 < sim.in_most_repeats <= sim._trials["room"]
+        sim._trials["room"] = sim.in_most_repeats - 1
+        with monkeypatch.context() as m:
+            if how == "no plan":
+                m.setattr(simulator, "resident_trials_plan", lambda *a: None)
+            else:
+                sim._trials["insisted"] = False
+                m.setattr(simulator, "trials_pay", lambda *a: True)
+                m.setattr(sim, "_setup_trials", _no_memory)
+            outs.append(sim.run(90))
+        assert sim._trials is None
+        _same(sim, outs, raster, st)
+
+
+def _no_memory():
+    raise torch.OutOfMemoryError("none")
