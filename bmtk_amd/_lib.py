@@ -68,7 +68,7 @@ class Glif3Bwd(C.Structure):
 
 
 EVENTS_INCONSISTENT = 1     # BMTK_EVENTS_INCONSISTENT
-ABI_VERSION = 33  # BMTK_AMD_ABI_VERSION of include/bmtk_amd.h that the mirrors above were written for
+ABI_VERSION = 34  # BMTK_AMD_ABI_VERSION of include/bmtk_amd.h that the mirrors above were written for
 
 # name -> (restype, argtypes); every symbol include/bmtk_amd.h declares
 SIGNATURES = {
@@ -111,7 +111,8 @@ SIGNATURES = {
     "bmtk_glif3_simulate_fwd": (c_int32, [C.POINTER(Glif3Sim), c_int64, c_int64, c_void_p]),
     "bmtk_csr_receptors_used": (c_int32, [c_int64] + [c_void_p] * 4),
     "bmtk_csr_pack_cells": (c_int32, [c_int64, c_int32] + [c_void_p] * 3),
-    "bmtk_csr_weight_reach": (c_int32, [c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
+    "bmtk_csr_weight_reach": (c_int32, [c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
+    "bmtk_csr_pack_whole": (c_int32, [c_int64, c_int32, c_void_p, c_void_p, c_void_p]),
     "bmtk_events_check": (c_int32, [c_int64, c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p]),
     "bmtk_events_repeated": (c_int32, [c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
     "bmtk_events_by_trial": (c_int32, [c_int32, c_int64, c_int64, c_int32] + [c_void_p] * 6),

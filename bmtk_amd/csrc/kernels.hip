@@ -307,17 +307,36 @@ __global__ __launch_bounds__(kBlock) void compact_write_fused_kernel(const uint6
     }
 }
 
+// By which the weights of a table are known again, whatever their order: the sum of a synapse's target and weight, mixed (the finaliser
+// of splitmix64, Steele, Lea and Flood 2014).
+__device__ __forceinline__ unsigned long long synapse_mark(unsigned target, unsigned weight_bits)
+{
+    unsigned long long z = ((unsigned long long)weight_bits << 32 | target) + 0x9E3779B97F4A7C15ull;
+    z = (z ^ z >> 30) * 0xBF58476D1CE4E5B9ull;
+    z = (z ^ z >> 27) * 0x94D049BB133111EBull;
+    return z ^ z >> 31;
+}
+__device__ __forceinline__ void add_mark(unsigned long long *mark, unsigned long long own)
+{
+#pragma unroll
+    for (int step = kWave / 2; step > 0; step >>= 1) own += __shfl_xor(own, step, kWave);
+    if (lane_id() == 0) atomicAdd(mark, own);
+}
+
 // What 32-bit sums of arrivals have to know of a table's weights, in one pass: the lowest power of two that a set bit of some weight
 // stands for, the largest size (both reduced per wavefront first), and how much could reach each target at once, in multiples of 2^-10
 // rounded up.  Bounded by the additions, 47 ps each: 2.9 ms for 62 M synapses, where a count in doubles and ten array operations took 9.
 __global__ __launch_bounds__(kBlock) void weight_reach_kernel(int64_t nnz, const int32_t *__restrict__ indices, const float *__restrict__ weights,
-                                                              unsigned long long *__restrict__ reach, int32_t *__restrict__ found)
+                                                              unsigned long long *__restrict__ reach, int32_t *__restrict__ found,
+                                                              unsigned long long *__restrict__ mark)
 {
     int lowest = 0, largest = 0;
+    unsigned long long own = 0ull;
     for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < nnz; i += (int64_t)gridDim.x * kBlock) {
         const unsigned bits = __float_as_uint(weights[i]) & 0x7FFFFFFFu, exponent = bits >> 23;
         const unsigned mantissa = (bits & 0x7FFFFFu) | (exponent ? 0x800000u : 0u);
         largest = max(largest, (int)bits);
+        own += synapse_mark((unsigned)indices[i], __float_as_uint(weights[i]));
         if (mantissa == 0u) continue;
         lowest = min(lowest, (int)max(exponent, 1u) - 150 + __ffs((int)mantissa) - 1);
         // (sizes of 2^30 and more, infinities and NaN are told by found[1])
@@ -328,10 +347,23 @@ __global__ __launch_bounds__(kBlock) void weight_reach_kernel(int64_t nnz, const
         lowest = min(lowest, __shfl_xor(lowest, step, kWave));
         largest = max(largest, __shfl_xor(largest, step, kWave));
     }
+    add_mark(mark, own);
     if (lane_id() == 0) {
         atomicMin(found, lowest);
         atomicMax(found + 1, largest);
     }
+}
+
+// The weights of packed records as whole numbers of 2^-k (scale = 2^k).  One read and one write of the records.
+__global__ __launch_bounds__(kBlock) void pack_whole_kernel(int64_t nnz, float scale, uint2 *__restrict__ packed, unsigned long long *__restrict__ mark)
+{
+    unsigned long long own = 0ull;
+    for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < nnz; i += (int64_t)gridDim.x * kBlock) {
+        const uint2 sy = packed[i];
+        own += synapse_mark(sy.x & 0xFFFFFFu, sy.y);
+        packed[i].y = (unsigned)(int)(__uint_as_float(sy.y) * scale);
+    }
+    add_mark(mark, own);
 }
 
 // Input event lists looked over, a wavefront per step.  Bounded by launches and the one look at `found` that follows: the same in
@@ -681,14 +713,25 @@ int bmtk_spikes_compact_bits(const uint64_t *zbits, int64_t n, int32_t *ids, int
     return compact_from_bits(zbits, n, ids, count, block_count, (hipStream_t)stream);
 }
 
-int bmtk_csr_weight_reach(int64_t nnz, const int32_t *indices, const float *weights, uint64_t *reach, int32_t *found, void *stream)
+int bmtk_csr_weight_reach(int64_t nnz, const int32_t *indices, const float *weights, uint64_t *reach, int32_t *found, uint64_t *mark, void *stream)
 {
-    BMTK_REQUIRE(nnz >= 0 && found && reach && (nnz == 0 || (indices && weights)), "csr_weight_reach: bad sizes or null pointers");
+    BMTK_REQUIRE(nnz >= 0 && found && reach && mark && (nnz == 0 || (indices && weights)), "csr_weight_reach: bad sizes or null pointers");
     if (nnz == 0) return BMTK_OK;
     const int64_t blocks = (nnz + kBlock - 1) / kBlock;
     hipLaunchKernelGGL(weight_reach_kernel, dim3((unsigned)(blocks < 4096 ? blocks : 4096)), dim3(kBlock), 0, (hipStream_t)stream, nnz, indices,
-                       weights, reinterpret_cast<unsigned long long *>(reach), found);
+                       weights, reinterpret_cast<unsigned long long *>(reach), found, reinterpret_cast<unsigned long long *>(mark));
     BMTK_CHECK_LAUNCH("csr_weight_reach");
+    return BMTK_OK;
+}
+
+int bmtk_csr_pack_whole(int64_t nnz, int32_t k, bmtk_synapse *packed, uint64_t *mark, void *stream)
+{
+    BMTK_REQUIRE(nnz >= 0 && k >= 0 && k <= 30 && mark && (nnz == 0 || packed), "csr_pack_whole: bad sizes or null pointers");
+    if (nnz == 0) return BMTK_OK;
+    const int64_t blocks = (nnz + kBlock - 1) / kBlock;
+    hipLaunchKernelGGL(pack_whole_kernel, dim3((unsigned)(blocks < 4096 ? blocks : 4096)), dim3(kBlock), 0, (hipStream_t)stream, nnz, ldexpf(1.0f, k),
+                       reinterpret_cast<uint2 *>(packed), reinterpret_cast<unsigned long long *>(mark));
+    BMTK_CHECK_LAUNCH("csr_pack_whole");
     return BMTK_OK;
 }
 

@@ -192,25 +192,26 @@ def fixed_point_shift(tables, n_neurons):
 
 def whole_numbers(rec, inp, n_neurons):
     """Whether the sums of arrivals fit 32-bit whole numbers of a power of two that every weight is a multiple of: (k, how often a step may
-    repeat an input id) for multiples of 2^-k pA, or None.  A synapse has one delay, so what it brings to a sum comes from the
+    repeat an input id, mark by which the weights are known again) for multiples of 2^-k pA, or None.  A synapse has one delay, so what it brings to a sum comes from the
     events of one step: all synapses of a neuron once, and those of the inputs once more for every time that a step may repeat their id, have
     to come to less than half of what 32 bits hold (the other half is for arrivals under way where ``step`` is set back)."""
     lib, tables = _lib.load(), [t for t in (inp, rec) if t is not None and t.nnz]
     if not tables:
-        return 0, 1 << 30
+        return 0, 1 << 30, 0
     dev = tables[0].weights.device
-    reach, found = torch.zeros(n_neurons, dtype=torch.int64, device=dev), torch.zeros(2, dtype=torch.int32, device=dev)
+    reach, found = torch.zeros(n_neurons, dtype=torch.int64, device=dev), torch.zeros(4, dtype=torch.int32, device=dev)
+    mark = found[2:].view(torch.int64)
     of_inputs = torch.zeros(1, device=dev)
     for t in tables:      # (the inputs first, so that what they come to is known by itself)
-        _lib.check(lib.bmtk_csr_weight_reach(t.nnz, _p(t.indices), _p(t.weights), _p(reach), _p(found), _stream()))
+        _lib.check(lib.bmtk_csr_weight_reach(t.nnz, _p(t.indices), _p(t.weights), _p(reach), _p(found), _p(mark), _stream()))
         if t is inp:
             of_inputs = reach.max()
-    (lowest, largest), of_inputs, most = found.tolist(), float(of_inputs.max()) / 1024.0, float(reach.max()) / 1024.0
+    (lowest, largest, *_), of_inputs, most = found.tolist(), float(of_inputs.max()) / 1024.0, float(reach.max()) / 1024.0
     k = -lowest
     left = 2.0 ** 30 - most * 2.0 ** k
     if largest >= 0x4E800000 or k > 30 or left <= 0.0:      # (2^30 as a float's bits)
         return None
-    return k, math.ceil(left / max(1.0, of_inputs * 2.0 ** k)) - 1
+    return k, math.ceil(left / max(1.0, of_inputs * 2.0 ** k)) - 1, int(mark)
 
 
 def fused_pays(n_neurons, batch, n_synapses, class_table, rate_hz, h_ms=1.0):
@@ -522,7 +523,7 @@ class Glif3Simulator:
             small = resident_trials_plan(self.n, self.batch, self.L, n_cu, None, 4) if self.batch > 1 else None
             whole = whole_numbers(self.rec, self.inp, self.n) if small and (plan is None or plan_cost(small) <= plan_cost(plan)) else None
             if whole:
-                plan = dict(small, whole=whole[0] + 1, room=whole[1])
+                plan = dict(small, whole=whole[0] + 1, room=whole[1], mark=whole[2])
             elif plan and self.batch > 1:
                 plan, used = self._fixed_point_plan()
         if plan and not self._trials_possible(plan, resident_trials != "auto"):
@@ -580,7 +581,8 @@ class Glif3Simulator:
 
     def _setup_trials(self):
         """Tables and buffers of the form with resident trials: recurrent and input rows as one table sorted by target,
-        the bounds of every workgroup's segment of every row, the ring behind a call and the ballot history."""
+        the bounds of every workgroup's segment of every row, the ring behind a call and the ballot history.  False where they cannot be
+        had any more: 32-bit sums, weights that somebody has written to since these were chosen, and no room for 64-bit ones."""
         tr, n = self._trials, self.n
         groups = tr["groups"]
         seg = torch.empty(n + self.n_inputs, groups + 1, dtype=torch.int32, device=self.dev)
@@ -602,7 +604,11 @@ class Glif3Simulator:
             tr["ring"] = torch.zeros(self.batch, self.L - 1, NREC, n, device=self.dev, dtype=torch.int64 if self.batch > 1 else torch.float32)
         tr["whole"] = 0 if tr.get("few") else tr.get("whole", 0)
         if tr["whole"]:
-            packed[:, 1] = (packed.view(torch.float32)[:, 1] * 2.0 ** (tr["whole"] - 1)).to(torch.int32)
+            mark = torch.zeros(1, dtype=torch.int64, device=self.dev)
+            _lib.check(self.lib.bmtk_csr_pack_whole(at, tr["whole"] - 1, _p(packed), _p(mark), _stream()))
+            if int(mark) != tr["mark"]:
+                self._trials_in_fixed_point()
+                return not self._trials.get("whole") and self._setup_trials()
         elif self.sum_shift:
             packed.view(torch.float32)[:, 1] *= 2.0 ** self.sum_shift
         cells, extra = None, 2 * tr["span"]
@@ -619,6 +625,7 @@ class Glif3Simulator:
         segment = int(math.ceil(math.log2(max(1.0, at / float(max(1, row)) / groups))))
         tr.update(seg=seg, packed=packed, cells=cells, extra=extra, max_team_shift=min(6, segment),
                   hist=torch.zeros(tr["ways"], 4, n_words(n) + 1, dtype=torch.int64, device=self.dev))
+        return True
 
     def _trials_run(self, s, n_steps):
         """Fill ``s`` for a call in the form with resident trials.  Returns what has to live until it is launched."""
@@ -649,11 +656,11 @@ class Glif3Simulator:
 
     def _run_trials(self, n_steps, stretch, bits, saved):
         """A call in the form with resident trials, ``stretch`` steps at a time.  False, and nothing done, if that was the
-        constructor's choice and there is no memory for it."""
+        constructor's choice and there is no memory for it, or its tables cannot be had any more."""
         scratch = {}
         try:
-            if self._trials["seg"] is None:
-                self._setup_trials()
+            if self._trials["seg"] is None and not self._setup_trials():
+                return False
             if saved is not None:
                 scratch = dict(v=torch.empty(stretch * self.ne, device=self.dev),
                                flags=torch.empty(stretch * self.ne, dtype=torch.uint8, device=self.dev))

@@ -49,7 +49,7 @@ extern "C" {
 
 /* Bumped whenever a struct layout or a signature below changes; bmtk_amd_abi_version() returns the value the
  * library was built with. */
-#define BMTK_AMD_ABI_VERSION 33
+#define BMTK_AMD_ABI_VERSION 34
 int bmtk_amd_abi_version(void);
 const char *bmtk_amd_last_error(void);
 /* sizeof(bmtk_glif3_sim) as the library was compiled, for bindings that mirror the struct */
@@ -503,8 +503,14 @@ int bmtk_csr_pack_cells(int64_t nnz, int32_t span, const uint32_t *cells, bmtk_s
 
 /* reach[target] += |weight| in multiples of 2^-10, each rounded up (weights of 2^30 and more, infinities and NaN left out), over the
  * synapses of a table whose indices are targets; found[0] = the lowest power of two that a set bit of some weight stands for if that is lower,
- * found[1] = the bits of the largest |weight| if that is larger.  The caller clears them. */
-int bmtk_csr_weight_reach(int64_t nnz, const int32_t *indices, const float *weights, uint64_t *reach, int32_t *found, void *stream);
+ * found[1] = the bits of the largest |weight| if that is larger; mark[0] += a number by which targets and weights are known again, in any
+ * order.  The caller clears them. */
+int bmtk_csr_weight_reach(int64_t nnz, const int32_t *indices, const float *weights, uint64_t *reach, int32_t *found, uint64_t *mark, void *stream);
+
+/* Packed records of the standard packing in place: the weight becomes the 32-bit whole number of 2^-k (0 to 30) that it is, for
+ * bmtk_glif3_sim.rb_whole = k + 1; mark[0] += what bmtk_csr_weight_reach adds for these targets and weights: where the two differ,
+ * the weights are not those that it looked at. */
+int bmtk_csr_pack_whole(int64_t nnz, int32_t k, bmtk_synapse *packed, uint64_t *mark, void *stream);
 
 /* Looks over per-step event lists (in_events[in_ptr[t] .. in_ptr[t + 1]) are the ids of step t; in_ptr has n_steps + 1 entries)
  * before anything else reads them: found[0] |= BMTK_EVENTS_INCONSISTENT where in_ptr does not ascend from 0 to n_events or an id

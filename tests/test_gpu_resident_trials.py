@@ -488,7 +488,7 @@ def test_weights_that_32_bit_sums_take():
                                            np.ones(w.size, np.int64), np.zeros(w.size, np.int64), rows, n)
     quarters = np.round(rng.normal(0, 20, 400)) / 4
     rec, inp = table(quarters), table(np.full(100, 2.0), 10)
-    k, room = simulator.whole_numbers(rec, inp, n)
+    k, room, _ = simulator.whole_numbers(rec, inp, n)
     of_inputs = np.bincount(inp.indices.cpu().numpy(), minlength=n) * 2.0
     together = of_inputs + np.bincount(rec.indices.cpu().numpy(), np.abs(rec.weights.cpu().numpy()), n)
     assert k == 2 and (together.max() + room * of_inputs.max()) * 4 < 2 ** 30 <= (together.max() + (room + 1) * of_inputs.max()) * 4
@@ -596,6 +596,23 @@ def test_repeated_events_where_64_bit_sums_do_not_fit(monkeypatch):
             outs.append(sim.run(90))
         assert sim._trials is None
         _same(sim, outs, raster, st)
+
+
+@pytest.mark.parametrize("which", ["rec", "inp"])
+@pytest.mark.parametrize("scale", [0.3, 2.0 ** 12])
+def test_weights_written_to_before_the_first_run(scale, which):
+    """Weights that no longer are what 32-bit sums were chosen by, in place, behind the constructor: sums of 64 bits of the new ones."""
+    cfg, _, _ = _case(700, 6, 4)
+    sim = _sim(cfg, 6, resident_trials=True)
+    assert sim._trials["whole"] == 3
+    getattr(sim, which).weights.data.mul_(scale)
+    key = which + "_src"
+    indptr, indices, w, d, r = cfg[key]
+    cfg[key] = indptr, indices, w * np.float32(scale), d, r
+    new = _sim(cfg, 6, resident_trials=True)
+    outs, want = ([s.run(50), s.run(100)] for s in (sim, new))
+    assert sim._trials["whole"] == 0
+    _same(sim, outs, np.concatenate([new.raster(o["bits"]).cpu().numpy() for o in want]), new.state.to_numpy())
 
 
 def _no_memory():
