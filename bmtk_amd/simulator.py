@@ -898,7 +898,7 @@ class Glif3Simulator:
             if (not torch.is_tensor(in_events) or in_ptr.dtype != torch.int64 or in_events.dtype != torch.int32
                     or in_ptr.dim() != 1 or in_events.dim() != 1 or not in_ptr.numel()):
                 raise ValueError("device input event lists are inconsistent")
-            in_ptr, in_events = in_ptr.contiguous(), in_events.contiguous()
+            in_ptr, in_events = in_ptr.to(self.dev).contiguous(), in_events.to(self.dev).contiguous()
             look = True
         else:
             in_ptr = np.ascontiguousarray(in_ptr, np.int64)
@@ -917,11 +917,10 @@ class Glif3Simulator:
     def _look_over_events(self, in_ptr, in_events, n_ids):
         """ValueError for lists that are not what they should be; how often a step repeats an id at most, the same of each step, and the running
         sum of the repeats of the steps with the ids themselves where a form at hand asks for them, or None."""
-        ptr, events = in_ptr.to(self.dev), in_events.to(self.dev)
-        steps = ptr.numel() - 1
+        steps = in_ptr.numel() - 1
         found = torch.zeros(2 * steps + 3, dtype=torch.int32, device=self.dev)  # ... and behind the three words what each step repeats
         repeats, longest = found[3:steps + 3], found[steps + 3:]
-        _lib.check(self.lib.bmtk_events_check(steps, _p(ptr), events.numel(), _p(events), n_ids, _p(repeats), _p(longest), _p(found), _stream()))
+        _lib.check(self.lib.bmtk_events_check(steps, _p(in_ptr), in_events.numel(), _p(in_events), n_ids, _p(repeats), _p(longest), _p(found), _stream()))
         bad, count, most = found[:3].tolist()
         if bad & _lib.EVENTS_INCONSISTENT:
             raise ValueError("device input event lists are inconsistent")
@@ -932,7 +931,7 @@ class Glif3Simulator:
         first = torch.zeros(steps + 1, dtype=torch.int64, device=self.dev)
         torch.cumsum(repeats, 0, out=first[1:])
         again = torch.empty(count, dtype=torch.int32, device=self.dev)
-        _lib.check(self.lib.bmtk_events_repeated(steps, _p(ptr), _p(events), _p(first), _p(again), _stream()))
+        _lib.check(self.lib.bmtk_events_repeated(steps, _p(in_ptr), _p(in_events), _p(first), _p(again), _stream()))
         return most, longest, (first, again)
 
     def _struct(self, bits=None, record=None):

@@ -82,3 +82,20 @@ def test_lists_with_faults_are_refused(sim):
         with pytest.raises(ValueError, match="inconsistent"):
             sim.set_input_events(*device(p, e))
     assert sim.in_ptr is kept
+
+
+def test_tensors_in_host_memory_are_taken_to_the_device(sim):
+    """... before the lists at hand give way to them: as arrays are."""
+    import torch
+    ptr, events = _lists([3, 0, 70, 300, 20, 1, 0, 0, 5, 9], 5, True)
+    outs = []
+    for make in (lambda a: torch.as_tensor(a, device="cuda"), torch.as_tensor):
+        sim.set_input_events(make(ptr), make(events))
+        assert sim.in_ptr.is_cuda and sim.in_events.is_cuda
+        sim.step = 0
+        for t in (sim.state.V, sim.state.asc, sim.state.y1, sim.state.y2, sim.state.ref, sim.ring, sim.work_bits, sim.fuse_any):
+            t.zero_()
+        outs.append((sim.run(10)["bits"], sim.state.y1.clone()))
+    assert float(outs[0][1].abs().sum()) > 0
+    for a, b in zip(*outs):
+        assert torch.equal(a, b)
