@@ -640,8 +640,9 @@ int simulate_resident_batch(const bmtk_glif3_sim &s, int64_t step0, int64_t n_st
                  "glif3_simulate_fwd: rb_extra must lie in 0..2 * rb_span with rb_cells (batches; spans above 1024 need it or rb_whole) and be 2 * rb_span without");
     BMTK_REQUIRE(s.sum_shift >= 0 && s.sum_shift <= BMTK_SUM_SHIFT_MAX, "glif3_simulate_fwd: sum_shift must lie in 0..BMTK_SUM_SHIFT_MAX");
     const bool whole = s.rb_whole != 0;
-    BMTK_REQUIRE(s.rb_whole >= 0 && s.rb_whole <= 33 + s.sum_shift && !(whole && (batch == 1 || s.rb_cells)),
-                 "glif3_simulate_fwd: rb_whole must lie in 0..33 + sum_shift and is for batches without rb_cells");
+    // (a kept sum is 33 + sum_shift - rb_whole bits further up than a 32-bit one, which 64 bits hold up to 32)
+    BMTK_REQUIRE(!whole || (s.rb_whole > s.sum_shift && s.rb_whole <= 33 + s.sum_shift && batch > 1 && !s.rb_cells),
+                 "glif3_simulate_fwd: rb_whole must be 0 or lie in sum_shift + 1..sum_shift + 33 and is for batches without rb_cells");
     BMTK_REQUIRE(W >= 1 && W <= batch && s.rb_team_shift >= 0 && s.rb_team_shift <= 6 && s.rb_list >= kWave,
                  "glif3_simulate_fwd: rb_ways must lie in 1..batch, rb_team_shift in 0..6, rb_list from 64 on");
     BMTK_REQUIRE(s.rb_seg && s.rb_packed && s.rb_ring && s.rb_hist && s.res_sync, "glif3_simulate_fwd: resident trials need rb_* and res_sync");

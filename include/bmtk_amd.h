@@ -413,7 +413,7 @@ typedef struct bmtk_glif3_sim {
                                         * planes of rb_span, third and fourth behind these; from bit 4 on, where the neuron's third
                                         * stands among its workgroup's.  NULL (one trial; spans up to 1024; rb_whole): four planes */
     int32_t rb_extra;                  /* third and fourth sums of a workgroup's neurons at most; without rb_cells 2 * rb_span */
-    int32_t rb_whole;                  /* batches without rb_cells; 0, or k + 1: the weight field of rb_packed holds a 32-bit whole number of 2^-k pA
+    int32_t rb_whole;                  /* batches without rb_cells; 0, or k + 1, sum_shift + 1 to sum_shift + 33: the weight field of rb_packed holds a 32-bit whole number of 2^-k pA
                                         * (exactly), and so do the sums in LDS: what may reach a receptor of a neuron in a step must
                                         * stay below 2^31 of them.  rb_ring keeps its 64 bits and unit.  Half the LDS a sum */
     /* Fixed-point sums of the fused and the resident form: their tables (fuse_packed, rb_packed) hold the weights times

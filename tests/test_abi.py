@@ -91,6 +91,22 @@ def test_argument_validation_needs_no_gpu():
     assert _lib.RECORD_COUNT_STRIDE == stride
 
 
+@pytest.mark.parametrize("shift,whole,taken", [(0, 1, True), (0, 33, True), (0, -1, False), (0, 34, False), (1, 1, False), (1, 2, True), (1, 34, True),
+                                               (1, 35, False), (40, 8, False), (120, 1, False), (120, 121, True), (120, 153, True)])
+def test_whole_numbers_keep_within_64_bits(shift, whole, taken):
+    """Sums of 32 bits are kept shifted by 33 + sum_shift - rb_whole, which has to be a shift that 64 bits allow.  (What is taken is
+    refused by what is looked at next, more slots than LDS holds.)"""
+    buf = ctypes.create_string_buffer(64)
+    s = _lib.Glif3Sim()
+    for name in ("V", "asc", "y1", "y2", "ref", "prop", "ring", "work_bits", "rb_seg", "rb_packed", "rb_ring", "rb_hist", "res_sync"):
+        setattr(s, name, ctypes.addressof(buf))
+    s.n_neurons, s.batch, s.ring_slots, s.h, s.prop_stride = 100, 4, 60, 1.0, 100
+    s.rb_span, s.rb_groups, s.rb_ways, s.rb_list, s.rb_extra, s.sum_shift, s.rb_whole = 1024, 1, 1, 64, 2048, shift, whole
+    lib = _lib.load()
+    assert lib.bmtk_glif3_simulate_fwd(ctypes.byref(s), 0, 1, None) == -1
+    assert (b"does not fit in LDS" if taken else b"rb_whole") in lib.bmtk_amd_last_error()
+
+
 def test_ops_refuse_to_run_without_a_gpu():
     import torch
     if torch.cuda.is_available():
