@@ -329,8 +329,9 @@ extern "C" int bmtk_glif3_simulate_fwd(const bmtk_glif3_sim *sim, int64_t step0,
         BMTK_REQUIRE(s.res_span % 64 == 0 && s.res_span <= 1024, "glif3_simulate_fwd: res_span must be a multiple of 64, at most 1024");
         BMTK_REQUIRE(s.res_groups == (ne + s.res_span - 1) / s.res_span, "glif3_simulate_fwd: res_groups must equal ceil(ne/res_span)");
         BMTK_REQUIRE(s.res_sync, "glif3_simulate_fwd: resident mode needs res_sync");
-        BMTK_REQUIRE(!has_rec || s.rec_seg, "glif3_simulate_fwd: resident mode needs rec_seg");
-        BMTK_REQUIRE(!has_inp || s.inp_seg, "glif3_simulate_fwd: resident mode needs inp_seg");
+        // (one workgroup walks whole rows)
+        BMTK_REQUIRE(!has_rec || s.rec_seg || s.res_groups == 1, "glif3_simulate_fwd: resident mode needs rec_seg");
+        BMTK_REQUIRE(!has_inp || s.inp_seg || s.res_groups == 1, "glif3_simulate_fwd: resident mode needs inp_seg");
         BMTK_REQUIRE((size_t)s.ring_slots * GLIF3_NREC * s.res_span * sizeof(float) +
                              (s.res_groups == 1 ? solo_lds_extra(s.res_span) : kResLdsExtra) <= kResLdsBytes,
                      "glif3_simulate_fwd: ring slice does not fit in LDS beside the active-row list");

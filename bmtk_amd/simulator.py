@@ -825,10 +825,7 @@ class Glif3Simulator:
             return
         groups = -(-self.ne // span)
         if groups == 1:
-            # (whole rows are read, in any order: their bounds are the row's)
-            for t in (self.rec, self.inp):
-                if t is not None:
-                    setattr(self, "rec_seg" if t is self.rec else "inp_seg", torch.stack([t.indptr[:-1], t.indptr[1:]], 1))
+            # (whole rows are read, in any order)
             self.res_span, self.res_groups, self.res_fired = span, groups, None
             return
         if self.rec is not None:

@@ -107,6 +107,22 @@ def test_whole_numbers_keep_within_64_bits(shift, whole, taken):
     assert (b"does not fit in LDS" if taken else b"rb_whole") in lib.bmtk_amd_last_error()
 
 
+@pytest.mark.parametrize("table", ["rec", "inp"])
+def test_only_several_workgroups_need_segment_offsets(table):
+    """(What is taken is refused by what is looked at next, more slots than LDS holds.)"""
+    buf = ctypes.create_string_buffer(64)
+    s = _lib.Glif3Sim()
+    for name in ("V", "asc", "y1", "y2", "ref", "prop", "ring", "work_bits", "res_sync", "in_ptr", "in_events", "inp_indptr", "inp_packed", "rec_indptr",
+                 "rec_packed", "rec_seg", "inp_seg"):
+        setattr(s, name, None if name == table + "_seg" else ctypes.addressof(buf))
+    s.n_inputs, s.batch, s.ring_slots, s.h, s.prop_stride, s.res_span = 10, 1, 60, 1.0, 2000, 1024
+    lib = _lib.load()
+    for n, groups, message in ((1000, 1, b"does not fit in LDS"), (2000, 2, table.encode() + b"_seg")):
+        s.n_neurons, s.res_groups = n, groups
+        assert lib.bmtk_glif3_simulate_fwd(ctypes.byref(s), 0, 1, None) == -1
+        assert message in lib.bmtk_amd_last_error()
+
+
 def test_ops_refuse_to_run_without_a_gpu():
     import torch
     if torch.cuda.is_available():
