@@ -44,7 +44,7 @@ class Glif3Sim(C.Structure):
         ("spike_bits", c_void_p), ("spike_bits_stride", c_int64),
         ("save_v", c_void_p), ("save_flags", c_void_p),
         ("probe_col", c_void_p), ("probe_v", c_void_p), ("probe_stride", c_int64), ("probe_every", c_int32),
-        ("_pad1", c_int32),
+        ("res_step_events", c_int32),
         ("spike_step", c_void_p), ("spike_elem", c_void_p), ("spike_frac", c_void_p),
         ("spike_cap", c_int64), ("spike_count", c_void_p), ("spike_ways", c_int32), ("res_min_delay", c_int32),
     ]
@@ -68,7 +68,7 @@ class Glif3Bwd(C.Structure):
 
 
 EVENTS_INCONSISTENT = 1     # BMTK_EVENTS_INCONSISTENT
-ABI_VERSION = 34  # BMTK_AMD_ABI_VERSION of include/bmtk_amd.h that the mirrors above were written for
+ABI_VERSION = 35  # BMTK_AMD_ABI_VERSION of include/bmtk_amd.h that the mirrors above were written for
 
 # name -> (restype, argtypes); every symbol include/bmtk_amd.h declares
 SIGNATURES = {

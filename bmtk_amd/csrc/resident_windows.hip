@@ -525,7 +525,10 @@ __global__ __launch_bounds__(kWinBlock) void sim_window_kernel(bmtk_glif3_sim s,
 // Steps of a window, ring slots and all; false where the form by single steps is the faster one: the spikes arrive too early for
 // windows of several steps, or the ring has no room.  A window of two steps pays while three wavefronts hold no neurons (us per step,
 // windows / single steps, delays of 8 steps: 450 cells 0.77 / 0.97, 640 1.07 / 1.16, 780 1.21 / 1.28, 900 1.6 / 1.57), one of three always (900
-// cells, 10 steps 1.25 / 1.55).  With ballots from the history (a delay offset beyond what LDS keeps) the offset is all that counts.
+// cells, 10 steps 1.25 / 1.55).  Where nearly all wavefronts hold neurons, windows of more input events than their lists hold are not
+// for them (all rows are looked up by wavefronts that have an update to do; us per step, windows of three steps / single steps, 1,000 inputs
+// of 110 synapses a cell: 900 cells 58 events a step 4.66 / 4.71, 72 5.48 / 5.48, 91 6.69 / 6.50, 113 7.95 / 7.60, 139 9.29 / 9.11; 840 cells 72 5.02 / 5.35, 91
+// 6.34 / 6.35, 113 7.59 / 7.42; with three wavefronts free windows stay ahead, 832 cells 91 6.09 / 6.30, 139 8.54 / 8.90).  With ballots from the history (a delay offset beyond what LDS keeps) the offset is all that counts.
 static bool plan_windows(const bmtk_glif3_sim &s, int hist, Window &w, size_t &lds)
 {
     const int longest = s.ring_slots - 1, B = s.delay_offset;
@@ -548,6 +551,7 @@ static bool plan_windows(const bmtk_glif3_sim &s, int hist, Window &w, size_t &l
         if (w.slots < s.ring_slots) w.slots = s.ring_slots;
         lds = window_lds_bytes(w.slots, w.steps, w.span, w.record);
         if (lds + kWinStaticLds > kResLdsBytes) continue;
+        if (least == 3 && (int64_t)s.res_step_events * w.steps > kWinItems) continue;
         w.inp_lds = bounds > 0 && lds + bounds + kWinStaticLds <= kResLdsBytes;
         if (w.inp_lds) lds += bounds;
         const size_t own = s.rec_indptr ? (size_t)(s.n_neurons + 1) * sizeof(int) : 0;

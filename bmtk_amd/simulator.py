@@ -980,6 +980,7 @@ class Glif3Simulator:
             s.rec_seg, s.inp_seg = _p(self.rec_seg), _p(self.inp_seg)
             s.res_fired = _p(self.res_fired)
             s.res_min_delay = self.least_delay
+            s.res_step_events = min(-(-self.in_events.numel() // max(1, self.in_steps)), 1 << 30) if self.in_ptr is not None else 0
             if self.res_unified is not None and s.inp_packed and self.res_groups > 1:
                 s.inp_packed = s.rec_packed      # the input offsets count from the start of the joint table
         if bits is not None:

@@ -49,7 +49,7 @@ extern "C" {
 
 /* Bumped whenever a struct layout or a signature below changes; bmtk_amd_abi_version() returns the value the
  * library was built with. */
-#define BMTK_AMD_ABI_VERSION 34
+#define BMTK_AMD_ABI_VERSION 35
 int bmtk_amd_abi_version(void);
 const char *bmtk_amd_last_error(void);
 /* sizeof(bmtk_glif3_sim) as the library was compiled, for bindings that mirror the struct */
@@ -438,7 +438,7 @@ typedef struct bmtk_glif3_sim {
     float *probe_v;
     int64_t probe_stride;
     int32_t probe_every;         /* >= 1 */
-    int32_t _pad1;
+    int32_t res_step_events;     /* single-workgroup form: input events of a step, about; 0: not known (chooses between its forms only) */
     /* optional spike record with sub-step crossing fractions, appended with
      * atomics (unordered within a step); all NULL to disable */
     int32_t *spike_step;

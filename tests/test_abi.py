@@ -123,6 +123,17 @@ def test_only_several_workgroups_need_segment_offsets(table):
         assert message in lib.bmtk_amd_last_error()
 
 
+@pytest.mark.parametrize("n,events,steps", [(900, 0, 3), (900, 72, 3), (900, 85, 3), (900, 86, 0), (900, 1 << 30, 0), (833, 86, 0), (832, 86, 4), (832, 10000, 4), (450, 10000, 6)])
+def test_windows_of_more_events_than_their_lists_hold(n, events, steps):
+    """... are not for networks of more than 13 wavefronts of neurons."""
+    buf = ctypes.create_string_buffer(64)
+    s = _lib.Glif3Sim()
+    s.n_neurons, s.n_inputs, s.batch, s.res_groups, s.res_span = n, 1000, 1, 1, -(-n // 64) * 64
+    s.delay_offset, s.ring_slots, s.hist_slots, s.res_min_delay, s.res_step_events = 19, 2, 22, 1, events
+    s.spike_count = s.spike_frac = s.inp_indptr = s.rec_indptr = ctypes.addressof(buf)
+    assert _lib.load().bmtk_resident_window_steps(ctypes.byref(s)) == steps
+
+
 def test_ops_refuse_to_run_without_a_gpu():
     import torch
     if torch.cuda.is_available():
