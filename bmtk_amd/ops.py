@@ -222,11 +222,11 @@ class SynapseTable:
             if nnz:
                 fine = fine & (indices.min() >= 0) & (indices.max() < n_cols) & (d.min() >= 1) & (d.max() < ring_slots) & (r.max() < NREC)
             if n_rows:
-                least, most = torch.aminmax(indptr[1:] - indptr[:-1])
-                ok, least, max_row = torch.stack([fine.to(least.dtype), least, most]).tolist()
-                ok = bool(ok) and least >= 0
-            else:
-                ok = bool(fine)
+                # (compared, not subtracted: a difference of 32-bit numbers can come out positive where they descend)
+                fine = fine & (indptr[1:] >= indptr[:-1]).all()
+                most = (indptr[1:] - indptr[:-1]).max()
+                fine, max_row = torch.stack([fine.to(most.dtype), most]).tolist()
+            ok = bool(fine)
         if not ok:
             raise ValueError("inconsistent synapse table (indptr, index range, delay range or receptor range)")
         return cls(indptr, indices, w, d, r, n_rows=n_rows, max_row=max_row)
