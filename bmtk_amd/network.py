@@ -88,7 +88,7 @@ def check_csr(csr, n_rows, n_cols, ring_slots):
     values unchecked, so a table that fails here must never be launched on."""
     indptr, indices, w, d, r = csr
     nnz = int(indptr[-1])
-    if indptr.size != n_rows + 1 or indptr[0] != 0 or np.any(np.diff(indptr) < 0):
+    if indptr.size != n_rows + 1 or indptr[0] != 0 or np.any(indptr[1:] < indptr[:-1]):
         raise ValueError("indptr must be non-decreasing, start at 0 and have n_rows+1 entries")
     for name, a in (("indices", indices), ("weights", w), ("delays", d), ("receptors", r)):
         if a.size != nnz:

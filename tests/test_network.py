@@ -86,7 +86,7 @@ def test_input_event_lists_are_validated():
         net.check_input_events(np.array([0, 3, 2, 5], np.int64), np.array([3, 7, 0, 4, 9], np.int32), 10)
 
 
-@pytest.mark.parametrize("table", ["device"])
+@pytest.mark.parametrize("table", ["device", "host"])
 @pytest.mark.parametrize("indptr,taken", [((0, 1, 1, 3), True), ((0, 0, 0, 3), True), ((0, 2, 1, 3), False), ((1, 1, 2, 3), False), ((0, 1, 2, 2), False),
                                           ((0, -1, 2, 3), False), ((0, 2 ** 31 - 1, -2, 3), False), ((0, 1, -2 ** 31, 3), False)])
 def test_row_bounds_that_descend_are_refused(table, indptr, taken):
@@ -94,11 +94,12 @@ def test_row_bounds_that_descend_are_refused(table, indptr, taken):
     import torch
     from bmtk_amd.ops import SynapseTable
     csr = (np.array(indptr, np.int32), np.array([0, 1, 2], np.int32), np.ones(3, np.float32), np.ones(3, np.uint8), np.zeros(3, np.uint8))
-    adopt = {"device": lambda: SynapseTable.from_device([torch.as_tensor(a) for a in csr], 3, 3, 4)}[table]
+    adopt = {"device": lambda: SynapseTable.from_device([torch.as_tensor(a) for a in csr], 3, 3, 4),
+             "host": lambda: net.check_csr(csr, 3, 3, 4)}[table]
     if taken:
         adopt()
         return
-    with pytest.raises(ValueError, match="indptr"):
+    with pytest.raises(ValueError, match="indptr|entries"):
         adopt()
 
 
