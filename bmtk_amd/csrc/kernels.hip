@@ -325,7 +325,8 @@ __device__ __forceinline__ void add_mark(unsigned long long *mark, unsigned long
 
 // What 32-bit sums of arrivals have to know of a table's weights, in one pass: the lowest power of two that a set bit of some weight
 // stands for, the largest size (both reduced per wavefront first), and how much could reach each target at once, in multiples of 2^-10
-// rounded up.  Bounded by the additions, 47 ps each: 2.9 ms for 62 M synapses, where a count in doubles and ten array operations took 9.
+// rounded up.  Bounded by the additions, 47 ps each: 4.1 ms for 77 M synapses (3.8 without the mark), where a count in doubles and ten array
+// operations took 9 for 62 M.
 __global__ __launch_bounds__(kBlock) void weight_reach_kernel(int64_t nnz, const int32_t *__restrict__ indices, const float *__restrict__ weights,
                                                               unsigned long long *__restrict__ reach, int32_t *__restrict__ found,
                                                               unsigned long long *__restrict__ mark)
@@ -368,7 +369,8 @@ __global__ __launch_bounds__(kBlock) void pack_whole_kernel(int64_t nnz, float s
 
 // Input event lists looked over, a wavefront per step.  Bounded by launches and the one look at `found` that follows: the same in
 // array operations (marks at every step's start, differences, comparisons, reductions, four of them waited for) took 270 us a
-// call, 350 with repeats to list, beside runs of 1.5 to 2.3 ms; this takes 55, and 105 with repeats.
+// call, 350 with repeats to list, beside runs of 1.5 to 2.3 ms; this takes 55, and 60 with repeats, 70 where a step has 2,800 events.
+// 1 to 4 of those are for how often a step repeats one id.
 __global__ __launch_bounds__(kBlock) void events_check_kernel(int64_t n_steps, const int64_t *__restrict__ in_ptr, int64_t n_events,
                                                               const int32_t *__restrict__ in_events, int64_t n_ids, int32_t *__restrict__ repeats,
                                                               int32_t *__restrict__ longest, unsigned *__restrict__ found)

@@ -12,10 +12,10 @@
 //      trial a segment holds tens of synapses, which one lane would take one after the other.
 // Neither state nor arrival sums cross the memory system, and of the table only the segments of rows that fired.
 //
-// Sums are 64-bit fixed point, exact and independent of the order, as in the fused batched driver (and an integer
-// addition in LDS costs 28 clocks per wavefront where a float's costs 194).  Slot t-1 is folded and cleared before the
+// Sums are exact and independent of the order: 64-bit fixed point as in the fused batched driver, or 32-bit whole numbers where the
+// weights allow them (rb_whole, half the room; an integer addition in LDS costs 28 clocks per wavefront where a float's costs 194).  Slot t-1 is folded and cleared before the
 // spikes of step t-1 are added, so that ring_slots - 1 slots suffice: 160 bytes of LDS per neuron and trial at delays of
-// up to five steps with sums for all four receptors.  Behind a call the arrivals still ahead wait in rb_ring, trial by trial.
+// up to five steps with 64-bit sums for all four receptors.  Behind a call the arrivals still ahead wait in rb_ring, trial by trial.
 //
 // Where that saves launches a neuron has sums only for the receptors that some synapse of it ends on (rb_cells): of four ports the cells
 // of a population mostly use two, which is 80 bytes, and with two neurons to a thread (1088 to 1920 a workgroup) twice the
@@ -23,7 +23,7 @@
 // conflicts), the rarer third and fourth stand behind; a record names its cell, so that the pull asks nothing.  A step then takes 1.2 to 1.4
 // times as long: update 0.7 -> 1.4 us (the issue of two neurons' instructions), the pull's chain as before with twice the
 // synapses in a segment.  At 2.2 sums a neuron, 200 steps: 51,978 x 32 in 4 launches of 32 workgroups a trial 5.85 ms, in 8 of 63 8.03;
-// 20,011 x 20 in one launch 1.47, in two 1.74.  230,924 x 8 have no room for two trials either way.
+// 20,011 x 20 in one launch 1.47, in two 1.74.  230,924 x 8 have room for two trials with 32-bit sums only.
 //
 // What bounds it: a step is a chain of dependent loads (lists, segment bounds, synapses), 2.5 us at the smallest sizes,
 // whatever the number of trials side by side; then the table's segments, which every trial reads for itself.  Per step and

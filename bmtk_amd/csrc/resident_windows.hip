@@ -9,7 +9,7 @@
 // A spike of step u arrives from step u + E + 1 on, E = delay offset + smallest residual delay - 1.  Let a window be the
 // steps [T, T+S).  Its updates use up the ring slots [T, T+S), which earlier windows have completed.  Delivered beside them are
 // the spikes and events of the steps u in [T+S-1-E, T+2S-2-E]: their first arrivals lie in the next window, their last at
-// most 2S-2 + (largest - smallest delay) + 1 steps from T, which is the ring's length.  Their rows are listed a window ahead, from
+// most 2S-1 + (largest - smallest delay) steps from T: a ring of one slot more.  Their rows are listed a window ahead, from
 // ballots of steps before T-S: 3S-1 <= E.  In front of the first window its own share is delivered, behind the last one what
 // the call still owes, so that state and ring are left exactly as the other drivers leave them.
 //
@@ -23,7 +23,9 @@
 // cell holds its four receptors side by side, so that an update takes them with one read and clears them with one write, and an
 // update folds the arrivals of its own step (the sum that the other forms leave to the step after: the same roundings).  A wavefront's
 // roles are compiled apart: with one loop for all, spilled registers, whose reloads wait for every load and store under way,
-// made it 0.52 us a step, and lists made by the wavefronts that take the rows 0.46.
+// made it 0.52 us a step, and lists made by the wavefronts that take the rows 0.46.  One loop spills still, that of wavefronts with neurons
+// where fewer than three others are left to take rows (more than 640 cells), which holds every role: 56 of the kernel's 108 scratch
+// instructions, once a window each, none within a step or a row; the others stand before and behind the loops.
 //   450 cells at 0.1 ms, delays of 20 steps, 5 Hz of 1,000 inputs, with record: 0.34 us a step (single steps: 1.03); 900 cells: 1.05 (1.5);
 //   450 cells at 0.001 ms, delays of 2,000 steps: 0.31 (0.74).
 #include <type_traits>

@@ -58,10 +58,15 @@ RES_LDS_EXTRA = RES_ACT_ENTRIES * 4 + 256   # the list plus the kernel's static 
 SOLO_LDS_PER_ELEMENT = 4 * 4
 SOLO_LDS_EXTRA = 10240 + 2048
 RB_WIDE_SPAN = 1920             # neurons of a workgroup at most with two to a thread
-RB_TWO_COST = 1.35              # a step of resident trials with two neurons to a thread against one (51,978 x 32: 1.40, 20,011 x 20: 1.3)
-# ... with sums as 32-bit whole numbers (230,924 x 8: 1.27).  They take less time in as many launches too, no conversion of each weight
-# among other things: 200 steps with sums of 64 / 32 bits 5,000 x 16 630 / 614 us, 10,000 x 8 742 / 594, 31,000 x 8 1,091 / 902, 2,000 x 40 620 / 593, 60,000 x 4
-# 1,163 / 975, 4,000 x 64 1,030 / 878; two to a thread 51,978 x 32 5,484 / 4,901, 20,011 x 20 1,212 / 1,060, 100,000 x 4 2,406 / 2,020, 31,000 x 64
+# A launch of resident trials with two neurons to a thread against one.  Sums for the receptors in use only against all four sums of
+# one: 51,978 x 32 1.46, 20,011 x 20 1.41, 100,000 x 4 1.52, 120,000 x 16 1.32 (spans of 1472 to 1728 / 832 to 960)
+RB_TWO_COST = 1.35
+RB_FEW_COST = 1.07              # one to a thread, sums for the receptors in use only (51,978 x 32 1.11, 20,011 x 20 1.07, 230,924 x 8 1.05, 10,000 x 8 1.08, 2,000 x 40 1.07)
+# Two to a thread with sums as 32-bit whole numbers.  What counts is where few launches are saved, spans of 1408 to 1536 in the place of
+# 1024: five launches to four 128,000 x 10 1.05, four to three 128,000 x 8 1.04, 50,000 x 20 1.16, 62,000 x 16 1.17, 32,000 x 32 1.20, 15,500 x 64 1.21.  Where half of
+# them are saved, or more than a third, it may cost more: 51,978 x 32 1.18, 31,000 x 64 1.26, 230,924 x 8 and 20,011 x 20 1.33, 100,000 x 4 1.43, 120,000 x 16 1.51.
+# They take less time in as many launches too, no conversion of each weight among other things: 200 steps with sums of 64 / 32 bits
+# 5,000 x 16 630 / 614 us, 10,000 x 8 742 / 594, 31,000 x 8 1,091 / 902, 2,000 x 40 620 / 593, 60,000 x 4 1,163 / 975, 4,000 x 64 1,030 / 878; two to a thread 51,978 x 32 5,484 / 4,901, 20,011 x 20 1,212 / 1,060, 100,000 x 4 2,406 / 2,020, 31,000 x 64
 # 6,239 / 5,363; in half the launches 230,924 x 8 5,376 / 3,401 (100 steps), 120,000 x 16 12,264 / 9,702
 RB_TWO_COST_WHOLE = 1.22
 RB_LIST_MIN, RB_LDS_STATIC = 2000, 256   # the form with resident trials: least room (words) for its lists of rows, static LDS
@@ -135,9 +140,9 @@ def resident_trials_plan(n_neurons, batch, ring_slots, n_cu, third=None, sum_byt
         span = -(-(-(-n_neurons // cus)) // 64) * 64
         return plan(span, 1, 1) if 1024 < span <= RB_WIDE_SPAN and places(span) >= RB_LIST_MIN else None
     best, best_cost = None, None
-    # (of equals the first: few sums cost 0.1 us a step to tell apart)
+    # (of equals the first)
     kinds = (((False, 1024, 1.0), (False, RB_WIDE_SPAN, RB_TWO_COST_WHOLE)) if sum_bytes == 4 else
-             ((False, 1024, 1.0), (True, 1024, 1.05), (True, RB_WIDE_SPAN, RB_TWO_COST))[:1 if third is None else 3])
+             ((False, 1024, 1.0), (True, 1024, RB_FEW_COST), (True, RB_WIDE_SPAN, RB_TWO_COST))[:1 if third is None else 3])
     for few, most, cost in kinds:
         most = next((span for span in range(most, 0, -64) if places(span, few) >= RB_LIST_MIN), 0)
         if not most or -(-n_neurons // most) > cus:

@@ -458,7 +458,7 @@ typedef struct bmtk_glif3_sim {
     int32_t spike_ways;
     /* Single-workgroup form: no synapse of the two packed tables has a delay (as its record holds it, after the delay offset)
      * below this many steps; 0 or 1: not known.  With delay_offset it says how long after its spike a first arrival comes,
-     * and the form runs up to half that many steps (8 at most) between two barriers. */
+     * and the form runs up to a third of that many steps (8 at most) between two barriers. */
     int32_t res_min_delay;
 } bmtk_glif3_sim;
 
