@@ -369,8 +369,8 @@ __global__ __launch_bounds__(kBlock) void pack_whole_kernel(int64_t nnz, float s
 
 // Input event lists looked over, a wavefront per step.  Bounded by launches and the one look at `found` that follows: the same in
 // array operations (marks at every step's start, differences, comparisons, reductions, four of them waited for) took 270 us a
-// call, 350 with repeats to list, beside runs of 1.5 to 2.3 ms; this takes 55, and 60 with repeats, 70 where a step has 2,800 events.
-// 1 to 4 of those are for how often a step repeats one id.
+// call, 350 with repeats to list, beside runs of 1.5 to 2.3 ms; this takes 55, and 60 with repeats, 67 where a step has 2,800 events.
+// 1 to 2 of those are for how often a step repeats one id.
 __global__ __launch_bounds__(kBlock) void events_check_kernel(int64_t n_steps, const int64_t *__restrict__ in_ptr, int64_t n_events,
                                                               const int32_t *__restrict__ in_events, int64_t n_ids, int32_t *__restrict__ repeats,
                                                               int32_t *__restrict__ longest, unsigned *__restrict__ found)
@@ -388,6 +388,7 @@ __global__ __launch_bounds__(kBlock) void events_check_kernel(int64_t n_steps, c
         else
             for (int64_t base = p0; base < p1; base += kTogether * kWave) {
                 int32_t id[kTogether], before[kTogether];
+                unsigned long long same[kTogether], any = 0ull;
 #pragma unroll
                 for (int u = 0; u < kTogether; ++u) {
                     const int64_t p = min(base + u * kWave + lane, p1 - 1);
@@ -399,21 +400,31 @@ __global__ __launch_bounds__(kBlock) void events_check_kernel(int64_t n_steps, c
                     const int64_t p = base + u * kWave + lane;
                     if (p < p1 && (id[u] < 0 || id[u] >= n_ids)) bad |= BMTK_EVENTS_INCONSISTENT;
                     if (p < p1 && id[u] < before[u]) bad |= BMTK_EVENTS_UNORDERED;
-                    unsigned long long same = __ballot(p > p0 && p < p1 && id[u] == before[u]);
-                    if (same == 0ull) {
+                    same[u] = __ballot(p > p0 && p < p1 && id[u] == before[u]);
+                    any |= same[u];
+                }
+                // (one branch for what is usual: a branch each made a hand-over of 2,784 events a step, 1 in 200 a repeat, 2.5 us longer)
+                if (any == 0ull) {
+                    run = 0u;
+                    continue;
+                }
+#pragma unroll
+                for (int u = 0; u < kTogether; ++u) {
+                    unsigned long long on = same[u];
+                    if (on == 0ull) {
                         run = 0u;
                         continue;
                     }
-                    again += (unsigned)__popcll(same);
-                    if (same == ~0ull) {
+                    again += (unsigned)__popcll(on);
+                    if (on == ~0ull) {
                         run += kWave;
                         of_one = max(of_one, run);
                         continue;
                     }
-                    of_one = max(of_one, run + (unsigned)__ffsll((long long)~same) - 1u);
-                    run = (unsigned)__clzll((long long)~same);
+                    of_one = max(of_one, run + (unsigned)__ffsll((long long)~on) - 1u);
+                    run = (unsigned)__clzll((long long)~on);
                     unsigned on_end = 0u;
-                    for (; same; same &= same << 1) ++on_end;
+                    for (; on; on &= on << 1) ++on_end;
                     of_one = max(of_one, on_end);
                 }
             }

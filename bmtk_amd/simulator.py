@@ -211,12 +211,12 @@ def whole_numbers(rec, inp, n_neurons):
         _lib.check(lib.bmtk_csr_weight_reach(t.nnz, _p(t.indices), _p(t.weights), _p(reach), _p(found), _p(mark), _stream()))
         if t is inp:
             of_inputs = reach.max()
-    (lowest, largest, *_), of_inputs, most = found.tolist(), float(of_inputs.max()) / 1024.0, float(reach.max()) / 1024.0
+    (lowest, largest, *_), mark, of_inputs, most = found.tolist(), int(mark), float(of_inputs.max()) / 1024.0, float(reach.max()) / 1024.0
     k = -lowest
     left = 2.0 ** 30 - most * 2.0 ** k
     if largest >= 0x4E800000 or k > 30 or left <= 0.0:      # (2^30 as a float's bits)
         return None
-    return k, math.ceil(left / max(1.0, of_inputs * 2.0 ** k)) - 1, int(mark)
+    return k, math.ceil(left / max(1.0, of_inputs * 2.0 ** k)) - 1, mark
 
 
 def fused_pays(n_neurons, batch, n_synapses, class_table, rate_hz, h_ms=1.0):
@@ -921,17 +921,18 @@ class Glif3Simulator:
         sum of the repeats of the steps with the ids themselves where a form at hand asks for them, or None."""
         steps = in_ptr.numel() - 1
         found = torch.zeros(2 * steps + 3, dtype=torch.int32, device=self.dev)  # ... and behind the three words what each step repeats
-        repeats, longest = found[3:steps + 3], found[steps + 3:]
-        _lib.check(self.lib.bmtk_events_check(steps, _p(in_ptr), in_events.numel(), _p(in_events), n_ids, _p(repeats), _p(longest), _p(found), _stream()))
+        at = _p(found)
+        _lib.check(self.lib.bmtk_events_check(steps, _p(in_ptr), in_events.numel(), _p(in_events), n_ids, at + 12, at + 12 + 4 * steps, at, _stream()))
         bad, count, most = found[:3].tolist()
         if bad & _lib.EVENTS_INCONSISTENT:
             raise ValueError("device input event lists are inconsistent")
         if bad:
             raise ValueError("input events must be ascending within every step")
+        longest = found[steps + 3:] if most else None
         if not count or (self.pull_inp_table is None and self.fuse_table is None):
             return most, longest, None
         first = torch.zeros(steps + 1, dtype=torch.int64, device=self.dev)
-        torch.cumsum(repeats, 0, out=first[1:])
+        torch.cumsum(found[3:steps + 3], 0, out=first[1:])
         again = torch.empty(count, dtype=torch.int32, device=self.dev)
         _lib.check(self.lib.bmtk_events_repeated(steps, _p(in_ptr), _p(in_events), _p(first), _p(again), _stream()))
         return most, longest, (first, again)
