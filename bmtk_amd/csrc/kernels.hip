@@ -325,7 +325,7 @@ __device__ __forceinline__ void add_mark(unsigned long long *mark, unsigned long
 
 // What 32-bit sums of arrivals have to know of a table's weights, in one pass: the lowest power of two that a set bit of some weight
 // stands for, the largest size (both reduced per wavefront first), and how much could reach each target at once, in multiples of 2^-10
-// rounded up.  Bounded by the additions, 47 ps each: 4.1 ms for 77 M synapses (3.8 without the mark), where a count in doubles and ten array
+// rounded up.  Bounded by the additions, 47 ps each: 3.9 ms for 77 M synapses (3.6 without the mark), where a count in doubles and ten array
 // operations took 9 for 62 M.
 __global__ __launch_bounds__(kBlock) void weight_reach_kernel(int64_t nnz, const int32_t *__restrict__ indices, const float *__restrict__ weights,
                                                               unsigned long long *__restrict__ reach, int32_t *__restrict__ found,
