@@ -923,16 +923,16 @@ class Glif3Simulator:
         found = torch.zeros(2 * steps + 3, dtype=torch.int32, device=self.dev)  # ... and behind the three words what each step repeats
         at = _p(found)
         _lib.check(self.lib.bmtk_events_check(steps, _p(in_ptr), in_events.numel(), _p(in_events), n_ids, at + 12, at + 12 + 4 * steps, at, _stream()))
+        repeats, longest = found[3:steps + 3], found[steps + 3:]    # (while the device looks)
         bad, count, most = found[:3].tolist()
         if bad & _lib.EVENTS_INCONSISTENT:
             raise ValueError("device input event lists are inconsistent")
         if bad:
             raise ValueError("input events must be ascending within every step")
-        longest = found[steps + 3:] if most else None
         if not count or (self.pull_inp_table is None and self.fuse_table is None):
             return most, longest, None
         first = torch.zeros(steps + 1, dtype=torch.int64, device=self.dev)
-        torch.cumsum(found[3:steps + 3], 0, out=first[1:])
+        torch.cumsum(repeats, 0, out=first[1:])
         again = torch.empty(count, dtype=torch.int32, device=self.dev)
         _lib.check(self.lib.bmtk_events_repeated(steps, _p(in_ptr), _p(in_events), _p(first), _p(again), _stream()))
         return most, longest, (first, again)
