@@ -204,15 +204,15 @@ def whole_numbers(rec, inp, n_neurons):
     if not tables:
         return 0, 1 << 30, 0
     dev = tables[0].weights.device
-    reach, found = torch.zeros(n_neurons, dtype=torch.int64, device=dev), torch.zeros(4, dtype=torch.int32, device=dev)
-    mark = found[2:].view(torch.int64)
-    of_inputs = torch.zeros(1, device=dev)
+    reach, found = torch.zeros(n_neurons, dtype=torch.int64, device=dev), torch.zeros(2, dtype=torch.int64, device=dev)
+    of_inputs, mark = found.new_zeros(1), found[1:]     # (the first word: two of 32 bits)
     for t in tables:      # (the inputs first, so that what they come to is known by itself)
         _lib.check(lib.bmtk_csr_weight_reach(t.nnz, _p(t.indices), _p(t.weights), _p(reach), _p(found), _p(mark), _stream()))
         if t is inp:
-            of_inputs = reach.max()
-    (lowest, largest, *_), mark, of_inputs, most = found.tolist(), int(mark), float(of_inputs.max()) / 1024.0, float(reach.max()) / 1024.0
-    k = -lowest
+            of_inputs = reach.max().view(1)
+    both, mark, of_inputs, most = torch.cat([found, of_inputs, reach.max().view(1)]).tolist()     # (one look at the device)
+    lowest, largest = np.array([both]).view(np.int32).tolist()
+    k, of_inputs, most = -lowest, of_inputs / 1024.0, most / 1024.0
     left = 2.0 ** 30 - most * 2.0 ** k
     if largest >= 0x4E800000 or k > 30 or left <= 0.0:      # (2^30 as a float's bits)
         return None
@@ -608,12 +608,10 @@ class Glif3Simulator:
         if tr.get("ring") is None:
             tr["ring"] = torch.zeros(self.batch, self.L - 1, NREC, n, device=self.dev, dtype=torch.int64 if self.batch > 1 else torch.float32)
         tr["whole"] = 0 if tr.get("few") else tr.get("whole", 0)
+        mark = None
         if tr["whole"]:
             mark = torch.zeros(1, dtype=torch.int64, device=self.dev)
             _lib.check(self.lib.bmtk_csr_pack_whole(at, tr["whole"] - 1, _p(packed), _p(mark), _stream()))
-            if int(mark) != tr["mark"]:
-                self._trials_in_fixed_point()
-                return not self._trials.get("whole") and self._setup_trials()
         elif self.sum_shift:
             packed.view(torch.float32)[:, 1] *= 2.0 ** self.sum_shift
         cells, extra = None, 2 * tr["span"]
@@ -630,6 +628,9 @@ class Glif3Simulator:
         segment = int(math.ceil(math.log2(max(1.0, at / float(max(1, row)) / groups))))
         tr.update(seg=seg, packed=packed, cells=cells, extra=extra, max_team_shift=min(6, segment),
                   hist=torch.zeros(tr["ways"], 4, n_words(n) + 1, dtype=torch.int64, device=self.dev))
+        if mark is not None and int(mark) != tr["mark"]:     # (looked at with all else under way)
+            self._trials_in_fixed_point()
+            return not self._trials.get("whole") and self._setup_trials()
         return True
 
     def _trials_run(self, s, n_steps):
