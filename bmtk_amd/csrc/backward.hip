@@ -492,36 +492,78 @@ __global__ __launch_bounds__(kBlkThreads) void bwd_gather_blocked_kernel(bmtk_gl
     if (do_inp) bwd_inp_grad_waves(a, q, (int)blockIdx.x * kBlkWaves + wave, (int)gridDim.x * kBlkWaves);
 }
 
+// `x` of lane kU of the lane's own group of kLp (8 or 16) lanes
+template <int kLp, int kU>
+__device__ __forceinline__ unsigned of_row(unsigned x)
+{
+    static_assert(kLp == 8 || kLp == 16, "lane groups of half a 32-lane swizzle or less");
+    return (unsigned)__builtin_amdgcn_ds_swizzle((int)x, (kU << 5) | (32 - kLp));
+}
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+constexpr int kBlkBurst = 3;         // batches of sixteen records a row that are asked for at once
+constexpr int kBlkLengthKeys = 128;  // rows of a sweep are sorted by the length of their segment, up to this
+
+// records `at` and `at + 1` (any `at`: sixteen bytes on a boundary of eight)
+__device__ __forceinline__ uint4 pair_at(const uint2 *__restrict__ rows, int at)
+{
+    struct __attribute__((packed, aligned(8))) Pair {
+        unsigned x, y, z, w;
+    };
+    const Pair r = *reinterpret_cast<const Pair *>(rows + at);
+    return make_uint4(r.x, r.y, r.z, r.w);
+}
+
+// LDS of bwd_gather_blocked2_kernel behind the partial sums, by rows of a sweep
+constexpr size_t blk2_sort_bytes(size_t rows_sweep)
+{
+    return rows_sweep * (2 * sizeof(unsigned long long) + 2 * sizeof(int2) + 3 * sizeof(uint16_t)) + 2 * kBlkLengthKeys * sizeof(unsigned);
+}
+
 // TWO steps, t = q.t and t-1, in one pass over the blocked table (batches above 16: lp >= 8).  gz of step t reads
 // the adjoint slots t+1 .. t+L-1, gz of step t-1 the slots t .. t+L-2, and slot t only depends on what the state
 // adjoint of step t+1 left behind (it is psc0 times the adjoint of y1 BEFORE step t is undone): both sums can be taken
 // before the state adjoint of step t runs.  Per synapse the record, its weight, the trip round the row's lanes, the
 // row's bounds and the loop around them are paid once for two steps; the two adjoint rows (same target and
 // receptor, neighbouring slots) are fetched side by side.  The weight gradient rides along for both steps with ONE
-// read-modify-write per record.  Partial sums: gz[x] for step t, gz[8 + x] for step t-1.  Everything else as in
-// bwd_gather_blocked_kernel, except that a row's two partial sums take 32 bytes of LDS per lane (half as many rows
-// per sweep).
-template <bool kGrad, bool kNe24>
-__global__ __launch_bounds__(kBlkThreads) void bwd_gather_blocked2_kernel(bmtk_glif3_bwd a, BwdStep q, int lp, int rows_cu,
-                                                                          int sweeps, int gpw, int use_order, int do_inp)
+// read-modify-write per record.  Partial sums: gz[x] for step t, gz[8 + x] for step t-1.  A row's two partial sums take
+// 32 bytes of LDS per lane (half as many rows per sweep as in bwd_gather_blocked_kernel).
+//
+// What bounds it: a compute unit gets its loads back in the order in which it asked for them.  Adjoint rows that the L2 holds
+// come at one 128-byte row per 2.3 clocks (33 TB/s over the chip), but every record that has to come from memory holds up
+// the rows asked for behind it: 100 M rows beside a 400 MB stream of records take 420 us without the stream, 614 with a
+// piece of it fetched now and then, 457 with eight pieces at once, all wavefronts of a workgroup together.  So the records
+// (and bounds) of a whole visit are asked for at once, a visit ahead, behind a barrier; the barriers also keep the
+// wavefronts within a range, so that its adjoint rows stay in the L2 (misses 46 M -> 12 M lines of 107 M).  And a wavefront's
+// eight rows take as long as the longest of them: 30 % of the lanes' work at 42 records a segment, which is why a sweep's rows
+// are sorted by the length of their segment before every range (and by whether they fired: the gradient's work).
+// 51978 neurons x 32 trials, in-degree 1000, us per launch: as before 1025, with bursts and barriers 880, rows sorted 787, a visit
+// ahead and two records a lane 750; of these 35 are the gradients' read-modify-writes and 50 the input gradients in the tail.
+// Tried: records without a place in the caches (nontemporal, 3 % slower), gradients as atomic additions (1 %), their
+// old values fetched with the records (spills, 2 %).
+template <int kLp, bool kGrad, bool kNe24>
+__global__ __launch_bounds__(kBlkThreads) void bwd_gather_blocked2_kernel(bmtk_glif3_bwd a, BwdStep q, int rows_cu, int sweeps,
+                                                                          int gpw, int use_order, int do_inp)
 {
-    extern __shared__ float4 blk_acc[];  // [kBlkWaves][gpw][2][kWave], then the row order (uint16 per place)
-    constexpr int kF = kBlkInFlight;
+    // partial sums [rows of a sweep][2][kLp], the sweep's fired trials, segment bounds, places in the order of the visits and
+    // rows, the counters of the sort, then the row order (uint16 per place)
+    extern __shared__ float4 blk_acc[];
+    constexpr int kBurst = kBlkBurst;
+    constexpr int per = kWave / kLp;
     const int batch = a.batch;
     const int64_t n = a.n_neurons, ne = n * batch;
     const int L = a.ring_slots;
-    const int lane = lane_id(), wave = threadIdx.x / kWave;
+    const int lane = lane_id(), wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
     const int x = blockIdx.x & 7;
     const int P = a.blk_count >> 3;
-    const int per = kWave / lp;
-    const int grp = lane / lp, b4 = (lane - grp * lp) * 4;
+    const int grp = lane / kLp, in_row = lane & (kLp - 1), b4 = in_row * 4, c8 = in_row & 7;
     const bool lane_on = b4 < batch;
-    const unsigned long long grp_lanes = (lp == kWave ? ~0ull : ((1ull << lp) - 1ull)) << (grp * lp);
+    const unsigned long long grp_lanes = ((1ull << kLp) - 1ull) << (grp * kLp);
     const int64_t row_lo = (int64_t)(blockIdx.x >> 3) * rows_cu;
     const int64_t row_hi = row_lo + rows_cu < n ? row_lo + rows_cu : n;
     const uint2 *__restrict__ rows = reinterpret_cast<const uint2 *>(a.blk_packed);
     const char *__restrict__ ring = reinterpret_cast<const char *>(a.lam_ring);
-    const unsigned lane_off = (unsigned)b4 * 4u;
+    const unsigned lane_off = (unsigned)(lane_on ? b4 : 0) * 4u;  // (lanes without a trial read what the row's first lane reads)
     const unsigned q_lo = (unsigned)(q.t % L) * 4u, q_wrap = q_lo - 4u * (unsigned)L;
     const unsigned ne32 = (unsigned)ne, batch32 = (unsigned)batch;
     // from a synapse's cell for step t to its cell for step t-1: one slot down, or L-1 slots up from slot 0 (bytes)
@@ -530,14 +572,19 @@ __global__ __launch_bounds__(kBlkThreads) void bwd_gather_blocked2_kernel(bmtk_g
         const unsigned dq = tdr >> 24;
         const unsigned plane = min(dq + q_lo, dq + q_wrap);  // (slot of step t + delay) * 4 + receptor
         const unsigned elem = mad_u24(tdr, batch32, kNe24 ? mul_u24(plane, ne32) : plane * ne32);
-        off_t = (elem << 2) + lane_off;
+        off_t = elem << 2;
         off_p = off_t + (plane < 4u ? slot_up : slot_down);
     };
-    float4 *acc = blk_acc + (size_t)wave * gpw * 2 * kWave + lane;
+    const int rows_sweep = kBlkWaves * gpw * per;
+    unsigned long long *fired_l = reinterpret_cast<unsigned long long *>(blk_acc + (size_t)rows_sweep * 2 * kLp);  // [2][rows_sweep]
+    int2 *bounds_l = reinterpret_cast<int2 *>(fired_l + 2 * rows_sweep);             // [2][rows_sweep], by visit of even and odd ranges
+    unsigned *count_l = reinterpret_cast<unsigned *>(bounds_l + 2 * rows_sweep);     // [2 * kBlkLengthKeys]
+    uint16_t *visit_l = reinterpret_cast<uint16_t *>(count_l + 2 * kBlkLengthKeys);  // [2][rows_sweep]: place of a visit's row
+    uint16_t *wanted_l = visit_l + 2 * rows_sweep;                                   // by place: whether its row has visits
+    uint16_t *order = wanted_l + rows_sweep;
     const uint64_t *__restrict__ bits_t = a.spike_bits + q.row * a.spike_bits_stride;
     const uint64_t *__restrict__ bits_p = a.spike_bits + (q.row - 1) * a.spike_bits_stride;
-    uint16_t *order = reinterpret_cast<uint16_t *>(blk_acc + (size_t)kBlkWaves * gpw * 2 * kWave);
-    const int places = sweeps * kBlkWaves * gpw * per;
+    const int places = sweeps * rows_sweep;
     if (kGrad && use_order) {  // rows whose source fired in one of the two steps first (see bwd_gather_blocked_kernel)
         __shared__ unsigned scan_l[2][kBlkWaves];
         unsigned fm = 0u, n_mine = 0u;
@@ -574,169 +621,267 @@ __global__ __launch_bounds__(kBlkThreads) void bwd_gather_blocked2_kernel(bmtk_g
         for (int i = rows_cu + (int)threadIdx.x; i < places; i += kBlkThreads) order[i] = 0xFFFFu;
         __syncthreads();
     }
-    auto row_of = [&](int sw, int k) -> int64_t {
-        const int place = ((sw * gpw + k) * kBlkWaves + wave) * per + grp;
-        if (kGrad && use_order) {
-            const unsigned local = order[place];
-            return local == 0xFFFFu ? row_hi : row_lo + local;
-        }
-        return place < rows_cu ? row_lo + place : row_hi;
+    // the row at a place of sweep sw, counted from the workgroup's first (0xFFFFFFFF: none)
+    auto row_at = [&](int sw, int place) -> unsigned {
+        place += sw * rows_sweep;
+        if (kGrad && use_order) return order[place] == 0xFFFFu ? ~0u : order[place];
+        return place < rows_cu && row_lo + place < row_hi ? (unsigned)place : ~0u;
     };
-    // trials of this lane with a non-zero surrogate derivative in the step of record row `rec_row`
-    auto active_trials = [&](int64_t rec_row, int64_t j) -> unsigned {
-        if (!a.save_flags) return 0xFu;
-        const int64_t e = j * batch + b4;
-        const uint32_t f4 = *reinterpret_cast<const uint32_t *>(a.save_flags + rec_row * ne + e);
-        const float4 v4 = *reinterpret_cast<const float4 *>(a.save_v + rec_row * ne + e);
-        const int64_t col = a.class_id ? (int64_t)a.class_id[j] : j;
-        const float th = a.prop[GLIF3_TH * a.prop_stride + col];
-        const float v[4] = {v4.x, v4.y, v4.z, v4.w};
-        unsigned act = 0u;
-#pragma unroll
-        for (int c = 0; c < 4; ++c)
-            if (((f4 >> (8 * c)) & BMTK_F_INTEGRATING) && fabsf((v[c] - th) / th) < 1.0f) act |= 1u << c;
-        return act;
-    };
+    for (int i = threadIdx.x; i < 2 * kBlkLengthKeys; i += kBlkThreads) count_l[i] = 0u;
     for (int sw = 0; sw < sweeps; ++sw) {
-        // per row group one byte in each word: bits 0-3 the lane's trials with a non-zero surrogate derivative in
-        // the step, bits 4-7 those in which the source fired (kGrad); masks_t for step t, masks_p for step t-1
-        unsigned long long masks_t = 0ull, masks_p = 0ull;
-        for (int k = 0; k < gpw; ++k) {
-            const int64_t j = row_of(sw, k);
-            unsigned at = 0u, ap = 0u, mt = 0u, mp = 0u;
-            if (j < row_hi && lane_on) {
-                at = active_trials(q.row, j);
-                ap = active_trials(q.row - 1, j);
-                if (kGrad) {
-                    mt = (unsigned)(trial_mask(bits_t, j, batch, 0, batch) >> b4) & 0xFu;
-                    mp = (unsigned)(trial_mask(bits_p, j, batch, 0, batch) >> b4) & 0xFu;
+        // The places of a lane group, k = 0 .. gpw-1: what belongs to their rows for the whole sweep.
+        // active: four bits a place, the lane's trials with a non-zero surrogate derivative; of step t, and 16 up of step t-1
+        unsigned active = 0u;
+        {
+            constexpr int kPlaces = kBlkMaxGroups / 2;
+            // (no branches around the loads: those of all places travel together, where there is no row the last one's)
+            uint32_t f4[kPlaces][2];
+            float4 v4[kPlaces][2];
+            float th[kPlaces];
+            unsigned long long fired[kPlaces][2];
+            bool have[kPlaces];
+#pragma unroll
+            for (int k = 0; k < kPlaces; ++k) {
+                const unsigned local = k < gpw ? row_at(sw, (k * kBlkWaves + wave) * per + grp) : ~0u;
+                have[k] = local != ~0u && row_lo + local < row_hi;
+                const int64_t j = have[k] ? row_lo + local : n - 1, e = j * batch + (lane_on ? b4 : 0);
+                th[k] = a.prop[GLIF3_TH * a.prop_stride + (a.class_id ? (int64_t)a.class_id[j] : j)];
+#pragma unroll
+                for (int s = 0; s < 2; ++s) {
+                    f4[k][s] = *reinterpret_cast<const uint32_t *>(a.save_flags + (q.row - s) * ne + e);
+                    v4[k][s] = *reinterpret_cast<const float4 *>(a.save_v + (q.row - s) * ne + e);
+                    if (kGrad) {
+                        const uint64_t *bits = s == 0 ? bits_t : bits_p;
+                        const int64_t bit = j * batch;
+                        const int sh = (int)(bit & 63);
+                        const bool two = sh + batch > 64;
+                        const unsigned long long lo = bits[bit >> 6], hi = bits[(bit >> 6) + (two ? 1 : 0)];
+                        fired[k][s] = lo >> sh | (two ? hi << (64 - sh) : 0ull);
+                        if (batch < 64) fired[k][s] &= (1ull << batch) - 1ull;
+                    }
                 }
             }
-            masks_t |= (unsigned long long)(at | (mt << 4)) << (8 * k);
-            masks_p |= (unsigned long long)(ap | (mp << 4)) << (8 * k);
-            acc[(2 * k) * kWave] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            acc[(2 * k + 1) * kWave] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+#pragma unroll
+            for (int k = 0; k < kPlaces; ++k) {
+                if (k >= gpw) break;
+                const int place = (k * kBlkWaves + wave) * per + grp;
+                unsigned act = 0u;
+#pragma unroll
+                for (int s = 0; s < 2; ++s) {
+                    const float v[4] = {v4[k][s].x, v4[k][s].y, v4[k][s].z, v4[k][s].w};
+#pragma unroll
+                    for (int c = 0; c < 4; ++c)
+                        if (((f4[k][s] >> (8 * c)) & BMTK_F_INTEGRATING) && fabsf((v[c] - th[k]) / th[k]) < 1.0f) act |= 1u << (16 * s + c);
+                }
+                if (!have[k] || !lane_on) act = 0u;
+                active |= act << (4 * k);
+                const bool spiked = kGrad && have[k] && (fired[k][0] | fired[k][1]) != 0ull;
+                // (rows none of whose trials needs a sum, and whose source did not fire, have no visits)
+                const bool wanted = (__ballot(act != 0u) & grp_lanes) != 0ull || spiked;
+                if (in_row == 0) {
+                    wanted_l[place] = wanted ? 1u : 0u;
+                    if (kGrad) {
+                        fired_l[place] = spiked ? fired[k][0] : 0ull;
+                        fired_l[rows_sweep + place] = spiked ? fired[k][1] : 0ull;
+                    }
+                }
+                blk_acc[(size_t)place * 2 * kLp + in_row] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                blk_acc[(size_t)place * 2 * kLp + kLp + in_row] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            }
         }
-        const unsigned long long masks_any = masks_t | masks_p;
-        auto row_range = [&](int ph, int k, int &p, int &p1) {
-            p = p1 = 0;
-            if (ph >= P) return;
-            const bool want = ((masks_any >> (8 * k)) & 0xFFull) != 0ull;
-            const int64_t j = row_of(sw, k);
-            if ((__ballot(want) & grp_lanes) != 0ull && j < row_hi) {
-                const int32_t *__restrict__ ip = a.blk_indptr + (int64_t)(x * P + ph) * n + j;
-                p = ip[0];
-                p1 = ip[1];
+        __syncthreads();
+        // thread i keeps the segment bounds of the row at place i for the range ahead
+        const bool sorts = (int)threadIdx.x < rows_sweep;
+        const unsigned my_row = sorts && wanted_l[threadIdx.x] ? row_at(sw, (int)threadIdx.x) : ~0u;
+        const bool my_fired = kGrad && sorts && (fired_l[threadIdx.x] | fired_l[rows_sweep + threadIdx.x]) != 0ull;
+        int2 ahead = make_int2(0, 0);
+        auto ask_bounds = [&](int ph) {
+            ahead = make_int2(0, 0);
+            if (ph < P && my_row != ~0u) {
+                const int32_t *__restrict__ ip = a.blk_indptr + (int64_t)(x * P + ph) * n + row_lo + my_row;
+                ahead = make_int2(ip[0], ip[1]);
             }
         };
-        int p_next, p1_next;
-        row_range(0, 0, p_next, p1_next);
+        // The rows in the order of their visits to a range: those whose source fired first, the longer segments before the
+        // shorter (a wavefront takes as long as the longest of its eight rows), by counting.  Which of two equal ones
+        // comes first does not matter: a row's sum is its own.
+        auto sort_visits = [&](int ph) {
+            int key = 0;
+            unsigned rank = 0u;
+            if (sorts) {
+                key = kBlkLengthKeys - 1 - min(ahead.y - ahead.x, kBlkLengthKeys - 1) + (my_fired ? 0 : kBlkLengthKeys);
+                rank = atomicAdd(count_l + key, 1u);
+            }
+            __syncthreads();
+            if (wave == 0) {
+                unsigned c[2 * kBlkLengthKeys / kWave], sum = 0u;
+#pragma unroll
+                for (int i = 0; i < 2 * kBlkLengthKeys / kWave; ++i) {
+                    c[i] = count_l[lane * (2 * kBlkLengthKeys / kWave) + i];
+                    sum += c[i];
+                }
+                unsigned at = wave_inclusive_scan(sum) - sum;
+#pragma unroll
+                for (int i = 0; i < 2 * kBlkLengthKeys / kWave; ++i) {
+                    count_l[lane * (2 * kBlkLengthKeys / kWave) + i] = at;
+                    at += c[i];
+                }
+            }
+            __syncthreads();
+            if (sorts) {
+                const unsigned at = (ph & 1) * rows_sweep + count_l[key] + rank;
+                visit_l[at] = (uint16_t)threadIdx.x;
+                bounds_l[at] = ahead;
+            }
+            ask_bounds(ph + 1);
+            __syncthreads();
+            if (threadIdx.x < 2 * kBlkLengthKeys) count_l[threadIdx.x] = 0u;  // (there is a barrier before the next count)
+        };
+        ask_bounds(0);
+        sort_visits(0);
+        // A visit's records, kBurst batches of sixteen a row (lane c8 of a row takes records 2 c8 and 2 c8 + 1 of each), are
+        // asked for a visit ahead and by all wavefronts together.
+        uint4 rec[kBurst];
+        int p = 0, p1 = 0, place = 0;
+        auto burst = [&](uint4 (&r)[kBurst], int from, int end) {
+            const int last = max(end, 2) - 2;  // (a pair past the row's end is the last two records before it)
+#pragma unroll
+            for (int m = 0; m < kBurst; ++m) r[m] = pair_at(rows, min(from + 16 * m + 2 * c8, last));
+        };
+        auto visit_at = [&](int ph, int k, int &from, int &end, int &of) {
+            const int at = (ph & 1) * rows_sweep + (k * kBlkWaves + wave) * per + grp;
+            from = bounds_l[at].x;
+            end = bounds_l[at].y;
+            of = visit_l[at];
+        };
+        visit_at(0, 0, p, p1, place);
+        burst(rec, p, p1);
         for (int ph = 0; ph < P; ++ph) {
             for (int k = 0; k < gpw; ++k) {
-                int p = p_next;
-                const int p1 = p1_next;
-                row_range(k + 1 < gpw ? ph : ph + 1, k + 1 < gpw ? k + 1 : 0, p_next, p1_next);
-                if (__ballot(p < p1) == 0ull) continue;
-                const unsigned mine_t = (unsigned)(masks_t >> (8 * k + 4)) & 0xFu, mine_p = (unsigned)(masks_p >> (8 * k + 4)) & 0xFu;
-                const int p1_lane = ((masks_any >> (8 * k)) & 0xFFull) != 0ull ? p1 : 0;
-                const bool row_fired = kGrad && (__ballot((mine_t | mine_p) != 0u) & grp_lanes) != 0ull;
-                const int in_row = lane - grp * lp;
-                const int c8 = in_row & 7, first = grp * lp;
+                const bool more = k + 1 < gpw || ph + 1 < P;
+                int p_next = 0, p1_next = 0, place_next = place;
+                uint4 rec_next[kBurst];
+                __syncthreads();
+                if (k + 1 == gpw && ph + 1 < P) sort_visits(ph + 1);
+                if (more) visit_at(k + 1 < gpw ? ph : ph + 1, k + 1 < gpw ? k + 1 : 0, p_next, p1_next, place_next);
+                burst(rec_next, p_next, p1_next);
+                auto on = [&]() {
+                    p = p_next;
+                    p1 = p1_next;
+                    place = place_next;
+#pragma unroll
+                    for (int m = 0; m < kBurst; ++m) rec[m] = rec_next[m];
+                };
+                if (__ballot(p < p1) == 0ull) {
+                    on();
+                    continue;
+                }
+                const unsigned mine_t = kGrad ? (unsigned)(fired_l[place] >> b4) & 0xFu : 0u;
+                const unsigned mine_p = kGrad ? (unsigned)(fired_l[rows_sweep + place] >> b4) & 0xFu : 0u;
+                const unsigned long long fired_lanes = kGrad ? __ballot((mine_t | mine_p) != 0u) : 0ull;
+                const bool row_fired = (fired_lanes & grp_lanes) != 0ull;
                 float4 s_t = make_float4(0.0f, 0.0f, 0.0f, 0.0f), s_p = s_t;
-                struct Shared {
-                    uint2 r[kF / 8];
-                };
-                auto fetch = [&](int ahead) {
-                    Shared f;
+                auto sixteen = [&](uint4 own) {
+                    // the lane's own two records first: past the row's end they are record 0 with weight 0 (the same arithmetic and
+                    // the same loads for every lane); their cells are worked out once and passed round with the weights.
+                    // (A pair that begins with the row's last record was fetched one record early.)
+                    const int left = p1 - p - 2 * c8;
+                    const bool some = left > 0, both = left > 1, shifted = left == 1 && p1 > 1;
+                    unsigned own_t[2], own_p[2];
+                    cell_offs(shifted ? own.z : some ? own.x : 0u, own_t[0], own_p[0]);
+                    cell_offs(both ? own.z : 0u, own_t[1], own_p[1]);
+                    const unsigned own_w[2] = {shifted ? own.w : some ? own.y : 0u, both ? own.w : 0u};
+                    auto eight = [&](auto second) {
+                        constexpr int kSecond = decltype(second)::value;
+                        const bool grad_now = kGrad && (fired_lanes & __ballot(p < p1)) != 0ull;
+                        float keep = 0.0f;
+                        auto four = [&](auto which) {
+                            constexpr int h = 4 * decltype(which)::value, l = 4 * kSecond + h / 2;  // (two records a lane)
+                            const unsigned off_t[4] = {of_row<kLp, l>(own_t[0]), of_row<kLp, l>(own_t[1]), of_row<kLp, l + 1>(own_t[0]), of_row<kLp, l + 1>(own_t[1])};
+                            const unsigned off_p[4] = {of_row<kLp, l>(own_p[0]), of_row<kLp, l>(own_p[1]), of_row<kLp, l + 1>(own_p[0]), of_row<kLp, l + 1>(own_p[1])};
+                            float4 vt[4], vp[4];
 #pragma unroll
-                    for (int i = 0; i < kF / 8; ++i) f.r[i] = rows[p + ahead + 8 * i + c8];
-                    return f;
-                };
-                auto record = [&](const Shared &have, int u) {
-                    return make_uint2((unsigned)__shfl((int)have.r[u / 8].x, first + (u & 7), kWave),
-                                      (unsigned)__shfl((int)have.r[u / 8].y, first + (u & 7), kWave));
-                };
-                Shared cur = fetch(0), nxt = cur;
-                auto work = [&](const Shared &have, Shared &ahead) {
-                    float keep = 0.0f;
-                    const bool grad_now = kGrad && __ballot(row_fired && p < p1) != 0ull;
-                    float4 vt[kF], vp[kF];
-                    float w[kF];
+                            for (int u = 0; u < 4; ++u) {
+                                vt[u] = *reinterpret_cast<const float4 *>(ring + (off_t[u] + lane_off));
+                                vp[u] = *reinterpret_cast<const float4 *>(ring + (off_p[u] + lane_off));
+                            }
+                            const unsigned w[4] = {of_row<kLp, l>(own_w[0]), of_row<kLp, l>(own_w[1]), of_row<kLp, l + 1>(own_w[0]), of_row<kLp, l + 1>(own_w[1])};
 #pragma unroll
-                    for (int u = 0; u < kF; ++u) {
-                        const uint2 sy = record(have, u);
-                        const bool valid = p + u < p1_lane;
-                        // (lanes past their row's end take record 0 with weight 0: one select, then the same
-                        // arithmetic and the same two loads for every lane.  With the select on the address instead,
-                        // the compiler branched around the loads and waited for each of them.)
-                        unsigned off_t, off_p;
-                        cell_offs(valid ? sy.x : 0u, off_t, off_p);
-                        w[u] = valid ? __uint_as_float(sy.y) : 0.0f;
-                        vt[u] = *reinterpret_cast<const float4 *>(ring + off_t);
-                        vp[u] = *reinterpret_cast<const float4 *>(ring + off_p);
-                    }
-                    ahead = fetch(kF);
+                            for (int u = 0; u < 4; ++u) {
+                                const float wu = __uint_as_float(w[u]);
+                                s_t.x = fmaf(wu, vt[u].x, s_t.x);
+                                s_t.y = fmaf(wu, vt[u].y, s_t.y);
+                                s_t.z = fmaf(wu, vt[u].z, s_t.z);
+                                s_t.w = fmaf(wu, vt[u].w, s_t.w);
+                                s_p.x = fmaf(wu, vp[u].x, s_p.x);
+                                s_p.y = fmaf(wu, vp[u].y, s_p.y);
+                                s_p.z = fmaf(wu, vp[u].z, s_p.z);
+                                s_p.w = fmaf(wu, vp[u].w, s_p.w);
+                            }
+                            if (grad_now) {
+                                // gradient of a record: over the row's lanes, the adjoint entries of the trials in which the
+                                // source fired, of step t and of step t-1 (see bwd_gather_blocked_kernel)
 #pragma unroll
-                    for (int u = 0; u < kF; ++u) {
-                        s_t.x = fmaf(w[u], vt[u].x, s_t.x);
-                        s_t.y = fmaf(w[u], vt[u].y, s_t.y);
-                        s_t.z = fmaf(w[u], vt[u].z, s_t.z);
-                        s_t.w = fmaf(w[u], vt[u].w, s_t.w);
-                        s_p.x = fmaf(w[u], vp[u].x, s_p.x);
-                        s_p.y = fmaf(w[u], vp[u].y, s_p.y);
-                        s_p.z = fmaf(w[u], vp[u].z, s_p.z);
-                        s_p.w = fmaf(w[u], vp[u].w, s_p.w);
-                    }
-                    if (grad_now) {
-                        // gradient of a record: over the row's lanes, the adjoint entries of the trials in which the
-                        // source fired, of step t and of step t-1 (see bwd_gather_blocked_kernel)
-#pragma unroll
-                        for (int u = 0; u < kF; ++u) {
-                            float g = ((mine_t & 1u) ? vt[u].x : 0.0f) + ((mine_t & 2u) ? vt[u].y : 0.0f) +
-                                      ((mine_t & 4u) ? vt[u].z : 0.0f) + ((mine_t & 8u) ? vt[u].w : 0.0f);
-                            g += ((mine_p & 1u) ? vp[u].x : 0.0f) + ((mine_p & 2u) ? vp[u].y : 0.0f) +
-                                 ((mine_p & 4u) ? vp[u].z : 0.0f) + ((mine_p & 8u) ? vp[u].w : 0.0f);
-                            g += dpp_move<0xB1>(g);
-                            g += dpp_move<0x4E>(g);
-                            g += dpp_move<0x141>(g);
-                            if (lp > 8) g += dpp_move<0x140>(g);
-                            keep = in_row == u ? g : keep;
-                        }
-                    }
-                    if (grad_now && row_fired && in_row < kF && p + in_row < p1) a.d_blk_w[p + in_row] += keep;
-                    p = min(p + kF, p1);  // (a lane whose segment has ended stays at its end: BMTK_BLOCKED_PAD)
+                                for (int u = 0; u < 4; ++u) {
+                                    float g = ((mine_t & 1u) ? vt[u].x : 0.0f) + ((mine_t & 2u) ? vt[u].y : 0.0f) +
+                                              ((mine_t & 4u) ? vt[u].z : 0.0f) + ((mine_t & 8u) ? vt[u].w : 0.0f);
+                                    g += ((mine_p & 1u) ? vp[u].x : 0.0f) + ((mine_p & 2u) ? vp[u].y : 0.0f) +
+                                         ((mine_p & 4u) ? vp[u].z : 0.0f) + ((mine_p & 8u) ? vp[u].w : 0.0f);
+                                    g += dpp_move<0xB1>(g);
+                                    g += dpp_move<0x4E>(g);
+                                    g += dpp_move<0x141>(g);
+                                    if (kLp > 8) g += dpp_move<0x140>(g);
+                                    keep = in_row == h + u ? g : keep;
+                                }
+                            }
+                        };
+                        four(std::integral_constant<int, 0>{});
+                        if (__ballot(p + 4 < p1) != 0ull) four(std::integral_constant<int, 1>{});
+                        if (grad_now && row_fired && in_row < 8 && p + in_row < p1) a.d_blk_w[p + in_row] += keep;
+                        p = min(p + 8, p1);
+                    };
+                    eight(std::integral_constant<int, 0>{});
+                    if (__ballot(p < p1) != 0ull) eight(std::integral_constant<int, 1>{});
                 };
                 while (true) {
-                    work(cur, nxt);
+#pragma unroll
+                    for (int m = 0; m < kBurst; ++m) {
+                        if (__ballot(p < p1) == 0ull) break;
+                        sixteen(rec[m]);
+                    }
                     if (__ballot(p < p1) == 0ull) break;
-                    work(nxt, cur);
-                    if (__ballot(p < p1) == 0ull) break;
+                    burst(rec, p, p1);  // (segments longer than a burst)
                 }
-                float4 t = acc[(2 * k) * kWave];
+                float4 *acc = blk_acc + (size_t)place * 2 * kLp + in_row;
+                float4 t = acc[0];
                 t.x += s_t.x;
                 t.y += s_t.y;
                 t.z += s_t.z;
                 t.w += s_t.w;
-                acc[(2 * k) * kWave] = t;
-                t = acc[(2 * k + 1) * kWave];
+                acc[0] = t;
+                t = acc[kLp];
                 t.x += s_p.x;
                 t.y += s_p.y;
                 t.z += s_p.z;
                 t.w += s_p.w;
-                acc[(2 * k + 1) * kWave] = t;
+                acc[kLp] = t;
+                on();
             }
         }
+        __syncthreads();  // (a row's sums were last added to by whichever wavefront its last visit fell to)
         for (int k = 0; k < gpw; ++k) {
-            const int64_t j = row_of(sw, k);
-            if (j < row_hi && lane_on) {
-                const unsigned at = (unsigned)(masks_t >> (8 * k)) & 0xFu, ap = (unsigned)(masks_p >> (8 * k)) & 0xFu;
-                float4 t = acc[(2 * k) * kWave];
-                *reinterpret_cast<float4 *>(a.gz + (int64_t)x * ne + j * batch + b4) =
-                    make_float4((at & 1u) ? t.x : 0.0f, (at & 2u) ? t.y : 0.0f, (at & 4u) ? t.z : 0.0f, (at & 8u) ? t.w : 0.0f);
-                t = acc[(2 * k + 1) * kWave];
-                *reinterpret_cast<float4 *>(a.gz + (int64_t)(8 + x) * ne + j * batch + b4) =
-                    make_float4((ap & 1u) ? t.x : 0.0f, (ap & 2u) ? t.y : 0.0f, (ap & 4u) ? t.z : 0.0f, (ap & 8u) ? t.w : 0.0f);
-            }
+            const int place = (k * kBlkWaves + wave) * per + grp;
+            const unsigned local = row_at(sw, place);
+            if (local == ~0u || row_lo + local >= row_hi || !lane_on) continue;
+            const int64_t j = row_lo + local;
+            const unsigned at = active >> (4 * k), ap = active >> (16 + 4 * k);
+            // (written once, read by the next launch: not kept in the L2 that the adjoint rows are to stay in)
+            const f32x4 *sums = reinterpret_cast<const f32x4 *>(blk_acc) + (size_t)place * 2 * kLp + in_row;
+            const f32x4 st = sums[0], sp = sums[kLp];
+            __builtin_nontemporal_store(f32x4{(at & 1u) ? st.x : 0.0f, (at & 2u) ? st.y : 0.0f, (at & 4u) ? st.z : 0.0f, (at & 8u) ? st.w : 0.0f},
+                                        reinterpret_cast<f32x4 *>(a.gz + (int64_t)x * ne + j * batch + b4));
+            __builtin_nontemporal_store(f32x4{(ap & 1u) ? sp.x : 0.0f, (ap & 2u) ? sp.y : 0.0f, (ap & 4u) ? sp.z : 0.0f, (ap & 8u) ? sp.w : 0.0f},
+                                        reinterpret_cast<f32x4 *>(a.gz + (int64_t)(8 + x) * ne + j * batch + b4));
         }
     }
     // the input-weight gradients of both steps, in the kernel's tail
@@ -1303,10 +1448,27 @@ __device__ __forceinline__ int64_t first_event_of(const int32_t *__restrict__ ev
     return at_least ? lo + (__ffsll((long long)at_least) - 1) : hi;
 }
 
+// The run of events of one source that begins at `at` (lo <= at < hi, the events of a step): its source and its end, which
+// is `at` where the event before is of the same source.  Called by a whole wavefront with the same arguments in every lane:
+// one load answers all of it for runs of up to 62 events.
+__device__ __forceinline__ int64_t run_at(const int32_t *__restrict__ events, int64_t lo, int64_t at, int64_t hi, int batch, int &j)
+{
+    const int64_t mine = at - 1 + lane_id();  // (lane 0: the event before)
+    const int source = event_source(events[mine < lo ? lo : mine < hi ? mine : hi - 1], batch);
+    j = __builtin_amdgcn_readlane(source, 1);
+    const unsigned long long same = __ballot(mine >= lo && mine < hi && source == j);
+    if (same & 1ull) return at;
+    const unsigned long long other = ~(same >> 1);  // (bit 63 is set: the shift brings in a zero)
+    int64_t end = at + __ffsll((long long)other) - 1;
+    while (end == at + 63 && end < hi && event_source(events[end], batch) == j) ++at, ++end;
+    return end;
+}
+
 // The same for steps t = q.t and t-1 in ONE launch.  Two wavefronts must never update one source's row at a time, so
 // a source with events in both steps belongs to the wavefront that holds the first event of its run in step t,
 // which looks its run of step t-1 up (the events of a step are sorted) and adds both with one read-modify-write;
-// runs of step t-1 whose source has no event in step t are taken by the holder of their first event.
+// runs of step t-1 whose source has no event in step t are taken by the holder of their first event.  The two steps'
+// events are dealt out from the two ends of the wavefronts: with fewer events than wavefronts few get a chain of each.
 __device__ __forceinline__ void bwd_inp_grad2_waves(const bmtk_glif3_bwd &a, const BwdStep &q, int wave, int n_waves)
 {
     const int batch = a.batch;
@@ -1315,22 +1477,23 @@ __device__ __forceinline__ void bwd_inp_grad2_waves(const bmtk_glif3_bwd &a, con
     const int64_t k0 = a.in_ptr[q.t], k1 = a.in_ptr[q.t + 1];
     const int64_t m0 = a.in_ptr[q.t - 1], m1 = k0;  // (in_ptr[t-1] .. in_ptr[t]: the events of step t-1)
     for (int64_t k = k0 + wave; k < k1; k += n_waves) {
-        const int j = event_source(a.in_events[k], batch);
-        if (k > k0 && event_source(a.in_events[k - 1], batch) == j) continue;
-        int64_t k_end = k + 1;
-        while (k_end < k1 && event_source(a.in_events[k_end], batch) == j) ++k_end;
+        int j, same;
+        const int64_t k_end = run_at(a.in_events, k0, k, k1, batch, j);
+        if (k_end == k) continue;
         const int64_t m = first_event_of(a.in_events, m0, m1, j, batch);
         int64_t m_end = m;
-        while (m_end < m1 && event_source(a.in_events[m_end], batch) == j) ++m_end;
+        if (m < m1) {
+            m_end = run_at(a.in_events, m0, m, m1, batch, same);
+            if (same != j) m_end = m;
+        }
         inp_grad_row(a, j, slot_t, k, k_end, slot_p, m, m_end);
     }
-    for (int64_t m = m0 + wave; m < m1; m += n_waves) {
-        const int j = event_source(a.in_events[m], batch);
-        if (m > m0 && event_source(a.in_events[m - 1], batch) == j) continue;
+    for (int64_t m = m0 + (n_waves - 1 - wave); m < m1; m += n_waves) {
+        int j;
+        const int64_t m_end = run_at(a.in_events, m0, m, m1, batch, j);
+        if (m_end == m) continue;
         const int64_t k = first_event_of(a.in_events, k0, k1, j, batch);
         if (k < k1 && event_source(a.in_events[k], batch) == j) continue;  // the source's run of step t takes it along
-        int64_t m_end = m + 1;
-        while (m_end < m1 && event_source(a.in_events[m_end], batch) == j) ++m_end;
         inp_grad_row(a, j, slot_p, m, m_end, 0, 0, 0);
     }
 }
@@ -1384,6 +1547,15 @@ const void *blocked_variant(bool grad, bool ne24, bool wide)
 #undef BMTK_BLK
 }
 
+const void *blocked2_variant(bool lp16, bool grad, bool ne24)
+{
+#define BMTK_BLK2(l, g) (ne24 ? reinterpret_cast<const void *>(bwd_gather_blocked2_kernel<l, g, true>) \
+                              : reinterpret_cast<const void *>(bwd_gather_blocked2_kernel<l, g, false>))
+    if (lp16) return grad ? BMTK_BLK2(16, true) : BMTK_BLK2(16, false);
+    return grad ? BMTK_BLK2(8, true) : BMTK_BLK2(8, false);
+#undef BMTK_BLK2
+}
+
 // launch geometry of bwd_gather_blocked_kernel for a network on the current device
 struct BlockedPlan {
     unsigned grid;
@@ -1426,7 +1598,7 @@ int blocked_plan(const bmtk_glif3_bwd &a, BlockedPlan &pl)
     const int64_t cap2 = (int64_t)kBlkWaves * (kBlkMaxGroups / 2) * per;
     pl.sweeps2 = (int)((rows_cu + cap2 - 1) / cap2);
     pl.gpw2 = (int)((rows_cu + (int64_t)pl.sweeps2 * kBlkWaves * per - 1) / ((int64_t)pl.sweeps2 * kBlkWaves * per));
-    pl.lds2 = (size_t)kBlkWaves * pl.gpw2 * 2 * kWave * sizeof(float4);
+    pl.lds2 = (size_t)kBlkWaves * pl.gpw2 * 2 * kWave * sizeof(float4) + blk2_sort_bytes((size_t)kBlkWaves * pl.gpw2 * per);
     const size_t order_bytes2 = (size_t)pl.sweeps2 * kBlkWaves * pl.gpw2 * per * sizeof(uint16_t);
     pl.use_order2 = (pl.lds2 + order_bytes2 <= kBlkLdsMax && rows_cu <= 16 * kBlkThreads && rows_cu < 0xFFFF) ? 1 : 0;
     if (pl.use_order2) pl.lds2 += order_bytes2;
@@ -1445,12 +1617,8 @@ int blocked_plan(const bmtk_glif3_bwd &a, BlockedPlan &pl)
     }
     static bool asked2[64];
     if (dev >= 0 && dev < 64 && !asked2[dev]) {
-        const void *pair[4] = {reinterpret_cast<const void *>(bwd_gather_blocked2_kernel<true, true>),
-                               reinterpret_cast<const void *>(bwd_gather_blocked2_kernel<true, false>),
-                               reinterpret_cast<const void *>(bwd_gather_blocked2_kernel<false, true>),
-                               reinterpret_cast<const void *>(bwd_gather_blocked2_kernel<false, false>)};
-        for (int g = 0; g < 4; ++g) {
-            const hipError_t err = hipFuncSetAttribute(pair[g], hipFuncAttributeMaxDynamicSharedMemorySize, (int)kBlkLdsMax);
+        for (int g = 0; g < 8; ++g) {
+            const hipError_t err = hipFuncSetAttribute(blocked2_variant(g & 4, g & 2, g & 1), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kBlkLdsMax);
             if (err != hipSuccess) {
                 set_error("transposed propagation: cannot reserve LDS: %s", hipGetErrorString(err));
                 return BMTK_E_LAUNCH;
@@ -1497,14 +1665,10 @@ int blocked2_launch(const bmtk_glif3_bwd &a, const BwdStep &q, const BlockedPlan
     const bool ne24 = a.n_neurons * (int64_t)a.batch < (1ll << 24);
     bmtk_glif3_bwd args = a;
     BwdStep step = q;
-    int lp = pl.lp, rows_cu = pl.rows_cu, sweeps = pl.sweeps2, gpw = pl.gpw2, use_order = pl.use_order2;
+    int rows_cu = pl.rows_cu, sweeps = pl.sweeps2, gpw = pl.gpw2, use_order = pl.use_order2;
     int do_inp = inp_grad ? 1 : 0;
-    void *params[] = {&args, &step, &lp, &rows_cu, &sweeps, &gpw, &use_order, &do_inp};
-    const void *fn = grad ? (ne24 ? reinterpret_cast<const void *>(bwd_gather_blocked2_kernel<true, true>)
-                                  : reinterpret_cast<const void *>(bwd_gather_blocked2_kernel<true, false>))
-                          : (ne24 ? reinterpret_cast<const void *>(bwd_gather_blocked2_kernel<false, true>)
-                                  : reinterpret_cast<const void *>(bwd_gather_blocked2_kernel<false, false>));
-    const hipError_t err = hipLaunchKernel(fn, dim3(pl.grid), dim3(kBlkThreads), params, pl.lds2, st);
+    void *params[] = {&args, &step, &rows_cu, &sweeps, &gpw, &use_order, &do_inp};
+    const hipError_t err = hipLaunchKernel(blocked2_variant(pl.lp > 8, grad, ne24), dim3(pl.grid), dim3(kBlkThreads), params, pl.lds2, st);
     if (err != hipSuccess) {
         set_error("transposed propagation (two steps): launch failed: %s", hipGetErrorString(err));
         return BMTK_E_LAUNCH;

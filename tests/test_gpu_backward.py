@@ -8,7 +8,7 @@ import torch
 
 from oracle import glif3_oracle as orc
 from oracle import glif3_adjoint_ref as adj
-from bmtk_amd import synthetic, training
+from bmtk_amd import ops, synthetic, training
 from bmtk_amd.simulator import Glif3Simulator
 
 pytestmark = pytest.mark.gpu
@@ -309,6 +309,46 @@ def test_blocked_form_with_the_gradient_in_source_major_order():
         torch.cuda.synchronize()
         assert float((b.d_rec_w - want.d_rec_w).abs().max()) <= 1e-6 * float(want.d_rec_w.abs().max()), two_steps
         assert torch.equal(b.lam_V, want.lam_V) and torch.equal(b.lam_ring, want.lam_ring)
+
+
+@pytest.mark.parametrize("batch", [20, 32, 36, 64])
+def test_two_step_gather_at_every_edge_of_its_bursts(batch):
+    """Rows whose segments of one target range have 0, 1, 2, ... records, at the edges of what a lane (2), half a batch (8), a
+    batch (16) and a burst (48) hold, past the longest length that is told apart when rows are sorted (127), one single record at
+    the very start of the table, and several bursts: the adjoint state of the form that takes one step at a time, bit for
+    bit, and its gradients to 1e-6 of the largest."""
+    lengths = [1, 0, 2, 3, 4, 5, 7, 8, 9, 15, 16, 17, 31, 32, 33, 47, 48, 49, 95, 96, 97, 127, 128, 129, 200, 301]
+    rng = np.random.default_rng(batch)
+    n, n_blocks = 203, 8
+    span = -(-n // n_blocks)
+    cfg = _net(batch, 21, n=n, steps=41)
+    src, tgt = [], []
+    for j in range(n):
+        # (row 0: its one record is the first of the table; the others' segments of one range and a few records elsewhere)
+        m, at = lengths[j % len(lengths)], j % n_blocks if j else 0
+        t = np.concatenate([rng.integers(at * span, min(n, (at + 1) * span), m), rng.integers(0, n, 0 if j == 0 else 3)])
+        src += [j] * t.size
+        tgt += t.tolist()
+    src, tgt = np.array(src), np.array(tgt)
+    w = (rng.integers(1, 9, src.size) * 0.25 * np.where(src % 5 == 0, -1.0, 1.0)).astype(np.float32)
+    rec = ops.SynapseTable.from_edges(src, tgt, w, rng.integers(1, cfg["L"], src.size).astype(np.uint8),
+                                      rng.integers(0, 4, src.size).astype(np.uint8), n, n)
+    assert rec.indptr[1].item() == 1
+    sim = Glif3Simulator(n, cfg["par"], cfg["h"], batch=batch, rec=(rec.indptr, rec.indices, rec.weights, rec.delays, rec.receptors),
+                         inp=cfg["inp_src"], ring_slots=cfg["L"], resident=False)
+    sim.set_input_events(cfg["in_ptr"], cfg["in_events"])
+    fwd = sim.run(41, save_state=True)
+    dl = torch.as_tensor(rng.normal(size=(41, n * batch)).astype(np.float32), device="cuda")
+    one = training.Glif3Bptt(sim, dampening=0.3, blocked=True, n_blocks=n_blocks, two_steps=False)
+    two = training.Glif3Bptt(sim, dampening=0.3, blocked=True, n_blocks=n_blocks, two_steps=True)
+    for b in (one, two):
+        b.backward(fwd, dl_dz=dl)
+    for name in ("lam_V", "lam_asc", "lam_y1", "lam_y2", "lam_ring"):
+        assert torch.equal(getattr(one, name), getattr(two, name)), name
+    for name in ("d_rec_w", "d_inp_w"):
+        got, want = getattr(two, name), getattr(one, name)
+        assert float(want.abs().max()) > 0
+        assert float((got - want).abs().max()) <= 1e-6 * float(want.abs().max()), name
 
 
 @pytest.mark.parametrize("seed", range(10))
