@@ -70,6 +70,28 @@ __global__ __launch_bounds__(kBlock) void pull_anyrel_kernel(const uint64_t *__r
     any_rel[j] = (uint8_t)m;
 }
 
+// The same facts and the masks themselves, source by source: pair[j * (L + 1) + d] = the trials in which source j fired in the
+// step held by history row (slot_now - d) mod L, d = 0 .. L, of which the last is the first again.  What a synapse of delay d
+// has to know for the two arrival steps of pull2_pair_kernel, places d and d + 1, then lies in one place.  batch <= 64.
+template <typename Mask>
+__global__ __launch_bounds__(kBlock) void pull_pair_kernel(const uint64_t *__restrict__ hist, int64_t hist_stride, int L, int batch, int64_t n_src,
+                                                           int slot_now, Mask *__restrict__ pair, uint8_t *__restrict__ any_rel,
+                                                           const int32_t *__restrict__ pulled)
+{
+    const int64_t j = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (j >= n_src) return;
+    Mask *__restrict__ to = pair + j * (L + 1);
+    unsigned any = 0u;
+    for (int d = 0; d < L; ++d) {
+        const int r = (slot_now + L - d) % L;
+        const Mask m = pulled && !pulled[r] ? (Mask)0 : (Mask)source_mask(hist + (int64_t)r * hist_stride, (int)j, batch, 0, batch);
+        to[d] = m;
+        if (d == 0) to[L] = m;
+        any |= (m != 0 ? 1u : 0u) << d;
+    }
+    any_rel[j] = (uint8_t)any;
+}
+
 constexpr int kPullBlock = 1024;  // 16 wavefronts share one staged activity map
 // per wavefront: 4 x 64 accumulators of 8 bytes and a stage of 64 entries of 8 bytes
 constexpr size_t kPullAccBytes = (size_t)(kPullBlock / kWave) * (GLIF3_NREC + 1) * kWave * sizeof(unsigned long long);
@@ -384,6 +406,247 @@ __global__ __launch_bounds__(kPullBlock) void pull2_kernel(const uint64_t *__res
     } while (b0.row < n_tgt);
 }
 
+// The rows a wavefront takes from its workgroup's counter, one by one, as a stream of blocks (PullCursor gives every wavefront
+// the same number of rows).  The next row and its bounds are fetched a row ahead.
+template <int kChunks>
+struct RowCursor {
+    const int32_t *__restrict__ indptr;
+    int *counter;
+    int end;           // past the workgroup's last row
+    int row, q, p1;    // row at hand (end: none), what is left of it
+    int nrow, np0, np1;
+    bool at_start;
+
+    __device__ __forceinline__ void look_ahead()
+    {
+        int r = 0;
+        if (lane_id() == 0) r = atomicAdd(counter, 1);
+        nrow = min(__builtin_amdgcn_readfirstlane(r), end);
+        if (nrow < end) {
+            np0 = indptr[nrow];
+            np1 = indptr[nrow + 1];
+        }
+    }
+    __device__ __forceinline__ void advance()
+    {
+        row = nrow;
+        q = np0;
+        p1 = np1;
+        if (row < end) look_ahead();
+    }
+    __device__ __forceinline__ void start(const int32_t *ip, int *ctr, int last)
+    {
+        indptr = ip;
+        counter = ctr;
+        end = last;
+        np0 = np1 = 0;
+        look_ahead();
+        advance();
+    }
+    __device__ __forceinline__ PullBlock next()
+    {
+        if (row >= end) return PullBlock{end, 0, 0, false, false, 0};
+        PullBlock b{row, q, p1, false, false, 0};
+        q += kChunks * kWave;
+        if (q >= p1) {
+            b.last = true;
+            advance();
+        }
+        return b;
+    }
+};
+
+// the first row that begins at position `at` of the table or behind it; a whole wavefront looks, 64 rows at a time
+__device__ __forceinline__ int row_from(const int32_t *__restrict__ indptr, int n_rows, int64_t at)
+{
+    int lo = 0, hi = n_rows;  // the answer lies in lo .. hi
+    while (lo < hi) {
+        const int step = (hi - lo + kWave - 1) / kWave, r = lo + lane_id() * step;
+        const int before = __popcll(__ballot(r < hi && (int64_t)indptr[r] < at));
+        if (before == 0) return lo;
+        hi = min(hi, lo + before * step);
+        lo += (before - 1) * step + 1;
+    }
+    return lo;
+}
+
+// pull2_kernel for histories of up to 8 rows, as many bytes of LDS as there are sources, and batches of up to 64 trials.
+//
+// What bounds it: at low rates the stream of the table (52 M synapses x 64 trials: 416 MB, 65 us at the rate of a bare read; 121 us at
+// 0.3 Hz), at higher ones an L2 line for every synapse whose source fired and the additions.  Against pull2_kernel: one
+// fetch answers both arrival steps (pull_pair_kernel lays the trials out for it) and one stage serves both, so that 14 % (5 Hz) to 36 %
+// (20 Hz) fewer lines are asked for; the trials of 64 synapses travel while those before are added; wavefronts take rows from
+// a counter and workgroups begin where their share of the synapses does (in-degrees with a spread of a half: the
+// last of 4,096 wavefronts with 13 rows each had half as much again to do).  us per call, pull2_kernel / this, 51,978 targets x 64 at
+// in-degree 1000: 134 / 121 at 0.3 Hz, 158 / 141 at 1, 276 / 241 at 5, 532 / 366 at 20; 20,000 x 48 at 500, 5 Hz: 82 / 59; 8,000 x 16
+// at 300: 19.8 / 16.1.  Tried: blocks of 8,192 synapses shared by the workgroup between barriers, whose fetches then come
+// in bursts (147 / 156 / 261 / 438 us at the four rates, without the row counter, where this took 129 / 153 / 263 / 416).
+template <typename Mask>
+struct PullPair {
+    Mask b, a;  // trials for arrival step t (place d), for t - 1 (place d + 1)
+};
+template <typename Mask>
+__device__ __forceinline__ PullPair<Mask> pair_at(const Mask *__restrict__ pair, unsigned at)
+{
+    struct __attribute__((packed, aligned(sizeof(Mask)))) Two {
+        Mask b, a;
+    };
+    const Two t = *reinterpret_cast<const Two *>(pair + at);
+    return PullPair<Mask>{t.b, t.a};
+}
+constexpr int kPairChunks = 4;         // 64-synapse chunks per block of a wavefront
+constexpr int kPairStage = 2 * kWave;  // entries of a wavefront's stage: fewer than 64 left over and up to 64 new ones
+template <typename Mask, bool kAuto>
+__global__ __launch_bounds__(kPullBlock) void pull2_pair_kernel(const Mask *__restrict__ pair, int L, int batch, const int32_t *__restrict__ indptr,
+                                                                const bmtk_synapse *__restrict__ packed, float *__restrict__ out_a,
+                                                                float *__restrict__ out_b, int64_t n_tgt, int64_t ne, int slot_now,
+                                                                const uint4 *__restrict__ any_rel, int n_16, const int32_t *__restrict__ ctrl)
+{
+    extern __shared__ unsigned long long pull_lds[];  // accumulators [wave][step][4][64], stages [wave][128], map
+    bool add_a = false, add_b = false;
+    if (kAuto) {
+        int pulled = 0;
+        for (int r = 0; r < L; ++r) pulled |= ctrl[r];
+        if (!pulled) return;
+        add_a = ctrl[kAutoRows + (slot_now + L - 1) % L] != 0;
+        add_b = ctrl[kAutoRows + slot_now] != 0;
+    }
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
+    constexpr int kWaves = kPullBlock / kWave;
+    unsigned long long *acc = pull_lds + wave * (2 * GLIF3_NREC * kWave);
+    uint2 *stage = reinterpret_cast<uint2 *>(pull_lds + kWaves * 2 * GLIF3_NREC * kWave) + wave * kPairStage;
+    uint4 *any_l = reinterpret_cast<uint4 *>(pull_lds + kWaves * (2 * GLIF3_NREC * kWave + kPairStage));
+    const uint8_t *any_b = reinterpret_cast<const uint8_t *>(any_l);
+    const unsigned lane = (unsigned)lane_id(), uL = (unsigned)L;
+    auto fetch = [&](unsigned long long *dst, const PullBlock &blk) {
+        const bool some = blk.base < blk.p1;
+        const char *__restrict__ src = reinterpret_cast<const char *>(packed) + (some ? (size_t)blk.base * 8u : (size_t)0);
+        const unsigned last = some ? (unsigned)(blk.p1 - blk.base) - 1u : 0u;
+#pragma unroll
+        for (int u = 0; u < kPairChunks; ++u)
+            dst[u] = __builtin_nontemporal_load(
+                reinterpret_cast<const unsigned long long *>(src + min(lane + u * kWave, last) * 8u));
+    };
+    // the workgroup's rows: as many synapses for every workgroup, and its wavefronts take the rows one by one; the activity map
+    // comes into LDS meanwhile
+    __shared__ int share[3];  // first row, past the last, the next one to take
+    if (wave < 2) {
+        const int64_t part = blockIdx.x + wave, nnz = indptr[n_tgt];
+        // (below some 8 M synapses the search for the rows costs more than workgroups of unequal work: 1 M synapses x 64 trials 18.8 / 16.6 us
+        // with and without, 10 M x 48 60.4 / 59.0, 13 M x 64 80.6 / 82.0, 52 M x 64 243 / 249)
+        const int r = part == gridDim.x ? (int)n_tgt : nnz < (8 << 20) ? (int)(n_tgt * part / gridDim.x) : row_from(indptr, (int)n_tgt, nnz * part / gridDim.x);
+        if (lane == 0) {
+            share[wave] = r;
+            if (wave == 0) share[2] = r;
+        }
+    } else {
+        for (int i = (int)threadIdx.x - 2 * kWave; i < n_16; i += kPullBlock - 2 * kWave) any_l[i] = any_rel[i];
+    }
+#pragma unroll
+    for (int r = 0; r < 2 * GLIF3_NREC; ++r) acc[r * kWave + lane] = 0ull;
+    __syncthreads();
+    const int row_end = share[1];
+    RowCursor<kPairChunks> cursor;
+    cursor.start(indptr, &share[2], row_end);
+    PullBlock b0 = cursor.next();
+    if (b0.row >= row_end) return;
+    unsigned long long d0[kPairChunks], d1[kPairChunks];
+    fetch(d0, b0);
+    PullBlock b1 = cursor.next();
+    fetch(d1, b1);
+    // (sums of at least 128 bytes a row are not kept in the L2 that the trials of the sources lie in; shorter pieces of a line are)
+    const bool whole_lines = batch >= 32;
+    int staged = 0;  // entries in the stage (same in all lanes)
+    // Staged synapses, 64 at a time: their trials of both arrival steps are asked for with one fetch, and added to while the next
+    // ones' are on their way.
+    PullPair<Mask> asked{0, 0};
+    unsigned long long *asked_to = nullptr;
+    float asked_w = 0.0f;
+    int asked_n = 0;
+    auto add = [&]() {
+        const unsigned long long w = to_fixed(asked_w);
+        Mask a = (int)lane < asked_n ? asked.a : 0, b = (int)lane < asked_n ? asked.b : 0;  // (not before: it waits for the fetch)
+        while (a | b) {
+            if (a) {
+                atomicAdd(asked_to + (sizeof(Mask) == 8 ? __ffsll((long long)a) : __ffs((int)a)) - 1, w);
+                a &= a - 1;
+            }
+            if (b) {
+                atomicAdd(asked_to + GLIF3_NREC * kWave + (sizeof(Mask) == 8 ? __ffsll((long long)b) : __ffs((int)b)) - 1, w);
+                b &= b - 1;
+            }
+        }
+    };
+    // (the first `n` entries of the stage)
+    auto work_off = [&](int n) {
+        const uint2 e = stage[lane];  // {source | ... | receptor << 24 | delay << 26, weight}
+        PullPair<Mask> m = pair_at(pair, (int)lane < n ? __umul24(e.x & 0xFFFFFFu, uL + 1u) + (e.x >> 26) : 0u);
+        add();
+        asked = m;
+        asked_n = n;
+        asked_to = acc + ((e.x >> 24) & 3u) * kWave;
+        asked_w = __uint_as_float(e.y);
+    };
+    auto work_done = [&]() {
+        add();
+        asked_n = 0;
+    };
+    auto turn = [&](PullBlock &cb, unsigned long long *cd) {
+        const unsigned left = cb.base < cb.p1 ? (unsigned)(cb.p1 - cb.base) : 0u;
+        // bit d of a source's byte = fired d steps before the step whose row is slot_now, which holds step t - L; a synapse of
+        // delay d asks for bit d on behalf of step t and bit d + 1, bit L being bit 0, for t - 1
+        unsigned word[kPairChunks];
+#pragma unroll
+        for (int u = 0; u < kPairChunks; ++u) {
+            const unsigned tdr = (unsigned)cd[u], m = any_b[tdr & 0xFFFFFFu];
+            word[u] = (m | (m << uL)) >> (tdr >> 26);
+        }
+#pragma unroll
+        for (int u = 0; u < kPairChunks; ++u) {
+            const bool hit = lane + u * kWave < left && (word[u] & 3u) != 0u;
+            const unsigned long long who = __ballot(hit);
+            const int n = __popcll(who);
+            if (n == 0) continue;
+            if (hit) stage[staged + lane_prefix(who)] = make_uint2((unsigned)cd[u], (unsigned)(cd[u] >> 32));
+            staged += n;
+            if (staged >= kWave) {
+                work_off(kWave);
+                staged -= kWave;
+                if ((int)lane < staged) stage[lane] = stage[kWave + lane];
+            }
+        }
+        if (cb.last) {
+            work_off(staged);
+            work_done();
+            staged = 0;
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+#pragma unroll
+                for (int r = 0; r < GLIF3_NREC; ++r) {
+                    unsigned long long *cell = acc + (k * GLIF3_NREC + r) * kWave + lane;
+                    if ((int)lane < batch) {
+                        float *out = (k ? out_b : out_a) + (int64_t)r * ne + cb.row * batch + lane;
+                        const float sum = from_fixed(*cell);
+                        if (kAuto && (k ? add_b : add_a))
+                            *out += sum;
+                        else if (whole_lines)
+                            __builtin_nontemporal_store(sum, out);
+                        else
+                            *out = sum;
+                    }
+                    *cell = 0ull;
+                }
+            }
+        }
+        cb = cursor.next();
+        fetch(cd, cb);
+    };
+    do {  // (one way out, after a whole round of the buffers: see pull_kernel)
+        turn(b0, d0);
+        turn(b1, d1);
+    } while (b0.row < row_end);
+}
+
 // bmtk_csr_propagate_auto, first launch: the spikes of step `step` as events, if they are few.  Every workgroup
 // reads the number of active elements and decides the same way; up to cnt_max the elements' rows are walked and
 // their weights pushed into the ring (fp32 atomics), above it nothing happens here and the step is left to the
@@ -430,13 +693,17 @@ __global__ __launch_bounds__(kBlock) void auto_anymap_kernel(const uint64_t *__r
     if ((lane_id() & 31) == 0 && j < (int64_t)n_w32 * 32) any_row[j >> 5] = (uint32_t)(m >> (lane_id() & 32));
 }
 
+// masks of pull_pair_kernel, 64 bits each, up to a boundary of 16 bytes
+constexpr int64_t pair_bytes(int64_t L, int64_t n_src) { return (n_src * (L + 1) * 8 + 15) / 16 * 16; }
+
 }  // namespace bmtk
 
 extern "C" int64_t bmtk_csr_propagate_pull_workspace_bytes(int32_t L, int64_t n_src)
 {
     if (L <= 0 || n_src <= 0) return 0;
     // one bit per (row, source), or one byte per source (the two-step form with up to 8 rows): the larger of the two
-    const int64_t bits = (int64_t)L * ((n_src + 31) / 32) * 4, bytes = (n_src + 15) / 16 * 16;
+    // (and, for that form, the trials of every source and row)
+    const int64_t bits = (int64_t)L * ((n_src + 31) / 32) * 4, bytes = (n_src + 15) / 16 * 16 + (L <= 8 ? bmtk::pair_bytes(L, n_src) : 0);
     return bits > bytes ? bits : bytes;
 }
 
@@ -584,10 +851,65 @@ extern "C" int bmtk_csr_propagate_auto(const int32_t *active, const int32_t *n_a
     return BMTK_OK;
 }
 
+// what arrives in two steps by pull2_pair_kernel; `work` holds pair_bytes(L, n_src) bytes of masks, then one byte per source
+namespace bmtk {
+static int pair_launch(const uint64_t *hist, int64_t hist_stride, int L, int64_t n_src, int batch, const int32_t *indptr, const bmtk_synapse *packed,
+                       float *out_a, float *out_b, int64_t n_tgt, int slot_now, void *work, const int32_t *ctrl, const char *who, hipStream_t st)
+{
+    const int n_16 = (int)((n_src + 15) / 16);
+    uint8_t *any_rel = (uint8_t *)work + pair_bytes(L, n_src);
+    const bool narrow = batch <= 32;
+    const dim3 build((unsigned)((n_src + kBlock - 1) / kBlock));
+    if (narrow)
+        hipLaunchKernelGGL(pull_pair_kernel<uint32_t>, build, dim3(kBlock), 0, st, hist, hist_stride, L, batch, n_src, slot_now, (uint32_t *)work, any_rel, ctrl);
+    else
+        hipLaunchKernelGGL(pull_pair_kernel<unsigned long long>, build, dim3(kBlock), 0, st, hist, hist_stride, L, batch, n_src, slot_now,
+                           (unsigned long long *)work, any_rel, ctrl);
+    int dev = 0;
+    (void)hipGetDevice(&dev);
+    static int cu_count[64];
+    int n_cu = (dev >= 0 && dev < 64) ? cu_count[dev] : 0;
+    if (n_cu <= 0) {
+        n_cu = 256;
+        (void)hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev);
+        if (dev >= 0 && dev < 64) cu_count[dev] = n_cu;
+    }
+    const unsigned rows_per_block = kPullBlock / kWave;
+    const unsigned want = (unsigned)((n_tgt + rows_per_block - 1) / rows_per_block);
+    const void *const kernels[2][2] = {
+        {reinterpret_cast<const void *>(pull2_pair_kernel<unsigned long long, false>), reinterpret_cast<const void *>(pull2_pair_kernel<unsigned long long, true>)},
+        {reinterpret_cast<const void *>(pull2_pair_kernel<uint32_t, false>), reinterpret_cast<const void *>(pull2_pair_kernel<uint32_t, true>)}};
+    const void *kernel = kernels[narrow][ctrl != nullptr];
+    static bool asked[2][2][64];
+    if (dev >= 0 && dev < 64 && !asked[narrow][ctrl != nullptr][dev]) {
+        const hipError_t err = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kPull2LdsMax);
+        if (err != hipSuccess) {
+            set_error("%s: cannot reserve %zu bytes of LDS: %s", who, kPull2LdsMax, hipGetErrorString(err));
+            return BMTK_E_LAUNCH;
+        }
+        asked[narrow][ctrl != nullptr][dev] = true;
+    }
+    const void *pair = work;
+    int L_arg = L, batch_arg = batch, slot = slot_now, n_map = n_16;
+    int64_t tgt = n_tgt, ne = n_tgt * (int64_t)batch;
+    const uint8_t *map = any_rel;
+    void *args[] = {&pair, &L_arg, &batch_arg, &indptr, &packed, &out_a, &out_b, &tgt, &ne, &slot, &map, &n_map, &ctrl};
+    const hipError_t err = hipLaunchKernel(kernel, dim3(want < (unsigned)n_cu ? want : (unsigned)n_cu), dim3(kPullBlock), args,
+                                           (size_t)n_16 * 16 + kPull2AccBytes, st);
+    if (err != hipSuccess) {
+        set_error("%s: launch failed: %s", who, hipGetErrorString(err));
+        return BMTK_E_LAUNCH;
+    }
+    BMTK_CHECK_LAUNCH("pull of two arrival steps");
+    return BMTK_OK;
+}
+}  // namespace bmtk
+
 extern "C" int64_t bmtk_csr_propagate_auto2_workspace_bytes(int32_t L, int64_t n_src)
 {
     if (L <= 0 || n_src <= 0) return 0;
-    return 2 * bmtk::kAutoRows * 4 + (n_src + 15) / 16 * 16;  // the record of pushed steps, then one byte per source
+    // the record of pushed steps, then what pull_pair_kernel lays out and one byte per source
+    return 2 * bmtk::kAutoRows * 4 + bmtk::pair_bytes(L, n_src) + (n_src + 15) / 16 * 16;
 }
 
 extern "C" int bmtk_csr_propagate_auto2(const int32_t *active_a, const int32_t *n_active_a, const int32_t *active_b,
@@ -631,6 +953,9 @@ extern "C" int bmtk_csr_propagate_auto2(const int32_t *active_a, const int32_t *
                            (int)(step % L), (int)scatter_max_active, ctrl, 0);
     }
     int slot_now = (int)((step + 1) % L);  // the row the spikes of step + 1 will take: it holds step + 1 - L
+    if (batch <= kWave)
+        return pair_launch(spike_hist, hist_stride, L, n_src, batch, tgt_indptr, tgt_packed, ring + (int64_t)(step % L) * GLIF3_NREC * ne,
+                           ring + (int64_t)slot_now * GLIF3_NREC * ne, n_tgt, slot_now, any_rel, ctrl, "csr_propagate_auto2", st);
     hipLaunchKernelGGL(pull_anyrel_kernel, dim3((unsigned)((n_src + kBlock - 1) / kBlock)), dim3(kBlock), 0, st, spike_hist,
                        hist_stride, L, batch, n_src, slot_now, any_rel, (const int32_t *)ctrl);
     int dev = 0;
@@ -646,16 +971,15 @@ extern "C" int bmtk_csr_propagate_auto2(const int32_t *active_a, const int32_t *
     const unsigned want = (unsigned)((n_tgt + rows_per_block - 1) / rows_per_block);
     const dim3 grid(want < (unsigned)n_cu ? want : (unsigned)n_cu, (unsigned)((batch + kWave - 1) / kWave));
     BMTK_REQUIRE(grid.y <= 65535, "csr_propagate_auto2: batch too large");
-    const void *kernel = batch == kWave ? reinterpret_cast<const void *>(pull2_kernel<true, true, true>)
-                                        : reinterpret_cast<const void *>(pull2_kernel<false, true, true>);
-    static bool asked[2][64];
-    if (dev >= 0 && dev < 64 && !asked[batch == kWave][dev]) {
+    const void *kernel = reinterpret_cast<const void *>(pull2_kernel<false, true, true>);
+    static bool asked[64];
+    if (dev >= 0 && dev < 64 && !asked[dev]) {
         const hipError_t err = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kPull2LdsMax);
         if (err != hipSuccess) {
             set_error("csr_propagate_auto2: cannot reserve %zu bytes of LDS: %s", kPull2LdsMax, hipGetErrorString(err));
             return BMTK_E_LAUNCH;
         }
-        asked[batch == kWave][dev] = true;
+        asked[dev] = true;
     }
     // what the steps not pushed send to steps `step` and `step + 1`, into (or onto) those steps' ring slots
     float *out_a = ring + (int64_t)(step % L) * GLIF3_NREC * ne, *out_b = ring + (int64_t)slot_now * GLIF3_NREC * ne;
@@ -692,6 +1016,9 @@ extern "C" int bmtk_csr_propagate_pull2(const uint64_t *spike_hist, int64_t hist
     // kernel then asks one question per synapse instead of two), else one bit per row and source
     const int n_16 = (int)((n_src + 15) / 16);
     const bool byte_map = L <= 8 && (size_t)n_16 * 16 + kPull2AccBytes <= kPull2LdsMax;
+    if (byte_map && batch <= kWave)
+        return pair_launch(spike_hist, hist_stride, L, n_src, batch, indptr, packed, syn2, syn2 + GLIF3_NREC * n_tgt * batch, n_tgt,
+                           (int)(t_arrive % L), workspace, nullptr, "csr_propagate_pull2", (hipStream_t)stream);
     const int n_w32 = byte_map ? n_16 : (int)((n_src + 31) / 32);
     const size_t lds = (byte_map ? (size_t)n_16 * 16 : (size_t)L * n_w32 * 4) + kPull2AccBytes;
     BMTK_REQUIRE(lds <= kPull2LdsMax, "csr_propagate_pull2: L * n_src too large for the activity map in LDS");
@@ -718,18 +1045,19 @@ extern "C" int bmtk_csr_propagate_pull2(const uint64_t *spike_hist, int64_t hist
     const unsigned want = (unsigned)((n_tgt + rows_per_block - 1) / rows_per_block);
     const dim3 grid(want < (unsigned)n_cu ? want : (unsigned)n_cu, (unsigned)((batch + kWave - 1) / kWave));
     BMTK_REQUIRE(grid.y <= 65535, "csr_propagate_pull2: batch too large");
-    const void *const kernels[2][2] = {
-        {reinterpret_cast<const void *>(pull2_kernel<false, false, false>), reinterpret_cast<const void *>(pull2_kernel<false, true, false>)},
-        {reinterpret_cast<const void *>(pull2_kernel<true, false, false>), reinterpret_cast<const void *>(pull2_kernel<true, true, false>)}};
-    const void *kernel = kernels[batch == kWave][byte_map];
-    static bool asked[2][2][64];
-    if (dev >= 0 && dev < 64 && !asked[batch == kWave][byte_map][dev]) {
+    // (byte map: batches above 64 only)
+    const int form = byte_map ? 1 : batch == kWave ? 2 : 0;
+    const void *const kernels[3] = {reinterpret_cast<const void *>(pull2_kernel<false, false, false>), reinterpret_cast<const void *>(pull2_kernel<false, true, false>),
+                                    reinterpret_cast<const void *>(pull2_kernel<true, false, false>)};
+    const void *kernel = kernels[form];
+    static bool asked[3][64];
+    if (dev >= 0 && dev < 64 && !asked[form][dev]) {
         const hipError_t err = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kPull2LdsMax);
         if (err != hipSuccess) {
             set_error("csr_propagate_pull2: cannot reserve %zu bytes of LDS: %s", kPull2LdsMax, hipGetErrorString(err));
             return BMTK_E_LAUNCH;
         }
-        asked[batch == kWave][byte_map][dev] = true;
+        asked[form][dev] = true;
     }
     int64_t ne = n_tgt * (int64_t)batch;
     int slot_now = (int)(t_arrive % L), n_map = n_w32;

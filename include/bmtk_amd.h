@@ -143,7 +143,8 @@ typedef struct bmtk_synapse {
  * bits below 2^-32 are dropped.  The cost is one read of the table per step plus one mask fetch per synapse with
  * an active source.  L must exceed the largest delay; L * hist_stride must stay below 2^29 words; the bit map,
  * L * ceil(n_src/32) * 4 bytes, must fit in 40 KB of LDS (n_src <= 54,000 at L = 6).  The workspace size is the
- * larger of that map and n_src bytes rounded up to 16 (the map of bmtk_csr_propagate_pull2). */
+ * larger of that map and, for L <= 8, what bmtk_csr_propagate_pull2 lays out: 8 (L + 1) n_src bytes of trials and n_src
+ * bytes of its map, either rounded up to 16. */
 int64_t bmtk_csr_propagate_pull_workspace_bytes(int32_t L, int64_t n_src);
 int bmtk_csr_propagate_pull(const uint64_t *spike_hist, int64_t hist_stride, int32_t L, int64_t n_src, int32_t batch,
                             const int32_t *indptr, const bmtk_synapse *packed, float *syn, int64_t n_tgt,
@@ -187,7 +188,8 @@ int bmtk_csr_propagate_auto(const int32_t *active, const int32_t *n_active, int6
  * limits as bmtk_csr_propagate_pull, except that the map may take up to 70 KB of LDS.  With L <= 8 and n_src <=
  * 70 KB the map is kept source-major instead, one byte per source whose bit d says "fired d steps before the
  * step whose row t_arrive's spikes will take": one LDS read then answers both questions a synapse asks (6 % faster
- * at 0.2 Hz at 51,978 x batch 64); bmtk_csr_propagate_pull_workspace_bytes covers both forms of the map. */
+ * at 0.2 Hz at 51,978 x batch 64).  For batches of up to 64 the trials themselves are then laid out source by source too,
+ * so that one fetch serves both arrival steps.  bmtk_csr_propagate_pull_workspace_bytes covers all of it. */
 int bmtk_csr_propagate_pull2(const uint64_t *spike_hist, int64_t hist_stride, int32_t L, int64_t n_src, int32_t batch,
                              const int32_t *indptr, const bmtk_synapse *packed, float *syn2, int64_t n_tgt,
                              int64_t t_arrive, void *workspace, void *stream);
@@ -200,8 +202,8 @@ int bmtk_csr_propagate_pull2(const uint64_t *spike_hist, int64_t hist_stride, in
  * `step` and `step + 1`.  After the call ring slots step mod L and (step + 1) mod L hold everything that arrives in
  * those two steps; the caller consumes and clears both before the next call.  L at most 8 (the activity map is one
  * byte per source) and n_src bytes within 70 KB of LDS; workspace of bmtk_csr_propagate_auto2_workspace_bytes bytes,
- * zeroed before the first call.  At 51,978 x batch 64 a pair of steps left to the pull costs one table pass, 116 -
- * 435 us at 0.2 - 20 Hz, against two passes of 100 - 275 us each with the one-step switch. */
+ * zeroed before the first call.  At 51,978 x batch 64 a pair of steps left to the pull costs one table pass, 121 -
+ * 366 us at 0.3 - 20 Hz, against two passes of 100 - 275 us each with the one-step switch. */
 int64_t bmtk_csr_propagate_auto2_workspace_bytes(int32_t L, int64_t n_src);
 int bmtk_csr_propagate_auto2(const int32_t *active_a, const int32_t *n_active_a, const int32_t *active_b,
                              const int32_t *n_active_b, int64_t max_active, const uint64_t *spike_hist,

@@ -248,6 +248,29 @@ def test_two_step_pull_equals_two_pulls(batch, p, n_src, L):
         assert float(one[0].abs().max()) > 0 and not torch.equal(one[0], one[1])
 
 
+@pytest.mark.parametrize("n_tgt,nnz,batch,power", [(3, 4000, 64, 1.0), (5000, 70000, 33, 6.0), (9001, 8500000, 32, 3.0), (40000, 8400000, 8, 8.0)])
+def test_two_step_pull_of_rows_of_very_unequal_length(n_tgt, nnz, batch, power):
+    """Targets drawn as n * x**power: rows from several tenths of the table down to none, empty ones first and last, on either side
+    of the size from which workgroups begin at their share of the synapses.  Equal to two calls of the one-step form, bit for bit."""
+    g = torch.Generator(device="cuda").manual_seed(n_tgt)
+    n_src, L = 700, 6
+    tgt = (torch.rand(nnz, device="cuda", generator=g, dtype=torch.float64) ** power * (n_tgt - 2)).long() + (1 if n_tgt > 3 else 0)
+    src = torch.randint(0, n_src, (nnz,), device="cuda", generator=g)
+    table = ops.SynapseTable.from_edges(tgt, src, torch.randn(nnz, device="cuda", generator=g),
+                                        torch.randint(1, L, (nnz,), device="cuda", generator=g, dtype=torch.uint8),
+                                        torch.randint(0, 4, (nnz,), device="cuda", generator=g, dtype=torch.uint8), n_tgt, n_src)
+    hist = torch.zeros(L, ops.n_words(n_src * batch) + 1, dtype=torch.int64, device="cuda")
+    for row in hist:
+        row[:-1] = to_dev(bits_of((torch.rand(n_src * batch, device="cuda", generator=g) < 0.01).to(torch.uint8).cpu().numpy()))[:row.numel() - 1]
+    one = torch.full((2, 4, n_tgt * batch), 7.0, device="cuda")
+    two = torch.full((2, 4, n_tgt * batch), -3.0, device="cuda")
+    ops.csr_propagate_pull(hist, n_src, table, one[0], n_tgt, batch, 2 * L - 1)
+    ops.csr_propagate_pull(hist, n_src, table, one[1], n_tgt, batch, 2 * L)
+    ops.csr_propagate_pull2(hist, n_src, table, two, n_tgt, batch, 2 * L)
+    # (the one-step pull of step t - 1 reads the row of step t - 1 as that of step t - 1 - L: no delay is that long)
+    assert torch.equal(one, two) and float(two.abs().max()) > 0
+
+
 @pytest.mark.parametrize("batch,L", [(64, 6), (5, 6), (32, 8), (64, 2), (1, 3)])
 def test_two_step_auto_delivery_equals_the_oracle(batch, L):
     """``ops.AutoPropagator2`` (bmtk_csr_propagate_auto2): called every second step, each of the two new steps goes
