@@ -120,16 +120,23 @@ struct StepArgs {
 // per workgroup, 18.1 / 19.5 with two, 24.4 with one; transposing the table on its way into LDS (an integer
 // division per word, one word per load) took 19.8 / 20.2 with four tiles.  By measured bytes the launch then moves
 // 5.95 TB/s where the form with a column per neuron moved 6.15 TB/s on the same machine.
+//
+// While all workgroups of one tile are resident at once (eight on a compute unit: 524,288 elements on 256 of them) there is
+// nothing to share the staging with, and four tiles a workgroup leave compute units idle: 30,011 elements are 30 workgroups.  One tile / four,
+// us: 5,000 elements 3.3 / 5.7, 30,011 3.6 / 6.0, 100,000 4.2 / 6.3, 200,000 5.7 / 7.2, 400,000 8.6 / 9.6, 2^20 24.9 / 22.6.
 constexpr int kStepTiles = 4;
+constexpr int kStepResident = 2048;  // workgroups of 256 threads that 256 compute units hold
 
-template <bool kLdsTable>
+// kTilesOrNone: tiles of a workgroup that stages the class table in LDS; 0: the table is not staged
+template <int kTilesOrNone>
 __global__ __launch_bounds__(kBlock) void glif3_step_kernel(StepArgs a)
 {
     extern __shared__ __align__(16) float step_table[];  // [GLIF3_NPROP][columns] when kLdsTable
-    // with the table in LDS a workgroup takes kStepTiles tiles of 256 elements, so that staging the table is
+    // with the table in LDS a workgroup of a large launch takes kStepTiles tiles of 256 elements, so that staging the table is
     // shared by several tiles.  The state of all tiles is asked for first, before the table is staged: the loads
     // of the tiles travel together, and the staging runs while they are on their way.
-    constexpr int kTiles = kLdsTable ? kStepTiles : 1;
+    constexpr bool kLdsTable = kTilesOrNone > 0;
+    constexpr int kTiles = kLdsTable ? kTilesOrNone : 1;
     Glif3Elem s[kTiles];
     float syn[kTiles][GLIF3_NREC], I[kTiles];
     int64_t e[kTiles], col[kTiles];
@@ -621,11 +628,14 @@ int bmtk_glif3_step_fwd(int64_t n_neurons, int32_t batch, float *V, float *asc, 
     // a class table of up to 48 KB (423 classes) is staged in LDS by every workgroup (sixteen bytes per load: a
     // table that is not 16-byte aligned is read through the caches instead)
     const size_t table_bytes = (size_t)prop_stride * GLIF3_NPROP * sizeof(float);
-    if (class_id && table_bytes <= 48u * 1024u && ((uintptr_t)prop & 15u) == 0)
-        hipLaunchKernelGGL(glif3_step_kernel<true>, dim3((grid + kStepTiles - 1) / kStepTiles), dim3(kBlock), table_bytes,
-                           (hipStream_t)stream, a);
-    else
-        hipLaunchKernelGGL(glif3_step_kernel<false>, dim3(grid), dim3(kBlock), 0, (hipStream_t)stream, a);
+    if (class_id && table_bytes <= 48u * 1024u && ((uintptr_t)prop & 15u) == 0) {
+        if (grid <= kStepResident)
+            hipLaunchKernelGGL(glif3_step_kernel<1>, dim3(grid), dim3(kBlock), table_bytes, (hipStream_t)stream, a);
+        else
+            hipLaunchKernelGGL(glif3_step_kernel<kStepTiles>, dim3((grid + kStepTiles - 1) / kStepTiles), dim3(kBlock), table_bytes,
+                               (hipStream_t)stream, a);
+    } else
+        hipLaunchKernelGGL(glif3_step_kernel<0>, dim3(grid), dim3(kBlock), 0, (hipStream_t)stream, a);
     BMTK_CHECK_LAUNCH("glif3_step_fwd");
     return BMTK_OK;
 }
