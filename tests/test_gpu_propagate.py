@@ -24,6 +24,20 @@ def test_compaction_is_flatnonzero(n, p):
         np.testing.assert_array_equal(ids[:c].cpu().numpy(), want)
 
 
+@pytest.mark.parametrize("n", [1, 64, 65, 4095, 4097, 65535, 65536, 65537, 131071, 131072, 131073])
+@pytest.mark.parametrize("p", [0.0, 0.03, 0.2, 1.0])
+def test_compaction_of_bits_on_either_side_of_one_launch(n, p):
+    """Words of a wavefront's lanes, two words a lane and the size from which two launches take over; bits beyond n are set."""
+    rng = np.random.default_rng(n)
+    z = (rng.random(n) < p).astype(np.uint8)
+    words = np.zeros(ops.n_words(n) + 1, np.uint64)
+    words[:-1] = np.packbits(np.concatenate([z, np.ones(ops.n_words(n) * 64 - n, np.uint8)]), bitorder="little").view(np.uint64)
+    c = ops.SpikeCompactor(n)
+    ids, count = c(to_dev(words.view(np.int64)))
+    assert int(count) == int(z.sum())
+    np.testing.assert_array_equal(ids[:int(count)].cpu().numpy(), np.flatnonzero(z))
+
+
 def test_compaction_other_paths():
     """Flags that do not start on a 16-byte boundary (the packing then goes through the one-flag-per-thread kernel),
     non-zero flags other than 1, and an input beyond the size the fused two-launch form takes."""
