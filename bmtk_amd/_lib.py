@@ -68,7 +68,7 @@ class Glif3Bwd(C.Structure):
 
 
 EVENTS_INCONSISTENT = 1     # BMTK_EVENTS_INCONSISTENT
-ABI_VERSION = 35  # BMTK_AMD_ABI_VERSION of include/bmtk_amd.h that the mirrors above were written for
+ABI_VERSION = 36  # BMTK_AMD_ABI_VERSION of include/bmtk_amd.h that the mirrors above were written for
 
 # name -> (restype, argtypes); every symbol include/bmtk_amd.h declares
 SIGNATURES = {
@@ -86,6 +86,7 @@ SIGNATURES = {
     "bmtk_spikes_compact_noalloc": (c_int32, [c_void_p, c_int64, c_void_p, c_void_p, c_void_p]),
     "bmtk_csr_propagate_scatter": (c_int32, [c_void_p, c_void_p, c_int64, c_int32, c_void_p, c_void_p, c_void_p,
                                              c_void_p, c_void_p, c_void_p, c_int32, c_int64, c_int64, c_void_p]),
+    "bmtk_csr_propagate_scatter_ranges": (c_int32, [c_void_p, c_void_p, c_int32] + [c_void_p] * 6 + [c_int32] * 3 + [c_void_p, c_int32, c_int64, c_int64, c_void_p]),
     "bmtk_csr_propagate_gather": (c_int32, [c_void_p, c_int64, c_int32, c_void_p, c_void_p, c_void_p, c_void_p,
                                             c_void_p, c_void_p, c_int32, c_int64, c_int64, c_void_p]),
     "bmtk_csr_propagate_auto_workspace_bytes": (c_int64, [c_int32, c_int64]),

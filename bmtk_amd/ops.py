@@ -5,6 +5,8 @@ Layout: element e = neuron*batch + trial; state tensors are flat ``[ne]`` or
 ``[k, ne]``; the ring buffer is ``[L, 4, ne]``; spike bits are uint64 words
 stored in int64 tensors of ``ceil(ne/64)+1`` entries.
 """
+import functools
+import math
 from dataclasses import dataclass
 
 import numpy as np
@@ -160,6 +162,25 @@ def spikes_compact(z):
 
 
 BLOCKED_PAD = 16  # BMTK_BLOCKED_PAD of include/bmtk_amd.h
+
+
+@functools.lru_cache(maxsize=256)
+def _range_rows_min(row, ne, ring_slots):
+    """Rows of ``row`` synapses on average from which scatter_ranges_kernel takes less time than an atomic per event (in us, fitted to one
+    MI355X: 5,000 to 200,000 targets, rows of 100 to 500; the two agree within 10 % where the forms cross).  An event's atomic takes
+    48 ps, and so does a line of sixteen cells that a workgroup adds to the ring at the end, once for however many events; a row costs
+    every workgroup a look; cells have to be cleared and gone through."""
+    lines = (ring_slots - 1) * NREC * ne / 16.0
+
+    def gain(rows):
+        events = rows * row
+        return 48e-6 * (events - lines * (1.0 - math.exp(-events / lines))) - (0.8 + 1.45e-5 * ne) - rows * (0.5e-3 + 16e-6 * row)
+    rows = 16
+    while rows < (1 << 24) and gain(rows) <= 0.0:
+        rows *= 1.1
+    return int(rows) if rows < (1 << 24) else 0
+
+
 
 
 @dataclass
@@ -347,6 +368,32 @@ class SynapseTable:
             raise ValueError("synapse table rows are not sorted by index")
         return seg
 
+    RANGES = 256             # workgroups of delivery by target ranges (csr_propagate_scatter), each with
+    RANGE_LDS = 150 << 10    # as many bytes of LDS for its cells
+
+    def range_rows_min(self, n_tgt, batch, ring_slots):
+        """Active elements from which delivery by target ranges is expected to be the faster form, 0: never (cells of a range
+        that do not fit a workgroup, or rows so short that the offsets would outgrow the table)."""
+        span = -(-n_tgt // self.RANGES)
+        if 16 * ring_slots * span * batch > self.RANGE_LDS or self.nnz < max(1, 100 * self.n_rows) or self.delays.dtype != torch.uint8:
+            return 0
+        return _range_rows_min(self.nnz / self.n_rows, n_tgt * batch, ring_slots)
+
+    def ranges(self, n_tgt):
+        """Segment offsets of the rows by ``RANGES`` ranges of targets, or None for a table whose rows are not sorted by index.
+        Made once per table and row bounds (synchronises then; None while a graph is being captured)."""
+        plan = getattr(self, "_ranges", None)
+        if plan is None or plan[0] is not self.indptr or plan[1] != (self.indptr._version, n_tgt):
+            if torch.cuda.is_current_stream_capturing():
+                return None
+            made_of = (self.indptr._version, n_tgt)
+            try:
+                seg = self.segment_offsets(-(-n_tgt // self.RANGES), self.RANGES)
+            except ValueError:
+                seg = None
+            plan = self._ranges = (self.indptr, made_of, seg)
+        return plan[2]
+
     def pointers(self):
         nnz = self.nnz
         return (_p(self.indptr, torch.int32, self.n_rows + 1, "indptr"), _p(self.indices, torch.int32, nnz, "indices"),
@@ -356,13 +403,23 @@ class SynapseTable:
 
 
 def csr_propagate_scatter(active, n_active, table, ring, n_tgt, batch, step, max_active=None):
-    """Event-driven delivery of the active element list through a source-major table."""
+    """Event-driven delivery of the active element list through a source-major table.  Tables whose rows are sorted by index
+    keep offsets of their rows from the first call that could use them on: steps with many events are then delivered by ranges of targets
+    (``SynapseTable.range_rows_min``)."""
     lib = _lib.load()
     L = ring.shape[0]
     if ring.numel() != L * NREC * n_tgt * batch:
         raise ValueError("ring must be [L, 4, n_tgt*batch]")
     if max_active is None:
         max_active = active.numel()
+    rows_min = table.range_rows_min(n_tgt, batch, L)
+    if 0 < rows_min <= max_active:
+        seg = table.ranges(n_tgt)
+        if seg is not None:
+            _lib.check(lib.bmtk_csr_propagate_scatter_ranges(
+                _p(active, torch.int32, None, "active"), _p(n_active, torch.int32, 1, "n_active"), batch, *table.pointers(), _p(seg),
+                -(-n_tgt // table.RANGES), table.RANGES, rows_min, _p(ring, torch.float32), L, n_tgt, int(step), _stream()))
+            return
     _lib.check(lib.bmtk_csr_propagate_scatter(
         _p(active, torch.int32, None, "active"), _p(n_active, torch.int32, 1, "n_active"), max_active, batch,
         *table.pointers(), _p(ring, torch.float32), L, n_tgt, int(step), _stream()))

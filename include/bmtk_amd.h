@@ -49,7 +49,7 @@ extern "C" {
 
 /* Bumped whenever a struct layout or a signature below changes; bmtk_amd_abi_version() returns the value the
  * library was built with. */
-#define BMTK_AMD_ABI_VERSION 35
+#define BMTK_AMD_ABI_VERSION 36
 int bmtk_amd_abi_version(void);
 const char *bmtk_amd_last_error(void);
 /* sizeof(bmtk_glif3_sim) as the library was compiled, for bindings that mirror the struct */
@@ -111,6 +111,16 @@ int bmtk_csr_propagate_scatter(const int32_t *active, const int32_t *n_active, i
                                const int32_t *indptr, const int32_t *indices, const float *weights,
                                const uint8_t *delays, const uint8_t *receptors,
                                float *ring, int32_t L, int64_t n_tgt, int64_t step, void *stream);
+
+/* The same by target ranges for steps with at least rows_min active elements: n_ranges workgroups each own `span` targets, add what
+ * the active rows send there in LDS and add their cells to the ring (atomically) at the end.  seg: bmtk_csr_segment_offsets of the
+ * table with `span` and n_ranges, rows sorted by target; it only says where a range's synapses lie in a row: indices, weights,
+ * delays and receptors are read as they are now (synapses that have left their range are still delivered, one by one), row
+ * bounds must be those that seg was made from.  L * 4 * span * batch cells must fit 150 KB. */
+int bmtk_csr_propagate_scatter_ranges(const int32_t *active, const int32_t *n_active, int32_t batch, const int32_t *indptr,
+                                      const int32_t *indices, const float *weights, const uint8_t *delays,
+                                      const uint8_t *receptors, const uint32_t *seg, int32_t span, int32_t n_ranges,
+                                      int32_t rows_min, float *ring, int32_t L, int64_t n_tgt, int64_t step, void *stream);
 
 /* The same sums taken row by row over the TARGET-MAJOR table from the spike
  * bits of the emitting step: deterministic (each ring cell is updated by one

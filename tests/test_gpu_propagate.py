@@ -233,6 +233,94 @@ def test_pull_matches_oracle(batch, p):
     assert np.abs(want).max() > 0
 
 
+@pytest.mark.parametrize("n,batch,L,k", [(1, 1, 6, 400), (255, 1, 6, 300), (257, 3, 6, 250), (5000, 1, 6, 120), (1023, 8, 2, 150), (70, 1, 63, 200), (30011, 2, 6, 100)])
+def test_delivery_by_target_ranges_equals_the_walk(n, batch, L, k, monkeypatch):
+    """Fewer, as many and more targets than ranges, ranges without targets, several trials, two slots and many: what an atomic per event
+    gives, bit for bit (quarter-pA weights: exact sums in any order), from no active element to all."""
+    rng = np.random.default_rng(n + batch)
+    src, tgt, w, d, r = _edges(rng, n, n, n * k, max_delay=L - 1)
+    w = (np.round(w * 4) / 4).astype(np.float32)
+    table = ops.SynapseTable.from_edges(src, tgt, w, d, r, n, n)
+    if table.nnz < 100 * n or table.range_rows_min(n, batch, L) == 0:
+        pytest.skip("not a table for ranges")
+    seg = table.ranges(n)
+    assert seg is not None and table.ranges(n) is seg
+    from bmtk_amd import _lib
+    start = torch.as_tensor(np.round(rng.normal(0, 10, (L, 4, n * batch)) * 4) / 4, device="cuda", dtype=torch.float32)
+    for share in (0.0, 0.01, 0.2, 1.0):
+        on = np.flatnonzero(rng.random(n * batch) < share).astype(np.int32)
+        ids, count = to_dev(np.concatenate([on, np.full(1, -7, np.int32)])), to_dev(np.array([on.size], np.int32))
+        want, got = start.clone(), start.clone()
+        monkeypatch.setattr(ops.SynapseTable, "range_rows_min", lambda *a: 0)
+        ops.csr_propagate_scatter(ids, count, table, want, n, batch, 13, max_active=n * batch)
+        monkeypatch.undo()
+        for rows_min in (0, 1 << 30):
+            got.copy_(start)
+            _lib.check(_lib.load().bmtk_csr_propagate_scatter_ranges(ids.data_ptr(), count.data_ptr(), batch, *table.pointers(), seg.data_ptr(),
+                                                                     -(-n // 256), 256, rows_min, got.data_ptr(), L, n, 13, ops._stream()))
+            assert torch.equal(want, got), (share, rows_min)
+        got.copy_(start)
+        ops.csr_propagate_scatter(ids, count, table, got, n, batch, 13, max_active=n * batch)
+        assert torch.equal(want, got)
+
+
+def test_delivery_by_target_ranges_follows_a_table_that_is_written_to():
+    """Weights, delays, receptors and targets changed in place behind the offsets; rows whose order is lost; other row bounds; a table
+    that was never sorted: always what an atomic per event gives."""
+    rng = np.random.default_rng(3)
+    n, L, nnz = 600, 6, 600 * 150
+    src, tgt, w, d, r = _edges(rng, n, n, nnz)
+    w = (np.round(w * 4) / 4).astype(np.float32)
+    table = ops.SynapseTable.from_edges(src, tgt, w, d, r, n, n)
+    ids, count = torch.arange(n, device="cuda", dtype=torch.int32), torch.tensor([n], device="cuda", dtype=torch.int32)
+
+    def check(t):
+        want, got = torch.zeros(L, 4, n, device="cuda"), torch.zeros(L, 4, n, device="cuda")
+        from bmtk_amd import _lib
+        _lib.check(_lib.load().bmtk_csr_propagate_scatter(ids.data_ptr(), count.data_ptr(), n, 1, *t.pointers(), want.data_ptr(), L, n, 4, ops._stream()))
+        ops.csr_propagate_scatter(ids, count, t, got, n, 1, 4)
+        assert torch.equal(want, got) and float(want.abs().max()) > 0
+
+    assert 0 < table.range_rows_min(n, 1, L) <= n
+    check(table)
+    seg = table.ranges(n)
+    table.weights.mul_(-2)
+    table.delays.copy_(torch.randint(1, L, (nnz,), device="cuda"))
+    table.receptors.copy_(torch.randint(0, 4, (nnz,), device="cuda"))
+    check(table)
+    table.indices.copy_(torch.randint(0, n, (nnz,), device="cuda"))      # targets leave their ranges, rows are no longer in order
+    check(table)
+    assert table.ranges(n) is seg
+    table.indptr[1:-1] = torch.arange(1, n, device="cuda") * (nnz // n)  # other rows
+    check(table)
+    assert table.ranges(n) is None
+    for order in (torch.arange(nnz - 1, -1, -1, device="cuda"), torch.arange(nnz, device="cuda")):
+        t = ops.SynapseTable.from_edges(src, tgt, w, d, r, n, n)
+        rows = torch.repeat_interleave(torch.arange(n, device="cuda"), (t.indptr[1:] - t.indptr[:-1]).long())
+        by = torch.sort(rows[order], stable=True).indices
+        t.indices, t.weights = t.indices[order][by].contiguous(), t.weights[order][by].contiguous()
+        check(t)
+        assert (t.ranges(n) is None) == (order[0].item() != 0)
+
+
+@pytest.mark.parametrize("span,n_groups", [(7, 30), (64, 4), (1, 211), (300, 1), (100, 2)])
+def test_segment_offsets_are_what_a_search_finds(span, n_groups):
+    """Empty rows, rows of one synapse and of several chunks, repeated targets, targets beyond the last group, first and last groups empty."""
+    rng = np.random.default_rng(span)
+    lens = rng.integers(0, 200, 50)
+    lens[[0, 3, 49]] = 0
+    lens[[1, 4]] = 1, 64
+    indptr = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    idx = np.concatenate([np.sort(rng.integers(0, 211, m)) for m in lens]).astype(np.int32)
+    one = np.ones(idx.size, np.uint8)
+    t = ops.SynapseTable(to_dev(indptr), to_dev(idx), to_dev(one.astype(np.float32)), to_dev(one), to_dev(one), n_rows=50, max_row=200)
+    want = np.stack([indptr[j] + np.searchsorted(idx[indptr[j]:indptr[j + 1]], np.arange(n_groups + 1) * span) for j in range(50)])
+    np.testing.assert_array_equal(t.segment_offsets(span, n_groups).cpu().numpy(), want)
+    t.indices[indptr[-1] - 1] = 0
+    with pytest.raises(ValueError):
+        t.segment_offsets(span, n_groups)
+
+
 @pytest.mark.parametrize("batch,p,n_src,L", [(1, 0.3, 211, 6), (5, 0.2, 211, 6), (32, 0.05, 1500, 6), (64, 0.01, 211, 6),
                                               (64, 0.3, 211, 6), (100, 0.1, 97, 6), (130, 0.05, 211, 6),
                                               (64, 0.05, 211, 2), (32, 0.05, 400, 8), (64, 0.05, 211, 9), (5, 0.2, 300, 14)])
