@@ -181,8 +181,6 @@ def _range_rows_min(row, ne, ring_slots):
     return int(rows) if rows < (1 << 24) else 0
 
 
-
-
 @dataclass
 class SynapseTable:
     """Device copy of a synapse table (see ``bmtk_amd.network``)."""
@@ -377,21 +375,27 @@ class SynapseTable:
         span = -(-n_tgt // self.RANGES)
         if 16 * ring_slots * span * batch > self.RANGE_LDS or self.nnz < max(1, 100 * self.n_rows) or self.delays.dtype != torch.uint8:
             return 0
+        if ring_slots < 2 or n_tgt * batch < 1:   # (refused by the call itself)
+            return 0
         return _range_rows_min(self.nnz / self.n_rows, n_tgt * batch, ring_slots)
 
     def ranges(self, n_tgt):
         """Segment offsets of the rows by ``RANGES`` ranges of targets, or None for a table whose rows are not sorted by index.
-        Made once per table and row bounds (synchronises then; None while a graph is being captured)."""
+        Made once per table and row bounds (synchronises then).  None while a graph is being captured: its replays would read the
+        offsets after other row bounds have replaced them."""
+        if torch.cuda.is_current_stream_capturing():
+            return None
         plan = getattr(self, "_ranges", None)
+        stream = _stream()
         if plan is None or plan[0] is not self.indptr or plan[1] != (self.indptr._version, n_tgt):
-            if torch.cuda.is_current_stream_capturing():
-                return None
             made_of = (self.indptr._version, n_tgt)
             try:
                 seg = self.segment_offsets(-(-n_tgt // self.RANGES), self.RANGES)
             except ValueError:
                 seg = None
-            plan = self._ranges = (self.indptr, made_of, seg)
+            plan = self._ranges = (self.indptr, made_of, seg, stream)
+        elif plan[2] is not None and plan[3] != stream:
+            plan[2].record_stream(torch.cuda.current_stream())   # (replaced offsets are not reused under a launch of another stream)
         return plan[2]
 
     def pointers(self):

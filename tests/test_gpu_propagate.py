@@ -303,6 +303,37 @@ def test_delivery_by_target_ranges_follows_a_table_that_is_written_to():
         assert (t.ranges(n) is None) == (order[0].item() != 0)
 
 
+def test_a_captured_delivery_follows_row_bounds_written_later():
+    """A captured call keeps no offsets: its replays read the row bounds of their own time."""
+    rng = np.random.default_rng(5)
+    n, L, nnz = 600, 6, 600 * 150
+    src, tgt, w, d, r = _edges(rng, n, n, nnz)
+    w = (np.round(w * 4) / 4).astype(np.float32)
+    table = ops.SynapseTable.from_edges(src, tgt, w, d, r, n, n)
+    ids, count = torch.arange(n, device="cuda", dtype=torch.int32), torch.tensor([n], device="cuda", dtype=torch.int32)
+    got, want = torch.zeros(L, 4, n, device="cuda"), torch.zeros(L, 4, n, device="cuda")
+    ops.csr_propagate_scatter(ids, count, table, got, n, 1, 4)
+    assert table.ranges(n) is not None
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got.zero_()
+        ops.csr_propagate_scatter(ids, count, table, got, n, 1, 4)
+    for bounds in (None, torch.arange(1, n, device="cuda") * (nnz // n), torch.arange(1, n, device="cuda") * 3):
+        if bounds is not None:
+            table.indptr[1:-1] = bounds
+        ops.csr_propagate_scatter(ids, count, table, want.zero_(), n, 1, 4)
+        graph.replay()
+        assert torch.equal(want, got)
+    other = torch.cuda.Stream()
+    other.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(other):
+        ops.csr_propagate_scatter(ids, count, table, got.zero_(), n, 1, 4)
+    torch.cuda.current_stream().wait_stream(other)
+    assert torch.equal(want, got)
+    with pytest.raises(RuntimeError):
+        ops.csr_propagate_scatter(ids, count, table, torch.zeros(1, 4, n, device="cuda"), n, 1, 4)
+
+
 @pytest.mark.parametrize("span,n_groups", [(7, 30), (64, 4), (1, 211), (300, 1), (100, 2)])
 def test_segment_offsets_are_what_a_search_finds(span, n_groups):
     """Empty rows, rows of one synapse and of several chunks, repeated targets, targets beyond the last group, first and last groups empty."""
