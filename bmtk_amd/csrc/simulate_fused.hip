@@ -206,6 +206,65 @@ __device__ __forceinline__ unsigned long long input_word(const int64_t *__restri
     return m;
 }
 
+// The same for steps t .. t + n_sub - 1 (at most two) and the 64 words from `w0` on, by a whole wavefront: lane l gets word w0 + l
+// of either step.  `words`: 128 words of LDS of the wavefront's own.  What it costs is trips to memory, on a wavefront whose group
+// waits for it: where the words' events begin is looked for with 64 probes a round, in both steps at once, and the events
+// themselves come 64 at a time.  A bisection per lane and step was up to twice twelve trips, one after
+// the other: 3,001 neurons x 12 trials, 1,000 inputs 14.6 -> 13.9 us a launch (12.2 without input events); 51,978 x 32 the same 187.
+__device__ __forceinline__ void input_words(const int64_t *__restrict__ in_ptr, const int32_t *__restrict__ in_events, int64_t t, int n_sub,
+                                            int w0, int per_word, unsigned long long *words, unsigned long long (&m)[2])
+{
+    const int lane = lane_id();
+    const int64_t id0 = (int64_t)w0 * per_word, id1 = id0 + (int64_t)kWave * per_word;
+    int64_t at[2], to[2], end[2];  // where the words' events begin lies in at .. to
+#pragma unroll
+    for (int sub = 0; sub < 2; ++sub) {
+        at[sub] = in_ptr[sub < n_sub ? t + sub : t];
+        end[sub] = to[sub] = sub < n_sub ? in_ptr[t + sub + 1] : at[sub];
+        words[sub * kWave + lane] = 0ull;
+    }
+    while (at[0] < to[0] || at[1] < to[1]) {
+        int64_t step[2];
+        bool before[2];
+#pragma unroll
+        for (int sub = 0; sub < 2; ++sub) {
+            step[sub] = (to[sub] - at[sub] + kWave - 1) / kWave;
+            const int64_t r = at[sub] + lane * step[sub];
+            before[sub] = r < to[sub] && (int64_t)in_events[r] < id0;
+        }
+#pragma unroll
+        for (int sub = 0; sub < 2; ++sub) {
+            const int n = __popcll(__ballot(before[sub]));
+            if (n == 0) {
+                to[sub] = at[sub];
+            } else {
+                to[sub] = min(to[sub], at[sub] + n * step[sub]);
+                at[sub] += (n - 1) * step[sub] + 1;
+            }
+        }
+    }
+    bool more[2] = {true, true};
+    while (more[0] || more[1]) {
+        int64_t ev[2];
+#pragma unroll
+        for (int sub = 0; sub < 2; ++sub) ev[sub] = more[sub] && at[sub] + lane < end[sub] ? (int64_t)in_events[at[sub] + lane] : id1;
+#pragma unroll
+        for (int sub = 0; sub < 2; ++sub) {
+            const bool here = ev[sub] >= id0 && ev[sub] < id1;
+            if (here) {
+                const unsigned in = (unsigned)(ev[sub] - id0), w = in / (unsigned)per_word;
+                atomicOr(words + sub * kWave + w, 1ull << (in - w * (unsigned)per_word));
+            }
+            more[sub] = __ballot(here) == ~0ull;
+            at[sub] += kWave;
+        }
+    }
+    __builtin_amdgcn_wave_barrier();
+    m[0] = words[lane];
+    m[1] = words[kWave + lane];
+    asm volatile("" : : : "memory");  // (the room is used for something else next)
+}
+
 // kRows: neurons of a group, 64 / batch.  kBytes: the activity map holds one byte per source, bit (t mod 8) = the source
 // fired in some trial of step t -- one LDS read then answers both questions a synapse asks -- which takes histories of
 // at most 8 rows and as many bytes of LDS as there are sources.  Otherwise it holds one bit per 2^shift sources and history row.
@@ -269,8 +328,7 @@ __global__ __launch_bounds__(kFuseBlock) void sim_fused_kernel(bmtk_glif3_sim s,
     const unsigned long long field = batch == 64 ? ~0ull : ((1ull << batch) - 1ull);
     if (wave == kFuseWaves - 1 && (q.in_bits || q.map_write >= 0)) {
         // ---- the workgroup's share of the input events of the launch's steps as bits of their history rows: a
-        //      lane per 64-bit word, which holds the trials of kRows sources; the events of a step are ascending, so a
-        //      word's events are one run of the list, found by bisection.  (Read by later launches.)  The wavefront
+        //      lane per 64-bit word, which holds the trials of kRows sources.  (Read by later launches.)  The wavefront
         //      then takes groups like the others, which have taken a few more meanwhile. ----
         uint8_t *map_new = reinterpret_cast<uint8_t *>(s.fuse_any + (int64_t)max(q.map_write, 0) * q.n_w32);
         // the bits of the map's bytes that belong to the launch's steps
@@ -278,15 +336,15 @@ __global__ __launch_bounds__(kFuseBlock) void sim_fused_kernel(bmtk_glif3_sim s,
         const unsigned step_bits = (q.n_sub > 0 ? step_bit0 : 0u) | (q.n_sub > 1 ? step_bit1 : 0u);
         const int in_word0 = (int)(s.fuse_in_base / kRows);
         const int per_word = kRows * batch;
-        for (int w = bid * kWave + (int)lane; w < q.n_in_words; w += q.n_main * kWave) {
+        for (int w0 = bid * kWave; w0 < q.n_in_words; w0 += q.n_main * kWave) {
             unsigned long long bits[2] = {0ull, 0ull};
-            for (int sub = 0; sub < q.n_sub; ++sub) {
-                if (q.in_bits) {
-                    const int64_t t = q.t0 + sub;
-                    const unsigned long long m = input_word(s.in_ptr, s.in_events, t, w, per_word);
-                    s.work_bits[(t % H) * s.fuse_hist_stride + in_word0 + w] = m;
-                    bits[sub] = m;
-                }
+            const int w = w0 + (int)lane;
+            if (q.in_bits) input_words(s.in_ptr, s.in_events, q.t0, q.n_sub, w0, per_word, reinterpret_cast<unsigned long long *>(stage), bits);
+            if (w >= q.n_in_words) break;
+            if (q.in_bits) {
+#pragma unroll
+                for (int sub = 0; sub < 2; ++sub)
+                    if (sub < q.n_sub) s.work_bits[((q.t0 + sub) % H) * s.fuse_hist_stride + in_word0 + w] = bits[sub];
             }
 #pragma unroll
             for (int f = 0; f < kRows; ++f) {

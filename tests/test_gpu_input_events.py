@@ -99,3 +99,38 @@ def test_tensors_in_host_memory_are_taken_to_the_device(sim):
     assert float(outs[0][1].abs().sum()) > 0
     for a, b in zip(*outs):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("batch", [8, 12, 20, 64])
+@pytest.mark.parametrize("repeats", [False, True])
+def test_input_words_of_the_fused_form(batch, repeats):
+    """Steps with no event, one, a wavefront's load and one more or less, and every id; the first and the last source; several runs of
+    64 words: bit for bit what separate launches deliver."""
+    import torch
+    n_in = 1500
+    ids = n_in * batch
+    counts = [0, 1, 2, 0, 63, 64, 65, 4095, 4096, 4097, ids, ids - 1, 0, 0, 130, 1, 0, 300, 64, 0]
+    cfg = synthetic.small_glif3_network(n=70, n_in=n_in, steps=len(counts), seed=batch, in_fanout=3, batch=batch, in_w_scale=3.0)
+    for key in ("rec_src", "inp_src"):
+        indptr, indices, w, d, r = cfg[key]
+        cfg[key] = (indptr, indices, (np.round(w * 4.0) / 4.0 + np.sign(w) * 0.25).astype(np.float32), d, r)
+    rng = np.random.default_rng(batch)
+    steps = [np.sort(rng.choice(ids, min(c, ids), replace=False)) for c in counts]
+    steps[1][:] = ids - 1
+    steps[15][:] = 0
+    if repeats:
+        for s in steps:
+            s[1::5] = s[:-1:5][:s[1::5].size]
+    ptr = np.concatenate([[0], np.cumsum([s.size for s in steps])]).astype(np.int64)
+    events = np.concatenate(steps).astype(np.int32)
+    outs = []
+    for fused in (True, False):
+        sim = Glif3Simulator(cfg["n"], cfg["par"], cfg["h"], batch=batch, rec=cfg["rec_src"], inp=cfg["inp_src"], class_id=cfg["class_id"],
+                             resident=False, pull=True, fused=fused)
+        assert (sim.fuse_table is not None) == fused
+        sim.set_input_events(ptr, events)
+        bits = torch.cat([sim.raster(sim.run(k)["bits"]) for k in (1, 8, 11)])
+        outs.append((bits, *(getattr(sim.state, k) for k in ("V", "asc", "y1", "y2", "ref"))))
+    assert int(outs[0][0].sum()) > 0
+    for a, b in zip(*outs):
+        assert torch.equal(a, b)
