@@ -68,7 +68,7 @@ class Glif3Bwd(C.Structure):
 
 
 EVENTS_INCONSISTENT = 1     # BMTK_EVENTS_INCONSISTENT
-ABI_VERSION = 36  # BMTK_AMD_ABI_VERSION of include/bmtk_amd.h that the mirrors above were written for
+ABI_VERSION = 37  # BMTK_AMD_ABI_VERSION of include/bmtk_amd.h that the mirrors above were written for
 
 # name -> (restype, argtypes); every symbol include/bmtk_amd.h declares
 SIGNATURES = {
@@ -129,6 +129,7 @@ SIGNATURES = {
     "bmtk_microbench_atomics": (c_int32, [c_void_p, c_int64, c_int32, c_int32, c_int32, c_void_p]),
     "bmtk_microbench_hop": (c_int32, [c_void_p, c_void_p, c_int32, c_int32, c_int32, C.c_uint32, c_void_p]),
     "bmtk_spike_counts": (c_int32, [c_void_p, c_int64, c_int64, c_int64, c_void_p, c_void_p]),
+    "bmtk_rate_mse": (c_int32, [c_void_p, c_int64, c_int32, c_int64, c_void_p, c_int64] + [c_void_p] * 5),
 }
 
 

@@ -23,16 +23,44 @@ def spike_counts(bits, ne):
     return counts
 
 
+def _plain(counts, n_steps, batch, pop_id, targets):
+    """Whether the call is what bmtk_rate_mse takes: its types and layouts on the current device, and nobody who follows the
+    operations (gradients by the targets, tracing, transforms, modes)."""
+    tensors = (counts, pop_id, targets)
+    if any(type(t) is not torch.Tensor or not t.is_cuda or t.get_device() != torch.cuda.current_device() for t in tensors):
+        return False
+    if any(torch._C._functorch.is_functorch_wrapped_tensor(t) or t.is_conj() or t.is_neg() for t in tensors):
+        return False
+    if torch.jit.is_tracing() or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack() or torch.autograd.forward_ad._current_level >= 0:
+        return False
+    return (type(n_steps) is int and n_steps > 0 and type(batch) is int and batch > 0 and counts.dtype == torch.int32 and pop_id.dtype == torch.int64
+            and targets.dtype == torch.float32 and not targets.requires_grad and pop_id.dim() == 1 and targets.dim() == 2
+            and pop_id.numel() > 0 and counts.numel() == pop_id.numel() * batch and targets.shape[0] == batch and targets.shape[1] > 0
+            and counts.is_contiguous() and pop_id.is_contiguous() and targets.is_contiguous())
+
+
 def rate_mse(counts, n_steps, batch, pop_id, targets):
     """MSE between population rates and targets, and its derivative per spike.
 
     counts  int32 [n*batch] spikes per element; pop_id int64 [n] population of
     every neuron; targets float [batch, n_pops] in spikes per neuron per step.
     The rate of population p in trial b is mean over its neurons and steps of z.
-    Returns (loss, dl_dz_const float32 [n*batch])."""
-    dev = counts.device
+    Returns (loss, dl_dz_const float32 [n*batch]).
+
+    Two launches and one look at the device; as array operations (every other form of the arguments) it is some 25 launches,
+    which a training step of a small network waits for."""
     n = pop_id.numel()
     n_pops = targets.shape[1]
+    if _plain(counts, n_steps, batch, pop_id, targets):
+        dev = counts.device
+        work = torch.zeros(n_pops * (batch + 1) + 1, dtype=torch.int64, device=dev)
+        loss, per_spike = torch.empty((), dtype=torch.float32, device=dev), torch.empty(counts.numel(), dtype=torch.float32, device=dev)
+        _lib.check(_lib.load().bmtk_rate_mse(_p(counts), n, batch, n_steps, _p(pop_id), n_pops, _p(targets), _p(work), _p(loss), _p(per_spike),
+                                             _stream()))
+        if work[-1].item():
+            raise RuntimeError("pop_id outside 0..{}".format(n_pops - 1))
+        return loss, per_spike
+    dev = counts.device
     size = torch.bincount(pop_id, minlength=n_pops).to(torch.float32)
     c = counts.view(n, batch).to(torch.float32)
     rate = torch.zeros(n_pops, batch, device=dev).index_add_(0, pop_id, c) / (size.view(-1, 1) * n_steps)

@@ -49,7 +49,7 @@ extern "C" {
 
 /* Bumped whenever a struct layout or a signature below changes; bmtk_amd_abi_version() returns the value the
  * library was built with. */
-#define BMTK_AMD_ABI_VERSION 36
+#define BMTK_AMD_ABI_VERSION 37
 int bmtk_amd_abi_version(void);
 const char *bmtk_amd_last_error(void);
 /* sizeof(bmtk_glif3_sim) as the library was compiled, for bindings that mirror the struct */
@@ -690,6 +690,12 @@ int bmtk_csr_propagate_bwd_blocked_plan(int64_t n_neurons, int32_t batch, int32_
 /* Number of spikes of every element over n_steps rows of spike bits: counts[e] (int32). */
 int bmtk_spike_counts(const uint64_t *spike_bits, int64_t stride, int64_t n_steps, int64_t ne, int32_t *counts,
                       void *stream);
+
+/* Mean square of (rate of population p in trial b - targets[b * n_pops + p]) and its derivative by the spikes of every element
+ * (the same in every step).  A rate is spikes per neuron and step; pop_id: the population of every neuron.  work: n_pops * batch +
+ * n_pops + 1 words, zero; the last is 1 afterwards if some pop_id lies outside 0 .. n_pops - 1 (such neurons are left out). */
+int bmtk_rate_mse(const int32_t *counts, int64_t n_neurons, int32_t batch, int64_t n_steps, const int64_t *pop_id, int64_t n_pops,
+                  const float *targets, int64_t *work, float *loss, float *per_spike, void *stream);
 
 /* ---------------------------------------------------------------------------
  * Three measurements the kernels' design rests on, kept in the library so that they can be repeated

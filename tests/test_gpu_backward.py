@@ -433,3 +433,54 @@ def test_swept_form_equals_the_parts(n, batch, steps, p_conn):
     one.backward(whole, dl_dz=torch.cat(dl))
     for name in ("lam_V", "lam_asc", "lam_y1", "lam_y2"):
         assert torch.equal(getattr(one, name), getattr(swept, name)), name
+
+
+@pytest.mark.parametrize("steps", [1, 15, 16, 17, 33])
+@pytest.mark.parametrize("ne", [1, 64, 65, 1000, 4096])
+def test_spike_counts(ne, steps):
+    words = ops.n_words(ne) + 1
+    g = torch.Generator(device="cuda").manual_seed(ne + steps)
+    bits = torch.randint(-2**62, 2**62, (steps, words), device="cuda", generator=g) * 3
+    want = ((bits.unsqueeze(-1) >> torch.arange(64, device="cuda")) & 1).flatten(1)[:, :ne].sum(0)
+    assert torch.equal(training.spike_counts(bits, ne), want.to(torch.int32))
+
+
+@pytest.mark.parametrize("n,batch,n_pops", [(1, 1, 1), (300, 12, 17), (257, 5, 1), (1000, 64, 63), (1000, 64, 64), (5000, 3, 4096), (3, 4, 40)])
+def test_rate_loss_matches_64_bits(n, batch, n_pops):
+    """Sums in LDS and beyond, populations without a neuron (no rate: the loss is no number, the others' derivatives are).  Two fp32
+    divisions and a difference after exact sums: some units in the last place of rate and target."""
+    rng = np.random.default_rng(n)
+    counts = rng.poisson(3.0, (n, batch)).astype(np.int32)
+    pop = rng.permutation(np.concatenate([np.arange(min(n, n_pops)), rng.integers(0, n_pops, max(0, n - n_pops))]))
+    targets = rng.uniform(0, 0.05, (batch, n_pops)).astype(np.float32)
+    args = (torch.as_tensor(counts, device="cuda").view(-1), 200, batch, torch.as_tensor(pop, device="cuda"), torch.as_tensor(targets, device="cuda"))
+    assert training._plain(*args)
+    loss, g = training.rate_mse(*args)
+    size = np.bincount(pop, minlength=n_pops).astype(np.float64)
+    total = np.zeros((n_pops, batch))
+    np.add.at(total, pop, counts)
+    with np.errstate(all="ignore"):
+        err = (total / (size[:, None] * 200)).T - targets
+        want = 2 * err / (batch * n_pops) / (size * 200)
+    assert loss.shape == () and loss.dtype == g.dtype == torch.float32
+    if size.min() > 0:
+        assert float(loss) == pytest.approx((err ** 2).mean(), rel=1e-6)
+    else:
+        assert np.isnan(float(loss))
+    scale = 2 * 0.2 / (batch * n_pops) / (size * 200)   # (of a derivative: rates and targets stay below 0.2)
+    np.testing.assert_array_less(np.abs(g.cpu().numpy().reshape(n, batch) - want.T[pop]) / scale[pop][:, None], 4 * 2.0 ** -23)
+    # what the kernel does not take goes the general way, with the same result
+    for other in ((args[0].long(), *args[1:]), (args[0], 200.0, *args[2:]), (*args[:4], args[4].t().contiguous().t()), (*args[:4], args[4].clone().requires_grad_())):
+        assert not training._plain(*other) or other[4].is_contiguous()
+        if size.min() > 0:
+            loss2, g2 = training.rate_mse(*other)
+            assert float(loss2) == pytest.approx(float(loss), rel=1e-6)
+            assert loss2.requires_grad == other[4].requires_grad
+            np.testing.assert_allclose(g2.detach().cpu().numpy(), g.cpu().numpy(), rtol=1e-4, atol=float(scale[size > 0].max()) * 1e-6)
+
+
+def test_rate_loss_refuses_populations_that_do_not_exist():
+    counts, targets = torch.ones(8, dtype=torch.int32, device="cuda"), torch.zeros(2, 3, device="cuda")
+    for bad in (-1, 3, 1 << 40):
+        with pytest.raises(RuntimeError):
+            training.rate_mse(counts, 10, 2, torch.tensor([0, 1, bad, 2], device="cuda"), targets)
