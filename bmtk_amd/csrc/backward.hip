@@ -1089,6 +1089,12 @@ struct SweepElem {
 // read the slots t .. t+L-1, others write slots t-1 and t-2.  Slot s holds psc0 times the adjoint of y1 before step s is
 // undone; slot t was written by the launch before (bwd_seed_slot_kernel at the start of a call).
 //
+// No array of the kernel is indexed at run time: a choice of one of four trials' values by the lane's place made the sums and potentials an array
+// in scratch memory, whose stores waited for the loads (and the records asked for before them) ahead of the first turn.  us per two
+// steps, with scratch / without: 3001 x 12, in-degree 200: 19.6 / 16.2; 3001 x 32, 100: 25.1 / 18.0; 20000 x 16, 150: 114.5 / 92.6; 12000 x 32, 120: 85.3 / 66.7;
+// 12000 x 12, 400: 92.5 / 89.0; 14000 x 16, 200: 71.3 / 71.7.  Tried: eight synapses in flight for rows of a wavefront's own (1800 x 32, 600: 29.8 -> 26.5, but
+// 3001 x 4, 200: 12.5 -> 15.2, spilled registers), two turns in flight (spilled registers: 17 to 18.5 against 16.2).
+//
 // Per step, gather and state adjoint as launches of their own against this form: 3001 neurons x batch 12, in-degree 200:
 // 21.8 -> 10.2 us; 6920 x 16, in-degree 525: 56 -> 33; 30000 x 16, in-degree 300: 194 -> 124.  What bounds it: at the smallest sizes the chain
 // row bounds -> records -> adjoint rows -> state (a launch starts with cold L2s, 1 to 2.5 us a link), above some 5,000 rows
@@ -1275,12 +1281,14 @@ __global__ __launch_bounds__(kSweepThreads, kSweepPerCu) void bwd_sweep_kernel(b
                 sum[s].w += __shfl_xor(sum[s].w, off, kWave);
             }
         auto undo = [&](int c) {
+            // (of values: a choice between members of a struct became a place in scratch memory, whose stores waited for the loads)
+            auto pick = [c](float x0, float x1, float x2, float x3) { return c == 0 ? x0 : c == 1 ? x1 : c == 2 ? x2 : x3; };
             float g[2] = {0.0f, 0.0f}, v[2] = {0.0f, 0.0f};
             unsigned f[2] = {0u, 0u};
 #pragma unroll
             for (int s = 0; s < kSteps; ++s) {
-                g[s] = c == 0 ? sum[s].x : c == 1 ? sum[s].y : c == 2 ? sum[s].z : sum[s].w;
-                v[s] = c == 0 ? v4[s].x : c == 1 ? v4[s].y : c == 2 ? v4[s].z : v4[s].w;
+                g[s] = pick(sum[s].x, sum[s].y, sum[s].z, sum[s].w);
+                v[s] = pick(v4[s].x, v4[s].y, v4[s].z, v4[s].w);
                 f[s] = (f4[s] >> (8 * c)) & 0xFFu;
             }
             el.undo(a, q, pr, e4 + c, ne, g, v, f);
