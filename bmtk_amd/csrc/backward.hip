@@ -12,6 +12,7 @@ struct BwdStep {
     int64_t t;    // absolute step being differentiated
     int64_t row;  // its row in the forward record
     int parts;    // partial sums gz[parts][ne] that the transposed propagation left (1, or 8 from the blocked form)
+    int slot;     // t % ring_slots (divided on the host: a 64-bit remainder is 150 scalar instructions, one after the other)
 };
 
 __device__ __forceinline__ float surrogate(float U, float th, float dampening)
@@ -73,7 +74,7 @@ __global__ __launch_bounds__(kBlock) void bwd_gather_kernel(bmtk_glif3_bwd a, Bw
         if (lane_on && sub == 0) a.gz[e] = 0.0f;
         return;
     }
-    const int slot0 = (int)(q.t % L);
+    const int slot0 = q.slot;
     const int p0 = a.rec_indptr[j], p1 = a.rec_indptr[j + 1];
     const uint2 *__restrict__ rows = reinterpret_cast<const uint2 *>(a.rec_packed);
     const float *__restrict__ ring = a.lam_ring + tile0 + b;
@@ -149,7 +150,7 @@ __global__ __launch_bounds__(kBlock) void bwd_gather4_kernel(bmtk_glif3_bwd a, B
         if (lane_on && sub == 0) *reinterpret_cast<float4 *>(a.gz + e) = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         return;
     }
-    const int slot0 = (int)(q.t % L);
+    const int slot0 = q.slot;
     const int p0 = a.rec_indptr[j], p1 = a.rec_indptr[j + 1];
     const uint2 *__restrict__ rows = reinterpret_cast<const uint2 *>(a.rec_packed);
     const float *__restrict__ ring = a.lam_ring + b4;
@@ -254,7 +255,7 @@ __global__ __launch_bounds__(kBlkThreads) void bwd_gather_blocked_kernel(bmtk_gl
     // delay*4 + receptor, so (slot0 + delay) % L * 4 + receptor = min(u, u - 4L) with u = slot0*4 + that byte
     const char *__restrict__ ring = reinterpret_cast<const char *>(a.lam_ring);
     const unsigned lane_off = (unsigned)b4 * 4u;
-    const unsigned q_lo = (unsigned)(q.t % L) * 4u, q_wrap = q_lo - 4u * (unsigned)L;
+    const unsigned q_lo = (unsigned)q.slot * 4u, q_wrap = q_lo - 4u * (unsigned)L;
     const unsigned ne32 = (unsigned)ne, batch32 = (unsigned)batch;
     auto cell_off = [&](unsigned tdr) -> unsigned {
         const unsigned dq = tdr >> 24;
@@ -564,7 +565,7 @@ __global__ __launch_bounds__(kBlkThreads) void bwd_gather_blocked2_kernel(bmtk_g
     const uint2 *__restrict__ rows = reinterpret_cast<const uint2 *>(a.blk_packed);
     const char *__restrict__ ring = reinterpret_cast<const char *>(a.lam_ring);
     const unsigned lane_off = (unsigned)(lane_on ? b4 : 0) * 4u;  // (lanes without a trial read what the row's first lane reads)
-    const unsigned q_lo = (unsigned)(q.t % L) * 4u, q_wrap = q_lo - 4u * (unsigned)L;
+    const unsigned q_lo = (unsigned)q.slot * 4u, q_wrap = q_lo - 4u * (unsigned)L;
     const unsigned ne32 = (unsigned)ne, batch32 = (unsigned)batch;
     // from a synapse's cell for step t to its cell for step t-1: one slot down, or L-1 slots up from slot 0 (bytes)
     const unsigned slot_down = 0u - 16u * ne32, slot_up = 16u * ne32 * (unsigned)(L - 1);
@@ -965,7 +966,7 @@ __device__ __forceinline__ void bwd_state_block(const bmtk_glif3_bwd &a, const B
         l1[k] = a.lam_y1[k * ne + e];
         l2[k] = a.lam_y2[k * ne + e];
     }
-    float *slot = a.lam_ring + (int64_t)(q.t % a.ring_slots) * GLIF3_NREC * ne + e;
+    float *slot = a.lam_ring + (int64_t)q.slot * GLIF3_NREC * ne + e;
 #pragma unroll
     for (int k = 0; k < GLIF3_NREC; ++k) slot[k * ne] = p.psc0[k] * l1[k];
     const float sg = (f & BMTK_F_INTEGRATING) ? spike_adjoint(a, p, q.row, e, ne, 0, q.parts) : 0.0f;
@@ -1008,12 +1009,13 @@ __global__ __launch_bounds__(kBlock) void bwd_state2_kernel(bmtk_glif3_bwd a, Bw
     const float sg_t = (f_t & BMTK_F_INTEGRATING) ? spike_adjoint(a, p, q.row, e, ne, 0, 8) : 0.0f;
     const float sg_p = (f_p & BMTK_F_INTEGRATING) ? spike_adjoint(a, p, q.row - 1, e, ne, 8, 8) : 0.0f;
     state_adjoint_step(lV, lA, l1, l2, p, a.h, f_t, sg_t);
-    float *slot = a.lam_ring + (int64_t)((q.t - 1) % L) * GLIF3_NREC * ne + e;
+    const int before = q.slot == 0 ? L - 1 : q.slot - 1;
+    float *slot = a.lam_ring + (int64_t)before * GLIF3_NREC * ne + e;
 #pragma unroll
     for (int k = 0; k < GLIF3_NREC; ++k) slot[k * ne] = p.psc0[k] * l1[k];
     state_adjoint_step(lV, lA, l1, l2, p, a.h, f_p, sg_p);
     if (write_after) {
-        slot = a.lam_ring + (int64_t)((q.t + L - 2) % L) * GLIF3_NREC * ne + e;
+        slot = a.lam_ring + (int64_t)(before == 0 ? L - 1 : before - 1) * GLIF3_NREC * ne + e;
 #pragma unroll
         for (int k = 0; k < GLIF3_NREC; ++k) slot[k * ne] = p.psc0[k] * l1[k];
     }
@@ -1051,7 +1053,7 @@ struct SweepElem {
                                          const float (&g)[2], const float (&v)[2], const unsigned (&f)[2])
     {
         const int L = a.ring_slots;
-        int slot = (int)(q.t % L);
+        int slot = q.slot;
 #pragma unroll
         for (int s = 0; s < (kTwo ? 2 : 1); ++s) {
             float gs = g[s];
@@ -1139,7 +1141,7 @@ __global__ __launch_bounds__(kSweepThreads, kSweepPerCu) void bwd_sweep_kernel(b
     const uint2 *__restrict__ rows = reinterpret_cast<const uint2 *>(a.rec_packed);
     const char *__restrict__ ring = reinterpret_cast<const char *>(a.lam_ring);
     const unsigned lane_off = (unsigned)(lane_on ? b4 : 0) * 4u;
-    const unsigned q_lo = (unsigned)(q.t % L) * 4u, q_wrap = q_lo - 4u * (unsigned)L;
+    const unsigned q_lo = (unsigned)q.slot * 4u, q_wrap = q_lo - 4u * (unsigned)L;
     const unsigned ne32 = (unsigned)ne, batch32 = (unsigned)batch;
     // from a synapse's cell for step t to its cell for step t-1: one slot down, or L-1 slots up from slot 0 (bytes)
     const unsigned slot_down = 0u - 16u * ne32, slot_up = 16u * ne32 * (unsigned)(L - 1);
@@ -1333,7 +1335,7 @@ __global__ __launch_bounds__(kBlock) void bwd_rec_grad_kernel(bmtk_glif3_bwd a, 
     const int64_t j = (int64_t)blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave;
     if (j >= a.n_neurons) return;
     const uint64_t *__restrict__ bits = a.spike_bits + q.row * a.spike_bits_stride;
-    const int slot0 = (int)(q.t % L);
+    const int slot0 = q.slot;
     const int p0 = a.rec_indptr[j], p1 = a.rec_indptr[j + 1];
     const uint2 *__restrict__ rows = reinterpret_cast<const uint2 *>(a.rec_packed);
     for (int tile0 = 0; tile0 < batch; tile0 += kWave) {
@@ -1424,7 +1426,7 @@ __device__ __forceinline__ void inp_grad_row(const bmtk_glif3_bwd &a, int j, int
 __device__ __forceinline__ void bwd_inp_grad_waves(const bmtk_glif3_bwd &a, const BwdStep &q, int wave, int n_waves)
 {
     const int batch = a.batch;
-    const int slot0 = (int)(q.t % a.ring_slots);
+    const int slot0 = q.slot;
     const int64_t k0 = a.in_ptr[q.t], k1 = a.in_ptr[q.t + 1];
     for (int64_t k = k0 + wave; k < k1; k += n_waves) {
         const int j = event_source(a.in_events[k], batch);
@@ -1481,7 +1483,7 @@ __device__ __forceinline__ void bwd_inp_grad2_waves(const bmtk_glif3_bwd &a, con
 {
     const int batch = a.batch;
     const int L = a.ring_slots;
-    const int slot_t = (int)(q.t % L), slot_p = (int)((q.t - 1) % L);
+    const int slot_t = q.slot, slot_p = q.slot == 0 ? L - 1 : q.slot - 1;
     const int64_t k0 = a.in_ptr[q.t], k1 = a.in_ptr[q.t + 1];
     const int64_t m0 = a.in_ptr[q.t - 1], m1 = k0;  // (in_ptr[t-1] .. in_ptr[t]: the events of step t-1)
     for (int64_t k = k0 + wave; k < k1; k += n_waves) {
@@ -1901,7 +1903,7 @@ extern "C" int bmtk_glif3_simulate_bwd(const bmtk_glif3_bwd *bwd, int64_t step0,
             hipLaunchKernelGGL(bwd_seed_slot_kernel, dim3(elem_grid), dim3(kBlock), 0, st, a, (int)((step0 + k_top) % a.ring_slots));
         while (k_top >= 0) {
             const bool two = k_top >= 1;
-            rc = sweep_launch(a, sp, BwdStep{step0 + k_top, k_top, 1}, two, st);
+            rc = sweep_launch(a, sp, BwdStep{step0 + k_top, k_top, 1, (int)((step0 + k_top) % a.ring_slots)}, two, st);
             if (rc != BMTK_OK) return rc;
             k_top -= two ? 2 : 1;
         }
@@ -1914,11 +1916,11 @@ extern "C" int bmtk_glif3_simulate_bwd(const bmtk_glif3_bwd *bwd, int64_t step0,
     if (blocked && a.gz_planes >= 16 && pl.lp >= 8 && n_steps >= 2) {
         hipLaunchKernelGGL(bwd_seed_slot_kernel, dim3(elem_grid), dim3(kBlock), 0, st, a, (int)((step0 + k_top) % a.ring_slots));
         for (; k_top >= 1; k_top -= 2) {
-            BwdStep q{step0 + k_top, k_top, 8};
+            BwdStep q{step0 + k_top, k_top, 8, (int)((step0 + k_top) % a.ring_slots)};
             const int rc = blocked2_launch(a, q, pl, a.d_blk_w != nullptr, inp_grad, st);
             if (rc != BMTK_OK) return rc;
             if (a.d_rec_w && !a.d_blk_w) {  // (before the state adjoint, which overwrites a slot step t-1's gradient reads)
-                const BwdStep before{q.t - 1, q.row - 1, 8};
+                const BwdStep before{q.t - 1, q.row - 1, 8, (int)((q.t - 1) % a.ring_slots)};
                 hipLaunchKernelGGL(bwd_rec_grad_kernel, dim3(rows_grid), dim3(kBlock), 0, st, a, q);
                 hipLaunchKernelGGL(bwd_rec_grad_kernel, dim3(rows_grid), dim3(kBlock), 0, st, a, before);
             }
@@ -1926,7 +1928,7 @@ extern "C" int bmtk_glif3_simulate_bwd(const bmtk_glif3_bwd *bwd, int64_t step0,
         }
     }
     for (int64_t k = k_top; k >= 0; --k) {
-        BwdStep q{step0 + k, k, blocked ? 8 : 1};
+        BwdStep q{step0 + k, k, blocked ? 8 : 1, (int)((step0 + k) % a.ring_slots)};
         // The recurrent weight gradient of step t reads the adjoint slots t+1 .. t+L-1, which the state adjoint of
         // this step (it writes slot t) leaves alone: it can ride along with the transposed propagation, which
         // reads the same slots before the state adjoint runs.  Batches of more than one tile keep the kernel of
@@ -1964,7 +1966,7 @@ extern "C" int bmtk_glif3_step_bwd(const bmtk_glif3_bwd *bwd, int64_t step0, int
     BMTK_REQUIRE(gz_parts == 1 || gz_parts == 8, "glif3_step_bwd: gz holds 1 sum or 8 partial sums per element");
     const bmtk_glif3_bwd &a = *bwd;
     const int64_t ne = a.n_neurons * (int64_t)a.batch;
-    BwdStep q{step0 + k, k, gz_parts};
+    BwdStep q{step0 + k, k, gz_parts, (int)((step0 + k) % a.ring_slots)};
     hipLaunchKernelGGL(bwd_state_kernel, dim3((unsigned)((ne + kBlock - 1) / kBlock)), dim3(kBlock), 0,
                        (hipStream_t)stream, a, q, 0);
     BMTK_CHECK_LAUNCH("glif3_step_bwd");
@@ -1978,7 +1980,7 @@ extern "C" int bmtk_csr_weight_grad(const bmtk_glif3_bwd *bwd, int64_t step0, in
     BMTK_REQUIRE(step0 >= 0 && k >= 0, "csr_weight_grad: step0 and k must be non-negative");
     const bmtk_glif3_bwd &a = *bwd;
     BMTK_REQUIRE(a.d_rec_w || a.d_inp_w, "csr_weight_grad: neither d_rec_w nor d_inp_w is given");
-    BwdStep q{step0 + k, k, 1};
+    BwdStep q{step0 + k, k, 1, (int)((step0 + k) % a.ring_slots)};
     if (a.d_rec_w)
         hipLaunchKernelGGL(bwd_rec_grad_kernel, dim3((unsigned)((a.n_neurons + kBlock / kWave - 1) / (kBlock / kWave))),
                            dim3(kBlock), 0, (hipStream_t)stream, a, q);
@@ -2007,7 +2009,7 @@ extern "C" int bmtk_csr_propagate_bwd(const int32_t *indptr, const bmtk_synapse 
     a.rec_packed = packed;
     a.lam_ring = const_cast<float *>(lam_ring);
     a.gz = gz;
-    BwdStep q{step, 0, 1};
+    BwdStep q{step, 0, 1, (int)(step % L)};
     const unsigned rows_grid = (unsigned)((n_neurons + kBlock / kWave - 1) / (kBlock / kWave));
     int bp = 1;
     while (bp < batch && bp < kWave) bp <<= 1;
@@ -2042,7 +2044,7 @@ extern "C" int bmtk_csr_propagate_bwd_blocked(const int32_t *blk_indptr, const b
     int rc = blocked_check(a, "csr_propagate_bwd_blocked");
     if (rc == BMTK_OK) rc = blocked_plan(a, pl);
     if (rc != BMTK_OK) return rc;
-    BwdStep q{step, 0, 8};
+    BwdStep q{step, 0, 8, (int)(step % a.ring_slots)};
     rc = blocked_launch(a, q, pl, false, false, (hipStream_t)stream);
     if (rc != BMTK_OK) return rc;
     BMTK_CHECK_LAUNCH("csr_propagate_bwd_blocked");

@@ -72,6 +72,9 @@ struct FusedLaunch {
     int repeats;         // the repeated ids of the launch's steps are delivered as events
     int H;               // rows of the history (L + 4)
     int Lr;              // slots of the ring (L + 2)
+    // (divisions are the host's: a 64-bit remainder is 150 scalar instructions, and a group's closing work needed four)
+    int hist_row[3];     // history rows of steps t0-1, t0, t0+1
+    int ring_slot[3];    // ring slots of steps t0-1, t0, t0+1
     int n_w32;           // words per row of the activity map of bits; words of one map of bytes
     int shift;           // sources per bit of the activity map: 2^shift
     int team;            // wavefronts that share a group (1: every wavefront takes groups of its own from the workgroup's counter)
@@ -300,7 +303,9 @@ __global__ __launch_bounds__(kFuseBlock) void sim_fused_kernel(bmtk_glif3_sim s,
     if (!kBytes) {
         // the activity rows of the steps the NEXT launch writes start empty (no launch reads them before)
         for (int k = 0; k < 2; ++k) {
-            uint32_t *__restrict__ next = s.fuse_any + ((q.t0 + q.n_sub + k) % H) * q.n_w32;
+            int row = q.hist_row[1] + q.n_sub + k;
+            row = row >= H ? row - H : row;
+            uint32_t *__restrict__ next = s.fuse_any + (int64_t)row * q.n_w32;
             for (int i = bid * kFuseBlock + (int)threadIdx.x; i < q.n_w32; i += q.n_main * kFuseBlock) next[i] = 0u;
         }
     }
@@ -317,8 +322,8 @@ __global__ __launch_bounds__(kFuseBlock) void sim_fused_kernel(bmtk_glif3_sim s,
         } else {
             // the activity maps of the steps t0-1 .. t0-L, one after the other
             for (int k = 0; k < L; ++k) {
-                const int64_t u = q.t0 - 1 - k;
-                const uint32_t *__restrict__ src = s.fuse_any + (((u % H) + H) % H) * q.n_w32;
+                const int row = q.hist_row[0] - k;
+                const uint32_t *__restrict__ src = s.fuse_any + (int64_t)(row < 0 ? row + H : row) * q.n_w32;
                 for (int i = threadIdx.x; i < q.n_w32; i += kFuseBlock) any_l[k * q.n_w32 + i] = src[i];
             }
         }
@@ -344,7 +349,7 @@ __global__ __launch_bounds__(kFuseBlock) void sim_fused_kernel(bmtk_glif3_sim s,
             if (q.in_bits) {
 #pragma unroll
                 for (int sub = 0; sub < 2; ++sub)
-                    if (sub < q.n_sub) s.work_bits[((q.t0 + sub) % H) * s.fuse_hist_stride + in_word0 + w] = bits[sub];
+                    if (sub < q.n_sub) s.work_bits[(int64_t)q.hist_row[1 + sub] * s.fuse_hist_stride + in_word0 + w] = bits[sub];
             }
 #pragma unroll
             for (int f = 0; f < kRows; ++f) {
@@ -355,8 +360,8 @@ __global__ __launch_bounds__(kFuseBlock) void sim_fused_kernel(bmtk_glif3_sim s,
                         map_new[source] = (uint8_t)((map_old[source] & ~step_bits) | (on0 ? step_bit0 : 0u) | (on1 ? step_bit1 : 0u));
                 } else {
                     const unsigned g = (unsigned)source >> q.shift;
-                    if (on0) atomicOr(s.fuse_any + (q.t0 % H) * q.n_w32 + (g >> 5), 1u << (g & 31u));
-                    if (on1) atomicOr(s.fuse_any + ((q.t0 + 1) % H) * q.n_w32 + (g >> 5), 1u << (g & 31u));
+                    if (on0) atomicOr(s.fuse_any + (int64_t)q.hist_row[1] * q.n_w32 + (g >> 5), 1u << (g & 31u));
+                    if (on1) atomicOr(s.fuse_any + (int64_t)q.hist_row[2] * q.n_w32 + (g >> 5), 1u << (g & 31u));
                 }
             }
         }
@@ -378,7 +383,8 @@ __global__ __launch_bounds__(kFuseBlock) void sim_fused_kernel(bmtk_glif3_sim s,
                 const int p1 = s.inp_indptr[j + 1];
                 for (int p = s.inp_indptr[j] + (int)lane; p < p1; p += kWave) {
                     const uint2 sy = rows[p];
-                    const int slot = (int)((t + (int64_t)(sy.x >> 26)) % q.Lr);
+                    int slot = q.ring_slot[1 + sub] + (int)(sy.x >> 26);  // (delays are below L, Lr is L + 2)
+                    slot = slot >= q.Lr ? slot - q.Lr : slot;
                     const int64_t i = sy.x & 0xFFFFFFu;
                     atomicAdd(s.ring + ((int64_t)(slot * GLIF3_NREC + (int)((sy.x >> 24) & 3u)) * ne + i * batch + b),
                               __uint_as_float(sy.y));
@@ -414,8 +420,8 @@ __global__ __launch_bounds__(kFuseBlock) void sim_fused_kernel(bmtk_glif3_sim s,
     // once, where the two ways meet again.
     // ring map: bit i of row (u % Lr) = some ring cell of neuron i in slot u % Lr holds an arrival (set where
     // repeated ids are delivered, cleared by the neuron's owner when it takes the cells along); behind the activity map
-    auto ring_row = [&](FuseArgs sp, FuseLaunchArgs qp, int64_t step) -> uint32_t * {
-        return in_memory(sp->fuse_any) + (kBytes ? 2 : (int64_t)qp->H) * qp->n_w32 + ((step % qp->Lr + qp->Lr) % qp->Lr) * ((n + 31) >> 5);
+    auto ring_row = [&](FuseArgs sp, FuseLaunchArgs qp, int slot) -> uint32_t * {
+        return in_memory(sp->fuse_any) + (kBytes ? 2 : (int64_t)qp->H) * qp->n_w32 + (int64_t)slot * ((n + 31) >> 5);
     };
     auto load_group = [&](int grp) {
         const FuseArgs sp = fresh_args();
@@ -426,8 +432,8 @@ __global__ __launch_bounds__(kFuseBlock) void sim_fused_kernel(bmtk_glif3_sim s,
         const int64_t col = sp->class_id ? (int64_t)in_memory(sp->class_id)[row] : (int64_t)row;
         pr.load(in_memory(sp->prop), sp->prop_stride, col);
         if (qp->use_ring) {
-            ring_word0 = ring_row(sp, qp, qp->t0 - 1)[row >> 5];
-            ring_word1 = ring_row(sp, qp, qp->t0)[row >> 5];
+            ring_word0 = ring_row(sp, qp, qp->ring_slot[0])[row >> 5];
+            ring_word1 = ring_row(sp, qp, qp->ring_slot[1])[row >> 5];
         }
         if (kBytes) byte_old = reinterpret_cast<const uint8_t *>(in_memory(sp->fuse_any) + (int64_t)max(qp->map_read, 0) * qp->n_w32)[row];
         if (qp->n_sub > 0) {
@@ -450,9 +456,9 @@ __global__ __launch_bounds__(kFuseBlock) void sim_fused_kernel(bmtk_glif3_sim s,
         const bool on = in_group && row < n;  // this lane holds an element
         const unsigned e0 = (unsigned)(grp * kRows) * (unsigned)batch, e = e0 + lane, boff = e * 4u;
         // the ring cells of one slot, where an id repeated within a step reached this neuron (rare)
-        auto take_ring = [&](int64_t step, unsigned word, float (&a)[GLIF3_NREC]) {
+        auto take_ring = [&](int slot, unsigned word, float (&a)[GLIF3_NREC]) {
             if (qp->use_ring && on && ((word >> ((unsigned)row & 31u)) & 1u)) {
-                float *cells = in_memory(sp->ring) + (int64_t)((step % qp->Lr + qp->Lr) % qp->Lr) * GLIF3_NREC * ne;
+                float *cells = in_memory(sp->ring) + (int64_t)slot * GLIF3_NREC * ne;
                 float v[GLIF3_NREC];
 #pragma unroll
                 for (int k = 0; k < GLIF3_NREC; ++k) v[k] = ldf(cells, k, boff);
@@ -461,10 +467,10 @@ __global__ __launch_bounds__(kFuseBlock) void sim_fused_kernel(bmtk_glif3_sim s,
                     stf(cells, k, boff, 0.0f);
                     a[k] = v[k] + a[k];
                 }
-                if (first_trial) atomicAnd(ring_row(sp, qp, step) + (row >> 5), ~(1u << ((unsigned)row & 31u)));
+                if (first_trial) atomicAnd(ring_row(sp, qp, slot) + (row >> 5), ~(1u << ((unsigned)row & 31u)));
             }
         };
-        if (qp->fold0) take_ring(qp->t0 - 1, ring_word0, a0);
+        if (qp->fold0) take_ring(qp->ring_slot[0], ring_word0, a0);
         if (qp->n_sub == 0) {
             // closing launch: what arrived in the last step enters y1, as at the end of that step
             if (on) {
@@ -503,7 +509,7 @@ __global__ __launch_bounds__(kFuseBlock) void sim_fused_kernel(bmtk_glif3_sim s,
             }
             // the group's elements are one word of spike bits
             const unsigned long long m = __ballot(spike);
-            if (lane == 0) in_memory(sp->work_bits)[(t % qp->H) * sp->fuse_hist_stride + grp] = m;
+            if (lane == 0) in_memory(sp->work_bits)[qp->hist_row[1 + sub] * sp->fuse_hist_stride + grp] = m;
             if (sp->spike_bits) {
                 // the same bits in the run's output, element after element: where a group fills its 64 bits a word of
                 // its own, otherwise pieces of one or two words (cleared by the driver)
@@ -521,7 +527,7 @@ __global__ __launch_bounds__(kFuseBlock) void sim_fused_kernel(bmtk_glif3_sim s,
                 fired_bits |= row_fired ? (sub == 0 ? step_bit0 : step_bit1) : 0u;
             } else if (m != 0ull && on && first_trial && row_fired) {
                 const unsigned g = (unsigned)row >> qp->shift;
-                atomicOr(in_memory(sp->fuse_any) + (t % qp->H) * qp->n_w32 + (g >> 5), 1u << (g & 31u));
+                atomicOr(in_memory(sp->fuse_any) + (int64_t)qp->hist_row[1 + sub] * qp->n_w32 + (g >> 5), 1u << (g & 31u));
             }
             if (sp->spike_count && m != 0ull) {
                 // one counter bump per wavefront, record slots handed out in lane order
@@ -543,7 +549,7 @@ __global__ __launch_bounds__(kFuseBlock) void sim_fused_kernel(bmtk_glif3_sim s,
         };
         one_step(0, qp->fold0 != 0, a0, qp->probe_row0);
         if (qp->n_sub == 2) {
-            take_ring(qp->t0, ring_word1, a1);
+            take_ring(qp->ring_slot[1], ring_word1, a1);
             one_step(1, true, a1, qp->probe_row1);
         }
         if (on) {
@@ -624,7 +630,7 @@ __global__ __launch_bounds__(kFuseBlock) void sim_fused_kernel(bmtk_glif3_sim s,
     // second adds the weights.  A group's closing work waits for its last masks the same way and is done in the turn
     // after the group's last block.
     unsigned head = 0u, tail = 0u;   // entries head .. tail-1 (mod kFuseStage) are parked; same in all lanes
-    unsigned arrive = (unsigned)(((q.t0 - 1) % H + H) % H);
+    const unsigned arrive = (unsigned)q.hist_row[0];
     unsigned pend_acc = 0u, pend_shift = 0u;
     unsigned long long pend_w = 0ull, pend_m = 0ull;
     bool pend_any = false;           // masks are on their way (same in all lanes)
@@ -948,6 +954,10 @@ int simulate_fused(const bmtk_glif3_sim &s, int64_t step0, int64_t n_steps, hipS
         q.n_sub = closing ? 0 : (int)(n_steps - k < 2 ? n_steps - k : 2);
         q.t0 = step0 + k;
         q.out_row = k;
+        for (int i = 0; i < 3; ++i) {
+            q.hist_row[i] = (int)((q.t0 + i - 1 + q.H) % q.H);
+            q.ring_slot[i] = (int)((q.t0 + i - 1 + q.Lr) % q.Lr);
+        }
         q.probe_row0 = closing ? -1 : probe_row(q.t0);
         q.probe_row1 = q.n_sub == 2 ? probe_row(q.t0 + 1) : -1;
         q.fold0 = k > 0 ? 1 : 0;
