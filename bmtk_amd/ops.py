@@ -372,31 +372,31 @@ class SynapseTable:
     def range_rows_min(self, n_tgt, batch, ring_slots):
         """Active elements from which delivery by target ranges is expected to be the faster form, 0: never (cells of a range
         that do not fit a workgroup, or rows so short that the offsets would outgrow the table)."""
-        span = -(-n_tgt // self.RANGES)
-        if 16 * ring_slots * span * batch > self.RANGE_LDS or self.nnz < max(1, 100 * self.n_rows) or self.delays.dtype != torch.uint8:
+        nnz = self.indices.numel()
+        if nnz < max(1, 100 * self.n_rows) or 16 * ring_slots * -(-n_tgt // self.RANGES) * batch > self.RANGE_LDS or self.delays.dtype != torch.uint8:
             return 0
         if ring_slots < 2 or n_tgt * batch < 1:   # (refused by the call itself)
             return 0
-        return _range_rows_min(self.nnz / self.n_rows, n_tgt * batch, ring_slots)
+        return _range_rows_min(nnz / self.n_rows, n_tgt * batch, ring_slots)
 
     def ranges(self, n_tgt):
         """Segment offsets of the rows by ``RANGES`` ranges of targets, or None for a table whose rows are not sorted by index.
         Made once per table and row bounds (synchronises then).  None while a graph is being captured: its replays would read the
         offsets after other row bounds have replaced them."""
-        if torch.cuda.is_current_stream_capturing():
+        if torch._C._cuda_isCurrentStreamCapturing():
             return None
+        indptr = self.indptr
         plan = getattr(self, "_ranges", None)
-        stream = _stream()
-        if plan is None or plan[0] is not self.indptr or plan[1] != (self.indptr._version, n_tgt):
-            made_of = (self.indptr._version, n_tgt)
+        if plan is None or plan[0] is not indptr or plan[1] != indptr._version or plan[2] != n_tgt:
+            version = indptr._version
             try:
                 seg = self.segment_offsets(-(-n_tgt // self.RANGES), self.RANGES)
             except ValueError:
                 seg = None
-            plan = self._ranges = (self.indptr, made_of, seg, stream)
-        elif plan[2] is not None and plan[3] != stream:
-            plan[2].record_stream(torch.cuda.current_stream())   # (replaced offsets are not reused under a launch of another stream)
-        return plan[2]
+            plan = self._ranges = (indptr, version, n_tgt, seg, _stream())
+        elif plan[3] is not None and plan[4] != _stream():
+            plan[3].record_stream(torch.cuda.current_stream())   # (replaced offsets are not reused under a launch of another stream)
+        return plan[3]
 
     def pointers(self):
         nnz = self.nnz

@@ -150,9 +150,9 @@ class Glif3Bptt:
         self.d_inp_w = torch.zeros(sim.inp.nnz, device=dev) if sim.inp is not None and sim.in_ptr is not None else None
 
     def zero(self):
-        for t in (self.lam_V, self.lam_asc, self.lam_y1, self.lam_y2, self.lam_ring, self.gz, self.d_rec_w, self.d_inp_w):
-            if t is not None:
-                t.zero_()
+        # (all in a launch or two: eight small ones were 55 us of a training step, these 15)
+        torch._foreach_zero_([t for t in (self.lam_V, self.lam_asc, self.lam_y1, self.lam_y2, self.lam_ring, self.gz, self.d_rec_w, self.d_inp_w)
+                              if t is not None])
 
     def _struct(self, fwd, dl_dz_const, dl_dz, blocked):
         sim, saved, bits = self.sim, fwd["saved"], fwd["bits"]
