@@ -11,10 +11,12 @@ Flags that matter for results:
 import os
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 PKG = os.path.dirname(HERE)
 LIB = os.path.join(PKG, "libbmtk_amd.so")
+PTR = os.path.join(PKG, "_ptr.so")
 SOURCES = ["kernels.hip", "propagate_pull.hip", "simulate.hip", "simulate_fused.hip", "resident.hip", "resident_solo.hip", "resident_windows.hip", "resident_batch.hip", "backward.hip", "poisson.hip", "microbench.hip"]
 FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared", "-ffp-contract=off",
          "-munsafe-fp-atomics", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
@@ -32,7 +34,25 @@ def build(verbose=False, extra=()):
         raise RuntimeError("hipcc failed:\n" + out)
     if verbose and out.strip():
         print(out)
+    build_ptr(verbose)
     return LIB
+
+
+def build_ptr(verbose=False):
+    """The pointer checks of ``ops._p`` as a Python module (host code)."""
+    import torch
+    from torch.utils import cpp_extension
+    lib_dir = os.path.join(os.path.dirname(torch.__file__), "lib")
+    cmd = ([os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-w",
+            "-D_GLIBCXX_USE_CXX11_ABI={}".format(int(torch._C._GLIBCXX_USE_CXX11_ABI))]
+           + ["-I" + d for d in cpp_extension.include_paths() + [sysconfig.get_paths()["include"]]]
+           + ["-o", PTR, os.path.join(HERE, "ptr.cpp"), "-L" + lib_dir, "-ltorch_python", "-ltorch_cpu", "-lc10"])
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    res = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    if res.returncode != 0:
+        raise RuntimeError("compiling ptr.cpp failed:\n" + res.stdout)
+    return PTR
 
 
 if __name__ == "__main__":

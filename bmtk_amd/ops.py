@@ -43,6 +43,14 @@ def _p(t, dtype=None, numel=None, name="tensor"):
     return t.data_ptr()
 
 
+try:  # (the same checks in native code, where it has been built)
+    from . import _ptr
+    _ptr.set_general(_p)
+    _p = _ptr.ptr
+except ImportError:
+    pass
+
+
 def n_words(ne):
     return (ne + 63) // 64
 

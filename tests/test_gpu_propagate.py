@@ -511,3 +511,30 @@ def test_auto_delivery_picks_a_form_on_the_device_and_the_ring_is_the_oracles(ba
             assert seen == {True} or 0 in counts
         elif thr == ne:
             assert seen == {False}
+
+
+def test_native_pointer_checks_are_the_general_ones():
+    """What passes gives the tensor's pointer, what does not the general way's exception, word for word."""
+    from bmtk_amd import _ptr
+    general = next(f for f in gc_functions() if f.__name__ == "_p")
+    x = torch.zeros(4, 6, device="cuda")
+    calls = [(None,), (x,), (x, torch.float32), (x, torch.float32, 24), (x, None, 3, "x"), (x[1:],), (x[:0],), (torch.nn.Parameter(x),), (x.requires_grad_(),),
+             (x.detach().to(torch.complex64).conj(),), (x, torch.int32, 24, "ring"), (x, torch.float32, 25, "ring"), (x.t(), None, None, "t"), (x[:, :2],), (x.cpu(),),
+             (x, torch.float32, 24.0), (x, torch.float32, 1 << 70), (x, "float"), (x.to_sparse(),), (5,), ()]
+    for args in calls:
+        outs = []
+        for f in (_ptr.ptr, general):
+            try:
+                outs.append(f(*args))
+            except Exception as exc:
+                outs.append((type(exc), str(exc)))
+        assert outs[0] == outs[1], args
+    assert _ptr.ptr(x, name="y") == x.data_ptr() and ops._p is _ptr.ptr
+    with pytest.raises(ValueError, match="y holds 24"):
+        _ptr.ptr(x, numel=25, name="y")
+
+
+def gc_functions():
+    import gc
+    import types
+    return [f for f in gc.get_objects() if isinstance(f, types.FunctionType) and f.__module__ == "bmtk_amd.ops"]
