@@ -238,8 +238,8 @@ def bench_propagation(torch, steps=200, warmup=20, modes=PROPAGATION_MODES, rate
             if traffic is not None and two:
                 traffic /= 2                                            # per arrival step, like the time below
             entry = {"kernel": {"auto": "auto_push_kernel or pull_kernel, chosen on the device",
-                                "auto2": "auto2: auto_push_kernel or pull2_kernel, chosen on the device for each of the two steps of a call",
-                                "pull2": "pull2_kernel: the arrivals of two steps per launch, half a launch per step"}
+                                "auto2": "auto2: auto_push_kernel or pull2_pair_kernel, chosen on the device for each of the two steps of a call",
+                                "pull2": "pull2_pair_kernel: the arrivals of two steps per launch, half a launch per step"}
                                .get(mode, mode + "_kernel"),
                      "workload": "propagation N=51978 nnz=%d batch=64 rate=%gHz" % (t_src.nnz, rate),
                      "events_per_launch": events, "active_elements_per_launch": active,

@@ -1093,7 +1093,7 @@ struct SweepElem {
 //
 // No array of the kernel is indexed at run time: a choice of one of four trials' values by the lane's place made the sums and potentials an array
 // in scratch memory, whose stores waited for the loads (and the records asked for before them) ahead of the first turn.  us per two
-// steps, with scratch / without: 3001 x 12, in-degree 200: 19.6 / 16.2; 3001 x 32, 100: 25.1 / 18.0; 20000 x 16, 150: 114.5 / 92.6; 12000 x 32, 120: 85.3 / 66.7;
+// steps, with scratch / without: 3001 x 12, in-degree 200: 19.6 / 16.2 (15.2 since the host divides by the ring's length); 3001 x 32, 100: 25.1 / 18.0; 20000 x 16, 150: 114.5 / 92.6; 12000 x 32, 120: 85.3 / 66.7;
 // 12000 x 12, 400: 92.5 / 89.0; 14000 x 16, 200: 71.3 / 71.7.  Tried: eight synapses in flight for rows of a wavefront's own (1800 x 32, 600: 29.8 -> 26.5, but
 // 3001 x 4, 200: 12.5 -> 15.2, spilled registers), two turns in flight (spilled registers: 17 to 18.5 against 16.2).
 //
