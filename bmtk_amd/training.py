@@ -74,7 +74,7 @@ def rate_mse(counts, n_steps, batch, pop_id, targets):
 class Glif3Bptt:
     """Reverse-time adjoint over a recorded forward run of a ``Glif3Simulator``: of a batch, or of a single trial
     built with ``resident=False``.  (A batch whose simulator leaves ``resident`` at "auto" runs the forward part with
-    resident trials where they pay: 1.76 instead of 2.19 ms a step of training at 3,001 neurons x 12 trials x 100 steps.)"""
+    resident trials where they pay: 1.18 instead of 1.52 ms a step of training at 3,001 neurons x 12 trials x 100 steps.)"""
 
     # A synapse costs the swept form more once the L2s no longer hold the adjoint ring; the blocked form has a fixed part per
     # row and range, which long rows share among more synapses.  Measured on one MI355X, whole calls of 40 steps, us per step
@@ -84,7 +84,11 @@ class Glif3Bptt:
     # 97/81 160/120; 27011 x 8 (21) 43/53 67/76 107/112 186/174; 51978 x 4 (20) 77/81 127/128 212/195 403/350.  The forms cross
     # where the ring times the cube root of the in-degree reaches these marks: lower for batches whose adjoint rows (four
     # bytes a trial) are no whole lines of 64 bytes, so that the swept form's gathers fetch what they do not use.
-    BLOCKED_MIN_RING_MB = 31.0          # at in-degree 400, batch a multiple of 16
+    BLOCKED_MIN_RING_MB = 31.0          # at in-degree 400, 16 trials
+    # 32, 48 and 64 trials, where the blocked form takes two steps per pass: ring times square root of the in-degree.  Swept / blocked as they
+    # are now (us per step): 9003 x 32 at in-degree 250 34/36, 400 47/43, 750 76/59; 7000 x 32, 600 47/45; 11000 x 32, 200 34/38;
+    # 13000 x 32, 120 35/37; 15000 x 32, 220 52/47; 5000 x 64, 300 42/38; 6500 x 64, 150 39/38; 4000 x 48, 900 64/53
+    BLOCKED_MIN_RING_MB_TWO = 25.5
     BLOCKED_MIN_RING_MB_RAGGED = 22.0, 20.0   # other batches up to 16, and above (where it takes two steps per pass)
     BLOCKED_MIN_RING_MB_FOUR = 17.0     # four trials: a quarter of a line
     # Four trials through a table of more than 150 MB, which does not stay in the memory-side cache beside the rest: launches of
@@ -96,9 +100,25 @@ class Glif3Bptt:
     def blocked_pays(cls, n, batch, ring_slots, nnz):
         """Whether the blocked form is expected to take less time per step than the swept form."""
         ring_mb = ring_slots * NREC * n * batch * 4e-6
+        if batch % 16 == 0 and batch > 16:
+            return ring_mb * (nnz / (400.0 * n)) ** 0.5 >= cls.BLOCKED_MIN_RING_MB_TWO
         least = (cls.BLOCKED_MIN_RING_MB if batch % 16 == 0 else cls.BLOCKED_MIN_RING_MB_FOUR if batch <= 4
                  else cls.BLOCKED_MIN_RING_MB_RAGGED[batch > 16])
         return ring_mb * (nnz / (400.0 * n)) ** (1.0 / 3.0) >= least
+
+    @staticmethod
+    def target_ranges(n, batch, ring_slots, nnz, two_steps=True):
+        """Target ranges of the blocked table.  Two steps per pass (batches above 16): what counts is how long a row's segments are, a
+        segment has its fixed part.  us per two steps with 8 / 16 / 24 / 32 ranges: 52000 x 32, in-degree 100 280/291/313/335; 25000 x 40, 120
+        212/226/246/270; 12000 x 64, 150 132/135/141/152; 45000 x 40, 200 517/503/530/563; 31000 x 64, 300 490/462/472/489; 20000 x 20, 300
+        148/145/149/156; 40000 x 24, 400 390/368/366/372; 30011 x 32, 600 331/314/315/319; 20011 x 20, 700 256/248/244/244; 15000 x 32, 800
+        183/182/179/182; 51978 x 32, 1000 888/838/809/812.  Measured up to 200 MB of adjoint ring; larger ones, and one step per pass,
+        are left to the share of a ring that an L2 holds."""
+        if batch <= 16 or not two_steps or ring_slots * NREC * n * batch * 4 > 200e6:
+            from . import ops
+            return ops.blocked_table_blocks(n, batch, ring_slots)
+        in_degree = nnz / n
+        return 8 if in_degree < 175.0 else 16 if in_degree < 600.0 else 24
 
     @classmethod
     def plain_pays(cls, batch, nnz):
@@ -110,7 +130,7 @@ class Glif3Bptt:
         source-major table (its adjoint ring ``lam_ring`` has two slots more than ``sim.L``); ``blocked``: the recurrent
         table regrouped by target range for the transposed propagation; neither: a launch per part and step, any batch.
         None leaves the choice to ``blocked_pays`` and ``plain_pays`` where the batch (a multiple of 4 up to 64) allows it.  ``n_blocks``:
-        number of target ranges, a multiple of 8 (None: ``ops.blocked_table_blocks``); ``two_steps``: let the blocked form
+        number of target ranges, a multiple of 8 (None: ``target_ranges``); ``two_steps``: let the blocked form
         take two steps per pass over its table (batches above 16; ``gz`` then holds the partial sums of both)."""
         if sim.res_span or sim.delay_offset:
             raise ValueError("the backward pass needs a simulator built with resident=False (or a batch) and delay_offset 0")
@@ -138,8 +158,7 @@ class Glif3Bptt:
         self.d_rec_w = torch.zeros(sim.rec.nnz, device=dev) if sim.rec is not None else None
         self.blk = None
         if blocked:
-            from . import ops
-            self.n_blocks = int(n_blocks or ops.blocked_table_blocks(sim.n, sim.batch, sim.L))
+            self.n_blocks = int(n_blocks or self.target_ranges(sim.n, sim.batch, sim.L, sim.rec.nnz, two_steps))
             if self.n_blocks % 8:
                 raise ValueError("n_blocks must be a multiple of 8")
             self.blk = sim.rec.blocked(sim.n, self.n_blocks)

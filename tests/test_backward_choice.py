@@ -20,3 +20,30 @@ def test_choice_is_within_a_tenth_of_the_fastest(n, batch, k, swept, blocked, pl
 
 def test_a_table_without_synapses_is_no_reason_for_ranges():
     assert not Glif3Bptt.blocked_pays(51978, 32, 6, 0)
+
+
+# two steps per pass as they are now: neurons, trials, in-degree, us per step swept / blocked
+TWO_STEPS = [(7000, 32, 600, 47.3, 45.0), (5000, 64, 300, 41.6, 38.3), (9003, 32, 250, 33.7, 35.5), (11000, 32, 200, 34.1, 37.5), (4000, 48, 900, 64.1, 53.2),
+             (9003, 32, 400, 46.6, 42.6), (13000, 32, 120, 35.4, 36.5), (6500, 64, 150, 39.4, 37.6), (9003, 32, 120, 23.4, 29.9), (9003, 32, 750, 75.5, 58.5),
+             (15000, 32, 220, 51.9, 47.4), (15000, 32, 500, 92.3, 72.2), (20011, 20, 200, 87.9, 63.0), (20011, 20, 700, 246.6, 136.8), (6000, 64, 500, 69.3, 54.7),
+             (12000, 64, 150, 80.4, 65.4)]
+
+
+@pytest.mark.parametrize("n,batch,k,swept,blocked", TWO_STEPS)
+def test_choice_for_two_steps_per_pass(n, batch, k, swept, blocked):
+    assert (blocked if Glif3Bptt.blocked_pays(n, batch, 6, n * k) else swept) <= 1.05 * min(swept, blocked)
+
+
+# neurons, trials, in-degree, us per two steps with 8 / 16 / 24 target ranges
+RANGES = [(52000, 32, 100, 280.4, 291.4, 312.8), (25000, 40, 120, 211.7, 225.7, 246.1), (12000, 64, 150, 132.1, 135.1, 141.0), (45000, 40, 200, 516.5, 503.4, 530.0),
+          (31000, 64, 300, 489.9, 461.7, 472.1), (20000, 20, 300, 147.6, 145.1, 148.7), (40000, 24, 400, 389.8, 368.1, 366.3), (30011, 32, 600, 331.4, 314.3, 315.1),
+          (20011, 20, 700, 256.3, 248.4, 243.9), (15000, 32, 800, 183.0, 181.8, 179.0), (51978, 32, 1000, 887.8, 837.8, 809.4)]
+
+
+@pytest.mark.parametrize("n,batch,k,eight,sixteen,more", RANGES)
+def test_number_of_target_ranges(n, batch, k, eight, sixteen, more):
+    took = {8: eight, 16: sixteen, 24: more}[Glif3Bptt.target_ranges(n, batch, 6, n * k)]
+    assert took <= 1.01 * min(eight, sixteen, more)
+    from bmtk_amd import ops
+    assert Glif3Bptt.target_ranges(n, batch, 6, n * k, two_steps=False) == ops.blocked_table_blocks(n, batch, 6)
+    assert Glif3Bptt.target_ranges(4 * n, 64, 6, 4 * n * k) == ops.blocked_table_blocks(4 * n, 64, 6) or 4 * n * 64 * 96 <= 200e6
