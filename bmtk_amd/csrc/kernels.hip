@@ -584,15 +584,17 @@ __global__ __launch_bounds__(kBlock) void scatter_kernel(const int32_t *__restri
 
 // The same sums by owners of target ranges, for steps with many events: workgroup g takes what the active rows send to targets
 // g * span .. (g + 1) * span - 1, adds it up in LDS, and adds its cells to the ring at the end, sixteen neighbours to a line, where
-// an atomic per event is a line per event.  `seg` (bmtk_csr_segment_offsets) says where in a row a range's synapses lie; what they are is
-// read from the table as it is now, and a synapse whose target is not in its range goes to the ring by itself.
+// an atomic per event is a line per event.  `seg` (bmtk_csr_segment_offsets) only proposes where to cut a row among the workgroups: the
+// cuts are held within the row's bounds as the table has them now, the first and last piece begin and end there, and a synapse whose target
+// is not in its range goes to the ring by itself.  Whatever was written to the table since, every synapse of a row is delivered once.
 //
-// What bounds it: lines asked for by a compute unit (a segment's bounds and its four arrays, 2.3 clocks each) and the chain count ->
-// elements -> bounds -> synapses.  Neighbouring ranges share the lines of a row and go to one XCD: dealt out in turn, every XCD
-// read every active row (16.4 us instead of 12.0 at 1,380 rows of 300 into 30,011 targets, 64 instead of 54 at 4,600 x 500 into 100,000).
-// us per call, an atomic per event / by ranges: 5,000 targets, 115,000 events 8.5 / 5.8; 12,000, 110,000 8.4 / 5.6; 30,011, 90,000
-// 6.8 / 5.9, 414,000 23.3 / 12.0; 60,000, 90,000 6.6 / 6.7, 414,000 23.4 / 15.4; 100,000, 150,000 9.7 / 9.4, 2.3 M 116 / 54; 200,000, 150,000 9.6 / 11.1,
-// 500,000 26.9 / 21.7, 2.3 M 114 / 63: below rows_min active elements it is the walk above.
+// What bounds it: lines asked for by a compute unit (a piece's cuts, its row's bounds and its four arrays, 2.3 clocks each) and the chain
+// count -> elements -> cuts -> synapses.  Neighbouring ranges share the lines of a row and go to one XCD: dealt out in turn, every XCD
+// read every active row (16.4 us instead of 12.0 at 1,380 rows of 300 into 30,011 targets, 64 instead of 54 at 4,600 x 500 into 100,000, both
+// before the row bounds were read, which costs 5 %; without them a rewritten indptr would be delivered by the rows it had before).
+// us per call, an atomic per event / by ranges: 5,000 targets, 115,000 events 8.2 / 6.2; 12,000, 110,000 7.4 / 6.4; 30,011, 90,000
+// 6.4 / 6.6, 414,000 22.5 / 13.2; 60,000, 90,000 6.5 / 7.4, 414,000 22.2 / 15.8; 100,000, 150,000 9.4 / 10.9, 2.3 M 114 / 56; 200,000, 150,000 9.3 / 14.2,
+// 500,000 26.6 / 26.0, 2.3 M 113 / 66: below rows_min active elements it is the walk above.
 constexpr int kRangeThreads = 1024;
 constexpr size_t kRangeLdsMax = 150u * 1024u;
 __global__ __launch_bounds__(kRangeThreads) void scatter_ranges_kernel(const int32_t *__restrict__ active, const int32_t *__restrict__ n_active,
@@ -613,16 +615,21 @@ __global__ __launch_bounds__(kRangeThreads) void scatter_ranges_kernel(const int
     const unsigned n_here = (unsigned)max((int64_t)0, min((int64_t)span, n_tgt - t0));
     constexpr int kAhead = 4;  // synapses of a segment in flight
     struct Row {
-        int b, p, p1;
+        int b;
+        unsigned p, p1;  // (unsigned: a step past the end of 2^31 - 1 synapses stays behind it)
     };
+    struct __attribute__((packed, aligned(4))) Two {
+        int at, to;
+    };
+    const int inner = g == 0 ? 0 : -1, end = g == (int)gridDim.x - 1 ? 0x7FFFFFFF : 0;  // (the first piece begins with its row, the last ends with it)
     auto look = [&](int k) {
-        Row r{0, 0, 0};
+        Row r{0, 0u, 0u};
         if (k < cnt) {
             const int e = active[k], j = batch == 1 ? e : (int)((uint32_t)e / (uint32_t)batch);
-            const uint32_t *at = seg + (int64_t)j * n_seg + g;
+            const Two cut = *reinterpret_cast<const Two *>(seg + (int64_t)j * n_seg + g), now = *reinterpret_cast<const Two *>(t.indptr + j);
             r.b = e - j * batch;
-            r.p = (int)at[0];
-            r.p1 = (int)at[1];
+            r.p = (unsigned)max(now.at, min(cut.at & inner, now.to));
+            r.p1 = (unsigned)max(now.at, min(cut.to | end, now.to));
         }
         return r;
     };
@@ -631,7 +638,7 @@ __global__ __launch_bounds__(kRangeThreads) void scatter_ranges_kernel(const int
     __syncthreads();
     for (int k = threadIdx.x; k < cnt; k += kRangeThreads) {
         const Row next = look(k + kRangeThreads);
-        for (int p = row.p; p < row.p1; p += kAhead) {
+        for (unsigned p = row.p; p < row.p1; p += kAhead) {
             int i[kAhead], d[kAhead], r[kAhead];
             float w[kAhead];
 #pragma unroll

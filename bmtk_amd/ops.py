@@ -175,14 +175,14 @@ BLOCKED_PAD = 16  # BMTK_BLOCKED_PAD of include/bmtk_amd.h
 @functools.lru_cache(maxsize=256)
 def _range_rows_min(row, ne, ring_slots):
     """Rows of ``row`` synapses on average from which scatter_ranges_kernel takes less time than an atomic per event (in us, fitted to one
-    MI355X: 5,000 to 200,000 targets, rows of 100 to 500; the two agree within 10 % where the forms cross).  An event's atomic takes
+    MI355X: 5,000 to 200,000 targets, rows of 100 to 500; where it says the forms cross they are within 6 % of one another).  An event's atomic takes
     48 ps, and so does a line of sixteen cells that a workgroup adds to the ring at the end, once for however many events; a row costs
     every workgroup a look; cells have to be cleared and gone through."""
     lines = (ring_slots - 1) * NREC * ne / 16.0
 
     def gain(rows):
         events = rows * row
-        return 48e-6 * (events - lines * (1.0 - math.exp(-events / lines))) - (0.8 + 1.45e-5 * ne) - rows * (0.5e-3 + 16e-6 * row)
+        return 48e-6 * (events - lines * (1.0 - math.exp(-events / lines))) - (0.6 + 1.0e-5 * ne) - rows * (1.45e-3 + 17e-6 * row)
     rows = 16
     while rows < (1 << 24) and gain(rows) <= 0.0:
         rows *= 1.1
@@ -389,19 +389,20 @@ class SynapseTable:
 
     def ranges(self, n_tgt):
         """Segment offsets of the rows by ``RANGES`` ranges of targets, or None for a table whose rows are not sorted by index.
-        Made once per table and row bounds (synchronises then).  None while a graph is being captured: its replays would read the
-        offsets after other row bounds have replaced them."""
+        Made once per table and row bounds (synchronises then).  What a delivery adds does not depend on them: bounds rewritten in a way
+        that the version counter does not see (a replayed graph, ``.data``, a caller's kernel) make it slower, not wrong.  None while a
+        graph is being captured: its replays would read the offsets after others have replaced them."""
         if torch._C._cuda_isCurrentStreamCapturing():
             return None
         indptr = self.indptr
         plan = getattr(self, "_ranges", None)
-        if plan is None or plan[0] is not indptr or plan[1] != indptr._version or plan[2] != n_tgt:
+        if plan is None or plan[0] is not indptr or plan[1] != indptr._version or plan[2] != (n_tgt, self.n_rows):
             version = indptr._version
             try:
                 seg = self.segment_offsets(-(-n_tgt // self.RANGES), self.RANGES)
             except ValueError:
                 seg = None
-            plan = self._ranges = (indptr, version, n_tgt, seg, _stream())
+            plan = self._ranges = (indptr, version, (n_tgt, self.n_rows), seg, _stream())
         elif plan[3] is not None and plan[4] != _stream():
             plan[3].record_stream(torch.cuda.current_stream())   # (replaced offsets are not reused under a launch of another stream)
         return plan[3]

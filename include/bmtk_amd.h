@@ -114,9 +114,9 @@ int bmtk_csr_propagate_scatter(const int32_t *active, const int32_t *n_active, i
 
 /* The same by target ranges for steps with at least rows_min active elements: n_ranges workgroups each own `span` targets, add what
  * the active rows send there in LDS and add their cells to the ring (atomically) at the end.  seg: bmtk_csr_segment_offsets of the
- * table with `span` and n_ranges, rows sorted by target; it only says where a range's synapses lie in a row: indices, weights,
- * delays and receptors are read as they are now (synapses that have left their range are still delivered, one by one), row
- * bounds must be those that seg was made from.  L * 4 * span * batch cells must fit 150 KB. */
+ * table with `span` and n_ranges, rows sorted by target; it only says where a range's synapses lie in a row: row bounds, indices,
+ * weights, delays and receptors are read as they are now, and whatever of them was written to since, every synapse of a row is delivered
+ * once (those outside their range one by one).  seg must ascend within a row.  L * 4 * span * batch cells must fit 150 KB. */
 int bmtk_csr_propagate_scatter_ranges(const int32_t *active, const int32_t *n_active, int32_t batch, const int32_t *indptr,
                                       const int32_t *indices, const float *weights, const uint8_t *delays,
                                       const uint8_t *receptors, const uint32_t *seg, int32_t span, int32_t n_ranges,

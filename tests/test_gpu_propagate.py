@@ -334,6 +334,53 @@ def test_a_captured_delivery_follows_row_bounds_written_later():
         ops.csr_propagate_scatter(ids, count, table, torch.zeros(1, 4, n, device="cuda"), n, 1, 4)
 
 
+def test_delivery_by_target_ranges_of_row_bounds_written_unseen():
+    """Row bounds rewritten behind the version counter (a captured write replayed, ``.data``, a DLPack view): shifted and shortened rows,
+    all synapses in one row, rows outside their old bounds.  Always what an atomic per event gives, with the offsets of before."""
+    rng = np.random.default_rng(7)
+    n, L, nnz = 600, 6, 600 * 150
+    src, tgt, w, d, r = _edges(rng, n, n, nnz)
+    w = (np.round(w * 4) / 4).astype(np.float32)
+    table = ops.SynapseTable.from_edges(src, tgt, w, d, r, n, n)
+    on = np.union1d(rng.choice(n, n // 2, replace=False), [0, 299, n - 1]).astype(np.int32)
+    ids, count = to_dev(on), to_dev(np.array([on.size], np.int32))
+    from bmtk_amd import _lib
+
+    def walked():
+        want = torch.zeros(L, 4, n, device="cuda")
+        _lib.check(_lib.load().bmtk_csr_propagate_scatter(ids.data_ptr(), count.data_ptr(), n, 1, *table.pointers(), want.data_ptr(), L, n, 4, ops._stream()))
+        return want
+
+    def ranged():
+        got = torch.zeros(L, 4, n, device="cuda")
+        ops.csr_propagate_scatter(ids, count, table, got, n, 1, 4)
+        return got
+
+    assert 0 < table.range_rows_min(n, 1, L) <= on.size and torch.equal(ranged(), walked())
+    before = walked()
+    i = torch.arange(1, n, device="cuda", dtype=torch.int32)
+    bounds = [i * (nnz // n), i * 3, (i >= 300).to(torch.int32) * nnz, torch.full_like(i, nnz), torch.full_like(i, 0), nnz - (n - i) * 140]
+    fresh = torch.zeros_like(i)
+    graph = torch.cuda.CUDAGraph()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.graph(graph, stream=side):
+        torch.add(fresh, 0, out=table.indptr[1:-1])
+    table.ranges(n)          # (the capture itself was counted, its replays are not)
+    seg = table.ranges(n)
+    for b in bounds:
+        fresh.copy_(b)
+        graph.replay()
+        want, got = walked(), ranged()
+        assert torch.equal(want, got) and not torch.equal(want, before)
+        assert table.ranges(n) is seg
+    view = torch.from_dlpack(table.indptr.detach())
+    for how in (table.indptr.data, view):
+        for b in bounds:
+            how[1:-1] = b
+            assert torch.equal(walked(), ranged())
+
+
 @pytest.mark.parametrize("span,n_groups", [(7, 30), (64, 4), (1, 211), (300, 1), (100, 2)])
 def test_segment_offsets_are_what_a_search_finds(span, n_groups):
     """Empty rows, rows of one synapse and of several chunks, repeated targets, targets beyond the last group, first and last groups empty."""
