@@ -396,8 +396,8 @@ class SynapseTable:
             return None
         indptr = self.indptr
         plan = getattr(self, "_ranges", None)
-        if plan is None or plan[0] is not indptr or plan[1] != indptr._version or plan[2] != (n_tgt, self.n_rows):
-            version = indptr._version
+        version = None if indptr.is_inference() else indptr._version   # (tensors made under inference_mode count no writes)
+        if plan is None or plan[0] is not indptr or plan[1] != version or plan[2] != (n_tgt, self.n_rows):
             try:
                 seg = self.segment_offsets(-(-n_tgt // self.RANGES), self.RANGES)
             except ValueError:

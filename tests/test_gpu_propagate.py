@@ -381,6 +381,38 @@ def test_delivery_by_target_ranges_of_row_bounds_written_unseen():
             assert torch.equal(walked(), ranged())
 
 
+@pytest.mark.parametrize("sort", [True, False])
+def test_delivery_by_target_ranges_of_a_table_made_under_inference_mode(sort):
+    """Such tensors have no version counter: delivered in the mode and after it, also where row bounds were rewritten in the mode."""
+    rng = np.random.default_rng(8)
+    n, L, nnz = 600, 6, 600 * 150
+    src, tgt, w, d, r = _edges(rng, n, n, nnz)
+    w = (np.round(w * 4) / 4).astype(np.float32)
+    from bmtk_amd import _lib
+    with torch.inference_mode():
+        table = ops.SynapseTable.from_edges(src, tgt, w, d, r, n, n)
+        if not sort:
+            table.indices = table.indices.flip(0).contiguous()
+    assert table.indptr.is_inference()
+    on = np.union1d(rng.choice(n, n // 2, replace=False), [0, n - 1]).astype(np.int32)
+    ids, count = to_dev(on), to_dev(np.array([on.size], np.int32))
+
+    def check():
+        want, got = torch.zeros(L, 4, n, device="cuda"), torch.zeros(L, 4, n, device="cuda")
+        _lib.check(_lib.load().bmtk_csr_propagate_scatter(ids.data_ptr(), count.data_ptr(), n, 1, *table.pointers(), want.data_ptr(), L, n, 4, ops._stream()))
+        ops.csr_propagate_scatter(ids, count, table, got, n, 1, 4)
+        assert torch.equal(want, got) and float(want.abs().max()) > 0
+
+    assert 0 < table.range_rows_min(n, 1, L) <= on.size
+    check()
+    with torch.inference_mode():
+        check()
+        table.indptr[1:-1] = torch.arange(1, n, device="cuda") * 3
+        check()
+    check()
+    assert (table.ranges(n) is not None) == sort
+
+
 @pytest.mark.parametrize("span,n_groups", [(7, 30), (64, 4), (1, 211), (300, 1), (100, 2)])
 def test_segment_offsets_are_what_a_search_finds(span, n_groups):
     """Empty rows, rows of one synapse and of several chunks, repeated targets, targets beyond the last group, first and last groups empty."""
