@@ -388,8 +388,9 @@ class SynapseTable:
         return _range_rows_min(nnz / self.n_rows, n_tgt * batch, ring_slots)
 
     def ranges(self, n_tgt):
-        """Segment offsets of the rows by ``RANGES`` ranges of targets, or None for a table whose rows are not sorted by index.
-        Made once per table and row bounds (synchronises then).  What a delivery adds does not depend on them: bounds rewritten in a way
+        """Segment offsets of the rows by ``RANGES`` ranges of targets, or None for a table whose rows are not sorted by index and where
+        there is no room for them: 1,028 bytes a row (at the 100 synapses from which a row is worth it as many again as its synapses take),
+        kept as long as the table.  Made once per table and row bounds (synchronises then).  What a delivery adds does not depend on them: bounds rewritten in a way
         that the version counter does not see (a replayed graph, ``.data``, a caller's kernel) make it slower, not wrong.  None while a
         graph is being captured: its replays would read the offsets after others have replaced them."""
         if torch._C._cuda_isCurrentStreamCapturing():
@@ -400,7 +401,7 @@ class SynapseTable:
         if plan is None or plan[0] is not indptr or plan[1] != version or plan[2] != (n_tgt, self.n_rows):
             try:
                 seg = self.segment_offsets(-(-n_tgt // self.RANGES), self.RANGES)
-            except ValueError:
+            except (ValueError, torch.OutOfMemoryError):
                 seg = None
             plan = self._ranges = (indptr, version, (n_tgt, self.n_rows), seg, _stream())
         elif plan[3] is not None and plan[4] != _stream():

@@ -413,6 +413,27 @@ def test_delivery_by_target_ranges_of_a_table_made_under_inference_mode(sort):
     assert (table.ranges(n) is not None) == sort
 
 
+def test_delivery_where_the_offsets_find_no_room(monkeypatch):
+    """The walk takes the call, and does not ask for the memory again."""
+    rng = np.random.default_rng(9)
+    n, L, nnz = 600, 6, 600 * 150
+    src, tgt, w, d, r = _edges(rng, n, n, nnz)
+    w = (np.round(w * 4) / 4).astype(np.float32)
+    table, other = (ops.SynapseTable.from_edges(src, tgt, w, d, r, n, n) for _ in range(2))
+    ids, count = torch.arange(n, device="cuda", dtype=torch.int32), torch.tensor([n], device="cuda", dtype=torch.int32)
+    want, got = torch.zeros(L, 4, n, device="cuda"), torch.zeros(L, 4, n, device="cuda")
+    ops.csr_propagate_scatter(ids, count, other, want, n, 1, 4)
+    asked = []
+
+    def no_room(self, *a):
+        asked.append(a)
+        raise torch.OutOfMemoryError("none left")
+    monkeypatch.setattr(ops.SynapseTable, "segment_offsets", no_room)
+    for _ in range(2):
+        ops.csr_propagate_scatter(ids, count, table, got.zero_(), n, 1, 4)
+        assert torch.equal(want, got) and len(asked) == 1
+
+
 @pytest.mark.parametrize("span,n_groups", [(7, 30), (64, 4), (1, 211), (300, 1), (100, 2)])
 def test_segment_offsets_are_what_a_search_finds(span, n_groups):
     """Empty rows, rows of one synapse and of several chunks, repeated targets, targets beyond the last group, first and last groups empty."""
