@@ -408,6 +408,17 @@ class SynapseTable:
             plan[3].record_stream(torch.cuda.current_stream())   # (replaced offsets are not reused under a launch of another stream)
         return plan[3]
 
+    def pull_workspace(self, need, device):
+        """``need`` bytes of scratch memory for a pull, which one launch of a call writes and the next reads: the calling stream's own.  The
+        last stream's is kept (what is let go belongs to the stream that worked with it, so that it is not reused under its launches); a
+        graph being captured gets memory of its own, which neither later calls nor other graphs write to."""
+        if torch._C._cuda_isCurrentStreamCapturing():
+            return torch.empty(need // 4 + 1, dtype=torch.int32, device=device)
+        kept, stream = getattr(self, "_pull_ws", None), _stream()
+        if kept is None or kept[0] != stream or kept[1].numel() * 4 < need:
+            kept = self._pull_ws = (stream, torch.empty(need // 4 + 1, dtype=torch.int32, device=device))
+        return kept[1]
+
     def pointers(self):
         nnz = self.nnz
         return (_p(self.indptr, torch.int32, self.n_rows + 1, "indptr"), _p(self.indices, torch.int32, nnz, "indices"),
@@ -462,10 +473,7 @@ def csr_propagate_pull(spike_hist, n_src, table, syn, n_tgt, batch, t_arrive):
     L = spike_hist.shape[0]
     if table.max_delay() >= L:
         raise ValueError("spike history of {} steps is shorter than the largest delay".format(L))
-    ws = getattr(table, "_pull_ws", None)
-    need = lib.bmtk_csr_propagate_pull_workspace_bytes(L, n_src)
-    if ws is None or ws.numel() * 4 < need:
-        ws = table._pull_ws = torch.zeros(need // 4 + 1, dtype=torch.int32, device=syn.device)
+    ws = table.pull_workspace(lib.bmtk_csr_propagate_pull_workspace_bytes(L, n_src), syn.device)
     _lib.check(lib.bmtk_csr_propagate_pull(_p(spike_hist, torch.int64), spike_hist.shape[1], L, n_src, batch,
                                            _p(table.indptr), _p(table.packed()), _p(syn, torch.float32), n_tgt,
                                            int(t_arrive), _p(ws), _stream()))
@@ -481,10 +489,7 @@ def csr_propagate_pull2(spike_hist, n_src, table, syn2, n_tgt, batch, t_arrive):
     L = spike_hist.shape[0]
     if table.max_delay() >= L:
         raise ValueError("spike history of {} steps is shorter than the largest delay".format(L))
-    ws = getattr(table, "_pull_ws", None)
-    need = lib.bmtk_csr_propagate_pull_workspace_bytes(L, n_src)
-    if ws is None or ws.numel() * 4 < need:
-        ws = table._pull_ws = torch.zeros(need // 4 + 1, dtype=torch.int32, device=syn2.device)
+    ws = table.pull_workspace(lib.bmtk_csr_propagate_pull_workspace_bytes(L, n_src), syn2.device)
     _lib.check(lib.bmtk_csr_propagate_pull2(_p(spike_hist, torch.int64), spike_hist.shape[1], L, n_src, batch,
                                             _p(table.indptr), _p(table.packed()), _p(syn2, torch.float32), n_tgt,
                                             int(t_arrive), _p(ws), _stream()))

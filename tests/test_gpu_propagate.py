@@ -481,6 +481,51 @@ def test_two_step_pull_equals_two_pulls(batch, p, n_src, L):
         assert float(one[0].abs().max()) > 0 and not torch.equal(one[0], one[1])
 
 
+@pytest.mark.parametrize("batch,L,two", [(64, 6, True), (12, 6, True), (64, 9, True), (100, 6, True), (64, 6, False)])
+def test_pulls_of_one_table_on_two_streams_and_in_a_graph(batch, L, two):
+    """Two streams at work at once with histories of their own, and a captured call replayed beside them:
+    none reads what another call has laid out."""
+    rng = np.random.default_rng(batch + L)
+    n_src, n_tgt, reps = 20000, 3000, 30
+    src, tgt, w, d, r = _edges(rng, n_src, n_tgt, 400000, max_delay=L - 1)
+    table = ops.SynapseTable.from_numpy(net.coo_to_csr(src, tgt, w, d, r, n_rows=n_tgt, major="target"))
+    words = ops.n_words(n_src * batch)
+    hist = [torch.zeros(L, words + 1, dtype=torch.int64, device="cuda") for _ in range(3)]
+    for h in hist:
+        h[:, :-1] = torch.as_tensor(rng.integers(0, 2**62, (L, words)) & rng.integers(0, 2**62, (L, words)) & rng.integers(0, 2**62, (L, words)), device="cuda")
+    out = lambda: torch.zeros(2 if two else 1, 4, n_tgt * batch, device="cuda")  # noqa: E731
+
+    def pull(h, to):
+        if two:
+            ops.csr_propagate_pull2(h, n_src, table, to, n_tgt, batch, L)
+        else:
+            ops.csr_propagate_pull(h, n_src, table, to, n_tgt, batch, L)
+
+    want = [out() for _ in hist]
+    for h, x in zip(hist, want):
+        pull(h, x)
+        torch.cuda.synchronize()
+    assert not torch.equal(want[0], want[1])
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    got = [[out() for _ in range(reps)] for _ in streams]
+    graph, replayed = torch.cuda.CUDAGraph(), out()
+    with torch.cuda.graph(graph):
+        pull(hist[2], replayed)
+    torch.cuda.synchronize()
+    for k in range(reps):
+        for s, h, g in zip(streams, hist, got):
+            with torch.cuda.stream(s):
+                pull(h, g[k])
+        replayed.zero_()
+        graph.replay()
+        if k % 10 == 9:
+            torch.cuda.current_stream().synchronize()
+            assert torch.equal(replayed, want[2])
+    torch.cuda.synchronize()
+    for g, x in zip(got, want):
+        assert all(torch.equal(y, x) for y in g)
+
+
 @pytest.mark.parametrize("n_tgt,nnz,batch,power", [(3, 4000, 64, 1.0), (5000, 70000, 33, 6.0), (9001, 8500000, 32, 3.0), (40000, 8400000, 8, 8.0)])
 def test_two_step_pull_of_rows_of_very_unequal_length(n_tgt, nnz, batch, power):
     """Targets drawn as n * x**power: rows from several tenths of the table down to none, empty ones first and last, on either side
