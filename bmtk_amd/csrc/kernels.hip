@@ -121,11 +121,16 @@ struct StepArgs {
 // division per word, one word per load) took 19.8 / 20.2 with four tiles.  By measured bytes the launch then moves
 // 5.95 TB/s where the form with a column per neuron moved 6.15 TB/s on the same machine.
 //
-// While all workgroups of one tile are resident at once (eight on a compute unit: 524,288 elements on 256 of them) there is
-// nothing to share the staging with, and four tiles a workgroup leave compute units idle: 30,011 elements are 30 workgroups.  One tile / four,
-// us: 5,000 elements 3.3 / 5.7, 30,011 3.6 / 6.0, 100,000 4.2 / 6.3, 200,000 5.7 / 7.2, 400,000 8.6 / 9.6, 2^20 24.9 / 22.6.
+// While all workgroups of one tile are resident at once there is nothing to share the staging with, and four tiles a workgroup leave compute
+// units idle: 30,011 elements are 30 workgroups.  Seven of them fit a compute unit by their 72 registers a thread, fewer by the table: five
+// of 250 classes (29 KB), three of 423 (49 KB).  One tile / four, us a call (of a loop of calls: not below 5.2 on the host), by classes:
+//   37: 200,000 elements 5.4 / 6.2, 440,000 7.1 / 7.4, 524,288 7.9 / 7.8     111: 5.3 / 6.4, 7.2 / 7.7, 8.4 / 7.9     176: 5.2 / 6.9, 7.7 / 8.0, 8.9 / 8.4
+//   200 (six): 350,000 7.0 / 7.9, 400,000 8.1 / 8.0          250 (five): 327,680 6.6 / 7.9, 350,000 8.8 / 8.2
+//   300 (four): 262,144 6.2 / 7.5, 327,680 8.5 / 8.2         423 (three): 196,608 5.7 / 7.6, 230,924 8.9 / 8.1, 524,288 13.0 / 9.8
+// (kernels alone at 5,000, 30,011 and 100,000 elements: 111 classes 3.7 / 5.6, 3.8 / 6.1, 4.2 / 6.3; 423 classes 4.8 / 6.8, 4.9 / 7.4, 5.5 / 7.6.)
 constexpr int kStepTiles = 4;
-constexpr int kStepResident = 2048;  // workgroups of 256 threads that 256 compute units hold
+constexpr int kStepPerCu = 7;                 // workgroups of one tile on a compute unit
+constexpr size_t kLdsPerCu = 160u * 1024u, kLdsUnit = 1280u;  // LDS of a compute unit, and what it is given out in
 
 // kTilesOrNone: tiles of a workgroup that stages the class table in LDS; 0: the table is not staged
 template <int kTilesOrNone>
@@ -743,6 +748,21 @@ __global__ __launch_bounds__(kBlock) void gather_kernel(const uint64_t *__restri
 
 using namespace bmtk;
 
+// of the current device (asked for once)
+static unsigned compute_units()
+{
+    static int count[64];
+    int dev = 0;
+    (void)hipGetDevice(&dev);
+    int n = dev >= 0 && dev < 64 ? count[dev] : 0;
+    if (n <= 0) {
+        n = 256;
+        (void)hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev);
+        if (dev >= 0 && dev < 64) count[dev] = n;
+    }
+    return (unsigned)n;
+}
+
 extern "C" {
 
 int bmtk_amd_abi_version(void) { return BMTK_AMD_ABI_VERSION; }
@@ -781,7 +801,9 @@ int bmtk_glif3_step_fwd(int64_t n_neurons, int32_t batch, float *V, float *asc, 
     // table that is not 16-byte aligned is read through the caches instead)
     const size_t table_bytes = (size_t)prop_stride * GLIF3_NPROP * sizeof(float);
     if (class_id && table_bytes <= 48u * 1024u && ((uintptr_t)prop & 15u) == 0) {
-        if (grid <= kStepResident)
+        const size_t fit = kLdsPerCu / ((table_bytes + kLdsUnit - 1) / kLdsUnit * kLdsUnit);
+        const unsigned per_cu = fit < (size_t)kStepPerCu ? (unsigned)fit : (unsigned)kStepPerCu;
+        if (grid <= per_cu * compute_units())
             hipLaunchKernelGGL(glif3_step_kernel<1>, dim3(grid), dim3(kBlock), table_bytes, (hipStream_t)stream, a);
         else
             hipLaunchKernelGGL(glif3_step_kernel<kStepTiles>, dim3((grid + kStepTiles - 1) / kStepTiles), dim3(kBlock), table_bytes,

@@ -139,13 +139,15 @@ def test_class_table_in_any_size_and_alignment_equals_one_column_per_neuron(clas
             np.testing.assert_array_equal(got[name][0][k], v, err_msg="%s %s" % (name, k))
 
 
-@pytest.mark.parametrize("n,batch", [(255, 1), (257, 1), (524288, 1), (524289, 1), (525313, 1), (174763, 3), (174762, 3)])
-def test_class_table_with_one_and_with_several_tiles_a_workgroup(n, batch):
-    """On either side of the 2,048 workgroups up to which each takes one tile of 256 elements, with a last workgroup of one element: state,
-    spikes, cleared arrivals and fractions of one column per neuron, bit for bit."""
+@pytest.mark.parametrize("n,batch,classes", [(255, 1, 9), (257, 1, 9), (524288, 1, 9), (524289, 1, 9), (525313, 1, 9), (174763, 3, 9), (174762, 3, 9),
+                                             (458752, 1, 9), (458753, 1, 9), (152918, 3, 9), (393216, 1, 200), (393217, 1, 200), (196608, 1, 423),
+                                             (196609, 1, 423), (65537, 3, 423), (300, 1, 423)])
+def test_class_table_with_one_and_with_several_tiles_a_workgroup(n, batch, classes):
+    """On either side of the workgroups of one tile of 256 elements that are resident at once (seven on each of 256 compute units, fewer by
+    the table's size), with a last workgroup of one element: state, spikes, cleared arrivals and fractions of one column per neuron, bit for bit."""
     rng = np.random.default_rng(n)
-    par = synthetic.random_cells(rng, 9)
-    class_id = rng.integers(0, 9, n).astype(np.int32)
+    par = synthetic.random_cells(rng, classes)
+    class_id = rng.integers(0, classes, n).astype(np.int32)
     p32 = orc.precompute(par, 1.0).astype(np.float32)
     st0 = synthetic.random_state(rng, par, n, batch, class_id)
     arrivals, current = rng.normal(0, 300, (4, n * batch)).astype(np.float32), rng.normal(5000, 2000, n * batch).astype(np.float32)
