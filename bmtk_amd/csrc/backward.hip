@@ -537,17 +537,19 @@ constexpr size_t blk2_sort_bytes(size_t rows_sweep)
 // (and bounds) of a whole visit are asked for at once, a visit ahead, behind a barrier; the barriers also keep the
 // wavefronts within a range, so that its adjoint rows stay in the L2 (misses 46 M -> 12 M lines of 107 M).  And a wavefront's
 // eight rows take as long as the longest of them: 30 % of the lanes' work at 42 records a segment, which is why a sweep's rows
-// are sorted by the length of their segment before every range (and by whether they fired: the gradient's work).
+// are sorted by the length of their segment before every range (and by whether they fired: the gradient's work).  Rows that fired are not gathered into
+// sweeps of their own, as bwd_gather_blocked_kernel gathers them: within a sweep the sort does it, and sweeps of like work are no slower (us per step with a list
+// of all rows / without, one row in five fired: 51978 x 32, in-degree 1000: 416 / 413; 100000 x 32, 300: 470 / 455; 30000 x 64, 600: 317 / 310).
 // 51978 neurons x 32 trials, in-degree 1000, us per launch: as before 1025, with bursts and barriers 880, rows sorted 787, a visit
 // ahead and two records a lane 750; of these 35 are the gradients' read-modify-writes and 50 the input gradients in the tail.
 // Tried: records without a place in the caches (nontemporal, 3 % slower), gradients as atomic additions (1 %), their
 // old values fetched with the records (spills, 2 %).
 template <int kLp, bool kGrad, bool kNe24>
 __global__ __launch_bounds__(kBlkThreads) void bwd_gather_blocked2_kernel(bmtk_glif3_bwd a, BwdStep q, int rows_cu, int sweeps,
-                                                                          int gpw, int use_order, int do_inp)
+                                                                          int gpw, int do_inp)
 {
-    // partial sums [rows of a sweep][2][kLp], the sweep's fired trials, segment bounds, places in the order of the visits and
-    // rows, the counters of the sort, then the row order (uint16 per place)
+    // partial sums [rows of a sweep][2][kLp], the sweep's fired trials, segment bounds, the counters of the sort, places in the
+    // order of the visits
     extern __shared__ float4 blk_acc[];
     constexpr int kBurst = kBlkBurst;
     constexpr int per = kWave / kLp;
@@ -582,50 +584,11 @@ __global__ __launch_bounds__(kBlkThreads) void bwd_gather_blocked2_kernel(bmtk_g
     unsigned *count_l = reinterpret_cast<unsigned *>(bounds_l + 2 * rows_sweep);     // [2 * kBlkLengthKeys]
     uint16_t *visit_l = reinterpret_cast<uint16_t *>(count_l + 2 * kBlkLengthKeys);  // [2][rows_sweep]: place of a visit's row
     uint16_t *wanted_l = visit_l + 2 * rows_sweep;                                   // by place: whether its row has visits
-    uint16_t *order = wanted_l + rows_sweep;
     const uint64_t *__restrict__ bits_t = a.spike_bits + q.row * a.spike_bits_stride;
     const uint64_t *__restrict__ bits_p = a.spike_bits + (q.row - 1) * a.spike_bits_stride;
-    const int places = sweeps * rows_sweep;
-    if (kGrad && use_order) {  // rows whose source fired in one of the two steps first (see bwd_gather_blocked_kernel)
-        __shared__ unsigned scan_l[2][kBlkWaves];
-        unsigned fm = 0u, n_mine = 0u;
-        for (int i = 0; (int)threadIdx.x + i * kBlkThreads < rows_cu; ++i) {
-            const int64_t j = row_lo + threadIdx.x + i * kBlkThreads;
-            if (j < row_hi && (trial_mask(bits_t, j, batch, 0, batch) | trial_mask(bits_p, j, batch, 0, batch)) != 0ull)
-                fm |= 1u << i;
-            ++n_mine;
-        }
-        const unsigned c1 = (unsigned)__popc(fm), c0 = n_mine - c1;
-        const unsigned in1 = wave_inclusive_scan(c1), in0 = wave_inclusive_scan(c0);
-        if (lane == kWave - 1) {
-            scan_l[0][wave] = in0;
-            scan_l[1][wave] = in1;
-        }
-        __syncthreads();
-        unsigned base0 = 0u, base1 = 0u, total1 = 0u;
-#pragma unroll
-        for (int w = 0; w < kBlkWaves; ++w) {
-            if (w < wave) {
-                base0 += scan_l[0][w];
-                base1 += scan_l[1][w];
-            }
-            total1 += scan_l[1][w];
-        }
-        unsigned at1 = base1 + in1 - c1, at0 = total1 + base0 + in0 - c0;
-        for (unsigned i = 0; i < n_mine; ++i) {
-            const unsigned local = threadIdx.x + i * kBlkThreads;
-            if ((fm >> i) & 1u)
-                order[at1++] = (uint16_t)local;
-            else
-                order[at0++] = (uint16_t)local;
-        }
-        for (int i = rows_cu + (int)threadIdx.x; i < places; i += kBlkThreads) order[i] = 0xFFFFu;
-        __syncthreads();
-    }
     // the row at a place of sweep sw, counted from the workgroup's first (0xFFFFFFFF: none)
     auto row_at = [&](int sw, int place) -> unsigned {
         place += sw * rows_sweep;
-        if (kGrad && use_order) return order[place] == 0xFFFFu ? ~0u : order[place];
         return place < rows_cu && row_lo + place < row_hi ? (unsigned)place : ~0u;
     };
     for (int i = threadIdx.x; i < 2 * kBlkLengthKeys; i += kBlkThreads) count_l[i] = 0u;
@@ -1663,7 +1626,7 @@ struct BlockedPlan {
     int lp, rows_cu, sweeps, gpw, use_order;
     size_t lds;
     // the two-step kernel: twice the LDS per row, hence half as many row groups per wavefront and sweep
-    int sweeps2, gpw2, use_order2;
+    int sweeps2, gpw2;
     size_t lds2;
 };
 constexpr size_t kBlkLdsMax = 160u * 1024u - 256u;  // a compute unit's LDS less the kernel's static part
@@ -1700,9 +1663,6 @@ int blocked_plan(const bmtk_glif3_bwd &a, BlockedPlan &pl)
     pl.sweeps2 = (int)((rows_cu + cap2 - 1) / cap2);
     pl.gpw2 = (int)((rows_cu + (int64_t)pl.sweeps2 * kBlkWaves * per - 1) / ((int64_t)pl.sweeps2 * kBlkWaves * per));
     pl.lds2 = (size_t)kBlkWaves * pl.gpw2 * 2 * kWave * sizeof(float4) + blk2_sort_bytes((size_t)kBlkWaves * pl.gpw2 * per);
-    const size_t order_bytes2 = (size_t)pl.sweeps2 * kBlkWaves * pl.gpw2 * per * sizeof(uint16_t);
-    pl.use_order2 = (pl.lds2 + order_bytes2 <= kBlkLdsMax && rows_cu <= 16 * kBlkThreads && rows_cu < 0xFFFF) ? 1 : 0;
-    if (pl.use_order2) pl.lds2 += order_bytes2;
     static bool asked[8][64];
     const void *variants[8];
     for (int g = 0; g < 8; ++g) variants[g] = blocked_variant(g & 4, g & 2, g & 1);
@@ -1766,9 +1726,9 @@ int blocked2_launch(const bmtk_glif3_bwd &a, const BwdStep &q, const BlockedPlan
     const bool ne24 = a.n_neurons * (int64_t)a.batch < (1ll << 24);
     bmtk_glif3_bwd args = a;
     BwdStep step = q;
-    int rows_cu = pl.rows_cu, sweeps = pl.sweeps2, gpw = pl.gpw2, use_order = pl.use_order2;
+    int rows_cu = pl.rows_cu, sweeps = pl.sweeps2, gpw = pl.gpw2;
     int do_inp = inp_grad ? 1 : 0;
-    void *params[] = {&args, &step, &rows_cu, &sweeps, &gpw, &use_order, &do_inp};
+    void *params[] = {&args, &step, &rows_cu, &sweeps, &gpw, &do_inp};
     const hipError_t err = hipLaunchKernel(blocked2_variant(pl.lp > 8, grad, ne24), dim3(pl.grid), dim3(kBlkThreads), params, pl.lds2, st);
     if (err != hipSuccess) {
         set_error("transposed propagation (two steps): launch failed: %s", hipGetErrorString(err));
