@@ -90,6 +90,10 @@ class Glif3Bptt:
     # 13000 x 32, 120 35/37; 15000 x 32, 220 52/47; 5000 x 64, 300 42/38; 6500 x 64, 150 39/38; 4000 x 48, 900 64/53
     BLOCKED_MIN_RING_MB_TWO = 25.5
     BLOCKED_MIN_RING_MB_RAGGED = 22.0, 20.0   # other batches up to 16, and above (where it takes two steps per pass)
+    # more than 16 trials and two_steps=False, whole lines and others, times the cube root.  Swept / blocked, us per step: 9003 x 32, in-degree 750 75/82;
+    # 15000 x 32, 220 55/67, 500 95/94; 20011 x 32, 220 84/84; 30011 x 32, 120 101/110, 400 222/175; 15013 x 20, 220 60/68, 750 161/133; 12000 x 24, 300
+    # 60/68; 8000 x 40, 300 58/70; 12000 x 40, 300 104/93
+    BLOCKED_MIN_RING_MB_ONE = 50.0, 32.0
     BLOCKED_MIN_RING_MB_FOUR = 17.0     # four trials: a quarter of a line
     # Four trials through a table of more than 150 MB, which does not stay in the memory-side cache beside the rest: launches of
     # their own for the parts (27011 x 4, in-degree 750: 139 against 147 swept; 33123 x 4, 598: 155 against 187 and 169 blocked;
@@ -97,12 +101,13 @@ class Glif3Bptt:
     PLAIN_MIN_TABLE_BYTES = 150e6
 
     @classmethod
-    def blocked_pays(cls, n, batch, ring_slots, nnz):
-        """Whether the blocked form is expected to take less time per step than the swept form."""
+    def blocked_pays(cls, n, batch, ring_slots, nnz, two_steps=True):
+        """Whether the blocked form is expected to take less time per step than the swept form.  ``two_steps``: as it will be built."""
         ring_mb = ring_slots * NREC * n * batch * 4e-6
-        if batch % 16 == 0 and batch > 16:
+        if batch % 16 == 0 and batch > 16 and two_steps:
             return ring_mb * (nnz / (400.0 * n)) ** 0.5 >= cls.BLOCKED_MIN_RING_MB_TWO
-        least = (cls.BLOCKED_MIN_RING_MB if batch % 16 == 0 else cls.BLOCKED_MIN_RING_MB_FOUR if batch <= 4
+        least = (cls.BLOCKED_MIN_RING_MB_ONE[batch % 16 != 0] if batch > 16 and not two_steps else
+                 cls.BLOCKED_MIN_RING_MB if batch % 16 == 0 else cls.BLOCKED_MIN_RING_MB_FOUR if batch <= 4
                  else cls.BLOCKED_MIN_RING_MB_RAGGED[batch > 16])
         return ring_mb * (nnz / (400.0 * n)) ** (1.0 / 3.0) >= least
 
@@ -150,7 +155,7 @@ class Glif3Bptt:
         if blocked and not can_block:
             raise ValueError("the blocked table needs a recurrent table and a batch that is a multiple of 4 up to 64")
         if blocked is None and not swept:
-            blocked = can_block and (swept is False or not can_sweep or self.blocked_pays(sim.n, sim.batch, sim.L, sim.rec.nnz))
+            blocked = can_block and (swept is False or not can_sweep or self.blocked_pays(sim.n, sim.batch, sim.L, sim.rec.nnz, two_steps))
             swept = not blocked and can_sweep and swept is None and not self.plain_pays(sim.batch, sim.rec.nnz)
         self.swept, blocked = bool(swept), bool(blocked)
         # (the swept form writes the adjoint slots of two steps ahead while others are still read)

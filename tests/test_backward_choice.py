@@ -34,6 +34,19 @@ def test_choice_for_two_steps_per_pass(n, batch, k, swept, blocked):
     assert (blocked if Glif3Bptt.blocked_pays(n, batch, 6, n * k) else swept) <= 1.05 * min(swept, blocked)
 
 
+# one step per pass: neurons, trials, in-degree, us per step swept / blocked
+ONE_STEP = [(9003, 32, 400, 45.8, 61.1), (9003, 32, 750, 75.1, 82.3), (7000, 32, 600, 45.8, 60.5), (15000, 32, 220, 55.3, 67.2), (15000, 32, 500, 95.2, 93.7),
+            (5000, 64, 300, 41.3, 56.9), (4000, 48, 900, 62.9, 73.2), (30011, 32, 120, 101.0, 110.4), (20011, 32, 220, 83.7, 84.1), (20011, 32, 60, 45.9, 63.8),
+            (30011, 32, 400, 222.1, 174.7), (51978, 32, 220, 277.5, 248.6), (40000, 64, 150, 320.3, 337.8), (9003, 20, 400, 53.8, 63.0), (15013, 20, 220, 59.9, 67.7),
+            (15013, 20, 750, 161.1, 132.5), (25013, 20, 300, 175.0, 123.1), (12000, 24, 300, 59.5, 67.5), (20000, 24, 300, 127.2, 103.9), (8000, 40, 300, 58.4, 69.6),
+            (12000, 40, 300, 103.8, 93.2)]
+
+
+@pytest.mark.parametrize("n,batch,k,swept,blocked", ONE_STEP)
+def test_choice_for_one_step_per_pass(n, batch, k, swept, blocked):
+    assert (blocked if Glif3Bptt.blocked_pays(n, batch, 6, n * k, two_steps=False) else swept) <= 1.1 * min(swept, blocked)
+
+
 # neurons, trials, in-degree, us per two steps with 8 / 16 / 24 target ranges
 RANGES = [(52000, 32, 100, 280.4, 291.4, 312.8), (25000, 40, 120, 211.7, 225.7, 246.1), (12000, 64, 150, 132.1, 135.1, 141.0), (45000, 40, 200, 516.5, 503.4, 530.0),
           (31000, 64, 300, 489.9, 461.7, 472.1), (20000, 20, 300, 147.6, 145.1, 148.7), (40000, 24, 400, 389.8, 368.1, 366.3), (30011, 32, 600, 331.4, 314.3, 315.1),

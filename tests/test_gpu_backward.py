@@ -251,6 +251,14 @@ def test_backward_parts_argument_errors():
     assert "neither" in lib.bmtk_amd_last_error().decode()
 
 
+def test_choice_of_form_is_told_the_steps_per_pass(monkeypatch):
+    cfg = _net(32, 4, steps=5)
+    sim = Glif3Simulator(cfg["n"], cfg["par"], cfg["h"], batch=32, rec=cfg["rec_src"], inp=cfg["inp_src"], ring_slots=cfg["L"], resident=False)
+    monkeypatch.setattr(training.Glif3Bptt, "blocked_pays", staticmethod(lambda n, batch, ring_slots, nnz, two_steps=True: two_steps))
+    two, one = training.Glif3Bptt(sim), training.Glif3Bptt(sim, two_steps=False)
+    assert two.blk is not None and not two.swept and one.blk is None and one.swept
+
+
 @pytest.mark.parametrize("batch,seed,n_blocks,steps", [(32, 9, 16, 70), (64, 3, 8, 69), (20, 5, 8, 33), (32, 11, 8, 3),
                                                         (32, 12, 8, 4)])
 def test_two_steps_per_pass_of_the_blocked_form_equal_one(batch, seed, n_blocks, steps):
