@@ -139,15 +139,13 @@ def test_class_table_in_any_size_and_alignment_equals_one_column_per_neuron(clas
             np.testing.assert_array_equal(got[name][0][k], v, err_msg="%s %s" % (name, k))
 
 
-@pytest.mark.parametrize("n,batch,classes", [(255, 1, 9), (257, 1, 9), (524288, 1, 9), (524289, 1, 9), (525313, 1, 9), (174763, 3, 9), (174762, 3, 9),
-                                             (458752, 1, 9), (458753, 1, 9), (152918, 3, 9), (393216, 1, 200), (393217, 1, 200), (196608, 1, 423),
-                                             (196609, 1, 423), (65537, 3, 423), (300, 1, 423)])
-def test_class_table_with_one_and_with_several_tiles_a_workgroup(n, batch, classes):
-    """On either side of the workgroups of one tile of 256 elements that are resident at once (seven on each of 256 compute units, fewer by
-    the table's size), with a last workgroup of one element: state, spikes, cleared arrivals and fractions of one column per neuron, bit for bit."""
+@pytest.mark.parametrize("n,batch", [(255, 1), (257, 1), (524288, 1), (524289, 1), (525313, 1), (174763, 3), (174762, 3)])
+def test_class_table_with_one_and_with_several_tiles_a_workgroup(n, batch):
+    """On either side of the 2,048 workgroups up to which each takes one tile of 256 elements, with a last workgroup of one element: state,
+    spikes, cleared arrivals and fractions of one column per neuron, bit for bit."""
     rng = np.random.default_rng(n)
-    par = synthetic.random_cells(rng, classes)
-    class_id = rng.integers(0, classes, n).astype(np.int32)
+    par = synthetic.random_cells(rng, 9)
+    class_id = rng.integers(0, 9, n).astype(np.int32)
     p32 = orc.precompute(par, 1.0).astype(np.float32)
     st0 = synthetic.random_state(rng, par, n, batch, class_id)
     arrivals, current = rng.normal(0, 300, (4, n * batch)).astype(np.float32), rng.normal(5000, 2000, n * batch).astype(np.float32)
@@ -160,6 +158,29 @@ def test_class_table_with_one_and_with_several_tiles_a_workgroup(n, batch, class
             ops.glif3_step_fwd(st, prop, 1.0, batch=batch, class_id=cid, syn=syn, clear_syn=True, i_ext=to_dev(current), z=z, zbits=zb, frac=frac)
         got.append((st.V, st.asc, st.y1, st.y2, st.ref, syn, zb, z, frac))
     assert float(got[0][8].abs().max()) > 0 and float(got[0][5].abs().max()) == 0
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("n,batch,classes", [(458752, 1, 9), (458753, 1, 9), (152918, 3, 9), (393216, 1, 200), (393217, 1, 200), (196608, 1, 423),
+                                             (196609, 1, 423), (65537, 3, 423), (300, 1, 423)])
+def test_class_table_on_either_side_of_the_workgroups_resident_at_once(n, batch, classes):
+    """One tile of 256 elements a workgroup while all workgroups are resident at once (seven on each of 256 compute units, fewer by the table's
+    size), several beyond, with a last workgroup of one element: state, spikes and fractions of one column per neuron, bit for bit."""
+    rng = np.random.default_rng(n)
+    par = synthetic.random_cells(rng, classes)
+    class_id = rng.integers(0, classes, n).astype(np.int32)
+    p32 = orc.precompute(par, 1.0).astype(np.float32)
+    st0 = synthetic.random_state(rng, par, n, batch, class_id)
+    arrivals, current = rng.normal(0, 300, (4, n * batch)).astype(np.float32), rng.normal(5000, 2000, n * batch).astype(np.float32)
+    got = []
+    for prop, cid in ((to_dev(np.ascontiguousarray(p32[:, class_id])), None), (to_dev(p32), to_dev(class_id))):
+        st, syn = ops.Glif3State.from_numpy(st0), to_dev(arrivals)
+        zb, frac = torch.zeros(ops.n_words(n * batch) + 1, dtype=torch.int64, device="cuda"), torch.zeros(n * batch, device="cuda")
+        for _ in range(2):
+            ops.glif3_step_fwd(st, prop, 1.0, batch=batch, class_id=cid, syn=syn, clear_syn=True, i_ext=to_dev(current), zbits=zb, frac=frac)
+        got.append((st.V, st.asc, st.y1, st.y2, st.ref, syn, zb, frac))
+    assert float(got[0][7].abs().max()) > 0
     for a, b in zip(*got):
         assert torch.equal(a, b)
 
