@@ -526,6 +526,41 @@ def test_pulls_of_one_table_on_two_streams_and_in_a_graph(batch, L, two):
         assert all(torch.equal(y, x) for y in g)
 
 
+@pytest.mark.parametrize("two", [True, False])
+def test_pulls_of_one_table_from_two_threads_share_no_scratch_memory(monkeypatch, two):
+    """A call that begins while another thread's is under way, on the same stream, works in memory of its own: the launches of the two
+    may come in any order."""
+    import threading
+    from bmtk_amd import _lib
+    rng = np.random.default_rng(3)
+    n, L, batch = 500, 6, 64
+    src, tgt, w, d, r = _edges(rng, n, n, 20000)
+    table = ops.SynapseTable.from_numpy(net.coo_to_csr(src, tgt, w, d, r, n_rows=n, major="target"))
+    hist = torch.zeros(L, ops.n_words(n * batch) + 1, dtype=torch.int64, device="cuda")
+    hist[:, :-1] = 0x0101010101010101
+    name, f = ("bmtk_csr_propagate_pull2", ops.csr_propagate_pull2) if two else ("bmtk_csr_propagate_pull", ops.csr_propagate_pull)
+    real, scratch = _lib.load(), []
+    out = [torch.zeros(2 if two else 1, 4, n * batch, device="cuda") for _ in range(2)]
+
+    class Lib:
+        def __getattr__(self, what):
+            return getattr(real, what) if what != name else self.pull
+
+        def pull(self, *args):
+            scratch.append(args[-2])
+            if len(scratch) == 1:
+                other = threading.Thread(target=f, args=(hist, n, table, out[1], n, batch, L))
+                other.start()
+                other.join()
+            return getattr(real, name)(*args)
+
+    monkeypatch.setattr(_lib, "load", lambda *a, **k: lib)
+    lib = Lib()
+    f(hist, n, table, out[0], n, batch, L)
+    assert len(scratch) == 2 and scratch[0] != scratch[1]
+    assert torch.equal(*out) and float(out[0].abs().max()) > 0
+
+
 @pytest.mark.parametrize("n_tgt,nnz,batch,power", [(3, 4000, 64, 1.0), (5000, 70000, 33, 6.0), (9001, 8500000, 32, 3.0), (40000, 8400000, 8, 8.0)])
 def test_two_step_pull_of_rows_of_very_unequal_length(n_tgt, nnz, batch, power):
     """Targets drawn as n * x**power: rows from several tenths of the table down to none, empty ones first and last, on either side
