@@ -366,9 +366,10 @@ class SynapseTable:
         """uint32 [n_rows, n_groups+1] offsets of the first synapse per row whose index is >= g*span
         (stored in an int32 tensor, ``out`` if given).  Raises if a row is not sorted by index."""
         lib = _lib.load()
+        bounds = _p(self.indptr, torch.int32, self.n_rows + 1, "indptr"), _p(self.indices, torch.int32, None, "indices")
         seg = torch.empty(self.n_rows, n_groups + 1, dtype=torch.int32, device=self.indices.device) if out is None else out
         flag = torch.zeros(1, dtype=torch.int32, device=self.indices.device)
-        _lib.check(lib.bmtk_csr_segment_offsets(self.n_rows, _p(self.indptr), _p(self.indices), span, n_groups,
+        _lib.check(lib.bmtk_csr_segment_offsets(self.n_rows, *bounds, span, n_groups,
                                                 _p(seg, torch.int32, self.n_rows * (n_groups + 1), "out"), _p(flag), _stream()))
         if int(flag.item()):
             raise ValueError("synapse table rows are not sorted by index")

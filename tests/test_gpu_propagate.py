@@ -434,6 +434,21 @@ def test_delivery_where_the_offsets_find_no_room(monkeypatch):
         assert torch.equal(want, got) and len(asked) == 1
 
 
+@pytest.mark.parametrize("field,dtype", [("indices", torch.int16), ("indices", torch.int64), ("indptr", torch.int64), ("indptr", torch.int16)])
+def test_delivery_and_segment_offsets_refuse_other_types_before_reading_them(field, dtype):
+    rng = np.random.default_rng(10)
+    n, L, nnz = 600, 6, 600 * 150
+    table = ops.SynapseTable.from_edges(*_edges(rng, n, n, nnz), n, n)
+    setattr(table, field, getattr(table, field).to(dtype))
+    ids, count = torch.arange(n, device="cuda", dtype=torch.int32), torch.tensor([n], device="cuda", dtype=torch.int32)
+    assert 0 < table.range_rows_min(n, 1, L) <= n
+    with pytest.raises(TypeError, match=field):
+        ops.csr_propagate_scatter(ids, count, table, torch.zeros(L, 4, n, device="cuda"), n, 1, 4)
+    with pytest.raises(TypeError, match=field):
+        table.segment_offsets(7, 30)
+    assert getattr(table, "_ranges", None) is None
+
+
 @pytest.mark.parametrize("span,n_groups", [(7, 30), (64, 4), (1, 211), (300, 1), (100, 2)])
 def test_segment_offsets_are_what_a_search_finds(span, n_groups):
     """Empty rows, rows of one synapse and of several chunks, repeated targets, targets beyond the last group, first and last groups empty."""
