@@ -319,59 +319,51 @@ __global__ __launch_bounds__(kBlock) void compact_write_fused_kernel(const uint6
     }
 }
 
-// The bits of up to kOneLaunchWords words in ONE launch of one workgroup: a wavefront holds a run of up to kWordsPerLane x 64 words in
-// registers, counts them, and writes its ids behind those of the wavefronts before it.  What bounds it is the launch and three trips: one
-// launch against two, 4.6 % of the elements on, us: 5,000 elements 2.1 / 3.4, 30,011 2.3 / 3.9, 65,536 2.7 / 4.4, 131,072 3.5 / 4.4; and the
-// host is through with it 3.2 us earlier.  (With three elements in ten on, as no spikes are, one workgroup is no faster: 30,011 5.5 / 5.6.)
-constexpr int kOneBlock = 1024, kWordsPerLane = 1;
-constexpr int64_t kOneLaunchWords = (int64_t)kOneBlock * kWordsPerLane;
-__global__ __launch_bounds__(kOneBlock) void compact_one_kernel(const uint64_t *__restrict__ bits, int64_t n_words, int64_t n,
-                                                                int32_t *__restrict__ ids, int32_t *__restrict__ count)
+// The bits of up to kOneLaunchWords words in ONE launch of one workgroup: a thread holds a word, a wavefront counts its 64 and writes
+// its ids behind those of the wavefronts before it.  What bounds it with few of them on is the launch and three trips, with many the
+// instructions of one compute unit.  One launch / two, us in a captured graph, 4.6 % on: 5,000 elements 1.9 / 3.4, 30,011 2.1 / 3.9, 65,536 2.4 / 3.9
+// (in a loop of calls 4.0 / 6.9, the host's time); three in ten on: 30,011 5.1 / 5.6, 49,152 5.9 / 6.0, 65,536 6.8 / 5.9 (loop 6.9 / 6.9); all on: 65,536 6.9 / 11.6.
+// It ends at a word a thread: with two words a thread 131,072 elements took 3.4 / 4.0 at 4.6 % on, but 15.2 / 6.4 at three in ten.  The scalar base and
+// mask of the dense way: 8.3 -> 6.8 at 65,536 with three in ten on.
+constexpr int kOneLaunchWords = 1024;
+__global__ __launch_bounds__(kOneLaunchWords) void compact_one_kernel(const uint64_t *__restrict__ bits, int64_t n_words, int64_t n,
+                                                                      int32_t *__restrict__ ids, int32_t *__restrict__ count)
 {
-    __shared__ unsigned total_l[kOneBlock / kWave];
-    const int lane = lane_id(), wave = threadIdx.x / kWave;
-    const int per = (int)((n_words + kOneBlock - 1) / kOneBlock);
-    const int64_t first = (int64_t)wave * per * kWave;
-    unsigned long long v[kWordsPerLane];
-    unsigned in[kWordsPerLane], own = 0u;
-#pragma unroll
-    for (int i = 0; i < kWordsPerLane; ++i) v[i] = i < per ? load_word(bits, first + i * kWave + lane, n_words, n) : 0ull;
-#pragma unroll
-    for (int i = 0; i < kWordsPerLane; ++i) {
-        in[i] = wave_inclusive_scan((unsigned)__popcll(v[i]));
-        own += (unsigned)__builtin_amdgcn_readlane((int)in[i], kWave - 1);
-    }
-    if (lane == 0) total_l[wave] = own;
+    constexpr int kWaves = kOneLaunchWords / kWave;
+    __shared__ unsigned total_l[kWaves];
+    const int lane = lane_id(), wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
+    const unsigned long long v = load_word(bits, threadIdx.x, n_words, n);
+    const unsigned in = wave_inclusive_scan((unsigned)__popcll(v));
+    const unsigned here = (unsigned)__builtin_amdgcn_readlane((int)in, kWave - 1);
+    if (lane == 0) total_l[wave] = here;
     __syncthreads();
     unsigned at = 0u, total = 0u;
 #pragma unroll
-    for (int w = 0; w < kOneBlock / kWave; ++w) {
+    for (int w = 0; w < kWaves; ++w) {
         if (w < wave) at += total_l[w];
         total += total_l[w];
     }
     if (threadIdx.x == 0) *count = (int32_t)total;
-#pragma unroll
-    for (int i = 0; i < kWordsPerLane; ++i) {
-        const unsigned here = (unsigned)__builtin_amdgcn_readlane((int)in[i], kWave - 1);
-        if (here > 8 * kWave) {
-            // many of them: word by word, so that a store's ids lie side by side
+    if (here > 8 * kWave) {
+        // many of them: word by word, so that a store's ids lie side by side
+        const int32_t first = wave * kWave * 64 + lane;
+        at = (unsigned)__builtin_amdgcn_readfirstlane((int)at);
 #pragma unroll 16
-            for (int l = 0; l < kWave; ++l) {
-                const unsigned long long m = bcast_u64(v[i], l);
-                if ((m >> lane) & 1ull) ids[at + lane_prefix(m)] = (int32_t)((first + i * kWave + l) << 6) + lane;
-                at += (unsigned)__popcll(m);
-            }
-            continue;
+        for (int l = 0; l < kWave; ++l) {
+            const unsigned long long m = bcast_u64(v, l);
+            int32_t *__restrict__ to = ids + at;  // (a scalar base: the lanes' part is their place in the word)
+            if (__builtin_amdgcn_inverse_ballot_w64(m)) to[lane_prefix(m)] = first + 64 * l;
+            at += (unsigned)__popcll(m);
         }
-        unsigned pos = at + in[i] - (unsigned)__popcll(v[i]);
-        const int32_t base = (int32_t)((first + i * kWave + lane) << 6);
-        unsigned long long m = v[i];
-        while (m) {
-            const int b = __ffsll((long long)m) - 1;
-            m &= m - 1ull;
-            ids[pos++] = base + b;
-        }
-        at += here;
+        return;
+    }
+    unsigned pos = at + in - (unsigned)__popcll(v);
+    const int32_t base = (int32_t)(threadIdx.x << 6);
+    unsigned long long m = v;
+    while (m) {
+        const int b = __ffsll((long long)m) - 1;
+        m &= m - 1ull;
+        ids[pos++] = base + b;
     }
 }
 
@@ -830,7 +822,7 @@ static int compact_from_bits(const uint64_t *bits, int64_t n, int32_t *ids, int3
     const int64_t n_words = n_words_of(n);
     const int n_blocks = (int)n_blocks_of(n);
     if (n_words <= kOneLaunchWords) {
-        hipLaunchKernelGGL(compact_one_kernel, dim3(1), dim3(kOneBlock), 0, stream, bits, n_words, n, ids, count);
+        hipLaunchKernelGGL(compact_one_kernel, dim3(1), dim3(kOneLaunchWords), 0, stream, bits, n_words, n, ids, count);
         BMTK_CHECK_LAUNCH("spikes_compact");
         return BMTK_OK;
     }
