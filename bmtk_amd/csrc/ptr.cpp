@@ -1,7 +1,7 @@
 // _ptr.ptr(tensor, dtype=None, numel=None, name="tensor"): the device pointer of a tensor after the checks of ops._p, which
 // every operation makes of every argument.  Asked through Python they are five calls a tensor, 0.34 us, here 0.07; an update in a caller's own step
 // loop has nine tensors, and such a loop (30,011 neurons) waits for the host: 23.5 -> 19.3 us a step.  Whatever is not a plain device tensor that passes, errors
-// included, goes to the function given to set_general (ops' own).
+// included, goes to the function given to set_general (ops' own).  built_for: the torch whose headers it was compiled with.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
@@ -69,4 +69,12 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_ptr", nullptr, -1, methods, nullp
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__ptr() { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit__ptr()
+{
+    PyObject *m = PyModule_Create(&module);
+    if (m != nullptr && PyModule_AddStringConstant(m, "built_for", BMTK_AMD_TORCH) != 0) {
+        Py_DECREF(m);
+        return nullptr;
+    }
+    return m;
+}

@@ -43,12 +43,19 @@ def _p(t, dtype=None, numel=None, name="tensor"):
     return t.data_ptr()
 
 
-try:  # (the same checks in native code, where it has been built)
-    from . import _ptr
-    _ptr.set_general(_p)
-    _p = _ptr.ptr
-except ImportError:
-    pass
+def _native(general):
+    """The same checks in native code, where that has been built for this torch (it reads a tensor's fields in place)."""
+    try:
+        from . import _ptr
+    except ImportError:
+        return general
+    if getattr(_ptr, "built_for", None) != str(torch.__version__):
+        return general
+    _ptr.set_general(general)
+    return _ptr.ptr
+
+
+_p = _native(_p)
 
 
 def n_words(ne):
