@@ -487,6 +487,17 @@ def test_rate_loss_matches_64_bits(n, batch, n_pops):
             np.testing.assert_allclose(g2.detach().cpu().numpy(), g.cpu().numpy(), rtol=1e-4, atol=float(scale[size > 0].max()) * 1e-6)
 
 
+def test_rate_loss_forms_that_the_kernel_does_not_take():
+    n, batch, n_pops = 300, 12, 17
+    counts, pop = torch.zeros(n * batch, dtype=torch.int32, device="cuda"), torch.arange(n, device="cuda") % n_pops
+    targets = torch.full((batch, n_pops), 0.01, device="cuda")
+    args = (counts, 200, batch, pop, targets)
+    assert training._plain(*args)
+    for at, other in ((0, counts.long()), (0, counts.repeat_interleave(2)[::2]), (0, counts.cpu()), (1, 200.0), (1, np.int64(200)), (3, pop.int()),
+                      (4, targets.t().contiguous().t()), (4, targets.clone().requires_grad_()), (4, targets.double())):
+        assert not training._plain(*args[:at], other, *args[at + 1:])
+
+
 def test_rate_loss_refuses_populations_that_do_not_exist():
     counts, targets = torch.ones(8, dtype=torch.int32, device="cuda"), torch.zeros(2, 3, device="cuda")
     for bad in (-1, 3, 1 << 40):
